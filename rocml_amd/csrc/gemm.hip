@@ -5,6 +5,7 @@
 #include "common.h"
 #include "gemm_tile.h"
 #include "gemm_mfma.h"
+#include "gemm_pingpong.h"
 
 ROCML_LAST_ERROR_FN(gemm)
 
@@ -56,6 +57,39 @@ static int launch_mfma_tile_as(const void* x, int ldx, const void* w, int ldw, v
     return 0;
 }
 
+// The same for the 256x256 kernel: one block a CU walks through its share of the tiles (and K pieces).
+template <int EPI>
+static int launch_pingpong(const void* x, int ldx, const void* w, int ldw, void* out, int ldo, int m, int n, int k,
+                           int splits, void* workspace, SplitPlan plan, hipStream_t stream) {
+    static bool ready = false;
+    if (!ready) {
+        if (allow_lds(gemm_pingpong_kernel<EPI>, pingpong::LDS_BYTES, "gemm")) return 1;
+        if (allow_lds(gemm_pingpong_kernel<EPI_F32>, pingpong::LDS_BYTES, "gemm")) return 1;
+        ready = true;
+    }
+    const int tiles_m = ceil_div(m, 256), n_tiles = tiles_m * ceil_div(n, 256);
+    int k_per_split = splits <= 1 ? k : round_up(ceil_div(k, splits), GM_BK);
+    splits = ceil_div(k, k_per_split);
+    const int items = n_tiles * splits, cus = cu_count() / 8 * 8;
+    const int blocks = cus > 0 && round_up(items, 8) > cus ? cus : round_up(items, 8);
+    if (splits <= 1) {
+        gemm_pingpong_kernel<EPI><<<blocks, 512, pingpong::LDS_BYTES, stream>>>(
+            (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, out, ldo, m, n, k, tiles_m, n_tiles, k, 0, items);
+        return 0;
+    }
+    gemm_pingpong_kernel<EPI_F32><<<blocks, 512, pingpong::LDS_BYTES, stream>>>(
+        (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, workspace, n, m, n, k, tiles_m, n_tiles, k_per_split, (long long)m * n, items);
+    if (plan.defer && ldo == n) {
+        *plan.deferred = splits;
+        return 0;
+    }
+    gemm_splitk_reduce_kernel<EPI><<<ceil_div((long long)m * n, 256), 256, 0, stream>>>((const float*)workspace, out, ldo, m, n, splits);
+    return 0;
+}
+
+// Its loads address a tile's rows by 31-bit offsets.
+static bool pingpong_fits(int ldx, int ldw) { return (long long)(ldx > ldw ? ldx : ldw) * 512 < 0x7fff0000ll; }
+
 // The tile shapes of the many-rows kernel, as rows x columns of a block's tile: 128x128 (four waves
 // of 64x64, two blocks a CU), 256x256 (eight waves of 128x64), 256x192 (eight of 64x96), 128x192
 // (four of 64x96), 256x96 (four of 64x96, the whole of up to 256 rows against a narrow strip of
@@ -66,24 +100,23 @@ using GemmTile64x256 = GemmTile<1, 4, 2, 2>;
 
 // What a tile shape costs: microseconds per 64-wide K stage for a CU that holds as many blocks of it
 // as fit (`cap`), when half the chip or less is at work (`light`) and when all of it is (`full`: the
-// memory system is shared and the clock drops under load), and, for the shape of which two fit,
-// for a CU that holds one alone.  Measured on the Qwen3-8B and 14B products at 80 to 8192 rows.
-struct TileKind { int bm, bn, cap; double light, full, alone; int shape; };
+// memory system is shared and the clock drops under load), for the shape of which two fit,
+// for a CU that holds one alone, and what a launch costs beside its stages (`fixed`).
+struct TileKind { int bm, bn, cap; double light, full, alone, fixed; int shape; };
 static const TileKind TILE_KINDS[] = {
-    {128, 128, 2, 1.21, 1.25, 0.88, 1}, {256, 256, 1, 1.55, 1.85, 0.0, 2}, {256, 192, 1, 1.22, 1.50, 0.0, 3},
-    {128, 192, 1, 1.00, 1.04, 0.0, 4},  {256, 96, 1, 1.03, 1.12, 0.0, 5},  {64, 256, 1, 0.93, 1.05, 0.0, 6}};
+    {128, 128, 2, 0.91, 1.03, 0.62, 2.8, 1}, {256, 256, 1, 1.11, 1.37, 0.0, 5.8, 2}, {256, 192, 1, 1.03, 1.32, 0.0, 6.6, 3},
+    {128, 192, 1, 0.74, 0.83, 0.0, 4.8, 4},  {256, 96, 1, 0.80, 0.86, 0.0, 4.4, 5},  {64, 256, 1, 0.70, 0.78, 0.0, 2.7, 6}};
 
 // An estimate of a product's time in microseconds with tiles of `kind` and K cut into `pieces`
 // (each piece the work of a block of its own, 32-bit partial sums written once here and read once
 // by whoever adds them): the rounds of blocks the chip holds at a time, each round as long as its
 // K stages at the rate of the CUs' load, but no shorter than the busiest CU needs to pull its
-// blocks' operands (36 GB/s a CU: with few rows it is the weights' arrival that a block waits for,
+// blocks' operands (60 GB/s a CU: with few rows it is the weights' arrival that a block waits for,
 // and more, smaller blocks pull more at a time); a fixed part for the launch; the bytes the
 // epilogue moves; never less than the weights need to arrive at all.  The constants were fitted
-// to measurements of 103 products (the Qwen3-8B, 14B and 0.6B shapes at 52 to 8192 rows, six tile
-// shapes, one to eight pieces): the choice made on this estimate is 0.9 % behind the best choice
-// on average and within 5 % for nine in ten.
-static double tile_cost(const TileKind& kind, int pieces, int m, int n, int k, int epi, int cus) {
+// to 16 products (the Qwen3-8B, 14B, 0.6B and the 2B designs' layers) at 96 to 8192 rows, each
+// shape with whole K: the estimate is 4.5 to 6 % off (root mean square) per shape.
+static double tile_cost(const TileKind& kind, int pieces, int m, int n, int k, int epi, bool defer, int cus) {
     long long tiles = (long long)ceil_div(m, kind.bm) * ceil_div(n, kind.bn);
     int k_per_piece = round_up(ceil_div(k, pieces), GM_BK);
     pieces = ceil_div(k, k_per_piece);
@@ -99,15 +132,15 @@ static double tile_cost(const TileKind& kind, int pieces, int m, int n, int k, i
     long long rounds = blocks / slots, rest = blocks % slots;
     double t = (double)rounds * stages * stage_us(slots) + (rest ? stages * stage_us(rest) : 0.0);
     double pulled = (double)(kind.bn + (m < kind.bm ? m : kind.bm)) * k_per_piece * 2.0 * (double)ceil_div(blocks, (long long)cus);
-    if (t < pulled / 36.0e3) t = pulled / 36.0e3;
-    t += 3.0;
+    if (t < pulled / 60.0e3) t = pulled / 60.0e3;
+    t += kind.fixed;
     double moved = epi_gated(epi) ? (double)m * n
                    : pieces > 1      ? (double)m * n * 4.0 * pieces
                                      : (double)m * n * 4.0 * (epi == EPI_ACC ? 2.0 : 1.0);
-    t += moved / 2.0e6;
+    t += moved / (pieces > 1 ? 4.0e6 : 8.0e6);                       // (partial sums leave when all blocks end together)
     double floor_us = (double)n * k * 2.0 / 5.5e6;                  // the weights at 5.5 TB/s
     if (t < floor_us) t = floor_us;
-    if (pieces > 1) t += (double)pieces * m * n * 4.0 / 5.0e6;      // the partial sums read again
+    if (pieces > 1) t += (double)pieces * m * n * 4.0 / 5.0e6 + (defer ? 0.0 : 4.0);   // read again, by a kernel of their own unless deferred
     return t;
 }
 
@@ -126,21 +159,23 @@ static int launch_mfma_tile(const void* x, int ldx, const void* w, int ldw, void
     if (shape == 0) {
         double best = 1e30;
         for (const auto& kind : TILE_KINDS) {
+            if (kind.shape == 2 && !pingpong_fits(ldx, ldw)) continue;
             for (int pieces = 1; pieces <= 8 && pieces <= plan.max_splits; ++pieces) {
                 if (pieces > 1 && (epi_gated(EPI) || k / pieces < 256 || !workspace ||
                                    (long long)pieces * m * n * (long long)sizeof(float) > workspace_bytes))
                     break;
-                double t = tile_cost(kind, pieces, m, n, k, EPI, cus);
+                double t = tile_cost(kind, pieces, m, n, k, EPI, plan.defer && ldo == n, cus);
                 if (t < best) { best = t; shape = kind.shape; splits = pieces; }
             }
         }
     }
+    if (shape == 2 && !pingpong_fits(ldx, ldw)) shape = 1;
     switch (shape) {
         case 6: return launch_mfma_tile_as<EPI, GemmTile64x256>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
         case 5: return launch_mfma_tile_as<EPI, GemmTile256x96>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
         case 4: return launch_mfma_tile_as<EPI, GemmTile128x192>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
         case 3: return launch_mfma_tile_as<EPI, GemmTile192>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
-        case 2: return launch_mfma_tile_as<EPI, GemmTile256>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
+        case 2: return launch_pingpong<EPI>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
         default: return launch_mfma_tile_as<EPI, GemmTile128>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
     }
 }

@@ -4,14 +4,17 @@
 //
 // Kernels:
 //  * gemm_mfma_kernel, many rows (prefill): an output tile per block, each wave a grid of
-//    v_mfma_f32_32x32x16_bf16 tiles (128x64 per wave in the 256-wide shapes, 64x64 in the
-//    128x128 one); K staged 64 at a time through double-buffered LDS with one barrier per stage;
-//    rows padded by 16 bytes so that 128-bit LDS reads of 16 rows fall into 16 different bank
-//    groups.  The idea of the tiling (big tile per block, a grid of fragments per wave, padded
-//    double-buffered LDS) is the reference's WMMA kernel
+//    v_mfma_f32_16x16x32_bf16 tiles (64x64 or 64x96 per wave); K staged 64 at a time through
+//    double-buffered LDS with one barrier per stage; rows padded by 16 bytes so that 128-bit LDS
+//    reads of 16 rows fall into 16 different bank groups.  The idea of the tiling (big tile per
+//    block, a grid of fragments per wave, padded double-buffered LDS) is the reference's WMMA kernel
 //    (rocml-kernels/kernels/gemm_xwt_wmma_impl.h:211-378); layouts, sizes and the instruction
 //    schedule are for wave64 MFMA.  Blocks are renumbered so that each of the 8 XCDs works on a
-//    contiguous range of tiles and its L2 sees few weight panels.
+//    contiguous range of tiles and its L2 sees few weight panels.  256x256 tiles are
+//    gemm_pingpong_kernel's (gemm_pingpong.h).
+//    The 16x16x32 product and not 32x32x16: under load the chip is held by its power, and fed from
+//    registers with random operands the first sustains 2.0 PFLOP/s where the second sustains 1.76
+//    (half the traffic to the sums' registers per operation); in these kernels it is 4 to 16 %.
 //  * gemm_skinny_kernel, few rows (decode, M <= 64): memory-bound; a block owns 16 weight rows
 //    per wave and a K range.  Weights go straight from global memory into MFMA operand
 //    registers (v_mfma_f32_16x16x32_bf16), 8 loads of 16 bytes in flight per lane; the
@@ -54,7 +57,10 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f +
 template <int EPI>
 __device__ __forceinline__ float gated_mul(float g, float u) {
     if (EPI == EPI_RELUGLU) return fmaxf(g, 0.f) * u;
-    return silu_mul(g, u);
+    // silu(g) * u with the hardware's exponential and reciprocal (one unit in the last place each): the result is rounded
+    // to 8 bits, and the exact division and exponential were 5 % of the 256x256 product (1,101 against 1,047 us at
+    // 8192 x 24576 x 4096)
+    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504088896341f)) * u;
 }
 
 // The scale of a norm whose product-side half was done by the producer of the residual stream
@@ -185,17 +191,8 @@ __device__ __forceinline__ void epilogue_store(void* out, size_t idx, float v) {
 }
 
 // ---- many rows ---------------------------------------------------------------------------
-// One kernel, two shapes (see GemmTile below): 256x256 with eight waves (two per SIMD, each
-// 128x64) for products wide enough to give every CU such a tile, 128x128 with four waves of
-// 64x64 (two blocks per CU) for the rest.  (256x128 with four waves of 128x64 was tried: one
-// wave per SIMD has nobody to cover for it while it waits for weights from HBM.  Reading four
-// bytes of every row's line some stages ahead, to pull it into L2, was tried too: the extra
-// requests cost more than the earlier arrival gains, also when only one block of every tile
-// column (for the weights) and one column in four (for the activations) does it.  Loading the operands straight into LDS
-// (global_load_lds_dwordx4, K staged 32 at a time in five unpadded, XOR-swizzled buffers) was
-// tried as well and gave the same results about 7% slower: a barrier every 16 products per wave,
-// and the compiler answers such loads with a full wait on the LDS counter before the first
-// product of every stage.)
+// One kernel, several shapes (see GemmTile below) with whole K or pieces of it; which one a product gets is the
+// host's estimate (tile_cost in gemm.hip).
 constexpr int GM_BK = 64;
 constexpr int GM_BAND = 8;                             // tile rows of a band (see the kernel)
 constexpr int GM_ROW = GM_BK / 8 + 1;                 // u32x4_t per LDS row, one of padding
@@ -203,7 +200,8 @@ constexpr int GM_ROW = GM_BK / 8 + 1;                 // u32x4_t per LDS row, on
 template <int WAVES_M_, int WAVES_N_, int TM_, int TN_>
 struct GemmTile {
     static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;   // waves along M and N
-    static constexpr int TM = TM_, TN = TN_;                        // 32x32 MFMA tiles per wave
+    static constexpr int TM = TM_, TN = TN_;                        // a wave's tile in units of 32x32
+    static constexpr int MT = 2 * TM, NT = 2 * TN;                  // 16-row operand tiles per wave
     static constexpr int BM = WAVES_M * TM * 32, BN = WAVES_N * TN * 32;
     static constexpr int THREADS = 64 * WAVES_M * WAVES_N;
     static constexpr int PASS_ROWS = THREADS / 8;                   // tile rows one pass loads
@@ -211,45 +209,82 @@ struct GemmTile {
     static constexpr int LDS_BYTES = 2 * (BM + BN) * GM_ROW * 16;   // two stages
 };
 using GemmTile128 = GemmTile<2, 2, 2, 2>;
-using GemmTile256 = GemmTile<2, 4, 4, 2>;       // eight waves (two per SIMD), 128x64 each
+using GemmTile256 = GemmTile<2, 4, 4, 2>;       // eight waves (two per SIMD), 128x64 each: gemm_pingpong_kernel
 using GemmTile192 = GemmTile<4, 2, 2, 3>;       // 256 rows x 192 columns, eight waves of 64x96
 
-// Accumulator element e of a lane: row 8*(e/4) + 4*(lane/32) + e%4, column lane%32.
+// Operand tiles whose columns are dealt to the lanes together: a lane's sums of `tile_deal` tiles are 4 * tile_deal
+// neighbouring columns of a row and leave in one store, and the four lanes of a row store 64 bytes side by side (32 for
+// the gated result of the 96-wide waves).  Pieces of 16 bytes 64 bytes apart instead made four times the requests and the
+// 32-bit products of 512 rows 25 % slower.
 template <int EPI, typename T>
-__device__ __forceinline__ void tile_epilogue(f32x16_t (&acc)[T::TM][T::TN], void* out, int ldo, int m, int n,
+constexpr int tile_deal() {
+    return epi_gated(EPI) ? (T::NT % 4 == 0 ? 4 : 2) : EPI == EPI_BF16 || EPI == EPI_RELU2 ? 2 : 1;
+}
+
+// Where weight row r of a block's tile lies in LDS, so that the sums come out as above.
+template <int DEAL>
+__device__ __forceinline__ int tile_lds_row(int r) {
+    int in = r % (16 * DEAL);
+    return r - in + in / 4 % DEAL * 16 + in / (4 * DEAL) * 4 + in % 4;
+}
+
+// acc[i][j][e]: row 16*i + lane%16 of the wave's rows; tile j = d * DEAL + t holds column
+// d * DEAL*16 + lane/16 * DEAL*4 + 4*t + e of its columns.
+template <int EPI, typename T>
+__device__ __forceinline__ void tile_epilogue(f32x4_t (&acc)[T::MT][T::NT], void* out, int ldo, int m, int n,
                                               int m0, int n0, int wm, int wn, int lane) {
+    constexpr int DEAL = tile_deal<EPI, T>();
+    constexpr bool NARROW = EPI == EPI_BF16 || EPI == EPI_RELU2 || epi_gated(EPI);
+    constexpr int PER = epi_gated(EPI) ? 2 * DEAL : 4 * DEAL;        // values of a store
+    static_assert(PER * (NARROW ? 2 : 4) <= 16 && T::NT % DEAL == 0, "one store of at most 16 bytes");
+    const int n_out = epi_gated(EPI) ? n >> 1 : n;
+    const bool aligned = ((size_t)out % (PER * (NARROW ? 2 : 4))) == 0 && ldo % PER == 0;
 #pragma unroll
-    for (int i = 0; i < T::TM; ++i)
+    for (int i = 0; i < T::MT; ++i) {
+        int gm = m0 + (wm * T::MT + i) * 16 + (lane & 15);
+        if (gm >= m) continue;
 #pragma unroll
-        for (int j = 0; j < T::TN; ++j) {
-            int gn = n0 + (wn * T::TN + j) * 32 + (lane & 31);
-            if (epi_gated(EPI)) {
-                // Neighbouring lanes hold neighbouring columns: the even one the gate, the odd one
-                // the up value of one output column.  Of two neighbouring rows the even lane
-                // finishes the first and the odd lane the second: one exchange per pair of rows,
-                // and every lane has half of the exponentials and stores.
-                bool odd = lane & 1;
+        for (int d = 0; d < T::NT / DEAL; ++d) {
+            int gn = n0 + wn * T::NT * 16 + (d * 4 + (lane >> 4)) * 4 * DEAL;
+            int go = epi_gated(EPI) ? gn >> 1 : gn;
+            size_t at = (size_t)gm * ldo + go;
+            float v[PER];
 #pragma unroll
-                for (int e = 0; e < 16; e += 2) {
-                    float first = acc[i][j][e], second = acc[i][j][e + 1];
-                    float got = __shfl_xor(odd ? first : second, 1, 64);    // even: up of row e; odd: gate of row e+1
-                    float gate = odd ? got : first, up = odd ? second : got;
-                    int gm = m0 + (wm * T::TM + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3) + (odd ? 1 : 0);
-                    if (gm < m && (gn | 1) < n)
-                        ((bf16_t*)out)[(size_t)gm * ldo + (gn >> 1)] = f32_to_bf16(gated_mul<EPI>(gate, up));
+            for (int c = 0; c < PER; ++c) {
+                if (epi_gated(EPI)) v[c] = gated_mul<EPI>(acc[i][d * DEAL + c / 2][2 * c % 4], acc[i][d * DEAL + c / 2][2 * c % 4 + 1]);
+                else v[c] = acc[i][d * DEAL + c / 4][c % 4];
+                if (EPI == EPI_RELU2) { v[c] = fmaxf(v[c], 0.f); v[c] *= v[c]; }
+            }
+            if (aligned && go + PER <= n_out) {
+                if constexpr (NARROW) {
+                    uint32_t pk[PER / 2];
+#pragma unroll
+                    for (int h = 0; h < PER / 2; ++h) pk[h] = f32x2_to_bf16x2(v[2 * h], v[2 * h + 1]);
+                    if constexpr (PER == 8) *(u32x4_t*)((bf16_t*)out + at) = u32x4_t{pk[0], pk[1], pk[2], pk[3]};
+                    else *(uint2*)((bf16_t*)out + at) = make_uint2(pk[0], pk[1]);
+                } else {
+                    f32x4_t* to = (f32x4_t*)((float*)out + at);
+                    f32x4_t four = {v[0], v[1], v[2], v[3]};
+                    if (EPI == EPI_ACC) four += *to;
+                    *to = four;
                 }
                 continue;
             }
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                int gm = m0 + (wm * T::TM + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-                if (gm < m && gn < n) epilogue_store<EPI>(out, (size_t)gm * ldo + gn, acc[i][j][e]);
+            for (int c = 0; c < PER; ++c) {
+                if (go + c >= n_out) break;
+                if (NARROW) ((bf16_t*)out)[at + c] = f32_to_bf16(v[c]);
+                else if (EPI == EPI_ACC) ((float*)out)[at + c] += v[c];
+                else ((float*)out)[at + c] = v[c];
             }
         }
+    }
 }
 
+// (two waves a SIMD for every shape: with one, the compiler keeps sums in the accumulation registers and moves them to and
+// fro around every product)
 template <int EPI, typename T>
-__global__ void __launch_bounds__(T::THREADS)
+__global__ void __launch_bounds__(T::THREADS, 2)
 gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ w, int ldw,
                  void* __restrict__ out, int ldo, int m, int n, int k, int tiles_m, int n_tiles,
                  int k_per_split, long long split_stride) {
@@ -259,14 +294,13 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     extern __shared__ u32x4_t gm_smem[];              // [2 stages][A: BM rows | B: BN rows][GM_ROW]
     constexpr int STAGE = (T::BM + T::BN) * GM_ROW;
     constexpr int NREG = T::PA + T::PB;               // 16-byte pieces a thread moves per K stage
-    constexpr int PROD = T::TM * T::TN;               // products per 16-wide K slice
-    constexpr int KK = GM_BK / 16;                    // slices per stage
-    static_assert(KK == 4, "the schedule below is written for four slices per stage");
-    // piece r is stored after product r * SPAN / NREG of the first three slices (SPAN products);
-    // its register is refilled one product later when every store has a free product behind it,
-    // else right behind the store
-    constexpr int SPAN = 3 * PROD;
-    static_assert(SPAN >= NREG, "the stores must fit into the first three slices");
+    constexpr int GROUPS = 2 * T::MT;                 // groups of NT products (one operand tile of x) per stage
+    // Products of a stage before the barrier: the last groups of the second slice come behind it.  A stage's stores are
+    // spread over the products before it: piece r is stored after product r * SPAN / NREG; its register is refilled one
+    // product later when every store has a free product behind it, else right behind the store.
+    constexpr int TAIL = 3;
+    constexpr int SPAN = (GROUPS - TAIL) * T::NT;
+    static_assert(SPAN >= NREG, "the stores must fit before the barrier");
     constexpr bool REFILL_LATER = SPAN >= 2 * NREG;
     int per_xcd = gridDim.x / 8;
     int logical = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
@@ -288,28 +322,26 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     int wm = wave / T::WAVES_N, wn = wave % T::WAVES_N;
     int lrow = tid >> 3, lkc = tid & 7;
     int nk = (k + GM_BK - 1) / GM_BK;
-    f32x16_t acc[T::TM][T::TN];
+    f32x4_t acc[T::MT][T::NT];
 #pragma unroll
-    for (int i = 0; i < T::TM; ++i)
+    for (int i = 0; i < T::MT; ++i)
 #pragma unroll
-        for (int j = 0; j < T::TN; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+        for (int j = 0; j < T::NT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-    // Schedule of one K stage (64 wide = four slices of 16), written out by hand and pinned with
+    // Schedule of one K stage (64 wide = two slices of 32), written out by hand and pinned with
     // scheduling barriers, because left alone the compiler sinks every LDS read to its first use
     // and gathers the stores behind the products:
-    //  * the operand pieces of the next slice are read from LDS before the products of the
-    //    current slice are issued (two register sets);
+    //  * an operand tile of x is read from LDS three groups of products before its own (a ring of
+    //    four), a slice's weights during the slice before it (two register sets);
     //  * the pieces of the next stage, loaded from global memory one stage ago, are stored to the
-    //    other LDS buffer between the products of slices 0 to 2 (evenly: LDS takes a 128-bit
+    //    other LDS buffer between the products before the barrier (evenly: LDS takes a 128-bit
     //    store at a quarter of the rate of a read, and bunched stores hold up the operand reads
     //    behind them), and each register is refilled from the stage after that: the memory pipes
     //    work while the matrix core does, and a load has a whole stage to arrive;
-    //  * the one barrier of a stage stands after slice 2.  By then every wave has stored its
-    //    pieces of the next stage and has read the last pieces of this one, so during slice 3 the
-    //    first operands of the next stage are fetched and the matrix core does not wait for LDS
-    //    when the stage changes.
+    //  * the one barrier of a stage stands three groups before its end.  By then every wave has
+    //    stored its pieces of the next stage and has read the last pieces of this one, so during the
+    //    last groups the first operands of the next stage are fetched and the matrix core does not
+    //    wait for LDS when the stage changes.
     // Loads go to clamped addresses and are used as they come: rows beyond M or N only feed
     // outputs that are never stored, and a piece beyond K is zeroed when it is stored to LDS.
     // Nothing in the loop is conditional, so the count of outstanding loads is known at every
@@ -323,11 +355,11 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
         int row = lrow + T::PASS_ROWS * (is_a ? r : r - T::PA);
         src[r] = is_a ? x + (size_t)min(m0 + row, m - 1) * ldx + lkc * 8
                       : w + (size_t)min(n0 + row, n - 1) * ldw + lkc * 8;
-        dst[r] = (is_a ? 0 : T::BM * GM_ROW) + row * GM_ROW + lkc;
+        dst[r] = (is_a ? row : T::BM + tile_lds_row<tile_deal<EPI, T>()>(row)) * GM_ROW + lkc;
     }
     const u32x4_t zero = {0u, 0u, 0u, 0u};
-    int fa = (wm * T::TM * 32 + (lane & 31)) * GM_ROW + (lane >> 5);
-    int fb = T::BM * GM_ROW + (wn * T::TN * 32 + (lane & 31)) * GM_ROW + (lane >> 5);
+    int fa = (wm * T::MT * 16 + (lane & 15)) * GM_ROW + (lane >> 4);
+    int fb = (T::BM + wn * T::NT * 16 + (lane & 15)) * GM_ROW + (lane >> 4);
     // offset of this thread's piece in stage kt, or back to the row's start when it is beyond K
 #define GM_KOFF(kt_) ((kt_) * GM_BK + lkc * 8 < k ? (kt_) * GM_BK : -lkc * 8)
     {
@@ -342,34 +374,45 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
         for (int r = 0; r < NREG; ++r) reg[r] = *(const u32x4_t*)(src[r] + o1);
     }
     __syncthreads();
-    bf16x8_t a[2][T::TM], b[2][T::TN];
+    // operands: a ring of four tiles of x, three groups ahead of the products; two sets of the weights' tiles, one a slice
+    bf16x8_t a[4], b[2][T::NT];
 #pragma unroll
-    for (int i = 0; i < T::TM; ++i) a[0][i] = as_frag4(gm_smem[fa + i * 32 * GM_ROW]);
+    for (int j = 0; j < T::NT; ++j) b[0][j] = as_frag4(gm_smem[fb + j * 16 * GM_ROW]);
 #pragma unroll
-    for (int j = 0; j < T::TN; ++j) b[0][j] = as_frag4(gm_smem[fb + j * 32 * GM_ROW]);
+    for (int i = 0; i < TAIL; ++i) a[i] = as_frag4(gm_smem[fa + i * 16 * GM_ROW]);
     for (int kt = 0; kt < nk; ++kt) {
         const u32x4_t* cur = gm_smem + (kt & 1) * STAGE;
         u32x4_t* nxt = gm_smem + ((kt + 1) & 1) * STAGE;
         bool in1 = (kt + 1) * GM_BK + lkc * 8 < k;    // is the piece held in registers inside K
         int o2 = GM_KOFF(kt + 2);
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-            int c = kk & 1;
-            const u32x4_t* from = kk + 1 < KK ? cur + (kk + 1) * 2 : nxt;   // slice 3 fetches the next stage's slice 0
+        for (int g = 0; g < GROUPS; ++g) {
+            constexpr int MT = T::MT, NT = T::NT;
+            const int slice = g / MT, i = g % MT;
+            if (g == GROUPS - TAIL) __syncthreads();  // (compiles to nothing in the other groups: g is unrolled)
+            // the tile of x three groups ahead, of the next stage behind the barrier
+            const int ga = g + TAIL;
+            const u32x4_t* from = ga < GROUPS ? cur : nxt;
+            a[ga & 3] = as_frag4(from[fa + (ga % MT) * 16 * GM_ROW + (ga % GROUPS) / MT * 4]);
+            // the next slice's weights: spread over the first slice, right behind the barrier for the next stage
+            if (slice == 0) {
 #pragma unroll
-            for (int i = 0; i < T::TM; ++i) a[c ^ 1][i] = as_frag4(from[fa + i * 32 * GM_ROW]);
+                for (int j = 0; j < NT; ++j)
+                    if (j * MT / NT == i) b[1][j] = as_frag4(cur[fb + j * 16 * GM_ROW + 4]);
+            } else if (g >= GROUPS - TAIL) {
 #pragma unroll
-            for (int j = 0; j < T::TN; ++j) b[c ^ 1][j] = as_frag4(from[fb + j * 32 * GM_ROW]);
+                for (int j = 0; j < NT; ++j)
+                    if (j * TAIL / NT == g - (GROUPS - TAIL)) b[0][j] = as_frag4(nxt[fb + j * 16 * GM_ROW]);
+            }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int q = 0; q < PROD; ++q) {
-                acc[q / T::TN][q % T::TN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                    a[c][q / T::TN], b[c][q % T::TN], acc[q / T::TN][q % T::TN], 0, 0, 0);
+            for (int j = 0; j < NT; ++j) {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[slice][j], a[g & 3], acc[i][j], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 // the piece whose place is product s of the stage: r with r * SPAN / NREG == s
-                int slot = kk * PROD + q;
+                const int slot = g * NT + j;
                 int r = (slot * NREG + SPAN - 1) / SPAN;
-                bool here = kk < 3 && r < NREG && r * SPAN / NREG == slot;
+                bool here = slot < SPAN && r < NREG && r * SPAN / NREG == slot;
                 int rp = ((slot - 1) * NREG + SPAN - 1) / SPAN;      // the piece one product earlier
                 bool before = slot >= 1 && slot - 1 < SPAN && rp < NREG && rp * SPAN / NREG == slot - 1;
                 if (here) {
@@ -380,7 +423,6 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (kk == 2) __syncthreads();
         }
     }
 #undef GM_KOFF

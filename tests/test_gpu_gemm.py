@@ -62,6 +62,27 @@ def test_bfloat16_algorithms(m, n, k, algo):
     assert float((acc.double() - (ref + base.double())).abs().max()) < 2e-5 * scale, "accumulating"
 
 
+@pytest.mark.parametrize("m,n,k", [(4200, 4400, 72), (4100, 4609, 8), (2305, 8200, 200)])
+@pytest.mark.parametrize("epilogue", [None, "swiglu", "relu2"])
+def test_more_tiles_than_compute_units(m, n, k, epilogue):
+    """256x256 tiles of which a block walks through several (306, 323 and 330 of them), the rest of K not a whole stage; the
+    operands are column ranges of wider matrices that hold NaN beside them."""
+    n -= n % 2 if epilogue == "swiglu" else 0
+    x, w = _operands(m, n, k, torch.bfloat16, 7)
+    wide_x, wide_w = torch.full((m, k + 64), float("nan"), dtype=torch.bfloat16, device="cuda"), torch.full(
+        (n, k + 72), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide_x[:, 8:8 + k], wide_w[:, 16:16 + k] = x, w
+    ref = _ref(x, w)
+    if epilogue == "swiglu":
+        ref = torch.nn.functional.silu(ref[:, 0::2]) * ref[:, 1::2]
+    elif epilogue == "relu2":
+        ref = ref.clamp(min=0) ** 2
+    out = torch.empty(ref.shape, dtype=torch.float32 if epilogue is None else torch.bfloat16, device="cuda")
+    ops.gemm(wide_x[:, 8:8 + k], wide_w[:, 16:16 + k], out, algo=TILE256, epilogue=epilogue)
+    # 32-bit sums of at most 200 products; a bfloat16 result is rounded to 8 bits
+    assert float((out.double() - ref).abs().max()) < (2e-5 if epilogue is None else 5e-3) * max(1.0, float(ref.abs().max()))
+
+
 def test_strided_rows_and_refusals():
     from rocml_amd.errors import KernelError
     big = torch.randn(40, 200, device="cuda").to(torch.bfloat16)
