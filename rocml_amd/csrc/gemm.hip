@@ -25,28 +25,28 @@ static int allow_lds(K kernel, int bytes, const char* name) {
 
 struct SplitPlan { int defer; int* deferred; RowScale rs; int max_splits; };   // max_splits: the most K pieces the caller wants
 
-template <int EPI, typename T>
+template <int EPI, typename T, typename E = bf16_t>
 static int launch_mfma_tile_as(const void* x, int ldx, const void* w, int ldw, void* out, int ldo, int m,
                                int n, int k, int splits, void* workspace, SplitPlan plan, hipStream_t stream) {
     static bool ready = false;
     if (!ready) {
-        if (allow_lds(gemm_mfma_kernel<EPI, T>, T::LDS_BYTES, "gemm")) return 1;
-        if (allow_lds(gemm_mfma_kernel<EPI_F32, T>, T::LDS_BYTES, "gemm")) return 1;
+        if (allow_lds(gemm_mfma_kernel<EPI, T, E>, T::LDS_BYTES, "gemm")) return 1;
+        if (allow_lds(gemm_mfma_kernel<EPI_F32, T, E>, T::LDS_BYTES, "gemm")) return 1;
         ready = true;
     }
     int tiles_m = ceil_div(m, T::BM), tiles_n = ceil_div(n, T::BN);
     int n_tiles = tiles_m * tiles_n;
     if (splits <= 1) {
-        gemm_mfma_kernel<EPI, T><<<round_up(n_tiles, 8), T::THREADS, T::LDS_BYTES, stream>>>(
-            (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, out, ldo, m, n, k, tiles_m, n_tiles, k, 0);
+        gemm_mfma_kernel<EPI, T, E><<<round_up(n_tiles, 8), T::THREADS, T::LDS_BYTES, stream>>>(
+            (const E*)x, ldx, (const E*)w, ldw, out, ldo, m, n, k, tiles_m, n_tiles, k, 0);
         return 0;
     }
     // K cut in pieces: 32-bit partial sums [piece][M][N] in the workspace, added in order by the
     // caller's next kernel or by the reduce kernel here
-    int k_per_split = round_up(ceil_div(k, splits), GM_BK);
+    int k_per_split = round_up(ceil_div(k, splits), 128 / (int)sizeof(E));
     splits = ceil_div(k, k_per_split);
-    gemm_mfma_kernel<EPI_F32, T><<<round_up(n_tiles * splits, 8), T::THREADS, T::LDS_BYTES, stream>>>(
-        (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, workspace, n, m, n, k, tiles_m, n_tiles, k_per_split,
+    gemm_mfma_kernel<EPI_F32, T, E><<<round_up(n_tiles * splits, 8), T::THREADS, T::LDS_BYTES, stream>>>(
+        (const E*)x, ldx, (const E*)w, ldw, workspace, n, m, n, k, tiles_m, n_tiles, k_per_split,
         (long long)m * n);
     if (plan.defer && ldo == n) {
         *plan.deferred = splits;
@@ -86,6 +86,8 @@ static int launch_pingpong(const void* x, int ldx, const void* w, int ldw, void*
     gemm_splitk_reduce_kernel<EPI><<<ceil_div((long long)m * n, 256), 256, 0, stream>>>((const float*)workspace, out, ldo, m, n, splits);
     return 0;
 }
+
+#include "gemm_f32.h"
 
 // Its loads address a tile's rows by 31-bit offsets.
 static bool pingpong_fits(int ldx, int ldw) { return (long long)(ldx > ldw ? ldx : ldw) * 512 < 0x7fff0000ll; }
@@ -622,6 +624,25 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
                          workspace, workspace_bytes,
                          plan, stream);
 #undef BY_EPI
+        if (rc) return rc;
+        ROCML_CHECK_LAUNCH("gemm");
+        return 0;
+    }
+    // 32-bit operands in 16-byte pieces: the 32-bit matrix instructions, the few-rows kernel while its reads of the
+    // activations (every block reads them all) stay below the weights'
+    bool f32_pieces = x_dtype == ROCML_F32 && w_dtype == ROCML_F32 && out_dtype == ROCML_F32 && k % 4 == 0 && ldx % 4 == 0 &&
+                      ldw % 4 == 0 && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
+    if (f32_pieces && algo == ALGO_AUTO) {
+        SplitPlan plan{defer, deferred_splits, RowScale{}, max_splits >= 1 && max_splits < 16 ? max_splits : 16};
+        const float *xf = (const float*)x, *wf = (const float*)w;
+        float* of = (float*)out;
+        int rc;
+#define F32_BY_EPI(fn, ...)                                                                  \
+        (epi == EPI_ACC ? fn<EPI_ACC>(__VA_ARGS__) : epi == EPI_SWIGLU ? fn<EPI_SWIGLU>(__VA_ARGS__) \
+         : epi == EPI_RELUGLU ? fn<EPI_RELUGLU>(__VA_ARGS__) : fn<EPI_F32>(__VA_ARGS__))
+        if (m <= 32) rc = F32_BY_EPI(launch_f32_rows, xf, ldx, wf, ldw, of, ldo, m, n, k, stream);
+        else rc = F32_BY_EPI(launch_f32_tile, xf, ldx, wf, ldw, of, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
+#undef F32_BY_EPI
         if (rc) return rc;
         ROCML_CHECK_LAUNCH("gemm");
         return 0;

@@ -193,7 +193,7 @@ __device__ __forceinline__ void epilogue_store(void* out, size_t idx, float v) {
 // ---- many rows ---------------------------------------------------------------------------
 // One kernel, several shapes (see GemmTile below) with whole K or pieces of it; which one a product gets is the
 // host's estimate (tile_cost in gemm.hip).
-constexpr int GM_BK = 64;
+constexpr int GM_BK = 64;                             // bfloat16 values of a stage: 128 bytes of a row
 constexpr int GM_BAND = 8;                             // tile rows of a band (see the kernel)
 constexpr int GM_ROW = GM_BK / 8 + 1;                 // u32x4_t per LDS row, one of padding
 
@@ -216,8 +216,9 @@ using GemmTile192 = GemmTile<4, 2, 2, 3>;       // 256 rows x 192 columns, eight
 // neighbouring columns of a row and leave in one store, and the four lanes of a row store 64 bytes side by side (32 for
 // the gated result of the 96-wide waves).  Pieces of 16 bytes 64 bytes apart instead made four times the requests and the
 // 32-bit products of 512 rows 25 % slower.
-template <int EPI, typename T>
+template <int EPI, typename T, typename E = bf16_t>
 constexpr int tile_deal() {
+    if (sizeof(E) == 4) return epi_gated(EPI) ? 2 : 1;
     return epi_gated(EPI) ? (T::NT % 4 == 0 ? 4 : 2) : EPI == EPI_BF16 || EPI == EPI_RELU2 ? 2 : 1;
 }
 
@@ -230,11 +231,11 @@ __device__ __forceinline__ int tile_lds_row(int r) {
 
 // acc[i][j][e]: row 16*i + lane%16 of the wave's rows; tile j = d * DEAL + t holds column
 // d * DEAL*16 + lane/16 * DEAL*4 + 4*t + e of its columns.
-template <int EPI, typename T>
+template <int EPI, typename T, typename E = bf16_t>
 __device__ __forceinline__ void tile_epilogue(f32x4_t (&acc)[T::MT][T::NT], void* out, int ldo, int m, int n,
                                               int m0, int n0, int wm, int wn, int lane) {
-    constexpr int DEAL = tile_deal<EPI, T>();
-    constexpr bool NARROW = EPI == EPI_BF16 || EPI == EPI_RELU2 || epi_gated(EPI);
+    constexpr int DEAL = tile_deal<EPI, T, E>();
+    constexpr bool NARROW = sizeof(E) == 2 && (EPI == EPI_BF16 || EPI == EPI_RELU2 || epi_gated(EPI));
     constexpr int PER = epi_gated(EPI) ? 2 * DEAL : 4 * DEAL;        // values of a store
     static_assert(PER * (NARROW ? 2 : 4) <= 16 && T::NT % DEAL == 0, "one store of at most 16 bytes");
     const int n_out = epi_gated(EPI) ? n >> 1 : n;
@@ -251,7 +252,10 @@ __device__ __forceinline__ void tile_epilogue(f32x4_t (&acc)[T::MT][T::NT], void
             float v[PER];
 #pragma unroll
             for (int c = 0; c < PER; ++c) {
-                if (epi_gated(EPI)) v[c] = gated_mul<EPI>(acc[i][d * DEAL + c / 2][2 * c % 4], acc[i][d * DEAL + c / 2][2 * c % 4 + 1]);
+                if (epi_gated(EPI)) {
+                    float gate = acc[i][d * DEAL + c / 2][2 * c % 4], up = acc[i][d * DEAL + c / 2][2 * c % 4 + 1];
+                    v[c] = sizeof(E) == 4 && EPI == EPI_SWIGLU ? silu_mul(gate, up) : gated_mul<EPI>(gate, up);
+                }
                 else v[c] = acc[i][d * DEAL + c / 4][c % 4];
                 if (EPI == EPI_RELU2) { v[c] = fmaxf(v[c], 0.f); v[c] *= v[c]; }
             }
@@ -283,9 +287,10 @@ __device__ __forceinline__ void tile_epilogue(f32x4_t (&acc)[T::MT][T::NT], void
 
 // (two waves a SIMD for every shape: with one, the compiler keeps sums in the accumulation registers and moves them to and
 // fro around every product)
-template <int EPI, typename T>
+// E: the operands' type, bf16_t or float (then a slice of a stage is 16 values of K, multiplied four times four)
+template <int EPI, typename T, typename E = bf16_t>
 __global__ void __launch_bounds__(T::THREADS, 2)
-gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ w, int ldw,
+gemm_mfma_kernel(const E* __restrict__ x, int ldx, const E* __restrict__ w, int ldw,
                  void* __restrict__ out, int ldo, int m, int n, int k, int tiles_m, int n_tiles,
                  int k_per_split, long long split_stride) {
     // With split_stride != 0 the K range is cut into pieces of k_per_split; piece p of a tile is
@@ -298,7 +303,8 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     // Products of a stage before the barrier: the last groups of the second slice come behind it.  A stage's stores are
     // spread over the products before it: piece r is stored after product r * SPAN / NREG; its register is refilled one
     // product later when every store has a free product behind it, else right behind the store.
-    constexpr int TAIL = 3;
+    constexpr int TAIL = T::MT >= 4 ? 3 : 1;
+    constexpr int PIECE = 16 / sizeof(E), BK = 8 * PIECE;     // values of a 16-byte piece and of a stage
     constexpr int SPAN = (GROUPS - TAIL) * T::NT;
     static_assert(SPAN >= NREG, "the stores must fit before the barrier");
     constexpr bool REFILL_LATER = SPAN >= 2 * NREG;
@@ -321,7 +327,7 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int wm = wave / T::WAVES_N, wn = wave % T::WAVES_N;
     int lrow = tid >> 3, lkc = tid & 7;
-    int nk = (k + GM_BK - 1) / GM_BK;
+    int nk = (k + BK - 1) / BK;
     f32x4_t acc[T::MT][T::NT];
 #pragma unroll
     for (int i = 0; i < T::MT; ++i)
@@ -331,14 +337,14 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     // Schedule of one K stage (64 wide = two slices of 32), written out by hand and pinned with
     // scheduling barriers, because left alone the compiler sinks every LDS read to its first use
     // and gathers the stores behind the products:
-    //  * an operand tile of x is read from LDS three groups of products before its own (a ring of
+    //  * an operand tile of x is read from LDS TAIL groups of products before its own (a ring of
     //    four), a slice's weights during the slice before it (two register sets);
     //  * the pieces of the next stage, loaded from global memory one stage ago, are stored to the
     //    other LDS buffer between the products before the barrier (evenly: LDS takes a 128-bit
     //    store at a quarter of the rate of a read, and bunched stores hold up the operand reads
     //    behind them), and each register is refilled from the stage after that: the memory pipes
     //    work while the matrix core does, and a load has a whole stage to arrive;
-    //  * the one barrier of a stage stands three groups before its end.  By then every wave has
+    //  * the one barrier of a stage stands TAIL groups before its end.  By then every wave has
     //    stored its pieces of the next stage and has read the last pieces of this one, so during the
     //    last groups the first operands of the next stage are fetched and the matrix core does not
     //    wait for LDS when the stage changes.
@@ -347,24 +353,24 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     // Nothing in the loop is conditional, so the count of outstanding loads is known at every
     // wait; the last stages load and store pieces nobody reads.
     u32x4_t reg[NREG];
-    const bf16_t* src[NREG];
+    const E* src[NREG];
     int dst[NREG];                                    // LDS index of the piece within a stage
 #pragma unroll
     for (int r = 0; r < NREG; ++r) {
         bool is_a = r < T::PA;
         int row = lrow + T::PASS_ROWS * (is_a ? r : r - T::PA);
-        src[r] = is_a ? x + (size_t)min(m0 + row, m - 1) * ldx + lkc * 8
-                      : w + (size_t)min(n0 + row, n - 1) * ldw + lkc * 8;
-        dst[r] = (is_a ? row : T::BM + tile_lds_row<tile_deal<EPI, T>()>(row)) * GM_ROW + lkc;
+        src[r] = is_a ? x + (size_t)min(m0 + row, m - 1) * ldx + lkc * PIECE
+                      : w + (size_t)min(n0 + row, n - 1) * ldw + lkc * PIECE;
+        dst[r] = (is_a ? row : T::BM + tile_lds_row<tile_deal<EPI, T, E>()>(row)) * GM_ROW + lkc;
     }
     const u32x4_t zero = {0u, 0u, 0u, 0u};
     int fa = (wm * T::MT * 16 + (lane & 15)) * GM_ROW + (lane >> 4);
     int fb = (T::BM + wn * T::NT * 16 + (lane & 15)) * GM_ROW + (lane >> 4);
     // offset of this thread's piece in stage kt, or back to the row's start when it is beyond K
-#define GM_KOFF(kt_) ((kt_) * GM_BK + lkc * 8 < k ? (kt_) * GM_BK : -lkc * 8)
+#define GM_KOFF(kt_) ((kt_) * BK + lkc * PIECE < k ? (kt_) * BK : -lkc * PIECE)
     {
         int o0 = GM_KOFF(0);
-        bool in0 = lkc * 8 < k;
+        bool in0 = lkc * PIECE < k;
 #pragma unroll
         for (int r = 0; r < NREG; ++r) reg[r] = *(const u32x4_t*)(src[r] + o0);
 #pragma unroll
@@ -374,40 +380,47 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
         for (int r = 0; r < NREG; ++r) reg[r] = *(const u32x4_t*)(src[r] + o1);
     }
     __syncthreads();
-    // operands: a ring of four tiles of x, three groups ahead of the products; two sets of the weights' tiles, one a slice
-    bf16x8_t a[4], b[2][T::NT];
+    // operands: a ring of four tiles of x, TAIL groups ahead of the products; two sets of the weights' tiles, one a slice
+    u32x4_t a[4], b[2][T::NT];
 #pragma unroll
-    for (int j = 0; j < T::NT; ++j) b[0][j] = as_frag4(gm_smem[fb + j * 16 * GM_ROW]);
+    for (int j = 0; j < T::NT; ++j) b[0][j] = gm_smem[fb + j * 16 * GM_ROW];
 #pragma unroll
-    for (int i = 0; i < TAIL; ++i) a[i] = as_frag4(gm_smem[fa + i * 16 * GM_ROW]);
+    for (int i = 0; i < TAIL; ++i) a[i] = gm_smem[fa + i * 16 * GM_ROW];
     for (int kt = 0; kt < nk; ++kt) {
         const u32x4_t* cur = gm_smem + (kt & 1) * STAGE;
         u32x4_t* nxt = gm_smem + ((kt + 1) & 1) * STAGE;
-        bool in1 = (kt + 1) * GM_BK + lkc * 8 < k;    // is the piece held in registers inside K
+        bool in1 = (kt + 1) * BK + lkc * PIECE < k;    // is the piece held in registers inside K
         int o2 = GM_KOFF(kt + 2);
 #pragma unroll
         for (int g = 0; g < GROUPS; ++g) {
             constexpr int MT = T::MT, NT = T::NT;
             const int slice = g / MT, i = g % MT;
             if (g == GROUPS - TAIL) __syncthreads();  // (compiles to nothing in the other groups: g is unrolled)
-            // the tile of x three groups ahead, of the next stage behind the barrier
+            // the tile of x TAIL groups ahead, of the next stage behind the barrier
             const int ga = g + TAIL;
             const u32x4_t* from = ga < GROUPS ? cur : nxt;
-            a[ga & 3] = as_frag4(from[fa + (ga % MT) * 16 * GM_ROW + (ga % GROUPS) / MT * 4]);
+            a[ga & 3] = from[fa + (ga % MT) * 16 * GM_ROW + (ga % GROUPS) / MT * 4];
             // the next slice's weights: spread over the first slice, right behind the barrier for the next stage
             if (slice == 0) {
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
-                    if (j * MT / NT == i) b[1][j] = as_frag4(cur[fb + j * 16 * GM_ROW + 4]);
+                    if (j * MT / NT == i) b[1][j] = cur[fb + j * 16 * GM_ROW + 4];
             } else if (g >= GROUPS - TAIL) {
 #pragma unroll
                 for (int j = 0; j < NT; ++j)
-                    if (j * TAIL / NT == g - (GROUPS - TAIL)) b[0][j] = as_frag4(nxt[fb + j * 16 * GM_ROW]);
+                    if (j * TAIL / NT == g - (GROUPS - TAIL)) b[0][j] = nxt[fb + j * 16 * GM_ROW];
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[slice][j], a[g & 3], acc[i][j], 0, 0, 0);
+                if constexpr (sizeof(E) == 2) {
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag4(b[slice][j]), as_frag4(a[g & 3]), acc[i][j], 0, 0, 0);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(b[slice][j][e]), __uint_as_float(a[g & 3][e]),
+                                                                         acc[i][j], 0, 0, 0);
+                }
                 __builtin_amdgcn_sched_barrier(0);
                 // the piece whose place is product s of the stage: r with r * SPAN / NREG == s
                 const int slot = g * NT + j;
@@ -426,7 +439,7 @@ gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
         }
     }
 #undef GM_KOFF
-    tile_epilogue<EPI, T>(acc, out, ldo, m, n, m0, n0, wm, wn, lane);
+    tile_epilogue<EPI, T, E>(acc, out, ldo, m, n, m0, n0, wm, wn, lane);
 }
 
 // ---- few rows ----------------------------------------------------------------------------

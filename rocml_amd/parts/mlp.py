@@ -38,6 +38,8 @@ class GatedMlp(FeedForward):
             self.epilogue = None          # the products' epilogues know the bare activations only
         self.spec = spec
         self.dtype = ctx.dtype
+        # the epilogue is the matrix-core kernels', which take K in pieces of 16 bytes
+        self.fused = self.epilogue is not None and spec.hidden % (8 if ctx.dtype == torch.bfloat16 else 4) == 0
         self.w_gate_up: Optional[torch.Tensor] = None
         self.w_down: Optional[torch.Tensor] = None
 
@@ -53,17 +55,15 @@ class GatedMlp(FeedForward):
         gate, up = tensors["gate_proj.weight"], tensors["up_proj.weight"]
         self.w_gate_up = torch.stack([gate, up], dim=1).reshape(2 * gate.shape[0], gate.shape[1]).contiguous()
         self.w_down = tensors["down_proj.weight"]
-        self.fused = self.epilogue is not None and self.dtype == torch.bfloat16 and self.spec.hidden % 8 == 0
 
     def activation_bytes(self, n_tokens: int) -> int:
         s = self.spec
         size = 2 if self.dtype == torch.bfloat16 else 4
-        fused = self.epilogue is not None and self.dtype == torch.bfloat16 and s.hidden % 8 == 0
-        return n_tokens * s.intermediate * (size + (0 if fused else 8))
+        return n_tokens * s.intermediate * (size + (0 if self.fused else 8))
 
     def takes_row_scale(self, step) -> bool:
         # the gated epilogue of the few-rows products applies it
-        return self.w_gate_up is not None and self.fused and step.n_tokens <= ops.ROW_SCALE_MAX_ROWS
+        return self.w_gate_up is not None and self.fused and self.dtype == torch.bfloat16 and step.n_tokens <= ops.ROW_SCALE_MAX_ROWS
 
     def forward(self, step, xn, x_accum) -> None:
         s = self.spec

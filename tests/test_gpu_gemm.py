@@ -62,6 +62,32 @@ def test_bfloat16_algorithms(m, n, k, algo):
     assert float((acc.double() - (ref + base.double())).abs().max()) < 2e-5 * scale, "accumulating"
 
 
+# rows around 16 and 32 (the few-rows kernel's tiles) and beyond; K of a run of 64, less, and runs with a rest; N that is no tile;
+# products cut along K (narrow, deep) and whole
+@pytest.mark.parametrize("m,n,k", [(1, 5, 4), (2, 384, 96), (16, 300, 1028), (17, 51, 640), (32, 4112, 260), (33, 70, 68), (64, 64, 32),
+                                   (130, 1000, 4100), (700, 130, 2052), (5, 20000, 64)])
+def test_float32_matrix_cores(m, n, k):
+    x, w = _operands(m, n, k, torch.float32, 5)
+    wide = torch.full((m, k + 8), float("nan"), device="cuda")
+    wide[:, 4:4 + k] = x
+    ref = _ref(x, w)
+    scale = max(1.0, float(ref.abs().max()))
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+    out = torch.full((m, n), float("nan"), device="cuda")
+    ops.gemm(wide[:, 4:4 + k], w, out, workspace=ws)
+    assert float((out.double() - ref).abs().max()) < 1e-5 * scale
+    base = torch.randn(m, n, device="cuda")
+    acc = base.clone()
+    ops.gemm(x, w, acc, accumulate=True, workspace=ws)
+    assert float((acc.double() - (ref + base.double())).abs().max()) < 1e-5 * scale
+    if n % 2 == 0:
+        for epilogue, act in (("swiglu", torch.nn.functional.silu), ("relu_glu", torch.relu)):
+            h = torch.full((m, n // 2), float("nan"), device="cuda")
+            ops.gemm(x, w, h, workspace=ws, epilogue=epilogue)
+            want = act(ref[:, 0::2]) * ref[:, 1::2]
+            assert float((h.double() - want).abs().max()) < 2e-5 * max(1.0, float(want.abs().max())), epilogue
+
+
 @pytest.mark.parametrize("m,n,k", [(4200, 4400, 72), (4100, 4609, 8), (2305, 8200, 200)])
 @pytest.mark.parametrize("epilogue", [None, "swiglu", "relu2"])
 def test_more_tiles_than_compute_units(m, n, k, epilogue):
