@@ -5,6 +5,7 @@
 // matrix cores; everything else, and the whole 32-bit path, runs the plain kernel.
 #include "common.h"
 #include "attention_generic.h"
+#include "attention_f32.h"
 #include "attention_mfma.h"
 #include "attention_latent.h"
 
@@ -274,9 +275,34 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
         ROCML_CHECK_LAUNCH("attention");
         return 0;
     }
+    AttnExtra ex{dv, v_in_k, chunk, slopes, sink, sinks, softcap, keep_first};
+    // the 32-bit path: the matrix cores' own 32-bit products, for the head sizes that fill their tiles
+    bool f32_ok = dtype == ROCML_F32 && plain_features && page_size == AF_PAGE && hkv <= 65535 && n_seqs <= 65535 &&
+                  ((uintptr_t)q | (uintptr_t)out | (uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0 &&
+                  (d == 16 || d == 32 || d == 48 || d == 64 || d == 96 || d == 112 || d == 128 || d == 192 || d == 256);
+    if (f32_ok && algo == ATTN_AUTO) {
+        AttnF32Args a{(const float*)q, (const float*)kcache, (const float*)vcache, (float*)out, block_table, token_seq, token_pos,
+                      cu_seqlens, bt_width, hq, hkv, window, scale, ex};
+        int rc;
+#define AF_SIZE(KD_) rc = launch_attn_f32<KD_>(a, n_tokens, n_seqs, max_new, cu_count(), stream)
+        switch (d / 16) {
+            case 1: AF_SIZE(1); break;
+            case 2: AF_SIZE(2); break;
+            case 3: AF_SIZE(3); break;
+            case 4: AF_SIZE(4); break;
+            case 6: AF_SIZE(6); break;
+            case 7: AF_SIZE(7); break;
+            case 8: AF_SIZE(8); break;
+            case 12: AF_SIZE(12); break;
+            default: AF_SIZE(16); break;
+        }
+#undef AF_SIZE
+        if (rc) return rc;
+        ROCML_CHECK_LAUNCH("attention");
+        return 0;
+    }
     dim3 grid(n_tokens, hq);
     size_t lds = (size_t)(d + AG_BLOCK) * sizeof(float);
-    AttnExtra ex{dv, v_in_k, chunk, slopes, sink, sinks, softcap, keep_first};
     if (dtype == ROCML_F32)
         attn_generic_kernel<float><<<grid, AG_BLOCK, lds, stream>>>(
             (const float*)q, (float*)out, (const float*)kcache, (const float*)vcache, block_table,

@@ -485,3 +485,39 @@ def test_decode_over_tens_of_thousands_of_keys(length, window, n_splits):
 @pytest.mark.parametrize("length,window", [(32768, None), (32768, 5000), (40960, None)])
 def test_a_chunk_deep_in_a_long_sequence(length, window):
     _long_case(length, 256, 4, 2, 128, window, 0, seed=32)
+
+
+# (query heads, kv heads, head size, [(context length, new tokens)]): one token a sequence and a few (the token kernel), tiles of
+# 64 rows with a rest, 20 heads a kv head, a block table of 8 pages and more (more waves a block)
+F32 = [(4, 2, 16, [(1, 1), (129, 1), (64, 1)]), (5, 5, 48, [(70, 60), (3, 3), (200, 1)]), (3, 1, 112, [(65, 2), (300, 4)]),
+       (16, 8, 128, [(600, 1), (37, 1)]), (16, 8, 128, [(300, 300), (129, 65), (64, 8)]), (20, 1, 64, [(520, 1), (9, 1)]),
+       (40, 2, 32, [(90, 21)]), (8, 2, 256, [(700, 1)]), (4, 4, 256, [(130, 70)]), (6, 3, 192, [(100, 33)])]
+F32_MASKS = [{}, {"window": 65}, {"window": 20, "keep_first": 3}, {"window": 64, "keep_first": 70, "sink": True}, {"chunk": 50, "slopes": True},
+             {"softcap": 5.0, "sinks": True}]
+
+
+@pytest.mark.parametrize("hq,hkv,d,seqs", F32)
+@pytest.mark.parametrize("mask", F32_MASKS)
+def test_float32_matrix_cores_against_the_plain_kernel(hq, hkv, d, seqs, mask):
+    """Every mask at every shape; what lies behind a sequence's end in its last page is NaN, which no result may see."""
+    dev, _, _, _ = _build(seqs, hq, hkv, d, torch.float32, 11)
+    for b, (length, _) in enumerate(seqs):
+        if length % PAGE:
+            page = int(dev["table"][b, length // PAGE])
+            dev["kc"][page, :, length % PAGE:] = float("nan")
+            dev["vc"][page, :, :, length % PAGE:] = float("nan")
+    kw = {k: v for k, v in mask.items() if k in ("window", "keep_first", "chunk", "softcap", "sink")}
+    g = torch.Generator().manual_seed(12)
+    if mask.get("slopes"):
+        kw["slopes"] = (torch.rand(hq, generator=g) * 0.1).cuda()
+    if mask.get("sinks"):
+        kw.update(sink=True, sinks=torch.randn(hq, generator=g).cuda())
+    got = []
+    for algo in (0, PLAIN):
+        out = torch.full_like(dev["q"], float("nan"))
+        ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, d ** -0.5,
+                      algo=algo, cu_seqlens=dev["cu"], max_new=max(n for _, n in seqs), q_counts=[n for _, n in seqs],
+                      max_len=max(length for length, _ in seqs), **kw)
+        got.append(out.double())
+    # both are 32-bit: sums of up to 256 products and 700 probabilities in another order
+    assert float((got[0] - got[1]).abs().max()) < 1e-5
