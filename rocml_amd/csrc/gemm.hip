@@ -640,7 +640,7 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
 #define F32_BY_EPI(fn, ...)                                                                  \
         (epi == EPI_ACC ? fn<EPI_ACC>(__VA_ARGS__) : epi == EPI_SWIGLU ? fn<EPI_SWIGLU>(__VA_ARGS__) \
          : epi == EPI_RELUGLU ? fn<EPI_RELUGLU>(__VA_ARGS__) : fn<EPI_F32>(__VA_ARGS__))
-        if (m <= 32) rc = F32_BY_EPI(launch_f32_rows, xf, ldx, wf, ldw, of, ldo, m, n, k, stream);
+        if (m <= 32) rc = F32_BY_EPI(launch_f32_rows, xf, ldx, wf, ldw, of, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else rc = F32_BY_EPI(launch_f32_tile, xf, ldx, wf, ldw, of, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
 #undef F32_BY_EPI
         if (rc) return rc;

@@ -65,7 +65,7 @@ def test_bfloat16_algorithms(m, n, k, algo):
 # rows around 16 and 32 (the few-rows kernel's tiles) and beyond; K of a run of 64, less, and runs with a rest; N that is no tile;
 # products cut along K (narrow, deep) and whole
 @pytest.mark.parametrize("m,n,k", [(1, 5, 4), (2, 384, 96), (16, 300, 1028), (17, 51, 640), (32, 4112, 260), (33, 70, 68), (64, 64, 32),
-                                   (130, 1000, 4100), (700, 130, 2052), (5, 20000, 64)])
+                                   (130, 1000, 4100), (700, 130, 2052), (5, 20000, 64), (3, 100, 2052), (20, 1024, 3076)])
 def test_float32_matrix_cores(m, n, k):
     x, w = _operands(m, n, k, torch.float32, 5)
     wide = torch.full((m, k + 8), float("nan"), device="cuda")
@@ -80,6 +80,11 @@ def test_float32_matrix_cores(m, n, k):
     acc = base.clone()
     ops.gemm(x, w, acc, accumulate=True, workspace=ws)
     assert float((acc.double() - (ref + base.double())).abs().max()) < 1e-5 * scale
+    acc = base.clone()
+    pieces = ops.gemm(x, w, acc, accumulate=True, workspace=ws, defer=True)
+    if pieces:
+        acc += ws[:pieces * m * n * 4].view(torch.float32).view(pieces, m, n).sum(0)
+    assert float((acc.double() - (ref + base.double())).abs().max()) < 1e-5 * scale, pieces
     if n % 2 == 0:
         for epilogue, act in (("swiglu", torch.nn.functional.silu), ("relu_glu", torch.relu)):
             h = torch.full((m, n // 2), float("nan"), device="cuda")
