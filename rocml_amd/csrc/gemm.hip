@@ -420,7 +420,7 @@ static int launch_kpar(const void* x, int ldx, const void* w, int ldw, void* out
                        void* workspace, long long workspace_bytes, SplitPlan plan, hipStream_t stream) {
     int n_tiles = ceil_div(n, 16);
     int splits = 4 * cu_count() / n_tiles;
-    int by_k = k / 1024;
+    int by_k = ceil_div(k, 1024);                      // (a wave then has one chunk of 256)
     if (splits > by_k) splits = by_k;
     if (splits > plan.max_splits) splits = plan.max_splits;
     if (splits < 1 || epi_gated(EPI)) splits = 1;
@@ -484,6 +484,14 @@ ROCML_EXPORT int rocml_splitk_reduce(const float* partials, void* out, int out_d
     return 0;
 }
 
+// Waves of a block of the kernel below: few enough that a wave's share of K is one chunk of 256, for one trip to memory
+// (microseconds at one row: 1024 x 2048 5.8 with four waves, 4.8 with eight; 1024 x 3072 7.6, 6.8 and 6.1 with twelve);
+// beyond 3072 the count of eight or twelve with fewer chunks (4096 x 12288: 21.5 and 21.0; 2048 x 6144: 10.3 and 10.0).
+static int prescale_waves(int k) {
+    if (k <= 3072) return k <= 1024 ? 4 : k <= 2048 ? 8 : 12;
+    return ceil_div(ceil_div(k, 12), 256) < ceil_div(ceil_div(k, 8), 256) ? 12 : 8;
+}
+
 // resid[M, N] += X * W^T for at most 16 rows of bfloat16 operands, whole sums, and the next norm
 // prepared: xg[M, N] = bfloat16(resid * gain) and ssq[M][ceil(N / 16)], the sums of squares of
 // every 16 columns of a row (see gemm_residual_prescale_kernel).
@@ -494,6 +502,7 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
     ROCML_REQUIRE(m <= 16, "gemm_residual_prescale: at most 16 rows, got %d", m);
     ROCML_REQUIRE(ldx >= k && ldw >= k && ldr >= n && ldg >= n, "gemm_residual_prescale: row strides (%d, %d, %d, %d) too small",
                   ldx, ldw, ldr, ldg);
+    ROCML_REQUIRE(ldx < (1 << 26) && ldw < (1 << 26), "gemm_residual_prescale: 16 rows of the operands exceed 31-bit offsets");
     ROCML_REQUIRE(k % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0,
                   "gemm_residual_prescale: K and the operands' row strides must be multiples of 8 and the pointers "
                   "16-byte aligned (K=%d ldx=%d ldw=%d)", k, ldx, ldw);
@@ -502,16 +511,17 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
     ROCML_REQUIRE(resid && gain && xg && ssq, "gemm_residual_prescale: null pointer");
     if (m == 0) return 0;
     int tiles = ceil_div(n, 16);
-    ROCML_REQUIRE(waves == 0 || waves == 4 || waves == 8 || waves == 16, "gemm_residual_prescale: 4, 8 or 16 waves, got %d", waves);
-    // waves: 0 = choose: eight a block when each still gets 512 of K and the chip holds all blocks
-    // of eight at once, else four
-    if (waves == 0) waves = (k >= 4096 && tiles <= cu_count()) ? 8 : 4;
-#define GRP_LAUNCH(W_)                                                                                          \
-    gemm_residual_prescale_kernel<W_><<<tiles, 64 * W_, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, resid, \
+    ROCML_REQUIRE(waves == 0 || waves == 4 || waves == 8 || waves == 12 || waves == 16,
+                  "gemm_residual_prescale: 4, 8, 12 or 16 waves, got %d", waves);
+    if (waves == 0) waves = prescale_waves(k);
+    const bool one = round_up(ceil_div(k, waves), 32) <= 256;
+#define GRP_LAUNCH(W_, ONE_)                                                                                    \
+    gemm_residual_prescale_kernel<W_, ONE_><<<tiles, 64 * W_, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, resid, \
                                                                      ldr, gain, (bf16_t*)xg, ldg, ssq, tiles, m, n, k)
-    if (waves == 16) GRP_LAUNCH(16);
-    else if (waves == 8) GRP_LAUNCH(8);
-    else GRP_LAUNCH(4);
+    if (waves == 16) { if (one) GRP_LAUNCH(16, true); else GRP_LAUNCH(16, false); }
+    else if (waves == 12) { if (one) GRP_LAUNCH(12, true); else GRP_LAUNCH(12, false); }
+    else if (waves == 8) { if (one) GRP_LAUNCH(8, true); else GRP_LAUNCH(8, false); }
+    else { if (one) GRP_LAUNCH(4, true); else GRP_LAUNCH(4, false); }
 #undef GRP_LAUNCH
     ROCML_CHECK_LAUNCH("gemm_residual_prescale");
     return 0;
@@ -521,17 +531,18 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
 // stream and norm the result.  Its blocks own 16 columns and all of K, so the chip must hold them in
 // one round, and a CU pulls a block's weight rows at a limited rate, so K must be short or the
 // blocks must be nearly one a CU.  Measured in replayed graphs against the product cut along K over
-// blocks plus the norm kernel (us): 4096 x 4096 10.3 against 13.8 at 1 row, 12.1 against 14.5 at
-// 8, 13.0 against 14.8 at 16; 1024 x 3072 7.6 against 9.2 at 1 row, 9.4 against 9.7 at 16;
-// 4096 x 12288 22.8 against 25.6 at 2 rows, 25.3 against 26.6 at 8, 27.9 against 27.3 at 12 (every
-// block reads all activations, which is what more rows cost); 2560 x 9728 (160 blocks) 18.4 against
-// 17.4 and 5120 x 5120 (320 blocks, more than a round) 19.2 against 17.9 at 1 row: not taken.
+// blocks (the norm kernel behind it takes 4.4 more; us): 4096 x 4096 8.4 against 8.1 at 1 row, 9.5 against 8.4 at
+// 8, 10.9 against 9.0 at 16; 1024 x 3072 6.1 against 5.6 at 1 row, 8.2 against 5.9 at 16; 2048 x 6144 10.0 against 7.8 at
+// 1 row, 11.1 against 7.6 at 4, 12.1 against 7.7 at 8; 4096 x 12288 21.5 against 20.6 at 1 row, 24.0 against 20.9 at 8 (every
+// block reads all activations, which is what more rows cost); 2560 x 9728 (160 blocks) 15.9 against
+// 11.6 at 1 row and 5120 x 5120 (320 blocks, more than a round): not taken.
 ROCML_EXPORT int rocml_gemm_residual_prescale_pays(int m, int n, int k) {
     if (m < 1 || m > 16 || k % 8 != 0) return 0;
     int tiles = ceil_div(n, 16);
     const int cus = cu_count();
     if (tiles > cus) return 0;
     if (k <= 4096) return 1;
+    if (k <= 8192 && m <= 4 && 2 * tiles >= cus) return 1;
     return k <= 12288 && m <= 8 && 10 * tiles >= 9 * cus;
 }
 
@@ -614,7 +625,21 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
         // blocks as well and a wave is left with one chunk; the few-rows kernel is 10 to 15 %
         // faster there.  Beyond two rows the activations
         // read from L2 cost more than the block sharing of the few-rows kernel.
-        bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && m <= 2 && !gated && 2 * (n / 16) >= 3 * cus);
+        // But where K in pieces of 1024 leaves a wave one chunk of 256 and the blocks are at most two a CU (one and a half
+        // beyond 8 rows), it is one trip to memory without staging and with half the partial sums: microseconds at 1 and 8
+        // rows against the few-rows kernel 4.3 and 4.5 for 5.6 and 5.8 at 4096 x 1024, 4.3 and 4.6 for 5.6 and 5.7 at
+        // 2048 x 2048, 6.3 and 6.6 for 6.5 and 6.5 at 4096 x 2048 (512 blocks), 7.9 and 8.5 for 7.7 at 6144 x 2048 (768).
+        const long long pieces = ceil_div(k, 1024), kpar_blocks = ceil_div(n, 16) * pieces;
+        bool one_trip = m <= 16 && !gated && (pieces == 1 || workspace) && pieces <= plan.max_splits &&
+                        2 * kpar_blocks <= (m <= 8 ? 4 : 3) * (long long)cus && pieces * m * n * 4 <= workspace_bytes + (pieces == 1 ? (1ll << 60) : 0);
+        // The gated product, which cannot be cut along K: up to 8 rows and K of 2048 (microseconds at 1 and 8 rows against the
+        // few-rows kernel: 12288 x 2048 11.5 and 12.6 for 15.0 and 14.6, 8192 x 2048 8.6 and 9.5 for 12.6 and 12.2, 6144 x 1024
+        // 6.1 and 6.6 for 6.9; at 16 rows 14.8 for 15.1, 10.8 for 12.3 and 7.3 for 7.0), and up to two rows and K of 4096 in
+        // whole chunks (24576 x 4096 36.8 for 38.0; 41.5 for 36.4 at 8 rows; 19456 x 2560, whose waves end in a half chunk, 22.0 for 22.0).
+        one_trip = one_trip || (gated && ((m <= 8 && k <= 2048) || (m <= 2 && k <= 4096 && k % 1024 == 0)));
+        bool offsets_fit = ldx < (1 << 26) && ldw < (1 << 26);       // (its 16 rows are addressed by 31-bit offsets)
+        bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && offsets_fit &&
+                                               (one_trip || (m <= 2 && !gated && 2 * (n / 16) >= 3 * cus)));
         if (kpar) rc = BY_EPI(launch_kpar, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else if (skinny) rc = BY_EPI(launch_skinny_m, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else rc = BY_EPI(launch_mfma_tile, x, ldx, w, ldw, out, ldo, m, n, k,

@@ -43,6 +43,18 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;   // 16 bytes as a
 
 __device__ __forceinline__ bf16x8_t as_frag4(u32x4_t v) { return __builtin_bit_cast(bf16x8_t, v); }
 
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ga_buffer(const void* base, long long bytes) {
+    // raw buffer (stride 0), 32-bit data format; the range check is on the byte offset
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)min(bytes, (long long)0x7fffffff), 0x00020000);
+}
+
+// An operand row's 16 bytes at `offset`, zeros (and no traffic) where `in` does not hold: no branch and no select behind a
+// load, either of which makes the wave wait for it on the spot.
+constexpr uint32_t BUF_NOWHERE = 0x80000000u;         // beyond every such buffer
+__device__ __forceinline__ u32x4_t buf_piece(__amdgpu_buffer_rsrc_t buf, bool in, uint32_t offset) {
+    return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(buf, in ? offset : BUF_NOWHERE, 0, 0));
+}
+
 // EPI_SWIGLU: weight rows come in pairs (gate_j, up_j); the output is bfloat16 [M, N/2] with
 // out[m][j] = silu(gate) * up (rocml-kernels/kernels/silu_mul.hip:12-20), formed from the 32-bit
 // accumulators so that gate and up are never rounded or written.
@@ -585,10 +597,6 @@ gemm_skinny_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restri
 // bytes of 16 * WAVES rows must fit 31 bits.
 constexpr uint32_t GA_NOWHERE = 0x80000000u;         // an offset beyond any buffer here
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t ga_buffer(const void* base, long long bytes) {
-    // raw buffer (stride 0), 32-bit data format; the range check is on the byte offset
-    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)min(bytes, (long long)0x7fffffff), 0x00020000);
-}
 
 template <int MT, int EPI, bool PARTIAL, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
@@ -744,21 +752,19 @@ gemm_kpar_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     int quarter = (((be - bs + 3) / 4) + 31) / 32 * 32;
     int ks = min(be, bs + wave * quarter), ke = min(be, ks + quarter);
     bool xok = col < m;
-    const bf16_t* wsafe = w + (size_t)min(tile * 16 + col, n - 1) * ldw;
-    const bf16_t* xsafe = x + (size_t)min(col, m - 1) * ldx;
-    const bf16_t* wp = wsafe + g * 8;
-    const bf16_t* xp = xsafe + g * 8;
+    const int rows_here = min(16, n - tile * 16);
+    const __amdgpu_buffer_rsrc_t wbuf = ga_buffer(w + (size_t)tile * 16 * ldw, ((long long)(rows_here - 1) * ldw + k) * 2);
+    const __amdgpu_buffer_rsrc_t xbuf = ga_buffer(x, ((long long)(m - 1) * ldx + k) * 2);
+    const uint32_t woff = ((uint32_t)col * (uint32_t)ldw + g * 8) * 2u, xoff = ((uint32_t)col * (uint32_t)ldx + g * 8) * 2u;
     u32x4_t wc[8], xc[8], wn[8], xn[8];
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    // No select behind a load (see the few-rows kernel): clamped addresses, and the activations
-    // of a piece beyond K are zeroed just before they are multiplied.
-#define GK_LOAD(kb_, wd_, xd_)                                                \
-    _Pragma("unroll") for (int j = 0; j < 8; ++j) {                           \
-        bool in_ = (kb_) + j * 32 + g * 8 < ke;                               \
-        wd_[j] = *(const u32x4_t*)(in_ ? wp + (kb_) + j * 32 : wsafe);        \
-        xd_[j] = *(const u32x4_t*)(in_ ? xp + (kb_) + j * 32 : xsafe);        \
+#define GK_LOAD(kb_, wd_, xd_)                                                                     \
+    _Pragma("unroll") for (int j = 0; j < 8; ++j) {                                                \
+        bool in_ = (kb_) + j * 32 + g * 8 < ke;                                                    \
+        wd_[j] = buf_piece(wbuf, in_ && col < rows_here, woff + (uint32_t)((kb_) + j * 32) * 2u);  \
+        xd_[j] = buf_piece(xbuf, in_ && xok, xoff + (uint32_t)((kb_) + j * 32) * 2u);              \
     }
-    if (ks < ke) GK_LOAD(ks, wc, xc)
+    GK_LOAD(ks, wc, xc)
     // (the rows' scales for the gated epilogue: formed by the last wave while its first loads are
     // on their way, handed to the first wave through LDS)
     constexpr bool SCALES = epi_gated(EPI) && !PARTIAL;
@@ -773,12 +779,8 @@ gemm_kpar_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     for (int kb = ks; kb < ke; kb += GK_KC) {
         bool more = kb + GK_KC < ke;
         if (more) GK_LOAD(kb + GK_KC, wn, xn)
-        const u32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            u32x4_t xv = kb + j * 32 + g * 8 < ke ? xc[j] : zero;
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag4(wc[j]), as_frag4(xv), acc, 0, 0, 0);
-        }
+        for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag4(wc[j]), as_frag4(xc[j]), acc, 0, 0, 0);
         if (more) {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
@@ -825,7 +827,9 @@ gemm_kpar_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
 // multiplies them by 1 / sqrt(sum of ssq[row] / N + eps): the norm's scale is one number per row
 // and commutes with the product.  A decode step of a few sequences is priced by the kernels that
 // follow one another, not by bytes; this takes two norms out of every layer.
-template <int WAVES>
+// ONE: a wave's share of K is at most one chunk of 256, so everything is asked for in one trip and half the registers do
+// (which sixteen waves a block need).
+template <int WAVES, bool ONE>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ w, int ldw,
                               float* resid, int ldr, const float* __restrict__ gain, bf16_t* __restrict__ xg, int ldg,
@@ -836,24 +840,19 @@ gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_
     int tile = blockIdx.x;
     int share = (((k + WAVES - 1) / WAVES) + 31) / 32 * 32;
     int ks = min(k, wave * share), ke = min(k, ks + share);
-    const bf16_t* wsafe = w + (size_t)min(tile * 16 + col, n - 1) * ldw;
-    const bf16_t* xsafe = x + (size_t)min(col, m - 1) * ldx;
-    const bf16_t* wp = wsafe + g * 8;
-    const bf16_t* xp = xsafe + g * 8;
-    u32x4_t wc[8], xc[8], wn[8], xn[8];
+    const int rows_here = min(16, n - tile * 16);
+    const __amdgpu_buffer_rsrc_t wbuf = ga_buffer(w + (size_t)tile * 16 * ldw, ((long long)(rows_here - 1) * ldw + k) * 2);
+    const __amdgpu_buffer_rsrc_t xbuf = ga_buffer(x, ((long long)(m - 1) * ldx + k) * 2);
+    const uint32_t woff = ((uint32_t)col * (uint32_t)ldw + g * 8) * 2u, xoff = ((uint32_t)col * (uint32_t)ldx + g * 8) * 2u;
+    u32x4_t wc[8], xc[8], wn[ONE ? 1 : 8], xn[ONE ? 1 : 8];
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    bool xrow = col < m;        // lanes of rows beyond M load no activations (their sums are not stored)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) xc[j] = xn[j] = u32x4_t{0u, 0u, 0u, 0u};
-    // (no select behind a load: clamped addresses; a piece beyond the wave's K range is zeroed on
-    // the activation side just before it is multiplied)
-#define GR_LOAD(kb_, wd_, xd_)                                                \
-    _Pragma("unroll") for (int j = 0; j < 8; ++j) {                           \
-        bool in_ = (kb_) + j * 32 + g * 8 < ke;                               \
-        wd_[j] = *(const u32x4_t*)(in_ ? wp + (kb_) + j * 32 : wsafe);        \
-        if (xrow) xd_[j] = *(const u32x4_t*)(in_ ? xp + (kb_) + j * 32 : xsafe); \
+#define GR_LOAD(kb_, wd_, xd_)                                                                     \
+    _Pragma("unroll") for (int j = 0; j < 8; ++j) {                                                \
+        bool in_ = (kb_) + j * 32 + g * 8 < ke;                                                    \
+        wd_[j] = buf_piece(wbuf, in_ && col < rows_here, woff + (uint32_t)((kb_) + j * 32) * 2u);  \
+        xd_[j] = buf_piece(xbuf, in_ && col < m, xoff + (uint32_t)((kb_) + j * 32) * 2u);          \
     }
-    if (ks < ke) GR_LOAD(ks, wc, xc)
+    GR_LOAD(ks, wc, xc)
     // The first wave finishes the block's outputs: what it needs of the residual stream and of the
     // gain is asked for now, so that it has arrived when the sums are ready.
     int n0 = tile * 16 + g * 4;
@@ -865,20 +864,21 @@ gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_
         gn = *(const float4*)(gain + n0);
         asm volatile("" ::: "memory");          // (the loads stay here)
     }
+    __builtin_amdgcn_sched_barrier(0);          // (and so do the operands': sunk to their products they arrive one by one)
     for (int kb = ks; kb < ke; kb += GK_KC) {
-        bool more = kb + GK_KC < ke;
-        if (more) GR_LOAD(kb + GK_KC, wn, xn)
-        const u32x4_t zero = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            u32x4_t xv = kb + j * 32 + g * 8 < ke ? xc[j] : zero;
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag4(wc[j]), as_frag4(xv), acc, 0, 0, 0);
+        bool more = !ONE && kb + GK_KC < ke;
+        if constexpr (!ONE) {
+            if (more) GR_LOAD(kb + GK_KC, wn, xn)
         }
-        if (more) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                wc[j] = wn[j];
-                xc[j] = xn[j];
+        for (int j = 0; j < 8; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_frag4(wc[j]), as_frag4(xc[j]), acc, 0, 0, 0);
+        if constexpr (!ONE) {
+            if (more) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    wc[j] = wn[j];
+                    xc[j] = xn[j];
+                }
             }
         }
     }
