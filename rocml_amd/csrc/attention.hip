@@ -170,7 +170,8 @@ static int launch_latent(const LatentArgs& a, hipStream_t stream) {
         a.q, a.out, a.cache, a.block_table, a.bt_width, a.cu_seqlens, a.n_seqs, a.token_pos, a.n_heads, a.dk, a.dv,
         a.scale * LOG2E, a.window, n_splits, part_o, part_ml);
     if (n_splits > 1)
-        attn_latent_reduce_kernel<<<(unsigned)rows, a.dv > 256 ? 256 : a.dv > 128 ? 128 : 64, 0, stream>>>(part_o, part_ml, a.out, n_splits, a.dv);
+        attn_latent_reduce_kernel<<<(unsigned)rows, (ALR_GROUPS * (a.dv / 4) + 63) / 64 * 64, (64 + ALR_GROUPS * a.dv) * sizeof(float), stream>>>(
+            part_o, part_ml, a.out, n_splits, a.dv);
     return 0;
 }
 
