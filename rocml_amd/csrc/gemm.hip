@@ -423,7 +423,7 @@ static int launch_kpar(const void* x, int ldx, const void* w, int ldw, void* out
     int by_k = ceil_div(k, 1024);                      // (a wave then has one chunk of 256)
     if (splits > by_k) splits = by_k;
     if (splits > plan.max_splits) splits = plan.max_splits;
-    if (splits < 1 || epi_gated(EPI)) splits = 1;
+    if (splits < 1 || epi_gated(EPI) || (k <= 2048 && !(plan.defer && ldo == n))) splits = 1;   // whole sums spare the reduce kernel
     long long per_split = (long long)m * n * sizeof(float);
     if (splits > 1 && (long long)splits * per_split > workspace_bytes)
         splits = workspace ? (int)(workspace_bytes / per_split) : 1;
@@ -630,13 +630,15 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
         // rows against the few-rows kernel 4.3 and 4.5 for 5.6 and 5.8 at 4096 x 1024, 4.3 and 4.6 for 5.6 and 5.7 at
         // 2048 x 2048, 6.3 and 6.6 for 6.5 and 6.5 at 4096 x 2048 (512 blocks), 7.9 and 8.5 for 7.7 at 6144 x 2048 (768).
         const long long pieces = ceil_div(k, 1024), kpar_blocks = ceil_div(n, 16) * pieces;
-        bool one_trip = m <= 16 && !gated && (pieces == 1 || workspace) && pieces <= plan.max_splits &&
+        bool one_trip = m <= 16 && !gated && (pieces == 1 || (workspace && plan.defer && ldo == n)) && pieces <= plan.max_splits &&
                         2 * kpar_blocks <= (m <= 8 ? 4 : 3) * (long long)cus && pieces * m * n * 4 <= workspace_bytes + (pieces == 1 ? (1ll << 60) : 0);
         // The gated product, which cannot be cut along K: up to 8 rows and K of 2048 (microseconds at 1 and 8 rows against the
         // few-rows kernel: 12288 x 2048 11.5 and 12.6 for 15.0 and 14.6, 8192 x 2048 8.6 and 9.5 for 12.6 and 12.2, 6144 x 1024
         // 6.1 and 6.6 for 6.9; at 16 rows 14.8 for 15.1, 10.8 for 12.3 and 7.3 for 7.0), and up to two rows and K of 4096 in
         // whole chunks (24576 x 4096 36.8 for 38.0; 41.5 for 36.4 at 8 rows; 19456 x 2560, whose waves end in a half chunk, 22.0 for 22.0).
-        one_trip = one_trip || (gated && ((m <= 8 && k <= 2048) || (m <= 2 && k <= 4096 && k % 1024 == 0)));
+        // A product whose pieces nobody adds pays a kernel for them: the same rule.
+        bool whole = gated || !(plan.defer && ldo == n);
+        one_trip = one_trip || (whole && ((m <= 8 && k <= 2048 && n <= 48 * cus) || (m <= 2 && k <= 4096 && k % 1024 == 0)));
         bool offsets_fit = ldx < (1 << 26) && ldw < (1 << 26);       // (its 16 rows are addressed by 31-bit offsets)
         bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && offsets_fit &&
                                                (one_trip || (m <= 2 && !gated && 2 * (n / 16) >= 3 * cus)));
