@@ -82,6 +82,13 @@ template <> struct Elem<bf16_t> {
     static __device__ __forceinline__ void store(bf16_t* p, float v) { *p = f32_to_bf16(v); }
 };
 
+// ---- buffers --------------------------------------------------------------------
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ga_buffer(const void* base, long long bytes) {
+    // raw buffer (stride 0), 32-bit data format; the range check is on the byte offset
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)min(bytes, (long long)0x7fffffff), 0x00020000);
+}
+constexpr uint32_t BUF_NOWHERE = 0x80000000u;         // an offset beyond every such buffer: the load gives zeros
+
 // ---- wave64 reductions --------------------------------------------------------
 constexpr int WAVE = 64;
 

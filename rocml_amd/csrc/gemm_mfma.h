@@ -43,14 +43,8 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;   // 16 bytes as a
 
 __device__ __forceinline__ bf16x8_t as_frag4(u32x4_t v) { return __builtin_bit_cast(bf16x8_t, v); }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t ga_buffer(const void* base, long long bytes) {
-    // raw buffer (stride 0), 32-bit data format; the range check is on the byte offset
-    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, (int)min(bytes, (long long)0x7fffffff), 0x00020000);
-}
-
 // An operand row's 16 bytes at `offset`, zeros (and no traffic) where `in` does not hold: no branch and no select behind a
 // load, either of which makes the wave wait for it on the spot.
-constexpr uint32_t BUF_NOWHERE = 0x80000000u;         // beyond every such buffer
 __device__ __forceinline__ u32x4_t buf_piece(__amdgpu_buffer_rsrc_t buf, bool in, uint32_t offset) {
     return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(buf, in ? offset : BUF_NOWHERE, 0, 0));
 }
