@@ -62,6 +62,32 @@ def test_bfloat16_algorithms(m, n, k, algo):
     assert float((acc.double() - (ref + base.double())).abs().max()) < 2e-5 * scale, "accumulating"
 
 
+# one chunk of 256 a wave, one and a rest, K in pieces of 1024 with a rest; N that is no tile; rows to either side of the rule's limits
+@pytest.mark.parametrize("m,n,k", [(1, 40, 8), (3, 1000, 1024), (8, 2047, 1032), (9, 2048, 2048), (16, 520, 3080), (8, 4096, 2048), (2, 70, 264)])
+def test_few_rows_in_one_trip(m, n, k):
+    """The operands are column ranges of wider matrices that hold NaN beside them; whole sums, deferred pieces and the gated
+    activation, by the library's own choice of kernel."""
+    x, w = _operands(m, n, k, torch.bfloat16, 9)
+    wide_x, wide_w = torch.full((m, k + 16), float("nan"), dtype=torch.bfloat16, device="cuda"), torch.full(
+        (n, k + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide_x[:, 8:8 + k], wide_w[:, :k] = x, w
+    x, w = wide_x[:, 8:8 + k], wide_w[:, :k]
+    ref = _ref(x, w)
+    scale = max(1.0, float(ref.abs().max()))
+    ws = torch.empty(16 << 20, dtype=torch.uint8, device="cuda")
+    for defer in (False, True):
+        acc = torch.ones(m, n, device="cuda")
+        pieces = ops.gemm(x, w, acc, accumulate=True, workspace=ws, defer=defer)
+        if pieces:
+            acc += ws[:pieces * m * n * 4].view(torch.float32).view(pieces, m, n).sum(0)
+        assert float((acc.double() - 1 - ref).abs().max()) < 2e-5 * scale, (defer, pieces)
+    if n % 2 == 0:
+        h = torch.empty(m, n // 2, dtype=torch.bfloat16, device="cuda")
+        ops.gemm(x, w, h, workspace=ws, epilogue="swiglu")
+        want = torch.nn.functional.silu(ref[:, 0::2]) * ref[:, 1::2]
+        assert float((h.double() - want).abs().max()) < 5e-3 * max(1.0, float(want.abs().max()))
+
+
 # rows around 16 and 32 (the few-rows kernel's tiles) and beyond; K of a run of 64, less, and runs with a rest; N that is no tile;
 # products cut along K (narrow, deep) and whole
 @pytest.mark.parametrize("m,n,k", [(1, 5, 4), (2, 384, 96), (16, 300, 1028), (17, 51, 640), (32, 4112, 260), (33, 70, 68), (64, 64, 32),
@@ -198,7 +224,7 @@ def test_many_rows_with_k_cut_in_pieces(m, n, k):
     assert float((out16.double() - ref).abs().max()) < 5e-3 * scale
 
 
-@pytest.mark.parametrize("waves", [0, 4, 8])
+@pytest.mark.parametrize("waves", [0, 4, 8, 12, 16])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (3, 100, 72), (8, 4096, 1032), (16, 130, 4096), (7, 515, 264), (2, 88, 12288)])
 def test_residual_sum_that_prepares_the_next_norm(m, n, k, waves):
     """resid += x W^T with whole sums, xg = bfloat16(resid * gain), and per 16 columns the sum of
