@@ -99,11 +99,47 @@ __device__ __forceinline__ void af_values(const af_f32x4_t (&p)[NT], Row vrow, a
         }
 }
 
+__device__ __forceinline__ bool af_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
+
+// Adds what the page's infinite and NaN values give the rows that see their keys; every other value has had its product.
+// values: the page's [D][64] in memory.
 template <int KD>
-__global__ void __launch_bounds__(256)
+__device__ __forceinline__ void af_add_odd_values(const af_f32x4_t (&p)[4], const float* values, af_f32x4_t (&o)[KD], const AttnF32Args& a,
+                                                  int first_key, int lane, int pos, int lo) {
+#pragma unroll 1
+    for (int k = 0; k < AF_PAGE; ++k) {
+        float mine = 0.f;                             // the probability that lane l%16 + 16 (k%16 / 4) holds of key k
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mine = t * 16 + e == (k & ~12) ? p[t][e] : mine;
+        const float w = __shfl(mine, (lane & 15) + (k & 12) * 4, 64);
+        const int key = first_key + k;
+        const bool seen = key <= pos && (key >= lo || key < a.ex.keep_first);
+        int at = (lane >> 4) * 4 * AF_PAGE + k;
+        asm volatile("" : "+v"(at));                  // (addresses formed before the loop, or all loads at once, would take
+#pragma unroll                                        //  registers that the kernel is short of)
+        for (int c = 0; c < KD; ++c) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = values[at + (c * 16 + e) * AF_PAGE];
+                if (seen && !af_finite(v)) o[c][e] = fmaf(w, v, o[c][e]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// (registers for as many blocks as find room in a CU's LDS)
+constexpr int af_prompt_lds(int d) { return (AF_PAGE * (d + 4) + d * (AF_PAGE + 4)) * 4; }
+constexpr int af_prompt_blocks(int d) { return 160 * 1024 / af_prompt_lds(d) < 4 ? 160 * 1024 / af_prompt_lds(d) : 4; }
+
+template <int KD>
+__global__ void __launch_bounds__(256, af_prompt_blocks(KD * 16))
 attn_f32_prompt_kernel(AttnF32Args a) {
     constexpr int D = KD * 16, KS = D + 4, VS = AF_PAGE + 4;      // padded rows: 16 rows fall into different banks
     extern __shared__ float af_smem[];
+    __shared__ int odd_page;                          // the last page that holds an infinite or NaN value
     float *ks = af_smem, *vs = af_smem + AF_PAGE * KS;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int seq = blockIdx.y, kvh = blockIdx.z, group = a.hq / a.hkv;
@@ -125,23 +161,34 @@ attn_f32_prompt_kernel(AttnF32Args a) {
         o[c] = af_f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
     float m = -INFINITY, l = 0.f;
+    if (threadIdx.x == 0) odd_page = -1;
     for (int p = 0; p <= last_pos / AF_PAGE; ++p) {
         if (p >= kept_pages && p < lo_page) continue;
         const size_t at = ((size_t)pages[p] * a.hkv + kvh) * AF_PAGE * D;
-        const int known = last_pos - p * AF_PAGE;     // values behind it are another sequence's, if any
+        // Values behind `known` are another sequence's, if any.  The page's values meet the probabilities of 16 rows at once,
+        // and zero times infinity is NaN: a row must not see the infinite or NaN value of a key it does not see (a later
+        // token's, or one before its window).  Such values are left out of the products and added to the rows that see them.
+        const int known = last_pos - p * AF_PAGE;
         __syncthreads();
         for (int i = threadIdx.x; i < AF_PAGE * D / 4; i += 256) {
             *(af_f32x4_t*)(ks + i / (D / 4) * KS + i % (D / 4) * 4) = *(const af_f32x4_t*)(a.kcache + at + i * 4);
             af_f32x4_t v = *(const af_f32x4_t*)(a.vcache + at + i * 4);
             int key = i % (AF_PAGE / 4) * 4;
+            bool odd = false;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = key + e <= known ? v[e] : 0.f;
+            for (int e = 0; e < 4; ++e) {
+                bool here = key + e <= known, finite = af_finite(v[e]);
+                odd = odd || (here && !finite);
+                v[e] = here && finite ? v[e] : 0.f;
+            }
+            if (odd) odd_page = p;
             *(af_f32x4_t*)(vs + i / (AF_PAGE / 4) * VS + key) = v;
         }
         __syncthreads();
         af_scores<KD, 4>(q, [&](int kt, int c) { return *(const af_f32x4_t*)(ks + (kt * 16 + (lane & 15)) * KS + c * 16 + (lane >> 4) * 4); }, s);
         af_softmax<KD, 4>(s, o, m, l, a, p * AF_PAGE, lane, pos, lo, slope);
         af_values<KD, 4>(s, [&](int c, int kt) { return *(const af_f32x4_t*)(vs + (c * 16 + (lane & 15)) * VS + kt * 16 + (lane >> 4) * 4); }, o);
+        if (odd_page == p) af_add_odd_values<KD>(s, a.vcache + at, o, a, p * AF_PAGE, lane, pos, lo);
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
@@ -253,7 +300,7 @@ template <int KD>
 static int launch_attn_f32(const AttnF32Args& a, int n_tokens, int n_seqs, int max_new, int cus, hipStream_t stream) {
     constexpr int D = KD * 16;
     const int group = a.hq / a.hkv;
-    constexpr int PROMPT_LDS = (AF_PAGE * (D + 4) + D * (AF_PAGE + 4)) * 4;
+    constexpr int PROMPT_LDS = af_prompt_lds(D);
     constexpr int MANY = D <= 128 ? 16 : 8;           // (registers: a tile's keys and values, the queries and the sums)
     constexpr int FEW_LDS = 4 * 16 * (D + 6) * 4, MANY_LDS = MANY * 16 * (D + 6) * 4;
     static bool ready = false;

@@ -521,3 +521,32 @@ def test_float32_matrix_cores_against_the_plain_kernel(hq, hkv, d, seqs, mask):
         got.append(out.double())
     # both are 32-bit: sums of up to 256 products and 700 probabilities in another order
     assert float((got[0] - got[1]).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("hq,hkv,d,seqs", [(4, 2, 16, [(130, 130), (64, 40)]), (16, 8, 128, [(300, 300), (129, 65)]), (3, 1, 112, [(200, 70)]),
+                                           (8, 2, 256, [(150, 90)]), (20, 1, 64, [(70, 70)])])
+@pytest.mark.parametrize("mask", F32_MASKS)
+def test_float32_prompt_rows_do_not_see_what_unseen_keys_hold(hq, hkv, d, seqs, mask):
+    """Infinite and NaN values at some positions of every sequence reach the rows that see those positions, and no others: the
+    plain kernel visits seen keys only."""
+    dev, _, _, _ = _build(seqs, hq, hkv, d, torch.float32, 21)
+    for b, (length, n_new) in enumerate(seqs):
+        for at, value, column in ((0, float("inf"), 1), (length - n_new // 2, float("nan"), 3), (length - n_new // 2 + 1, float("inf"), d - 1),
+                                  (length - n_new // 3, -float("inf"), 5), (length - 2, float("nan"), 0)):
+            dev["vc"][int(dev["table"][b, at // PAGE]), :, column, at % PAGE] = value
+    kw = {k: v for k, v in mask.items() if k in ("window", "keep_first", "chunk", "softcap", "sink")}
+    g = torch.Generator().manual_seed(22)
+    if mask.get("slopes"):
+        kw["slopes"] = (torch.rand(hq, generator=g) * 0.1).cuda()
+    if mask.get("sinks"):
+        kw.update(sink=True, sinks=torch.randn(hq, generator=g).cuda())
+    got = []
+    for algo in (0, PLAIN):
+        out = torch.full_like(dev["q"], float("nan"))
+        ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, d ** -0.5,
+                      algo=algo, cu_seqlens=dev["cu"], max_new=max(n for _, n in seqs), q_counts=[n for _, n in seqs],
+                      max_len=max(length for length, _ in seqs), **kw)
+        got.append(out.double())
+    assert not got[1].isfinite().all() and got[1].isfinite().any()
+    # (the finite ones: as in the test above)
+    torch.testing.assert_close(got[0], got[1], rtol=0.0, atol=1e-5, equal_nan=True)
