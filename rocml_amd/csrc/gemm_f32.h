@@ -83,8 +83,7 @@ gemm_f32_rows_kernel(const float* __restrict__ x, int ldx, const float* __restri
             first += red[v][row / 16][row % 16][epi_gated(EPI) ? 2 * c : c];
             if (epi_gated(EPI)) second += red[v][row / 16][row % 16][2 * c + 1];
         }
-        if (EPI == EPI_SWIGLU) first = silu_mul(first, second);
-        if (EPI == EPI_RELUGLU) first = fmaxf(first, 0.f) * second;
+        if (epi_gated(EPI)) first = gated_mul<EPI>(first, second);
         *to = EPI == EPI_ACC ? *to + first : first;
     }
 }

@@ -63,10 +63,7 @@ __device__ __forceinline__ float silu_mul(float g, float u) { return g / (1.0f +
 template <int EPI>
 __device__ __forceinline__ float gated_mul(float g, float u) {
     if (EPI == EPI_RELUGLU) return fmaxf(g, 0.f) * u;
-    // silu(g) * u with the hardware's exponential and reciprocal (one unit in the last place each): the result is rounded
-    // to 8 bits, and the exact division and exponential were 5 % of the 256x256 product (1,101 against 1,047 us at
-    // 8192 x 24576 x 4096)
-    return g * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(g * -1.44269504088896341f)) * u;
+    return silu_mul(g, u);
 }
 
 // The scale of a norm whose product-side half was done by the producer of the residual stream
@@ -260,7 +257,7 @@ __device__ __forceinline__ void tile_epilogue(f32x4_t (&acc)[T::MT][T::NT], void
             for (int c = 0; c < PER; ++c) {
                 if (epi_gated(EPI)) {
                     float gate = acc[i][d * DEAL + c / 2][2 * c % 4], up = acc[i][d * DEAL + c / 2][2 * c % 4 + 1];
-                    v[c] = sizeof(E) == 4 && EPI == EPI_SWIGLU ? silu_mul(gate, up) : gated_mul<EPI>(gate, up);
+                    v[c] = gated_mul<EPI>(gate, up);
                 }
                 else v[c] = acc[i][d * DEAL + c / 4][c % 4];
                 if (EPI == EPI_RELU2) { v[c] = fmaxf(v[c], 0.f); v[c] *= v[c]; }

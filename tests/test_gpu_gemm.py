@@ -181,6 +181,32 @@ def test_gated_epilogue(m, n, k, algo):
         assert float((out32.double().cpu() - ref.cpu()).abs().max()) < 2e-5 * max(1.0, float(ref.abs().max()))
 
 
+@pytest.mark.parametrize("m,algo", [(1, KPAR), (8, SKINNY), (40, SKINNY), (130, TILE), (130, TILE64X256), (130, TILE192), (300, TILE256)])
+def test_gated_results_are_the_exact_ones_rounded_once(m, algo):
+    """silu(gate) * up over the whole range in which exp(-gate) is finite, formed in 32-bit: the stored bfloat16 is the rounding of
+    a number within four units in the last place (exponential, sum, division and product) of the exact one."""
+    half = 1 << 16
+    g = torch.Generator().manual_seed(31)
+    gate = torch.rand(half, generator=g) * 118 - 88              # [-88, 30)
+    parts, rest = [], gate
+    for _ in range(3):                                           # a 32-bit number is the sum of three of 8 bits
+        parts.append(rest.bfloat16())
+        rest = rest - parts[-1].float()
+    assert not rest.any()
+    w = torch.zeros(half, 2, 8, dtype=torch.bfloat16)
+    w[:, 0, :3] = torch.stack(parts, -1)
+    w[:, 1, 3] = 2.0 ** 60                                       # (what a gate of -88 leaves of it is an ordinary number)
+    x = torch.zeros(m, 8, dtype=torch.bfloat16)
+    x[:, :4] = 1.0
+    out = torch.empty(m, half, dtype=torch.bfloat16, device="cuda")
+    ops.gemm(x.cuda(), w.view(2 * half, 8).cuda(), out, algo=algo, epilogue="swiglu")
+    exact = gate.double() / (1 + torch.exp(-gate.double())) * 2.0 ** 60
+    exact = exact.cuda()
+    step = torch.exp2(torch.floor(torch.log2(exact.abs().clamp_min(1e-300))) - 8)      # half a bfloat16 step
+    off = (out.double() - exact).abs() - step - 4 * 2.0 ** -23 * exact.abs()
+    assert float((off / exact.abs().clamp_min(1e-300)).max()) <= 0
+
+
 def test_deferred_split_sums():
     """A product split along K may leave its partial sums to the caller; adding them in split
     order gives the product."""
