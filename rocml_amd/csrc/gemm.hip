@@ -431,12 +431,16 @@ static int launch_kpar(const void* x, int ldx, const void* w, int ldw, void* out
     int k_per_split = round_up(ceil_div(k, splits), 128);
     splits = ceil_div(k, k_per_split);
     dim3 grid(n_tiles, splits);
+    const bool far = ldx >= NEAR_STRIDE || ldw >= NEAR_STRIDE;
+#define KPAR(PARTIAL_, FAR_, ...) \
+    gemm_kpar_kernel<EPI, PARTIAL_, FAR_><<<grid, GK_THREADS, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, __VA_ARGS__)
     if (splits == 1) {
-        gemm_kpar_kernel<EPI, false><<<grid, GK_THREADS, 0, stream>>>(
-            (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, out, ldo, m, n, k, k_per_split, plan.rs);
+        if (far) KPAR(false, true, out, ldo, m, n, k, k_per_split, plan.rs);
+        else KPAR(false, false, out, ldo, m, n, k, k_per_split, plan.rs);
     } else {
-        gemm_kpar_kernel<EPI, true><<<grid, GK_THREADS, 0, stream>>>(
-            (const bf16_t*)x, ldx, (const bf16_t*)w, ldw, workspace, n, m, n, k, k_per_split, RowScale{});
+        if (far) KPAR(true, true, workspace, n, m, n, k, k_per_split, RowScale{});
+        else KPAR(true, false, workspace, n, m, n, k, k_per_split, RowScale{});
+#undef KPAR
         if (plan.defer && ldo == n) {
             *plan.deferred = splits;
             return 0;
@@ -639,9 +643,7 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
         // A product whose pieces nobody adds pays a kernel for them: the same rule.
         bool whole = gated || !(plan.defer && ldo == n);
         one_trip = one_trip || (whole && ((m <= 8 && k <= 2048 && n <= 48 * cus) || (m <= 2 && k <= 4096 && k % 1024 == 0)));
-        bool offsets_fit = ldx < (1 << 26) && ldw < (1 << 26);       // (its 16 rows are addressed by 31-bit offsets)
-        bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && offsets_fit &&
-                                               (one_trip || (m <= 2 && !gated && 2 * (n / 16) >= 3 * cus)));
+        bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && (one_trip || (m <= 2 && !gated && 2 * (n / 16) >= 3 * cus)));
         if (kpar) rc = BY_EPI(launch_kpar, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else if (skinny) rc = BY_EPI(launch_skinny_m, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else rc = BY_EPI(launch_mfma_tile, x, ldx, w, ldw, out, ldo, m, n, k,

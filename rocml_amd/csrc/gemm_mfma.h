@@ -43,11 +43,34 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;   // 16 bytes as a
 
 __device__ __forceinline__ bf16x8_t as_frag4(u32x4_t v) { return __builtin_bit_cast(bf16x8_t, v); }
 
-// An operand row's 16 bytes at `offset`, zeros (and no traffic) where `in` does not hold: no branch and no select behind a
-// load, either of which makes the wave wait for it on the spot.
-__device__ __forceinline__ u32x4_t buf_piece(__amdgpu_buffer_rsrc_t buf, bool in, uint32_t offset) {
-    return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(buf, in ? offset : BUF_NOWHERE, 0, 0));
-}
+// Rows of an operand of which lane l reads row l%16, 16 bytes at a time, zeros (and no traffic) where `in` does not hold.  By
+// default the rows are a buffer: no branch and no select behind a load, either of which makes the wave wait for it on the
+// spot; the sixteenth row must then lie within 31 bits of bytes.  FAR: rows further apart, by 64-bit addresses.
+constexpr int NEAR_STRIDE = 1 << 26;                  // strides below it keep 16 rows within reach
+template <bool FAR>
+struct OperandRows {
+    __amdgpu_buffer_rsrc_t buf;
+    const bf16_t* row;
+    uint32_t offset;
+    __device__ __forceinline__ OperandRows(const bf16_t* base, int ld, int rows, int k, int lane) {
+        const int r = lane & 15, piece = (lane >> 4) * 8;
+        if constexpr (FAR) {
+            row = base + (size_t)min(r, rows - 1) * ld + piece;
+        } else {
+            buf = ga_buffer(base, ((long long)(rows - 1) * ld + k) * 2);
+            offset = ((uint32_t)r * (uint32_t)ld + piece) * 2u;
+        }
+    }
+    __device__ __forceinline__ u32x4_t load(bool in, int at) const {
+        if constexpr (FAR) {
+            u32x4_t v = {0u, 0u, 0u, 0u};
+            if (in) v = *(const u32x4_t*)(row + at);
+            return v;
+        } else {
+            return __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(buf, in ? offset + (uint32_t)at * 2u : BUF_NOWHERE, 0, 0));
+        }
+    }
+};
 
 // EPI_SWIGLU: weight rows come in pairs (gate_j, up_j); the output is bfloat16 [M, N/2] with
 // out[m][j] = silu(gate) * up (rocml-kernels/kernels/silu_mul.hip:12-20), formed from the 32-bit
@@ -731,7 +754,7 @@ gemm_skinny_ahead_kernel(const bf16_t* x, int ldx, const bf16_t* w, int ldw, voi
 // are added in wave order through LDS, then comes the epilogue (or the split-K partial store).
 constexpr int GK_KC = 256, GK_THREADS = 256;
 
-template <int EPI, bool PARTIAL>
+template <int EPI, bool PARTIAL, bool FAR>
 __global__ void __launch_bounds__(GK_THREADS)
 gemm_kpar_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ w, int ldw,
                  void* __restrict__ out, int ldo, int m, int n, int k, int k_per_split, RowScale rs) {
@@ -744,16 +767,14 @@ gemm_kpar_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
     int ks = min(be, bs + wave * quarter), ke = min(be, ks + quarter);
     bool xok = col < m;
     const int rows_here = min(16, n - tile * 16);
-    const __amdgpu_buffer_rsrc_t wbuf = ga_buffer(w + (size_t)tile * 16 * ldw, ((long long)(rows_here - 1) * ldw + k) * 2);
-    const __amdgpu_buffer_rsrc_t xbuf = ga_buffer(x, ((long long)(m - 1) * ldx + k) * 2);
-    const uint32_t woff = ((uint32_t)col * (uint32_t)ldw + g * 8) * 2u, xoff = ((uint32_t)col * (uint32_t)ldx + g * 8) * 2u;
+    const OperandRows<FAR> wrows(w + (size_t)tile * 16 * ldw, ldw, rows_here, k, lane), xrows(x, ldx, m, k, lane);
     u32x4_t wc[8], xc[8], wn[8], xn[8];
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #define GK_LOAD(kb_, wd_, xd_)                                                                     \
     _Pragma("unroll") for (int j = 0; j < 8; ++j) {                                                \
         bool in_ = (kb_) + j * 32 + g * 8 < ke;                                                    \
-        wd_[j] = buf_piece(wbuf, in_ && col < rows_here, woff + (uint32_t)((kb_) + j * 32) * 2u);  \
-        xd_[j] = buf_piece(xbuf, in_ && xok, xoff + (uint32_t)((kb_) + j * 32) * 2u);              \
+        wd_[j] = wrows.load(in_ && col < rows_here, (kb_) + j * 32);                               \
+        xd_[j] = xrows.load(in_ && xok, (kb_) + j * 32);                                           \
     }
     GK_LOAD(ks, wc, xc)
     // (the rows' scales for the gated epilogue: formed by the last wave while its first loads are
@@ -832,16 +853,14 @@ gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_
     int share = (((k + WAVES - 1) / WAVES) + 31) / 32 * 32;
     int ks = min(k, wave * share), ke = min(k, ks + share);
     const int rows_here = min(16, n - tile * 16);
-    const __amdgpu_buffer_rsrc_t wbuf = ga_buffer(w + (size_t)tile * 16 * ldw, ((long long)(rows_here - 1) * ldw + k) * 2);
-    const __amdgpu_buffer_rsrc_t xbuf = ga_buffer(x, ((long long)(m - 1) * ldx + k) * 2);
-    const uint32_t woff = ((uint32_t)col * (uint32_t)ldw + g * 8) * 2u, xoff = ((uint32_t)col * (uint32_t)ldx + g * 8) * 2u;
+    const OperandRows<false> wrows(w + (size_t)tile * 16 * ldw, ldw, rows_here, k, lane), xrows(x, ldx, m, k, lane);
     u32x4_t wc[8], xc[8], wn[ONE ? 1 : 8], xn[ONE ? 1 : 8];
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #define GR_LOAD(kb_, wd_, xd_)                                                                     \
     _Pragma("unroll") for (int j = 0; j < 8; ++j) {                                                \
         bool in_ = (kb_) + j * 32 + g * 8 < ke;                                                    \
-        wd_[j] = buf_piece(wbuf, in_ && col < rows_here, woff + (uint32_t)((kb_) + j * 32) * 2u);  \
-        xd_[j] = buf_piece(xbuf, in_ && col < m, xoff + (uint32_t)((kb_) + j * 32) * 2u);          \
+        wd_[j] = wrows.load(in_ && col < rows_here, (kb_) + j * 32);                               \
+        xd_[j] = xrows.load(in_ && col < m, (kb_) + j * 32);                                       \
     }
     GR_LOAD(ks, wc, xc)
     // The first wave finishes the block's outputs: what it needs of the residual stream and of the

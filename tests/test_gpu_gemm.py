@@ -159,6 +159,43 @@ def test_strided_rows_and_refusals():
         ops.gemm(x.cpu(), w, out)
 
 
+@pytest.fixture(scope="module")
+def sixteen_far_rows():
+    """Room for 16 rows that lie 2^27 numbers apart, more than 31 bits of bytes in all."""
+    return torch.empty(15 * (1 << 27) + 4096, dtype=torch.bfloat16, device="cuda")
+
+
+def _far(t, room):
+    wide = room[:(t.shape[0] - 1) * (1 << 27) + t.shape[1]].as_strided(t.shape, (1 << 27, 1))
+    wide.copy_(t)
+    return wide
+
+
+@pytest.mark.parametrize("m,n,k,which", [(16, 40, 264, "x"), (3, 16, 1032, "w"), (9, 70, 64, "x"), (1, 13, 3080, "w")])
+def test_few_rows_far_apart(m, n, k, which, sixteen_far_rows):
+    """The K-parallel kernel with operand rows beyond each other's 31-bit reach: whole sums, K pieces, the gated activation."""
+    x, w = _operands(m, n, k, torch.bfloat16, 14)
+    ref = _ref(x, w)
+    tol = 2e-5 * max(1.0, float(ref.abs().max()))
+    if which == "x":
+        x = _far(x, sixteen_far_rows)
+    else:
+        w = _far(w, sixteen_far_rows)
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+    for algo in ([0, KPAR] if which == "x" else [KPAR]):
+        out = torch.full((m, n), float("nan"), device="cuda")
+        ops.gemm(x, w, out, algo=algo, workspace=ws)
+        assert float((out.double() - ref).abs().max()) < tol
+        pieces = ops.gemm(x, w, out, algo=algo, workspace=ws, defer=True)
+        got = ws[:pieces * m * n * 4].view(torch.float32).view(pieces, m, n).sum(0) if pieces else out
+        assert float((got.double() - ref).abs().max()) < tol, pieces
+    if n % 2 == 0:
+        h = torch.empty(m, n // 2, dtype=torch.bfloat16, device="cuda")
+        ops.gemm(x, w, h, algo=KPAR, workspace=ws, epilogue="swiglu")
+        want = torch.nn.functional.silu(ref[:, 0::2]) * ref[:, 1::2]
+        assert float((h.double() - want).abs().max()) < 5e-3 * max(1.0, float(want.abs().max()))
+
+
 @pytest.mark.parametrize("algo", [PLAIN, TILE, SKINNY, KPAR, TILE256, TILE192, TILE128X192, TILE256X96, TILE64X256])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (7, 448, 96), (25, 300, 520), (41, 130, 1032), (64, 1000, 264), (130, 256, 128), (300, 2048, 512)])
 def test_gated_epilogue(m, n, k, algo):
