@@ -506,7 +506,6 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
     ROCML_REQUIRE(m <= 16, "gemm_residual_prescale: at most 16 rows, got %d", m);
     ROCML_REQUIRE(ldx >= k && ldw >= k && ldr >= n && ldg >= n, "gemm_residual_prescale: row strides (%d, %d, %d, %d) too small",
                   ldx, ldw, ldr, ldg);
-    ROCML_REQUIRE(ldx < (1 << 26) && ldw < (1 << 26), "gemm_residual_prescale: 16 rows of the operands exceed 31-bit offsets");
     ROCML_REQUIRE(k % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0,
                   "gemm_residual_prescale: K and the operands' row strides must be multiples of 8 and the pointers "
                   "16-byte aligned (K=%d ldx=%d ldw=%d)", k, ldx, ldw);
@@ -519,10 +518,11 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
                   "gemm_residual_prescale: 4, 8, 12 or 16 waves, got %d", waves);
     if (waves == 0) waves = prescale_waves(k);
     const bool one = round_up(ceil_div(k, waves), 32) <= 256;
-#define GRP_LAUNCH(W_, ONE_)                                                                                    \
-    gemm_residual_prescale_kernel<W_, ONE_><<<tiles, 64 * W_, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, resid, \
+#define GRP_LAUNCH(W_, ...)                                                                                     \
+    gemm_residual_prescale_kernel<W_, __VA_ARGS__><<<tiles, 64 * W_, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, resid, \
                                                                      ldr, gain, (bf16_t*)xg, ldg, ssq, tiles, m, n, k)
-    if (waves == 16) { if (one) GRP_LAUNCH(16, true); else GRP_LAUNCH(16, false); }
+    if (ldx >= NEAR_STRIDE || ldw >= NEAR_STRIDE) GRP_LAUNCH(4, false, true);
+    else if (waves == 16) { if (one) GRP_LAUNCH(16, true); else GRP_LAUNCH(16, false); }
     else if (waves == 12) { if (one) GRP_LAUNCH(12, true); else GRP_LAUNCH(12, false); }
     else if (waves == 8) { if (one) GRP_LAUNCH(8, true); else GRP_LAUNCH(8, false); }
     else { if (one) GRP_LAUNCH(4, true); else GRP_LAUNCH(4, false); }

@@ -841,7 +841,7 @@ gemm_kpar_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
 // follow one another, not by bytes; this takes two norms out of every layer.
 // ONE: a wave's share of K is at most one chunk of 256, so everything is asked for in one trip and half the registers do
 // (which sixteen waves a block need).
-template <int WAVES, bool ONE>
+template <int WAVES, bool ONE, bool FAR = false>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ w, int ldw,
                               float* resid, int ldr, const float* __restrict__ gain, bf16_t* __restrict__ xg, int ldg,
@@ -853,7 +853,7 @@ gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_
     int share = (((k + WAVES - 1) / WAVES) + 31) / 32 * 32;
     int ks = min(k, wave * share), ke = min(k, ks + share);
     const int rows_here = min(16, n - tile * 16);
-    const OperandRows<false> wrows(w + (size_t)tile * 16 * ldw, ldw, rows_here, k, lane), xrows(x, ldx, m, k, lane);
+    const OperandRows<FAR> wrows(w + (size_t)tile * 16 * ldw, ldw, rows_here, k, lane), xrows(x, ldx, m, k, lane);
     u32x4_t wc[8], xc[8], wn[ONE ? 1 : 8], xn[ONE ? 1 : 8];
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #define GR_LOAD(kb_, wd_, xd_)                                                                     \

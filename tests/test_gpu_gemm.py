@@ -320,6 +320,27 @@ def test_residual_sum_that_prepares_the_next_norm(m, n, k, waves):
                                    torch.zeros(17, n, dtype=torch.bfloat16, device="cuda"), torch.zeros(17, tiles, device="cuda"))
 
 
+@pytest.mark.parametrize("m,n,k,which", [(16, 40, 264, "x"), (3, 16, 1032, "w"), (11, 130, 4096, "x")])
+def test_residual_sum_of_rows_far_apart(m, n, k, which, sixteen_far_rows):
+    """The same with operand rows beyond each other's 31-bit reach."""
+    x, w = _operands(m, n, k, torch.bfloat16, 15)
+    want = 1.0 + _ref(x, w)
+    if which == "x":
+        x = _far(x, sixteen_far_rows)
+    else:
+        w = _far(w, sixteen_far_rows)
+    tiles = (n + 15) // 16
+    resid, gain = torch.ones(m, n, device="cuda"), torch.linspace(0.5, 1.5, n, device="cuda")
+    xg, ssq = torch.empty(m, n, dtype=torch.bfloat16, device="cuda"), torch.empty(m, tiles, device="cuda")
+    for waves in (0, 8):
+        resid.fill_(1.0)
+        ops.gemm_residual_prescale(x, w, resid, gain, xg, ssq, waves=waves)
+        assert float((resid.double() - want).abs().max()) < 2e-5 * max(1.0, float(want.abs().max()))
+        assert float((xg.double() - want * gain.double()).abs().max()) < 5e-3 * float((want * gain.double()).abs().max())
+        squares = torch.nn.functional.pad(want ** 2, (0, tiles * 16 - n)).view(m, tiles, 16).sum(-1)
+        assert float((ssq.double() - squares).abs().max()) < 1e-4 * float(squares.max())
+
+
 @pytest.mark.parametrize("algo", [0, SKINNY, KPAR])
 @pytest.mark.parametrize("m,n,k,parts", [(1, 64, 64, 4), (2, 24576, 4096, 256), (8, 448, 96, 6), (16, 1000, 264, 17), (13, 300, 1032, 64)])
 def test_gated_epilogue_applies_a_row_scale(m, n, k, parts, algo):
