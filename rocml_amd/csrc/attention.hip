@@ -362,8 +362,6 @@ ROCML_EXPORT int rocml_attention_decode_fused(const float* qkv, int ld, int qkv_
                       (qkv_splits == 1 || (qkv_split_stride >= (long long)n_tokens * ld && qkv_split_stride % 4 == 0)),
                   "fused decode attention: projection rows of %d values (need %d, a multiple of 4, 16-byte aligned), "
                   "split stride %lld", ld, rows * d, qkv_split_stride);
-    ROCML_REQUIRE(qkv_splits == 1 || ((qkv_splits - 1) * qkv_split_stride + ld) * 4 < 0x7fffffffll,
-                  "fused decode attention: partial sums beyond 31-bit offsets");
     ROCML_REQUIRE((q_gain == nullptr) == (k_gain == nullptr) && (cos_t == nullptr) == (sin_t == nullptr),
                   "fused decode attention: gains and rotation tables come in pairs");
     if (n_tokens == 0) return 0;

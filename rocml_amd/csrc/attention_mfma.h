@@ -206,7 +206,11 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
         // rotation), and without a branch: the pieces beyond the projection's are zeros from beyond the buffer.  Under a
         // condition each was a trip to memory of its own, behind the keys and values
         // (a block a kv head at 64 keys 8.2 -> 7.8 us, one sequence of 560 8.8 -> 8.0, eight of 2,100 19.9 -> 19.2).
-        const __amdgpu_buffer_rsrc_t proj = ga_buffer(tok, ((long long)(pj.n_splits - 1) * pj.split_stride + pj.ld) * 4);
+        // (a buffer a K piece, empty where there is none: its offsets are those of one row)
+        __amdgpu_buffer_rsrc_t proj[4];
+#pragma unroll
+        for (int sp = 0; sp < 4; ++sp)
+            proj[sp] = ga_buffer(tok + (sp < pj.n_splits ? sp * pj.split_stride : 0), sp < pj.n_splits ? (long long)pj.ld * 4 : 0);
         const int rot = EXTRA ? pj.rot : D, half = rot / 2;
         const bool scaled = pj.row_ssq != nullptr, whole4 = scaled && (pj.row_parts & 3) == 0;
         const float* ssq = scaled ? pj.row_ssq + (size_t)t * pj.row_parts : tok;
@@ -226,7 +230,7 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
 #pragma unroll
                     for (int sp = 0; sp < 4; ++sp)
                         raw[i][j][sp] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
-                            proj, sp < pj.n_splits ? at + (uint32_t)(j * 64 + sp * pj.split_stride) * 4u : BUF_NOWHERE, 0, 0));
+                            proj[sp], at + (uint32_t)(j * 64) * 4u, 0, 0));
                 gain[i] = r[i] < group ? pj.q_gain : (r[i] == group ? pj.k_gain : nullptr);
                 const float* from = gain[i] ? gain[i] : tok;
 #pragma unroll

@@ -284,6 +284,30 @@ def test_decode_fused_applies_a_row_scale():
             assert float((a - b).abs().max()) <= 1e-2 * float(a.abs().max())
 
 
+def test_decode_fused_takes_partial_sums_that_lie_far_apart():
+    """K pieces of the projection more than 31 bits of bytes apart (rows much wider than the projection) give the same bits as
+    the same pieces side by side."""
+    hq, hkv, d, splits = 4, 2, 64, 5
+    seqs = [(70, 1), (200, 1)]
+    rows, ld = (hq + 2 * hkv) * d, 90_000_000
+    g = torch.Generator().manual_seed(23)
+    sums = torch.randn(splits, 2, rows, generator=g).cuda()
+    wide = torch.empty(splits, 2, ld, device="cuda")
+    wide[:, :, :rows] = sums
+    angle = torch.rand(2, d // 2, generator=g) * 6.28
+    cos, sin, gain = torch.cos(angle).cuda(), torch.sin(angle).cuda(), torch.ones(d, device="cuda")
+    ws = torch.empty(32 << 20, dtype=torch.uint8, device="cuda")
+    got = []
+    for qkv in (sums, wide):
+        dev, _, _, _ = _build(seqs, hq, hkv, d, torch.bfloat16, 24)
+        out = torch.full((2, hq * d), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ops.attention_decode_fused(qkv, out, dev["kc"], dev["vc"], dev["table"], None, dev["tok_pos"], hq, hkv, d, d ** -0.5, gain, gain,
+                                   1e-5, cos, sin, workspace=ws, max_len=200, n_splits=2)
+        got.append((out, dev["kc"], dev["vc"]))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 def test_decode_fused_without_norm_or_rotation():
     _fused_case([(77, 1), (200, 1)], 8, 4, 128, 2, 3, None, seed=12, norm=False)
     _fused_case([(77, 1), (200, 1)], 8, 4, 128, 1, 0, None, seed=13, rotate=False)
