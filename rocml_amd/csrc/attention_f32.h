@@ -131,7 +131,7 @@ __device__ __forceinline__ void af_add_odd_values(const af_f32x4_t (&p)[4], cons
 }
 
 // (registers for as many blocks as find room in a CU's LDS)
-constexpr int af_prompt_lds(int d) { return (AF_PAGE * (d + 4) + d * (AF_PAGE + 4)) * 4; }
+constexpr int af_prompt_lds(int d) { return (AF_PAGE * (d + 4) + d * (AF_PAGE + 4) + 4) * 4; }
 constexpr int af_prompt_blocks(int d) { return 160 * 1024 / af_prompt_lds(d) < 4 ? 160 * 1024 / af_prompt_lds(d) : 4; }
 
 template <int KD>
@@ -139,8 +139,10 @@ __global__ void __launch_bounds__(256, af_prompt_blocks(KD * 16))
 attn_f32_prompt_kernel(AttnF32Args a) {
     constexpr int D = KD * 16, KS = D + 4, VS = AF_PAGE + 4;      // padded rows: 16 rows fall into different banks
     extern __shared__ float af_smem[];
-    __shared__ int odd_page;                          // the last page that holds an infinite or NaN value
     float *ks = af_smem, *vs = af_smem + AF_PAGE * KS;
+    float& odd_page = vs[D * VS];                     // the last page that holds an infinite or NaN value (a variable of its own
+                                                      // before the rows would put them at an odd multiple of 4 bytes, and one
+                                                      // that is no float would make the page table's reads vector loads)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int seq = blockIdx.y, kvh = blockIdx.z, group = a.hq / a.hkv;
     const int t0 = a.cu_seqlens[seq], count = a.cu_seqlens[seq + 1] - t0;
@@ -161,34 +163,41 @@ attn_f32_prompt_kernel(AttnF32Args a) {
         o[c] = af_f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
     float m = -INFINITY, l = 0.f;
-    if (threadIdx.x == 0) odd_page = -1;
+    if (threadIdx.x == 0) odd_page = -1.f;
     for (int p = 0; p <= last_pos / AF_PAGE; ++p) {
         if (p >= kept_pages && p < lo_page) continue;
         const size_t at = ((size_t)pages[p] * a.hkv + kvh) * AF_PAGE * D;
         // Values behind `known` are another sequence's, if any.  The page's values meet the probabilities of 16 rows at once,
         // and zero times infinity is NaN: a row must not see the infinite or NaN value of a key it does not see (a later
-        // token's, or one before its window).  Such values are left out of the products and added to the rows that see them.
+        // token's, or one before its window).  Such values are taken out of the page and added to the rows that see them.
         const int known = last_pos - p * AF_PAGE;
         __syncthreads();
+        float odd = 0.f;                              // NaN once a value was infinite or NaN
         for (int i = threadIdx.x; i < AF_PAGE * D / 4; i += 256) {
             *(af_f32x4_t*)(ks + i / (D / 4) * KS + i % (D / 4) * 4) = *(const af_f32x4_t*)(a.kcache + at + i * 4);
             af_f32x4_t v = *(const af_f32x4_t*)(a.vcache + at + i * 4);
             int key = i % (AF_PAGE / 4) * 4;
-            bool odd = false;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                bool here = key + e <= known, finite = af_finite(v[e]);
-                odd = odd || (here && !finite);
-                v[e] = here && finite ? v[e] : 0.f;
+                v[e] = key + e <= known ? v[e] : 0.f;
+                odd = fmaf(v[e], 0.f, odd);
             }
-            if (odd) odd_page = p;
             *(af_f32x4_t*)(vs + i / (AF_PAGE / 4) * VS + key) = v;
         }
+        if (!(odd == 0.f)) odd_page = (float)p;
         __syncthreads();
+        const bool repair = odd_page == (float)p;
+        if (repair) {
+            for (int i = threadIdx.x; i < AF_PAGE * D; i += 256) {
+                float& v = vs[i / AF_PAGE * VS + i % AF_PAGE];
+                if (!af_finite(v)) v = 0.f;
+            }
+            __syncthreads();
+        }
         af_scores<KD, 4>(q, [&](int kt, int c) { return *(const af_f32x4_t*)(ks + (kt * 16 + (lane & 15)) * KS + c * 16 + (lane >> 4) * 4); }, s);
         af_softmax<KD, 4>(s, o, m, l, a, p * AF_PAGE, lane, pos, lo, slope);
         af_values<KD, 4>(s, [&](int c, int kt) { return *(const af_f32x4_t*)(vs + (c * 16 + (lane & 15)) * VS + kt * 16 + (lane >> 4) * 4); }, o);
-        if (odd_page == p) af_add_odd_values<KD>(s, a.vcache + at, o, a, p * AF_PAGE, lane, pos, lo);
+        if (repair) af_add_odd_values<KD>(s, a.vcache + at, o, a, p * AF_PAGE, lane, pos, lo);
     }
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
