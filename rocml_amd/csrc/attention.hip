@@ -285,7 +285,7 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
         AttnF32Args a{(const float*)q, (const float*)kcache, (const float*)vcache, (float*)out, block_table, token_seq, token_pos,
                       cu_seqlens, bt_width, hq, hkv, window, scale, ex};
         int rc;
-#define AF_SIZE(KD_) rc = launch_attn_f32<KD_>(a, n_tokens, n_seqs, max_new, cu_count(), stream)
+#define AF_SIZE(KD_) rc = launch_attn_f32<KD_>(a, n_tokens, n_seqs > 0 ? q_counts : nullptr, n_seqs, max_new, max_len, cu_count(), stream)
         switch (d / 16) {
             case 1: AF_SIZE(1); break;
             case 2: AF_SIZE(2); break;

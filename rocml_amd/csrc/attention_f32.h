@@ -27,11 +27,13 @@ struct AttnF32Args {
     int bt_width, hq, hkv, window;
     float scale;
     AttnExtra ex;
+    int few = 0;                // with both kernels: sequences of at most so many query tokens are the token kernel's
 };
 
-// Scores of 16 rows with NT tiles of 16 keys: krow(t, c) is the lane's piece (16 c + 4 (l/16) .. + 3) of key 16 t + l%16.
-template <int KD, int NT, typename Row>
-__device__ __forceinline__ void af_scores(const af_f32x4_t (&q)[KD], Row krow, af_f32x4_t (&s)[NT]) {
+// Scores of 16 rows with NT tiles of 16 keys: krow(t, c) is the lane's piece (16 c + 4 (l/16) .. + 3) of key 16 t + l%16,
+// query(c) that of its row.
+template <int KD, int NT, typename Query, typename Row>
+__device__ __forceinline__ void af_scores(Query query, Row krow, af_f32x4_t (&s)[NT]) {
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
         // two sums, of the even and the odd places: a product waits 32 clocks for the one before it in its sum
@@ -39,11 +41,11 @@ __device__ __forceinline__ void af_scores(const af_f32x4_t (&q)[KD], Row krow, a
         s[t] = odd;
 #pragma unroll
         for (int c = 0; c < KD; ++c) {
-            af_f32x4_t a = krow(t, c);
+            af_f32x4_t a = krow(t, c), q = query(c);
 #pragma unroll
             for (int e = 0; e < 4; e += 2) {
-                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], q[c][e], s[t], 0, 0, 0);
-                odd = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e + 1], q[c][e + 1], odd, 0, 0, 0);
+                s[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], q[e], s[t], 0, 0, 0);
+                odd = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e + 1], q[e + 1], odd, 0, 0, 0);
             }
         }
         s[t] += odd;
@@ -147,7 +149,7 @@ attn_f32_prompt_kernel(AttnF32Args a) {
     const int seq = blockIdx.y, kvh = blockIdx.z, group = a.hq / a.hkv;
     const int t0 = a.cu_seqlens[seq], count = a.cu_seqlens[seq + 1] - t0;
     const int row0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * 64, n_rows = count * group;   // the longest rows first
-    if (row0 >= n_rows) return;
+    if (row0 >= n_rows || count <= a.few) return;
     const int row = min(row0 + wave * 16 + (lane & 15), n_rows - 1);
     const int t = t0 + row / group, h = kvh * group + row % group;
     const int pos = a.token_pos[t], lo = attn_first_key(pos, a.window, a.ex.chunk);
@@ -194,7 +196,7 @@ attn_f32_prompt_kernel(AttnF32Args a) {
             }
             __syncthreads();
         }
-        af_scores<KD, 4>(q, [&](int kt, int c) { return *(const af_f32x4_t*)(ks + (kt * 16 + (lane & 15)) * KS + c * 16 + (lane >> 4) * 4); }, s);
+        af_scores<KD, 4>([&](int c) { return q[c]; }, [&](int kt, int c) { return *(const af_f32x4_t*)(ks + (kt * 16 + (lane & 15)) * KS + c * 16 + (lane >> 4) * 4); }, s);
         af_softmax<KD, 4>(s, o, m, l, a, p * AF_PAGE, lane, pos, lo, slope);
         af_values<KD, 4>(s, [&](int c, int kt) { return *(const af_f32x4_t*)(vs + (c * 16 + (lane & 15)) * VS + kt * 16 + (lane >> 4) * 4); }, o);
         if (repair) af_add_odd_values<KD>(s, a.vcache + at, o, a, p * AF_PAGE, lane, pos, lo);
@@ -222,10 +224,19 @@ template <int KD, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
 attn_f32_token_kernel(AttnF32Args a) {
     constexpr int D = KD * 16, ROW = D + 4;
-    extern __shared__ float af_smem[];                // [WAVES][16][ROW], then maxima and sums [WAVES][16] each
-    float *os = af_smem, *ms = af_smem + WAVES * 16 * ROW, *ls = ms + WAVES * 16;
+    extern __shared__ float af_smem[];                // [WAVES][16][ROW], then maxima and sums [WAVES][16] each, then [16][ROW] queries
+    float *os = af_smem, *ms = af_smem + WAVES * 16 * ROW, *ls = ms + WAVES * 16, *qs = ls + WAVES * 16;
+    // Sixteen waves leave 128 registers a lane, which keys, values, queries and sums of 128 numbers a head fill: the queries
+    // stay in LDS then (in registers, seven others were spilled; 64 sequences of 1,000 keys: 118 and 105 us).
+    constexpr bool Q_IN_LDS = WAVES == 16 && KD == 8;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int t = blockIdx.x, kvh = blockIdx.y, group = a.hq / a.hkv, g0 = blockIdx.z * 16;
+    const int kvh = blockIdx.y, group = a.hq / a.hkv, g0 = blockIdx.z * 16;
+    int t = blockIdx.x;
+    if (a.few) {                                      // blocks for `few` tokens of every sequence
+        const int seq = t / a.few, at = t % a.few, t0 = a.cu_seqlens[seq], count = a.cu_seqlens[seq + 1] - t0;
+        if (count > a.few || at >= count) return;
+        t = __builtin_amdgcn_readfirstlane(t0 + at);
+    }
     const int h = kvh * group + min(g0 + (lane & 15), group - 1);
     const int pos = a.token_pos[t], lo = attn_first_key(pos, a.window, a.ex.chunk);
     const int* pages = a.block_table + (size_t)a.token_seq[t] * a.bt_width;
@@ -233,8 +244,14 @@ attn_f32_token_kernel(AttnF32Args a) {
     af_f32x4_t q[KD], o[KD], s[1];
 #pragma unroll
     for (int c = 0; c < KD; ++c) {
-        q[c] = *(const af_f32x4_t*)(a.q + ((size_t)t * a.hq + h) * D + c * 16 + (lane >> 4) * 4);
+        if (!Q_IN_LDS) q[c] = *(const af_f32x4_t*)(a.q + ((size_t)t * a.hq + h) * D + c * 16 + (lane >> 4) * 4);
         o[c] = af_f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    if (Q_IN_LDS) {
+        for (int c = wave; c < KD; c += WAVES)
+            *(af_f32x4_t*)(qs + (lane & 15) * ROW + c * 16 + (lane >> 4) * 4) =
+                *(const af_f32x4_t*)(a.q + ((size_t)t * a.hq + h) * D + c * 16 + (lane >> 4) * 4);
+        __syncthreads();
     }
     float m = -INFINITY, l = 0.f;
     // the pages of the kept first positions, then those of the window
@@ -255,7 +272,11 @@ attn_f32_token_kernel(AttnF32Args a) {
         if (KD <= 8)
 #pragma unroll
             for (int c = 0; c < KD; ++c) v[c] = *(const af_f32x4_t*)(vp + c * 16 * AF_PAGE);
-        af_scores<KD, 1>(q, [&](int, int c) { return k[c]; }, s);
+        if constexpr (Q_IN_LDS)
+            af_scores<KD, 1>([&](int c) { return *(const af_f32x4_t*)(qs + (lane & 15) * ROW + c * 16 + (lane >> 4) * 4); },
+                             [&](int, int c) { return k[c]; }, s);
+        else
+            af_scores<KD, 1>([&](int c) { return q[c]; }, [&](int, int c) { return k[c]; }, s);
         if (KD > 8)                                   // (beyond 128 numbers a head both do not fit the registers)
 #pragma unroll
             for (int c = 0; c < KD; ++c) v[c] = *(const af_f32x4_t*)(vp + c * 16 * AF_PAGE);
@@ -305,13 +326,55 @@ attn_f32_token_kernel(AttnF32Args a) {
     }
 }
 
+// Microseconds of both kernels over a step whose sequences have counts[b] query tokens (each `all` without counts) when those
+// of at most `few` go to the token kernel.  A page costs a block of 64 rows about 1 us per 16 numbers of a head and a block of
+// one token a quarter of it (its waves share the page), half as much again where the blocks are more than the CUs; measured
+// at heads of 32, 128 and 256: 1.4, 1.0 and 0.9, and 0.27 at all three.  How far back a sequence reaches is known of the longest
+// one only (`pages`): up to 64 tokens are taken to stand at the end of so much, more of them to be a whole prompt.
+static double af_cost(int few, const int* counts, int n_seqs, int all, int pages, int d, int group, int hkv, int cus) {
+    struct { double work = 0.0, longest = 0.0; } rows, token;       // pages of all blocks, and of the longest
+    for (int b = 0; b < n_seqs; ++b) {
+        int c = counts ? counts[b] : all;
+        if (c == 0) continue;
+        double reach = n_seqs == 1 || c <= AF_PAGE || ceil_div(c, AF_PAGE) > pages ? pages : ceil_div(c, AF_PAGE);
+        auto& k = c <= few ? token : rows;
+        k.work += reach * hkv * (c <= few ? (double)c * ceil_div(group, 16) : (double)ceil_div((long long)c * group, 64));
+        if (reach > k.longest) k.longest = reach;
+    }
+    double t = 0.0, page = d / 16.0;
+    if (rows.work > 0.0) t += 6.0 + page * (rows.work > cus * rows.longest ? rows.work / cus : rows.longest);
+    if (token.work > 0.0) t += 6.0 + 0.25 * page * (token.work > cus * token.longest ? 1.5 * token.work / cus : token.longest);
+    return t;
+}
+
+// The line between the two kernels for a step: the cheapest of the powers of two, none and all.  Blocks of 64 rows pay for
+// prompts; a few tokens behind a long context, or one token a sequence beside a prompt, leave them nearly empty and few, each
+// walking all pages by itself.  Microseconds at 8 heads of 256 on 2: 5 tokens behind 1,000 positions 196 in blocks of 64 rows,
+// 64 by token; 5 new ones 18 and 8; 300 ones beside 15 sequences of one token and 2,000 positions 481, and 232 with both kernels.
+static int af_few(const AttnF32Args& a, int d, const int* counts, int n_seqs, int max_new, int max_len, int cus) {
+    const int group = a.hq / a.hkv;
+    int pages = max_len > 0 ? ceil_div(max_len, AF_PAGE) : a.bt_width;
+    const int span = a.window > 0 ? a.window : a.ex.chunk;
+    if (span > 0) {
+        int seen = ceil_div(span, AF_PAGE) + 1 + ceil_div(a.ex.keep_first, AF_PAGE);
+        if (seen < pages) pages = seen;
+    }
+    int best = max_new;
+    double best_t = af_cost(max_new, counts, n_seqs, max_new, pages, d, group, a.hkv, cus);
+    for (long long few = 0; few < max_new && few <= 4096; few = few ? 2 * few : 1) {
+        double t = af_cost((int)few, counts, n_seqs, max_new, pages, d, group, a.hkv, cus);
+        if (t < best_t) { best = (int)few; best_t = t; }
+    }
+    return best;
+}
+
 template <int KD>
-static int launch_attn_f32(const AttnF32Args& a, int n_tokens, int n_seqs, int max_new, int cus, hipStream_t stream) {
+static int launch_attn_f32(AttnF32Args a, int n_tokens, const int* counts, int n_seqs, int max_new, int max_len, int cus, hipStream_t stream) {
     constexpr int D = KD * 16;
     const int group = a.hq / a.hkv;
     constexpr int PROMPT_LDS = af_prompt_lds(D);
     constexpr int MANY = D <= 128 ? 16 : 8;           // (registers: a tile's keys and values, the queries and the sums)
-    constexpr int FEW_LDS = 4 * 16 * (D + 6) * 4, MANY_LDS = MANY * 16 * (D + 6) * 4;
+    constexpr int FEW_LDS = 4 * 16 * (D + 6) * 4, MANY_LDS = MANY * 16 * (D + 6) * 4 + (MANY == 16 && D == 128 ? 16 * (D + 4) * 4 : 0);
     static bool ready = false;
     if (!ready) {
         const struct { const void* f; int bytes; } all[] = {{(const void*)attn_f32_prompt_kernel<KD>, PROMPT_LDS},
@@ -322,16 +385,25 @@ static int launch_attn_f32(const AttnF32Args& a, int n_tokens, int n_seqs, int m
                 return rocml_fail("attention: cannot reserve %d bytes of LDS", k.bytes);
         ready = true;
     }
-    // A tile of 64 rows is worth filling from 16 rows a sequence on.
-    if (a.cu_seqlens && n_seqs > 0 && (long long)max_new * group >= 16 && max_new > 1) {
+    const int few = a.cu_seqlens && n_seqs > 0 && max_new > 1 ? af_few(a, D, counts, n_seqs, max_new, max_len, cus) : 0x7fffffff;
+    long long by_token = 0, by_rows = 0;              // tokens of either kernel
+    for (int b = 0; few < max_new && b < n_seqs; ++b) {
+        int c = counts ? counts[b] : max_new;
+        (c <= few ? by_token : by_rows) += c;
+    }
+    // (a kernel that runs alone takes every sequence, whatever its count: a recorded step may be replayed with others)
+    if (by_rows > 0) {
+        if (by_token > 0) a.few = few;
         dim3 grid(ceil_div((long long)max_new * group, 64), n_seqs, a.hkv);
         attn_f32_prompt_kernel<KD><<<grid, 256, PROMPT_LDS, stream>>>(a);
-        return 0;
+        if (by_token == 0) return 0;
+    } else {
+        by_token = n_tokens;
     }
     // Waves a block by the room of the block table, which a recorded step keeps as its sequences grow: more than four where
     // the pages are many and the blocks are not.
-    dim3 grid(n_tokens, a.hkv, ceil_div(group, 16));
-    if (a.bt_width >= 8 && (long long)n_tokens * a.hkv <= 2ll * cus)
+    dim3 grid(a.few ? n_seqs * a.few : n_tokens, a.hkv, ceil_div(group, 16));
+    if (a.bt_width >= 8 && by_token * a.hkv <= 2ll * cus)
         attn_f32_token_kernel<KD, MANY><<<grid, 64 * MANY, MANY_LDS, stream>>>(a);
     else
         attn_f32_token_kernel<KD, 4><<<grid, 256, FEW_LDS, stream>>>(a);

@@ -574,3 +574,28 @@ def test_float32_prompt_rows_do_not_see_what_unseen_keys_hold(hq, hkv, d, seqs, 
     assert not got[1].isfinite().all() and got[1].isfinite().any()
     # (the finite ones: as in the test above)
     torch.testing.assert_close(got[0], got[1], rtol=0.0, atol=1e-5, equal_nan=True)
+
+
+# (query heads, kv heads, head size, [(context length, new tokens)]): one token (two, eight) a sequence beside prompts, which are
+# the other kernel's; a few tokens behind a long context, and 300 of them, on either side of the line
+@pytest.mark.parametrize("hq,hkv,d,seqs", [(16, 8, 128, [(300, 300), (2000, 1), (700, 1), (65, 1)]), (8, 2, 256, [(9, 1), (400, 400), (1500, 2), (130, 1)]),
+                                           (20, 1, 64, [(2200, 1), (3000, 3000), (900, 8)]), (4, 4, 48, [(1000, 1), (900, 900)]),
+                                           (16, 8, 128, [(1500, 16)]), (2, 2, 16, [(1200, 300)]), (34, 2, 32, [(400, 3), (390, 1)])])
+@pytest.mark.parametrize("mask", [{}, {"window": 65, "keep_first": 3}, {"chunk": 50, "slopes": True}])
+def test_float32_steps_that_mix_prompts_and_single_tokens(hq, hkv, d, seqs, mask):
+    """Every token gets its result from one of the two kernels, whichever the step's line gives it to, as from the plain one; and
+    the same without the host's counts, by which the line is drawn."""
+    dev, _, _, _ = _build(seqs, hq, hkv, d, torch.float32, 31)
+    kw = {k: v for k, v in mask.items() if k != "slopes"}
+    if mask.get("slopes"):
+        kw["slopes"] = (torch.rand(hq, generator=torch.Generator().manual_seed(32)) * 0.1).cuda()
+    counts = [n for _, n in seqs]
+    got = []
+    for algo, known in ((PLAIN, counts), (0, counts), (0, None)):
+        out = torch.full_like(dev["q"], float("nan"))
+        ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, d ** -0.5,
+                      algo=algo, cu_seqlens=dev["cu"], max_new=max(counts), q_counts=known, max_len=max(length for length, _ in seqs), **kw)
+        got.append(out.double())
+    # (both are 32-bit: sums of up to 256 products and 3,000 probabilities in another order)
+    assert float((got[1] - got[0]).abs().max()) < 1e-5
+    assert float((got[2] - got[0]).abs().max()) < 1e-5
