@@ -169,9 +169,12 @@ static int launch_latent(const LatentArgs& a, hipStream_t stream) {
     attn_latent_mfma_kernel<KD, DT, RT><<<dim3(a.tiles, n_splits), 256, L::BYTES, stream>>>(
         a.q, a.out, a.cache, a.block_table, a.bt_width, a.cu_seqlens, a.n_seqs, a.token_pos, a.n_heads, a.dk, a.dv,
         a.scale * LOG2E, a.window, n_splits, part_o, part_ml);
-    if (n_splits > 1)
-        attn_latent_reduce_kernel<<<(unsigned)rows, (ALR_GROUPS * (a.dv / 4) + 63) / 64 * 64, (64 + ALR_GROUPS * a.dv) * sizeof(float), stream>>>(
-            part_o, part_ml, a.out, n_splits, a.dv);
+    if (n_splits > 1) {
+        if (n_splits <= 8) launch_latent_reduce<1>(part_o, part_ml, a.out, rows, n_splits, a.dv, stream);
+        else if (n_splits <= 16) launch_latent_reduce<2>(part_o, part_ml, a.out, rows, n_splits, a.dv, stream);
+        else if (n_splits <= 32) launch_latent_reduce<4>(part_o, part_ml, a.out, rows, n_splits, a.dv, stream);
+        else launch_latent_reduce<8>(part_o, part_ml, a.out, rows, n_splits, a.dv, stream);
+    }
     return 0;
 }
 

@@ -263,49 +263,60 @@ attn_latent_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, 
 }
 
 // Log-sum-exp merge of the splits of a row: one block per row.  At most 64 splits: lane s of every wave fetches split s's
-// reference and sum, so these loads go out together.  Eight groups of threads take every eighth split each, four values a
-// thread, all eight loads in one trip while the weights are formed, and meet in LDS in group order (a thread a value with the
-// splits eight at a time was 14 trips at 51 splits of 512 values: 11.4 us, now 4.8).
-constexpr int ALR_GROUPS = 8;
-__global__ void __launch_bounds__(1024)
+// reference and sum, so these loads go out together.  GROUPS groups of threads, one for every eight splits, take every GROUPS th
+// split each, four values a thread, all eight loads in one trip while the weights are formed, and meet in LDS in group order.
+// A thread a value with the splits eight at a time was 14 trips at 51 splits of 512 values: 11.4 us, now 4.8.  Eight groups
+// whatever the number of splits left most of a block idle where the rows are many and their splits few: 8,192 rows of 512
+// values in two splits took 31 us longer.
+template <int GROUPS>
+__global__ void __launch_bounds__(128 * GROUPS)
 attn_latent_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                           bf16_t* __restrict__ out, int n_splits, int dv) {
-    extern __shared__ float alr_smem[];               // [64 weights][ALR_GROUPS][dv]
+    extern __shared__ float alr_smem[];               // [64 weights][GROUPS][dv]
     float *wgt = alr_smem, *sums = alr_smem + 64;
     size_t row = blockIdx.x;
     const float* ml = part_ml + row * n_splits * 2;
     const float* po = part_o + row * n_splits * dv;
     const int lane = threadIdx.x & 63, quads = dv / 4;
-    const int group = (int)threadIdx.x / quads, d = (int)threadIdx.x % quads * 4;   // (threads beyond the groups: group >= 8)
+    const int group = (int)threadIdx.x / quads, d = (int)threadIdx.x % quads * 4;   // (threads beyond the groups: group >= GROUPS)
     float2 mine = *(const float2*)(ml + 2 * min(lane, n_splits - 1));
     float4 v[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = *(const float4*)(po + (size_t)min(group + i * ALR_GROUPS, n_splits - 1) * dv + d);
+    for (int i = 0; i < 8; ++i) v[i] = *(const float4*)(po + (size_t)min(group + i * GROUPS, n_splits - 1) * dv + d);
     float ms = lane < n_splits ? mine.x : -INFINITY, ls = lane < n_splits ? mine.y : 0.f;
     float mm = wave_max(ms);
     float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mm);
     if (threadIdx.x < 64) wgt[lane] = w;              // (zero beyond the last split)
     float inv_l = 1.0f / wave_sum(ls * w);            // every wave computes the same sum
     __syncthreads();
-    if (group < ALR_GROUPS) {
-        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (group < GROUPS) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            int s = group + i * ALR_GROUPS;
+            int s = group + i * GROUPS;
             if (s >= n_splits) continue;
             float ws = wgt[s];
             acc.x = fmaf(v[i].x, ws, acc.x); acc.y = fmaf(v[i].y, ws, acc.y);
             acc.z = fmaf(v[i].z, ws, acc.z); acc.w = fmaf(v[i].w, ws, acc.w);
         }
-        *(float4*)(sums + group * dv + d) = acc;
+        if (GROUPS > 1) *(float4*)(sums + group * dv + d) = acc;
     }
-    __syncthreads();
-    if (group != 0) return;
-    float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (GROUPS > 1) {
+        __syncthreads();
+        if (group == 0) {
 #pragma unroll
-    for (int g = 0; g < ALR_GROUPS; ++g) {
-        float4 u = *(const float4*)(sums + g * dv + d);
-        t.x += u.x; t.y += u.y; t.z += u.z; t.w += u.w;
+            for (int g = 1; g < GROUPS; ++g) {
+                float4 u = *(const float4*)(sums + g * dv + d);
+                acc.x += u.x; acc.y += u.y; acc.z += u.z; acc.w += u.w;
+            }
+        }
     }
-    *(uint2*)(out + row * dv + d) = make_uint2(f32x2_to_bf16x2(t.x * inv_l, t.y * inv_l), f32x2_to_bf16x2(t.z * inv_l, t.w * inv_l));
+    if (group != 0) return;
+    *(uint2*)(out + row * dv + d) = make_uint2(f32x2_to_bf16x2(acc.x * inv_l, acc.y * inv_l), f32x2_to_bf16x2(acc.z * inv_l, acc.w * inv_l));
+}
+
+template <int GROUPS>
+static void launch_latent_reduce(const float* part_o, const float* part_ml, bf16_t* out, long long rows, int n_splits, int dv, hipStream_t stream) {
+    attn_latent_reduce_kernel<GROUPS><<<(unsigned)rows, (GROUPS * (dv / 4) + 63) / 64 * 64, (64 + (GROUPS > 1 ? GROUPS * dv : 0)) * sizeof(float), stream>>>(
+        part_o, part_ml, out, n_splits, dv);
 }

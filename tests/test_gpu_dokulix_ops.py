@@ -360,6 +360,29 @@ def test_matrix_core_kernel_for_latent_rows(H, DK, DV, window, decode):
     assert float(err.max()) < 2e-2 * max(1.0, float(ref.abs().max())), f"row {int(err.argmax())}, position {pos[int(err.argmax())]}"
 
 
+@pytest.mark.parametrize("splits", [1, 2, 8, 9, 16, 17, 32, 33, 60])
+@pytest.mark.parametrize("H,DK,DV", [(3, 576, 512), (20, 96, 64), (5, 48, 40)])
+def test_merge_of_latent_splits(H, DK, DV, splits):
+    """Three tokens over 4,000 keys; the room for partial results decides on the splits: the merge's numbers of threads to
+    either side of every line between them."""
+    from rocml_amd import ops
+    gen = torch.Generator().manual_seed(splits + DK)
+    T, n = 4000, 3
+    pages = (T + PAGE - 1) // PAGE
+    k = torch.randn(pages * PAGE, DK, generator=gen).to(torch.bfloat16)
+    q = torch.randn(n, H, DK, generator=gen).to(torch.bfloat16)
+    out = torch.full((n, H * DV), float("nan"), dtype=torch.bfloat16, device=DEV)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)                 # noqa: E731
+    ws = torch.empty(splits * n * H * (DV + 2) * 4, dtype=torch.uint8, device=DEV)
+    ops.attention(q.reshape(n, -1).to(DEV), out, k.view(pages, 1, PAGE, DK).to(DEV), None, i32([list(range(pages))]), i32([0] * n),
+                  i32([T - 3, T - 2, T - 1]), H, 1, DK, DK ** -0.5, algo=ops.ATTN_MFMA, workspace=ws, cu_seqlens=i32([0, n]), max_new=n,
+                  q_counts=[n], max_len=T, v_head_dim=DV, values_in_keys=True)
+    s = torch.einsum("thd,kd->thk", q.double(), k.double()) * DK ** -0.5
+    s.masked_fill_(torch.arange(pages * PAGE) > torch.tensor([T - 3, T - 2, T - 1])[:, None, None], float("-inf"))
+    ref = torch.einsum("thk,kd->thd", torch.softmax(s, -1), k[:, :DV].double())
+    assert float((out.double().cpu().view(n, H, DV) - ref).abs().max()) < 2e-2 * float(ref.abs().max())
+
+
 @pytest.mark.parametrize("tx", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("T,H,K,N,xs,os_", [(1, 3, 16, 24, 24, 32), (8, 16, 128, 512, 192, 576), (70, 4, 40, 20, 48, 20),
                                             (300, 2, 512, 128, 512, 128), (17, 6, 64, 32, 64, 32)])
