@@ -1411,46 +1411,50 @@ norm_add_vec_kernel(float* __restrict__ x, const float* __restrict__ y, const fl
     // With a few rows this is priced in trips to memory: everything the row needs is asked for at once (the next norm's
     // gain too), the K pieces GROUP at a time, and no load stands behind a branch or a select, where the wave would wait
     // for it: threads beyond the row's end read its start and count nothing.  Five rows of 2048 with four pieces: 9.2 -> 5.0 us.
+    // Waves wholly beyond the end of a short row read nothing (8,192 rows of 96 with one piece: 8.4 us, 11.2 if they do).
     __shared__ float scratch[EW_BLOCK / WAVE];
     size_t row = (size_t)blockIdx.x * n;
     int nv = n / 4;
     typedef __attribute__((ext_vector_type(4))) float vec4;       // (a choice between two of these stays in registers)
     const vec4 zero4 = {0.f, 0.f, 0.f, 0.f};
     constexpr int GROUP = VEC <= 2 ? 4 : VEC <= 4 ? 2 : 1;
+    const bool idle = VEC == 1 && (int)__builtin_amdgcn_readfirstlane(threadIdx.x) >= nv;
     const bool prepare = copy && next_gain;
     const float* ng = prepare ? next_gain : gain;
     const float* src = replace ? x : y;               // (read and not counted: the pieces are the whole of y)
-    vec4 yv[VEC], xv[VEC], gv[VEC], bv[VEC], nv4[VEC];
+    vec4 yv[VEC], xv[VEC], gv[VEC], bv[VEC], nv4[VEC], sum[VEC];
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) {
-        int i = threadIdx.x + j * EW_BLOCK;
-        int at = i < nv ? i : 0;
-        yv[j] = ((const vec4*)(src + row))[at];
-        xv[j] = ((const vec4*)(x + row))[at];
-        gv[j] = ((const vec4*)gain)[at];
-        nv4[j] = ((const vec4*)ng)[at];
-        bv[j] = zero4;
-        if (LAYER && bias) bv[j] = ((const vec4*)bias)[at];
-    }
-    // the K pieces of the product that made y, in split order
-    vec4 sum[VEC];
+    for (int j = 0; j < VEC; ++j) yv[j] = xv[j] = gv[j] = bv[j] = nv4[j] = sum[j] = zero4;
+    if (!idle) {
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) sum[j] = replace ? zero4 : yv[j];
-    for (int sp = 0; sp < n_splits; sp += GROUP) {
-        vec4 p[GROUP][VEC];
+        for (int j = 0; j < VEC; ++j) {
+            int i = threadIdx.x + j * EW_BLOCK;
+            int at = i < nv ? i : 0;
+            yv[j] = ((const vec4*)(src + row))[at];
+            xv[j] = ((const vec4*)(x + row))[at];
+            gv[j] = ((const vec4*)gain)[at];
+            nv4[j] = ((const vec4*)ng)[at];
+            if (LAYER && bias) bv[j] = ((const vec4*)bias)[at];
+        }
+        // the K pieces of the product that made y, in split order
 #pragma unroll
-        for (int q = 0; q < GROUP; ++q)
+        for (int j = 0; j < VEC; ++j) sum[j] = replace ? zero4 : yv[j];
+        for (int sp = 0; sp < n_splits; sp += GROUP) {
+            vec4 p[GROUP][VEC];
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) {
-                int i = threadIdx.x + j * EW_BLOCK;
-                p[q][j] = ((const vec4*)(partials + min(sp + q, n_splits - 1) * split_stride + row))[i < nv ? i : 0];
-            }
+            for (int q = 0; q < GROUP; ++q)
 #pragma unroll
-        for (int q = 0; q < GROUP; ++q)
+                for (int j = 0; j < VEC; ++j) {
+                    int i = threadIdx.x + j * EW_BLOCK;
+                    p[q][j] = ((const vec4*)(partials + min(sp + q, n_splits - 1) * split_stride + row))[i < nv ? i : 0];
+                }
 #pragma unroll
-            for (int j = 0; j < VEC; ++j) {
-                sum[j] = sp + q < n_splits ? sum[j] + p[q][j] : sum[j];
-            }
+            for (int q = 0; q < GROUP; ++q)
+#pragma unroll
+                for (int j = 0; j < VEC; ++j) {
+                    sum[j] = sp + q < n_splits ? sum[j] + p[q][j] : sum[j];
+                }
+        }
     }
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {

@@ -219,3 +219,27 @@ def test_refusals():
         ops.rmsnorm(x.cuda(), torch.ones(9).cuda(), 1e-5, torch.empty(2, 8).cuda())
     with pytest.raises(KernelError):
         ops.swiglu(torch.randn(2, 9).cuda(), torch.empty(2, 4).cuda())
+
+
+@pytest.mark.parametrize("n", [4, 96, 252, 260, 1000, 1028])
+@pytest.mark.parametrize("splits,replace", [(0, False), (1, True), (3, False), (5, True)])
+@pytest.mark.parametrize("layer", [False, True])
+def test_norm_add_rows_shorter_than_a_block(n, splits, replace, layer):
+    """Rows that end inside a wave and leave whole waves of a block without values: K pieces, the next norm, a copy."""
+    rows = 5
+    g = torch.Generator().manual_seed(n + splits)
+    x, y = torch.randn(rows, n, generator=g), torch.randn(rows, n, generator=g)
+    gain, bias, after = 1 + 0.2 * torch.randn(n, generator=g), 0.1 * torch.randn(n, generator=g), 1 + 0.2 * torch.randn(n, generator=g)
+    parts = torch.randn(splits, rows, n, generator=g) if splits else None
+    whole = (0 if replace else y.double()) + (parts.double().sum(0) if splits else 0)
+    mid = whole - whole.mean(-1, keepdim=True) if layer else whole
+    stream = x.double() + mid / torch.sqrt((mid ** 2).mean(-1, keepdim=True) + 1e-5) * gain.double() + (bias.double() if layer else 0)
+    normed = stream / torch.sqrt((stream ** 2).mean(-1, keepdim=True) + 1e-6) * after.double()
+    for prepared in (False, True):
+        xd, copy = x.cuda(), torch.full((rows, n), float("nan"), device="cuda")
+        if replace:
+            y = torch.full_like(y, float("nan"))
+        ops.norm_add(xd, y.cuda(), gain.cuda(), bias.cuda() if layer else None, 1e-5, layer, copy=copy, partials=None if parts is None else parts.cuda(),
+                     replace=replace, next_gain=after.cuda() if prepared else None, next_eps=1e-6)
+        assert float((xd.double().cpu() - stream).abs().max()) < 2e-5
+        assert float((copy.double().cpu() - (normed if prepared else stream)).abs().max()) < 2e-5
