@@ -423,7 +423,11 @@ static int launch_kpar(const void* x, int ldx, const void* w, int ldw, void* out
     int by_k = ceil_div(k, 1024);                      // (a wave then has one chunk of 256)
     if (splits > by_k) splits = by_k;
     if (splits > plan.max_splits) splits = plan.max_splits;
-    if (splits < 1 || epi_gated(EPI) || (k <= 2048 && !(plan.defer && ldo == n))) splits = 1;   // whole sums spare the reduce kernel
+    // Whole sums spare the reduce kernel: up to K of 2048, and up to 4096 while the blocks are at most one a CU and enough to pull
+    // the weights by themselves (microseconds at one row and K of 4096, in pieces and whole: 1024 columns 6.2 and 7.4, 1536 7.3
+    // and 7.4, 2048 7.7 and 7.4, 4096 11.9 and 9.4; the few-rows kernel 7.6, 7.7, 8.2 and 10.7).
+    const bool deferred = plan.defer && ldo == n;
+    if (splits < 1 || epi_gated(EPI) || (!deferred && (k <= 2048 || (k <= 4096 && 8 * n_tiles > 3 * cu_count() && n_tiles <= cu_count())))) splits = 1;
     long long per_split = (long long)m * n * sizeof(float);
     if (splits > 1 && (long long)splits * per_split > workspace_bytes)
         splits = workspace ? (int)(workspace_bytes / per_split) : 1;
@@ -640,9 +644,11 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
         // few-rows kernel: 12288 x 2048 11.5 and 12.6 for 15.0 and 14.6, 8192 x 2048 8.6 and 9.5 for 12.6 and 12.2, 6144 x 1024
         // 6.1 and 6.6 for 6.9; at 16 rows 14.8 for 15.1, 10.8 for 12.3 and 7.3 for 7.0), and up to two rows and K of 4096 in
         // whole chunks (24576 x 4096 36.8 for 38.0; 41.5 for 36.4 at 8 rows; 19456 x 2560, whose waves end in a half chunk, 22.0 for 22.0).
-        // A product whose pieces nobody adds pays a kernel for them: the same rule.
+        // A product whose pieces nobody adds pays a kernel for them: the same rule, but with K beyond 2048 for at most one block a
+        // CU (5000 x 4096 at one row: 13.1 whole and 16.1 in pieces, 12.5 in the few-rows kernel).
         bool whole = gated || !(plan.defer && ldo == n);
-        one_trip = one_trip || (whole && ((m <= 8 && k <= 2048 && n <= 48 * cus) || (m <= 2 && k <= 4096 && k % 1024 == 0)));
+        one_trip = one_trip || (whole && ((m <= 8 && k <= 2048 && n <= 48 * cus) ||
+                                          (m <= 2 && k <= 4096 && k % 1024 == 0 && (gated || n <= 16 * cus))));
         bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && (one_trip || (m <= 2 && !gated && 2 * (n / 16) >= 3 * cus)));
         if (kpar) rc = BY_EPI(launch_kpar, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else if (skinny) rc = BY_EPI(launch_skinny_m, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
