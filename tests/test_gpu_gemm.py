@@ -141,6 +141,21 @@ def test_more_tiles_than_compute_units(m, n, k, epilogue):
     assert float((out.double() - ref).abs().max()) < (2e-5 if epilogue is None else 5e-3) * max(1.0, float(ref.abs().max()))
 
 
+@pytest.mark.parametrize("m,n,k", [(4200, 4400, 72), (4100, 4609, 200)])
+def test_more_tiles_than_compute_units_into_the_stream(m, n, k):
+    """The same with the sums added to what is there, which reads memory while the next tile's operands are on their way, and
+    with a plain bfloat16 result."""
+    x, w = _operands(m, n, k, torch.bfloat16, 7)
+    ref = _ref(x, w)
+    base = torch.randn(m, n, device="cuda")
+    acc = base.clone()
+    ops.gemm(x, w, acc, accumulate=True, algo=TILE256)
+    assert float((acc.double() - (ref + base.double())).abs().max()) < 2e-5 * max(1.0, float(ref.abs().max()))
+    out16 = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    ops.gemm(x, w, out16, algo=TILE256)
+    assert float((out16.double() - ref).abs().max()) < 5e-3 * max(1.0, float(ref.abs().max()))
+
+
 def test_strided_rows_and_refusals():
     from rocml_amd.errors import KernelError
     big = torch.randn(40, 200, device="cuda").to(torch.bfloat16)
@@ -219,6 +234,19 @@ def test_gated_epilogue(m, n, k, algo):
         assert float((out32.double().cpu() - ref.cpu()).abs().max()) < 2e-5 * max(1.0, float(ref.abs().max()))
 
 
+@pytest.mark.parametrize("m,n,k,algo", [(1, 64, 64, PLAIN), (25, 300, 520, PLAIN), (130, 256, 30, 0), (7, 70, 33, 0)])
+def test_float32_gated_by_the_plain_kernel(m, n, k, algo):
+    """Asked for by number, and where K is no multiple of 4."""
+    x, w = _operands(m, n, k, torch.float32, 3)
+    full = _ref(x, w)
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+    for epilogue, act in (("swiglu", torch.nn.functional.silu), ("relu_glu", torch.relu)):
+        out = torch.empty(m, n // 2, device="cuda")
+        ops.gemm(x, w, out, algo=algo, workspace=ws, epilogue=epilogue)
+        ref = act(full[:, 0::2]) * full[:, 1::2]
+        assert float((out.double() - ref).abs().max()) < 2e-5 * max(1.0, float(ref.abs().max())), epilogue
+
+
 @pytest.mark.parametrize("m,algo", [(1, KPAR), (8, SKINNY), (40, SKINNY), (130, TILE), (130, TILE64X256), (130, TILE192), (300, TILE256)])
 def test_gated_results_are_the_exact_ones_rounded_once(m, algo):
     """silu(gate) * up over the whole range in which exp(-gate) is finite, formed in 32-bit: the stored bfloat16 is the rounding of
@@ -285,6 +313,38 @@ def test_many_rows_with_k_cut_in_pieces(m, n, k):
     small = torch.empty(m * n * 4, dtype=torch.uint8, device="cuda")
     out16 = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
     assert ops.gemm(x, w, out16, workspace=small, defer=True) == 0
+    assert float((out16.double() - ref).abs().max()) < 5e-3 * scale
+
+
+# sizes at which the library cuts K and takes 256x256 tiles, with remainders in M, N and K and a short last piece; the last has
+# more tiles and pieces than compute units, so that a block goes from one K piece to another
+@pytest.mark.parametrize("m,n,k,pieces", [(930, 3243, 5144, 3), (386, 3283, 7480, 7), (918, 2165, 5408, 5), (3101, 4979, 17224, 3)])
+def test_256x256_tiles_with_k_cut_in_pieces(m, n, k, pieces):
+    """Every piece holds the sums of its own range of K, the same bits as that range's product alone; added they are the product.
+    The operands are column ranges of wider matrices that hold NaN beside them."""
+    x, w = _operands(m, n, k, torch.bfloat16, 8)
+    wide_x, wide_w = torch.full((m, k + 64), float("nan"), dtype=torch.bfloat16, device="cuda"), torch.full(
+        (n, k + 72), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide_x[:, 8:8 + k], wide_w[:, 16:16 + k] = x, w
+    x, w = wide_x[:, 8:8 + k], wide_w[:, 16:16 + k]
+    ref = _ref(x, w)
+    scale = max(1.0, float(ref.abs().max()))
+    ws = torch.full((pieces * m * n,), float("nan"), device="cuda")
+    base = torch.randn(m, n, device="cuda")
+    acc = base.clone()
+    assert ops.gemm(x, w, acc, accumulate=True, workspace=ws, defer=True) == pieces and torch.equal(acc, base)
+    step = (-(-k // pieces) + 63) // 64 * 64
+    alone = torch.empty(m, n, device="cuda")
+    for p, sums in enumerate(ws.view(pieces, m, n)):
+        ops.gemm(x[:, p * step:(p + 1) * step], w[:, p * step:(p + 1) * step], alone, algo=TILE256)
+        assert torch.equal(sums, alone), p
+    ops.splitk_reduce(ws.view(pieces, m, n), acc, accumulate=True)
+    whole = base.clone()
+    assert ops.gemm(x, w, whole, accumulate=True, workspace=ws) == 0
+    assert torch.equal(whole, acc)
+    assert float((acc.double() - (ref + base.double())).abs().max()) < 2e-5 * scale
+    out16 = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    ops.gemm(x, w, out16, workspace=ws)
     assert float((out16.double() - ref).abs().max()) < 5e-3 * scale
 
 
