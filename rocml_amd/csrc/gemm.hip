@@ -543,14 +543,16 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
 // 8, 10.9 against 9.0 at 16; 1024 x 3072 6.1 against 5.6 at 1 row, 8.2 against 5.9 at 16; 2048 x 6144 10.0 against 7.8 at
 // 1 row, 11.1 against 7.6 at 4, 12.1 against 7.7 at 8; 4096 x 12288 21.5 against 20.6 at 1 row, 24.0 against 20.9 at 8 (every
 // block reads all activations, which is what more rows cost); 2560 x 9728 (160 blocks) 15.9 against
-// 11.6 at 1 row and 5120 x 5120 (320 blocks, more than a round): not taken.
+// 11.6 at 1 row and 5120 x 5120 (320 blocks, more than a round): not taken.  Between K of 4096 and 8192, up to 4 rows: as far as
+// a wave of twelve has two chunks (K of 6144) it is ahead of product and norm by 0.9 to 1.8 us at 2048 columns and 1.1 to 3.1
+// at 2560; a third chunk costs 0.8 to 1.5 us more than it saves at 2048 and up to 0.9 at 2560, and is 0.5 to 2.3 ahead at 3072.
 ROCML_EXPORT int rocml_gemm_residual_prescale_pays(int m, int n, int k) {
     if (m < 1 || m > 16 || k % 8 != 0) return 0;
     int tiles = ceil_div(n, 16);
     const int cus = cu_count();
     if (tiles > cus) return 0;
     if (k <= 4096) return 1;
-    if (k <= 8192 && m <= 4 && 2 * tiles >= cus) return 1;
+    if (k <= 8192 && m <= 4 && (k <= 6144 ? 2 : 4) * tiles >= (k <= 6144 ? 1 : 3) * cus) return 1;
     return k <= 12288 && m <= 8 && 10 * tiles >= 9 * cus;
 }
 

@@ -381,6 +381,16 @@ def test_residual_sum_that_prepares_the_next_norm(m, n, k, waves):
                                    torch.zeros(17, n, dtype=torch.bfloat16, device="cuda"), torch.zeros(17, tiles, device="cuda"))
 
 
+@pytest.mark.parametrize("m,n,k,pays", [(1, 2048, 4096, True), (4, 2048, 6144, True), (1, 2048, 6152, False), (4, 2560, 8192, False),
+                                        (4, 3072, 8192, True), (5, 3072, 8192, False), (8, 4096, 12288, True), (1, 4112, 4096, False)])
+def test_when_the_prepared_norm_pays(m, n, k, pays):
+    """The rule's lines for 256 compute units, from both ways' measured times."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the lines are those of 256 compute units")
+    x, w = torch.empty(m, k, dtype=torch.bfloat16, device="cuda"), torch.empty(n, k, dtype=torch.bfloat16, device="cuda")
+    assert ops.gemm_residual_prescale_pays(x, w) == pays
+
+
 @pytest.mark.parametrize("m,n,k,which", [(16, 40, 264, "x"), (3, 16, 1032, "w"), (11, 130, 4096, "x")])
 def test_residual_sum_of_rows_far_apart(m, n, k, which, sixteen_far_rows):
     """The same with operand rows beyond each other's 31-bit reach."""
