@@ -106,18 +106,21 @@ using GemmTile64x256 = GemmTile<1, 4, 2, 2>;
 // for a CU that holds one alone, and what a launch costs beside its stages (`fixed`).
 struct TileKind { int bm, bn, cap; double light, full, alone, fixed; int shape; };
 static const TileKind TILE_KINDS[] = {
-    {128, 128, 2, 0.91, 1.03, 0.62, 2.8, 1}, {256, 256, 1, 1.11, 1.37, 0.0, 5.8, 2}, {256, 192, 1, 1.03, 1.32, 0.0, 6.6, 3},
-    {128, 192, 1, 0.74, 0.83, 0.0, 4.8, 4},  {256, 96, 1, 0.80, 0.86, 0.0, 4.4, 5},  {64, 256, 1, 0.70, 0.78, 0.0, 2.7, 6}};
+    {128, 128, 2, 0.918, 1.14, 0.577, 3.24, 1}, {256, 256, 1, 1.099, 1.393, 0.0, 7.27, 2}, {256, 192, 1, 1.032, 1.316, 0.0, 5.04, 3},
+    {128, 192, 1, 0.683, 0.83, 0.0, 4.15, 4},   {256, 96, 1, 0.751, 0.835, 0.0, 4.08, 5},  {64, 256, 1, 0.72, 0.729, 0.0, 3.17, 6}};
 
 // An estimate of a product's time in microseconds with tiles of `kind` and K cut into `pieces`
 // (each piece the work of a block of its own, 32-bit partial sums written once here and read once
 // by whoever adds them): the rounds of blocks the chip holds at a time, each round as long as its
 // K stages at the rate of the CUs' load, but no shorter than the busiest CU needs to pull its
-// blocks' operands (60 GB/s a CU: with few rows it is the weights' arrival that a block waits for,
-// and more, smaller blocks pull more at a time); a fixed part for the launch; the bytes the
-// epilogue moves; never less than the weights need to arrive at all.  The constants were fitted
-// to 16 products (the Qwen3-8B, 14B, 0.6B and the 2B designs' layers) at 96 to 8192 rows, each
-// shape with whole K: the estimate is 4.5 to 6 % off (root mean square) per shape.
+// blocks' operands (70 GB/s a CU: with few rows it is the weights' arrival that a block waits for,
+// and more, smaller blocks pull more at a time); a fixed part for the launch and one for every further
+// round; the bytes the epilogue moves; never less than the weights need to arrive at all.
+// The constants are those with the least loss by the choice over 3,563 products (64 to 2,048 rows, 13 outputs from
+// 520 to 24576, K from 512 to 12288; left to the next kernel, whole, gated), each measured with all shapes and
+// one to eight pieces of which an estimate is within 1.6 of the best (55,713 times, weights from memory): the choice
+// is 0.6 % behind the best on average, more than 5 % behind for 132 of them and 23 % at worst.  (Fitted to the times
+// of whole K alone it had been 1.2 %, 319 and 41 %.)  The estimate itself is 9 to 14 % off (root mean square) per shape.
 static double tile_cost(const TileKind& kind, int pieces, int m, int n, int k, int epi, bool defer, int cus) {
     long long tiles = (long long)ceil_div(m, kind.bm) * ceil_div(n, kind.bn);
     int k_per_piece = round_up(ceil_div(k, pieces), GM_BK);
@@ -134,15 +137,15 @@ static double tile_cost(const TileKind& kind, int pieces, int m, int n, int k, i
     long long rounds = blocks / slots, rest = blocks % slots;
     double t = (double)rounds * stages * stage_us(slots) + (rest ? stages * stage_us(rest) : 0.0);
     double pulled = (double)(kind.bn + (m < kind.bm ? m : kind.bm)) * k_per_piece * 2.0 * (double)ceil_div(blocks, (long long)cus);
-    if (t < pulled / 60.0e3) t = pulled / 60.0e3;
-    t += kind.fixed;
+    if (t < pulled / 70.3e3) t = pulled / 70.3e3;
+    t += kind.fixed + 1.79 * (double)(rounds + (rest ? 1 : 0) - 1);
     double moved = epi_gated(epi) ? (double)m * n
                    : pieces > 1      ? (double)m * n * 4.0 * pieces
                                      : (double)m * n * 4.0 * (epi == EPI_ACC ? 2.0 : 1.0);
-    t += moved / (pieces > 1 ? 4.0e6 : 8.0e6);                       // (partial sums leave when all blocks end together)
-    double floor_us = (double)n * k * 2.0 / 5.5e6;                  // the weights at 5.5 TB/s
+    t += moved / (pieces > 1 ? 5.24e6 : 4.25e6);
+    double floor_us = (double)n * k * 2.0 / 5.87e6;                 // the weights at 5.9 TB/s
     if (t < floor_us) t = floor_us;
-    if (pieces > 1) t += (double)pieces * m * n * 4.0 / 5.0e6 + (defer ? 0.0 : 4.0);   // read again, by a kernel of their own unless deferred
+    if (pieces > 1) t += (double)pieces * m * n * 4.0 / 5.0e6 + (defer ? 0.0 : 3.96);   // read again, by a kernel of their own unless deferred
     return t;
 }
 

@@ -318,7 +318,7 @@ def test_many_rows_with_k_cut_in_pieces(m, n, k):
 
 # sizes at which the library cuts K and takes 256x256 tiles, with remainders in M, N and K and a short last piece; the last has
 # more tiles and pieces than compute units, so that a block goes from one K piece to another
-@pytest.mark.parametrize("m,n,k,pieces", [(930, 3243, 5144, 3), (386, 3283, 7480, 7), (918, 2165, 5408, 5), (3101, 4979, 17224, 3)])
+@pytest.mark.parametrize("m,n,k,pieces", [(1051, 2749, 5320, 4), (402, 4046, 9328, 7), (546, 3295, 7280, 6), (1309, 5576, 8816, 3)])
 def test_256x256_tiles_with_k_cut_in_pieces(m, n, k, pieces):
     """Every piece holds the sums of its own range of K, the same bits as that range's product alone; added they are the product.
     The operands are column ranges of wider matrices that hold NaN beside them."""
