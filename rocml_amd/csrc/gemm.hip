@@ -417,12 +417,15 @@ static int launch_skinny(const void* x, int ldx, const void* w, int ldw, void* o
 }
 
 // At most 16 rows: blocks of 16 weight rows, K split over the block's waves and, while there are
-// fewer than four blocks a CU, over blocks as well (each wave keeps at least 256 of K).
+// fewer than three blocks a CU, over blocks as well (in pieces of at most 1024: up to 256 of K a wave).
 template <int EPI>
 static int launch_kpar(const void* x, int ldx, const void* w, int ldw, void* out, int ldo, int m, int n, int k,
                        void* workspace, long long workspace_bytes, SplitPlan plan, hipStream_t stream) {
     int n_tiles = ceil_div(n, 16);
-    int splits = 4 * cu_count() / n_tiles;
+    // A CU holds three blocks, and four blocks of which the last waits cost more than they bring, but for K below 2048, where a
+    // wave has less than a chunk (microseconds at one row, four and three blocks a CU: 8192 x 9728 36.2 and 33.1, 8192 x 3072
+    // 14.6 and 12.4, 7168 x 6144 22.2 and 20.8; 8192 x 1536 8.2 and 8.9).
+    int splits = (k < 2048 ? 4 : 3) * cu_count() / n_tiles;
     int by_k = ceil_div(k, 1024);                      // (a wave then has one chunk of 256)
     if (splits > by_k) splits = by_k;
     if (splits > plan.max_splits) splits = plan.max_splits;
@@ -559,6 +562,40 @@ ROCML_EXPORT int rocml_gemm_residual_prescale_pays(int m, int n, int k) {
     return k <= 12288 && m <= 8 && 10 * tiles >= 9 * cus;
 }
 
+// Whether the kernel whose waves split K is the faster one for up to 16 rows where K in pieces of 1024 leaves a wave one chunk of
+// 256 and the next kernel adds the pieces: one trip to memory without staging and with half the partial sums of the few-rows
+// kernel.  Compared with that kernel on 6,594 products of 1 to 16 rows (15 outputs from 520 to 24576, K from 256 to 12288):
+//  * at most one block a CU: 10 to 25 % faster (4096 x 1024 5.0 us for 5.5 at one row, 2048 x 2048 4.4 for 5.4), but whole sums of
+//    640 to 896, which the few-rows kernel cuts in two small pieces, 2 to 20 % slower (2048 x 768 1.02 to 1.08 times at 3 to 16 rows);
+//  * more than one: the CUs with a block more than the others decide.  A chunk that is half full is still ahead (K of 512: 5 to
+//    12 %; of 256, where staging costs nothing, 12 % behind), two pieces where the second round is nearly whole (4096 x 1536 0.92
+//    times, 2560 x 1408 1.09 to 1.19), more pieces than two equal, with half the pieces for the next kernel; whole sums
+//    of 1024 are 6 to 20 % behind (5120 x 1024 6.2 us for 5.5 at one row, 7.2 for 6.0 at 16).
+// From 48 K outputs on the few-rows kernel leaves a K of up to 768 whole, and is 12 to 33 % behind.
+static bool kpar_pieces_pay(int m, int n, int k, int cus) {
+    const int pieces = ceil_div(k, 1024), blocks = ceil_div(n, 16) * pieces;
+    if (k > 512 && k <= 768 && (long long)m * n >= 48 * 1024) return true;
+    if (blocks <= cus) return pieces > 1 || k <= 512 || k > 960;
+    return k > 2048 || (k > 256 && k <= 512) || (pieces == 2 && 8 * blocks >= 14 * cus && ceil_div(k, 2) <= 960);
+}
+
+// The same for sums that must be whole (the gated product, or pieces that nobody would add), up to 8 rows.  K of up to 2048 (gated,
+// microseconds at 1 and 8 rows against the few-rows kernel: 12288 x 2048 11.5 and 13.0 for 14.0 and 13.7, 8192 x 2048 8.7 and 10.1
+// for 11.9 and 11.8, 6144 x 1024 5.3 and 6.0 for 6.0 and 6.0), and up to two rows K of 4096 in whole chunks (24576 x 4096 38.0 for
+// 39.1 at one row, 41.5 for 36.4 at 8).  With more than one block a CU the last chunk of a wave must be worth its trip, the more
+// so the more rows there are (times of the few-rows kernel's, 5120 columns: K of 1280 1.06 at 1 row, 1.10 at 4 and 1.17 at 8, 1536 0.98,
+// 1.06 and 1.12, 1792 0.88, 0.97 and 1.02; K of 256 1.03 to 1.16).  A product whose pieces nobody adds pays a kernel for them in the
+// few-rows kernel: there only K of 256 is behind (1.05 to 1.24), and K beyond 2048 is taken for at most one block a CU
+// (5000 x 4096 at one row: 13.1 whole, 16.1 in pieces, 12.5 in the few-rows kernel).
+static bool kpar_whole_pays(int m, int n, int k, bool gated, int cus) {
+    const bool narrow = n <= 16 * cus;                // at most one block a CU
+    if (m <= 2 && k <= 4096 && k % 1024 == 0 && (gated || narrow)) return true;
+    if (m > 8 || k > 2048 || n > 48 * cus) return false;
+    if (narrow) return true;
+    const int last = (k - 1) % 1024 + 1, least = 128 * (m <= 2 ? 2 : m);
+    return gated ? last > (least < 768 ? least : 768) : k > 256;
+}
+
 // algo: 0 = choose, 1 = plain tiled kernel, 2 = MFMA tile kernel (128x128 tiles), 3 = MFMA few-rows
 // kernel (M <= 64), 4 = MFMA kernel for at most 16 rows, 5 to 9 = MFMA tile kernel with 256x256,
 // 256x192, 128x192, 256x96 and 64x256 tiles.
@@ -631,30 +668,16 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
          : epi == EPI_ACC ? fn<EPI_ACC>(__VA_ARGS__)                 \
          : epi == EPI_RELU2 ? fn<EPI_RELU2>(__VA_ARGS__)             \
          : epi == EPI_RELUGLU ? fn<EPI_RELUGLU>(__VA_ARGS__) : fn<EPI_SWIGLU>(__VA_ARGS__))
-        // One or two rows (but not the gated product, which has its own choice of blocks): the
-        // kernel whose waves split K, unless the output is narrow (fewer than
-        // one and a half blocks of 16 weight rows a CU: 4096 or 5120 wide on 256 CUs, the products
-        // that return to the hidden size): its blocks are then so few that K must be cut across
-        // blocks as well and a wave is left with one chunk; the few-rows kernel is 10 to 15 %
-        // faster there.  Beyond two rows the activations
-        // read from L2 cost more than the block sharing of the few-rows kernel.
-        // But where K in pieces of 1024 leaves a wave one chunk of 256 and the blocks are at most two a CU (one and a half
-        // beyond 8 rows), it is one trip to memory without staging and with half the partial sums: microseconds at 1 and 8
-        // rows against the few-rows kernel 4.3 and 4.5 for 5.6 and 5.8 at 4096 x 1024, 4.3 and 4.6 for 5.6 and 5.7 at
-        // 2048 x 2048, 6.3 and 6.6 for 6.5 and 6.5 at 4096 x 2048 (512 blocks), 7.9 and 8.5 for 7.7 at 6144 x 2048 (768).
+        // The kernel whose waves split K: where K in pieces of 1024 leaves a wave one chunk, where sums must be whole, and
+        // for one or two rows against a wide output (at least one and a half blocks of 16 weight rows a CU; beyond two
+        // rows the activations read from L2 cost more than the block sharing of the few-rows kernel).
         const long long pieces = ceil_div(k, 1024), kpar_blocks = ceil_div(n, 16) * pieces;
-        bool one_trip = m <= 16 && !gated && (pieces == 1 || (workspace && plan.defer && ldo == n)) && pieces <= plan.max_splits &&
-                        2 * kpar_blocks <= (m <= 8 ? 4 : 3) * (long long)cus && pieces * m * n * 4 <= workspace_bytes + (pieces == 1 ? (1ll << 60) : 0);
-        // The gated product, which cannot be cut along K: up to 8 rows and K of 2048 (microseconds at 1 and 8 rows against the
-        // few-rows kernel: 12288 x 2048 11.5 and 12.6 for 15.0 and 14.6, 8192 x 2048 8.6 and 9.5 for 12.6 and 12.2, 6144 x 1024
-        // 6.1 and 6.6 for 6.9; at 16 rows 14.8 for 15.1, 10.8 for 12.3 and 7.3 for 7.0), and up to two rows and K of 4096 in
-        // whole chunks (24576 x 4096 36.8 for 38.0; 41.5 for 36.4 at 8 rows; 19456 x 2560, whose waves end in a half chunk, 22.0 for 22.0).
-        // A product whose pieces nobody adds pays a kernel for them: the same rule, but with K beyond 2048 for at most one block a
-        // CU (5000 x 4096 at one row: 13.1 whole and 16.1 in pieces, 12.5 in the few-rows kernel).
-        bool whole = gated || !(plan.defer && ldo == n);
-        one_trip = one_trip || (whole && ((m <= 8 && k <= 2048 && n <= 48 * cus) ||
-                                          (m <= 2 && k <= 4096 && k % 1024 == 0 && (gated || n <= 16 * cus))));
-        bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && (one_trip || (m <= 2 && !gated && 2 * (n / 16) >= 3 * cus)));
+        const bool deferred = plan.defer && ldo == n;
+        bool one_trip = m <= 16 && !gated && (pieces == 1 || (workspace && deferred)) && pieces <= plan.max_splits &&
+                        2 * kpar_blocks <= (m <= 8 ? 4 : 3) * (long long)cus && pieces * m * n * 4 <= workspace_bytes + (pieces == 1 ? (1ll << 60) : 0) &&
+                        (deferred ? kpar_pieces_pay(m, n, k, cus) : k > 256 || n <= 16 * cus);
+        bool whole = (gated || !deferred) && kpar_whole_pays(m, n, k, gated, cus);
+        bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && (one_trip || whole || (m <= 2 && !gated && 2 * (n / 16) >= 3 * cus)));
         if (kpar) rc = BY_EPI(launch_kpar, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else if (skinny) rc = BY_EPI(launch_skinny_m, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else rc = BY_EPI(launch_mfma_tile, x, ldx, w, ldw, out, ldo, m, n, k,

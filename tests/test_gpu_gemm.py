@@ -64,7 +64,8 @@ def test_bfloat16_algorithms(m, n, k, algo):
 
 # one chunk of 256 a wave, one and a rest, K in pieces of 1024 with a rest; N that is no tile; rows to either side of the rule's limits
 @pytest.mark.parametrize("m,n,k", [(1, 40, 8), (3, 1000, 1024), (8, 2047, 1032), (9, 2048, 2048), (16, 520, 3080), (8, 4096, 2048), (2, 70, 264),
-                                   (1, 1536, 4096), (2, 1552, 4096), (1, 4096, 3072), (2, 4112, 4096)])
+                                   (1, 1536, 4096), (2, 1552, 4096), (1, 4096, 3072), (2, 4112, 4096),
+                                   (1, 8208, 3080), (12, 4112, 640), (16, 2560, 1408), (4, 4112, 1280), (3, 4112, 256), (8, 4112, 1800)])
 def test_few_rows_in_one_trip(m, n, k):
     """The operands are column ranges of wider matrices that hold NaN beside them; whole sums, deferred pieces and the gated
     activation, by the library's own choice of kernel."""
