@@ -1,8 +1,8 @@
 // Attention over the paged key/value cache for gfx950.  One entry point for any step: the
 // query tokens of a step carry their sequence and position, keys and values are read from
 // the cache (the step's own keys were appended before), so prefill, decode and any cut of a
-// prompt run the same code.  bfloat16 with a head size that is a multiple of 32 runs on the
-// matrix cores; everything else, and the whole 32-bit path, runs the plain kernel.
+// prompt run the same code.  bfloat16 with a head size of 32, 64, 96, 128, 192 or 256 and 32-bit
+// with one that attention_f32.h takes run on the matrix cores; everything else runs the plain kernel.
 #include "common.h"
 #include "attention_generic.h"
 #include "attention_f32.h"
@@ -280,7 +280,9 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
         return 0;
     }
     AttnExtra ex{dv, v_in_k, chunk, slopes, sink, sinks, softcap, keep_first};
-    // the 32-bit path: the matrix cores' own 32-bit products, for the head sizes that fill their tiles
+    // the 32-bit path: the matrix cores' own 32-bit products, for head sizes that are whole tiles of 16.  Each size is three
+    // kernels of its own: the sizes of this library's models, test models included, and those of the bfloat16 kernels have them; others that would fit (80,
+    // 144, 160, ...) stay with the plain kernel.
     bool f32_ok = dtype == ROCML_F32 && plain_features && page_size == AF_PAGE && hkv <= 65535 && n_seqs <= 65535 &&
                   ((uintptr_t)q | (uintptr_t)out | (uintptr_t)kcache | (uintptr_t)vcache) % 16 == 0 &&
                   (d == 16 || d == 32 || d == 48 || d == 64 || d == 96 || d == 112 || d == 128 || d == 192 || d == 256);

@@ -1,6 +1,6 @@
 // Plain attention over the paged cache for any head size and either storage type: one
-// 256-thread block per (query token, query head).  It serves the 32-bit path (prefill and
-// decode) and every head size the fast kernels refuse.  The algebra is the reference's
+// 256-thread block per (query token, query head).  It serves every head size, page size and cache
+// layout that the matrix-core kernels (attention_mfma.h, attention_f32.h, attention_latent.h) refuse.  The algebra is the reference's
 // (rocml-kernels/kernels/attn_decode.hip:151-170, attn_prefill.hip:167-190): s_j = (q . k_j) *
 // scale, running maximum m, l = l * e^(m - m') + sum e^(s - m'), acc likewise, out = acc / l.
 // A query at position p sees keys [lo, p], lo = 0 or p - window + 1.  Keys are taken 256 at a

@@ -1,7 +1,7 @@
 // Matrix products of the decoder: out[M,N] (+)= X[M,K] * W[N,K]^T, weights row-major
 // [out, in] as the reference keeps them (rocml/src/weights/mod.rs:78-98).  bfloat16 operands
-// go to the MFMA kernels when their layout allows 16-byte loads; everything else, and the
-// whole 32-bit path, goes to the plain tiled kernel.
+// go to the MFMA kernels and 32-bit operands to the 32-bit matrix instructions (gemm_f32.h) when
+// their layout allows 16-byte loads; everything else goes to the plain tiled kernel.
 #include "common.h"
 #include "gemm_tile.h"
 #include "gemm_mfma.h"
@@ -526,7 +526,7 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
     int tiles = ceil_div(n, 16);
     ROCML_REQUIRE(waves == 0 || waves == 4 || waves == 8 || waves == 12 || waves == 16,
                   "gemm_residual_prescale: 4, 8, 12 or 16 waves, got %d", waves);
-    if (waves == 0) waves = prescale_waves(k);
+    if (waves == 0) waves = prescale_waves(k);       // (16 only for a caller that asks: 8.8 us for 8.4 with eight at K of 4096)
     const bool one = round_up(ceil_div(k, waves), 32) <= 256;
 #define GRP_LAUNCH(W_, ...)                                                                                     \
     gemm_residual_prescale_kernel<W_, __VA_ARGS__><<<tiles, 64 * W_, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, resid, \
@@ -692,7 +692,9 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
         return 0;
     }
     // 32-bit operands in 16-byte pieces: the 32-bit matrix instructions, the few-rows kernel while its reads of the
-    // activations (every block reads them all) stay below the weights'
+    // activations (every block reads them all) stay below the weights'.  Kernel, tiles and K pieces follow from the number of
+    // rows, so a row's sums are rounded in another order in another batch (by about 1e-6 of the row's largest sum); ALGO_PLAIN
+    // gives the same bits in every batch.
     bool f32_pieces = x_dtype == ROCML_F32 && w_dtype == ROCML_F32 && out_dtype == ROCML_F32 && k % 4 == 0 && ldx % 4 == 0 &&
                       ldw % 4 == 0 && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0);
     if (f32_pieces && algo == ALGO_AUTO) {

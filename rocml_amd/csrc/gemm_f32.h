@@ -124,7 +124,10 @@ static int launch_f32_rows(const float* x, int ldx, const float* w, int ldw, flo
 
 // Many rows: 128x128 tiles, or 64x64 where those leave CUs idle, K cut in pieces (32-bit partial sums, as everywhere) where
 // that still leaves CUs idle.  Bound by the matrix cores: a stage (32 of K) is 4,096 clocks for a 128x128 tile, 1,024 for a
-// 64x64 one, whatever else the CU holds.
+// 64x64 one, whatever else the CU holds.  The stage times of the estimate below are those clocks at some 2.1 GHz and a little
+// for the stage's turn; a full chip takes up to 2.2 and 0.75 us.  Of 42 products (six layers at 33 to 2,048 rows, both tiles,
+// one to eight pieces) the choice is 2.8 % behind the best on average, within 5 % for 32, 16 % behind at worst (574 rows,
+// 2048 x 6144: 161 us in three pieces of 128x128 tiles, 138 in eight of 64x64).
 using GemmTile64 = GemmTile<2, 2, 1, 1>;
 
 template <int EPI>

@@ -27,7 +27,8 @@
 //    product at every number of rows up to 64 (it cannot be cut along K, so the waves a block
 //    are what makes its blocks one round over the CUs), and for products cut along K whose
 //    blocks the host chose for the busiest CU.
-//  * gemm_kpar_kernel, one or two rows: the waves of a block split K and meet once in LDS.
+//  * gemm_kpar_kernel, up to 16 rows (one or two against a wide output; more where a wave's share of
+//    K is one chunk; the gated product up to 8): the waves of a block split K and meet once in LDS.
 //  * gemm_residual_prescale_kernel, up to 16 rows: whole sums into the residual stream and the
 //    next norm's operand in one pass.
 #pragma once
@@ -35,7 +36,6 @@
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
-typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;   // 16 bytes as a native vector: a
 // conditional between two of these is a register select, between two uint4 structs it goes

@@ -41,8 +41,9 @@ constexpr uint32_t NOWHERE = 0x80000000u;             // an offset beyond every 
 //  * a block a CU walks through its share of the tiles, and the parts of the next tile are asked for during the last two
 //    stages of this one, so that they arrive while the sums are written.
 // Measured (random operands; the kernel it replaced staged through registers with 32x32x16 products, one barrier a stage):
-// 8192 x 24576 x 4096 gated 1,370 -> 1,095 us (1.20 -> 1.51 PFLOP/s), 8192 x 4096 x 12288 into the stream 765 -> 580,
-// 2048 x 24576 x 4096 352 -> 284, 2048 x 6144 x 4096 94.7 -> 88.  A stage takes 2,519 clocks at 1.9 GHz; without the loads
+// 8192 x 24576 x 4096 gated 1,370 -> 1,161 us (1.20 -> 1.42 PFLOP/s), 8192 x 4096 x 12288 into the stream 765 -> 584,
+// 2048 x 24576 x 4096 gated 352 -> 287, 2048 x 6144 x 4096 94.7 -> 85 (launched one after another on one machine; the
+// gated one took 1,095 and 1,132 on others, and 5 % less with a silu of less than whole 32-bit precision).  A stage takes 2,519 clocks at 1.9 GHz; without the loads
 // 2,200 at 2.05, without the LDS reads 2,230, without both 2,160 at 2.2 (2.0 PFLOP/s): what is left is power and the
 // arrivals' share of the LDS.  Not kept: a ring of five half stages (all 160 KB of LDS, nine phases ahead): 2 % slower; six
 // reads in every phase instead of 8, 4, 8, 4: equal; without the raised priority around the products: equal.

@@ -1,11 +1,11 @@
 // Plain tiled matrix product C[M,N] (+)= X[M,K] * W[N,K]^T for any sizes and any of the
 // supported storage types, accumulating in 32-bit with fused multiply-add and no reduced-
-// precision matrix instruction.  It is the whole 32-bit path's product and the fallback of
-// the bfloat16 path for shapes the MFMA kernels refuse.  Tiling idea as in the reference's
+// precision matrix instruction.  It is the fallback of both paths for layouts the matrix-core
+// kernels refuse (K or row strides that are no whole 16-byte pieces).  Tiling idea as in the reference's
 // first GEMM (rocml-kernels/kernels/gemm_f16.hip:12-41), sized for a 256-thread block:
 // 64x64 outputs per block, 4x4 per thread, K staged 16 at a time through LDS.
-// Each output sums its K products in index order, so a row's result does not depend on
-// which other rows are in the batch.
+// Each output sums its K products in index order, so a row's result here does not depend on
+// which other rows are in the batch (the matrix-core kernels choose by the number of rows).
 #pragma once
 #include "common.h"
 
