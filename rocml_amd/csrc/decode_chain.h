@@ -1,0 +1,791 @@
+// A decode step's layers in one launch (gfx950, wave64, bfloat16): q/k/v projection, attention over the paged cache, output
+// projection, gated feed-forward, layer after layer, for one to four sequences of a model with small layers.
+//
+// What bounds it, and why it is one launch.  With a few rows of activations every product is a walk over its weights, and a
+// step used to be five or six dependent kernels a layer.  A kernel that follows another starts with nothing on its way to it:
+// launch, the first trip to memory and the last store are 4 to 5 us beside its bytes, and the weights, which depend on nothing,
+// wait with everything else.  Here a block (one a CU) takes the products' tiles and the attentions' heads of all layers in the
+// order in which they depend on each other: it asks for its weights (or its pages) first, then waits for its operands, so that
+// the next stages' weights are in registers while this stage's results travel.  From a block's store to the waiting blocks that
+// read it some 1.5 us pass.  A step of the Qwen3-0.6B shape (28 layers, replayed, to the logits): one sequence of 37 tokens
+// 943 -> 546 us, of 500 1,000 -> 619, of 5,000 1,122 -> 925; two of 30 and 700 1,034 -> 715; four up to 700 1,096 -> 821.
+// What is left of a layer (14.5 us) is five times a result's way to the next stage, each with a trip to memory behind its store.
+//
+// Measured on the way: two and three blocks a CU instead of one, 657 and 678 us against 558 (more weights ahead, but what asks
+// for operands is in the way of what answers); eight waves a block 648 against 548 (1.7B: 455 against 500); a wave of its own for
+// operands and results 994; a counter of flags beside plain data instead of words that carry their number 4.2 us from stage to
+// stage against 2.1; one counter of tickets for all 30 ns a ticket, 24 us a layer.
+//
+// Operands travel between blocks as 64-bit words {32 bits of data, 32 bits of the launch's and layer's number}, written and
+// read as relaxed atomics of agent scope, which pass by the L2s that the eight dies do not share: a word is either there whole
+// or not yet, so no flag, fence or order between words is needed.  A buffer is written again a layer later at the earliest:
+// its readers have then all published something that the writer's operands came from.  (Numbers repeat after 2^27 launches.)
+//
+// No wait can last: an item's place in the order is a ticket that a running block draws, and it waits only for items with lower
+// tickets.  The items are dealt over eight counters; of each counter's tickets the lowest unfinished one is held by a block that
+// runs and waits for nothing but finished items, or is the next that a running block draws.  That needs one running block for
+// each counter, which the first eight blocks of the grid are, and no block beside another whatever else the GPU runs.  Should a
+// wait last for seconds all the same, it ends, and the step's result is NaN.
+//
+// The algebra is that of the kernels the step otherwise runs (gemm_kpar_kernel, gemm_residual_prescale_kernel,
+// attn_decode_mfma_kernel FUSED): 32-bit sums on mfma_f32_16x16x32_bf16, the residual stream in 32 bits, the norm's scale
+// applied by the consumer of bfloat16(x * gain), partial results of key splits merged in split order.
+#pragma once
+#include "attention_mfma.h"
+
+typedef unsigned long long u64;
+typedef __attribute__((ext_vector_type(4))) uint32_t dc_u32x4_t;
+
+constexpr int DC_LAYERS = 32;           // layers of a launch (their pointers are kernel arguments)
+constexpr int DC_WAVES = 4, DC_THREADS = 64 * DC_WAVES;
+constexpr int DC_MAX_ROWS = 4;
+constexpr int DC_SHARDS = 8, DC_LINE = 16;      // ticket counters, 64-bit words between two of them (a line)
+constexpr int DC_D = 128;               // head size
+constexpr int DC_MAX_GROUP = 8;
+constexpr int DC_GROUP = 4;             // steps of K (32 wide) asked for together
+constexpr int DC_SHORT = 6, DC_LONG = 6;        // such groups on their way: a wave's whole share of a short K; of a longer one
+constexpr int DC_TILE = 16;             // weight rows of a tile
+constexpr int DC_MAX_TILES = 3;         // tiles of a block whose K is short
+constexpr int DC_MAX_LDS = 80 << 10;     // two launches beside each other fit a CU
+constexpr int DC_APART = 8;             // words between two tiles' sums of squares (side by side sixteen blocks write one line that all ask for: 24 against 20 us a layer)
+constexpr int DC_PAD = 64;              // bytes between two rows of activations in LDS
+constexpr u64 DC_PATIENCE = 400000000ull;       // ticks of 10 ns after which a wait gives up
+
+struct DcLayer {
+    const bf16_t *w_qkv, *w_o, *w_gu, *w_down;
+    const float *q_gain, *k_gain;       // per-head norms
+    const float* ffn_gain;              // the norm between attention and feed-forward
+    const float* next_gain;             // the next layer's first norm (last layer: null)
+    bf16_t *k, *v;                      // cache pages
+};
+
+// Word offsets of the buffers in the state (64-bit words).  The first DC_SHARDS lines hold the ticket counters, the next one the
+// mark of a wait that gave up.
+struct DcPlan {
+    int n_qkv, hq, hkv, hidden, inter, rows, splits, n_layers;
+    int items[6], per_layer;            // work items of a layer's stages, in order
+    int qkv_tiles, gu_tiles;            // tiles of an item of these stages
+    int y, part, part_ml, o, xa, xga, ssqa, h, xb, xgb, ssqb, words;
+    int lds;
+};
+
+struct DcArgs {
+    DcPlan p;
+    u64* state;
+    float* x;                           // [rows, hidden] residual stream, in and out
+    const bf16_t* xn;                   // [rows, hidden] the first layer's normed operand
+    const int* block_table; int bt_width;
+    const int* pos;
+    const float *cos_t, *sin_t;         // [rows, 64]
+    float scale_log2e, qk_eps, eps_mix, eps_ffn, inv_width;
+    DcLayer layer[DC_LAYERS];
+};
+
+__device__ __forceinline__ u64 dc_load(const u64* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void dc_store(u64* p, uint32_t data, uint32_t epoch) {
+    __hip_atomic_store(p, ((u64)epoch << 32) | data, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A wait that has gone on for long: true when it has to end.
+__device__ __forceinline__ bool dc_give_up(u64* state, int tries, u64& since) {
+    if (tries & 255) return false;
+    if (since == 0) since = wall_clock64();
+    if (dc_load(state + DC_SHARDS * DC_LINE) != 0) return true;
+    if (wall_clock64() - since < DC_PATIENCE) return false;
+    __hip_atomic_store(state + DC_SHARDS * DC_LINE, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
+// N words a lane at the addresses that at(i, offset) gives, all of them of this epoch when it returns.  The whole wave stays until the
+// last one is there.
+__device__ __forceinline__ const u64* dc_at(const u64* base, uint32_t bytes) { return (const u64*)((const char*)base + bytes); }
+template <int N, typename At>
+__device__ __forceinline__ void dc_collect(u64* state, uint32_t epoch, bool mine, uint32_t offset, At at, uint32_t (&v)[N]) {
+    u64 w[N], since = 0;
+    for (int tries = 1;; ++tries) {
+        asm volatile("" : "+v"(offset));        // (the addresses are formed in every turn: they do not wait in registers)
+#pragma unroll
+        for (int i = 0; i < N; ++i) w[i] = dc_load(at(i, offset));
+        bool ok = true;
+#pragma unroll
+        for (int i = 0; i < N; ++i) ok &= (uint32_t)(w[i] >> 32) == epoch;
+        if (__all(ok || !mine)) break;
+        if (dc_give_up(state, tries, since)) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) w[i] = 0x7fc07fc0u;         // NaN, as one 32-bit number and as two of 16
+            break;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = (uint32_t)w[i];
+}
+
+// A wave (the block's first) waits until one word of an earlier stage's result is there, one lane asking now and then: until then nothing of what
+// it waits for is near, and hundreds of blocks that ask for all their words all the time are in each other's way.
+__device__ __forceinline__ void dc_far_wait(u64* state, const u64* word, uint32_t epoch) {
+    u64 since = 0;
+    for (int tries = 1; (uint32_t)(__builtin_amdgcn_readfirstlane((int)(dc_load(word) >> 32))) != epoch; ++tries) {
+        __builtin_amdgcn_s_sleep(16);
+        if (dc_give_up(state, tries, since)) break;
+    }
+}
+
+// 1 / sqrt(mean square of a row + eps) from the sums of squares of its tiles, of which the lane has added up its first two
+// already; every lane gets it
+__device__ __forceinline__ float dc_row_scale(u64* state, const u64* ssq, int tiles, uint32_t epoch, float inv_width, float eps, int lane,
+                                              int from = 0, float ss = 0.f) {
+    for (int at = from + lane; at - lane < tiles; at += 64) {       // (a word every DC_APART)
+        uint32_t v[1];
+        bool mine = at < tiles;
+        dc_collect<1>(state, epoch, mine, mine ? at * (8u * DC_APART) : 0u, [&](int, uint32_t o) { return dc_at(ssq, o); }, v);
+        ss += mine ? __uint_as_float(v[0]) : 0.f;
+    }
+    return 1.0f / sqrtf(wave_sum(ss) * inv_width + eps);
+}
+
+// A block's place in the order: {launch, ticket} of its counter.  A block draws until its ticket lies behind its counter's last
+// item, so a counter is drawn from (items + blocks) times a launch; the last draw sets up the next launch.
+struct DcTickets {
+    u64* counter; uint32_t last;
+    __device__ __forceinline__ u64 draw() const { return __hip_atomic_fetch_add(counter, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    __device__ __forceinline__ void drawn(u64 mine, u64* next) const {
+        if ((uint32_t)mine == last) __hip_atomic_store(counter, ((mine >> 32) + 1) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *next = mine;
+    }
+};
+
+enum { DC_QKV = 0, DC_ATTN = 1, DC_MERGE = 2, DC_O = 3, DC_GU = 4, DC_DOWN = 5 };
+
+template <int V> struct DcInt { static constexpr int value = V; };
+
+// What a block works on, the same for all its threads.
+struct DcItem { int stage, layer, i; uint32_t epoch; };
+
+// LDS of a block.
+struct DcLds {
+    u64 next[2];                                // the item after this one, in turn
+    // the waves' sums (two of them in turn: the other waves go on to the next item while the first finishes this one)
+    float red[2][DC_MAX_TILES][DC_WAVES][DC_MAX_ROWS][DC_TILE];
+    float m[DC_WAVES][16], l[DC_WAVES][16];
+    float o[DC_WAVES][DC_MAX_GROUP][DC_D + 4];
+    bf16_t q[DC_MAX_GROUP][DC_D], k[DC_D], v[DC_D];
+    char x[];                                   // operands of a product, rows of 2 K + DC_PAD bytes
+};
+
+__device__ __forceinline__ int dc_k(const DcPlan& p, int stage) { return stage == DC_O ? p.hq * DC_D : stage == DC_DOWN ? p.inter : p.hidden; }
+
+// N rounds of 64 words of every row of operands (stride words apart) into LDS (pitch bytes apart), all asked for together.  SSQ:
+// with them the first two rounds of the rows' sums of squares.
+template <int M, int N, bool SSQ>
+__device__ __forceinline__ void dc_take(u64* st, uint32_t epoch, const u64* row, int stride, char* to, int pitch, const u64* ssq, int tiles,
+                                        int lane, float (&ss)[M]) {
+    constexpr int E = SSQ ? 2 : 0;
+    uint32_t v[M * (N + E)];
+    dc_collect<M * (N + E)>(st, epoch, true, lane * 8u, [&](int i, uint32_t o) {
+        const int m = i / (N + E), j = i % (N + E);
+        return j < N ? dc_at(row + (size_t)m * stride + j * 64, o)
+                     : dc_at(ssq + m * tiles * DC_APART, min(o + (j - N) * 512u, tiles * 8u - 8u) * DC_APART); }, v);
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        if constexpr (SSQ)
+            ss[m] = (lane < tiles ? __uint_as_float(v[m * (N + E) + N]) : 0.f) + (lane + 64 < tiles ? __uint_as_float(v[m * (N + E) + N + 1]) : 0.f);
+#pragma unroll
+        for (int i = 0; i < N; ++i) *(uint32_t*)(to + m * pitch + (i * 64 + lane) * 4) = v[m * (N + E) + i];
+    }
+}
+
+// SHORT: a wave's weights are all in its ring at once (separate code: one ring for both would be held twice).
+// One to three tiles of 16 weight rows times all rows of activations.  A wave has a quarter of K: it asks for its weights, takes
+// its share of the operands into LDS (nobody else reads it) and multiplies; the waves meet once, and the first one finishes.
+__device__ __forceinline__ int dc_tiles(const DcPlan& p, int stage) { return stage == DC_QKV ? p.qkv_tiles : stage == DC_GU ? p.gu_tiles : 1; }
+
+template <int M, bool SHORT>
+__device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, const DcItem& it, DcLds& sm, const DcTickets& tickets, int turn,
+                                           int wave, int lane) {
+    const DcPlan& p = a.p;
+    u64* st = a.state;
+    const int stage = it.stage, layer = it.layer;
+    const uint32_t epoch = it.epoch;
+    const bool residual = stage == DC_O || stage == DC_DOWN, head = layer == 0;
+    const int g = lane >> 4, col = lane & 15;
+    const int tiles = SHORT ? dc_tiles(p, stage) : 1, tile0 = it.i * tiles;
+    const bf16_t* w = stage == DC_QKV ? ly.w_qkv : stage == DC_O ? ly.w_o : stage == DC_GU ? ly.w_gu : ly.w_down;
+    const int k = dc_k(p, stage), share = k / DC_WAVES, first = wave * share, groups = share / (32 * DC_GROUP);
+    auto strip = ga_buffer(w + (size_t)tile0 * DC_TILE * k, (long long)tiles * DC_TILE * k * 2);
+    const uint32_t at = (uint32_t)(col * k + first + g * 8) * 2u;
+    constexpr int RING = SHORT ? DC_SHORT : DC_LONG;
+    dc_u32x4_t ring[RING][DC_GROUP];
+    auto request = [&](int r, int group, int tile) {
+        uint32_t from = group < groups && tile < tiles ? at : BUF_NOWHERE;
+        uint32_t behind = (uint32_t)(tile * DC_TILE * k) * 2u + group * (DC_GROUP * 64);
+#pragma unroll
+        for (int j = 0; j < DC_GROUP; ++j)
+            ring[r][j] = __builtin_bit_cast(dc_u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(strip, from, behind + j * 64, 0));
+    };
+    {
+        int group = 0, tile = 0;
+#pragma unroll
+        for (int r = 0; r < RING; ++r) {
+            request(r, group, tile);
+            if (++group == groups && SHORT) { group = 0; ++tile; }
+        }
+    }
+    // the first wave's lanes in the epilogue: a row of activations and one of 16 columns
+    const int orow = lane >> 4, ocol = tile0 * DC_TILE + col;
+    const bool mine = wave == 0 && orow < M;
+    const float* gain = stage == DC_O ? ly.ffn_gain : ly.next_gain;
+    float gv = 0.f, x_old = 0.f, ss[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) ss[m] = 0.f;
+    if (residual && mine) {
+        if (gain) gv = gain[ocol];
+        if (stage == DC_O && head) x_old = a.x[(size_t)orow * p.hidden + ocol];
+    }
+    asm volatile("" ::: "memory");              // (the requests stay before the waits)
+    __builtin_amdgcn_sched_barrier(0);
+    const int pitch = k * 2 + DC_PAD;
+    // (the next item is drawn when this one's turn is near: drawn with the weights it would be bound to a block that still waits
+    // while others have nothing to do, 37 against 30 us a layer; drawn at the end it would be waited for, 4 us a layer)
+    u64 drawn = 0;
+    if (stage == DC_QKV && head && wave == DC_WAVES - 1 && lane == 0) drawn = tickets.draw();
+    if (stage == DC_QKV && head) {
+#pragma unroll
+        for (int m = 0; m < M; ++m)
+            for (int i = lane; i < share / 2; i += 64)
+                *(uint32_t*)(sm.x + m * pitch + first * 2 + i * 4) = ((const uint32_t*)(a.xn + (size_t)m * k + first))[i];
+    } else {
+        const u64* src = stage == DC_QKV ? st + p.xgb : stage == DC_O ? st + p.o : stage == DC_GU ? st + p.xga : st + p.h;
+        const u64* far = stage == DC_QKV ? st + p.h : stage == DC_O ? st + p.y : stage == DC_GU ? st + p.o : st + p.xga;
+        const int n_far = stage == DC_QKV ? p.inter / 2 : stage == DC_O ? p.n_qkv : stage == DC_GU ? p.hq * DC_D / 2 : p.hidden / 2;
+        const uint32_t src_epoch = stage == DC_QKV ? epoch - 1 : epoch;
+        if (wave == 0) dc_far_wait(st, far + it.i * DC_LINE % n_far, src_epoch);
+        __syncthreads();
+        if (wave == DC_WAVES - 1 && lane == 0) drawn = tickets.draw();
+        if (residual && wave == 0 && !(stage == DC_O && head)) {
+            // (there before the operands are)
+            uint32_t v[1];
+            const u64* from = stage == DC_O ? st + p.xb : st + p.xa;
+            dc_collect<1>(st, stage == DC_O ? epoch - 1 : epoch, mine, mine ? (uint32_t)(orow * p.hidden + ocol) * 8u : 0u,
+                          [&](int, uint32_t o) { return dc_at(from, o); }, v);
+            x_old = __uint_as_float(v[0]);
+        }
+        int left = share / 128;
+        const u64* row = src + first / 2;
+        char* to = sm.x + first * 2;
+        auto take = [&](auto n, auto with_ssq) {
+            constexpr int N = decltype(n)::value;
+            dc_take<M, N, decltype(with_ssq)::value>(st, src_epoch, row, k / 2, to, pitch, st + p.ssqa, p.hidden / DC_TILE, lane, ss);
+            row += N * 64;
+            to += N * 256;
+            left -= N;
+        };
+        if (stage == DC_GU && wave == 0) {
+            if (left >= 4) take(DcInt<4>{}, DcInt<1>{});
+            else if (left >= 2) take(DcInt<2>{}, DcInt<1>{});
+            else take(DcInt<1>{}, DcInt<1>{});
+        }
+        while (left >= 6) take(DcInt<6>{}, DcInt<0>{});
+        if (left >= 4) take(DcInt<4>{}, DcInt<0>{});
+        if (left >= 2) take(DcInt<2>{}, DcInt<0>{});
+        if (left >= 1) take(DcInt<1>{}, DcInt<0>{});
+    }
+    if (wave == DC_WAVES - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const char* xs = sm.x + (M > 1 ? col % M : 0) * pitch + (first + g * 8) * 2;         // (columns beyond the rows repeat them)
+    auto multiply = [&](int r, int group) {
+        dc_u32x4_t xv[DC_GROUP];                // (read together: one by one each product waits for its own trip to LDS)
+#pragma unroll
+        for (int j = 0; j < DC_GROUP; ++j) xv[j] = *(const dc_u32x4_t*)(xs + (group * DC_GROUP + j) * 64);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < DC_GROUP; ++j)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, ring[r][j]), __builtin_bit_cast(bf16x8_t, xv[j]), acc, 0, 0, 0);
+    };
+    auto hand_over = [&](int tile) {
+        // element e of a lane: weight row 4g + e, row of activations col
+        if (col < M) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sm.red[turn][tile][wave][col][g * 4 + e] = acc[e];
+        }
+        acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    };
+    if constexpr (SHORT) {
+        int group = 0, tile = 0;
+#pragma unroll
+        for (int r = 0; r < RING; ++r) {
+            if (tile < tiles) {
+                multiply(r, group);
+                if (++group == groups) {
+                    hand_over(tile);
+                    group = 0;
+                    ++tile;
+                }
+            }
+        }
+    } else {
+        for (int g0 = 0; g0 < groups; g0 += RING) {
+#pragma unroll
+            for (int r = 0; r < RING; ++r) {
+                if (g0 + r < groups) multiply(r, g0 + r);
+                request(r, g0 + r + RING, 0);
+            }
+        }
+        hand_over(0);
+    }
+    float scale = 1.0f;
+    if (stage == DC_GU && wave == 0) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+            float mine_ = dc_row_scale(st, st + p.ssqa + m * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch, a.inv_width, a.eps_ffn, lane, 128, ss[m]);
+            scale = orow == m ? mine_ : scale;
+        }
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    for (int tile = 0; tile < tiles; ++tile) {
+        float v = 0.f;
+        const auto& red = sm.red[turn][tile];
+        if (orow < M) {
+            v = red[0][orow][col];
+#pragma unroll
+            for (int i = 1; i < DC_WAVES; ++i) v += red[i][orow][col];
+        }
+        if (stage == DC_QKV) {
+            if (orow < M) dc_store(st + p.y + (size_t)orow * p.n_qkv + ocol + tile * DC_TILE, __float_as_uint(v), epoch);
+        } else if (stage == DC_GU) {
+            // gate and up rows in turn: even lanes have a gate, their neighbour its up value
+            v *= scale;
+            float up = __shfl_xor(v, 1, 64);
+            float hv = v / (1.0f + expf(-v)) * up;
+            float hn = __shfl_xor(hv, 2, 64);
+            if (orow < M && (col & 3) == 0)
+                dc_store(st + p.h + (size_t)orow * (p.inter / 2) + (tile0 + tile) * 4 + col / 4, f32x2_to_bf16x2(hv, hn), epoch);
+        } else {
+            float r = x_old + v;
+            if (stage == DC_DOWN && layer == p.n_layers - 1) {
+                if (orow < M) a.x[(size_t)orow * p.hidden + ocol] = r;
+                return;
+            }
+            float xg = r * gv, xn = __shfl_xor(xg, 1, 64);
+            float sq = r * r;
+#pragma unroll
+            for (int off = 1; off < 16; off <<= 1) sq += __shfl_xor(sq, off, 64);
+            if (orow < M) {
+                const bool o = stage == DC_O;
+                if ((col & 1) == 0)
+                    dc_store(st + (o ? p.xga : p.xgb) + (size_t)orow * (p.hidden / 2) + ocol / 2, f32x2_to_bf16x2(xg, xn), epoch);
+                if (col == 0) dc_store(st + (o ? p.ssqa : p.ssqb) + (orow * (p.hidden / DC_TILE) + tile0) * DC_APART, __float_as_uint(sq), epoch);
+                dc_store(st + (o ? p.xa : p.xb) + (size_t)orow * p.hidden + ocol, __float_as_uint(r), epoch);
+            }
+        }
+    }
+}
+
+// One (token, kv head, split of its pages): the query heads of the kv head from the projection, the cached keys, and in the
+// block whose split holds the last page the step's own key and value, which it also appends.  Pages split, split + splits, ...;
+// a piece is 32 keys, the waves take pieces in turn, and a wave's first piece is asked for before the projection is waited for.
+__device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly, const DcItem& it, DcLds& sm, const DcTickets& tickets, int turn,
+                                             int wave, int lane) {
+    constexpr int D = DC_D, KD = D / 32, DT = D / 16, ROWS = (DC_MAX_GROUP + 2 + DC_WAVES - 1) / DC_WAVES;
+    const DcPlan& p = a.p;
+    u64* st = a.state;
+    const uint32_t epoch = it.epoch;
+    const int g = lane >> 4, col = lane & 15;
+    const int split = it.i % p.splits, kvh = it.i / p.splits % p.hkv, t = it.i / (p.splits * p.hkv);
+    const int group = p.hq / p.hkv;
+    const int* pages = a.block_table + (size_t)t * a.bt_width;
+    const int new_pos = a.pos[t], len = new_pos + 1;
+    const int n_pages = (len + AM_PAGE - 1) / AM_PAGE;
+    const int my_pages = split < n_pages ? (n_pages - split + p.splits - 1) / p.splits : 0;
+    const int n_pieces = my_pages * 2;
+    uint4 kbuf[2][KD], vbuf[DT];
+    auto request_keys = [&](int piece) {
+        int phys = pages[split + (piece >> 1) * p.splits];
+        const bf16_t* base = ly.k + (((size_t)phys * p.hkv + kvh) * AM_PAGE + (piece & 1) * 32) * D;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd)
+                kbuf[u][kd] = *(const uint4*)(base + (uint32_t)((8 * (col >> 2) + 4 * u + (col & 3)) * D + g * 8 + kd * 32));
+    };
+    auto request_values = [&](int piece) {
+        int phys = pages[split + (piece >> 1) * p.splits];
+        const bf16_t* base = ly.v + ((size_t)phys * p.hkv + kvh) * D * AM_PAGE + (piece & 1) * 32;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) vbuf[dt] = *(const uint4*)(base + (uint32_t)((dt * 16 + col) * AM_PAGE + g * 8));
+    };
+    if (wave < n_pieces) {
+        request_keys(wave);
+        request_values(wave);
+    }
+    const bool owner = new_pos / AM_PAGE % p.splits == split;
+    const int phys = pages[new_pos / AM_PAGE];
+    const int n_rows = group + (owner ? 2 : 0);
+    const float cs = a.cos_t[t * (D / 2) + lane], si = a.sin_t[t * (D / 2) + lane];
+    const float gq0 = ly.q_gain[lane], gq1 = ly.q_gain[lane + 64], gk0 = ly.k_gain[lane], gk1 = ly.k_gain[lane + 64];
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    float row_scale = 1.0f;
+    if (it.layer > 0) {
+        if (wave == 0) dc_far_wait(st, st + p.xgb + it.i * DC_LINE % (p.hidden / 2), epoch - 1);
+        __syncthreads();
+        row_scale = dc_row_scale(st, st + p.ssqb + t * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch - 1, a.inv_width, a.eps_mix, lane);
+    }
+    u64 drawn = 0;
+    if (wave == DC_WAVES - 1 && lane == 0) drawn = tickets.draw();
+    // a wave's rows of the projection together: a lane has the values lane and lane + 64 of each
+    {
+        const u64* tok = st + p.y + (size_t)t * p.n_qkv;
+        auto from = [&](int r) { return tok + (size_t)(r < group ? kvh * group + r : r == group ? p.hq + kvh : p.hq + p.hkv + kvh) * D; };
+        uint32_t raw[2 * ROWS];
+        dc_collect<2 * ROWS>(st, epoch, true, lane * 8u, [&](int i, uint32_t o) {
+            return dc_at(from(min(wave + i / 2 * DC_WAVES, n_rows - 1)) + (i & 1) * 64, o); }, raw);
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            int r = wave + DC_WAVES * i;
+            if (r >= n_rows) break;
+            float v0 = __uint_as_float(raw[2 * i]) * row_scale, v1 = __uint_as_float(raw[2 * i + 1]) * row_scale;
+            if (r <= group) {
+                float inv = 1.0f / sqrtf(wave_sum(fmaf(v1, v1, v0 * v0)) / (float)D + a.qk_eps);
+                v0 = v0 * inv * (r < group ? gq0 : gk0);
+                v1 = v1 * inv * (r < group ? gq1 : gk1);
+                // pairs (e, e + 64) are one lane's
+                float lo = v0 * cs - v1 * si, hi = v0 * si + v1 * cs;
+                v0 = lo;
+                v1 = hi;
+            }
+            bf16_t b0 = f32_to_bf16(v0), b1 = f32_to_bf16(v1);
+            bf16_t* dst = r < group ? sm.q[r] : r == group ? sm.k : sm.v;
+            dst[lane] = b0;
+            dst[lane + 64] = b1;
+            if (phys >= 0 && r >= group) {
+                const size_t head = (size_t)phys * p.hkv + kvh;
+                const int at = new_pos % AM_PAGE;
+                if (r == group) {
+                    ly.k[(head * AM_PAGE + at) * D + lane] = b0;
+                    ly.k[(head * AM_PAGE + at) * D + lane + 64] = b1;
+                } else {
+                    ly.v[(head * D + lane) * AM_PAGE + at] = b0;
+                    ly.v[(head * D + lane + 64) * AM_PAGE + at] = b1;
+                }
+            }
+        }
+    }
+    if (wave == DC_WAVES - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
+    __syncthreads();
+    // Q^T operand: column = head of the group (zero beyond it); read for every piece, registers are scarcer than LDS reads
+    auto query = [&](int kd) {
+        uint4 v = *(const uint4*)(&sm.q[col < group ? col : 0][kd * 32 + g * 8]);
+        bool ok = col < group;
+        v.x = ok ? v.x : 0u; v.y = ok ? v.y : 0u; v.z = ok ? v.z : 0u; v.w = ok ? v.w : 0u;
+        return __builtin_bit_cast(bf16x8_t, v);
+    };
+    float m = -INFINITY, l = 0.f;
+    f32x4_t o[DT];
+#pragma unroll
+    for (int i = 0; i < DT; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto scores = [&](int key0, int to, f32x4_t (&s)[2]) {
+        // element i of s[u] is key 8g + 4u + i, column = head
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            s[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd)
+                s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kbuf[u][kd]), query(kd), s[u], 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[u][i] = key0 + g * 8 + u * 4 + i < to ? s[u][i] * a.scale_log2e : -INFINITY;
+    };
+    auto add_values = [&](f32x4_t (&s)[2]) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[u][i]);
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        float m_new = fmaxf(m, mx);
+        float m_use = m_new == -INFINITY ? 0.f : m_new;
+        float corr = fast_exp2(m - m_use), sum = 0.f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[u][i] = fast_exp2(s[u][i] - m_use);
+                sum += s[u][i];
+            }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        l = l * corr + sum;
+        m = m_new;
+        uint4 pv = make_uint4(pack_bf16x2(s[0][0], s[0][1]), pack_bf16x2(s[0][2], s[0][3]),
+                              pack_bf16x2(s[1][0], s[1][1]), pack_bf16x2(s[1][2], s[1][3]));
+        bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pv);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            o[dt] = o[dt] * corr;
+            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vbuf[dt]), pf, o[dt], 0, 0, 0);
+        }
+    };
+    // (the step's own key is not yet in the cache where a block reads it; it comes last, from LDS)
+    const int cached = owner ? new_pos : len;
+    for (int piece = wave; piece < n_pieces; piece += DC_WAVES) {
+        f32x4_t s[2];
+        if (piece != wave) {
+            request_keys(piece);
+            request_values(piece);
+        }
+        scores((split + (piece >> 1) * p.splits) * AM_PAGE + (piece & 1) * 32, cached, s);
+        add_values(s);
+    }
+    asm volatile("" ::: "memory");
+    if (owner && wave == n_pieces % DC_WAVES) {
+        bool krow = col == 0, vrow = g == 0;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd) {
+                uint4 v = *(const uint4*)(sm.k + kd * 32 + g * 8);
+                bool take = krow && u == 0;
+                kbuf[u][kd] = make_uint4(take ? v.x : 0u, take ? v.y : 0u, take ? v.z : 0u, take ? v.w : 0u);
+            }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) vbuf[dt] = make_uint4(vrow ? (uint32_t)sm.v[dt * 16 + col] : 0u, 0u, 0u, 0u);
+        f32x4_t s[2];
+        scores(new_pos, new_pos + 1, s);
+        add_values(s);
+    }
+    // the waves' results in wave order; element i of o[dt] is d = 16 dt + 4g + i, column = head
+    if (col < group) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sm.o[wave][col][dt * 16 + g * 4 + i] = o[dt][i];
+    }
+    if (g == 0) {
+        sm.m[wave][col] = m;
+        sm.l[wave][col] = l;
+    }
+    __syncthreads();
+    for (int head = wave; head < group; head += DC_WAVES) {
+        const int d = lane * 2;
+        float mm = sm.m[0][head];
+#pragma unroll
+        for (int w = 1; w < DC_WAVES; ++w) mm = fmaxf(mm, sm.m[w][head]);
+        float ll = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll
+        for (int w = 0; w < DC_WAVES; ++w) {
+            float wgt = sm.m[w][head] == -INFINITY ? 0.f : fast_exp2(sm.m[w][head] - mm);
+            ll += sm.l[w][head] * wgt;
+            o0 += sm.o[w][head][d] * wgt;
+            o1 += sm.o[w][head][d + 1] * wgt;
+        }
+        int row = t * p.hq + kvh * group + head;
+        if (p.splits == 1) {
+            dc_store(st + p.o + (size_t)row * (D / 2) + lane, f32x2_to_bf16x2(o0 / ll, o1 / ll), epoch);
+        } else {
+            size_t slot = (size_t)row * p.splits + split;
+            dc_store(st + p.part + slot * D + d, __float_as_uint(o0), epoch);
+            dc_store(st + p.part + slot * D + d + 1, __float_as_uint(o1), epoch);
+            if (lane == 0) {
+                dc_store(st + p.part_ml + slot * 2, __float_as_uint(mm), epoch);
+                dc_store(st + p.part_ml + slot * 2 + 1, __float_as_uint(ll), epoch);
+            }
+        }
+    }
+    __syncthreads();                            // (the LDS is the next item's)
+}
+
+// The splits of one (token, query head) by log-sum-exp in split order, a quarter of them a wave.
+__device__ __forceinline__ void dc_merge(const DcArgs& a, const DcItem& it, DcLds& sm, const DcTickets& tickets, int turn, int wave, int lane) {
+    constexpr int D = DC_D;
+    const DcPlan& p = a.p;
+    u64* st = a.state;
+    const uint32_t epoch = it.epoch;
+    const int row = it.i;
+    if (wave == 0) dc_far_wait(st, st + p.y + row * DC_LINE % p.n_qkv, epoch);
+    __syncthreads();
+    u64 drawn = 0;
+    if (wave == DC_WAVES - 1 && lane == 0) drawn = tickets.draw();
+    const u64* ml = st + p.part_ml + (size_t)row * p.splits * 2;
+    bool mine = lane < p.splits;
+    uint32_t v[2];
+    dc_collect<2>(st, epoch, mine, mine ? lane * 16u : 0u, [&](int i, uint32_t o) { return dc_at(ml + i, o); }, v);
+    float ms = mine ? __uint_as_float(v[0]) : -INFINITY, ls = mine ? __uint_as_float(v[1]) : 0.f;
+    float mm = wave_max(ms);
+    float wgt = ms == -INFINITY ? 0.f : fast_exp2(ms - mm);
+    float inv_l = 1.0f / wave_sum(ls * wgt);    // every wave computes the same sum
+    const int quarter = (p.splits + DC_WAVES - 1) / DC_WAVES, s1 = min(p.splits, (wave + 1) * quarter);
+    float o0 = 0.f, o1 = 0.f;
+    for (int s0 = wave * quarter; s0 < s1; s0 += 4) {
+        uint32_t q[8];
+        dc_collect<8>(st, epoch, true, lane * 8u, [&](int i, uint32_t o) {
+            return dc_at(st + p.part + ((size_t)row * p.splits + min(s0 + i / 2, s1 - 1)) * D + (i & 1) * 64, o); }, q);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float ws = s0 + i < s1 ? __shfl(wgt, s0 + i, 64) : 0.f;
+            o0 += __uint_as_float(q[2 * i]) * ws;
+            o1 += __uint_as_float(q[2 * i + 1]) * ws;
+        }
+    }
+    sm.o[wave][0][lane] = o0;
+    sm.o[wave][0][lane + 64] = o1;
+    if (wave == DC_WAVES - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
+    __syncthreads();
+    if (wave == 0) {
+        float r[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int d = lane * 2 + j;
+            float sum = sm.o[0][0][d];
+#pragma unroll
+            for (int i = 1; i < DC_WAVES; ++i) sum += sm.o[i][0][d];
+            r[j] = sum * inv_l;
+        }
+        dc_store(st + p.o + (size_t)row * (D / 2) + lane, f32x2_to_bf16x2(r[0], r[1]), epoch);
+    }
+    __syncthreads();                            // (the LDS is the next item's)
+}
+
+template <int M>
+__global__ void __launch_bounds__(DC_THREADS) decode_chain_kernel(const DcArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char dc_lds[];
+    DcLds& sm = *(DcLds*)dc_lds;
+    const DcPlan& p = a.p;
+    const uint32_t total = (uint32_t)p.per_layer * p.n_layers, shard = blockIdx.x % DC_SHARDS;
+    // items shard, shard + DC_SHARDS, ...; every block of the counter draws one ticket behind them
+    const DcTickets tickets = {a.state + shard * DC_LINE, (total - shard + DC_SHARDS - 1) / DC_SHARDS + gridDim.x / DC_SHARDS - 1};
+    if (threadIdx.x == 0) tickets.drawn(tickets.draw(), sm.next);
+    __syncthreads();
+    for (int turn = 0;; turn ^= 1) {
+        const u64 drawn = sm.next[turn];
+        const uint32_t item = __builtin_amdgcn_readfirstlane((int)((uint32_t)drawn * DC_SHARDS + shard));
+        const uint32_t launch = __builtin_amdgcn_readfirstlane((int)(uint32_t)(drawn >> 32));
+        if (item >= total) break;
+        DcItem it;
+        it.layer = item / p.per_layer;
+        it.i = item - it.layer * p.per_layer;
+        it.stage = 0;
+#pragma unroll
+        for (int s = 0; s < 5; ++s)
+            if (it.stage == s && it.i >= p.items[s]) {
+                it.i -= p.items[s];
+                it.stage = s + 1;
+            }
+        // (numbers start at 2: the state starts as zeros, and a layer reads what the one before it numbered)
+        it.epoch = launch * (uint32_t)DC_LAYERS + (uint32_t)it.layer + 2u;
+        const DcLayer& ly = a.layer[it.layer];
+        // (told to be new in every turn: what the stages derive from it is not kept in registers beside the weights)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        if (it.stage == DC_ATTN) dc_attention(a, ly, it, sm, tickets, turn, wave, lane);
+        else if (it.stage == DC_MERGE) dc_merge(a, it, sm, tickets, turn, wave, lane);
+        else if (dc_tiles(p, it.stage) * dc_k(p, it.stage) <= DC_SHORT * DC_GROUP * 32 * DC_WAVES)
+            dc_product<M, true>(a, ly, it, sm, tickets, turn, wave, lane);
+        else dc_product<M, false>(a, ly, it, sm, tickets, turn, wave, lane);
+    }
+}
+
+// Whether a layer's sizes fit, and the plan of buffers and blocks (words of 64 bits).
+static bool dc_plan(DcPlan& p, int rows, int hidden, int hq, int hkv, int head_dim, int inter, int n_layers, int splits) {
+    if (rows < 1 || rows > DC_MAX_ROWS || head_dim != DC_D || hkv < 1 || hq < hkv || hq % hkv != 0 || hq / hkv > DC_MAX_GROUP) return false;
+    if (n_layers < 1 || n_layers > DC_LAYERS || splits < 1 || splits > 64) return false;
+    // a wave's quarter of K in whole groups of steps; strips of 16 weight rows whose offsets fit 31 bits
+    const int unit = 32 * DC_GROUP * DC_WAVES;
+    if (hidden < unit || inter < unit || hidden % unit != 0 || inter % unit != 0 || hq * (long long)DC_D % unit != 0) return false;
+    if (hidden > (1 << 20) || inter > (1 << 20) || hq > (1 << 13)) return false;
+    p.rows = rows; p.hidden = hidden; p.hq = hq; p.hkv = hkv; p.inter = inter; p.n_layers = n_layers; p.splits = splits;
+    p.n_qkv = (hq + 2 * hkv) * DC_D;
+    // short K: several tiles an item, as many as a wave's ring of weights holds (0.6B: 392 items a layer instead of 776)
+    auto tiles = [&](int n_tiles) {
+        const int groups = hidden / unit;
+        for (int t = DC_MAX_TILES; t > 1; --t)
+            if (t * groups <= DC_SHORT && n_tiles % t == 0) return t;
+        return 1;
+    };
+    p.qkv_tiles = tiles(p.n_qkv / DC_TILE);
+    p.gu_tiles = tiles(2 * inter / DC_TILE);
+    p.items[DC_QKV] = p.n_qkv / DC_TILE / p.qkv_tiles;
+    p.items[DC_ATTN] = rows * hkv * splits;
+    p.items[DC_MERGE] = splits > 1 ? rows * hq : 0;
+    p.items[DC_O] = hidden / DC_TILE;
+    p.items[DC_GU] = 2 * inter / DC_TILE / p.gu_tiles;
+    p.items[DC_DOWN] = hidden / DC_TILE;
+    p.per_layer = 0;
+    for (int s = 0; s < 6; ++s) p.per_layer += p.items[s];
+    int at = (DC_SHARDS + 1) * DC_LINE;
+    auto take = [&](long long words) { int here = at; at += (int)((words + 15) / 16 * 16); return here; };
+    p.y = take((long long)rows * p.n_qkv);
+    p.part = take(splits > 1 ? (long long)rows * hq * splits * DC_D : 0);
+    p.part_ml = take(splits > 1 ? (long long)rows * hq * splits * 2 : 0);
+    p.o = take((long long)rows * hq * DC_D / 2);
+    p.xa = take((long long)rows * hidden); p.xb = take((long long)rows * hidden);
+    p.xga = take((long long)rows * hidden / 2); p.xgb = take((long long)rows * hidden / 2);
+    p.ssqa = take((long long)rows * hidden / DC_TILE * DC_APART); p.ssqb = take((long long)rows * hidden / DC_TILE * DC_APART);
+    p.h = take((long long)rows * inter / 2);
+    p.words = at;
+    const int most_k = inter > hidden ? (inter > hq * DC_D ? inter : hq * DC_D) : (hidden > hq * DC_D ? hidden : hq * DC_D);
+    const long long product = (long long)rows * (most_k * 2LL + DC_PAD);
+    const long long lds = sizeof(DcLds) + product;
+    if (lds > DC_MAX_LDS) return false;
+    p.lds = (int)lds;
+    return true;
+}
+
+// Whether the chain is faster than the layers' own kernels: a matter of how long the weights' bytes take beside the stages'
+// latencies, and of how many words travel.  A layer of 31 MB of weights (Qwen3-0.6B) from one to four rows, above.  100 MB
+// (1.7B, 8 layers, to the logits): one row 536 -> 490 us, two 540 -> 546, four 580 -> 652.  202 MB (4B, 6 layers): one row 638 ->
+// 624 to 678; 386 MB (8B, 8 layers) 1,022 -> 1,154: while weights stream, a word's way takes several us.
+ROCML_EXPORT int rocml_decode_chain_pays(int rows, int hidden, int hq, int hkv, int head_dim, int inter) {
+    DcPlan p;
+    if (!dc_plan(p, rows, hidden, hq, hkv, head_dim, inter, 1, 1)) return 0;
+    const double mb = 2e-6 * hidden * ((double)p.n_qkv + (double)hq * DC_D + 3.0 * inter);
+    return mb <= (rows == 1 ? 128.0 : 64.0);
+}
+
+// 64-bit words of state that a chain of such layers needs; 0: not taken.
+ROCML_EXPORT int rocml_decode_chain_words(int rows, int hidden, int hq, int hkv, int head_dim, int inter, int n_layers, int splits) {
+    DcPlan p;
+    return dc_plan(p, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits) ? p.words : 0;
+}
+
+ROCML_EXPORT int rocml_decode_chain_max_layers() { return DC_LAYERS; }
+
+// layers: per layer the ten pointers of DcLayer.
+ROCML_EXPORT int rocml_decode_chain(void* state, long long state_words, float* x, const void* xn, const void* const* layers, int n_layers,
+                                    int rows, int hidden, int hq, int hkv, int head_dim, int inter, const int* block_table, int bt_width,
+                                    const int* token_pos, const float* cos_t, const float* sin_t, float scale, float qk_eps, float eps_mix,
+                                    float eps_ffn, int splits, hipStream_t stream) {
+    DcArgs a;
+    ROCML_REQUIRE(dc_plan(a.p, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits),
+                  "decode_chain: sizes not taken: rows=%d hidden=%d heads=%d/%d of %d inter=%d layers=%d splits=%d", rows, hidden, hq, hkv,
+                  head_dim, inter, n_layers, splits);
+    ROCML_REQUIRE(state && state_words >= a.p.words, "decode_chain: the state has %lld of %d words", state_words, a.p.words);
+    ROCML_REQUIRE(x && xn && layers && block_table && token_pos && cos_t && sin_t && bt_width > 0, "decode_chain: missing operand");
+    a.state = (u64*)state;
+    a.x = x; a.xn = (const bf16_t*)xn; a.block_table = block_table; a.bt_width = bt_width; a.pos = token_pos;
+    a.cos_t = cos_t; a.sin_t = sin_t;
+    a.scale_log2e = scale * AM_LOG2E; a.qk_eps = qk_eps; a.eps_mix = eps_mix; a.eps_ffn = eps_ffn; a.inv_width = 1.0f / (float)hidden;
+    for (int i = 0; i < n_layers; ++i) {
+        const void* const* f = layers + 10 * i;
+        for (int j = 0; j < 10; ++j) ROCML_REQUIRE(f[j] || (j == 7 && i == n_layers - 1), "decode_chain: layer %d lacks operand %d", i, j);
+        a.layer[i] = DcLayer{(const bf16_t*)f[0], (const bf16_t*)f[1], (const bf16_t*)f[2], (const bf16_t*)f[3], (const float*)f[4],
+                             (const float*)f[5], (const float*)f[6], (const float*)f[7], (bf16_t*)f[8], (bf16_t*)f[9]};
+    }
+    // a block a CU; a whole number for every counter
+    const int blocks = ceil_div(cu_count(), DC_SHARDS) * DC_SHARDS;
+    const auto kernel = rows == 1 ? decode_chain_kernel<1> : rows == 2 ? decode_chain_kernel<2> : rows == 3 ? decode_chain_kernel<3>
+                                                                                                            : decode_chain_kernel<4>;
+    if (a.p.lds > (64 << 10))
+        ROCML_REQUIRE(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, DC_MAX_LDS) == hipSuccess,
+                      "decode_chain: %d bytes of LDS were refused", a.p.lds);
+    kernel<<<blocks, DC_THREADS, a.p.lds, stream>>>(a);
+    ROCML_CHECK_LAUNCH("decode_chain");
+    return 0;
+}

@@ -189,6 +189,25 @@ class DecoderModel:
         return Cache(self.cache_requests(), max_tokens, self.dtype, self.device, max_seqs=max_seqs,
                      free_bytes=free, step_tokens=step_tokens, headroom=headroom)
 
+    def _chains(self, step: StepContext, cache: Cache) -> Dict[int, list]:
+        """The runs of schedule entries that ``ops.decode_chain`` takes in this step, as ``{first entry: its layers}``."""
+        chains: Dict[int, list] = {}
+        if step.max_new != 1 or step.n_tokens > ops.CHAIN_MAX_ROWS or step.n_tokens != step.n_seqs:
+            return chains
+        run: list = []
+        for i, entry in enumerate(self.spec.schedule):
+            block, layer = self.blocks[entry.layer], None
+            if entry.reads_cache_of is None and entry.offset_row is None and not entry.add_embedding and hasattr(block, "chain_layer"):
+                layer = block.chain_layer(step, self.entry_view(i, cache, step))
+            if layer is None or not ops.decode_chain_pays(layer, step.n_tokens):
+                run = []
+                continue
+            if run and len(run) < ops.decode_chain_max_layers() and layer.fits_behind(run[0]):
+                run.append(layer)
+            else:
+                run = chains[i] = [layer]
+        return chains
+
     # -- forward -----------------------------------------------------------------------
     def forward(self, step: StepContext, cache: Cache, block_tables: Dict[str, torch.Tensor],
                 want_rows: Optional[torch.Tensor], n_want: int) -> Optional[torch.Tensor]:
@@ -205,7 +224,19 @@ class DecoderModel:
             # entries that add the embedding's output to the stream later need it kept
             x0 = ws.get("model.x0", (step.n_tokens, s.hidden), torch.float32)
             ops.weighted_sum(x0, [x], [1.0])
+        chains = self._chains(step, cache)
+        behind = 0                      # entries before this one have run as part of a chain
         for i, entry in enumerate(s.schedule):
+            if i < behind:
+                continue
+            if i in chains:
+                layers, position = chains[i], chains[i][0].position
+                xn = self.blocks[entry.layer].chain_input(step, x)
+                cos, sin = position.tables(step)
+                words = ops.decode_chain_words(layers[0], step.n_tokens, len(layers))
+                ops.decode_chain(x, xn, layers, step.token_pos, cos, sin, ws.kept("model.chain", words, torch.int64), max_len=step.max_len)
+                behind = i + len(layers)
+                continue
             view = self.entry_view(i, cache, step)
             block = self.blocks[entry.layer]
             if entry.offset_row is not None:
@@ -220,7 +251,7 @@ class DecoderModel:
             hint = None
             if following is not None and (s.schedule[i + 1].offset_row is not None or s.schedule[i + 1].add_embedding):
                 following = None      # the stream changes between the two blocks: nothing can be prepared across
-            if getattr(block, "takes_next_norm", False) and hasattr(following, "entry_hint"):
+            if getattr(block, "takes_next_norm", False) and hasattr(following, "entry_hint") and i + 1 not in chains:
                 hint = following.entry_hint(step)
             if hint is not None:
                 block.forward(step, x, view, entry.reads_cache_of is None, next_norm=hint)

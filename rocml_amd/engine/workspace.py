@@ -46,6 +46,17 @@ class Workspace:
             self._views[(name, dtype, shape)] = view
         return view
 
+    def kept(self, name: str, n: int, dtype: torch.dtype) -> torch.Tensor:
+        """At least ``n`` numbers that start as zeros and keep what kernels leave in them from step to step (a buffer that
+        has to grow starts as zeros again)."""
+        key = f"kept.{name}/{dtype}"
+        buf = self._buffers.get(key)
+        if buf is None or buf.numel() < n:
+            buf = torch.zeros(n, dtype=dtype, device=self.device)
+            self._buffers[key] = buf
+            self.generation += 1
+        return buf
+
     def scratch(self) -> torch.Tensor:
         """Device memory kernels may use for partial results of one launch.  Partial sums
         that a deferred product left there are added to their target first."""

@@ -87,6 +87,10 @@ _SIGNATURES = {
                             _P, _I, _I, _P, _I, _I, _P, _LL, _I, _I, _I, _P, _I, _P, _F, _I, _P],
         "rocml_attention_decode_fused": [_P, _I, _I, _LL, _P, _P, _F, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P,
                                          _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _LL, _P, _I, _F, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
+        "rocml_decode_chain_pays": [_I, _I, _I, _I, _I, _I],
+        "rocml_decode_chain_words": [_I, _I, _I, _I, _I, _I, _I, _I],
+        "rocml_decode_chain_max_layers": [],
+        "rocml_decode_chain": [_P, _LL, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _F, _F, _F, _F, _I, _P],
         "rocml_attention_prefill_fused": [_P, _I, _P, _F, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _I,
                                           _P, _I, _P, _P],
     },
@@ -1164,6 +1168,113 @@ def attention_decode_fused(qkv: torch.Tensor, out: torch.Tensor, k_cache: torch.
 
 
 # ---- sampling ------------------------------------------------------------------------
+CHAIN_HEAD_DIM = 128        # the head size of a layer that decode_chain takes
+CHAIN_MAX_ROWS = 4          # most sequences of a step
+CHAIN_PAGE = 64             # positions of a cache page
+CHAIN_POINTERS = 10         # operands of a layer, in the order of ``ChainLayer.pointers``
+
+
+class ChainLayer:
+    """A layer as ``decode_chain`` runs it: ``x += o(attention(q, k, v of norm(x)))``, ``x += down(silu(gate) up of norm(x))``
+    with per-head norms and a rotation of whole heads on q and k.  The matrices, gains and cache of one layer."""
+
+    def __init__(self, w_qkv, w_o, w_gate_up, w_down, q_gain, k_gain, mix_gain, ffn_gain, k_cache, v_cache, block_table,
+                 n_heads: int, n_kv_heads: int, scale: float, qk_eps: float, mix_eps: float, ffn_eps: float, position):
+        self.w_qkv, self.w_o, self.w_gate_up, self.w_down = w_qkv, w_o, w_gate_up, w_down
+        self.q_gain, self.k_gain, self.mix_gain, self.ffn_gain = q_gain, k_gain, mix_gain, ffn_gain
+        self.k_cache, self.v_cache, self.block_table = k_cache, v_cache, block_table
+        self.n_heads, self.n_kv_heads = n_heads, n_kv_heads
+        self.scale, self.qk_eps, self.mix_eps, self.ffn_eps = scale, qk_eps, mix_eps, ffn_eps
+        self.position = position        # the part whose tables rotate q and k (equal specs share a step's tables)
+
+    @property
+    def hidden(self) -> int:
+        return self.w_qkv.shape[1]
+
+    @property
+    def inter(self) -> int:
+        return self.w_down.shape[1]
+
+    def fits_behind(self, other: "ChainLayer") -> bool:
+        """Whether this layer may follow ``other`` in one launch: the sizes, constants and tables of both are the same."""
+        return (self.hidden == other.hidden and self.inter == other.inter and self.n_heads == other.n_heads
+                and self.n_kv_heads == other.n_kv_heads and self.scale == other.scale and self.qk_eps == other.qk_eps
+                and self.mix_eps == other.mix_eps and self.ffn_eps == other.ffn_eps and self.position.spec == other.position.spec
+                and self.block_table.data_ptr() == other.block_table.data_ptr() and self.block_table.shape == other.block_table.shape)
+
+
+def decode_chain_max_layers() -> int:
+    return library("attention").rocml_decode_chain_max_layers()
+
+
+def decode_chain_splits(pages: int) -> int:
+    """Splits of the key range in ``decode_chain`` for a block table of ``pages`` pages: a block asks for two pages before it
+    waits for anything.  It depends on the step's shape only, so a recorded step can be replayed as the sequences grow."""
+    return 1 if pages <= 4 else min(64, (pages + 1) // 2)
+
+
+def decode_chain_pays(layer: ChainLayer, rows: int) -> bool:
+    """Whether the library's own rule says that ``decode_chain`` is the faster way for such layers and so many sequences."""
+    return bool(library("attention").rocml_decode_chain_pays(rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter))
+
+
+def decode_chain_words(layer: ChainLayer, rows: int, n_layers: int) -> int:
+    """64-bit words of state a chain of ``n_layers`` such layers needs for ``rows`` tokens (one per sequence); 0: not taken."""
+    return library("attention").rocml_decode_chain_words(
+        rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter, n_layers,
+        decode_chain_splits(layer.block_table.shape[1]))
+
+
+def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer], token_pos: torch.Tensor, cos: torch.Tensor,
+                 sin: torch.Tensor, state: torch.Tensor, max_len: int = 0) -> None:
+    """The layers of a decode step, one token per sequence, in one launch: ``x [rows, hidden]`` (32-bit) passes through them,
+    the new keys and values are appended.  ``xn``: the first layer's normed input in bfloat16.  ``state`` (int64) starts as
+    zeros and is the caller's to keep from call to call; launches that share it run one after the other.  ``max_len`` is what
+    ``--profile`` prices the call with."""
+    first = layers[0]
+    rows, hidden = x.shape
+    _dev(x, xn, token_pos, cos, sin, state, first.block_table)
+    _want(x, torch.float32, "residual stream")
+    _want(xn, torch.bfloat16, "normed operand")
+    _want(state, torch.int64, "state")
+    _want(token_pos, torch.int32, "positions")
+    _want(first.block_table, torch.int32, "block table")
+    n_qkv = (first.n_heads + 2 * first.n_kv_heads) * CHAIN_HEAD_DIM
+    if hidden != first.hidden or xn.shape != x.shape or token_pos.numel() != rows or first.block_table.shape[0] != rows:
+        raise KernelError(f"decode chain: {rows} rows of {hidden} do not fit the operands")
+    for t in (cos, sin):
+        _want(t, torch.float32, "rotation table")
+        if t.shape != (rows, CHAIN_HEAD_DIM // 2):
+            raise KernelError(f"rotation tables must be float32 {(rows, CHAIN_HEAD_DIM // 2)}")
+    pointers = (ctypes.c_void_p * (CHAIN_POINTERS * len(layers)))()
+    for i, c in enumerate(layers):
+        if not c.fits_behind(first):
+            raise KernelError("the layers of a decode chain must agree in sizes, constants and tables")
+        for w, shape in ((c.w_qkv, (n_qkv, hidden)), (c.w_o, (hidden, c.n_heads * CHAIN_HEAD_DIM)),
+                         (c.w_gate_up, (2 * c.inter, hidden)), (c.w_down, (hidden, c.inter))):
+            _want(w, torch.bfloat16, "weight")
+            if tuple(w.shape) != shape:
+                raise KernelError(f"decode chain: a weight is {tuple(w.shape)}, not {shape}")
+        for gain, n in ((c.q_gain, CHAIN_HEAD_DIM), (c.k_gain, CHAIN_HEAD_DIM), (c.mix_gain, hidden), (c.ffn_gain, hidden)):
+            _want(gain, torch.float32, "gain")
+            if gain.numel() != n:
+                raise KernelError(f"decode chain: a gain has {gain.numel()} values, not {n}")
+        pages = (c.k_cache.shape[0], c.n_kv_heads)
+        for t, shape in ((c.k_cache, pages + (CHAIN_PAGE, CHAIN_HEAD_DIM)), (c.v_cache, pages + (CHAIN_HEAD_DIM, CHAIN_PAGE))):
+            _want(t, torch.bfloat16, "cache")
+            if tuple(t.shape) != shape:
+                raise KernelError(f"decode chain: a cache is {tuple(t.shape)}, not {shape}")
+        following = layers[i + 1].mix_gain if i + 1 < len(layers) else None
+        operands = (c.w_qkv, c.w_o, c.w_gate_up, c.w_down, c.q_gain, c.k_gain, c.ffn_gain, following, c.k_cache, c.v_cache)
+        _dev(*operands)
+        for j, t in enumerate(operands):
+            pointers[CHAIN_POINTERS * i + j] = _ptr(t)
+    _check("attention", library("attention").rocml_decode_chain(
+        _ptr(state), state.numel(), _ptr(x), _ptr(xn), pointers, len(layers), rows, hidden, first.n_heads, first.n_kv_heads,
+        CHAIN_HEAD_DIM, first.inter, _ptr(first.block_table), first.block_table.shape[1], _ptr(token_pos), _ptr(cos), _ptr(sin),
+        first.scale, first.qk_eps, first.mix_eps, first.ffn_eps, decode_chain_splits(first.block_table.shape[1]), _stream()))
+
+
 ARGMAX_WORK_WORDS = 64      # 32-bit words of workspace per row for the two-stage argmax
 SAMPLE_SMALL_K = 64         # the largest top-k that the slice kernels of the sampler take
 

@@ -239,6 +239,20 @@ class Attention(Mixer):
             return 0
         return ops.decode_splits(step.n_tokens * self.spec.n_kv_heads, self.n_cus, min(cache.block_table.shape[1], 64))
 
+    def chain_operands(self, step, cache) -> Optional[dict]:
+        """What ``ops.decode_chain`` needs of this attention, or None where the layer or the step is not one it takes: one token
+        per sequence, bfloat16, heads of 128 with norms of their own and a rotation of the whole head, every key seen."""
+        s = self.spec
+        if (not self._fused_decode(step) or self.extras or s.bias or self.o_bias or s.window is not None or s.qk_norm is None
+                or s.head_dim != ops.CHAIN_HEAD_DIM or self.position is None or self.position.rot_dim != s.head_dim
+                or getattr(cache, "parts", None) is not None or step.n_tokens != step.n_seqs):
+            return None
+        if cache.k.dtype != self.dtype or cache.k.shape[2] != ops.CHAIN_PAGE or self.w_qkv.shape[0] != self.q_dim + 2 * self.kv_dim:
+            return None
+        return {"w_qkv": self.w_qkv, "w_o": self.w_o, "q_gain": self.q_gain, "k_gain": self.k_gain, "k_cache": cache.k,
+                "v_cache": cache.v, "block_table": cache.block_table, "n_heads": s.n_heads, "n_kv_heads": s.n_kv_heads,
+                "scale": s.scale, "qk_eps": s.qk_norm.eps, "position": self.position}
+
     def input_weight(self) -> Optional[torch.Tensor]:
         # only the path of the norm-and-rotation kernel, which takes rows of any stride; and the
         # projection must start at the buffer's first column

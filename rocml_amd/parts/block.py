@@ -119,6 +119,24 @@ class PreNormBlock(ConvInput, Part):
             return None               # the convolution needs the normed rows themselves
         return self._hint(step, self.mixer_norm, self.mixer)
 
+    def chain_layer(self, step, cache):
+        """This layer as ``ops.decode_chain`` runs it in a step, or None if it or the step is not one the chain takes."""
+        parts = (self.mixer, self.ffn)
+        norms = [n.prescale_hint() if hasattr(n, "prescale_hint") else None for n in (self.mixer_norm, self.ffn_norm)]
+        if self.input_conv is not None or None in norms or not all(hasattr(part, "chain_operands") for part in parts):
+            return None
+        mixer, ffn = self.mixer.chain_operands(step, cache), self.ffn.chain_operands(step)
+        if mixer is None or ffn is None:
+            return None
+        return ops.ChainLayer(mix_gain=norms[0].gain, ffn_gain=norms[1].gain, mix_eps=norms[0].eps, ffn_eps=norms[1].eps, **mixer, **ffn)
+
+    def chain_input(self, step, x: torch.Tensor) -> torch.Tensor:
+        """The first norm's output, for a chain that starts with this layer; ``x`` is complete behind it."""
+        xn, scale = self._norm(step, self.mixer_norm, x)
+        if scale is not None:
+            raise ConfigError("a chain of layers was handed an input without its norm's scale")
+        return xn
+
     def forward(self, step, x: torch.Tensor, cache, owns_cache: bool, next_norm=None) -> None:
         """``next_norm``: the hint of the norm that reads ``x`` after this block (``entry_hint`` of
         the block that runs next), or None."""

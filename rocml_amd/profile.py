@@ -114,6 +114,14 @@ def _prefill_fused_cost(qkv, out, k_cache, v_cache, block_table, token_pos, n_he
     return read_q + _nbytes(out, cos, sin) + kv, 4 * n_heads * head_dim * n_tokens * keys_per_query
 
 
+def _chain_cost(x, xn, layers, *a, **kw) -> Tuple[int, int]:
+    rows, seen = x.shape[0], kw.get("max_len", 0)
+    weights = sum(_nbytes(c.w_qkv, c.w_o, c.w_gate_up, c.w_down) for c in layers)
+    kv = sum(2 * rows * seen * c.n_kv_heads * c.k_cache.shape[3] * c.k_cache.element_size() for c in layers)
+    flops = sum(4 * c.n_heads * c.k_cache.shape[3] * rows * seen for c in layers)
+    return weights + kv + 2 * _nbytes(x), rows * weights + flops
+
+
 def _tensor_args_cost(skip: Tuple[int, ...] = (), flops_per_byte: float = 0.0) -> Callable:
     def cost(*a, **kw) -> Tuple[int, int]:
         tensors = [t for i, t in enumerate(a) if i not in skip] + list(kw.values())
@@ -132,6 +140,7 @@ _COSTS: Dict[str, Tuple[str, Callable]] = {
                   or kw.get("softcap") is not None or kw.get("keep_first")
                   else "attention", _attention_cost),
     "attention_decode_fused": ("attention (norm, rotation, append)", _fused_attention_cost),
+    "decode_chain": ("layers of a decode step", _chain_cost),
     "attention_prefill_fused": ("attention (query norm, rotation)", _prefill_fused_cost),
     "qk_norm_rope_append": ("q/k norm, rotation, append", _tensor_args_cost(skip=(11, 12))),   # not the whole cache
     "rmsnorm": ("rmsnorm", _tensor_args_cost(flops_per_byte=0.5)),

@@ -1,0 +1,169 @@
+"""The layers of a decode step in one launch (``ops.decode_chain``) against the same layers in 64 bits written here: the
+smallest sizes it takes, one, several and all of a wave's weights asked for at once, odd positions around page edges, one and
+many splits of the keys, one to four sequences; the state kept over calls of other sizes, and a recorded launch replayed.
+
+Bound: the operands of every product, q, k, v and probabilities carry 8 bits (a rounding error of up to 2^-9, 0.0011 root mean
+square), and a layer's result passes about eight such roundings, 0.0032; two layers and what the second makes of the first's
+error stay below 0.01 in the 2-norm of what the layers added."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from rocml_amd import ops  # noqa: E402
+
+D, PAGE, EPS = 128, 64, 1e-6
+DEV = "cuda:0"
+
+
+class _Position:
+    spec = "the test's"
+
+
+def _model(hidden, hq, hkv, inter, n_layers, lens, width, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+
+    def rand(*shape, scale=1.0):
+        return torch.randn(*shape, generator=g, device=DEV) * scale
+    n_pages = sum((n + PAGE) // PAGE for n in lens) + 3
+    order = torch.randperm(n_pages, generator=torch.Generator().manual_seed(seed)).tolist()
+    table = torch.full((len(lens), width), -1, dtype=torch.int32)
+    for b, n in enumerate(lens):
+        for i in range(n // PAGE + 1):
+            table[b, i] = order.pop()
+    table = table.to(DEV)
+    layers = []
+    for _ in range(n_layers):
+        w = [rand(r, c, scale=c ** -0.5).bfloat16() for r, c in (((hq + 2 * hkv) * D, hidden), (hidden, hq * D), (2 * inter, hidden), (hidden, inter))]
+        gains = [1.0 + rand(n, scale=0.1) for n in (D, D, hidden, hidden)]
+        k, v = rand(n_pages, hkv, PAGE, D).bfloat16(), rand(n_pages, hkv, D, PAGE).bfloat16()
+        layers.append(ops.ChainLayer(*w, *gains, k, v, table, hq, hkv, D ** -0.5, EPS, EPS, EPS, _Position()))
+    x = rand(len(lens), hidden)
+    inv = 1e4 ** (-torch.arange(0, D, 2, device=DEV, dtype=torch.float64) / D)
+    angle = torch.tensor(lens, device=DEV, dtype=torch.float64)[:, None] * inv
+    return layers, x, angle.cos().float(), angle.sin().float(), torch.tensor(lens, dtype=torch.int32, device=DEV)
+
+
+def _rms(x, gain):
+    return x / torch.sqrt((x * x).mean(-1, keepdim=True) + EPS) * gain.double()
+
+
+def _plain(layers, x, cos, sin, lens):
+    """The layers in 64 bits; the stream and each layer's new keys and values."""
+    x, kept = x.double(), []
+    for c in layers:
+        hq, hkv, n = c.n_heads, c.n_kv_heads, x.shape[0]
+        y = (_rms(x, c.mix_gain) @ c.w_qkv.double().T).view(n, hq + 2 * hkv, D)
+        q, k, v = _rms(y[:, :hq], c.q_gain), _rms(y[:, hq:hq + hkv], c.k_gain), y[:, hq + hkv:]
+
+        def turn(z):
+            a, b, co, si = z[..., :D // 2], z[..., D // 2:], cos.double()[:, None], sin.double()[:, None]
+            return torch.cat([a * co - b * si, a * si + b * co], -1)
+        q, k = turn(q), turn(k)
+        kept.append((k, v))
+        o = torch.empty(n, hq, D, dtype=torch.float64, device=DEV)
+        for b, ln in enumerate(lens):
+            pages = c.block_table[b, :ln // PAGE + 1].long()
+            ks = c.k_cache[pages].double().permute(0, 2, 1, 3).reshape(-1, hkv, D)[:ln]
+            vs = c.v_cache[pages].double().permute(0, 3, 1, 2).reshape(-1, hkv, D)[:ln]
+            ks, vs = torch.cat([ks, k[b:b + 1]]), torch.cat([vs, v[b:b + 1]])
+            for h in range(hq):
+                p = torch.softmax(ks[:, h * hkv // hq] @ q[b, h] * c.scale, 0)
+                o[b, h] = p @ vs[:, h * hkv // hq]
+        x = x + o.reshape(n, -1) @ c.w_o.double().T
+        gu = _rms(x, c.ffn_gain) @ c.w_gate_up.double().T
+        gate, up = gu[:, 0::2], gu[:, 1::2]
+        x = x + (gate * torch.sigmoid(gate) * up) @ c.w_down.double().T
+    return x, kept
+
+
+def _run(layers, x, cos, sin, pos, state):
+    xn = torch.empty(x.shape, dtype=torch.bfloat16, device=DEV)
+    ops.rmsnorm(x, layers[0].mix_gain, EPS, xn)
+    ops.decode_chain(x, xn, layers, pos, cos, sin, state)
+
+
+def _check(layers, x0, x, cos, sin, lens):
+    want, kept = _plain(layers, x0, cos, sin, lens)
+    added = want - x0.double()
+    assert torch.isfinite(x).all()
+    assert float((x.double() - want).norm() / added.norm()) < 0.01
+    for c, (k, v) in zip(layers, kept):
+        for b, ln in enumerate(lens):
+            page, at = int(c.block_table[b, ln // PAGE]), ln % PAGE
+            assert float((c.k_cache[page, :, at].double() - k[b]).norm() / k[b].norm()) < 0.01
+            assert float((c.v_cache[page, :, :, at].double() - v[b]).norm() / v[b].norm()) < 0.01
+
+
+CASES = [
+    # hidden, query heads, kv heads, intermediate, layers, positions, pages a table has room for
+    (512, 4, 4, 512, 1, [0], 1),                            # the smallest: one group of steps a wave, no key but the step's own
+    (512, 8, 1, 1024, 2, [63, 64], 2),                      # a group of eight heads; the last row of a page and the first of the next
+    (1024, 16, 8, 3072, 2, [37], 1),                        # three tiles an item
+    (1024, 16, 8, 3072, 2, [255, 0, 128], 4),               # as many pages as one split takes
+    (1024, 16, 8, 3072, 2, [256, 700, 1, 1023], 16),        # several splits, some without a page
+    (1536, 12, 4, 2560, 2, [300], 5),                       # three groups of steps, an odd number of pages
+    (2048, 16, 8, 6144, 2, [1000, 65], 64),                 # longer than the ring of weights; a split a page and more
+    (2560, 32, 8, 9728, 1, [129], 4),
+    (1024, 16, 8, 3072, 2, [9000], 256),                    # the most splits, several pages each
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[f"{c[0]}-{c[1]}-{c[3]}-{c[5]}" for c in CASES])
+def test_layers_in_one_launch(case):
+    hidden, hq, hkv, inter, n_layers, lens, width = case
+    layers, x0, cos, sin, pos = _model(hidden, hq, hkv, inter, n_layers, lens, width, seed=hidden + len(lens))
+    words = ops.decode_chain_words(layers[0], len(lens), n_layers)
+    assert words > 0
+    state = torch.zeros(words, dtype=torch.int64, device=DEV)
+    x = x0.clone()
+    _run(layers, x, cos, sin, pos, state)
+    _check(layers, x0, x, cos, sin, lens)
+    # the state is as good for the next launch, and the sums do not depend on timing
+    for _ in range(3):
+        again = x0.clone()
+        _run(layers, again, cos, sin, pos, state)
+        assert torch.equal(again, x)
+
+
+def test_one_state_for_launches_of_other_sizes():
+    small = _model(1024, 16, 8, 3072, 2, [70], 2, seed=1)
+    large = _model(1024, 16, 8, 3072, 3, [90, 500], 16, seed=2)
+    state = torch.zeros(max(ops.decode_chain_words(m[0][0], m[1].shape[0], len(m[0])) for m in (small, large)), dtype=torch.int64, device=DEV)
+    for layers, x0, cos, sin, pos in (small, large, small, large):
+        x = x0.clone()
+        _run(layers, x, cos, sin, pos, state)
+        _check(layers, x0, x, cos, sin, pos.tolist())
+
+
+def test_recorded_launch_replayed_with_other_inputs():
+    layers, x0, cos, sin, pos = _model(1024, 16, 8, 3072, 2, [130, 77], 4, seed=3)
+    state = torch.zeros(ops.decode_chain_words(layers[0], 2, 2), dtype=torch.int64, device=DEV)
+    x = x0.clone()
+    _run(layers, x, cos, sin, pos, state)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        _run(layers, x, cos, sin, pos, state)
+    for i in range(4):
+        fresh = x0 * (1.0 + 0.25 * i)
+        x.copy_(fresh)
+        graph.replay()
+        got = x.clone()
+        eager = fresh.clone()
+        _run(layers, eager, cos, sin, pos, state)
+        torch.cuda.synchronize()
+        assert torch.equal(got, eager)
+
+
+def test_what_the_chain_does_not_take():
+    layers, x0, cos, sin, pos = _model(512, 4, 4, 512, 1, [5], 1, seed=4)
+    state = torch.zeros(ops.decode_chain_words(layers[0], 1, 1), dtype=torch.int64, device=DEV)
+    xn = x0.bfloat16()
+    with pytest.raises(ops.KernelError):                    # a state that is too short
+        ops.decode_chain(x0, xn, layers, pos, cos, sin, state[:-16])
+    with pytest.raises(ops.KernelError):                    # more rows than it knows
+        many = _model(512, 4, 4, 512, 1, [5] * 5, 1, seed=4)
+        ops.decode_chain(many[1], many[1].bfloat16(), many[0], many[4], many[2], many[3], state)
+    assert ops.decode_chain_words(layers[0], 5, 1) == 0
+    odd = _model(768, 6, 2, 768, 1, [5], 1, seed=4)[0][0]    # no whole groups of steps in a wave's share of K
+    assert ops.decode_chain_words(odd, 1, 1) == 0 and not ops.decode_chain_pays(odd, 1)
