@@ -1,4 +1,4 @@
-// A decode step's layers in one launch (gfx950, wave64, bfloat16): q/k/v projection, attention over the paged cache, output
+// A decode step's layers in one launch (gfx950, wave64, bfloat16 and 32-bit): q/k/v projection, attention over the paged cache, output
 // projection, gated feed-forward, layer after layer, for one to four sequences of a model with small layers.
 //
 // What bounds it, and why it is one launch.  With a few rows of activations every product is a walk over its weights, and a
@@ -12,7 +12,7 @@
 // What is left of a layer (14.5 us) is five times a result's way to the next stage, each with a trip to memory behind its store.
 //
 // Measured on the way: two and three blocks a CU instead of one, 657 and 678 us against 558 (more weights ahead, but what asks
-// for operands is in the way of what answers); eight waves a block 648 against 548 (1.7B: 455 against 500); a wave of its own for
+// for operands is in the way of what answers); eight waves a block 648 against 548 (but see dc_plan); a wave of its own for
 // operands and results 994; a counter of flags beside plain data instead of words that carry their number 4.2 us from stage to
 // stage against 2.1; one counter of tickets for all 30 ns a ticket, 24 us a layer.
 //
@@ -28,16 +28,16 @@
 // wait last for seconds all the same, it ends, and the step's result is NaN.
 //
 // The algebra is that of the kernels the step otherwise runs (gemm_kpar_kernel, gemm_residual_prescale_kernel,
-// attn_decode_mfma_kernel FUSED): 32-bit sums on mfma_f32_16x16x32_bf16, the residual stream in 32 bits, the norm's scale
+// attn_decode_mfma_kernel FUSED; gemm_f32_rows_kernel, attn_f32_token_kernel): 32-bit sums, the residual stream in 32 bits, the norm's scale
 // applied by the consumer of bfloat16(x * gain), partial results of key splits merged in split order.
 #pragma once
+#include "attention_f32.h"
 #include "attention_mfma.h"
 
 typedef unsigned long long u64;
 typedef __attribute__((ext_vector_type(4))) uint32_t dc_u32x4_t;
 
 constexpr int DC_LAYERS = 32;           // layers of a launch (their pointers are kernel arguments)
-constexpr int DC_WAVES = 4, DC_THREADS = 64 * DC_WAVES;
 constexpr int DC_MAX_ROWS = 4;
 constexpr int DC_SHARDS = 8, DC_LINE = 16;      // ticket counters, 64-bit words between two of them (a line)
 constexpr int DC_D = 128;               // head size
@@ -46,17 +46,57 @@ constexpr int DC_GROUP = 4;             // steps of K (32 wide) asked for togeth
 constexpr int DC_SHORT = 6, DC_LONG = 6;        // such groups on their way: a wave's whole share of a short K; of a longer one
 constexpr int DC_TILE = 16;             // weight rows of a tile
 constexpr int DC_MAX_TILES = 3;         // tiles of a block whose K is short
-constexpr int DC_MAX_LDS = 80 << 10;     // two launches beside each other fit a CU
+constexpr int DC_MAX_LDS = 128 << 10;
 constexpr int DC_APART = 8;             // words between two tiles' sums of squares (side by side sixteen blocks write one line that all ask for: 24 against 20 us a layer)
 constexpr int DC_PAD = 64;              // bytes between two rows of activations in LDS
 constexpr u64 DC_PATIENCE = 400000000ull;       // ticks of 10 ns after which a wait gives up
 
+// The compute type's ways.  bfloat16: two values a word of operands, 32 of K a load, scores in powers of two.  32-bit: one, 16,
+// natural exponentials, and products of 4x4x1 in sixteen blocks: a block is four weight rows and four rows of activations at one
+// of the load's four places of K, so nothing is multiplied for rows that are not there (16x16x4 with four of its sixteen columns
+// in use takes four times the clocks, 2.7 us an item at K of 3,072).
+template <typename E> struct DcType;
+template <> struct DcType<bf16_t> {
+    static constexpr int PER_WORD = 2, STEP = 32;
+    static __device__ __forceinline__ float exp(float x) { return fast_exp2(x); }
+    static __device__ __forceinline__ bf16_t from(float v) { return f32_to_bf16(v); }
+    // element e of a lane: weight row 4 (l/16) + e, row of activations l%16
+    static __device__ __forceinline__ int x_row(int lane) { return lane & 15; }
+    static __device__ __forceinline__ void multiply(dc_u32x4_t w, dc_u32x4_t x, f32x4_t& acc) {
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), acc, 0, 0, 0);
+    }
+    static __device__ __forceinline__ void finish(f32x4_t&) {}
+    static __device__ __forceinline__ int w_row(int lane) { return (lane >> 4) * 4; }
+    static __device__ __forceinline__ bool holds(int lane, int rows) { return (lane & 15) < rows; }
+};
+template <> struct DcType<float> {
+    static constexpr int PER_WORD = 1, STEP = 16;
+    static __device__ __forceinline__ float exp(float x) { return expf(x); }
+    static __device__ __forceinline__ float from(float v) { return v; }
+    // element e of a lane: weight row 4 (l/4 % 4) + e, row of activations l%4, the places l/16 of K
+    static __device__ __forceinline__ int x_row(int lane) { return lane & 3; }
+    static __device__ __forceinline__ void multiply(dc_u32x4_t w, dc_u32x4_t x, f32x4_t& acc) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            acc = __builtin_amdgcn_mfma_f32_4x4x1f32(__uint_as_float(w[e]), __uint_as_float(x[e]), acc, 0, 0, 0);
+    }
+    static __device__ __forceinline__ void finish(f32x4_t& acc) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            acc[e] += __shfl_xor(acc[e], 16, 64);
+            acc[e] += __shfl_xor(acc[e], 32, 64);
+        }
+    }
+    static __device__ __forceinline__ int w_row(int lane) { return (lane >> 2) * 4; }
+    static __device__ __forceinline__ bool holds(int lane, int rows) { return lane < 16 && (lane & 3) < rows; }
+};
+
 struct DcLayer {
-    const bf16_t *w_qkv, *w_o, *w_gu, *w_down;
+    const void *w_qkv, *w_o, *w_gu, *w_down;
     const float *q_gain, *k_gain;       // per-head norms
     const float* ffn_gain;              // the norm between attention and feed-forward
     const float* next_gain;             // the next layer's first norm (last layer: null)
-    bf16_t *k, *v;                      // cache pages
+    void *k, *v;                        // cache pages
 };
 
 // Word offsets of the buffers in the state (64-bit words).  The first DC_SHARDS lines hold the ticket counters, the next one the
@@ -66,18 +106,18 @@ struct DcPlan {
     int items[6], per_layer;            // work items of a layer's stages, in order
     int qkv_tiles, gu_tiles;            // tiles of an item of these stages
     int y, part, part_ml, o, xa, xga, ssqa, h, xb, xgb, ssqb, words;
-    int lds;
+    int waves, lds;
 };
 
 struct DcArgs {
     DcPlan p;
     u64* state;
     float* x;                           // [rows, hidden] residual stream, in and out
-    const bf16_t* xn;                   // [rows, hidden] the first layer's normed operand
+    const void* xn;                     // [rows, hidden] the first layer's normed operand
     const int* block_table; int bt_width;
     const int* pos;
     const float *cos_t, *sin_t;         // [rows, 64]
-    float scale_log2e, qk_eps, eps_mix, eps_ffn, inv_width;
+    float scale, qk_eps, eps_mix, eps_ffn, inv_width;
     DcLayer layer[DC_LAYERS];
 };
 
@@ -162,14 +202,15 @@ template <int V> struct DcInt { static constexpr int value = V; };
 struct DcItem { int stage, layer, i; uint32_t epoch; };
 
 // LDS of a block.
+template <int W>
 struct DcLds {
     u64 next[2];                                // the item after this one, in turn
     // the waves' sums (two of them in turn: the other waves go on to the next item while the first finishes this one)
-    float red[2][DC_MAX_TILES][DC_WAVES][DC_MAX_ROWS][DC_TILE];
-    float m[DC_WAVES][16], l[DC_WAVES][16];
-    float o[DC_WAVES][DC_MAX_GROUP][DC_D + 4];
-    bf16_t q[DC_MAX_GROUP][DC_D], k[DC_D], v[DC_D];
-    char x[];                                   // operands of a product, rows of 2 K + DC_PAD bytes
+    float red[2][DC_MAX_TILES][W][DC_MAX_ROWS][DC_TILE];
+    float m[W][16], l[W][16];
+    float o[W][DC_MAX_GROUP][DC_D + 4];
+    float q[DC_MAX_GROUP][DC_D], k[DC_D], v[DC_D];      // (of the compute type)
+    char x[];                                   // operands of a product, rows of K values and DC_PAD bytes
 };
 
 __device__ __forceinline__ int dc_k(const DcPlan& p, int stage) { return stage == DC_O ? p.hq * DC_D : stage == DC_DOWN ? p.inter : p.hidden; }
@@ -195,13 +236,15 @@ __device__ __forceinline__ void dc_take(u64* st, uint32_t epoch, const u64* row,
 }
 
 // SHORT: a wave's weights are all in its ring at once (separate code: one ring for both would be held twice).
-// One to three tiles of 16 weight rows times all rows of activations.  A wave has a quarter of K: it asks for its weights, takes
+// One to three tiles of 16 weight rows times all rows of activations.  A wave has an equal share of K: it asks for its weights, takes
 // its share of the operands into LDS (nobody else reads it) and multiplies; the waves meet once, and the first one finishes.
 __device__ __forceinline__ int dc_tiles(const DcPlan& p, int stage) { return stage == DC_QKV ? p.qkv_tiles : stage == DC_GU ? p.gu_tiles : 1; }
 
-template <int M, bool SHORT>
-__device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, const DcItem& it, DcLds& sm, const DcTickets& tickets, int turn,
+template <typename E, int W, int M, bool SHORT>
+__device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, const DcItem& it, DcLds<W>& sm, const DcTickets& tickets, int turn,
                                            int wave, int lane) {
+    using T = DcType<E>;
+    constexpr int SIZE = sizeof(E), V = T::PER_WORD;
     const DcPlan& p = a.p;
     u64* st = a.state;
     const int stage = it.stage, layer = it.layer;
@@ -209,15 +252,15 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
     const bool residual = stage == DC_O || stage == DC_DOWN, head = layer == 0;
     const int g = lane >> 4, col = lane & 15;
     const int tiles = SHORT ? dc_tiles(p, stage) : 1, tile0 = it.i * tiles;
-    const bf16_t* w = stage == DC_QKV ? ly.w_qkv : stage == DC_O ? ly.w_o : stage == DC_GU ? ly.w_gu : ly.w_down;
-    const int k = dc_k(p, stage), share = k / DC_WAVES, first = wave * share, groups = share / (32 * DC_GROUP);
-    auto strip = ga_buffer(w + (size_t)tile0 * DC_TILE * k, (long long)tiles * DC_TILE * k * 2);
-    const uint32_t at = (uint32_t)(col * k + first + g * 8) * 2u;
+    const E* w = (const E*)(stage == DC_QKV ? ly.w_qkv : stage == DC_O ? ly.w_o : stage == DC_GU ? ly.w_gu : ly.w_down);
+    const int k = dc_k(p, stage), share = k / W, first = wave * share, groups = share / (T::STEP * DC_GROUP);
+    auto strip = ga_buffer(w + (size_t)tile0 * DC_TILE * k, (long long)tiles * DC_TILE * k * SIZE);
+    const uint32_t at = (uint32_t)(col * k + first) * SIZE + g * 16u;
     constexpr int RING = SHORT ? DC_SHORT : DC_LONG;
     dc_u32x4_t ring[RING][DC_GROUP];
     auto request = [&](int r, int group, int tile) {
         uint32_t from = group < groups && tile < tiles ? at : BUF_NOWHERE;
-        uint32_t behind = (uint32_t)(tile * DC_TILE * k) * 2u + group * (DC_GROUP * 64);
+        uint32_t behind = (uint32_t)(tile * DC_TILE * k) * SIZE + group * (DC_GROUP * 64);
 #pragma unroll
         for (int j = 0; j < DC_GROUP; ++j)
             ring[r][j] = __builtin_bit_cast(dc_u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(strip, from, behind + j * 64, 0));
@@ -243,24 +286,24 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
     }
     asm volatile("" ::: "memory");              // (the requests stay before the waits)
     __builtin_amdgcn_sched_barrier(0);
-    const int pitch = k * 2 + DC_PAD;
+    const int pitch = k * SIZE + DC_PAD;
     // (the next item is drawn when this one's turn is near: drawn with the weights it would be bound to a block that still waits
     // while others have nothing to do, 37 against 30 us a layer; drawn at the end it would be waited for, 4 us a layer)
     u64 drawn = 0;
-    if (stage == DC_QKV && head && wave == DC_WAVES - 1 && lane == 0) drawn = tickets.draw();
+    if (stage == DC_QKV && head && wave == W - 1 && lane == 0) drawn = tickets.draw();
     if (stage == DC_QKV && head) {
 #pragma unroll
         for (int m = 0; m < M; ++m)
-            for (int i = lane; i < share / 2; i += 64)
-                *(uint32_t*)(sm.x + m * pitch + first * 2 + i * 4) = ((const uint32_t*)(a.xn + (size_t)m * k + first))[i];
+            for (int i = lane; i < share / V; i += 64)
+                *(uint32_t*)(sm.x + m * pitch + first * SIZE + i * 4) = ((const uint32_t*)((const E*)a.xn + (size_t)m * k + first))[i];
     } else {
         const u64* src = stage == DC_QKV ? st + p.xgb : stage == DC_O ? st + p.o : stage == DC_GU ? st + p.xga : st + p.h;
         const u64* far = stage == DC_QKV ? st + p.h : stage == DC_O ? st + p.y : stage == DC_GU ? st + p.o : st + p.xga;
-        const int n_far = stage == DC_QKV ? p.inter / 2 : stage == DC_O ? p.n_qkv : stage == DC_GU ? p.hq * DC_D / 2 : p.hidden / 2;
+        const int n_far = stage == DC_QKV ? p.inter / V : stage == DC_O ? p.n_qkv : stage == DC_GU ? p.hq * DC_D / V : p.hidden / V;
         const uint32_t src_epoch = stage == DC_QKV ? epoch - 1 : epoch;
         if (wave == 0) dc_far_wait(st, far + it.i * DC_LINE % n_far, src_epoch);
         __syncthreads();
-        if (wave == DC_WAVES - 1 && lane == 0) drawn = tickets.draw();
+        if (wave == W - 1 && lane == 0) drawn = tickets.draw();
         if (residual && wave == 0 && !(stage == DC_O && head)) {
             // (there before the operands are)
             uint32_t v[1];
@@ -269,12 +312,12 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
                           [&](int, uint32_t o) { return dc_at(from, o); }, v);
             x_old = __uint_as_float(v[0]);
         }
-        int left = share / 128;
-        const u64* row = src + first / 2;
-        char* to = sm.x + first * 2;
+        int left = share / (64 * V);
+        const u64* row = src + first / V;
+        char* to = sm.x + first * SIZE;
         auto take = [&](auto n, auto with_ssq) {
             constexpr int N = decltype(n)::value;
-            dc_take<M, N, decltype(with_ssq)::value>(st, src_epoch, row, k / 2, to, pitch, st + p.ssqa, p.hidden / DC_TILE, lane, ss);
+            dc_take<M, N, decltype(with_ssq)::value>(st, src_epoch, row, k / V, to, pitch, st + p.ssqa, p.hidden / DC_TILE, lane, ss);
             row += N * 64;
             to += N * 256;
             left -= N;
@@ -289,12 +332,12 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
         if (left >= 2) take(DcInt<2>{}, DcInt<0>{});
         if (left >= 1) take(DcInt<1>{}, DcInt<0>{});
     }
-    if (wave == DC_WAVES - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
+    if (wave == W - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
 
     f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    const char* xs = sm.x + (M > 1 ? col % M : 0) * pitch + (first + g * 8) * 2;         // (columns beyond the rows repeat them)
+    const char* xs = sm.x + (M > 1 ? T::x_row(lane) % M : 0) * pitch + first * SIZE + g * 16;         // (columns beyond the rows repeat them)
     auto multiply = [&](int r, int group) {
         dc_u32x4_t xv[DC_GROUP];                // (read together: one by one each product waits for its own trip to LDS)
 #pragma unroll
@@ -302,13 +345,13 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int j = 0; j < DC_GROUP; ++j)
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, ring[r][j]), __builtin_bit_cast(bf16x8_t, xv[j]), acc, 0, 0, 0);
+            T::multiply(ring[r][j], xv[j], acc);
     };
     auto hand_over = [&](int tile) {
-        // element e of a lane: weight row 4g + e, row of activations col
-        if (col < M) {
+        T::finish(acc);
+        if (T::holds(lane, M)) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) sm.red[turn][tile][wave][col][g * 4 + e] = acc[e];
+            for (int e = 0; e < 4; ++e) sm.red[turn][tile][wave][T::x_row(lane)][T::w_row(lane) + e] = acc[e];
         }
         acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
     };
@@ -351,7 +394,7 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
         if (orow < M) {
             v = red[0][orow][col];
 #pragma unroll
-            for (int i = 1; i < DC_WAVES; ++i) v += red[i][orow][col];
+            for (int i = 1; i < W; ++i) v += red[i][orow][col];
         }
         if (stage == DC_QKV) {
             if (orow < M) dc_store(st + p.y + (size_t)orow * p.n_qkv + ocol + tile * DC_TILE, __float_as_uint(v), epoch);
@@ -360,9 +403,13 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
             v *= scale;
             float up = __shfl_xor(v, 1, 64);
             float hv = v / (1.0f + expf(-v)) * up;
-            float hn = __shfl_xor(hv, 2, 64);
-            if (orow < M && (col & 3) == 0)
-                dc_store(st + p.h + (size_t)orow * (p.inter / 2) + (tile0 + tile) * 4 + col / 4, f32x2_to_bf16x2(hv, hn), epoch);
+            u64* to = st + p.h + (size_t)orow * (p.inter / V) + (tile0 + tile) * (8 / V);
+            if constexpr (V == 2) {
+                float hn = __shfl_xor(hv, 2, 64);
+                if (orow < M && (col & 3) == 0) dc_store(to + col / 4, f32x2_to_bf16x2(hv, hn), epoch);
+            } else {
+                if (orow < M && (col & 1) == 0) dc_store(to + col / 2, __float_as_uint(hv), epoch);
+            }
         } else {
             float r = x_old + v;
             if (stage == DC_DOWN && layer == p.n_layers - 1) {
@@ -375,8 +422,9 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
             for (int off = 1; off < 16; off <<= 1) sq += __shfl_xor(sq, off, 64);
             if (orow < M) {
                 const bool o = stage == DC_O;
-                if ((col & 1) == 0)
-                    dc_store(st + (o ? p.xga : p.xgb) + (size_t)orow * (p.hidden / 2) + ocol / 2, f32x2_to_bf16x2(xg, xn), epoch);
+                u64* to = st + (o ? p.xga : p.xgb) + (size_t)orow * (p.hidden / V) + ocol / V;
+                if (V == 1) dc_store(to, __float_as_uint(xg), epoch);
+                else if ((col & 1) == 0) dc_store(to, f32x2_to_bf16x2(xg, xn), epoch);
                 if (col == 0) dc_store(st + (o ? p.ssqa : p.ssqb) + (orow * (p.hidden / DC_TILE) + tile0) * DC_APART, __float_as_uint(sq), epoch);
                 dc_store(st + (o ? p.xa : p.xb) + (size_t)orow * p.hidden + ocol, __float_as_uint(r), epoch);
             }
@@ -384,12 +432,223 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
     }
 }
 
+// What the waves of an attention item do with the cached keys: the first piece is asked for before the projection is waited for
+// (request_first), and behind the queries they multiply, their results meeting in LDS (run).
+template <typename E, int W> struct DcPieces;
+
+// bfloat16: a piece is 32 keys.
+template <int W> struct DcPieces<bf16_t, W> {
+    static constexpr int D = DC_D, KD = D / 32, DT = D / 16;
+    const DcArgs& a; const DcLayer& ly; const int* pages;
+    int kvh, split, my_pages, group, wave, lane;
+    uint4 kbuf[2][KD], vbuf[DT];
+
+    __device__ __forceinline__ void request(int piece) {
+        const int g = lane >> 4, col = lane & 15;
+        const size_t head = (size_t)pages[split + (piece >> 1) * a.p.splits] * a.p.hkv + kvh;
+        const bf16_t* kb = (const bf16_t*)ly.k + (head * AM_PAGE + (piece & 1) * 32) * D;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int kd = 0; kd < KD; ++kd)
+                kbuf[u][kd] = *(const uint4*)(kb + (uint32_t)((8 * (col >> 2) + 4 * u + (col & 3)) * D + g * 8 + kd * 32));
+        const bf16_t* vb = (const bf16_t*)ly.v + head * D * AM_PAGE + (piece & 1) * 32;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) vbuf[dt] = *(const uint4*)(vb + (uint32_t)((dt * 16 + col) * AM_PAGE + g * 8));
+    }
+    __device__ __forceinline__ void request_first() {
+        if (wave < my_pages * 2) request(wave);
+    }
+    __device__ __forceinline__ void run(DcLds<W>& sm, int cached, bool owner, int new_pos) {
+        const int g = lane >> 4, col = lane & 15, n_pieces = my_pages * 2;
+        const float scale_log2e = a.scale * AM_LOG2E;
+        const bf16_t *sq = (const bf16_t*)sm.q, *sk = (const bf16_t*)sm.k, *sv = (const bf16_t*)sm.v;
+        // Q^T operand: column = head of the group (zero beyond it); read for every piece, registers are scarcer than LDS reads
+        auto query = [&](int kd) {
+            uint4 v = *(const uint4*)(sq + (col < group ? col : 0) * D + kd * 32 + g * 8);
+            bool ok = col < group;
+            v.x = ok ? v.x : 0u; v.y = ok ? v.y : 0u; v.z = ok ? v.z : 0u; v.w = ok ? v.w : 0u;
+            return __builtin_bit_cast(bf16x8_t, v);
+        };
+        float m = -INFINITY, l = 0.f;
+        f32x4_t o[DT];
+#pragma unroll
+        for (int i = 0; i < DT; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        auto scores = [&](int key0, int to, f32x4_t (&s)[2]) {
+            // element i of s[u] is key 8g + 4u + i, column = head
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                s[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int kd = 0; kd < KD; ++kd)
+                    s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kbuf[u][kd]), query(kd), s[u], 0, 0, 0);
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) s[u][i] = key0 + g * 8 + u * 4 + i < to ? s[u][i] * scale_log2e : -INFINITY;
+        };
+        auto add_values = [&](f32x4_t (&s)[2]) {
+            float mx = -INFINITY;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[u][i]);
+            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            float m_new = fmaxf(m, mx);
+            float m_use = m_new == -INFINITY ? 0.f : m_new;
+            float corr = fast_exp2(m - m_use), sum = 0.f;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[u][i] = fast_exp2(s[u][i] - m_use);
+                    sum += s[u][i];
+                }
+            sum += __shfl_xor(sum, 16, 64);
+            sum += __shfl_xor(sum, 32, 64);
+            l = l * corr + sum;
+            m = m_new;
+            uint4 pv = make_uint4(pack_bf16x2(s[0][0], s[0][1]), pack_bf16x2(s[0][2], s[0][3]),
+                                  pack_bf16x2(s[1][0], s[1][1]), pack_bf16x2(s[1][2], s[1][3]));
+            bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pv);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                o[dt] = o[dt] * corr;
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vbuf[dt]), pf, o[dt], 0, 0, 0);
+            }
+        };
+        // (the step's own key is not yet in the cache where a block reads it; it comes last, from LDS)
+        for (int piece = wave; piece < n_pieces; piece += W) {
+            f32x4_t s[2];
+            if (piece != wave) request(piece);
+            scores((split + (piece >> 1) * a.p.splits) * AM_PAGE + (piece & 1) * 32, cached, s);
+            add_values(s);
+        }
+        asm volatile("" ::: "memory");
+        if (owner && wave == n_pieces % W) {
+            bool krow = col == 0, vrow = g == 0;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int kd = 0; kd < KD; ++kd) {
+                    uint4 v = *(const uint4*)(sk + kd * 32 + g * 8);
+                    bool take = krow && u == 0;
+                    kbuf[u][kd] = make_uint4(take ? v.x : 0u, take ? v.y : 0u, take ? v.z : 0u, take ? v.w : 0u);
+                }
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) vbuf[dt] = make_uint4(vrow ? (uint32_t)sv[dt * 16 + col] : 0u, 0u, 0u, 0u);
+            f32x4_t s[2];
+            scores(new_pos, new_pos + 1, s);
+            add_values(s);
+        }
+        // the waves' results in wave order; element i of o[dt] is d = 16 dt + 4g + i, column = head
+        if (col < group) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sm.o[wave][col][dt * 16 + g * 4 + i] = o[dt][i];
+        }
+        if (g == 0) {
+            sm.m[wave][col] = m;
+            sm.l[wave][col] = l;
+        }
+    }
+};
+
+// 32-bit: a piece is 16 keys, the helpers are attn_f32_token_kernel's.
+template <int W> struct DcPieces<float, W> {
+    static constexpr int D = DC_D, KD = D / 16;
+    const DcArgs& a; const DcLayer& ly; const int* pages;
+    int kvh, split, my_pages, group, wave, lane;
+    af_f32x4_t k[KD], v[KD];
+
+    __device__ __forceinline__ void request(int piece) {
+        const size_t at = ((size_t)pages[split + (piece >> 2) * a.p.splits] * a.p.hkv + kvh) * AF_PAGE * D;
+        const int in_page = (piece & 3) * 16;
+        const float* kp = (const float*)ly.k + at + (uint32_t)((in_page + (lane & 15)) * D + (lane >> 4) * 4);
+        const float* vp = (const float*)ly.v + at + (uint32_t)((lane & 15) * AF_PAGE + in_page + (lane >> 4) * 4);
+#pragma unroll
+        for (int c = 0; c < KD; ++c) k[c] = *(const af_f32x4_t*)(kp + c * 16);
+#pragma unroll
+        for (int c = 0; c < KD; ++c) v[c] = *(const af_f32x4_t*)(vp + c * 16 * AF_PAGE);
+    }
+    __device__ __forceinline__ void request_first() {
+        if (wave < my_pages * 4) request(wave);
+    }
+    __device__ __forceinline__ void run(DcLds<W>& sm, int cached, bool owner, int new_pos) {
+        AttnF32Args mask{};
+        mask.scale = a.scale;
+        const int n_pieces = my_pages * 4;
+        const float* q = sm.q[min(lane & 15, group - 1)] + (lane >> 4) * 4;
+        af_f32x4_t o[KD], s[1];
+#pragma unroll
+        for (int c = 0; c < KD; ++c) o[c] = af_f32x4_t{0.f, 0.f, 0.f, 0.f};
+        float m = -INFINITY, l = 0.f;
+        // keys first .. first + 15, of which those before `to` are seen
+        auto multiply = [&](int first, int to) {
+            af_scores<KD, 1>([&](int c) { return *(const af_f32x4_t*)(q + c * 16); }, [&](int, int c) { return k[c]; }, s);
+            af_softmax<KD, 1>(s, o, m, l, mask, first, lane, to - 1, 0, 0.f);
+            bool seen[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) seen[e] = first + (lane >> 4) * 4 + e < to;
+            af_values<KD, 1>(s, [&](int c, int) {
+                af_f32x4_t u = v[c];                  // a key that is not seen may hold anything: it is left out, not weighted by zero
+#pragma unroll
+                for (int e = 0; e < 4; ++e) u[e] = seen[e] ? u[e] : 0.f;
+                return u;
+            }, o);
+        };
+        for (int piece = wave; piece < n_pieces; piece += W) {
+            const int first = (split + (piece >> 2) * a.p.splits) * AF_PAGE + (piece & 3) * 16;
+            if (first >= cached) continue;
+            if (piece != wave) request(piece);
+            multiply(first, cached);
+        }
+        asm volatile("" ::: "memory");
+        // (the step's own key is not yet in the cache where a block reads it; it comes last, from LDS)
+        if (owner && wave == n_pieces % W) {
+#pragma unroll
+            for (int c = 0; c < KD; ++c) {
+                k[c] = *(const af_f32x4_t*)(sm.k + c * 16 + (lane >> 4) * 4);
+                v[c] = af_f32x4_t{sm.v[c * 16 + (lane & 15)], 0.f, 0.f, 0.f};
+            }
+            multiply(new_pos, new_pos + 1);
+        }
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        const int row = lane & 15;
+        if (lane < 16) {
+            sm.m[wave][lane] = m;
+            sm.l[wave][lane] = l;
+        }
+        if (row < group) {
+#pragma unroll
+            for (int c = 0; c < KD; ++c) *(af_f32x4_t*)(&sm.o[wave][row][c * 16 + (lane >> 4) * 4]) = o[c];
+        }
+    }
+};
+
+// Two neighbouring values of a (token, head)'s output.
+template <typename E>
+__device__ __forceinline__ void dc_store_pair(u64* out, int row, int lane, float v0, float v1, uint32_t epoch) {
+    if constexpr (DcType<E>::PER_WORD == 2) {
+        dc_store(out + (size_t)row * (DC_D / 2) + lane, f32x2_to_bf16x2(v0, v1), epoch);
+    } else {
+        dc_store(out + (size_t)row * DC_D + lane * 2, __float_as_uint(v0), epoch);
+        dc_store(out + (size_t)row * DC_D + lane * 2 + 1, __float_as_uint(v1), epoch);
+    }
+}
+
 // One (token, kv head, split of its pages): the query heads of the kv head from the projection, the cached keys, and in the
 // block whose split holds the last page the step's own key and value, which it also appends.  Pages split, split + splits, ...;
-// a piece is 32 keys, the waves take pieces in turn, and a wave's first piece is asked for before the projection is waited for.
-__device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly, const DcItem& it, DcLds& sm, const DcTickets& tickets, int turn,
+// the waves take their pieces in turn.
+template <typename E, int W>
+__device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly, const DcItem& it, DcLds<W>& sm, const DcTickets& tickets, int turn,
                                              int wave, int lane) {
-    constexpr int D = DC_D, KD = D / 32, DT = D / 16, ROWS = (DC_MAX_GROUP + 2 + DC_WAVES - 1) / DC_WAVES;
+    constexpr int D = DC_D, ROWS = (DC_MAX_GROUP + 2 + W - 1) / W;
+    using T = DcType<E>;
     const DcPlan& p = a.p;
     u64* st = a.state;
     const uint32_t epoch = it.epoch;
@@ -400,27 +659,8 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
     const int new_pos = a.pos[t], len = new_pos + 1;
     const int n_pages = (len + AM_PAGE - 1) / AM_PAGE;
     const int my_pages = split < n_pages ? (n_pages - split + p.splits - 1) / p.splits : 0;
-    const int n_pieces = my_pages * 2;
-    uint4 kbuf[2][KD], vbuf[DT];
-    auto request_keys = [&](int piece) {
-        int phys = pages[split + (piece >> 1) * p.splits];
-        const bf16_t* base = ly.k + (((size_t)phys * p.hkv + kvh) * AM_PAGE + (piece & 1) * 32) * D;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int kd = 0; kd < KD; ++kd)
-                kbuf[u][kd] = *(const uint4*)(base + (uint32_t)((8 * (col >> 2) + 4 * u + (col & 3)) * D + g * 8 + kd * 32));
-    };
-    auto request_values = [&](int piece) {
-        int phys = pages[split + (piece >> 1) * p.splits];
-        const bf16_t* base = ly.v + ((size_t)phys * p.hkv + kvh) * D * AM_PAGE + (piece & 1) * 32;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) vbuf[dt] = *(const uint4*)(base + (uint32_t)((dt * 16 + col) * AM_PAGE + g * 8));
-    };
-    if (wave < n_pieces) {
-        request_keys(wave);
-        request_values(wave);
-    }
+    DcPieces<E, W> piece{a, ly, pages, kvh, split, my_pages, group, wave, lane};
+    piece.request_first();
     const bool owner = new_pos / AM_PAGE % p.splits == split;
     const int phys = pages[new_pos / AM_PAGE];
     const int n_rows = group + (owner ? 2 : 0);
@@ -430,22 +670,22 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
     __builtin_amdgcn_sched_barrier(0);
     float row_scale = 1.0f;
     if (it.layer > 0) {
-        if (wave == 0) dc_far_wait(st, st + p.xgb + it.i * DC_LINE % (p.hidden / 2), epoch - 1);
+        if (wave == 0) dc_far_wait(st, st + p.xgb + it.i * DC_LINE % (p.hidden / T::PER_WORD), epoch - 1);
         __syncthreads();
         row_scale = dc_row_scale(st, st + p.ssqb + t * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch - 1, a.inv_width, a.eps_mix, lane);
     }
     u64 drawn = 0;
-    if (wave == DC_WAVES - 1 && lane == 0) drawn = tickets.draw();
+    if (wave == W - 1 && lane == 0) drawn = tickets.draw();
     // a wave's rows of the projection together: a lane has the values lane and lane + 64 of each
     {
         const u64* tok = st + p.y + (size_t)t * p.n_qkv;
         auto from = [&](int r) { return tok + (size_t)(r < group ? kvh * group + r : r == group ? p.hq + kvh : p.hq + p.hkv + kvh) * D; };
         uint32_t raw[2 * ROWS];
         dc_collect<2 * ROWS>(st, epoch, true, lane * 8u, [&](int i, uint32_t o) {
-            return dc_at(from(min(wave + i / 2 * DC_WAVES, n_rows - 1)) + (i & 1) * 64, o); }, raw);
+            return dc_at(from(min(wave + i / 2 * W, n_rows - 1)) + (i & 1) * 64, o); }, raw);
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
-            int r = wave + DC_WAVES * i;
+            int r = wave + W * i;
             if (r >= n_rows) break;
             float v0 = __uint_as_float(raw[2 * i]) * row_scale, v1 = __uint_as_float(raw[2 * i + 1]) * row_scale;
             if (r <= group) {
@@ -457,137 +697,43 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
                 v0 = lo;
                 v1 = hi;
             }
-            bf16_t b0 = f32_to_bf16(v0), b1 = f32_to_bf16(v1);
-            bf16_t* dst = r < group ? sm.q[r] : r == group ? sm.k : sm.v;
+            E b0 = T::from(v0), b1 = T::from(v1);
+            E* dst = r < group ? (E*)sm.q + r * D : r == group ? (E*)sm.k : (E*)sm.v;
             dst[lane] = b0;
             dst[lane + 64] = b1;
             if (phys >= 0 && r >= group) {
                 const size_t head = (size_t)phys * p.hkv + kvh;
                 const int at = new_pos % AM_PAGE;
                 if (r == group) {
-                    ly.k[(head * AM_PAGE + at) * D + lane] = b0;
-                    ly.k[(head * AM_PAGE + at) * D + lane + 64] = b1;
+                    ((E*)ly.k)[(head * AM_PAGE + at) * D + lane] = b0;
+                    ((E*)ly.k)[(head * AM_PAGE + at) * D + lane + 64] = b1;
                 } else {
-                    ly.v[(head * D + lane) * AM_PAGE + at] = b0;
-                    ly.v[(head * D + lane + 64) * AM_PAGE + at] = b1;
+                    ((E*)ly.v)[(head * D + lane) * AM_PAGE + at] = b0;
+                    ((E*)ly.v)[(head * D + lane + 64) * AM_PAGE + at] = b1;
                 }
             }
         }
     }
-    if (wave == DC_WAVES - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
+    if (wave == W - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
     __syncthreads();
-    // Q^T operand: column = head of the group (zero beyond it); read for every piece, registers are scarcer than LDS reads
-    auto query = [&](int kd) {
-        uint4 v = *(const uint4*)(&sm.q[col < group ? col : 0][kd * 32 + g * 8]);
-        bool ok = col < group;
-        v.x = ok ? v.x : 0u; v.y = ok ? v.y : 0u; v.z = ok ? v.z : 0u; v.w = ok ? v.w : 0u;
-        return __builtin_bit_cast(bf16x8_t, v);
-    };
-    float m = -INFINITY, l = 0.f;
-    f32x4_t o[DT];
-#pragma unroll
-    for (int i = 0; i < DT; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    auto scores = [&](int key0, int to, f32x4_t (&s)[2]) {
-        // element i of s[u] is key 8g + 4u + i, column = head
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            s[u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int kd = 0; kd < KD; ++kd)
-                s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kbuf[u][kd]), query(kd), s[u], 0, 0, 0);
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) s[u][i] = key0 + g * 8 + u * 4 + i < to ? s[u][i] * a.scale_log2e : -INFINITY;
-    };
-    auto add_values = [&](f32x4_t (&s)[2]) {
-        float mx = -INFINITY;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[u][i]);
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        float m_new = fmaxf(m, mx);
-        float m_use = m_new == -INFINITY ? 0.f : m_new;
-        float corr = fast_exp2(m - m_use), sum = 0.f;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                s[u][i] = fast_exp2(s[u][i] - m_use);
-                sum += s[u][i];
-            }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
-        l = l * corr + sum;
-        m = m_new;
-        uint4 pv = make_uint4(pack_bf16x2(s[0][0], s[0][1]), pack_bf16x2(s[0][2], s[0][3]),
-                              pack_bf16x2(s[1][0], s[1][1]), pack_bf16x2(s[1][2], s[1][3]));
-        bf16x8_t pf = __builtin_bit_cast(bf16x8_t, pv);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            o[dt] = o[dt] * corr;
-            o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vbuf[dt]), pf, o[dt], 0, 0, 0);
-        }
-    };
-    // (the step's own key is not yet in the cache where a block reads it; it comes last, from LDS)
-    const int cached = owner ? new_pos : len;
-    for (int piece = wave; piece < n_pieces; piece += DC_WAVES) {
-        f32x4_t s[2];
-        if (piece != wave) {
-            request_keys(piece);
-            request_values(piece);
-        }
-        scores((split + (piece >> 1) * p.splits) * AM_PAGE + (piece & 1) * 32, cached, s);
-        add_values(s);
-    }
-    asm volatile("" ::: "memory");
-    if (owner && wave == n_pieces % DC_WAVES) {
-        bool krow = col == 0, vrow = g == 0;
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int kd = 0; kd < KD; ++kd) {
-                uint4 v = *(const uint4*)(sm.k + kd * 32 + g * 8);
-                bool take = krow && u == 0;
-                kbuf[u][kd] = make_uint4(take ? v.x : 0u, take ? v.y : 0u, take ? v.z : 0u, take ? v.w : 0u);
-            }
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) vbuf[dt] = make_uint4(vrow ? (uint32_t)sm.v[dt * 16 + col] : 0u, 0u, 0u, 0u);
-        f32x4_t s[2];
-        scores(new_pos, new_pos + 1, s);
-        add_values(s);
-    }
-    // the waves' results in wave order; element i of o[dt] is d = 16 dt + 4g + i, column = head
-    if (col < group) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sm.o[wave][col][dt * 16 + g * 4 + i] = o[dt][i];
-    }
-    if (g == 0) {
-        sm.m[wave][col] = m;
-        sm.l[wave][col] = l;
-    }
+    piece.run(sm, owner ? new_pos : len, owner, new_pos);
     __syncthreads();
-    for (int head = wave; head < group; head += DC_WAVES) {
+    for (int head = wave; head < group; head += W) {
         const int d = lane * 2;
         float mm = sm.m[0][head];
 #pragma unroll
-        for (int w = 1; w < DC_WAVES; ++w) mm = fmaxf(mm, sm.m[w][head]);
+        for (int w = 1; w < W; ++w) mm = fmaxf(mm, sm.m[w][head]);
         float ll = 0.f, o0 = 0.f, o1 = 0.f;
 #pragma unroll
-        for (int w = 0; w < DC_WAVES; ++w) {
-            float wgt = sm.m[w][head] == -INFINITY ? 0.f : fast_exp2(sm.m[w][head] - mm);
+        for (int w = 0; w < W; ++w) {
+            float wgt = sm.m[w][head] == -INFINITY ? 0.f : T::exp(sm.m[w][head] - mm);
             ll += sm.l[w][head] * wgt;
             o0 += sm.o[w][head][d] * wgt;
             o1 += sm.o[w][head][d + 1] * wgt;
         }
         int row = t * p.hq + kvh * group + head;
         if (p.splits == 1) {
-            dc_store(st + p.o + (size_t)row * (D / 2) + lane, f32x2_to_bf16x2(o0 / ll, o1 / ll), epoch);
+            dc_store_pair<E>(st + p.o, row, lane, o0 / ll, o1 / ll, epoch);
         } else {
             size_t slot = (size_t)row * p.splits + split;
             dc_store(st + p.part + slot * D + d, __float_as_uint(o0), epoch);
@@ -601,8 +747,9 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
     __syncthreads();                            // (the LDS is the next item's)
 }
 
-// The splits of one (token, query head) by log-sum-exp in split order, a quarter of them a wave.
-__device__ __forceinline__ void dc_merge(const DcArgs& a, const DcItem& it, DcLds& sm, const DcTickets& tickets, int turn, int wave, int lane) {
+// The splits of one (token, query head) by log-sum-exp in split order, a run of them a wave.
+template <typename E, int W>
+__device__ __forceinline__ void dc_merge(const DcArgs& a, const DcItem& it, DcLds<W>& sm, const DcTickets& tickets, int turn, int wave, int lane) {
     constexpr int D = DC_D;
     const DcPlan& p = a.p;
     u64* st = a.state;
@@ -611,18 +758,18 @@ __device__ __forceinline__ void dc_merge(const DcArgs& a, const DcItem& it, DcLd
     if (wave == 0) dc_far_wait(st, st + p.y + row * DC_LINE % p.n_qkv, epoch);
     __syncthreads();
     u64 drawn = 0;
-    if (wave == DC_WAVES - 1 && lane == 0) drawn = tickets.draw();
+    if (wave == W - 1 && lane == 0) drawn = tickets.draw();
     const u64* ml = st + p.part_ml + (size_t)row * p.splits * 2;
     bool mine = lane < p.splits;
     uint32_t v[2];
     dc_collect<2>(st, epoch, mine, mine ? lane * 16u : 0u, [&](int i, uint32_t o) { return dc_at(ml + i, o); }, v);
     float ms = mine ? __uint_as_float(v[0]) : -INFINITY, ls = mine ? __uint_as_float(v[1]) : 0.f;
     float mm = wave_max(ms);
-    float wgt = ms == -INFINITY ? 0.f : fast_exp2(ms - mm);
+    float wgt = ms == -INFINITY ? 0.f : DcType<E>::exp(ms - mm);
     float inv_l = 1.0f / wave_sum(ls * wgt);    // every wave computes the same sum
-    const int quarter = (p.splits + DC_WAVES - 1) / DC_WAVES, s1 = min(p.splits, (wave + 1) * quarter);
+    const int run = (p.splits + W - 1) / W, s1 = min(p.splits, (wave + 1) * run);
     float o0 = 0.f, o1 = 0.f;
-    for (int s0 = wave * quarter; s0 < s1; s0 += 4) {
+    for (int s0 = wave * run; s0 < s1; s0 += 4) {
         uint32_t q[8];
         dc_collect<8>(st, epoch, true, lane * 8u, [&](int i, uint32_t o) {
             return dc_at(st + p.part + ((size_t)row * p.splits + min(s0 + i / 2, s1 - 1)) * D + (i & 1) * 64, o); }, q);
@@ -635,7 +782,7 @@ __device__ __forceinline__ void dc_merge(const DcArgs& a, const DcItem& it, DcLd
     }
     sm.o[wave][0][lane] = o0;
     sm.o[wave][0][lane + 64] = o1;
-    if (wave == DC_WAVES - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
+    if (wave == W - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
     __syncthreads();
     if (wave == 0) {
         float r[2];
@@ -644,18 +791,18 @@ __device__ __forceinline__ void dc_merge(const DcArgs& a, const DcItem& it, DcLd
             const int d = lane * 2 + j;
             float sum = sm.o[0][0][d];
 #pragma unroll
-            for (int i = 1; i < DC_WAVES; ++i) sum += sm.o[i][0][d];
+            for (int i = 1; i < W; ++i) sum += sm.o[i][0][d];
             r[j] = sum * inv_l;
         }
-        dc_store(st + p.o + (size_t)row * (D / 2) + lane, f32x2_to_bf16x2(r[0], r[1]), epoch);
+        dc_store_pair<E>(st + p.o, row, lane, r[0], r[1], epoch);
     }
     __syncthreads();                            // (the LDS is the next item's)
 }
 
-template <int M>
-__global__ void __launch_bounds__(DC_THREADS) decode_chain_kernel(const DcArgs a) {
+template <typename E, int W, int M>
+__global__ void __launch_bounds__(64 * W) decode_chain_kernel(const DcArgs a) {
     extern __shared__ __attribute__((aligned(16))) char dc_lds[];
-    DcLds& sm = *(DcLds*)dc_lds;
+    DcLds<W>& sm = *(DcLds<W>*)dc_lds;
     const DcPlan& p = a.p;
     const uint32_t total = (uint32_t)p.per_layer * p.n_layers, shard = blockIdx.x % DC_SHARDS;
     // items shard, shard + DC_SHARDS, ...; every block of the counter draws one ticket behind them
@@ -684,20 +831,25 @@ __global__ void __launch_bounds__(DC_THREADS) decode_chain_kernel(const DcArgs a
         int tid = threadIdx.x;
         asm volatile("" : "+v"(tid));
         const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-        if (it.stage == DC_ATTN) dc_attention(a, ly, it, sm, tickets, turn, wave, lane);
-        else if (it.stage == DC_MERGE) dc_merge(a, it, sm, tickets, turn, wave, lane);
-        else if (dc_tiles(p, it.stage) * dc_k(p, it.stage) <= DC_SHORT * DC_GROUP * 32 * DC_WAVES)
-            dc_product<M, true>(a, ly, it, sm, tickets, turn, wave, lane);
-        else dc_product<M, false>(a, ly, it, sm, tickets, turn, wave, lane);
+        if (it.stage == DC_ATTN) dc_attention<E, W>(a, ly, it, sm, tickets, turn, wave, lane);
+        else if (it.stage == DC_MERGE) dc_merge<E, W>(a, it, sm, tickets, turn, wave, lane);
+        else if (dc_tiles(p, it.stage) * dc_k(p, it.stage) <= DC_SHORT * DC_GROUP * DcType<E>::STEP * W)
+            dc_product<E, W, M, true>(a, ly, it, sm, tickets, turn, wave, lane);
+        else dc_product<E, W, M, false>(a, ly, it, sm, tickets, turn, wave, lane);
     }
 }
 
 // Whether a layer's sizes fit, and the plan of buffers and blocks (words of 64 bits).
-static bool dc_plan(DcPlan& p, int rows, int hidden, int hq, int hkv, int head_dim, int inter, int n_layers, int splits) {
+static bool dc_plan(DcPlan& p, int dtype, int rows, int hidden, int hq, int hkv, int head_dim, int inter, int n_layers, int splits) {
     if (rows < 1 || rows > DC_MAX_ROWS || head_dim != DC_D || hkv < 1 || hq < hkv || hq % hkv != 0 || hq / hkv > DC_MAX_GROUP) return false;
     if (n_layers < 1 || n_layers > DC_LAYERS || splits < 1 || splits > 64) return false;
-    // a wave's quarter of K in whole groups of steps; strips of 16 weight rows whose offsets fit 31 bits
-    const int unit = 32 * DC_GROUP * DC_WAVES;
+    // a wave's share of K in whole groups of steps; strips of 16 weight rows whose offsets fit 31 bits
+    if (dtype != ROCML_BF16 && dtype != ROCML_F32) return false;
+    const bool f32 = dtype == ROCML_F32;
+    // 32-bit and wide layers: eight waves a block, so that a wave's share of K fits its ring (1.7B, one row: 500 -> 455 us a step;
+    // 0.6B in bfloat16, whose shares fit four waves' rings, 548 -> 648)
+    p.waves = f32 || (hidden >= 2048 && hidden % 1024 == 0 && inter % 1024 == 0 && hq * DC_D % 1024 == 0) ? 8 : 4;
+    const int unit = (f32 ? 16 : 32) * DC_GROUP * p.waves, v = f32 ? 1 : 2, size = f32 ? 4 : 2;
     if (hidden < unit || inter < unit || hidden % unit != 0 || inter % unit != 0 || hq * (long long)DC_D % unit != 0) return false;
     if (hidden > (1 << 20) || inter > (1 << 20) || hq > (1 << 13)) return false;
     p.rows = rows; p.hidden = hidden; p.hq = hq; p.hkv = hkv; p.inter = inter; p.n_layers = n_layers; p.splits = splits;
@@ -724,68 +876,74 @@ static bool dc_plan(DcPlan& p, int rows, int hidden, int hq, int hkv, int head_d
     p.y = take((long long)rows * p.n_qkv);
     p.part = take(splits > 1 ? (long long)rows * hq * splits * DC_D : 0);
     p.part_ml = take(splits > 1 ? (long long)rows * hq * splits * 2 : 0);
-    p.o = take((long long)rows * hq * DC_D / 2);
+    p.o = take((long long)rows * hq * DC_D / v);
     p.xa = take((long long)rows * hidden); p.xb = take((long long)rows * hidden);
-    p.xga = take((long long)rows * hidden / 2); p.xgb = take((long long)rows * hidden / 2);
+    p.xga = take((long long)rows * hidden / v); p.xgb = take((long long)rows * hidden / v);
     p.ssqa = take((long long)rows * hidden / DC_TILE * DC_APART); p.ssqb = take((long long)rows * hidden / DC_TILE * DC_APART);
-    p.h = take((long long)rows * inter / 2);
+    p.h = take((long long)rows * inter / v);
     p.words = at;
     const int most_k = inter > hidden ? (inter > hq * DC_D ? inter : hq * DC_D) : (hidden > hq * DC_D ? hidden : hq * DC_D);
-    const long long product = (long long)rows * (most_k * 2LL + DC_PAD);
-    const long long lds = sizeof(DcLds) + product;
+    const long long product = (long long)rows * (most_k * (long long)size + DC_PAD);
+    const long long lds = (p.waves == 8 ? sizeof(DcLds<8>) : sizeof(DcLds<4>)) + product;
     if (lds > DC_MAX_LDS) return false;
     p.lds = (int)lds;
     return true;
 }
 
 // Whether the chain is faster than the layers' own kernels: a matter of how long the weights' bytes take beside the stages'
-// latencies, and of how many words travel.  A layer of 31 MB of weights (Qwen3-0.6B) from one to four rows, above.  100 MB
-// (1.7B, 8 layers, to the logits): one row 536 -> 490 us, two 540 -> 546, four 580 -> 652.  202 MB (4B, 6 layers): one row 638 ->
-// 624 to 678; 386 MB (8B, 8 layers) 1,022 -> 1,154: while weights stream, a word's way takes several us.
-ROCML_EXPORT int rocml_decode_chain_pays(int rows, int hidden, int hq, int hkv, int head_dim, int inter) {
+// latencies, and of how many words travel.  Steps to the logits, replayed, us:
+//   bfloat16, 0.6B (31 MB a layer): one row 943 -> 546, four 1,096 -> 821;
+//   1.7B (100 MB, 8 layers): one row 545 -> 431, two 547 -> 470, four 580 -> 550;
+//   4B (202 MB, 6 layers): one row 628 -> 623; 8B (386 MB, 6 layers): 841 -> 878: while weights stream, a word's way takes several us;
+//   32-bit, 0.6B (63 MB): one row 1,393 -> 807, four 1,705 -> 1,086, four of 1,000 keys 2,341 -> 1,236; 1.7B (201 MB): one row 887 -> 801.
+ROCML_EXPORT int rocml_decode_chain_pays(int dtype, int rows, int hidden, int hq, int hkv, int head_dim, int inter) {
     DcPlan p;
-    if (!dc_plan(p, rows, hidden, hq, hkv, head_dim, inter, 1, 1)) return 0;
-    const double mb = 2e-6 * hidden * ((double)p.n_qkv + (double)hq * DC_D + 3.0 * inter);
-    return mb <= (rows == 1 ? 128.0 : 64.0);
+    if (!dc_plan(p, dtype, rows, hidden, hq, hkv, head_dim, inter, 1, 1)) return 0;
+    const double mb = (dtype == ROCML_F32 ? 4e-6 : 2e-6) * hidden * ((double)p.n_qkv + (double)hq * DC_D + 3.0 * inter);
+    return mb <= (dtype == ROCML_F32 && rows == 1 ? 256.0 : 128.0);
 }
 
 // 64-bit words of state that a chain of such layers needs; 0: not taken.
-ROCML_EXPORT int rocml_decode_chain_words(int rows, int hidden, int hq, int hkv, int head_dim, int inter, int n_layers, int splits) {
+ROCML_EXPORT int rocml_decode_chain_words(int dtype, int rows, int hidden, int hq, int hkv, int head_dim, int inter, int n_layers, int splits) {
     DcPlan p;
-    return dc_plan(p, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits) ? p.words : 0;
+    return dc_plan(p, dtype, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits) ? p.words : 0;
 }
 
 ROCML_EXPORT int rocml_decode_chain_max_layers() { return DC_LAYERS; }
 
 // layers: per layer the ten pointers of DcLayer.
-ROCML_EXPORT int rocml_decode_chain(void* state, long long state_words, float* x, const void* xn, const void* const* layers, int n_layers,
+ROCML_EXPORT int rocml_decode_chain(int dtype, void* state, long long state_words, float* x, const void* xn, const void* const* layers, int n_layers,
                                     int rows, int hidden, int hq, int hkv, int head_dim, int inter, const int* block_table, int bt_width,
                                     const int* token_pos, const float* cos_t, const float* sin_t, float scale, float qk_eps, float eps_mix,
                                     float eps_ffn, int splits, hipStream_t stream) {
     DcArgs a;
-    ROCML_REQUIRE(dc_plan(a.p, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits),
+    ROCML_REQUIRE(dc_plan(a.p, dtype, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits),
                   "decode_chain: sizes not taken: rows=%d hidden=%d heads=%d/%d of %d inter=%d layers=%d splits=%d", rows, hidden, hq, hkv,
                   head_dim, inter, n_layers, splits);
     ROCML_REQUIRE(state && state_words >= a.p.words, "decode_chain: the state has %lld of %d words", state_words, a.p.words);
     ROCML_REQUIRE(x && xn && layers && block_table && token_pos && cos_t && sin_t && bt_width > 0, "decode_chain: missing operand");
     a.state = (u64*)state;
-    a.x = x; a.xn = (const bf16_t*)xn; a.block_table = block_table; a.bt_width = bt_width; a.pos = token_pos;
+    a.x = x; a.xn = xn; a.block_table = block_table; a.bt_width = bt_width; a.pos = token_pos;
     a.cos_t = cos_t; a.sin_t = sin_t;
-    a.scale_log2e = scale * AM_LOG2E; a.qk_eps = qk_eps; a.eps_mix = eps_mix; a.eps_ffn = eps_ffn; a.inv_width = 1.0f / (float)hidden;
+    a.scale = scale; a.qk_eps = qk_eps; a.eps_mix = eps_mix; a.eps_ffn = eps_ffn; a.inv_width = 1.0f / (float)hidden;
     for (int i = 0; i < n_layers; ++i) {
         const void* const* f = layers + 10 * i;
         for (int j = 0; j < 10; ++j) ROCML_REQUIRE(f[j] || (j == 7 && i == n_layers - 1), "decode_chain: layer %d lacks operand %d", i, j);
-        a.layer[i] = DcLayer{(const bf16_t*)f[0], (const bf16_t*)f[1], (const bf16_t*)f[2], (const bf16_t*)f[3], (const float*)f[4],
-                             (const float*)f[5], (const float*)f[6], (const float*)f[7], (bf16_t*)f[8], (bf16_t*)f[9]};
+        a.layer[i] = DcLayer{f[0], f[1], f[2], f[3], (const float*)f[4], (const float*)f[5], (const float*)f[6], (const float*)f[7],
+                             (void*)f[8], (void*)f[9]};
     }
     // a block a CU; a whole number for every counter
     const int blocks = ceil_div(cu_count(), DC_SHARDS) * DC_SHARDS;
-    const auto kernel = rows == 1 ? decode_chain_kernel<1> : rows == 2 ? decode_chain_kernel<2> : rows == 3 ? decode_chain_kernel<3>
-                                                                                                            : decode_chain_kernel<4>;
+    typedef void (*Kernel)(DcArgs);
+    static const Kernel kernels[3][DC_MAX_ROWS] = {
+        {decode_chain_kernel<float, 8, 1>, decode_chain_kernel<float, 8, 2>, decode_chain_kernel<float, 8, 3>, decode_chain_kernel<float, 8, 4>},
+        {decode_chain_kernel<bf16_t, 4, 1>, decode_chain_kernel<bf16_t, 4, 2>, decode_chain_kernel<bf16_t, 4, 3>, decode_chain_kernel<bf16_t, 4, 4>},
+        {decode_chain_kernel<bf16_t, 8, 1>, decode_chain_kernel<bf16_t, 8, 2>, decode_chain_kernel<bf16_t, 8, 3>, decode_chain_kernel<bf16_t, 8, 4>}};
+    const Kernel kernel = kernels[dtype == ROCML_F32 ? 0 : a.p.waves == 4 ? 1 : 2][rows - 1];
     if (a.p.lds > (64 << 10))
         ROCML_REQUIRE(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, DC_MAX_LDS) == hipSuccess,
                       "decode_chain: %d bytes of LDS were refused", a.p.lds);
-    kernel<<<blocks, DC_THREADS, a.p.lds, stream>>>(a);
+    kernel<<<blocks, 64 * a.p.waves, a.p.lds, stream>>>(a);
     ROCML_CHECK_LAUNCH("decode_chain");
     return 0;
 }

@@ -87,10 +87,10 @@ _SIGNATURES = {
                             _P, _I, _I, _P, _I, _I, _P, _LL, _I, _I, _I, _P, _I, _P, _F, _I, _P],
         "rocml_attention_decode_fused": [_P, _I, _I, _LL, _P, _P, _F, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P,
                                          _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _LL, _P, _I, _F, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
-        "rocml_decode_chain_pays": [_I, _I, _I, _I, _I, _I],
-        "rocml_decode_chain_words": [_I, _I, _I, _I, _I, _I, _I, _I],
+        "rocml_decode_chain_pays": [_I, _I, _I, _I, _I, _I, _I],
+        "rocml_decode_chain_words": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
         "rocml_decode_chain_max_layers": [],
-        "rocml_decode_chain": [_P, _LL, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _F, _F, _F, _F, _I, _P],
+        "rocml_decode_chain": [_I, _P, _LL, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _F, _F, _F, _F, _I, _P],
         "rocml_attention_prefill_fused": [_P, _I, _P, _F, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _I,
                                           _P, _I, _P, _P],
     },
@@ -1209,33 +1209,36 @@ def decode_chain_max_layers() -> int:
 
 def decode_chain_splits(pages: int) -> int:
     """Splits of the key range in ``decode_chain`` for a block table of ``pages`` pages: a block asks for two pages before it
-    waits for anything.  It depends on the step's shape only, so a recorded step can be replayed as the sequences grow."""
+    waits for anything, and a second turn costs less than a merge.  It depends on the step's shape only, so a recorded step can be
+    replayed as the sequences grow."""
     return 1 if pages <= 4 else min(64, (pages + 1) // 2)
 
 
 def decode_chain_pays(layer: ChainLayer, rows: int) -> bool:
     """Whether the library's own rule says that ``decode_chain`` is the faster way for such layers and so many sequences."""
-    return bool(library("attention").rocml_decode_chain_pays(rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter))
+    return bool(library("attention").rocml_decode_chain_pays(
+        _code(layer.w_qkv), rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter))
 
 
 def decode_chain_words(layer: ChainLayer, rows: int, n_layers: int) -> int:
     """64-bit words of state a chain of ``n_layers`` such layers needs for ``rows`` tokens (one per sequence); 0: not taken."""
     return library("attention").rocml_decode_chain_words(
-        rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter, n_layers,
+        _code(layer.w_qkv), rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter, n_layers,
         decode_chain_splits(layer.block_table.shape[1]))
 
 
 def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer], token_pos: torch.Tensor, cos: torch.Tensor,
                  sin: torch.Tensor, state: torch.Tensor, max_len: int = 0) -> None:
     """The layers of a decode step, one token per sequence, in one launch: ``x [rows, hidden]`` (32-bit) passes through them,
-    the new keys and values are appended.  ``xn``: the first layer's normed input in bfloat16.  ``state`` (int64) starts as
+    the new keys and values are appended.  ``xn``: the first layer's normed input in the compute type (bfloat16 or float32).  ``state`` (int64) starts as
     zeros and is the caller's to keep from call to call; launches that share it run one after the other.  ``max_len`` is what
     ``--profile`` prices the call with."""
     first = layers[0]
     rows, hidden = x.shape
     _dev(x, xn, token_pos, cos, sin, state, first.block_table)
     _want(x, torch.float32, "residual stream")
-    _want(xn, torch.bfloat16, "normed operand")
+    dtype = first.w_qkv.dtype
+    _want(xn, dtype, "normed operand")
     _want(state, torch.int64, "state")
     _want(token_pos, torch.int32, "positions")
     _want(first.block_table, torch.int32, "block table")
@@ -1252,7 +1255,7 @@ def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer]
             raise KernelError("the layers of a decode chain must agree in sizes, constants and tables")
         for w, shape in ((c.w_qkv, (n_qkv, hidden)), (c.w_o, (hidden, c.n_heads * CHAIN_HEAD_DIM)),
                          (c.w_gate_up, (2 * c.inter, hidden)), (c.w_down, (hidden, c.inter))):
-            _want(w, torch.bfloat16, "weight")
+            _want(w, dtype, "weight")
             if tuple(w.shape) != shape:
                 raise KernelError(f"decode chain: a weight is {tuple(w.shape)}, not {shape}")
         for gain, n in ((c.q_gain, CHAIN_HEAD_DIM), (c.k_gain, CHAIN_HEAD_DIM), (c.mix_gain, hidden), (c.ffn_gain, hidden)):
@@ -1261,7 +1264,7 @@ def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer]
                 raise KernelError(f"decode chain: a gain has {gain.numel()} values, not {n}")
         pages = (c.k_cache.shape[0], c.n_kv_heads)
         for t, shape in ((c.k_cache, pages + (CHAIN_PAGE, CHAIN_HEAD_DIM)), (c.v_cache, pages + (CHAIN_HEAD_DIM, CHAIN_PAGE))):
-            _want(t, torch.bfloat16, "cache")
+            _want(t, dtype, "cache")
             if tuple(t.shape) != shape:
                 raise KernelError(f"decode chain: a cache is {tuple(t.shape)}, not {shape}")
         following = layers[i + 1].mix_gain if i + 1 < len(layers) else None
@@ -1270,7 +1273,7 @@ def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer]
         for j, t in enumerate(operands):
             pointers[CHAIN_POINTERS * i + j] = _ptr(t)
     _check("attention", library("attention").rocml_decode_chain(
-        _ptr(state), state.numel(), _ptr(x), _ptr(xn), pointers, len(layers), rows, hidden, first.n_heads, first.n_kv_heads,
+        _code(first.w_qkv), _ptr(state), state.numel(), _ptr(x), _ptr(xn), pointers, len(layers), rows, hidden, first.n_heads, first.n_kv_heads,
         CHAIN_HEAD_DIM, first.inter, _ptr(first.block_table), first.block_table.shape[1], _ptr(token_pos), _ptr(cos), _ptr(sin),
         first.scale, first.qk_eps, first.mix_eps, first.ffn_eps, decode_chain_splits(first.block_table.shape[1]), _stream()))
 

@@ -241,9 +241,9 @@ class Attention(Mixer):
 
     def chain_operands(self, step, cache) -> Optional[dict]:
         """What ``ops.decode_chain`` needs of this attention, or None where the layer or the step is not one it takes: one token
-        per sequence, bfloat16, heads of 128 with norms of their own and a rotation of the whole head, every key seen."""
+        per sequence, heads of 128 with norms of their own and a rotation of the whole head, every key seen."""
         s = self.spec
-        if (not self._fused_decode(step) or self.extras or s.bias or self.o_bias or s.window is not None or s.qk_norm is None
+        if (step.max_new != 1 or self.separate_q or self.extras or self.v_head_dim != s.head_dim or self.pairing != "halves" or s.bias or self.o_bias or s.window is not None or s.qk_norm is None
                 or s.head_dim != ops.CHAIN_HEAD_DIM or self.position is None or self.position.rot_dim != s.head_dim
                 or getattr(cache, "parts", None) is not None or step.n_tokens != step.n_seqs):
             return None

@@ -67,7 +67,7 @@ class GatedMlp(FeedForward):
 
     def chain_operands(self, step) -> Optional[dict]:
         """What ``ops.decode_chain`` needs of this feed-forward, or None where it is not one it takes."""
-        if not self.fused or self.epilogue != "swiglu" or self.dtype != torch.bfloat16:
+        if not self.fused or self.epilogue != "swiglu":
             return None
         return {"w_gate_up": self.w_gate_up, "w_down": self.w_down}
 
