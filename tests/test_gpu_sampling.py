@@ -2,6 +2,8 @@
 out plainly here: penalty, greedy on temperature <= 0, temperature, top-k, softmax, top-p,
 draw.  Its own tests fix the cases: temperature 0 and top_k = 1 are argmax, draws stay inside
 the top-k set and the nucleus, a seed repeats its draws (rocml/src/sample.rs:214-295)."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -133,6 +135,32 @@ def test_small_top_k_on_slices_of_the_row(vocab, params):
         t = u * cum[-1]
         assert cum[tok] - p[tok] - 1e-4 * cum[-1] <= t <= cum[tok] + 1e-4 * cum[-1], (u, tok)
     assert len(set(got)) <= params.top_k
+
+
+@pytest.mark.parametrize("k", [5, 6, 20, 63, 64])
+@pytest.mark.parametrize("row", ["random", "descending", "equal", "two values", "three finite", "infinite"])
+def test_slices_hand_out_the_same_candidates_as_the_whole_row(row, k):
+    """The candidates of the slice kernels, whose waves rank a few values at once or select one after the other (from k of 6 and
+    up to 63, and with not too many values at the bound), at rows of ties and of few finite values: with a nucleus of everything
+    and hardly any difference in probability, draws over evenly spread uniform numbers meet every candidate and no other."""
+    vocab, batch = 9000, 256
+    g = torch.Generator().manual_seed(11)
+    x = torch.randn(vocab, generator=g)
+    if row == "descending":
+        x = x.sort(descending=True).values
+    elif row == "equal":
+        x = torch.full((vocab,), 0.25)
+    elif row == "two values":
+        x = (torch.arange(vocab) % 7 == 3).float()
+    elif row == "three finite":
+        x = torch.full((vocab,), -math.inf)
+        x[[5000, 17, 8999]] = torch.tensor([0.5, 0.25, 0.5])
+    elif row == "infinite":
+        x[torch.randperm(vocab, generator=g)[:8500]] = -math.inf
+    order = sorted((i for i in range(vocab) if x[i] > -math.inf), key=lambda i: (-float(x[i]), i))[:k]
+    got = _draw(x.expand(batch, vocab).contiguous(), [SamplingParams(temperature=500.0, top_k=k)] * batch,
+                [(i + 0.5) / batch for i in range(batch)])
+    assert set(got) == set(order)
 
 
 def test_ties_at_the_kth_value_keep_the_lowest_ids():
