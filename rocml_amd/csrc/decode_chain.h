@@ -1,5 +1,5 @@
-// A decode step's layers in one launch (gfx950, wave64, bfloat16 and 32-bit): q/k/v projection, attention over the paged cache, output
-// projection, gated feed-forward, layer after layer, for one to four sequences of a model with small layers.
+// A decode step's layers in one launch (gfx950, wave64, bfloat16 and 32-bit): q/k/v projection, attention over the paged cache,
+// output projection, gated feed-forward, layer after layer, for one to four sequences of a model with small layers.
 //
 // What bounds it, and why it is one launch.  With a few rows of activations every product is a walk over its weights, and a
 // step used to be five or six dependent kernels a layer.  A kernel that follows another starts with nothing on its way to it:
@@ -28,8 +28,8 @@
 // wait last for seconds all the same, it ends, and the step's result is NaN.
 //
 // The algebra is that of the kernels the step otherwise runs (gemm_kpar_kernel, gemm_residual_prescale_kernel,
-// attn_decode_mfma_kernel FUSED; gemm_f32_rows_kernel, attn_f32_token_kernel): 32-bit sums, the residual stream in 32 bits, the norm's scale
-// applied by the consumer of bfloat16(x * gain), partial results of key splits merged in split order.
+// attn_decode_mfma_kernel FUSED; gemm_f32_rows_kernel, attn_f32_token_kernel): 32-bit sums, the residual stream in 32 bits, the
+// norm's scale applied by the consumer of bfloat16(x * gain), partial results of key splits merged in split order.
 #pragma once
 #include "attention_f32.h"
 #include "attention_mfma.h"
@@ -42,12 +42,13 @@ constexpr int DC_MAX_ROWS = 4;
 constexpr int DC_SHARDS = 8, DC_LINE = 16;      // ticket counters, 64-bit words between two of them (a line)
 constexpr int DC_D = 128;               // head size
 constexpr int DC_MAX_GROUP = 8;
-constexpr int DC_GROUP = 4;             // steps of K (32 wide) asked for together
-constexpr int DC_SHORT = 6, DC_LONG = 6;        // such groups on their way: a wave's whole share of a short K; of a longer one
+constexpr int DC_GROUP = 4;             // loads of 16 bytes a lane asked for together
+constexpr int DC_RING = 6;              // such groups on their way
 constexpr int DC_TILE = 16;             // weight rows of a tile
 constexpr int DC_MAX_TILES = 3;         // tiles of a block whose K is short
 constexpr int DC_MAX_LDS = 128 << 10;
-constexpr int DC_APART = 8;             // words between two tiles' sums of squares (side by side sixteen blocks write one line that all ask for: 24 against 20 us a layer)
+// words between two tiles' sums of squares (side by side, sixteen blocks write one line that all ask for: 24 against 20 us a layer)
+constexpr int DC_APART = 8;
 constexpr int DC_PAD = 64;              // bytes between two rows of activations in LDS
 constexpr u64 DC_PATIENCE = 400000000ull;       // ticks of 10 ns after which a wait gives up
 
@@ -136,9 +137,10 @@ __device__ __forceinline__ bool dc_give_up(u64* state, int tries, u64& since) {
     return true;
 }
 
-// N words a lane at the addresses that at(i, offset) gives, all of them of this epoch when it returns.  The whole wave stays until the
-// last one is there.
 __device__ __forceinline__ const u64* dc_at(const u64* base, uint32_t bytes) { return (const u64*)((const char*)base + bytes); }
+
+// N words a lane at the addresses that at(i, offset) gives, all of them of this epoch when it returns.  The whole wave stays
+// until the last one is there.
 template <int N, typename At>
 __device__ __forceinline__ void dc_collect(u64* state, uint32_t epoch, bool mine, uint32_t offset, At at, uint32_t (&v)[N]) {
     u64 w[N], since = 0;
@@ -160,8 +162,8 @@ __device__ __forceinline__ void dc_collect(u64* state, uint32_t epoch, bool mine
     for (int i = 0; i < N; ++i) v[i] = (uint32_t)w[i];
 }
 
-// A wave (the block's first) waits until one word of an earlier stage's result is there, one lane asking now and then: until then nothing of what
-// it waits for is near, and hundreds of blocks that ask for all their words all the time are in each other's way.
+// The block's first wave waits until one word of an earlier stage's result is there, asking now and then: until then nothing of
+// what it waits for is near, and hundreds of blocks that ask for all their words all the time are in each other's way.
 __device__ __forceinline__ void dc_far_wait(u64* state, const u64* word, uint32_t epoch) {
     u64 since = 0;
     for (int tries = 1; (uint32_t)(__builtin_amdgcn_readfirstlane((int)(dc_load(word) >> 32))) != epoch; ++tries) {
@@ -256,8 +258,7 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
     const int k = dc_k(p, stage), share = k / W, first = wave * share, groups = share / (T::STEP * DC_GROUP);
     auto strip = ga_buffer(w + (size_t)tile0 * DC_TILE * k, (long long)tiles * DC_TILE * k * SIZE);
     const uint32_t at = (uint32_t)(col * k + first) * SIZE + g * 16u;
-    constexpr int RING = SHORT ? DC_SHORT : DC_LONG;
-    dc_u32x4_t ring[RING][DC_GROUP];
+    dc_u32x4_t ring[DC_RING][DC_GROUP];
     auto request = [&](int r, int group, int tile) {
         uint32_t from = group < groups && tile < tiles ? at : BUF_NOWHERE;
         uint32_t behind = (uint32_t)(tile * DC_TILE * k) * SIZE + group * (DC_GROUP * 64);
@@ -268,7 +269,7 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
     {
         int group = 0, tile = 0;
 #pragma unroll
-        for (int r = 0; r < RING; ++r) {
+        for (int r = 0; r < DC_RING; ++r) {
             request(r, group, tile);
             if (++group == groups && SHORT) { group = 0; ++tile; }
         }
@@ -358,7 +359,7 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
     if constexpr (SHORT) {
         int group = 0, tile = 0;
 #pragma unroll
-        for (int r = 0; r < RING; ++r) {
+        for (int r = 0; r < DC_RING; ++r) {
             if (tile < tiles) {
                 multiply(r, group);
                 if (++group == groups) {
@@ -369,11 +370,11 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
             }
         }
     } else {
-        for (int g0 = 0; g0 < groups; g0 += RING) {
+        for (int g0 = 0; g0 < groups; g0 += DC_RING) {
 #pragma unroll
-            for (int r = 0; r < RING; ++r) {
+            for (int r = 0; r < DC_RING; ++r) {
                 if (g0 + r < groups) multiply(r, g0 + r);
-                request(r, g0 + r + RING, 0);
+                request(r, g0 + r + DC_RING, 0);
             }
         }
         hand_over(0);
@@ -833,7 +834,7 @@ __global__ void __launch_bounds__(64 * W) decode_chain_kernel(const DcArgs a) {
         const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
         if (it.stage == DC_ATTN) dc_attention<E, W>(a, ly, it, sm, tickets, turn, wave, lane);
         else if (it.stage == DC_MERGE) dc_merge<E, W>(a, it, sm, tickets, turn, wave, lane);
-        else if (dc_tiles(p, it.stage) * dc_k(p, it.stage) <= DC_SHORT * DC_GROUP * DcType<E>::STEP * W)
+        else if (dc_tiles(p, it.stage) * dc_k(p, it.stage) <= DC_RING * DC_GROUP * DcType<E>::STEP * W)
             dc_product<E, W, M, true>(a, ly, it, sm, tickets, turn, wave, lane);
         else dc_product<E, W, M, false>(a, ly, it, sm, tickets, turn, wave, lane);
     }
@@ -858,7 +859,7 @@ static bool dc_plan(DcPlan& p, int dtype, int rows, int hidden, int hq, int hkv,
     auto tiles = [&](int n_tiles) {
         const int groups = hidden / unit;
         for (int t = DC_MAX_TILES; t > 1; --t)
-            if (t * groups <= DC_SHORT && n_tiles % t == 0) return t;
+            if (t * groups <= DC_RING && n_tiles % t == 0) return t;
         return 1;
     };
     p.qkv_tiles = tiles(p.n_qkv / DC_TILE);
