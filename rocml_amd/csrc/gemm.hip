@@ -511,7 +511,7 @@ static int prescale_waves(int k) {
 // every 16 columns of a row (see gemm_residual_prescale_kernel).
 ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void* w, int ldw, float* resid, int ldr,
                                               const float* gain, void* xg, int ldg, float* ssq, int m, int n, int k,
-                                              int waves, hipStream_t stream) {
+                                              int waves, const float* bias, hipStream_t stream) {
     ROCML_REQUIRE(m >= 0 && n > 0 && k > 0, "gemm_residual_prescale: bad sizes M=%d N=%d K=%d", m, n, k);
     ROCML_REQUIRE(m <= 16, "gemm_residual_prescale: at most 16 rows, got %d", m);
     ROCML_REQUIRE(ldx >= k && ldw >= k && ldr >= n && ldg >= n, "gemm_residual_prescale: row strides (%d, %d, %d, %d) too small",
@@ -519,8 +519,8 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
     ROCML_REQUIRE(k % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0,
                   "gemm_residual_prescale: K and the operands' row strides must be multiples of 8 and the pointers "
                   "16-byte aligned (K=%d ldx=%d ldw=%d)", k, ldx, ldw);
-    ROCML_REQUIRE((uintptr_t)resid % 16 == 0 && (uintptr_t)gain % 16 == 0 && (uintptr_t)xg % 8 == 0,
-                  "gemm_residual_prescale: the residual stream, the gain and the prepared operand must be aligned");
+    ROCML_REQUIRE((uintptr_t)resid % 16 == 0 && (uintptr_t)gain % 16 == 0 && (uintptr_t)xg % 8 == 0 && (uintptr_t)bias % 16 == 0,
+                  "gemm_residual_prescale: the residual stream, the gain, the bias and the prepared operand must be aligned");
     ROCML_REQUIRE(resid && gain && xg && ssq, "gemm_residual_prescale: null pointer");
     if (m == 0) return 0;
     int tiles = ceil_div(n, 16);
@@ -530,7 +530,7 @@ ROCML_EXPORT int rocml_gemm_residual_prescale(const void* x, int ldx, const void
     const bool one = round_up(ceil_div(k, waves), 32) <= 256;
 #define GRP_LAUNCH(W_, ...)                                                                                     \
     gemm_residual_prescale_kernel<W_, __VA_ARGS__><<<tiles, 64 * W_, 0, stream>>>((const bf16_t*)x, ldx, (const bf16_t*)w, ldw, resid, \
-                                                                     ldr, gain, (bf16_t*)xg, ldg, ssq, tiles, m, n, k)
+                                                                     ldr, gain, (bf16_t*)xg, ldg, ssq, tiles, m, n, k, bias)
     if (ldx >= NEAR_STRIDE || ldw >= NEAR_STRIDE) GRP_LAUNCH(4, false, true);
     else if (waves == 16) { if (one) GRP_LAUNCH(16, true); else GRP_LAUNCH(16, false); }
     else if (waves == 12) { if (one) GRP_LAUNCH(12, true); else GRP_LAUNCH(12, false); }

@@ -839,13 +839,14 @@ gemm_kpar_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict
 // multiplies them by 1 / sqrt(sum of ssq[row] / N + eps): the norm's scale is one number per row
 // and commutes with the product.  A decode step of a few sequences is priced by the kernels that
 // follow one another, not by bytes; this takes two norms out of every layer.
+// bias (or null): a number per column, added to the stream first.
 // ONE: a wave's share of K is at most one chunk of 256, so everything is asked for in one trip and half the registers do
 // (which sixteen waves a block need).
 template <int WAVES, bool ONE, bool FAR = false>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_t* __restrict__ w, int ldw,
                               float* resid, int ldr, const float* __restrict__ gain, bf16_t* __restrict__ xg, int ldg,
-                              float* __restrict__ ssq, int tiles, int m, int n, int k) {
+                              float* __restrict__ ssq, int tiles, int m, int n, int k, const float* __restrict__ bias) {
     __shared__ float red[WAVES][64][4];
     int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int g = lane >> 4, col = lane & 15;
@@ -872,6 +873,10 @@ gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_
     if (wave == 0 && vec) {
         r_old = *(const float4*)(resid + (size_t)col * ldr + n0);
         gn = *(const float4*)(gain + n0);
+        if (bias) {                             // (a kernel of its own for it takes 4.8 us)
+            const float4 b = *(const float4*)(bias + n0);
+            r_old.x += b.x; r_old.y += b.y; r_old.z += b.z; r_old.w += b.w;
+        }
         asm volatile("" ::: "memory");          // (the loads stay here)
     }
     __builtin_amdgcn_sched_barrier(0);          // (and so do the operands': sunk to their products they arrive one by one)
@@ -918,7 +923,7 @@ gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             if (n0 + e >= n) continue;
-            float r = resid[(size_t)col * ldr + n0 + e] + v[e];
+            float r = resid[(size_t)col * ldr + n0 + e] + (bias ? bias[n0 + e] : 0.f) + v[e];
             resid[(size_t)col * ldr + n0 + e] = r;
             xg[(size_t)col * ldg + n0 + e] = f32_to_bf16(r * gain[n0 + e]);
             ss = fmaf(r, r, ss);

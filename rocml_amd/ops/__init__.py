@@ -80,7 +80,7 @@ _SIGNATURES = {
         "rocml_splitk_reduce": [_P, _P, _I, _I, _I, _I, _I, _I, _P],
         "rocml_gemm_batched": [_P, _I, _I, _LL, _P, _I, _I, _LL, _P, _I, _I, _LL, _I, _I, _I, _I, _P, _I, _LL, _I, _P],
         "rocml_gemm_residual_prescale_pays": [_I, _I, _I],
-        "rocml_gemm_residual_prescale": [_P, _I, _P, _I, _P, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P],
+        "rocml_gemm_residual_prescale": [_P, _I, _P, _I, _P, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P, _P],
     },
     "attention": {
         "rocml_attention": [_P, _P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I,
@@ -867,12 +867,16 @@ def gemm_residual_prescale_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def gemm_residual_prescale(x: torch.Tensor, w: torch.Tensor, resid: torch.Tensor, gain: torch.Tensor,
-                           xg: torch.Tensor, ssq: torch.Tensor, waves: int = 0) -> None:
-    """``resid += x @ w.T`` (whole sums, at most 16 rows of bfloat16 operands) and, for the norm
+                           xg: torch.Tensor, ssq: torch.Tensor, waves: int = 0, bias: Optional[torch.Tensor] = None) -> None:
+    """``resid += x @ w.T`` (and ``bias``, float32, one number per column, if given; whole sums, at most 16 rows of bfloat16 operands) and, for the norm
     with ``gain`` that reads ``resid`` next: ``xg = bfloat16(resid * gain)`` and ``ssq[row][j]`` =
     the sum of squares of columns ``16 j .. 16 j + 15`` of the row.  The norm's output is
     ``xg * (1 / sqrt(ssq[row].sum() / N + eps))``; the scale commutes with the next product."""
-    _dev(gain, ssq)
+    _dev(gain, ssq, bias)
+    if bias is not None:
+        _want(bias, torch.float32, "bias")
+        if bias.numel() != w.shape[0]:
+            raise KernelError(f"the bias has {bias.numel()} numbers for {w.shape[0]} columns")
     for t in (x, w, resid, xg):
         if not t.is_cuda:
             raise KernelError("kernel arguments must be GPU tensors; this library has no CPU path")
@@ -892,7 +896,7 @@ def gemm_residual_prescale(x: torch.Tensor, w: torch.Tensor, resid: torch.Tensor
                           f"prepared {tuple(xg.shape)}, gain {gain.numel()}, sums {tuple(ssq.shape)} (need {(m, tiles)})")
     _check("gemm", library("gemm").rocml_gemm_residual_prescale(
         _ptr(x), max(x.stride(0), k), _ptr(w), w.stride(0), _ptr(resid), max(resid.stride(0), n), _ptr(gain), _ptr(xg),
-        max(xg.stride(0), n), _ptr(ssq), m, n, k, waves, _stream()))
+        max(xg.stride(0), n), _ptr(ssq), m, n, k, waves, _ptr(bias), _stream()))
 
 
 def splitk_reduce(partials: torch.Tensor, out: torch.Tensor, accumulate: bool = False) -> None:

@@ -358,10 +358,7 @@ class Attention(Mixer):
                               softcap=self.softcap, keep_first=self.keep_first)
         if s.gate:
             ops.sigmoid_gate(o, qkv[:, rows - self.g_dim:rows], group=self.v_head_dim if self.gate_per_head else 1)
-        if self.b_o is not None:
-            ws.flush_pending()
-            ops.add_row_vector(x_accum, self.b_o)
-        stream(step).add_product(o, self.w_o, x_accum)
+        stream(step).add_product(o, self.w_o, x_accum, bias=self.b_o)
 
 
 register_mixer("attention", Attention)

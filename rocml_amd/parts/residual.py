@@ -41,26 +41,31 @@ class ResidualStream:
         self.defer_overwrite = False
         self._prescaled = None
 
-    def add_product(self, a: torch.Tensor, w: torch.Tensor, target: torch.Tensor) -> None:
-        """``target += a @ w.T``.  The product may leave partial sums to the next norm
+    def add_product(self, a: torch.Tensor, w: torch.Tensor, target: torch.Tensor, bias: Optional[torch.Tensor] = None) -> None:
+        """``target += a @ w.T`` and ``bias`` (one 32-bit number per column) if given.  The product may leave partial sums to the next norm
         (``workspace.take_pending``), or have prepared that norm (``take_prescaled``)."""
         ws = self.workspace
         hint = self.next_norm
         self._prescaled = None
+        prepares = not self.overwrite and hint is not None and target.dtype == torch.float32 and hint.width == target.shape[1] \
+            and ops.gemm_residual_prescale_pays(a, w)
+        if bias is not None and (not prepares or bias.data_ptr() % 16 != 0):
+            ws.flush_pending()
+            ops.add_row_vector(target, bias)
+            bias = None
         if self.overwrite:
             ws.flush_pending()
             splits = ops.gemm(a, w, target, accumulate=False, workspace=ws.scratch(), defer=self.defer_overwrite)
             if splits:
                 ws.set_pending(target, splits, replace=True)
             return
-        if hint is not None and target.dtype == torch.float32 and hint.width == target.shape[1] \
-                and ops.gemm_residual_prescale_pays(a, w):
+        if prepares:
             ws.flush_pending()
             rows = target.shape[0]
             xg = ws.get("residual.prepared", tuple(target.shape), torch.bfloat16)
             parts = (target.shape[1] + ops.PRESCALE_TILE - 1) // ops.PRESCALE_TILE
             ssq = ws.get("residual.ssq", (rows, parts), torch.float32)
-            ops.gemm_residual_prescale(a, w, target, hint.gain, xg, ssq)
+            ops.gemm_residual_prescale(a, w, target, hint.gain, xg, ssq, bias=bias)
             self._prescaled = (target.data_ptr(), hint.gain.data_ptr(), xg, ops.RowScale(ssq, hint.eps, hint.width))
             return
         splits = ops.gemm(a, w, target, accumulate=True, workspace=ws.scratch(), defer=True)

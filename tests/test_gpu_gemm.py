@@ -382,6 +382,25 @@ def test_residual_sum_that_prepares_the_next_norm(m, n, k, waves):
                                    torch.zeros(17, n, dtype=torch.bfloat16, device="cuda"), torch.zeros(17, tiles, device="cuda"))
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 64, 64), (3, 102, 72), (8, 4096, 1032), (16, 130, 4096)])
+def test_residual_sum_with_a_bias(m, n, k):
+    """The bias is added to the stream in 32 bits before the product's sums: rows and columns in whole tiles and not (the
+    element-by-element end), against the sum in 64 bits."""
+    x, w = _operands(m, n, k, torch.bfloat16, 7)
+    g = torch.Generator().manual_seed(8)
+    base, bias = torch.randn(m, n, generator=g), torch.randn(n, generator=g)
+    gain = 1 + 0.2 * torch.randn(n, generator=g)
+    resid = base.cuda()
+    xg = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    ssq = torch.empty(m, (n + 15) // 16, device="cuda")
+    ops.gemm_residual_prescale(x, w, resid, gain.cuda(), xg, ssq, bias=bias.cuda())
+    want = base.double() + bias.double() + _ref(x, w).cpu()
+    assert float((resid.double().cpu() - want).abs().max()) < 2e-5 * max(1.0, float(want.abs().max()))
+    assert float((ssq.double().sum(-1).cpu() - (want ** 2).sum(-1)).abs().max()) < 1e-5 * float((want ** 2).sum(-1).max())
+    with pytest.raises(KernelError):
+        ops.gemm_residual_prescale(x, w, resid, gain.cuda(), xg, ssq, bias=torch.zeros(n + 1, device="cuda"))
+
+
 @pytest.mark.parametrize("m,n,k,pays", [(1, 2048, 4096, True), (4, 2048, 6144, True), (1, 2048, 6152, False), (4, 2560, 8192, False),
                                         (4, 3072, 8192, True), (5, 3072, 8192, False), (8, 4096, 12288, True), (1, 4112, 4096, False)])
 def test_when_the_prepared_norm_pays(m, n, k, pays):
