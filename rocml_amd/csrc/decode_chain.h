@@ -930,6 +930,7 @@ ROCML_EXPORT int rocml_decode_chain(int dtype, void* state, long long state_word
     for (int i = 0; i < n_layers; ++i) {
         const void* const* f = layers + 10 * i;
         for (int j = 0; j < 10; ++j) ROCML_REQUIRE(f[j] || (j == 7 && i == n_layers - 1), "decode_chain: layer %d lacks operand %d", i, j);
+        for (int j : {0, 1, 2, 3, 8, 9}) ROCML_REQUIRE((uintptr_t)f[j] % 16 == 0, "decode_chain: operand %d of layer %d is not aligned", j, i);
         a.layer[i] = DcLayer{f[0], f[1], f[2], f[3], (const float*)f[4], (const float*)f[5], (const float*)f[6], (const float*)f[7],
                              (void*)f[8], (void*)f[9]};
     }

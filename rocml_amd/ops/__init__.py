@@ -1199,6 +1199,17 @@ class ChainLayer:
     def inter(self) -> int:
         return self.w_down.shape[1]
 
+    def matrices(self):
+        return [w for w in (self.w_qkv, self.w_o, self.w_gate_up, self.w_down) if w is not None]
+
+    def lies_in_order(self) -> bool:
+        """Whether every operand lies whole and aligned in memory, as the chain's 16-byte loads take it; the layer's own kernels
+        take strided rows and other addresses too."""
+        gains = (self.q_gain, self.k_gain, self.mix_gain, self.ffn_gain)
+        return (all(t.is_contiguous() for t in (*self.matrices(), *gains, self.k_cache, self.v_cache, self.block_table))
+                and all(t.data_ptr() % 16 == 0 for t in (*self.matrices(), self.k_cache, self.v_cache))
+                and all(w.dtype == self.k_cache.dtype == self.v_cache.dtype for w in self.matrices()))
+
     def fits_behind(self, other: "ChainLayer") -> bool:
         """Whether this layer may follow ``other`` in one launch: the sizes, constants and tables of both are the same."""
         return (self.hidden == other.hidden and self.inter == other.inter and self.n_heads == other.n_heads
@@ -1219,8 +1230,9 @@ def decode_chain_splits(pages: int) -> int:
 
 
 def decode_chain_pays(layer: ChainLayer, rows: int) -> bool:
-    """Whether the library's own rule says that ``decode_chain`` is the faster way for such layers and so many sequences."""
-    return bool(library("attention").rocml_decode_chain_pays(
+    """Whether ``decode_chain`` takes the layer as it lies, and the library's own rule says that it is the faster way for such
+    layers and so many sequences."""
+    return layer.lies_in_order() and bool(library("attention").rocml_decode_chain_pays(
         _code(layer.w_qkv), rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter))
 
 

@@ -239,13 +239,18 @@ class Attention(Mixer):
             return 0
         return ops.decode_splits(step.n_tokens * self.spec.n_kv_heads, self.n_cus, min(cache.block_table.shape[1], 64))
 
+    def may_chain(self) -> bool:
+        """Whether there are steps in which ``chain_operands`` gives an answer."""
+        s = self.spec
+        return not (self.separate_q or self.extras or self.v_head_dim != s.head_dim or self.pairing != "halves" or s.bias or self.o_bias
+                    or s.window is not None or s.qk_norm is None or s.head_dim != ops.CHAIN_HEAD_DIM or self.position is None
+                    or self.position.rot_dim != s.head_dim)
+
     def chain_operands(self, step, cache) -> Optional[dict]:
         """What ``ops.decode_chain`` needs of this attention, or None where the layer or the step is not one it takes: one token
         per sequence, heads of 128 with norms of their own and a rotation of the whole head, every key seen."""
         s = self.spec
-        if (step.max_new != 1 or self.separate_q or self.extras or self.v_head_dim != s.head_dim or self.pairing != "halves" or s.bias or self.o_bias or s.window is not None or s.qk_norm is None
-                or s.head_dim != ops.CHAIN_HEAD_DIM or self.position is None or self.position.rot_dim != s.head_dim
-                or getattr(cache, "parts", None) is not None or step.n_tokens != step.n_seqs):
+        if step.max_new != 1 or step.n_tokens != step.n_seqs or not self.may_chain() or getattr(cache, "parts", None) is not None:
             return None
         if cache.k.dtype != self.dtype or cache.k.shape[2] != ops.CHAIN_PAGE or self.w_qkv.shape[0] != self.q_dim + 2 * self.kv_dim:
             return None

@@ -119,11 +119,17 @@ class PreNormBlock(ConvInput, Part):
             return None               # the convolution needs the normed rows themselves
         return self._hint(step, self.mixer_norm, self.mixer)
 
+    def may_chain(self) -> bool:
+        """Whether there are steps in which ``chain_layer`` gives an answer."""
+        return (self.input_conv is None and all(hasattr(n, "prescale_hint") for n in (self.mixer_norm, self.ffn_norm))
+                and all(hasattr(part, "may_chain") and part.may_chain() for part in (self.mixer, self.ffn)))
+
     def chain_layer(self, step, cache):
         """This layer as ``ops.decode_chain`` runs it in a step, or None if it or the step is not one the chain takes."""
-        parts = (self.mixer, self.ffn)
-        norms = [n.prescale_hint() if hasattr(n, "prescale_hint") else None for n in (self.mixer_norm, self.ffn_norm)]
-        if self.input_conv is not None or None in norms or not all(hasattr(part, "chain_operands") for part in parts):
+        if not self.may_chain():
+            return None
+        norms = [n.prescale_hint() for n in (self.mixer_norm, self.ffn_norm)]
+        if None in norms:
             return None
         mixer, ffn = self.mixer.chain_operands(step, cache), self.ffn.chain_operands(step)
         if mixer is None or ffn is None:

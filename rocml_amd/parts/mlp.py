@@ -65,9 +65,12 @@ class GatedMlp(FeedForward):
         # the gated epilogue of the few-rows products applies it
         return self.w_gate_up is not None and self.fused and self.dtype == torch.bfloat16 and step.n_tokens <= ops.ROW_SCALE_MAX_ROWS
 
+    def may_chain(self) -> bool:
+        return self.fused and self.epilogue == "swiglu"
+
     def chain_operands(self, step) -> Optional[dict]:
         """What ``ops.decode_chain`` needs of this feed-forward, or None where it is not one it takes."""
-        if not self.fused or self.epilogue != "swiglu":
+        if not self.may_chain():
             return None
         return {"w_gate_up": self.w_gate_up, "w_down": self.w_down}
 

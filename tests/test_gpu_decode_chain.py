@@ -167,5 +167,14 @@ def test_what_the_chain_does_not_take():
         many = _model(512, 4, 4, 512, 1, [5] * 5, 1, seed=4)
         ops.decode_chain(many[1], many[1].bfloat16(), many[0], many[4], many[2], many[3], state)
     assert ops.decode_chain_words(layers[0], 5, 1) == 0
+    layer = layers[0]                                       # operands that the layer's own kernels take and the chain's loads do not
+    assert ops.decode_chain_pays(layer, 1)
+    w = layer.w_o
+    layer.w_o = torch.empty(w.shape[0], w.shape[1] + 8, dtype=w.dtype, device=DEV)[:, :w.shape[1]]
+    assert not ops.decode_chain_pays(layer, 1)
+    layer.w_o = torch.empty(w.numel() + 1, dtype=w.dtype, device=DEV)[1:].view(w.shape)
+    assert not ops.decode_chain_pays(layer, 1)
+    with pytest.raises(ops.KernelError):
+        ops.decode_chain(x0, xn, [layer], pos, cos, sin, state)
     odd = _model(768, 6, 2, 768, 1, [5], 1, seed=4)[0][0]    # no whole groups of steps in a wave's share of K
     assert ops.decode_chain_words(odd, 1, 1) == 0 and not ops.decode_chain_pays(odd, 1)
