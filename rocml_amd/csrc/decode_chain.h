@@ -25,7 +25,8 @@
 // tickets.  The items are dealt over eight counters; of each counter's tickets the lowest unfinished one is held by a block that
 // runs and waits for nothing but finished items, or is the next that a running block draws.  That needs one running block for
 // each counter, which the first eight blocks of the grid are, and no block beside another whatever else the GPU runs.  Should a
-// wait last for seconds all the same, it ends, and the step's result is NaN.
+// wait last for seconds all the same, it ends, and the step's result is NaN: it leaves the launch's number as a mark, so that the
+// launch's other waits end too, while the next launch waits as if nothing had been.
 //
 // The algebra is that of the kernels the step otherwise runs (gemm_kpar_kernel, gemm_residual_prescale_kernel,
 // attn_decode_mfma_kernel FUSED; gemm_f32_rows_kernel, attn_f32_token_kernel): 32-bit sums, the residual stream in 32 bits, the
@@ -50,7 +51,8 @@ constexpr int DC_MAX_LDS = 128 << 10;
 // words between two tiles' sums of squares (side by side, sixteen blocks write one line that all ask for: 24 against 20 us a layer)
 constexpr int DC_APART = 8;
 constexpr int DC_PAD = 64;              // bytes between two rows of activations in LDS
-constexpr u64 DC_PATIENCE = 400000000ull;       // ticks of 10 ns after which a wait gives up
+constexpr long long DC_PATIENCE = 400000000ll;  // ticks of 10 ns after which a wait gives up
+constexpr int DC_POLLS = 256;                   // looks at a word between two looks at the clock and the mark
 
 // The compute type's ways.  bfloat16: two values a word of operands, 32 of K a load, scores in powers of two.  32-bit: one, 16,
 // natural exponentials, and products of 4x4x1 in sixteen blocks: a block is four weight rows and four rows of activations at one
@@ -101,7 +103,7 @@ struct DcLayer {
 };
 
 // Word offsets of the buffers in the state (64-bit words).  The first DC_SHARDS lines hold the ticket counters, the next one the
-// mark of a wait that gave up.
+// mark of a wait that gave up (dc_mark of its launch).
 struct DcPlan {
     int n_qkv, hq, hkv, hidden, inter, rows, splits, n_layers;
     int items[6], per_layer;            // work items of a layer's stages, in order
@@ -119,6 +121,8 @@ struct DcArgs {
     const int* pos;
     const float *cos_t, *sin_t;         // [rows, 64]
     float scale, qk_eps, eps_mix, eps_ffn, inv_width;
+    int between;                        // DC_POLLS - 1
+    long long patience;                 // DC_PATIENCE
     DcLayer layer[DC_LAYERS];
 };
 
@@ -127,13 +131,18 @@ __device__ __forceinline__ void dc_store(u64* p, uint32_t data, uint32_t epoch) 
     __hip_atomic_store(p, ((u64)epoch << 32) | data, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// A wait that has gone on for long: true when it has to end.
-__device__ __forceinline__ bool dc_give_up(u64* state, int tries, u64& since) {
-    if (tries & 255) return false;
+// What a launch leaves where a wait gave up, from the number that its words carry; never 0.
+__device__ __forceinline__ u64 dc_mark(uint32_t epoch) { return (epoch - 2u) / (uint32_t)DC_LAYERS + 1u; }
+
+// A wait that has gone on for long: true when it has to end, because this or another wait of the launch has lasted too long (a
+// mark that an earlier launch left does not count).
+__device__ __forceinline__ bool dc_give_up(const DcArgs& a, uint32_t epoch, int tries, u64& since) {
+    if (tries & a.between) return false;
+    u64* at = a.state + DC_SHARDS * DC_LINE;
     if (since == 0) since = wall_clock64();
-    if (dc_load(state + DC_SHARDS * DC_LINE) != 0) return true;
-    if (wall_clock64() - since < DC_PATIENCE) return false;
-    __hip_atomic_store(state + DC_SHARDS * DC_LINE, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (dc_load(at) == dc_mark(epoch)) return true;
+    if ((long long)(wall_clock64() - since) < a.patience) return false;
+    __hip_atomic_store(at, dc_mark(epoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
 }
 
@@ -142,7 +151,7 @@ __device__ __forceinline__ const u64* dc_at(const u64* base, uint32_t bytes) { r
 // N words a lane at the addresses that at(i, offset) gives, all of them of this epoch when it returns.  The whole wave stays
 // until the last one is there.
 template <int N, typename At>
-__device__ __forceinline__ void dc_collect(u64* state, uint32_t epoch, bool mine, uint32_t offset, At at, uint32_t (&v)[N]) {
+__device__ __forceinline__ void dc_collect(const DcArgs& a, uint32_t epoch, bool mine, uint32_t offset, At at, uint32_t (&v)[N]) {
     u64 w[N], since = 0;
     for (int tries = 1;; ++tries) {
         asm volatile("" : "+v"(offset));        // (the addresses are formed in every turn: they do not wait in registers)
@@ -152,7 +161,7 @@ __device__ __forceinline__ void dc_collect(u64* state, uint32_t epoch, bool mine
 #pragma unroll
         for (int i = 0; i < N; ++i) ok &= (uint32_t)(w[i] >> 32) == epoch;
         if (__all(ok || !mine)) break;
-        if (dc_give_up(state, tries, since)) {
+        if (dc_give_up(a, epoch, tries, since)) {
 #pragma unroll
             for (int i = 0; i < N; ++i) w[i] = 0x7fc07fc0u;         // NaN, as one 32-bit number and as two of 16
             break;
@@ -164,25 +173,25 @@ __device__ __forceinline__ void dc_collect(u64* state, uint32_t epoch, bool mine
 
 // The block's first wave waits until one word of an earlier stage's result is there, asking now and then: until then nothing of
 // what it waits for is near, and hundreds of blocks that ask for all their words all the time are in each other's way.
-__device__ __forceinline__ void dc_far_wait(u64* state, const u64* word, uint32_t epoch) {
+__device__ __forceinline__ void dc_far_wait(const DcArgs& a, const u64* word, uint32_t epoch) {
     u64 since = 0;
     for (int tries = 1; (uint32_t)(__builtin_amdgcn_readfirstlane((int)(dc_load(word) >> 32))) != epoch; ++tries) {
         __builtin_amdgcn_s_sleep(16);
-        if (dc_give_up(state, tries, since)) break;
+        if (dc_give_up(a, epoch, tries, since)) break;
     }
 }
 
 // 1 / sqrt(mean square of a row + eps) from the sums of squares of its tiles, of which the lane has added up its first two
 // already; every lane gets it
-__device__ __forceinline__ float dc_row_scale(u64* state, const u64* ssq, int tiles, uint32_t epoch, float inv_width, float eps, int lane,
+__device__ __forceinline__ float dc_row_scale(const DcArgs& a, const u64* ssq, int tiles, uint32_t epoch, float eps, int lane,
                                               int from = 0, float ss = 0.f) {
     for (int at = from + lane; at - lane < tiles; at += 64) {       // (a word every DC_APART)
         uint32_t v[1];
         bool mine = at < tiles;
-        dc_collect<1>(state, epoch, mine, mine ? at * (8u * DC_APART) : 0u, [&](int, uint32_t o) { return dc_at(ssq, o); }, v);
+        dc_collect<1>(a, epoch, mine, mine ? at * (8u * DC_APART) : 0u, [&](int, uint32_t o) { return dc_at(ssq, o); }, v);
         ss += mine ? __uint_as_float(v[0]) : 0.f;
     }
-    return 1.0f / sqrtf(wave_sum(ss) * inv_width + eps);
+    return 1.0f / sqrtf(wave_sum(ss) * a.inv_width + eps);
 }
 
 // A block's place in the order: {launch, ticket} of its counter.  A block draws until its ticket lies behind its counter's last
@@ -220,11 +229,11 @@ __device__ __forceinline__ int dc_k(const DcPlan& p, int stage) { return stage =
 // N rounds of 64 words of every row of operands (stride words apart) into LDS (pitch bytes apart), all asked for together.  SSQ:
 // with them the first two rounds of the rows' sums of squares.
 template <int M, int N, bool SSQ>
-__device__ __forceinline__ void dc_take(u64* st, uint32_t epoch, const u64* row, int stride, char* to, int pitch, const u64* ssq, int tiles,
+__device__ __forceinline__ void dc_take(const DcArgs& a, uint32_t epoch, const u64* row, int stride, char* to, int pitch, const u64* ssq, int tiles,
                                         int lane, float (&ss)[M]) {
     constexpr int E = SSQ ? 2 : 0;
     uint32_t v[M * (N + E)];
-    dc_collect<M * (N + E)>(st, epoch, true, lane * 8u, [&](int i, uint32_t o) {
+    dc_collect<M * (N + E)>(a, epoch, true, lane * 8u, [&](int i, uint32_t o) {
         const int m = i / (N + E), j = i % (N + E);
         return j < N ? dc_at(row + (size_t)m * stride + j * 64, o)
                      : dc_at(ssq + m * tiles * DC_APART, min(o + (j - N) * 512u, tiles * 8u - 8u) * DC_APART); }, v);
@@ -302,14 +311,14 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
         const u64* far = stage == DC_QKV ? st + p.h : stage == DC_O ? st + p.y : stage == DC_GU ? st + p.o : st + p.xga;
         const int n_far = stage == DC_QKV ? p.inter / V : stage == DC_O ? p.n_qkv : stage == DC_GU ? p.hq * DC_D / V : p.hidden / V;
         const uint32_t src_epoch = stage == DC_QKV ? epoch - 1 : epoch;
-        if (wave == 0) dc_far_wait(st, far + it.i * DC_LINE % n_far, src_epoch);
+        if (wave == 0) dc_far_wait(a, far + it.i * DC_LINE % n_far, src_epoch);
         __syncthreads();
         if (wave == W - 1 && lane == 0) drawn = tickets.draw();
         if (residual && wave == 0 && !(stage == DC_O && head)) {
             // (there before the operands are)
             uint32_t v[1];
             const u64* from = stage == DC_O ? st + p.xb : st + p.xa;
-            dc_collect<1>(st, stage == DC_O ? epoch - 1 : epoch, mine, mine ? (uint32_t)(orow * p.hidden + ocol) * 8u : 0u,
+            dc_collect<1>(a, stage == DC_O ? epoch - 1 : epoch, mine, mine ? (uint32_t)(orow * p.hidden + ocol) * 8u : 0u,
                           [&](int, uint32_t o) { return dc_at(from, o); }, v);
             x_old = __uint_as_float(v[0]);
         }
@@ -318,7 +327,7 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
         char* to = sm.x + first * SIZE;
         auto take = [&](auto n, auto with_ssq) {
             constexpr int N = decltype(n)::value;
-            dc_take<M, N, decltype(with_ssq)::value>(st, src_epoch, row, k / V, to, pitch, st + p.ssqa, p.hidden / DC_TILE, lane, ss);
+            dc_take<M, N, decltype(with_ssq)::value>(a, src_epoch, row, k / V, to, pitch, st + p.ssqa, p.hidden / DC_TILE, lane, ss);
             row += N * 64;
             to += N * 256;
             left -= N;
@@ -383,7 +392,7 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
     if (stage == DC_GU && wave == 0) {
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            float mine_ = dc_row_scale(st, st + p.ssqa + m * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch, a.inv_width, a.eps_ffn, lane, 128, ss[m]);
+            float mine_ = dc_row_scale(a, st + p.ssqa + m * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch, a.eps_ffn, lane, 128, ss[m]);
             scale = orow == m ? mine_ : scale;
         }
     }
@@ -671,9 +680,9 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
     __builtin_amdgcn_sched_barrier(0);
     float row_scale = 1.0f;
     if (it.layer > 0) {
-        if (wave == 0) dc_far_wait(st, st + p.xgb + it.i * DC_LINE % (p.hidden / T::PER_WORD), epoch - 1);
+        if (wave == 0) dc_far_wait(a, st + p.xgb + it.i * DC_LINE % (p.hidden / T::PER_WORD), epoch - 1);
         __syncthreads();
-        row_scale = dc_row_scale(st, st + p.ssqb + t * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch - 1, a.inv_width, a.eps_mix, lane);
+        row_scale = dc_row_scale(a, st + p.ssqb + t * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch - 1, a.eps_mix, lane);
     }
     u64 drawn = 0;
     if (wave == W - 1 && lane == 0) drawn = tickets.draw();
@@ -682,7 +691,7 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
         const u64* tok = st + p.y + (size_t)t * p.n_qkv;
         auto from = [&](int r) { return tok + (size_t)(r < group ? kvh * group + r : r == group ? p.hq + kvh : p.hq + p.hkv + kvh) * D; };
         uint32_t raw[2 * ROWS];
-        dc_collect<2 * ROWS>(st, epoch, true, lane * 8u, [&](int i, uint32_t o) {
+        dc_collect<2 * ROWS>(a, epoch, true, lane * 8u, [&](int i, uint32_t o) {
             return dc_at(from(min(wave + i / 2 * W, n_rows - 1)) + (i & 1) * 64, o); }, raw);
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) {
@@ -756,14 +765,14 @@ __device__ __forceinline__ void dc_merge(const DcArgs& a, const DcItem& it, DcLd
     u64* st = a.state;
     const uint32_t epoch = it.epoch;
     const int row = it.i;
-    if (wave == 0) dc_far_wait(st, st + p.y + row * DC_LINE % p.n_qkv, epoch);
+    if (wave == 0) dc_far_wait(a, st + p.y + row * DC_LINE % p.n_qkv, epoch);
     __syncthreads();
     u64 drawn = 0;
     if (wave == W - 1 && lane == 0) drawn = tickets.draw();
     const u64* ml = st + p.part_ml + (size_t)row * p.splits * 2;
     bool mine = lane < p.splits;
     uint32_t v[2];
-    dc_collect<2>(st, epoch, mine, mine ? lane * 16u : 0u, [&](int i, uint32_t o) { return dc_at(ml + i, o); }, v);
+    dc_collect<2>(a, epoch, mine, mine ? lane * 16u : 0u, [&](int i, uint32_t o) { return dc_at(ml + i, o); }, v);
     float ms = mine ? __uint_as_float(v[0]) : -INFINITY, ls = mine ? __uint_as_float(v[1]) : 0.f;
     float mm = wave_max(ms);
     float wgt = ms == -INFINITY ? 0.f : DcType<E>::exp(ms - mm);
@@ -772,7 +781,7 @@ __device__ __forceinline__ void dc_merge(const DcArgs& a, const DcItem& it, DcLd
     float o0 = 0.f, o1 = 0.f;
     for (int s0 = wave * run; s0 < s1; s0 += 4) {
         uint32_t q[8];
-        dc_collect<8>(st, epoch, true, lane * 8u, [&](int i, uint32_t o) {
+        dc_collect<8>(a, epoch, true, lane * 8u, [&](int i, uint32_t o) {
             return dc_at(st + p.part + ((size_t)row * p.splits + min(s0 + i / 2, s1 - 1)) * D + (i & 1) * 64, o); }, q);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -912,17 +921,21 @@ ROCML_EXPORT int rocml_decode_chain_words(int dtype, int rows, int hidden, int h
 
 ROCML_EXPORT int rocml_decode_chain_max_layers() { return DC_LAYERS; }
 
-// layers: per layer the ten pointers of DcLayer.
+// layers: per layer the ten pointers of DcLayer.  polls (a power of two), patience (ticks of 10 ns): when a wait gives up; 0 and
+// -1: as it is meant.
 ROCML_EXPORT int rocml_decode_chain(int dtype, void* state, long long state_words, float* x, const void* xn, const void* const* layers, int n_layers,
                                     int rows, int hidden, int hq, int hkv, int head_dim, int inter, const int* block_table, int bt_width,
                                     const int* token_pos, const float* cos_t, const float* sin_t, float scale, float qk_eps, float eps_mix,
-                                    float eps_ffn, int splits, hipStream_t stream) {
+                                    float eps_ffn, int splits, int polls, long long patience, hipStream_t stream) {
     DcArgs a;
     ROCML_REQUIRE(dc_plan(a.p, dtype, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits),
                   "decode_chain: sizes not taken: rows=%d hidden=%d heads=%d/%d of %d inter=%d layers=%d splits=%d", rows, hidden, hq, hkv,
                   head_dim, inter, n_layers, splits);
     ROCML_REQUIRE(state && state_words >= a.p.words, "decode_chain: the state has %lld of %d words", state_words, a.p.words);
     ROCML_REQUIRE(x && xn && layers && block_table && token_pos && cos_t && sin_t && bt_width > 0, "decode_chain: missing operand");
+    ROCML_REQUIRE(polls >= 0 && (polls & (polls - 1)) == 0, "decode_chain: %d looks are not a power of two", polls);
+    a.between = (polls > 0 ? polls : DC_POLLS) - 1;
+    a.patience = patience >= 0 ? patience : DC_PATIENCE;
     a.state = (u64*)state;
     a.x = x; a.xn = xn; a.block_table = block_table; a.bt_width = bt_width; a.pos = token_pos;
     a.cos_t = cos_t; a.sin_t = sin_t;

@@ -77,10 +77,10 @@ def _plain(layers, x, cos, sin, lens):
     return x, kept
 
 
-def _run(layers, x, cos, sin, pos, state):
+def _run(layers, x, cos, sin, pos, state, **how):
     xn = torch.empty(x.shape, dtype=layers[0].w_qkv.dtype, device=DEV)
     ops.rmsnorm(x, layers[0].mix_gain, EPS, xn)
-    ops.decode_chain(x, xn, layers, pos, cos, sin, state)
+    ops.decode_chain(x, xn, layers, pos, cos, sin, state, **how)
 
 
 def _check(layers, x0, x, cos, sin, lens):
@@ -155,6 +155,24 @@ def test_recorded_launch_replayed_with_other_inputs():
         _run(layers, eager, cos, sin, pos, state)
         torch.cuda.synchronize()
         assert torch.equal(got, eager)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_a_wait_that_ended_concerns_its_own_launch_only(dtype):
+    """A launch whose waits are told to end at once (every wait still ends by itself, the launch runs through) gives NaN; the next
+    one on the same state, whose waits look for a mark at every turn, gives what a fresh state gives."""
+    def model():
+        return _model(1024, 16, 8, 3072, 2, [70, 300], 5, seed=5, dtype=dtype)
+    layers, x0, cos, sin, pos = model()
+    state = torch.zeros(ops.decode_chain_words(layers[0], 2, 2), dtype=torch.int64, device=DEV)
+    x = x0.clone()
+    _run(layers, x, cos, sin, pos, state, polls=1, patience=0.0)
+    assert torch.isnan(x).any()
+    layers = model()[0]
+    for _ in range(3):
+        x = x0.clone()
+        _run(layers, x, cos, sin, pos, state, polls=1)
+        _check(layers, x0, x, cos, sin, pos.tolist())
 
 
 def test_what_the_chain_does_not_take():
