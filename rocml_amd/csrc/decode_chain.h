@@ -143,6 +143,7 @@ __device__ __forceinline__ bool dc_give_up(const DcArgs& a, uint32_t epoch, int 
     if (dc_load(at) == dc_mark(epoch)) return true;
     if ((long long)(wall_clock64() - since) < a.patience) return false;
     __hip_atomic_store(at, dc_mark(epoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");          // (there before the NaN that the wait gives travels on)
     return true;
 }
 
@@ -711,7 +712,10 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
             E* dst = r < group ? (E*)sm.q + r * D : r == group ? (E*)sm.k : (E*)sm.v;
             dst[lane] = b0;
             dst[lane + 64] = b1;
-            if (phys >= 0 && r >= group) {
+            // (what a wait that gave up has made of a key or value stays out of the cache: a page's next sequence may weight the
+            // row by zero, which does not take a NaN away)
+            const bool lost = r >= group && __any(v0 != v0 || v1 != v1) && dc_load(st + DC_SHARDS * DC_LINE) == dc_mark(epoch);
+            if (phys >= 0 && r >= group && !lost) {
                 const size_t head = (size_t)phys * p.hkv + kvh;
                 const int at = new_pos % AM_PAGE;
                 if (r == group) {

@@ -159,16 +159,14 @@ def test_recorded_launch_replayed_with_other_inputs():
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 def test_a_wait_that_ended_concerns_its_own_launch_only(dtype):
-    """A launch whose waits are told to end at once (every wait still ends by itself, the launch runs through) gives NaN; the next
-    one on the same state, whose waits look for a mark at every turn, gives what a fresh state gives."""
-    def model():
-        return _model(1024, 16, 8, 3072, 2, [70, 300], 5, seed=5, dtype=dtype)
-    layers, x0, cos, sin, pos = model()
+    """A launch whose waits are told to end at once (every wait still ends by itself, the launch runs through) gives NaN and leaves
+    none in the cache; the next one on the same state, whose waits look for a mark at every turn, gives what a fresh state gives."""
+    layers, x0, cos, sin, pos = _model(1024, 16, 8, 3072, 2, [70, 300], 5, seed=5, dtype=dtype)
     state = torch.zeros(ops.decode_chain_words(layers[0], 2, 2), dtype=torch.int64, device=DEV)
     x = x0.clone()
     _run(layers, x, cos, sin, pos, state, polls=1, patience=0.0)
     assert torch.isnan(x).any()
-    layers = model()[0]
+    assert all(torch.isfinite(t).all() for c in layers for t in (c.k_cache, c.v_cache))
     for _ in range(3):
         x = x0.clone()
         _run(layers, x, cos, sin, pos, state, polls=1)
