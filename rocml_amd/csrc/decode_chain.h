@@ -26,7 +26,7 @@
 // runs and waits for nothing but finished items, or is the next that a running block draws.  That needs one running block for
 // each counter, which the first eight blocks of the grid are, and no block beside another whatever else the GPU runs.  Should a
 // wait last for seconds all the same, it ends, and the step's result is NaN: it leaves the launch's number as a mark, so that the
-// launch's other waits end too, while the next launch waits as if nothing had been.
+// launch's other waits end too, while the next launch waits as if nothing had been, and tells the host (late).
 //
 // The algebra is that of the kernels the step otherwise runs (gemm_kpar_kernel, gemm_residual_prescale_kernel,
 // attn_decode_mfma_kernel FUSED; gemm_f32_rows_kernel, attn_f32_token_kernel): 32-bit sums, the residual stream in 32 bits, the
@@ -123,6 +123,7 @@ struct DcArgs {
     float scale, qk_eps, eps_mix, eps_ffn, inv_width;
     int between;                        // DC_POLLS - 1
     long long patience;                 // DC_PATIENCE
+    int* late;                          // host memory, or null: set to 1 when a wait gives up
     DcLayer layer[DC_LAYERS];
 };
 
@@ -143,6 +144,7 @@ __device__ __forceinline__ bool dc_give_up(const DcArgs& a, uint32_t epoch, int 
     if (dc_load(at) == dc_mark(epoch)) return true;
     if ((long long)(wall_clock64() - since) < a.patience) return false;
     __hip_atomic_store(at, dc_mark(epoch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (a.late) __hip_atomic_store(a.late, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");          // (there before the NaN that the wait gives travels on)
     return true;
 }
@@ -926,11 +928,12 @@ ROCML_EXPORT int rocml_decode_chain_words(int dtype, int rows, int hidden, int h
 ROCML_EXPORT int rocml_decode_chain_max_layers() { return DC_LAYERS; }
 
 // layers: per layer the ten pointers of DcLayer.  polls (a power of two), patience (ticks of 10 ns): when a wait gives up; 0 and
-// -1: as it is meant.
+// -1: as it is meant.  late: see DcArgs.
 ROCML_EXPORT int rocml_decode_chain(int dtype, void* state, long long state_words, float* x, const void* xn, const void* const* layers, int n_layers,
                                     int rows, int hidden, int hq, int hkv, int head_dim, int inter, const int* block_table, int bt_width,
                                     const int* token_pos, const float* cos_t, const float* sin_t, float scale, float qk_eps, float eps_mix,
-                                    float eps_ffn, int splits, int polls, long long patience, hipStream_t stream) {
+                                    float eps_ffn, int splits, int polls, long long patience, int* late,
+                                    hipStream_t stream) {
     DcArgs a;
     ROCML_REQUIRE(dc_plan(a.p, dtype, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits),
                   "decode_chain: sizes not taken: rows=%d hidden=%d heads=%d/%d of %d inter=%d layers=%d splits=%d", rows, hidden, hq, hkv,
@@ -940,6 +943,7 @@ ROCML_EXPORT int rocml_decode_chain(int dtype, void* state, long long state_word
     ROCML_REQUIRE(polls >= 0 && (polls & (polls - 1)) == 0, "decode_chain: %d looks are not a power of two", polls);
     a.between = (polls > 0 ? polls : DC_POLLS) - 1;
     a.patience = patience >= 0 ? patience : DC_PATIENCE;
+    a.late = late;
     a.state = (u64*)state;
     a.x = x; a.xn = xn; a.block_table = block_table; a.bt_width = bt_width; a.pos = token_pos;
     a.cos_t = cos_t; a.sin_t = sin_t;

@@ -18,7 +18,7 @@ import numpy as np
 import torch
 
 from ..cache import Cache
-from ..errors import CacheFullError, ContextOverflowError, RocmlError
+from ..errors import CacheFullError, ContextOverflowError, RocmlError, StepFailedError
 from .. import profile
 from .batch import StepContext, StepEntry, pack_step
 from .model import DecoderModel
@@ -60,6 +60,13 @@ class Engine:
     def length(self, slot: int) -> int:
         return self.cache.length(slot)
 
+    def check_steps(self) -> None:
+        """Raises if a step that has ended on the GPU gave no result (its logits are NaN: a wait between the blocks of a
+        launch lasted for seconds).  Told once; a step asks for those before it, whoever fetches results asks for the step they
+        came from.  The sequences of the step have to be released, the engine goes on."""
+        if self.workspace.was_late():
+            raise StepFailedError("a step ended without a result: its blocks waited for each other for too long")
+
     # -- the step ------------------------------------------------------------------------
     def step(self, entries: Sequence[StepEntry], device_ids: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
         """Runs the entries' tokens; returns ``[n_wanted, vocab]`` 32-bit logits on the
@@ -72,6 +79,7 @@ class Engine:
         spec = self.model.spec
         if not entries:
             return None
+        self.check_steps()
         if device_ids is not None:
             if any(len(e.tokens) != 1 for e in entries) or device_ids.numel() != len(entries) \
                     or device_ids.dtype != torch.int32 or not device_ids.is_cuda:

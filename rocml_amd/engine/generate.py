@@ -16,7 +16,7 @@ import time
 from dataclasses import dataclass, field
 from typing import FrozenSet, List, Optional, Sequence
 
-from ..errors import CacheFullError, RocmlError
+from ..errors import CacheFullError, RocmlError, StepFailedError
 from ..sampling.params import SamplingParams
 from ..sampling.sampler import SequenceSampling
 
@@ -69,6 +69,8 @@ class EngineBackend:
         self.sampler = sampler or DeviceSampler(engine.model.device)
         self.max_positions = engine.model.spec.max_positions
         self.run_ahead = run_ahead and hasattr(self.sampler, "sample_start")
+        # (called when ids have reached the host: the step they were drawn from has ended)
+        self._check_steps = getattr(engine, "check_steps", lambda: None)
         self._row_slots: Optional[List[int]] = None     # the slots whose logits the last step returned, row by row
         self._ahead = None                              # (slots, logits, slots still live, ids drawn) of a step launched ahead
 
@@ -121,7 +123,9 @@ class EngineBackend:
         """``may_continue[b]``: whether sequence ``b`` goes on after this token unless it is a
         stop token (the loop knows the limits); only those are run ahead."""
         if not self.run_ahead or self._row_slots is None or len(self._row_slots) != len(seqs):
-            return self.sampler.sample(logits, seqs)
+            drawn = self.sampler.sample(logits, seqs)
+            self._check_steps()
+            return drawn
         from .batch import StepEntry
         started = self.sampler.sample_start(logits, seqs)
         rows = [b for b in range(len(seqs)) if may_continue is None or may_continue[b]]
@@ -137,9 +141,12 @@ class EngineBackend:
                 # full cache) it changes nothing and the loop goes on step by step
                 ahead = self.engine.step([StepEntry(s, [0], [0]) for s in slots], device_ids=ids)
                 self._ahead = (slots, ahead, set(slots), {})
+            except StepFailedError:
+                raise
             except RocmlError:
                 self._ahead = None
         drawn = self.sampler.finish(started)
+        self._check_steps()
         if self._ahead is not None:
             self._ahead[3].update((self._row_slots[b], int(drawn[b])) for b in rows)
         return drawn

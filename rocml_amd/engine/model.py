@@ -236,7 +236,8 @@ class DecoderModel:
                 xn = self.blocks[entry.layer].chain_input(step, x)
                 cos, sin = position.tables(step)
                 words = ops.decode_chain_words(layers[0], step.n_tokens, len(layers))
-                ops.decode_chain(x, xn, layers, step.token_pos, cos, sin, ws.kept("model.chain", words, torch.int64), max_len=step.max_len)
+                ops.decode_chain(x, xn, layers, step.token_pos, cos, sin, ws.kept("model.chain", words, torch.int64), max_len=step.max_len,
+                                 late=ws.late())
                 behind = i + len(layers)
                 continue
             view = self.entry_view(i, cache, step)

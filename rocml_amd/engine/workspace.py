@@ -11,7 +11,7 @@ generation it was recorded in.
 from __future__ import annotations
 
 import math
-from typing import Dict, Tuple
+from typing import Dict, Optional, Tuple
 
 import torch
 
@@ -27,6 +27,7 @@ class Workspace:
         self._scratch_bytes = scratch_bytes
         self._scratch = None
         self._pending = None
+        self._late: Optional[torch.Tensor] = None
 
     def get(self, name: str, shape: Tuple[int, ...], dtype: torch.dtype) -> torch.Tensor:
         # (a step asks for the same few views over and over; building one costs as much as a launch)
@@ -56,6 +57,21 @@ class Workspace:
             self._buffers[key] = buf
             self.generation += 1
         return buf
+
+    def late(self) -> torch.Tensor:
+        """One number in host memory that a kernel sets to 1 when it ends without a result (see ``was_late``)."""
+        if self._late is None:
+            self._late = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        return self._late
+
+    def was_late(self) -> bool:
+        """Whether a kernel has ended without a result since the last time this was asked and true; asking costs no
+        synchronisation, a kernel that is still running counts when it has ended."""
+        if self._late is None or not int(self._late):
+            return False
+        torch.cuda.synchronize(self.device)         # (what was launched behind it read its results: told once)
+        self._late.zero_()
+        return True
 
     def scratch(self) -> torch.Tensor:
         """Device memory kernels may use for partial results of one launch.  Partial sums

@@ -43,5 +43,9 @@ class KernelError(RocmlError):
     """A HIP kernel refused its arguments, or the GPU runtime reported a failure."""
 
 
+class StepFailedError(RocmlError):
+    """A step that had been launched ended without a result; its sequences have to be released."""
+
+
 class ExtensionMissingError(RocmlError):
     """The compiled HIP library is missing and could not be built."""

@@ -286,6 +286,29 @@ def test_the_backend_may_run_ahead_of_the_host_without_changing_a_token(run_ahea
         assert useful <= ran <= useful + 2
 
 
+@pytest.mark.parametrize("when", ["as the ids arrive", "as the next step is launched"])
+@pytest.mark.parametrize("run_ahead", [True, False])
+def test_a_step_without_a_result_ends_the_loop_and_its_sequences(run_ahead, when):
+    """The engine tells of a step that gave no result when it is asked, or when the next step is launched, which must not look like a
+    step that was refused."""
+    from rocml_amd.engine.generate import EngineBackend
+    from rocml_amd.errors import StepFailedError
+
+    class Failing(_FakeEngine):
+        def check_steps(self):
+            if len(self.steps) >= 3:
+                raise StepFailedError("no result")
+
+        def step(self, entries, device_ids=None):
+            if when == "as the next step is launched":
+                self.check_steps()
+            return super().step(entries, device_ids)
+    engine = Failing(slots=2)
+    with pytest.raises(StepFailedError):
+        Generator(EngineBackend(engine, sampler=_FakeSampler(), run_ahead=run_ahead), max_batch=2).run([Request([1, 2, 3], 10), Request([4], 8)])
+    assert not engine.history and sorted(engine.cache.free) == [0, 1]
+
+
 def test_running_ahead_stops_at_the_models_last_position():
     from rocml_amd.engine.generate import EngineBackend
     engine = _FakeEngine(slots=2, max_positions=6)
