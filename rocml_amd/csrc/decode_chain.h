@@ -24,7 +24,9 @@
 // No wait can last: an item's place in the order is a ticket that a running block draws, and it waits only for items with lower
 // tickets.  The items are dealt over eight counters; of each counter's tickets the lowest unfinished one is held by a block that
 // runs and waits for nothing but finished items, or is the next that a running block draws.  That needs one running block for
-// each counter, which the first eight blocks of the grid are, and no block beside another whatever else the GPU runs.  Should a
+// each counter: a block gets its counter when it starts, in turn, so any eight running blocks of a launch are enough, whatever
+// else the GPU runs.  (By its place in the grid, which saves 1 % of a step, it would not do: a die starts its eighth of a grid by
+// itself, and of two such launches side by side each could fill a die that the other's blocks of one counter wait for.)  Should a
 // wait last for seconds all the same, it ends, and the step's result is NaN: it leaves the launch's number as a mark, so that the
 // launch's other waits end too, while the next launch waits as if nothing had been, and tells the host (late).
 //
@@ -52,7 +54,7 @@ constexpr int DC_MAX_LDS = 128 << 10;
 constexpr int DC_APART = 8;
 constexpr int DC_PAD = 64;              // bytes between two rows of activations in LDS
 constexpr long long DC_PATIENCE = 400000000ll;  // ticks of 10 ns after which a wait gives up
-constexpr int DC_POLLS = 256;                   // looks at a word between two looks at the clock and the mark
+constexpr int DC_POLLS = 256;                   // looks at a word between two looks at the clock and the mark (a power of two)
 
 // The compute type's ways.  bfloat16: two values a word of operands, 32 of K a load, scores in powers of two.  32-bit: one, 16,
 // natural exponentials, and products of 4x4x1 in sixteen blocks: a block is four weight rows and four rows of activations at one
@@ -103,7 +105,7 @@ struct DcLayer {
 };
 
 // Word offsets of the buffers in the state (64-bit words).  The first DC_SHARDS lines hold the ticket counters, the next one the
-// mark of a wait that gave up (dc_mark of its launch).
+// mark of a wait that gave up (dc_mark of its launch), the one behind it counts the blocks that have started.
 struct DcPlan {
     int n_qkv, hq, hkv, hidden, inter, rows, splits, n_layers;
     int items[6], per_layer;            // work items of a layer's stages, in order
@@ -121,7 +123,7 @@ struct DcArgs {
     const int* pos;
     const float *cos_t, *sin_t;         // [rows, 64]
     float scale, qk_eps, eps_mix, eps_ffn, inv_width;
-    int between;                        // DC_POLLS - 1
+    int first_try;                      // what a wait's looks are counted from: 1 (a test looks at the clock earlier)
     long long patience;                 // DC_PATIENCE
     int* late;                          // host memory, or null: set to 1 when a wait gives up
     DcLayer layer[DC_LAYERS];
@@ -138,7 +140,7 @@ __device__ __forceinline__ u64 dc_mark(uint32_t epoch) { return (epoch - 2u) / (
 // A wait that has gone on for long: true when it has to end, because this or another wait of the launch has lasted too long (a
 // mark that an earlier launch left does not count).
 __device__ __forceinline__ bool dc_give_up(const DcArgs& a, uint32_t epoch, int tries, u64& since) {
-    if (tries & a.between) return false;
+    if (tries & (DC_POLLS - 1)) return false;
     u64* at = a.state + DC_SHARDS * DC_LINE;
     if (since == 0) since = wall_clock64();
     if (dc_load(at) == dc_mark(epoch)) return true;
@@ -156,7 +158,7 @@ __device__ __forceinline__ const u64* dc_at(const u64* base, uint32_t bytes) { r
 template <int N, typename At>
 __device__ __forceinline__ void dc_collect(const DcArgs& a, uint32_t epoch, bool mine, uint32_t offset, At at, uint32_t (&v)[N]) {
     u64 w[N], since = 0;
-    for (int tries = 1;; ++tries) {
+    for (int tries = a.first_try;; ++tries) {
         asm volatile("" : "+v"(offset));        // (the addresses are formed in every turn: they do not wait in registers)
 #pragma unroll
         for (int i = 0; i < N; ++i) w[i] = dc_load(at(i, offset));
@@ -178,7 +180,7 @@ __device__ __forceinline__ void dc_collect(const DcArgs& a, uint32_t epoch, bool
 // what it waits for is near, and hundreds of blocks that ask for all their words all the time are in each other's way.
 __device__ __forceinline__ void dc_far_wait(const DcArgs& a, const u64* word, uint32_t epoch) {
     u64 since = 0;
-    for (int tries = 1; (uint32_t)(__builtin_amdgcn_readfirstlane((int)(dc_load(word) >> 32))) != epoch; ++tries) {
+    for (int tries = a.first_try; (uint32_t)(__builtin_amdgcn_readfirstlane((int)(dc_load(word) >> 32))) != epoch; ++tries) {
         __builtin_amdgcn_s_sleep(16);
         if (dc_give_up(a, epoch, tries, since)) break;
     }
@@ -215,16 +217,17 @@ template <int V> struct DcInt { static constexpr int value = V; };
 // What a block works on, the same for all its threads.
 struct DcItem { int stage, layer, i; uint32_t epoch; };
 
-// LDS of a block.
+// LDS of a block.  (The arrays are read 16 bytes at a time; at an odd multiple of 8 a step of 526 us takes 695.)
 template <int W>
 struct DcLds {
     u64 next[2];                                // the item after this one, in turn
+    uint32_t shard;                             // the block's ticket counter
     // the waves' sums (two of them in turn: the other waves go on to the next item while the first finishes this one)
-    float red[2][DC_MAX_TILES][W][DC_MAX_ROWS][DC_TILE];
-    float m[W][16], l[W][16];
-    float o[W][DC_MAX_GROUP][DC_D + 4];
-    float q[DC_MAX_GROUP][DC_D], k[DC_D], v[DC_D];      // (of the compute type)
-    char x[];                                   // operands of a product, rows of K values and DC_PAD bytes
+    alignas(16) float red[2][DC_MAX_TILES][W][DC_MAX_ROWS][DC_TILE];
+    alignas(16) float m[W][16], l[W][16];
+    alignas(16) float o[W][DC_MAX_GROUP][DC_D + 4];
+    alignas(16) float q[DC_MAX_GROUP][DC_D], k[DC_D], v[DC_D];      // (of the compute type)
+    alignas(16) char x[];                       // operands of a product, rows of K values and DC_PAD bytes
 };
 
 __device__ __forceinline__ int dc_k(const DcPlan& p, int stage) { return stage == DC_O ? p.hq * DC_D : stage == DC_DOWN ? p.inter : p.hidden; }
@@ -820,11 +823,21 @@ __global__ void __launch_bounds__(64 * W) decode_chain_kernel(const DcArgs a) {
     extern __shared__ __attribute__((aligned(16))) char dc_lds[];
     DcLds<W>& sm = *(DcLds<W>*)dc_lds;
     const DcPlan& p = a.p;
-    const uint32_t total = (uint32_t)p.per_layer * p.n_layers, shard = blockIdx.x % DC_SHARDS;
+    const uint32_t total = (uint32_t)p.per_layer * p.n_layers;
     // items shard, shard + DC_SHARDS, ...; every block of the counter draws one ticket behind them
-    const DcTickets tickets = {a.state + shard * DC_LINE, (total - shard + DC_SHARDS - 1) / DC_SHARDS + gridDim.x / DC_SHARDS - 1};
-    if (threadIdx.x == 0) tickets.drawn(tickets.draw(), sm.next);
+    auto counter = [&](uint32_t shard) {
+        return DcTickets{a.state + shard * DC_LINE, (total - shard + DC_SHARDS - 1) / DC_SHARDS + gridDim.x / DC_SHARDS - 1};
+    };
+    if (threadIdx.x == 0) {
+        // (a launch's blocks are a whole number for every counter, so the count goes on from launch to launch)
+        const u64 started = __hip_atomic_fetch_add(a.state + (DC_SHARDS + 1) * DC_LINE, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sm.shard = (uint32_t)(started % DC_SHARDS);
+        const DcTickets mine = counter(sm.shard);
+        mine.drawn(mine.draw(), sm.next);
+    }
     __syncthreads();
+    const uint32_t shard = __builtin_amdgcn_readfirstlane((int)sm.shard);
+    const DcTickets tickets = counter(shard);
     for (int turn = 0;; turn ^= 1) {
         const u64 drawn = sm.next[turn];
         const uint32_t item = __builtin_amdgcn_readfirstlane((int)((uint32_t)drawn * DC_SHARDS + shard));
@@ -887,7 +900,7 @@ static bool dc_plan(DcPlan& p, int dtype, int rows, int hidden, int hq, int hkv,
     p.items[DC_DOWN] = hidden / DC_TILE;
     p.per_layer = 0;
     for (int s = 0; s < 6; ++s) p.per_layer += p.items[s];
-    int at = (DC_SHARDS + 1) * DC_LINE;
+    int at = (DC_SHARDS + 2) * DC_LINE;
     auto take = [&](long long words) { int here = at; at += (int)((words + 15) / 16 * 16); return here; };
     p.y = take((long long)rows * p.n_qkv);
     p.part = take(splits > 1 ? (long long)rows * hq * splits * DC_D : 0);
@@ -927,12 +940,12 @@ ROCML_EXPORT int rocml_decode_chain_words(int dtype, int rows, int hidden, int h
 
 ROCML_EXPORT int rocml_decode_chain_max_layers() { return DC_LAYERS; }
 
-// layers: per layer the ten pointers of DcLayer.  polls (a power of two), patience (ticks of 10 ns): when a wait gives up; 0 and
-// -1: as it is meant.  late: see DcArgs.
+// layers: per layer the ten pointers of DcLayer.  polls (looks before a wait's first look at the clock), patience (ticks of
+// 10 ns): when a wait gives up; 0 and -1: as it is meant.  late: see DcArgs.  blocks: 0 for a block a CU; at least so many are started, and eight do.
 ROCML_EXPORT int rocml_decode_chain(int dtype, void* state, long long state_words, float* x, const void* xn, const void* const* layers, int n_layers,
                                     int rows, int hidden, int hq, int hkv, int head_dim, int inter, const int* block_table, int bt_width,
                                     const int* token_pos, const float* cos_t, const float* sin_t, float scale, float qk_eps, float eps_mix,
-                                    float eps_ffn, int splits, int polls, long long patience, int* late,
+                                    float eps_ffn, int splits, int polls, long long patience, int* late, int blocks,
                                     hipStream_t stream) {
     DcArgs a;
     ROCML_REQUIRE(dc_plan(a.p, dtype, rows, hidden, hq, hkv, head_dim, inter, n_layers, splits),
@@ -940,8 +953,8 @@ ROCML_EXPORT int rocml_decode_chain(int dtype, void* state, long long state_word
                   head_dim, inter, n_layers, splits);
     ROCML_REQUIRE(state && state_words >= a.p.words, "decode_chain: the state has %lld of %d words", state_words, a.p.words);
     ROCML_REQUIRE(x && xn && layers && block_table && token_pos && cos_t && sin_t && bt_width > 0, "decode_chain: missing operand");
-    ROCML_REQUIRE(polls >= 0 && (polls & (polls - 1)) == 0, "decode_chain: %d looks are not a power of two", polls);
-    a.between = (polls > 0 ? polls : DC_POLLS) - 1;
+    ROCML_REQUIRE(polls >= 0 && polls <= DC_POLLS, "decode_chain: %d looks", polls);
+    a.first_try = polls > 0 ? DC_POLLS + 1 - polls : 1;
     a.patience = patience >= 0 ? patience : DC_PATIENCE;
     a.late = late;
     a.state = (u64*)state;
@@ -956,7 +969,8 @@ ROCML_EXPORT int rocml_decode_chain(int dtype, void* state, long long state_word
                              (void*)f[8], (void*)f[9]};
     }
     // a block a CU; a whole number for every counter
-    const int blocks = ceil_div(cu_count(), DC_SHARDS) * DC_SHARDS;
+    ROCML_REQUIRE(blocks >= 0, "decode_chain: %d blocks", blocks);
+    blocks = ceil_div(blocks > 0 ? blocks : cu_count(), DC_SHARDS) * DC_SHARDS;
     typedef void (*Kernel)(DcArgs);
     static const Kernel kernels[3][DC_MAX_ROWS] = {
         {decode_chain_kernel<float, 8, 1>, decode_chain_kernel<float, 8, 2>, decode_chain_kernel<float, 8, 3>, decode_chain_kernel<float, 8, 4>},

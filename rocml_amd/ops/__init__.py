@@ -90,7 +90,7 @@ _SIGNATURES = {
         "rocml_decode_chain_pays": [_I, _I, _I, _I, _I, _I, _I],
         "rocml_decode_chain_words": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
         "rocml_decode_chain_max_layers": [],
-        "rocml_decode_chain": [_I, _P, _LL, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _F, _F, _F, _F, _I, _I, _LL, _P, _P],
+        "rocml_decode_chain": [_I, _P, _LL, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _F, _F, _F, _F, _I, _I, _LL, _P, _I, _P],
         "rocml_attention_prefill_fused": [_P, _I, _P, _F, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _I,
                                           _P, _I, _P, _P],
     },
@@ -1244,13 +1244,15 @@ def decode_chain_words(layer: ChainLayer, rows: int, n_layers: int) -> int:
 
 
 def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer], token_pos: torch.Tensor, cos: torch.Tensor,
-                 sin: torch.Tensor, state: torch.Tensor, max_len: int = 0, polls: int = 0, patience: float = -1.0, late: Optional[torch.Tensor] = None) -> None:
+                 sin: torch.Tensor, state: torch.Tensor, max_len: int = 0, polls: int = 0, patience: float = -1.0, late: Optional[torch.Tensor] = None,
+                 blocks: int = 0) -> None:
     """The layers of a decode step, one token per sequence, in one launch: ``x [rows, hidden]`` (32-bit) passes through them,
     the new keys and values are appended.  ``xn``: the first layer's normed input in the compute type (bfloat16 or float32).  ``state`` (int64) starts as
     zeros and is the caller's to keep from call to call; launches that share it run one after the other.  ``max_len`` is what
     ``--profile`` prices the call with.  A block's wait for another's result ends after ``patience`` seconds (about four), which is
-    looked at every ``polls`` looks at the result (256); the launch's results are then NaN, ``late`` (one int32 in pinned host memory) is
-    1, and the next launch is as good as any."""
+    looked at first after ``polls`` looks at the result (256); the launch's results are then NaN, ``late`` (one int32 in pinned host memory) is
+    1, and the next launch is as good as any.  ``blocks``: how many the launch
+    has (rounded up to a multiple of eight), one for each CU unless told otherwise."""
     first = layers[0]
     rows, hidden = x.shape
     _dev(x, xn, token_pos, cos, sin, state, first.block_table)
@@ -1296,7 +1298,7 @@ def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer]
         _code(first.w_qkv), _ptr(state), state.numel(), _ptr(x), _ptr(xn), pointers, len(layers), rows, hidden, first.n_heads, first.n_kv_heads,
         CHAIN_HEAD_DIM, first.inter, _ptr(first.block_table), first.block_table.shape[1], _ptr(token_pos), _ptr(cos), _ptr(sin),
         first.scale, first.qk_eps, first.mix_eps, first.ffn_eps, decode_chain_splits(first.block_table.shape[1]),
-        polls, -1 if patience < 0 else int(patience * 1e8), _ptr(late), _stream()))
+        polls, -1 if patience < 0 else int(patience * 1e8), _ptr(late), blocks, _stream()))
 
 
 ARGMAX_WORK_WORDS = 64      # 32-bit words of workspace per row for the two-stage argmax

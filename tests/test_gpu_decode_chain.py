@@ -157,6 +157,44 @@ def test_recorded_launch_replayed_with_other_inputs():
         assert torch.equal(got, eager)
 
 
+@pytest.mark.parametrize("case", [CASES[0], CASES[4], CASES[6]], ids=["smallest", "splits", "wide"])
+def test_as_few_blocks_as_there_may_be(case):
+    """Eight blocks, which each have a counter to themselves, give the same bits, and the state is as good for the next launch."""
+    hidden, hq, hkv, inter, n_layers, lens, width = case
+    layers, x0, cos, sin, pos = _model(hidden, hq, hkv, inter, n_layers, lens, width, 7)
+    state = torch.zeros(ops.decode_chain_words(layers[0], len(lens), n_layers), dtype=torch.int64, device=DEV)
+    x = x0.clone()
+    _run(layers, x, cos, sin, pos, state)
+    _check(layers, x0, x, cos, sin, lens)
+    for blocks in (8, 0, 24, 104, 8, 0):
+        again = x0.clone()
+        _run(layers, again, cos, sin, pos, state, blocks=blocks)
+        assert torch.equal(again, x), blocks
+
+
+def test_two_launches_side_by_side():
+    """Launches on two streams, which may each have some of the dies first."""
+    models = [_model(1024, 16, 8, 3072, 3, lens, 16, seed=len(lens)) for lens in ([700, 90], [800])]
+    states = [torch.zeros(ops.decode_chain_words(m[0][0], m[1].shape[0], 3), dtype=torch.int64, device=DEV) for m in models]
+    want = []
+    for (layers, x0, cos, sin, pos), state in zip(models, states):
+        x = x0.clone()
+        _run(layers, x, cos, sin, pos, state)
+        _check(layers, x0, x, cos, sin, pos.tolist())
+        want.append(x)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in models]
+    got = [[], []]
+    for _ in range(20):
+        for i, (layers, x0, cos, sin, pos) in enumerate(models):
+            with torch.cuda.stream(streams[i]):
+                x = x0.clone()
+                _run(layers, x, cos, sin, pos, states[i])
+                got[i].append(x)
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, w) for xs, w in zip(got, want) for x in xs)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
 def test_a_wait_that_ended_concerns_its_own_launch_only(dtype):
     """A launch whose waits are told to end at once (every wait still ends by itself, the launch runs through) gives NaN and leaves
