@@ -919,17 +919,24 @@ static bool dc_plan(DcPlan& p, int dtype, int rows, int hidden, int hq, int hkv,
     return true;
 }
 
-// Whether the chain is faster than the layers' own kernels: a matter of how long the weights' bytes take beside the stages'
-// latencies, and of how many words travel.  Steps to the logits, replayed, us:
-//   bfloat16, 0.6B (31 MB a layer): one row 943 -> 546, four 1,096 -> 821;
-//   1.7B (100 MB, 8 layers): one row 545 -> 431, two 547 -> 470, four 580 -> 550;
+// The most pages of a step's block table with which the chain is faster than the layers' own kernels; 0: never.  A matter of how
+// long the weights' bytes take beside the stages' latencies, of how many words travel, and of how many keys are seen: the attention
+// kernels have a piece of keys on its way while they multiply another, the chain, whose registers hold weights, has not.  Steps to
+// the logits, replayed, us:
+//   bfloat16, 0.6B (31 MB a layer), one row: 37 keys 943 -> 546, 5,000 1,071 -> 894, 20,000 1,299 -> 1,266, 32,000 1,546 -> 1,502, 40,000
+//     (1,024 pages in the table) 1,646 -> 1,685; two rows: 2,000 1,049 -> 747, 3,900 1,132 -> 960, 4,200 (128 pages) 1,149 -> 1,259; three: 2,000
+//     1,146 -> 929, 2,100 (64 pages) 1,118 -> 1,144; four: 300 1,026 -> 771, 2,000 1,172 -> 1,023, 2,100 1,174 -> 1,330, 16,000 2,201 -> 2,937;
+//   1.7B (100 MB, 8 layers), one row: 500 505 -> 401, 32,000 648 -> 611; two: 2,000 503 -> 464, 3,900 544 -> 502, 4,200 548 -> 571; four:
+//     500 518 -> 497, 2,000 563 -> 532, 2,100 556 -> 594;
 //   4B (202 MB, 6 layers): one row 628 -> 623; 8B (386 MB, 6 layers): 841 -> 878: while weights stream, a word's way takes several us;
-//   32-bit, 0.6B (63 MB): one row 1,393 -> 807, four 1,705 -> 1,086, four of 1,000 keys 2,341 -> 1,236; 1.7B (201 MB): one row 887 -> 801.
-ROCML_EXPORT int rocml_decode_chain_pays(int dtype, int rows, int hidden, int hq, int hkv, int head_dim, int inter) {
+//   32-bit, whose attention kernels walk a sequence's keys in few blocks: 0.6B (63 MB), one row of 500 1,827 -> 876, of 20,000 20,098 -> 2,053,
+//     four of 1,000 2,312 -> 1,447, of 20,000 20,499 -> 6,280; 1.7B (201 MB), one row of 500 944 -> 828, of 32,000 9,358 -> 1,219.
+ROCML_EXPORT int rocml_decode_chain_reach(int dtype, int rows, int hidden, int hq, int hkv, int head_dim, int inter) {
     DcPlan p;
     if (!dc_plan(p, dtype, rows, hidden, hq, hkv, head_dim, inter, 1, 1)) return 0;
     const double mb = (dtype == ROCML_F32 ? 4e-6 : 2e-6) * hidden * ((double)p.n_qkv + (double)hq * DC_D + 3.0 * inter);
-    return mb <= (dtype == ROCML_F32 && rows == 1 ? 256.0 : 128.0);
+    if (mb > (dtype == ROCML_F32 && rows == 1 ? 256.0 : 128.0)) return 0;
+    return dtype == ROCML_F32 ? 0x7fffffff : rows == 1 ? 512 : 128 / rows;
 }
 
 // 64-bit words of state that a chain of such layers needs; 0: not taken.

@@ -11,6 +11,7 @@ call raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Dict, Optional, Sequence
 
 import torch
@@ -87,7 +88,7 @@ _SIGNATURES = {
                             _P, _I, _I, _P, _I, _I, _P, _LL, _I, _I, _I, _P, _I, _P, _F, _I, _P],
         "rocml_attention_decode_fused": [_P, _I, _I, _LL, _P, _P, _F, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P,
                                          _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _LL, _P, _I, _F, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
-        "rocml_decode_chain_pays": [_I, _I, _I, _I, _I, _I, _I],
+        "rocml_decode_chain_reach": [_I, _I, _I, _I, _I, _I, _I],
         "rocml_decode_chain_words": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
         "rocml_decode_chain_max_layers": [],
         "rocml_decode_chain": [_I, _P, _LL, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _F, _F, _F, _F, _I, _I, _LL, _P, _I, _P],
@@ -1229,11 +1230,17 @@ def decode_chain_splits(pages: int) -> int:
     return 1 if pages <= 4 else min(64, (pages + 1) // 2)
 
 
+@functools.lru_cache(maxsize=256)
+def decode_chain_reach(dtype: torch.dtype, rows: int, hidden: int, n_heads: int, n_kv_heads: int, inter: int) -> int:
+    """The most pages a step's block table may have room for, with which ``decode_chain`` is the faster way for layers of these sizes
+    and so many sequences (the library's own rule); 0: it never is."""
+    return library("attention").rocml_decode_chain_reach(_DTYPE_CODE.get(dtype, -1), rows, hidden, n_heads, n_kv_heads, CHAIN_HEAD_DIM, inter)
+
+
 def decode_chain_pays(layer: ChainLayer, rows: int) -> bool:
-    """Whether ``decode_chain`` takes the layer as it lies, and the library's own rule says that it is the faster way for such
-    layers and so many sequences."""
-    return layer.lies_in_order() and bool(library("attention").rocml_decode_chain_pays(
-        _code(layer.w_qkv), rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter))
+    """Whether ``decode_chain`` takes the layer as it lies, and is the faster way in this step."""
+    return layer.lies_in_order() and layer.block_table.shape[1] <= decode_chain_reach(
+        layer.w_qkv.dtype, rows, layer.hidden, layer.n_heads, layer.n_kv_heads, layer.inter)
 
 
 def decode_chain_words(layer: ChainLayer, rows: int, n_layers: int) -> int:

@@ -48,3 +48,18 @@ def test_a_step_whose_wait_ended_is_told(monkeypatch):
     assert _generate(engine, prompts, 6) == want
     engine.cache.check()
     assert not engine.cache.lengths
+
+
+@pytest.mark.parametrize("lengths,chained", [([4031, 3], True), ([4100, 3], False), ([4100], True)])
+def test_long_sequences_run_the_layers_kernels(monkeypatch, lengths, chained):
+    """Two sequences share one launch up to 64 pages of keys (a table of 128 is refused), one sequence far beyond that; a sequence that
+    grows over the line in the middle goes on."""
+    engine = Engine(_model(2), max_tokens=16384, max_seqs=2)
+    calls = []
+    whole = ops.decode_chain
+    monkeypatch.setattr(ops, "decode_chain", lambda *a, **kw: (calls.append(1), whole(*a, **kw)))
+    prompts = [[i % 500 for i in range(n)] for n in lengths]
+    got = _generate(engine, prompts, 3)
+    assert bool(calls) == chained
+    again = _generate(engine, [p + g[:2] for p, g in zip(prompts, got)], 1)
+    assert [a[0] for a in again] == [g[2] for g in got]

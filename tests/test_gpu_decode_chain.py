@@ -211,6 +211,17 @@ def test_a_wait_that_ended_concerns_its_own_launch_only(dtype):
         _check(layers, x0, x, cos, sin, pos.tolist())
 
 
+@pytest.mark.parametrize("dtype,rows,hidden,inter,most", [
+    (torch.bfloat16, 1, 1024, 3072, 512), (torch.bfloat16, 2, 1024, 3072, 64), (torch.bfloat16, 3, 1024, 3072, 42), (torch.bfloat16, 4, 2048, 6144, 32),
+    (torch.float32, 4, 1024, 3072, 1 << 20), (torch.float32, 1, 2048, 6144, 1 << 20), (torch.float32, 2, 2048, 6144, 0), (torch.bfloat16, 1, 4096, 12288, 0)])
+def test_up_to_how_many_pages_it_pays(dtype, rows, hidden, inter, most):
+    hq = 2 * hidden // D
+    layer = _model(hidden, hq, 8, inter, 1, [5] * rows, 1, seed=9, dtype=dtype)[0][0]
+    for pages in (1, max(most, 1), most + 1):
+        layer.block_table = torch.zeros(rows, pages, dtype=torch.int32, device=DEV)
+        assert ops.decode_chain_pays(layer, rows) == (0 < pages <= most or most == 1 << 20), pages
+
+
 def test_what_the_chain_does_not_take():
     layers, x0, cos, sin, pos = _model(512, 4, 4, 512, 1, [5], 1, seed=4)
     state = torch.zeros(ops.decode_chain_words(layers[0], 1, 1), dtype=torch.int64, device=DEV)
