@@ -516,15 +516,18 @@ sample_kernel(const float* __restrict__ logits, float* __restrict__ work, int vo
 // shuffles.  The rules are those of sample_kernel above; a row is read once, by many CUs,
 // instead of a dozen times by one.
 //
-// Bound by chains of selections and counts, not by the row's bytes.  A wave ranks the few values that can be among its k best
-// all at once; where it has to select them one after the other, a selection is the wave's largest value by DPP moves (no trip
-// through the LDS crossbar) and the lanes that hold it by a ballot.  The waves' lists meet once, an entry's place being the
-// number of entries before it.  151,936 logits, k of 20: slices 24.3 -> 12.0 us (64 rows 62.6 -> 30.0), merge and draw 15.4 ->
-// 9.2; both with a selection for each of the k 20.0 and 9.4.  k of 64: 112 -> 70 us in all.
+// Bound by chains of selections and counts, not by the row's bytes.  A selection is the waves' largest values by DPP moves (no
+// trip through the LDS crossbar), the lanes that hold them by ballots, and the best of the waves' entries by one barrier: 1.1 us an
+// entry (64 rows 1.9), which is the way up to k of 8 (and at 64, where ranks would need more than a wave's lanes).  From there on a
+// wave ranks the few values that can be among its k best all at once, where there are not too many of them; its list and the
+// others' meet once, an entry's place being the number of entries before it.  151,936 logits, both kernels, us, at 1 and at 64
+// rows: k of 1 5.5 and 11.1 (6.2 and 12.0 with shuffles and two barriers a selection), k of 5 10.2 and 18.9 (ranked 13.3 and
+// 23.3), k of 8 13.7 and 26.0 (14.2 and 28.5), k of 12 ranked 18.4 and 35.2 (19.0 and 35.5), k of 20 21.0 and 41.7 (25.9 and 49.4), k of 64
+// 71 and 138 (each wave by itself 76 and 168).
 constexpr int SMALL_K = 64, SLICE_THREADS = 256, MAX_SLICES = 64;
 constexpr int NO_TOKEN = 0x7fffffff;
 constexpr int SLICE_CANDIDATES = 128;           // most values of a wave that are ranked all at once
-constexpr int SLICE_RANKED = 6;                 // k from which on that is faster (64 rows, k of 1: 21 us in all against 14, a selection costs 0.6 to 2)
+constexpr int SLICE_BLOCK = 8;                  // most k that the block selects together
 
 // The largest value of the wave (none of them NaN), in every lane.
 __device__ __forceinline__ float wave_max_moves(float v) {
@@ -608,29 +611,44 @@ sample_slice_topk_kernel(const float* __restrict__ logits, int vocab, int slice_
             if (v[e] > mine.v) { mine.v = v[e]; mine.i = base + e * SLICE_THREADS + tid; }
     };
     look();
+    if (k <= SLICE_BLOCK || k == SMALL_K) {             // the block selects, an entry after the other
+        for (int r = 0; r < k; ++r) {
+            const int from = wave_best_lane(mine);
+            if (lane == max(from, 0)) lists[wave][r] = from < 0 ? ArgMax{-INFINITY, NO_TOKEN} : mine;
+            __syncthreads();
+            ArgMax win = lists[0][r];
+            for (int w = 1; w < WAVES; ++w) win = better(win, lists[w][r]);
+            if (tid == 0) { out_v[r] = win.v; out_i[r] = win.i; }
+            if (r + 1 < k && win.i != NO_TOKEN && (win.i - base) % SLICE_THREADS == tid) {
+                const int we = (win.i - base) / SLICE_THREADS;
+#pragma unroll
+                for (int e = 0; e < EPT; ++e)
+                    if (e == we) v[e] = -INFINITY;
+                look();
+            }
+        }
+        return;
+    }
     int length = 0;
     // The k-th largest of the lanes' maxima bounds the wave's k-th largest value from below: the values not below it (some 24 of
-    // 1,024 at k of 20) are set aside and each finds its place by counting the better ones.  Too many of them (a large k, ties):
+    // 1,024 at k of 20) are set aside and each finds its place by counting the better ones.  Too many of them (ties, a large k):
     // one selection after the other.
-    int n_above = SLICE_CANDIDATES + 1;
-    if (k >= SLICE_RANKED && k < 64) {
-        int larger = 0;
-        for (int j = 0; j < 64; ++j) {
-            const float other = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.v), j));
-            larger += other > mine.v || (other == mine.v && j < lane);
-        }
-        const float bound = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.v),
-                                                                     __builtin_ctzll(__builtin_amdgcn_ballot_w64(larger == k - 1))));
-        n_above = 0;
+    int larger = 0;
+    for (int j = 0; j < 64; ++j) {
+        const float other = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.v), j));
+        larger += other > mine.v || (other == mine.v && j < lane);
+    }
+    const float bound = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine.v),
+                                                                 __builtin_ctzll(__builtin_amdgcn_ballot_w64(larger == k - 1))));
+    int n_above = 0;
 #pragma unroll
-        for (int e = 0; e < EPT; ++e) {
-            const bool in = v[e] >= bound && v[e] > -INFINITY;
-            const unsigned long long who = __builtin_amdgcn_ballot_w64(in);
-            if (who == 0) continue;
-            const int at = n_above + __builtin_popcountll(who & ((1ull << lane) - 1));
-            if (in && at < SLICE_CANDIDATES) above[wave][at] = {v[e], base + e * SLICE_THREADS + tid};
-            n_above += __builtin_popcountll(who);
-        }
+    for (int e = 0; e < EPT; ++e) {
+        const bool in = v[e] >= bound && v[e] > -INFINITY;
+        const unsigned long long who = __builtin_amdgcn_ballot_w64(in);
+        if (who == 0) continue;
+        const int at = n_above + __builtin_popcountll(who & ((1ull << lane) - 1));
+        if (in && at < SLICE_CANDIDATES) above[wave][at] = {v[e], base + e * SLICE_THREADS + tid};
+        n_above += __builtin_popcountll(who);
     }
     if (n_above <= SLICE_CANDIDATES) {
         length = min(k, n_above);

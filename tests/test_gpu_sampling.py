@@ -137,11 +137,11 @@ def test_small_top_k_on_slices_of_the_row(vocab, params):
     assert len(set(got)) <= params.top_k
 
 
-@pytest.mark.parametrize("k", [5, 6, 20, 63, 64])
+@pytest.mark.parametrize("k", [1, 2, 5, 6, 8, 9, 20, 63, 64])
 @pytest.mark.parametrize("row", ["random", "descending", "equal", "two values", "three finite", "infinite"])
 def test_slices_hand_out_the_same_candidates_as_the_whole_row(row, k):
-    """The candidates of the slice kernels, whose waves rank a few values at once or select one after the other (from k of 6 and
-    up to 63, and with not too many values at the bound), at rows of ties and of few finite values: with a nucleus of everything
+    """The candidates of the slice kernels, whose blocks select one after the other (up to k of 8 and at 64), or whose waves rank a few
+    values at once (or, with too many values at the bound, select one after the other), at rows of ties and of few finite values: with a nucleus of everything
     and hardly any difference in probability, draws over evenly spread uniform numbers meet every candidate and no other."""
     vocab, batch = 9000, 256
     g = torch.Generator().manual_seed(11)
