@@ -7,7 +7,6 @@
 #include "attention_generic.h"
 #include "attention_f32.h"
 #include "attention_mfma.h"
-#include "decode_chain.h"
 #include "attention_latent.h"
 
 ROCML_LAST_ERROR_FN(attention)

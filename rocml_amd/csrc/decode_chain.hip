@@ -33,9 +33,14 @@
 // The algebra is that of the kernels the step otherwise runs (gemm_kpar_kernel, gemm_residual_prescale_kernel,
 // attn_decode_mfma_kernel FUSED; gemm_f32_rows_kernel, attn_f32_token_kernel): 32-bit sums, the residual stream in 32 bits, the
 // norm's scale applied by the consumer of bfloat16(x * gain), partial results of key splits merged in split order.
-#pragma once
+//
+// A library of its own: a model that has no such layers does not load these kernels with those of its attention.
+#include "common.h"
+#include "attention_generic.h"
 #include "attention_f32.h"
 #include "attention_mfma.h"
+
+ROCML_LAST_ERROR_FN(decode_chain)
 
 typedef unsigned long long u64;
 typedef __attribute__((ext_vector_type(4))) uint32_t dc_u32x4_t;

@@ -88,10 +88,6 @@ _SIGNATURES = {
                             _P, _I, _I, _P, _I, _I, _P, _LL, _I, _I, _I, _P, _I, _P, _F, _I, _P],
         "rocml_attention_decode_fused": [_P, _I, _I, _LL, _P, _P, _F, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P,
                                          _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _LL, _P, _I, _F, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
-        "rocml_decode_chain_reach": [_I, _I, _I, _I, _I, _I, _I],
-        "rocml_decode_chain_words": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
-        "rocml_decode_chain_max_layers": [],
-        "rocml_decode_chain": [_I, _P, _LL, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _F, _F, _F, _F, _I, _I, _LL, _P, _I, _P],
         "rocml_attention_prefill_fused": [_P, _I, _P, _F, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _I,
                                           _P, _I, _P, _P],
     },
@@ -108,6 +104,12 @@ _SIGNATURES = {
     "sampling": {
         "rocml_sample": [_P, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P, _I, _P, _P],
         "rocml_argmax": [_P, _I, _I, _P, _P, _P],
+    },
+    "decode_chain": {
+        "rocml_decode_chain_reach": [_I, _I, _I, _I, _I, _I, _I],
+        "rocml_decode_chain_words": [_I, _I, _I, _I, _I, _I, _I, _I, _I],
+        "rocml_decode_chain_max_layers": [],
+        "rocml_decode_chain": [_I, _P, _LL, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P, _I, _P, _P, _P, _F, _F, _F, _F, _I, _I, _LL, _P, _I, _P],
     },
 }
 
@@ -1220,7 +1222,7 @@ class ChainLayer:
 
 
 def decode_chain_max_layers() -> int:
-    return library("attention").rocml_decode_chain_max_layers()
+    return library("decode_chain").rocml_decode_chain_max_layers()
 
 
 def decode_chain_splits(pages: int) -> int:
@@ -1234,7 +1236,7 @@ def decode_chain_splits(pages: int) -> int:
 def decode_chain_reach(dtype: torch.dtype, rows: int, hidden: int, n_heads: int, n_kv_heads: int, inter: int) -> int:
     """The most pages a step's block table may have room for, with which ``decode_chain`` is the faster way for layers of these sizes
     and so many sequences (the library's own rule); 0: it never is."""
-    return library("attention").rocml_decode_chain_reach(_DTYPE_CODE.get(dtype, -1), rows, hidden, n_heads, n_kv_heads, CHAIN_HEAD_DIM, inter)
+    return library("decode_chain").rocml_decode_chain_reach(_DTYPE_CODE.get(dtype, -1), rows, hidden, n_heads, n_kv_heads, CHAIN_HEAD_DIM, inter)
 
 
 def decode_chain_pays(layer: ChainLayer, rows: int) -> bool:
@@ -1245,7 +1247,7 @@ def decode_chain_pays(layer: ChainLayer, rows: int) -> bool:
 
 def decode_chain_words(layer: ChainLayer, rows: int, n_layers: int) -> int:
     """64-bit words of state a chain of ``n_layers`` such layers needs for ``rows`` tokens (one per sequence); 0: not taken."""
-    return library("attention").rocml_decode_chain_words(
+    return library("decode_chain").rocml_decode_chain_words(
         _code(layer.w_qkv), rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter, n_layers,
         decode_chain_splits(layer.block_table.shape[1]))
 
@@ -1301,7 +1303,7 @@ def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer]
         _dev(*operands)
         for j, t in enumerate(operands):
             pointers[CHAIN_POINTERS * i + j] = _ptr(t)
-    _check("attention", library("attention").rocml_decode_chain(
+    _check("decode_chain", library("decode_chain").rocml_decode_chain(
         _code(first.w_qkv), _ptr(state), state.numel(), _ptr(x), _ptr(xn), pointers, len(layers), rows, hidden, first.n_heads, first.n_kv_heads,
         CHAIN_HEAD_DIM, first.inter, _ptr(first.block_table), first.block_table.shape[1], _ptr(token_pos), _ptr(cos), _ptr(sin),
         first.scale, first.qk_eps, first.mix_eps, first.ffn_eps, decode_chain_splits(first.block_table.shape[1]),

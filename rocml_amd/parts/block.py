@@ -89,7 +89,8 @@ class PreNormBlock(ConvInput, Part):
         self.ffn = self.children.get("ffn")
         self.graph_safe = all(getattr(c, "graph_safe", True) for c in self.children.values())
         self.prompt_graph_safe = all(getattr(c, "prompt_graph_safe", False) for c in self.children.values())
-        self.kernel_families = tuple(f for c in self.children.values() for f in getattr(c, "kernel_families", ()))
+        self.kernel_families = tuple(f for c in self.children.values() for f in getattr(c, "kernel_families", ())) \
+            + (("decode_chain",) if self.may_chain() else ())
 
     def param_specs(self) -> Dict[str, ParamSpec]:
         return {f"{name}.{p}": spec for name, child in self.children.items()

@@ -115,3 +115,17 @@ def test_decode_splits_fill_the_chip_evenly():
     assert decode_splits(20 * 8, 256, 64) == 3          # 480 of 512 is near enough
     assert decode_splits(16 * 8, 256, 1) == 1           # one page in the table: nothing to split
     assert decode_splits(8, 256, 5) == 5 and decode_splits(4096, 256, 64) == 1
+
+
+@pytest.mark.parametrize("name,chained", [("tiny-a", False), ("tiny-b", False), ("qwen3-0.6b", True), ("qwen3-1.7b", True)])
+def test_only_models_with_such_layers_load_the_one_launch_decode_step(name, chained):
+    import torch
+
+    from rocml_amd.config import architecture_of
+    from rocml_amd.config.catalog import resolve
+    from rocml_amd.engine import DecoderModel
+    cfg = resolve(name).entry.config
+    arch = architecture_of(cfg)
+    model = DecoderModel(arch.to_spec(arch.read_config(cfg)), torch.bfloat16, device="meta")
+    assert ("decode_chain" in model.kernel_families()) == chained
+    assert {"elementwise", "gemm", "attention"} <= set(model.kernel_families())
