@@ -41,7 +41,8 @@ class DecoderModel:
         self.blocks = [build_block(b, ctx) for b in spec.layers]
         self.head = build_head(spec.head_spec(), ctx)
         # the blocks that steps of a few sequences may run in one launch with their neighbours (see _chains)
-        self.may_chain = [hasattr(b, "may_chain") and b.may_chain() for b in self.blocks]
+        # as their sizes, None for the others
+        self.chain_sizes = [b.chain_sizes() if hasattr(b, "may_chain") and b.may_chain() else None for b in self.blocks]
         # rows that schedule entries add to the residual stream before they run (32-bit)
         self.pass_offset: Optional[torch.Tensor] = None
         # matrices that parts of several layers read (each its own columns), by name; a step carries them
@@ -194,12 +195,15 @@ class DecoderModel:
     def _chains(self, step: StepContext, cache: Cache) -> Dict[int, list]:
         """The runs of schedule entries that ``ops.decode_chain`` takes in this step, as ``{first entry: its layers}``."""
         chains: Dict[int, list] = {}
-        if not any(self.may_chain) or step.max_new != 1 or step.n_tokens > ops.CHAIN_MAX_ROWS or step.n_tokens != step.n_seqs:
+        if not any(self.chain_sizes) or step.max_new != 1 or step.n_tokens > ops.CHAIN_MAX_ROWS or step.n_tokens != step.n_seqs:
+            return chains
+        pays = [sizes is not None and ops.decode_chain_reach(self.dtype, step.n_tokens, *sizes) > 0 for sizes in self.chain_sizes]
+        if not any(pays):
             return chains
         run: list = []
         for i, entry in enumerate(self.spec.schedule):
             block, layer = self.blocks[entry.layer], None
-            if entry.reads_cache_of is None and entry.offset_row is None and not entry.add_embedding and self.may_chain[entry.layer]:
+            if entry.reads_cache_of is None and entry.offset_row is None and not entry.add_embedding and pays[entry.layer]:
                 layer = block.chain_layer(step, self.entry_view(i, cache, step))
             if layer is None or not ops.decode_chain_pays(layer, step.n_tokens):
                 run = []

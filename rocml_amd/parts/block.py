@@ -125,6 +125,10 @@ class PreNormBlock(ConvInput, Part):
         return (self.input_conv is None and all(hasattr(n, "prescale_hint") for n in (self.mixer_norm, self.ffn_norm))
                 and all(hasattr(part, "may_chain") and part.may_chain() for part in (self.mixer, self.ffn)))
 
+    def chain_sizes(self):
+        """``(hidden, query heads, key/value heads, intermediate)`` of a block that may chain, for ``ops.decode_chain_reach``."""
+        return self.hidden, self.mixer.spec.n_heads, self.mixer.spec.n_kv_heads, self.ffn.spec.intermediate
+
     def chain_layer(self, step, cache):
         """This layer as ``ops.decode_chain`` runs it in a step, or None if it or the step is not one the chain takes."""
         if not self.may_chain():

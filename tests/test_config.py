@@ -129,3 +129,30 @@ def test_only_models_with_such_layers_load_the_one_launch_decode_step(name, chai
     model = DecoderModel(arch.to_spec(arch.read_config(cfg)), torch.bfloat16, device="meta")
     assert ("decode_chain" in model.kernel_families()) == chained
     assert {"elementwise", "gemm", "attention"} <= set(model.kernel_families())
+
+
+def test_a_step_asks_no_layer_whose_sizes_never_chain(monkeypatch):
+    """The rule of sizes is asked first: where it refuses all of them no layer is built, where it takes some only those are."""
+    import types
+
+    import torch
+
+    from rocml_amd import ops
+    from rocml_amd.config import architecture_of
+    from rocml_amd.config.catalog import resolve
+    from rocml_amd.engine import DecoderModel
+    cfg = dict(resolve("qwen3-8b").entry.config, num_hidden_layers=3)
+    arch = architecture_of(cfg)
+    model = DecoderModel(arch.to_spec(arch.read_config(cfg)), torch.bfloat16, device="meta")
+    sizes = (cfg["hidden_size"], cfg["num_attention_heads"], cfg["num_key_value_heads"], cfg["intermediate_size"])
+    assert model.chain_sizes == [sizes] * 3
+    asked = []
+    for block in model.blocks:
+        monkeypatch.setattr(block, "chain_layer", lambda step, view: asked.append(block))
+    monkeypatch.setattr(model, "entry_view", lambda i, cache, step: None)
+    step = types.SimpleNamespace(max_new=1, n_tokens=2, n_seqs=2)
+    monkeypatch.setattr(ops, "decode_chain_reach", lambda dtype, rows, *s: 0)
+    assert model._chains(step, None) == {} and not asked
+    model.chain_sizes[1] = None
+    monkeypatch.setattr(ops, "decode_chain_reach", lambda dtype, rows, *s: 64 if (dtype, rows, s) == (torch.bfloat16, 2, sizes) else 0)
+    assert model._chains(step, None) == {} and len(asked) == 2
