@@ -1203,7 +1203,7 @@ class ChainLayer:
         return self.w_down.shape[1]
 
     def matrices(self):
-        return [w for w in (self.w_qkv, self.w_o, self.w_gate_up, self.w_down) if w is not None]
+        return self.w_qkv, self.w_o, self.w_gate_up, self.w_down
 
     def lies_in_order(self) -> bool:
         """Whether every operand lies whole and aligned in memory, as the chain's 16-byte loads take it; the layer's own kernels

@@ -116,10 +116,11 @@ def _prefill_fused_cost(qkv, out, k_cache, v_cache, block_table, token_pos, n_he
 
 def _chain_cost(x, xn, layers, *a, **kw) -> Tuple[int, int]:
     rows, seen = x.shape[0], kw.get("max_len", 0)
-    weights = sum(_nbytes(c.w_qkv, c.w_o, c.w_gate_up, c.w_down) for c in layers)
+    weights = sum(_nbytes(*c.matrices()) for c in layers)
+    products = sum(2 * rows * w.numel() for c in layers for w in c.matrices())
     kv = sum(2 * rows * seen * c.n_kv_heads * c.k_cache.shape[3] * c.k_cache.element_size() for c in layers)
     flops = sum(4 * c.n_heads * c.k_cache.shape[3] * rows * seen for c in layers)
-    return weights + kv + 2 * _nbytes(x), rows * weights + flops
+    return weights + kv + 2 * _nbytes(x), products + flops
 
 
 def _tensor_args_cost(skip: Tuple[int, ...] = (), flops_per_byte: float = 0.0) -> Callable:

@@ -180,6 +180,25 @@ def test_profile_report_rows_and_roofline_columns():
     assert "t_min ms" in rep.to_human() and "report" in rep.to_json()
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_the_profile_counts_the_operations_of_a_chain_of_layers(dtype):
+    """Two operations a weight and row and four a head, value and key, whatever the weights' type."""
+    import torch
+    from rocml_amd import ops, profile
+    dt = getattr(torch, dtype)
+
+    def weight(r, c):
+        return torch.zeros(r, c, dtype=dt)
+    cache = torch.zeros(2, 2, 64, 128, dtype=dt)
+    layer = ops.ChainLayer(weight(1024, 512), weight(512, 512), weight(1024, 512), weight(512, 512), None, None, None, None, cache,
+                           cache.transpose(2, 3), None, 4, 2, 1.0, 1e-6, 1e-6, 1e-6, None)
+    x = torch.zeros(3, 512)
+    numbers = 1024 * 512 * 2 + 512 * 512 * 2
+    got_bytes, got_flops = profile._chain_cost(x, x, [layer, layer], max_len=100)
+    assert got_flops == 2 * (2 * 3 * numbers + 4 * 4 * 128 * 3 * 100)
+    assert got_bytes == 2 * (numbers + 2 * 3 * 100 * 2 * 128) * dt.itemsize + 2 * 3 * 512 * 4
+
+
 def test_profiler_wraps_the_launch_helpers_only_while_it_is_active():
     import torch
     from rocml_amd import ops, profile
