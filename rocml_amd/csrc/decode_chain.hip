@@ -25,7 +25,7 @@
 // tickets.  The items are dealt over eight counters; of each counter's tickets the lowest unfinished one is held by a block that
 // runs and waits for nothing but finished items, or is the next that a running block draws.  That needs one running block for
 // each counter: a block gets its counter when it starts, in turn, so any eight running blocks of a launch are enough, whatever
-// else the GPU runs.  (By its place in the grid, which saves 1 % of a step, it would not do: a die starts its eighth of a grid by
+// else the GPU runs.  (By its place in the grid, which saves up to 1 % of a step, it would not do: a die starts its eighth of a grid by
 // itself, and of two such launches side by side each could fill a die that the other's blocks of one counter wait for.)  Should a
 // wait last for seconds all the same, it ends, and the step's result is NaN: it leaves the launch's number as a mark, so that the
 // launch's other waits end too, while the next launch waits as if nothing had been, and tells the host (late).
@@ -204,14 +204,17 @@ __device__ __forceinline__ float dc_row_scale(const DcArgs& a, const u64* ssq, i
     return 1.0f / sqrtf(wave_sum(ss) * a.inv_width + eps);
 }
 
-// A block's place in the order: {launch, ticket} of its counter.  A block draws until its ticket lies behind its counter's last
-// item, so a counter is drawn from (items + blocks) times a launch; the last draw sets up the next launch.
+// A block's place in the order: {launch, ticket} of its counter, handed on as {launch, item}; the items shard, shard + DC_SHARDS,
+// ... are the counter's.  A block draws until its ticket lies behind its counter's last item, so a counter is drawn from (items +
+// blocks) times a launch; the last draw sets up the next launch.
 struct DcTickets {
-    u64* counter; uint32_t last;
-    __device__ __forceinline__ u64 draw() const { return __hip_atomic_fetch_add(counter, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    u64* state; uint32_t end;           // the number behind the items that the counter's last draw gives; its counter is end % DC_SHARDS
+    __device__ __forceinline__ u64* counter() const { return state + end % DC_SHARDS * DC_LINE; }
+    __device__ __forceinline__ u64 draw() const { return __hip_atomic_fetch_add(counter(), 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
     __device__ __forceinline__ void drawn(u64 mine, u64* next) const {
-        if ((uint32_t)mine == last) __hip_atomic_store(counter, ((mine >> 32) + 1) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        *next = mine;
+        const uint32_t item = (uint32_t)mine * DC_SHARDS + end % DC_SHARDS;
+        if (item == end) __hip_atomic_store(counter(), ((mine >> 32) + 1) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *next = (mine >> 32 << 32) | item;
     }
 };
 
@@ -226,7 +229,7 @@ struct DcItem { int stage, layer, i; uint32_t epoch; };
 template <int W>
 struct DcLds {
     u64 next[2];                                // the item after this one, in turn
-    uint32_t shard;                             // the block's ticket counter
+    uint32_t end;                               // see DcTickets
     // the waves' sums (two of them in turn: the other waves go on to the next item while the first finishes this one)
     alignas(16) float red[2][DC_MAX_TILES][W][DC_MAX_ROWS][DC_TILE];
     alignas(16) float m[W][16], l[W][16];
@@ -829,23 +832,21 @@ __global__ void __launch_bounds__(64 * W) decode_chain_kernel(const DcArgs a) {
     DcLds<W>& sm = *(DcLds<W>*)dc_lds;
     const DcPlan& p = a.p;
     const uint32_t total = (uint32_t)p.per_layer * p.n_layers;
-    // items shard, shard + DC_SHARDS, ...; every block of the counter draws one ticket behind them
-    auto counter = [&](uint32_t shard) {
-        return DcTickets{a.state + shard * DC_LINE, (total - shard + DC_SHARDS - 1) / DC_SHARDS + gridDim.x / DC_SHARDS - 1};
-    };
     if (threadIdx.x == 0) {
         // (a launch's blocks are a whole number for every counter, so the count goes on from launch to launch)
         const u64 started = __hip_atomic_fetch_add(a.state + (DC_SHARDS + 1) * DC_LINE, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        sm.shard = (uint32_t)(started % DC_SHARDS);
-        const DcTickets mine = counter(sm.shard);
+        const uint32_t shard = (uint32_t)(started % DC_SHARDS);
+        sm.end = ((total - shard + DC_SHARDS - 1) / DC_SHARDS + gridDim.x / DC_SHARDS - 1) * DC_SHARDS + shard;
+        const DcTickets mine = {a.state, sm.end};
         mine.drawn(mine.draw(), sm.next);
     }
     __syncthreads();
-    const uint32_t shard = __builtin_amdgcn_readfirstlane((int)sm.shard);
-    const DcTickets tickets = counter(shard);
+    uint32_t end = sm.end;
+    asm volatile("" : "+v"(end));               // (a vector register: scalar ones are scarcer, 535 us a step against 530)
+    const DcTickets tickets = {a.state, end};
     for (int turn = 0;; turn ^= 1) {
         const u64 drawn = sm.next[turn];
-        const uint32_t item = __builtin_amdgcn_readfirstlane((int)((uint32_t)drawn * DC_SHARDS + shard));
+        const uint32_t item = __builtin_amdgcn_readfirstlane((int)(uint32_t)drawn);
         const uint32_t launch = __builtin_amdgcn_readfirstlane((int)(uint32_t)(drawn >> 32));
         if (item >= total) break;
         DcItem it;
