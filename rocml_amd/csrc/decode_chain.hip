@@ -7,9 +7,10 @@
 // wait with everything else.  Here a block (one a CU) takes the products' tiles and the attentions' heads of all layers in the
 // order in which they depend on each other: it asks for its weights (or its pages) first, then waits for its operands, so that
 // the next stages' weights are in registers while this stage's results travel.  From a block's store to the waiting blocks that
-// read it some 1.5 us pass.  A step of the Qwen3-0.6B shape (28 layers, replayed, to the logits): one sequence of 37 tokens
-// 943 -> 546 us, of 500 1,000 -> 619, of 5,000 1,122 -> 925; two of 30 and 700 1,034 -> 715; four up to 700 1,096 -> 821.
-// What is left of a layer (14.5 us) is five times a result's way to the next stage, each with a trip to memory behind its store.
+// read it some 1.5 us pass.  A step of the Qwen3-0.6B shape (28 layers, replayed, to the logits): one sequence of 40 tokens
+// 967 -> 530 us, of 500 978 -> 587, of 5,000 1,071 -> 894; two of 2,000 1,049 -> 747; four of 300 1,026 -> 773 (with how many keys it is
+// slower: rocml_decode_chain_reach).  What is left of a layer (15.3 us) is five times a result's way to the next stage, each with a
+// trip to memory behind its store.
 //
 // Measured on the way: two and three blocks a CU instead of one, 657 and 678 us against 558 (more weights ahead, but what asks
 // for operands is in the way of what answers); eight waves a block 648 against 548 (but see dc_plan); a wave of its own for
@@ -929,9 +930,9 @@ static bool dc_plan(DcPlan& p, int dtype, int rows, int hidden, int hq, int hkv,
 // long the weights' bytes take beside the stages' latencies, of how many words travel, and of how many keys are seen: the attention
 // kernels have a piece of keys on its way while they multiply another, the chain, whose registers hold weights, has not.  Steps to
 // the logits, replayed, us:
-//   bfloat16, 0.6B (31 MB a layer), one row: 37 keys 943 -> 546, 5,000 1,071 -> 894, 20,000 1,299 -> 1,266, 32,000 1,546 -> 1,502, 40,000
+//   bfloat16, 0.6B (31 MB a layer), one row: 40 keys 967 -> 530, 5,000 1,071 -> 894, 20,000 1,299 -> 1,266, 32,000 1,546 -> 1,502, 40,000
 //     (1,024 pages in the table) 1,646 -> 1,685; two rows: 2,000 1,049 -> 747, 3,900 1,132 -> 960, 4,200 (128 pages) 1,149 -> 1,259; three: 2,000
-//     1,146 -> 929, 2,100 (64 pages) 1,118 -> 1,144; four: 300 1,026 -> 771, 2,000 1,172 -> 1,023, 2,100 1,174 -> 1,330, 16,000 2,201 -> 2,937;
+//     1,146 -> 929, 2,100 (64 pages) 1,118 -> 1,144; four: 300 1,026 -> 773, 2,000 1,172 -> 1,023, 2,100 1,174 -> 1,330, 16,000 2,201 -> 2,937;
 //   1.7B (100 MB, 8 layers), one row: 500 505 -> 401, 32,000 648 -> 611; two: 2,000 503 -> 464, 3,900 544 -> 502, 4,200 548 -> 571; four:
 //     500 518 -> 497, 2,000 563 -> 532, 2,100 556 -> 594;
 //   4B (202 MB, 6 layers): one row 628 -> 623; 8B (386 MB, 6 layers): 841 -> 878: while weights stream, a word's way takes several us;
