@@ -6,12 +6,14 @@
 #include "gemm_tile.h"
 #include "gemm_mfma.h"
 #include "gemm_pingpong.h"
+#include "gemm_ring.h"
 
 ROCML_LAST_ERROR_FN(gemm)
 
+// (the tile kernels by rows x columns of a block's tile)
 enum GemmAlgo : int { ALGO_AUTO = 0, ALGO_PLAIN = 1, ALGO_MFMA_TILE = 2, ALGO_MFMA_SKINNY = 3, ALGO_MFMA_KPAR = 4,
-                      ALGO_MFMA_TILE256 = 5, ALGO_MFMA_TILE192 = 6, ALGO_MFMA_TILE128X192 = 7, ALGO_MFMA_TILE256X96 = 8,
-                      ALGO_MFMA_TILE64X256 = 9 };
+                      ALGO_MFMA_TILE256 = 5, ALGO_MFMA_TILE256X192 = 6, ALGO_MFMA_TILE128X192 = 7, ALGO_MFMA_TILE256X128 = 8,
+                      ALGO_MFMA_TILE64X128 = 9, ALGO_MFMA_TILE64 = 10, ALGO_MFMA_TILE128X64 = 11, ALGO_MFMA_TILE128X256 = 12 };
 
 static int round_up(int a, int b) { return (a + b - 1) / b * b; }
 
@@ -57,6 +59,37 @@ static int launch_mfma_tile_as(const void* x, int ldx, const void* w, int ldw, v
     return 0;
 }
 
+// The ring kernel.
+template <int EPI, typename T, typename E = bf16_t>
+static int launch_ring(const void* x, int ldx, const void* w, int ldw, void* out, int ldo, int m,
+                       int n, int k, int splits, void* workspace, SplitPlan plan, hipStream_t stream) {
+    static bool ready = false;
+    if (!ready) {
+        if (allow_lds(gemm_ring_kernel<EPI, T, E>, T::LDS_BYTES, "gemm")) return 1;
+        if (allow_lds(gemm_ring_kernel<EPI_F32, T, E>, T::LDS_BYTES, "gemm")) return 1;
+        ready = true;
+    }
+    int tiles_m = ceil_div(m, T::BM), tiles_n = ceil_div(n, T::BN);
+    int n_tiles = tiles_m * tiles_n;
+    if (splits <= 1) {
+        gemm_ring_kernel<EPI, T, E><<<round_up(n_tiles, 8), T::THREADS, T::LDS_BYTES, stream>>>(
+            (const E*)x, ldx, (const E*)w, ldw, out, ldo, m, n, k, tiles_m, n_tiles, k, 0);
+        return 0;
+    }
+    int k_per_split = round_up(ceil_div(k, splits), 128 / (int)sizeof(E));
+    splits = ceil_div(k, k_per_split);
+    gemm_ring_kernel<EPI_F32, T, E><<<round_up(n_tiles * splits, 8), T::THREADS, T::LDS_BYTES, stream>>>(
+        (const E*)x, ldx, (const E*)w, ldw, workspace, n, m, n, k, tiles_m, n_tiles, k_per_split,
+        (long long)m * n);
+    if (plan.defer && ldo == n) {
+        *plan.deferred = splits;
+        return 0;
+    }
+    long long total = (long long)m * n;
+    gemm_splitk_reduce_kernel<EPI><<<ceil_div(total, 256), 256, 0, stream>>>((const float*)workspace, out, ldo, m, n, splits);
+    return 0;
+}
+
 // The same for the 256x256 kernel: one block a CU walks through its share of the tiles (and K pieces).
 template <int EPI>
 static int launch_pingpong(const void* x, int ldx, const void* w, int ldw, void* out, int ldo, int m, int n, int k,
@@ -87,102 +120,116 @@ static int launch_pingpong(const void* x, int ldx, const void* w, int ldw, void*
     return 0;
 }
 
-#include "gemm_f32.h"
-
-// Its loads address a tile's rows by 31-bit offsets.
-static bool pingpong_fits(int ldx, int ldw) { return (long long)(ldx > ldw ? ldx : ldw) * 512 < 0x7fff0000ll; }
-
-// The tile shapes of the many-rows kernel, as rows x columns of a block's tile: 128x128 (four waves
-// of 64x64, two blocks a CU), 256x256 (eight waves of 128x64), 256x192 (eight of 64x96), 128x192
-// (four of 64x96), 256x96 (four of 64x96, the whole of up to 256 rows against a narrow strip of
-// weights) and 64x256 (four of 64x64 side by side, for products of few rows).
-using GemmTile128x192 = GemmTile<2, 2, 2, 3>;
-using GemmTile256x96 = GemmTile<4, 1, 2, 3>;
-using GemmTile64x256 = GemmTile<1, 4, 2, 2>;
-
-// What a tile shape costs: microseconds per 64-wide K stage for a CU that holds as many blocks of it
-// as fit (`cap`), when half the chip or less is at work (`light`) and when all of it is (`full`: the
-// memory system is shared and the clock drops under load), for the shape of which two fit,
-// for a CU that holds one alone, and what a launch costs beside its stages (`fixed`).
-struct TileKind { int bm, bn, cap; double light, full, alone, fixed; int shape; };
+// The tile shapes of the many-rows kernels, as rows x columns of a block's tile (the number is the algorithm that asks for one):
+// 256x256 is gemm_pingpong_kernel's, 256x192 (eight waves of 64x96) gemm_mfma_kernel's, whose LDS stages are too large for a
+// ring of three, the others are the ring kernel's.  What one costs: how many blocks a CU holds (`cap`), microseconds per 64-wide
+// K stage for a CU that holds as many blocks as fit when half the chip or less is at work (`light`) and when all of it is
+// (`full`: the L2s are shared and the clock drops under load), for a CU that holds one of two (`alone`), what a launch costs
+// beside its stages (`fixed`) and every further round of blocks (`round`), the rate at which weights arrive (`weights`, TB/s) and
+// sums leave (`sums`).
+struct TileKind { int bm, bn, cap; double light, full, alone, fixed, round, weights, sums; int algo; };
 static const TileKind TILE_KINDS[] = {
-    {128, 128, 2, 0.918, 1.14, 0.577, 3.24, 1}, {256, 256, 1, 1.099, 1.393, 0.0, 7.27, 2}, {256, 192, 1, 1.032, 1.316, 0.0, 5.04, 3},
-    {128, 192, 1, 0.683, 0.83, 0.0, 4.15, 4},   {256, 96, 1, 0.751, 0.835, 0.0, 4.08, 5},  {64, 256, 1, 0.72, 0.729, 0.0, 3.17, 6}};
+    {256, 256, 1, 1.102, 1.465, 0.0, 11.18, 6.54, 3.41, 14.5, ALGO_MFMA_TILE256},  {256, 192, 1, 1.025, 1.319, 0.0, 9.71, 7.71, 5.51, 19.2, ALGO_MFMA_TILE256X192},
+    {128, 128, 1, 0.459, 0.529, 0.0, 3.68, 2.15, 5.26, 4.38, ALGO_MFMA_TILE},      {64, 64, 2, 0.474, 0.452, 0.253, 2.60, 0.69, 5.50, 5.08, ALGO_MFMA_TILE64},
+    {128, 64, 2, 0.682, 0.677, 0.385, 2.64, 0.77, 4.98, 4.78, ALGO_MFMA_TILE128X64}, {128, 192, 1, 0.617, 0.697, 0.0, 4.56, 3.11, 5.53, 4.91, ALGO_MFMA_TILE128X192},
+    {256, 128, 1, 0.665, 0.812, 0.0, 5.64, 4.17, 4.98, 6.29, ALGO_MFMA_TILE256X128}, {128, 256, 1, 0.780, 0.834, 0.0, 4.94, 3.35, 5.70, 5.39, ALGO_MFMA_TILE128X256},
+    {64, 128, 1, 0.385, 0.395, 0.0, 3.44, 1.79, 5.89, 4.74, ALGO_MFMA_TILE64X128}};
 
-// An estimate of a product's time in microseconds with tiles of `kind` and K cut into `pieces`
-// (each piece the work of a block of its own, 32-bit partial sums written once here and read once
-// by whoever adds them): the rounds of blocks the chip holds at a time, each round as long as its
-// K stages at the rate of the CUs' load, but no shorter than the busiest CU needs to pull its
-// blocks' operands (70 GB/s a CU: with few rows it is the weights' arrival that a block waits for,
-// and more, smaller blocks pull more at a time); a fixed part for the launch and one for every further
-// round; the bytes the epilogue moves; never less than the weights need to arrive at all.
-// The constants are those with the least loss by the choice over 3,563 products (64 to 2,048 rows, 13 outputs from
-// 520 to 24576, K from 512 to 12288; left to the next kernel, whole, gated), each measured with all shapes and
-// one to eight pieces of which an estimate is within 1.6 of the best (55,713 times, weights from memory): the choice
-// is 0.6 % behind the best on average, more than 5 % behind for 132 of them and 23 % at worst.  (Fitted to the times
-// of whole K alone it had been 1.2 %, 319 and 41 %.)  The estimate itself is 9 to 14 % off (root mean square) per shape.
+// An estimate of a product's time in microseconds with tiles of `kind` and K cut into `pieces` (each piece the work of a block of
+// its own, 32-bit partial sums written once here and read once by whoever adds them): the rounds of blocks the chip holds at a
+// time, each round its K stages at the rate of the CUs' load or at that of the weights that its blocks pull (a strip is read by
+// all tile rows at once, from memory once), whichever is slower, both where they are alike; a fixed part for the launch and one
+// for every further round; the bytes the epilogue moves.
+// The constants are a fit to 34,867 times of 2,719 products (17 to 3,000 rows, 18 outputs from 520 to 34816, K from 256 to 12288;
+// left to the next kernel, whole, gated; weights from memory), those within twice the best.  The estimate is 5 to 9 % off (root mean
+// square), the choice by it 0.9 % behind the best on average, more than 5 % for 186 products and 28 % at worst.
 static double tile_cost(const TileKind& kind, int pieces, int m, int n, int k, int epi, bool defer, int cus) {
-    long long tiles = (long long)ceil_div(m, kind.bm) * ceil_div(n, kind.bn);
-    int k_per_piece = round_up(ceil_div(k, pieces), GM_BK);
+    const int tiles_m = ceil_div(m, kind.bm);
+    const long long tiles = (long long)tiles_m * ceil_div(n, kind.bn);
+    const int k_per_piece = round_up(ceil_div(k, pieces), GM_BK);
     pieces = ceil_div(k, k_per_piece);
-    long long blocks = tiles * pieces, slots = (long long)cus * kind.cap;
-    double stages = (double)(k_per_piece / GM_BK);
+    const long long blocks = tiles * pieces, slots = (long long)cus * kind.cap;
+    const double stages = (double)(k_per_piece / GM_BK);
     auto stage_us = [&](long long together) {          // blocks on the chip at the same time, at most `slots`
-        double share = (double)together / (double)cus;
-        if (kind.cap == 2 && together <= cus) return kind.alone * (1.0 + 0.2 * (share > 0.5 ? share - 0.5 : 0.0));
-        double busy = (double)together / (double)slots;
+        double share = (double)together / (double)cus, busy = (double)together / (double)slots;
         double w = busy <= 0.5 ? 0.0 : busy >= 1.0 ? 1.0 : (busy - 0.5) * 2.0;
-        return kind.light + (kind.full - kind.light) * w;
+        double own = kind.light + (kind.full - kind.light) * w;
+        if (kind.cap == 2 && together <= cus) own = kind.alone * (1.0 + 0.2 * (share > 0.5 ? share - 0.5 : 0.0));
+        double arrive = (double)together / tiles_m * kind.bn * (GM_BK * 2.0) / (kind.weights * 1e6);
+        return cbrt(own * own * own + arrive * arrive * arrive);
     };
-    long long rounds = blocks / slots, rest = blocks % slots;
-    double t = (double)rounds * stages * stage_us(slots) + (rest ? stages * stage_us(rest) : 0.0);
-    double pulled = (double)(kind.bn + (m < kind.bm ? m : kind.bm)) * k_per_piece * 2.0 * (double)ceil_div(blocks, (long long)cus);
-    if (t < pulled / 70.3e3) t = pulled / 70.3e3;
-    t += kind.fixed + 1.79 * (double)(rounds + (rest ? 1 : 0) - 1);
-    double moved = epi_gated(epi) ? (double)m * n
-                   : pieces > 1      ? (double)m * n * 4.0 * pieces
-                                     : (double)m * n * 4.0 * (epi == EPI_ACC ? 2.0 : 1.0);
-    t += moved / (pieces > 1 ? 5.24e6 : 4.25e6);
-    double floor_us = (double)n * k * 2.0 / 5.87e6;                 // the weights at 5.9 TB/s
-    if (t < floor_us) t = floor_us;
+    const long long rounds = blocks / slots, rest = blocks % slots;
+    double t = (rounds ? (double)rounds * stages * stage_us(slots) : 0.0) + (rest ? stages * stage_us(rest) : 0.0);
+    t += kind.fixed + kind.round * (double)(rounds + (rest ? 1 : 0) - 1);
+    const double moved = epi_gated(epi) ? (double)m * n : (double)m * n * 4.0 * (pieces > 1 ? pieces : epi == EPI_ACC ? 2.0 : 1.0);
+    t += moved / (kind.sums * 1e6);
     if (pieces > 1) t += (double)pieces * m * n * 4.0 / 5.0e6 + (defer ? 0.0 : 3.96);   // read again, by a kernel of their own unless deferred
     return t;
 }
 
-// shape: 0 = choose, else a TileKind's number (then K stays whole).  The choice is the smallest
-// estimate over shapes and pieces.  What counts is the CU with the most work: 6144 columns are 24
-// tiles of 256, which with 2048 rows leave a quarter of the chip idle, or 32 tiles of 192, which
-// fill it; a product of 256 rows and 24576 columns is 384 tiles of 128x128, one and a half to a
-// CU, or 256 of 128x192, one each.  A product with few tiles (few rows, or a narrow output)
-// leaves most CUs idle while a few walk through all of K: then K is cut into up to 8 pieces.
-template <int EPI>
-static int launch_mfma_tile(const void* x, int ldx, const void* w, int ldw, void* out, int ldo, int m,
-                            int n, int k, int shape, void* workspace, long long workspace_bytes, SplitPlan plan,
-                            hipStream_t stream) {
-    int splits = 1;
-    const int cus = cu_count();
-    if (shape == 0) {
-        double best = 1e30;
-        for (const auto& kind : TILE_KINDS) {
-            if (kind.shape == 2 && !pingpong_fits(ldx, ldw)) continue;
-            for (int pieces = 1; pieces <= 8 && pieces <= plan.max_splits; ++pieces) {
-                if (pieces > 1 && (epi_gated(EPI) || k / pieces < 256 || !workspace ||
-                                   (long long)pieces * m * n * (long long)sizeof(float) > workspace_bytes))
-                    break;
-                double t = tile_cost(kind, pieces, m, n, k, EPI, plan.defer && ldo == n, cus);
-                if (t < best) { best = t; shape = kind.shape; splits = pieces; }
-            }
+// The 256x256 and the ring kernel address a tile's rows by 31-bit offsets.
+static bool rows_near(int ldx, int ldw, int size) { return (long long)(ldx > ldw ? ldx : ldw) * 256 * size < 0x7fff0000ll; }
+
+#include "gemm_f32.h"
+
+// algo: ALGO_AUTO = choose, else the tile kernel asked for (then K stays whole).  The choice is the smallest estimate over shapes and
+// pieces.  What counts is the CU with the most work: 6144 columns are 24 tiles of 256, which with 2048 rows leave a quarter of
+// the chip idle, or 32 tiles of 192, which fill it.  A product with few tiles (few rows, or a narrow output)
+// leaves most CUs idle while a few walk through all of K: then K is cut into pieces of at least 256 (512 where more than eight).
+struct TileChoice { int algo, pieces; };
+
+static TileChoice choose_tile(int m, int n, int k, int epi, bool defer, bool near, int most, int cus) {
+    // (a step asks for the same few products over and over: the last answers are kept)
+    struct Kept { int m, n, k, epi, defer, near, most, cus; TileChoice choice; };
+    static thread_local Kept kept[64];
+    Kept& slot = kept[((unsigned)n * 31u + (unsigned)k * 7u + (unsigned)m) % 64u];
+    if (slot.m == m && slot.n == n && slot.k == k && slot.epi == epi && slot.defer == defer && slot.near == near && slot.most == most && slot.cus == cus)
+        return slot.choice;
+    TileChoice choice{ALGO_MFMA_TILE256X192, 1};
+    double best = 1e30;
+    // From 256 rows and K of 4096 on, a K with a rest of a stage keeps 256x256 tiles and with them the number of pieces that a
+    // caller who adds them up has been given for such sizes (the ring in fewer pieces is 4 to 19 % faster: 402 x 4046 x 9328 73 us
+    // in seven, 61 in four); the estimates were fitted to whole stages.
+    const bool rest = k % GM_BK != 0 && k >= 4096 && m >= 256;
+    for (const auto& kind : TILE_KINDS) {
+        if (near ? rest && kind.algo != ALGO_MFMA_TILE256 : kind.algo != ALGO_MFMA_TILE256X192) continue;
+        for (int pieces = 1; pieces <= most && (pieces == 1 || k / pieces >= (pieces <= 8 ? 256 : 512)); ++pieces) {
+            double t = tile_cost(kind, pieces, m, n, k, epi, defer, cus);
+            if (t < best) { best = t; choice = {kind.algo, pieces}; }
         }
     }
-    if (shape == 2 && !pingpong_fits(ldx, ldw)) shape = 1;
-    switch (shape) {
-        case 6: return launch_mfma_tile_as<EPI, GemmTile64x256>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
-        case 5: return launch_mfma_tile_as<EPI, GemmTile256x96>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
-        case 4: return launch_mfma_tile_as<EPI, GemmTile128x192>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
-        case 3: return launch_mfma_tile_as<EPI, GemmTile192>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
-        case 2: return launch_pingpong<EPI>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
-        default: return launch_mfma_tile_as<EPI, GemmTile128>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
+    slot = Kept{m, n, k, epi, defer, near, most, cus, choice};
+    return choice;
+}
+
+template <int EPI>
+static int launch_mfma_tile(const void* x, int ldx, const void* w, int ldw, void* out, int ldo, int m,
+                            int n, int k, int algo, void* workspace, long long workspace_bytes, SplitPlan plan,
+                            hipStream_t stream) {
+    const bool near = rows_near(ldx, ldw, 2);
+    int splits = 1;
+    if (algo == ALGO_AUTO) {
+        long long most = epi_gated(EPI) || !workspace ? 1 : workspace_bytes / ((long long)m * n * (long long)sizeof(float));
+        most = most > 16 ? 16 : most;
+        most = most > plan.max_splits ? plan.max_splits : most;
+        TileChoice c = choose_tile(m, n, k, EPI, plan.defer && ldo == n, near, most < 1 ? 1 : (int)most, cu_count());
+        algo = c.algo;
+        splits = c.pieces;
     }
+    if (!near) algo = ALGO_MFMA_TILE256X192;
+#define RING(S_, ...) launch_ring<EPI, RingTile<GemmTile<__VA_ARGS__>, S_>>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream)
+    switch (algo) {
+        case ALGO_MFMA_TILE256: return launch_pingpong<EPI>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
+        case ALGO_MFMA_TILE256X192: return launch_mfma_tile_as<EPI, GemmTile192>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
+        case ALGO_MFMA_TILE128X192: return RING(4, 4, 2, 1, 3);
+        case ALGO_MFMA_TILE256X128: return RING(3, 4, 2, 2, 2);
+        case ALGO_MFMA_TILE64X128: return RING(6, 2, 2, 1, 2);
+        case ALGO_MFMA_TILE64: return RING(4, 2, 2, 1, 1);
+        case ALGO_MFMA_TILE128X64: return RING(3, 2, 2, 2, 1);
+        case ALGO_MFMA_TILE128X256: return RING(3, 2, 4, 2, 2);
+        default: return RING(4, 4, 2, 1, 2);
+    }
+#undef RING
 }
 
 // The two-steps-ahead kernel on a product that cannot be cut along K (the gated product), with
@@ -597,8 +644,8 @@ static bool kpar_whole_pays(int m, int n, int k, bool gated, int cus) {
 }
 
 // algo: 0 = choose, 1 = plain tiled kernel, 2 = MFMA tile kernel (128x128 tiles), 3 = MFMA few-rows
-// kernel (M <= 64), 4 = MFMA kernel for at most 16 rows, 5 to 9 = MFMA tile kernel with 256x256,
-// 256x192, 128x192, 256x96 and 64x256 tiles.
+// kernel (M <= 64), 4 = MFMA kernel for at most 16 rows, 5 to 12 = MFMA tile kernels with 256x256, 256x192, 128x192,
+// 256x128, 64x128, 64x64, 128x64 and 128x256 tiles.
 // accumulate: out += product (out must be 32-bit); this is the residual sum's epilogue.
 // epilogue: 0 = none; 1 = gated activation: W's rows are (gate_j, up_j) pairs and out is
 //   [M, N/2] = silu(gate) * up; 2 = the same with max(gate, 0) * up; 3 = max(sum, 0)^2, bfloat16.
@@ -629,7 +676,7 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
     ROCML_REQUIRE(ldx >= k && ldw >= k && ldo >= out_cols, "gemm: row strides (%d, %d, %d) below (K, K, N)",
                   ldx, ldw, ldo);
     ROCML_REQUIRE(!accumulate || out_dtype == ROCML_F32, "gemm: accumulation needs a 32-bit output");
-    ROCML_REQUIRE(algo >= ALGO_AUTO && algo <= ALGO_MFMA_TILE64X256, "gemm: unknown algorithm %d", algo);
+    ROCML_REQUIRE(algo >= ALGO_AUTO && algo <= ALGO_MFMA_TILE128X256, "gemm: unknown algorithm %d", algo);
     ROCML_REQUIRE(!defer || deferred_splits, "gemm: deferring needs a place to report the splits");
     if (m == 0) return 0;
     bool bf16_in = x_dtype == ROCML_BF16 && w_dtype == ROCML_BF16;
@@ -651,13 +698,16 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
                       "gemm: a row scale goes with the gated epilogue of at most 16 rows on the few-rows MFMA kernels "
                       "(M=%d parts=%d)", m, row_parts);
     if (use_mfma) {
-        // Up to 16 rows the few-rows kernels; up to 64 rows still for the gated product (it cannot
-        // cut K in pieces, which is what the tile kernel lives on with so few rows) and, up to 48
-        // rows, for every product but the widest (the output projection over the vocabulary): with
-        // blocks chosen for the busiest CU they are 1 to 7 % ahead of the tile kernel at 48 rows
-        // and 4 to 9 % behind it at 64.
+        // Up to 16 rows the few-rows kernels.  Beyond them the ring kernel's pieces of K are ahead of theirs (17 to 48 rows, 1,400 products
+        // left to the next kernel or not: 0.5 to 0.9 times their time) but for weights of some 110 MB and more up to 32 rows and 300 MB up
+        // to 48, whose blocks a CU are many either way (7168 x 8192 at 23 rows 27 us for 32, 19456 x 12288 at 35 99 for 119; 9728 x
+        // 8192 at 20 equal).  The gated product cannot be cut along K: up to 32 rows, and 48 where K is longer than twelve
+        // stages of the ring, the few-rows kernel (4 to 9 % ahead; behind by 16 % for K of up to 768 at 33 to 48 rows), and up to 64 for
+        // weights of 80 MB and more (19456 x 2560 at 64 27 us for 31, 34816 x 5120 74 for 76; 12288 x 2048 18 for 15).
         const int cus = cu_count();
-        bool few_rows = m <= 16 || (m <= 64 && (gated || (m <= 48 && n < 256 * cus)));
+        const long long weights = (long long)n * k;
+        bool few_rows = m <= 16 || (gated ? m <= 32 || (m <= 48 && k > 768) || (m <= 64 && weights >= 40000000)
+                                          : n < 256 * cus && weights >= (m <= 32 ? 56000000 : 150000000) && m <= 48);
         bool skinny = algo == ALGO_MFMA_SKINNY || (algo == ALGO_AUTO && few_rows);
         SplitPlan plan{defer, deferred_splits, RowScale{row_ssq, row_parts, row_eps, 1.0f / (float)k},
                        max_splits >= 1 && max_splits < 16 ? max_splits : 16};
@@ -680,12 +730,7 @@ ROCML_EXPORT int rocml_gemm(const void* x, int x_dtype, int ldx, const void* w, 
         bool kpar = algo == ALGO_MFMA_KPAR || (algo == ALGO_AUTO && (one_trip || whole || (m <= 2 && !gated && 2 * (n / 16) >= 3 * cus)));
         if (kpar) rc = BY_EPI(launch_kpar, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
         else if (skinny) rc = BY_EPI(launch_skinny_m, x, ldx, w, ldw, out, ldo, m, n, k, workspace, workspace_bytes, plan, stream);
-        else rc = BY_EPI(launch_mfma_tile, x, ldx, w, ldw, out, ldo, m, n, k,
-                         algo == ALGO_MFMA_TILE ? 1 : algo == ALGO_MFMA_TILE256 ? 2 : algo == ALGO_MFMA_TILE192 ? 3
-                         : algo == ALGO_MFMA_TILE128X192 ? 4 : algo == ALGO_MFMA_TILE256X96 ? 5
-                         : algo == ALGO_MFMA_TILE64X256 ? 6 : 0,
-                         workspace, workspace_bytes,
-                         plan, stream);
+        else rc = BY_EPI(launch_mfma_tile, x, ldx, w, ldw, out, ldo, m, n, k, algo, workspace, workspace_bytes, plan, stream);
 #undef BY_EPI
         if (rc) return rc;
         ROCML_CHECK_LAUNCH("gemm");

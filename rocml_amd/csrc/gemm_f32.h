@@ -122,12 +122,12 @@ static int launch_f32_rows(const float* x, int ldx, const float* w, int ldw, flo
     return 0;
 }
 
-// Many rows: 128x128 tiles, or 64x64 where those leave CUs idle, K cut in pieces (32-bit partial sums, as everywhere) where
-// that still leaves CUs idle.  Bound by the matrix cores: a stage (32 of K) is 4,096 clocks for a 128x128 tile, 1,024 for a
-// 64x64 one, whatever else the CU holds.  The stage times of the estimate below are those clocks at some 2.1 GHz and a little
-// for the stage's turn; a full chip takes up to 2.2 and 0.75 us.  Of 42 products (six layers at 33 to 2,048 rows, both tiles,
-// one to eight pieces) the choice is 2.8 % behind the best on average, within 5 % for 32, 16 % behind at worst (574 rows,
-// 2048 x 6144: 161 us in three pieces of 128x128 tiles, 138 in eight of 64x64).
+// Many rows: the ring kernel on 64x64 tiles (three blocks a CU) or 64x128, K cut in pieces (32-bit partial sums, as everywhere) where
+// whole K leaves CUs idle.  Bound by the matrix cores: a stage (32 of K) is 1,024 clocks for a 64x64 tile, whatever else the CU holds.
+// The constants of the estimate are a fit to 6,300 times of 1,105 products (33 to 1,500 rows, 18 outputs, K from 256 to 12288), 4 to
+// 7 % off (root mean square); the choice by it is 1 % behind the best of both on average, 17 % at worst.
+// Before the ring (operands staged through registers, 128x128 tiles beside 64x64), microseconds: 574 rows x 4096 x 1024 62 -> 52,
+// gated 6144 x 1024 76 -> 67, 1024 x 3072 42 -> 37 with three pieces for six; 1000 x 4096 x 2048 146 -> 130.
 using GemmTile64 = GemmTile<2, 2, 1, 1>;
 
 template <int EPI>
@@ -135,16 +135,17 @@ static int launch_f32_tile(const float* x, int ldx, const float* w, int ldw, flo
                            void* workspace, long long workspace_bytes, SplitPlan plan, hipStream_t stream) {
     const int cus = cu_count();
     double best = 1e30;
-    int edge = 128, splits = 1;
-    for (int e = 128; e >= 64; e -= 64)
+    int wide = 64, splits = 1;
+    for (int bn = 64; bn <= 128; bn += 64)
         for (int pieces = 1; pieces <= 8 && pieces <= plan.max_splits; ++pieces) {
             if (pieces > 1 && (epi_gated(EPI) || k / pieces < 128 || !workspace || (long long)pieces * m * n * 4 > workspace_bytes)) break;
-            long long blocks = (long long)ceil_div(m, e) * ceil_div(n, e) * pieces;
-            double stage = e == 128 ? 1.9 : 0.55;     // microseconds
-            double t = (double)ceil_div(blocks, (long long)cus) * ceil_div(ceil_div(k, pieces), 32) * stage + 3.0;
-            if (pieces > 1) t += (double)pieces * m * n * 8.0 / 4.0e6 + (plan.defer && ldo == n ? 0.0 : 4.0);
-            if (t < best) { best = t; edge = e; splits = pieces; }
+            long long blocks = (long long)ceil_div(m, 64) * ceil_div(n, bn) * pieces;
+            double stage = bn == 128 ? 1.042 : 0.538, fixed = bn == 128 ? 4.57 : 4.73;    // microseconds
+            double t = (double)ceil_div(blocks, (long long)cus) * ceil_div(ceil_div(k, pieces), 32) * stage + fixed;
+            if (pieces > 1) t += (double)pieces * m * n * 4.0 / 5.0e6 + (plan.defer && ldo == n ? 0.0 : 4.0);
+            if (t < best) { best = t; wide = bn; splits = pieces; }
         }
-    if (edge == 64) return launch_mfma_tile_as<EPI, GemmTile64, float>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
-    return launch_mfma_tile_as<EPI, GemmTile128, float>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
+    if (!rows_near(ldx, ldw, 4)) return launch_mfma_tile_as<EPI, GemmTile64, float>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
+    if (wide == 64) return launch_ring<EPI, RingTile<GemmTile64, 3>, float>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
+    return launch_ring<EPI, RingTile<GemmTile<2, 2, 1, 2>, 3>, float>(x, ldx, w, ldw, out, ldo, m, n, k, splits, workspace, plan, stream);
 }

@@ -4,14 +4,14 @@
 //
 // Kernels:
 //  * gemm_mfma_kernel, many rows (prefill): an output tile per block, each wave a grid of
-//    v_mfma_f32_16x16x32_bf16 tiles (64x64 or 64x96 per wave); K staged 64 at a time through
+//    v_mfma_f32_16x16x32_bf16 tiles (64x96 per wave); K staged 64 at a time through registers and
 //    double-buffered LDS with one barrier per stage; rows padded by 16 bytes so that 128-bit LDS
 //    reads of 16 rows fall into 16 different bank groups.  The idea of the tiling (big tile per
 //    block, a grid of fragments per wave, padded double-buffered LDS) is the reference's WMMA kernel
 //    (rocml-kernels/kernels/gemm_xwt_wmma_impl.h:211-378); layouts, sizes and the instruction
 //    schedule are for wave64 MFMA.  Blocks are renumbered so that each of the 8 XCDs works on a
 //    contiguous range of tiles and its L2 sees few weight panels.  256x256 tiles are
-//    gemm_pingpong_kernel's (gemm_pingpong.h).
+//    gemm_pingpong_kernel's (gemm_pingpong.h), all but 256x192 gemm_ring_kernel's (gemm_ring.h).
 //    The 16x16x32 product and not 32x32x16: under load the chip is held by its power, and fed from
 //    registers with random operands the first sustains 2.0 PFLOP/s where the second sustains 1.76
 //    (half the traffic to the sums' registers per operation); in these kernels it is 4 to 16 %.
@@ -23,9 +23,9 @@
 //    kernel), so results do not depend on timing
 //    (rocml-kernels/kernels/gemm_splitk_reduce.hip:4-10 has the same rule).
 //    gemm_skinny_ahead_kernel is the same with weights and activations requested two steps
-//    ahead and any number of waves a block from 2 to 16: for 17 to 64 rows, for the gated
-//    product at every number of rows up to 64 (it cannot be cut along K, so the waves a block
-//    are what makes its blocks one round over the CUs), and for products cut along K whose
+//    ahead and any number of waves a block from 2 to 16: for the gated
+//    product of up to 32 to 64 rows (it cannot be cut along K, so the waves a block
+//    are what makes its blocks one round over the CUs), for large weights up to 48 rows, and for products cut along K whose
 //    blocks the host chose for the busiest CU.
 //  * gemm_kpar_kernel, up to 16 rows (one or two against a wide output; more where a wave's share of
 //    K is one chunk; the gated product up to 8): the waves of a block split K and meet once in LDS.
@@ -217,7 +217,7 @@ __device__ __forceinline__ void epilogue_store(void* out, size_t idx, float v) {
 }
 
 // ---- many rows ---------------------------------------------------------------------------
-// One kernel, several shapes (see GemmTile below) with whole K or pieces of it; which one a product gets is the
+// Several kernels and shapes (see GemmTile below) with whole K or pieces of it; which one a product gets is the
 // host's estimate (tile_cost in gemm.hip).
 constexpr int GM_BK = 64;                             // bfloat16 values of a stage: 128 bytes of a row
 constexpr int GM_BAND = 8;                             // tile rows of a band (see the kernel)
@@ -234,7 +234,6 @@ struct GemmTile {
     static constexpr int PA = BM / PASS_ROWS, PB = BN / PASS_ROWS;  // passes per operand
     static constexpr int LDS_BYTES = 2 * (BM + BN) * GM_ROW * 16;   // two stages
 };
-using GemmTile128 = GemmTile<2, 2, 2, 2>;
 using GemmTile256 = GemmTile<2, 4, 4, 2>;       // eight waves (two per SIMD), 128x64 each: gemm_pingpong_kernel
 using GemmTile192 = GemmTile<4, 2, 2, 3>;       // 256 rows x 192 columns, eight waves of 64x96
 

@@ -502,3 +502,45 @@ def test_few_rows_products_with_chosen_blocks(m, n, k):
         assert float((partials.double().sum(0) - ref).abs().max()) < tol
     else:
         assert float((out.double() - ref).abs().max()) < tol
+
+
+# tiles of the ring kernel (rows x columns) by the algorithm that asks for them
+RING = {TILE: (128, 128), TILE128X192: (128, 192), TILE256X96: (256, 128), TILE64X256: (64, 128), 10: (64, 64), 11: (128, 64), 12: (128, 256)}
+
+
+@pytest.mark.parametrize("algo", sorted(RING))
+@pytest.mark.parametrize("k", [8, 64, 72, 192, 392, 904])       # less than a stage, whole ones, a rest; fewer stages than the ring and more
+@pytest.mark.parametrize("dm,dn", [(-1, 1), (0, 0), (1, -1)])
+def test_ring_tiles(algo, k, dm, dn):
+    """Around one tile and two, of operands with NaN beside them: whole sums and the gated activation."""
+    m, n = RING[algo][0] + dm, 2 * RING[algo][1] + 2 * dn
+    x, w = _operands(m, n, k, torch.bfloat16, 11)
+    wide_x, wide_w = torch.full((m, k + 16), float("nan"), dtype=torch.bfloat16, device="cuda"), torch.full(
+        (n, k + 8), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide_x[:, 8:8 + k], wide_w[:, :k] = x, w
+    x, w = wide_x[:, 8:8 + k], wide_w[:, :k]
+    ref = _ref(x, w)
+    out = torch.full((m, n), float("nan"), device="cuda")
+    ops.gemm(x, w, out, algo=algo)
+    assert float((out.double() - ref).abs().max()) < 2e-5 * max(1.0, float(ref.abs().max()))
+    h = torch.empty(m, n // 2, dtype=torch.bfloat16, device="cuda")
+    ops.gemm(x, w, h, algo=algo, epilogue="swiglu")
+    want = torch.nn.functional.silu(ref[:, 0::2]) * ref[:, 1::2]
+    assert float((h.double() - want).abs().max()) < 5e-3 * max(1.0, float(want.abs().max()))
+
+
+# runs of 512 of K and a rest, with and without pieces; both 32-bit tiles
+@pytest.mark.parametrize("m,n,k", [(33, 64, 508), (65, 130, 512), (200, 4100, 1028), (64, 6144, 1540), (574, 1024, 3072), (1000, 2048, 520)])
+def test_float32_sums_in_runs(m, n, k):
+    x, w = _operands(m, n, k, torch.float32, 12)
+    ref = _ref(x, w)
+    out = torch.full((m, n), float("nan"), device="cuda")
+    ops.gemm(x, w, out)
+    # a run's 512 products are added up with an error of a few times sqrt(512) * 2^-24 of their size at most: 2e-6 of the largest sum
+    assert float((out.double() - ref).abs().max()) < 2e-6 * max(1.0, float(ref.abs().max()))
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+    acc = torch.zeros(m, n, device="cuda")
+    pieces = ops.gemm(x, w, acc, accumulate=True, workspace=ws, defer=True)
+    if pieces:
+        acc += ws[:pieces * m * n * 4].view(torch.float32).view(pieces, m, n).sum(0)
+    assert float((acc.double() - ref).abs().max()) < 2e-6 * max(1.0, float(ref.abs().max())), pieces
