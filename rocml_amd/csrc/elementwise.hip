@@ -496,105 +496,203 @@ __global__ void qk_norm_rope_append_kernel(
     }
 }
 
-// Prompts: q and k rows of many tokens.  A wave takes ROWS rows and issues the loads of all of
-// them before it works on the first (one row per wave leaves too few bytes in flight and too
-// many tiny blocks to dispatch).  Only the case LOCAL_PAIR describes: whole head rotated, both
-// values of a pair in one lane, complete projections (no partial sums).
-template <typename TI, typename TO, int QK_PER_LANE, int ROWS>
-__global__ void __launch_bounds__(EW_BLOCK)
-qk_norm_rope_rows_kernel(
-    const TI* __restrict__ qkv, int ld, int n_tokens, int hq, int hkv, int d,
-    const float* __restrict__ q_gain, const float* __restrict__ k_gain, float eps,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
-    TO* __restrict__ q_out, TO* __restrict__ kcache, const int* __restrict__ block_table, int bt_width,
-    const int* __restrict__ token_seq, const int* __restrict__ token_pos, int page_size, int rows_per_token,
-    int first_row, const float* __restrict__ bias, float qt_coef, int qt_every, const float* __restrict__ span_inv) {
-    constexpr int HJ = QK_PER_LANE / 2;
-    int wave = threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1);
-    long long total = (long long)n_tokens * rows_per_token;
-    long long row0 = ((long long)blockIdx.x * QK_WAVES + wave) * ROWS;
-    float v[ROWS][QK_PER_LANE], cs[ROWS][HJ], sn[ROWS][HJ];
-    int tok[ROWS], rr[ROWS];
+// Values of many tokens at once (prompts): a block takes 64 consecutive tokens of the packed
+// batch, one key/value head and 32 of its values, stages them in LDS and writes them transposed.
+// In the transposed page a token is one 2- or 4-byte column; written token by token every store
+// would touch a cache line of its own, written this way the 64 lanes of a wave store 64
+// neighbouring positions of one row (they are neighbours wherever the tokens are consecutive
+// positions of one sequence inside one page, which is the rule in a prompt).
+// WIDE: 16 bytes a load (the rows, the head size and the columns' start allow it).
+constexpr int VT_TOKENS = 64, VT_VALUES = 32;
+
+struct ValueTiles { int col0, heads, d, along_tokens, wide; };   // first column, heads, head size, tiles along the tokens
+
+template <typename TI> struct Wide;                 // 16 bytes of a row as numbers
+template <> struct Wide<float> {
+    static constexpr int N = 4;
+    static __device__ __forceinline__ void load(const float* p, float (&v)[4]) {
+        float4 a = *(const float4*)p;
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    }
+};
+template <> struct Wide<bf16_t> {
+    static constexpr int N = 8;
+    static __device__ __forceinline__ void load(const bf16_t* p, float (&v)[8]) {
+        uint4 a = *(const uint4*)p;
+        const uint32_t w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
-    for (int i = 0; i < ROWS; ++i) {
-        long long row = min(row0 + i, total - 1);            // rows past the end repeat the last one, not stored
-        tok[i] = (int)(row / rows_per_token);
-        rr[i] = first_row + (int)(row - (long long)tok[i] * rows_per_token);
-        const TI* src = qkv + (size_t)tok[i] * ld + (size_t)rr[i] * d;
-#pragma unroll
-        for (int j = 0; j < QK_PER_LANE; ++j) v[i][j] = Elem<TI>::load(src + lane + j * WAVE);
-        if (bias) {
-#pragma unroll
-            for (int j = 0; j < QK_PER_LANE; ++j) v[i][j] += bias[(size_t)rr[i] * d + lane + j * WAVE];
-        }
-        if (cos_t) {
-#pragma unroll
-            for (int j = 0; j < HJ; ++j) {
-                cs[i][j] = cos_t[(size_t)tok[i] * (d / 2) + lane + j * WAVE];
-                sn[i][j] = sin_t[(size_t)tok[i] * (d / 2) + lane + j * WAVE];
-            }
+        for (int i = 0; i < 4; ++i) {
+            v[2 * i] = __uint_as_float(w[i] << 16);
+            v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
         }
     }
+};
+
+template <typename TI, typename TO>
+__device__ __forceinline__ void append_value_tile(const TI* __restrict__ qkv, int ld, int n_tokens, ValueTiles vt, int tile,
+                                                  TO* __restrict__ vcache, const int* __restrict__ block_table, int bt_width,
+                                                  const int* __restrict__ token_seq, const int* __restrict__ token_pos, int page_size,
+                                                  const float* __restrict__ bias) {
+    __shared__ float vt_stage[VT_TOKENS][VT_VALUES + 1];
+    const int t0 = tile % vt.along_tokens * VT_TOKENS, head = tile / vt.along_tokens % vt.heads, e0 = tile / vt.along_tokens / vt.heads * VT_VALUES;
+    const int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE, d = vt.d, col = vt.col0 + head * d;
+    // (asked for together with the values: the page's number is a trip behind them otherwise)
+    const int t = t0 + lane, pos = token_pos[min(t, n_tokens - 1)];
+    const int page = block_table[(size_t)token_seq[min(t, n_tokens - 1)] * bt_width + pos / page_size];
+    if (vt.wide) {
+        constexpr int N = Wide<TI>::N, PER_ROW = VT_VALUES / N, STEP = EW_BLOCK / PER_ROW, PASSES = VT_TOKENS / STEP;
+        float v[PASSES][N], b[N];
+        const int e = min(e0 + tid % PER_ROW * N, d - N);
 #pragma unroll
-    for (int i = 0; i < ROWS; ++i) {
-        bool is_q = rr[i] < hq;
+        for (int i = 0; i < PASSES; ++i) Wide<TI>::load(qkv + (size_t)min(t0 + tid / PER_ROW + STEP * i, n_tokens - 1) * ld + col + e, v[i]);
+#pragma unroll
+        for (int c = 0; c < N; ++c) b[c] = bias ? bias[col + e + c] : 0.f;
+#pragma unroll
+        for (int i = 0; i < PASSES; ++i)
+#pragma unroll
+            for (int c = 0; c < N; ++c) vt_stage[tid / PER_ROW + STEP * i][tid % PER_ROW * N + c] = v[i][c] + b[c];
+    } else {
+        // thread -> (token tid/32 + 8*i, value tid%32): 128 contiguous bytes per token row
+        float tmp[VT_TOKENS * VT_VALUES / EW_BLOCK];
+#pragma unroll
+        for (int i = 0; i < VT_TOKENS * VT_VALUES / EW_BLOCK; ++i) {
+            int j = min(t0 + (tid >> 5) + (EW_BLOCK / VT_VALUES) * i, n_tokens - 1), e = min(e0 + (tid & 31), d - 1);
+            tmp[i] = Elem<TI>::load(qkv + (size_t)j * ld + col + e);
+            if (bias) tmp[i] += bias[col + e];
+        }
+#pragma unroll
+        for (int i = 0; i < VT_TOKENS * VT_VALUES / EW_BLOCK; ++i) vt_stage[(tid >> 5) + (EW_BLOCK / VT_VALUES) * i][tid & 31] = tmp[i];
+    }
+    __syncthreads();
+    if (t >= n_tokens || page < 0) return;
+    TO* dst = vcache + ((size_t)page * vt.heads + head) * d * page_size + pos % page_size;
+#pragma unroll
+    for (int i = 0; i < VT_VALUES / (EW_BLOCK / WAVE); ++i) {
+        int el = wave + (EW_BLOCK / WAVE) * i;
+        if (e0 + el < d) Elem<TO>::store(dst + (size_t)(e0 + el) * page_size, vt_stage[lane][el]);
+    }
+}
+
+template <typename TI, typename TO>
+__global__ void __launch_bounds__(EW_BLOCK)
+v_append_tile_kernel(const TI* __restrict__ qkv, int ld, int n_tokens, ValueTiles vt, TO* __restrict__ vcache,
+                     const int* __restrict__ block_table, int bt_width, const int* __restrict__ token_seq,
+                     const int* __restrict__ token_pos, int page_size, const float* __restrict__ bias) {
+    append_value_tile(qkv, ld, n_tokens, vt, blockIdx.x, vcache, block_table, bt_width, token_seq, token_pos, page_size, bias);
+}
+
+__device__ __forceinline__ float4 row4(const float* p) { return *(const float4*)p; }
+__device__ __forceinline__ float4 row4(const bf16_t* p) {
+    uint2 a = *(const uint2*)p;
+    return make_float4(__uint_as_float(a.x << 16), __uint_as_float(a.x & 0xffff0000u), __uint_as_float(a.y << 16), __uint_as_float(a.y & 0xffff0000u));
+}
+
+// Prompts: q and k rows of many tokens, whole heads of D = 128 or 256 rotated (pairs (e, e + D/2)) or none, complete projections, and
+// behind them in the same launch the values' tiles.  D/8 lanes have a row, eight values each: four pairs, so a rotation needs no
+// exchange and every load and store is 16 (or 8) bytes; a wave works on 64 / (D/8) rows at once and asks for PASSES
+// such sets before it works on the first.  Bound by the bytes: a lane a value of four rows in turn (four-byte loads, two-byte
+// stores, a butterfly of six steps a row) took 8.6 us for 670 tokens of 24 rows and 66 for 8,192 of them, and the values 5 and 20 in
+// a launch of their own.
+template <typename TI, typename TO, int D, int PASSES>
+__global__ void __launch_bounds__(EW_BLOCK)
+qkv_rows_append_kernel(
+    const TI* __restrict__ qkv, int ld, int n_tokens, int hq, int hkv,
+    const float* __restrict__ q_gain, const float* __restrict__ k_gain, float eps,
+    const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+    TO* __restrict__ q_out, TO* __restrict__ kcache, TO* __restrict__ vcache, const int* __restrict__ block_table, int bt_width,
+    const int* __restrict__ token_seq, const int* __restrict__ token_pos, int page_size, unsigned rows_per_token,
+    int first_row, const float* __restrict__ bias, float qt_coef, int qt_every, const float* __restrict__ span_inv,
+    int row_blocks, ValueTiles vt) {
+    if ((int)blockIdx.x >= row_blocks) {
+        append_value_tile(qkv, ld, n_tokens, vt, blockIdx.x - row_blocks, vcache, block_table, bt_width, token_seq, token_pos, page_size, bias);
+        return;
+    }
+    constexpr int LANES = D / 8, SETS = WAVE / LANES;
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x & (WAVE - 1), e = lane % LANES * 4;
+    const unsigned total = (unsigned)n_tokens * rows_per_token;
+    const unsigned row0 = (blockIdx.x * QK_WAVES + wave) * (SETS * PASSES) + lane / LANES;
+    float4 lo[PASSES], hi[PASSES], cs[PASSES], sn[PASSES];
+    int tok[PASSES], rr[PASSES];
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        const unsigned row = min(row0 + i * SETS, total - 1);       // rows past the end repeat the last one, not stored
+        tok[i] = (int)(row / rows_per_token);
+        rr[i] = first_row + (int)(row - (unsigned)tok[i] * rows_per_token);
+        const TI* src = qkv + (size_t)tok[i] * ld + rr[i] * D + e;
+        lo[i] = row4(src);
+        hi[i] = row4(src + D / 2);
+        if (cos_t) {
+            cs[i] = row4(cos_t + (size_t)tok[i] * (D / 2) + e);
+            sn[i] = row4(sin_t + (size_t)tok[i] * (D / 2) + e);
+        }
+    }
+    auto add = [](float4& a, float4 b) { a.x += b.x; a.y += b.y; a.z += b.z; a.w += b.w; };
+    auto scale = [](float4& a, float f, float4 g) { a.x = a.x * f * g.x; a.y = a.y * f * g.y; a.z = a.z * f * g.z; a.w = a.w * f * g.w; };
+#pragma unroll
+    for (int i = 0; i < PASSES; ++i) {
+        const bool is_q = rr[i] < hq;
+        if (bias) {
+            add(lo[i], row4(bias + rr[i] * D + e));
+            add(hi[i], row4(bias + rr[i] * D + e + D / 2));
+        }
         const float* gain = is_q ? q_gain : k_gain;
         if (gain) {
             float inv;
             if (span_inv) {          // the norm spans the token's whole q (k) row: its factor is given, the gain is the head's part
                 inv = span_inv[(size_t)tok[i] * 2 + (is_q ? 0 : 1)];
-                gain += (size_t)(is_q ? rr[i] : rr[i] - hq) * d;
+                gain += (is_q ? rr[i] : rr[i] - hq) * D;
             } else {
-                float ss = 0.f;
+                float ss = lo[i].x * lo[i].x;
+                ss = fmaf(lo[i].y, lo[i].y, ss); ss = fmaf(lo[i].z, lo[i].z, ss); ss = fmaf(lo[i].w, lo[i].w, ss);
+                ss = fmaf(hi[i].x, hi[i].x, ss); ss = fmaf(hi[i].y, hi[i].y, ss); ss = fmaf(hi[i].z, hi[i].z, ss); ss = fmaf(hi[i].w, hi[i].w, ss);
 #pragma unroll
-                for (int j = 0; j < QK_PER_LANE; ++j) ss = fmaf(v[i][j], v[i][j], ss);
-                inv = 1.0f / sqrtf(wave_sum(ss) / (float)d + eps);
+                for (int off = LANES / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
+                inv = 1.0f / sqrtf(ss / (float)D + eps);
             }
-#pragma unroll
-            for (int j = 0; j < QK_PER_LANE; ++j) v[i][j] = v[i][j] * inv * gain[lane + j * WAVE];
+            scale(lo[i], inv, row4(gain + e));
+            scale(hi[i], inv, row4(gain + e + D / 2));
         }
         if (qt_every > 0 && is_q) {
-            float temp = query_temperature(token_pos[tok[i]], qt_coef, qt_every);
-#pragma unroll
-            for (int j = 0; j < QK_PER_LANE; ++j) v[i][j] *= temp;
+            const float temp = query_temperature(token_pos[tok[i]], qt_coef, qt_every);
+            const float4 one = make_float4(1.f, 1.f, 1.f, 1.f);
+            scale(lo[i], temp, one);
+            scale(hi[i], temp, one);
         }
         if (cos_t) {
-#pragma unroll
-            for (int j = 0; j < HJ; ++j) {
-                float lo = v[i][j], hi = v[i][j + HJ];
-                v[i][j] = lo * cs[i][j] - hi * sn[i][j];
-                v[i][j + HJ] = lo * sn[i][j] + hi * cs[i][j];
-            }
+            const float4 a = lo[i], b = hi[i], c = cs[i], n = sn[i];
+            lo[i] = make_float4(a.x * c.x - b.x * n.x, a.y * c.y - b.y * n.y, a.z * c.z - b.z * n.z, a.w * c.w - b.w * n.w);
+            hi[i] = make_float4(a.x * n.x + b.x * c.x, a.y * n.y + b.y * c.y, a.z * n.z + b.z * c.z, a.w * n.w + b.w * c.w);
         }
-        if (row0 + i >= total) continue;
+        if (row0 + i * SETS >= total) continue;
         TO* dst;
         if (is_q) {
-            dst = q_out + ((size_t)tok[i] * hq + rr[i]) * d;
+            dst = q_out + ((size_t)tok[i] * hq + rr[i]) * D;
         } else {
             int pos = token_pos[tok[i]];
             int page = block_table[(size_t)token_seq[tok[i]] * bt_width + pos / page_size];
             if (page < 0) continue;
-            dst = kcache + (((size_t)page * hkv + (rr[i] - hq)) * page_size + pos % page_size) * d;
+            dst = kcache + (((size_t)page * hkv + (rr[i] - hq)) * page_size + pos % page_size) * D;
         }
-#pragma unroll
-        for (int j = 0; j < QK_PER_LANE; ++j) Elem<TO>::store(dst + lane + j * WAVE, v[i][j]);
+        store4(dst + e, lo[i].x, lo[i].y, lo[i].z, lo[i].w);
+        store4(dst + e + D / 2, hi[i].x, hi[i].y, hi[i].z, hi[i].w);
     }
 }
 
 // Prompts: q and k rows without a norm (nor a stretch or biases), in 16-byte pieces, whatever the head size: a thread takes
 // four neighbouring pairs (e, e + rot/2) of a row, or four values beyond the rotated part.  d and rot are multiples of 8.
+// (bfloat16 rows that are only moved come as half as many 32-bit numbers: 8,448 tokens of 16 keys of 192 62 us by a wave a row.)
 template <typename TO>
 __global__ void __launch_bounds__(EW_BLOCK)
 rope_rows_vec_kernel(const float* __restrict__ qkv, int ld, int hq, int hkv, int d, const float* __restrict__ cos_t,
                      const float* __restrict__ sin_t, int rot, TO* __restrict__ q_out, TO* __restrict__ kcache,
                      const int* __restrict__ block_table, int bt_width, const int* __restrict__ token_seq,
-                     const int* __restrict__ token_pos, int page_size, int rows_per_token, int first_row, long long total) {
-    long long idx = (long long)blockIdx.x * EW_BLOCK + threadIdx.x;
+                     const int* __restrict__ token_pos, int page_size, unsigned rows_per_token, int first_row, unsigned total) {
+    const unsigned idx = blockIdx.x * EW_BLOCK + threadIdx.x;
     if (idx >= total) return;
-    const int half = rot / 2, pair_units = rot / 8, units = pair_units + (d - rot) / 4;
-    long long row = idx / units;
+    const int half = rot / 2, pair_units = rot / 8;
+    const unsigned units = pair_units + (d - rot) / 4, row = idx / units;
     int unit = (int)(idx - row * units);
-    int t = (int)(row / rows_per_token), r = first_row + (int)(row - (long long)t * rows_per_token);
+    int t = (int)(row / rows_per_token), r = first_row + (int)(row - (unsigned)t * rows_per_token);
     bool pairs = unit < pair_units;
     int e = pairs ? unit * 4 : rot + (unit - pair_units) * 4;
     const float* src = qkv + (size_t)t * ld + (size_t)r * d + e;
@@ -619,47 +717,6 @@ rope_rows_vec_kernel(const float* __restrict__ qkv, int ld, int hq, int hkv, int
     }
     store4(dst, lo.x * c.x - hi.x * s.x, lo.y * c.y - hi.y * s.y, lo.z * c.z - hi.z * s.z, lo.w * c.w - hi.w * s.w);
     store4(dst + half, lo.x * s.x + hi.x * c.x, lo.y * s.y + hi.y * c.y, lo.z * s.z + hi.z * c.z, lo.w * s.w + hi.w * c.w);
-}
-
-// Values of many tokens at once (prompts): a block takes 64 consecutive tokens of the packed
-// batch, one key/value head and 32 of its values, stages them in LDS and writes them transposed.
-// In the transposed page a token is one 2- or 4-byte column; written token by token every store
-// would touch a cache line of its own, written this way the 64 lanes of a wave store 64
-// neighbouring positions of one row (they are neighbours wherever the tokens are consecutive
-// positions of one sequence inside one page, which is the rule in a prompt).
-constexpr int VT_TOKENS = 64, VT_VALUES = 32;
-
-template <typename TI, typename TO>
-__global__ void __launch_bounds__(EW_BLOCK)
-v_append_tile_kernel(const TI* __restrict__ qkv, int ld, int n_tokens, int v_col0, int hkv, int d,
-                     TO* __restrict__ vcache, const int* __restrict__ block_table, int bt_width,
-                     const int* __restrict__ token_seq, const int* __restrict__ token_pos, int page_size,
-                     const float* __restrict__ bias) {
-    __shared__ float vt_stage[VT_TOKENS][VT_VALUES + 1];
-    int t0 = blockIdx.x * VT_TOKENS, head = blockIdx.y, e0 = blockIdx.z * VT_VALUES;
-    int tid = threadIdx.x, lane = tid & (WAVE - 1), wave = tid / WAVE;
-    // thread -> (token tid/32 + 8*i, value tid%32): 128 contiguous bytes per token row
-    float tmp[VT_TOKENS * VT_VALUES / EW_BLOCK];
-#pragma unroll
-    for (int i = 0; i < VT_TOKENS * VT_VALUES / EW_BLOCK; ++i) {
-        int j = min(t0 + (tid >> 5) + (EW_BLOCK / VT_VALUES) * i, n_tokens - 1), e = min(e0 + (tid & 31), d - 1);
-        tmp[i] = Elem<TI>::load(qkv + (size_t)j * ld + v_col0 + (size_t)head * d + e);
-        if (bias) tmp[i] += bias[v_col0 + (size_t)head * d + e];
-    }
-#pragma unroll
-    for (int i = 0; i < VT_TOKENS * VT_VALUES / EW_BLOCK; ++i) vt_stage[(tid >> 5) + (EW_BLOCK / VT_VALUES) * i][tid & 31] = tmp[i];
-    __syncthreads();
-    int t = t0 + lane;
-    if (t >= n_tokens) return;
-    int pos = token_pos[t];
-    int page = block_table[(size_t)token_seq[t] * bt_width + pos / page_size];
-    if (page < 0) return;
-    TO* dst = vcache + ((size_t)page * hkv + head) * d * page_size + pos % page_size;
-#pragma unroll
-    for (int i = 0; i < VT_VALUES / (EW_BLOCK / WAVE); ++i) {
-        int el = wave + (EW_BLOCK / WAVE) * i;
-        if (e0 + el < d) Elem<TO>::store(dst + (size_t)(e0 + el) * page_size, vt_stage[lane][el]);
-    }
 }
 
 ROCML_EXPORT int rocml_qk_norm_rope_append(
@@ -716,45 +773,62 @@ ROCML_EXPORT int rocml_qk_norm_rope_append(
     // both values of a rotation pair in one lane: whole head rotated, d = per_lane * 64
     // (and the pairs are (e, e + d/2): neighbours as pairs go through LDS)
     bool local_pair = per_lane >= 2 && (rot == 0 || (rot == d && pairing == 0)) && d == per_lane * WAVE && dv == d;
-    // many rows, none of them values: several rows per wave
-    bool many_rows = local_pair && per_lane <= 4 && n_splits == 1 && n_tokens >= VT_TOKENS && (v_tiled || !write_kv) && !span_self;
-    constexpr int MANY = 4;
-    // the same for rows without a norm, of any size that is a multiple of 8
     uintptr_t aligned = (uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)kcache | (uintptr_t)cos_t | (uintptr_t)sin_t;
-    bool plain_rows = in_dtype == ROCML_F32 && !many_rows && !q_gain && !k_gain && !bias && qt_every == 0 && n_splits == 1 &&
+    const int size = in_dtype == ROCML_F32 ? 4 : 2;
+    // many rows, none of them values: several rows per wave
+    bool many_rows = local_pair && per_lane <= 4 && n_splits == 1 && n_tokens >= VT_TOKENS && (v_tiled || !write_kv) && !span_self &&
+                     ld % 4 == 0 && ((aligned | (uintptr_t)q_gain | (uintptr_t)k_gain | (uintptr_t)bias) & 15) == 0 && rows < 1ll << 31;
+    // the same for rows without a norm, of any size that is a multiple of 8
+    bool plain_rows = !many_rows && !q_gain && !k_gain && !bias && qt_every == 0 && n_splits == 1 &&
                       n_tokens >= VT_TOKENS && (v_tiled || !write_kv) && d % 8 == 0 && rot % 8 == 0 && pairing == 0 && ld % 4 == 0 &&
                       (aligned & 15) == 0;
-    long long pieces = (long long)n_tokens * rows_per_token * (cos_t ? rot / 8 + (d - rot) / 4 : d / 4);
-    plain_rows = plain_rows && pieces < (1ll << 31) * EW_BLOCK;
-    int grid = many_rows ? ceil_div(rows, QK_WAVES * MANY) : ceil_div(rows, QK_WAVES);
+    const bool rotated = cos_t && rot;
+    const bool moved = in_dtype == ROCML_BF16 && out_dtype == ROCML_BF16 && !rotated && d % 16 == 0 && ld % 8 == 0;   // as 32-bit numbers
+    plain_rows = plain_rows && (in_dtype == ROCML_F32 || moved);
+    const int row_d = moved ? d / 2 : d, row_ld = moved ? ld / 2 : ld, row_rot = rotated ? rot : 0;
+    long long pieces = (long long)n_tokens * rows_per_token * (row_rot / 8 + (row_d - row_rot) / 4);
+    plain_rows = plain_rows && pieces < 1ll << 31;
+    ValueTiles vt{v_col0, hv, dv, v_tiled ? ceil_div(n_tokens, VT_TOKENS) : 0,
+                  (uintptr_t)qkv % 16 == 0 && (long long)ld * size % 16 == 0 && v_col0 * size % 16 == 0 && dv * size % 16 == 0};
+    const int v_blocks = vt.along_tokens * hv * ceil_div(dv, VT_VALUES);
+    ROCML_REQUIRE((long long)vt.along_tokens * hv * ceil_div(dv, VT_VALUES) < 1ll << 30, "qk_norm_rope_append: too many tokens %d", n_tokens);
+    int grid = ceil_div(rows, QK_WAVES);
     size_t lds = local_pair ? 0 : (size_t)QK_WAVES * d * sizeof(float);
 #define LAUNCH_N(TI, TO, N, LP)                                                                 \
     qk_norm_rope_append_kernel<TI, TO, N, LP><<<grid, EW_BLOCK, lds, stream>>>(                 \
         (const TI*)qkv, ld, n_tokens, hq, hkv, d, q_gain, k_gain, eps, cos_t, sin_t, rot,       \
         (TO*)q_out, (TO*)kcache, (TO*)vcache, block_table, bt_width, token_seq, token_pos,      \
         page_size, write_kv, n_splits, split_stride, rows_per_token, pairing, first_row, bias, dv, qt_coef, qt_every, span_inv, span_self, v_col0, hv)
-#define LAUNCH_ROWS(TI, TO, N)                                                                  \
-    qk_norm_rope_rows_kernel<TI, TO, N, MANY><<<grid, EW_BLOCK, 0, stream>>>(                   \
-        (const TI*)qkv, ld, n_tokens, hq, hkv, d, q_gain, k_gain, eps, rot ? cos_t : nullptr,   \
-        rot ? sin_t : nullptr, (TO*)q_out, (TO*)kcache, block_table, bt_width, token_seq,       \
-        token_pos, page_size, rows_per_token, first_row, bias, qt_coef, qt_every, span_inv)
+    // (few rows are spread over all CUs, many ask for four sets at a time)
+#define LAUNCH_ROWS(TI, TO, D_, PASSES_)                                                        \
+    {                                                                                           \
+        const int row_blocks = ceil_div(rows, QK_WAVES * (WAVE / (D_ / 8)) * PASSES_);          \
+        qkv_rows_append_kernel<TI, TO, D_, PASSES_><<<row_blocks + v_blocks, EW_BLOCK, 0, stream>>>( \
+            (const TI*)qkv, ld, n_tokens, hq, hkv, q_gain, k_gain, eps, rot ? cos_t : nullptr,  \
+            rot ? sin_t : nullptr, (TO*)q_out, (TO*)kcache, (TO*)vcache, block_table, bt_width, token_seq, \
+            token_pos, page_size, rows_per_token, first_row, bias, qt_coef, qt_every, span_inv, row_blocks, vt); \
+    }
 #define LAUNCH(TI, TO)                                                                          \
     {                                                                                           \
-        if (plain_rows) {                                                                       \
-            rope_rows_vec_kernel<TO><<<ceil_div(pieces, EW_BLOCK), EW_BLOCK, 0, stream>>>(      \
-                (const float*)qkv, ld, hq, hkv, d, cos_t, sin_t, cos_t ? rot : 0, (TO*)q_out, (TO*)kcache, block_table, bt_width, \
-                token_seq, token_pos, page_size, rows_per_token, first_row, pieces);            \
-        } else if (many_rows) { if (per_lane == 2) LAUNCH_ROWS(TI, TO, 2); else LAUNCH_ROWS(TI, TO, 4); } \
-        else if (per_lane == 1) LAUNCH_N(TI, TO, 1, false);                                     \
+        if (many_rows) {                                                                        \
+            if (d == 128) { if (rows >= 65536) LAUNCH_ROWS(TI, TO, 128, 4) else LAUNCH_ROWS(TI, TO, 128, 1) } \
+            else { if (rows >= 65536) LAUNCH_ROWS(TI, TO, 256, 4) else LAUNCH_ROWS(TI, TO, 256, 1) } \
+        } else if (plain_rows) {                                                                \
+            if (moved)                                                                          \
+                rope_rows_vec_kernel<float><<<ceil_div(pieces, EW_BLOCK), EW_BLOCK, 0, stream>>>( \
+                    (const float*)qkv, row_ld, hq, hkv, row_d, cos_t, sin_t, 0, (float*)q_out, (float*)kcache, block_table, bt_width, \
+                    token_seq, token_pos, page_size, rows_per_token, first_row, (unsigned)pieces); \
+            else                                                                                \
+                rope_rows_vec_kernel<TO><<<ceil_div(pieces, EW_BLOCK), EW_BLOCK, 0, stream>>>(  \
+                    (const float*)qkv, ld, hq, hkv, d, cos_t, sin_t, row_rot, (TO*)q_out, (TO*)kcache, block_table, bt_width, \
+                    token_seq, token_pos, page_size, rows_per_token, first_row, (unsigned)pieces); \
+        } else if (per_lane == 1) LAUNCH_N(TI, TO, 1, false);                                   \
         else if (per_lane == 2) { if (local_pair) LAUNCH_N(TI, TO, 2, true); else LAUNCH_N(TI, TO, 2, false); } \
         else if (per_lane == 4) { if (local_pair) LAUNCH_N(TI, TO, 4, true); else LAUNCH_N(TI, TO, 4, false); } \
         else { if (local_pair) LAUNCH_N(TI, TO, 8, true); else LAUNCH_N(TI, TO, 8, false); }    \
-        if (v_tiled) {                                                                          \
-            dim3 vgrid(ceil_div(n_tokens, VT_TOKENS), hv, ceil_div(dv, VT_VALUES));            \
-            v_append_tile_kernel<TI, TO><<<vgrid, EW_BLOCK, 0, stream>>>(                       \
-                (const TI*)qkv, ld, n_tokens, v_col0, hv, dv, (TO*)vcache, block_table,\
-                bt_width, token_seq, token_pos, page_size, bias);                               \
-        }                                                                                       \
+        if (v_tiled && !many_rows)                                                              \
+            v_append_tile_kernel<TI, TO><<<v_blocks, EW_BLOCK, 0, stream>>>(                    \
+                (const TI*)qkv, ld, n_tokens, vt, (TO*)vcache, block_table, bt_width, token_seq, token_pos, page_size, bias); \
     }
     if (in_dtype == ROCML_F32 && out_dtype == ROCML_F32) LAUNCH(float, float)
     else if (in_dtype == ROCML_F32 && out_dtype == ROCML_BF16) LAUNCH(float, bf16_t)
@@ -874,11 +948,22 @@ __global__ void add_row_vector_kernel(float* __restrict__ x, const float* __rest
     if (idx < total) x[idx] += b[idx % n];
 }
 
+__global__ void __launch_bounds__(EW_BLOCK)
+add_row_vector_vec_kernel(float* __restrict__ x, const float* __restrict__ b, unsigned quads, unsigned total) {
+    const unsigned idx = blockIdx.x * EW_BLOCK + threadIdx.x;
+    if (idx >= total) return;
+    float4 v = row4(x + (size_t)idx * 4), a = row4(b + idx % quads * 4);
+    *(float4*)(x + (size_t)idx * 4) = make_float4(v.x + a.x, v.y + a.y, v.z + a.z, v.w + a.w);
+}
+
 ROCML_EXPORT int rocml_add_row_vector(float* x, const float* b, int n_rows, int n, hipStream_t stream) {
     ROCML_REQUIRE(n_rows >= 0 && n > 0, "add_row_vector: bad sizes rows=%d n=%d", n_rows, n);
     long long total = (long long)n_rows * n;
     if (total == 0) return 0;
-    add_row_vector_kernel<<<ceil_div(total, EW_BLOCK), EW_BLOCK, 0, stream>>>(x, b, n, total);
+    if (n % 4 == 0 && (((uintptr_t)x | (uintptr_t)b) & 15) == 0 && total / 4 < 1ll << 31)
+        add_row_vector_vec_kernel<<<ceil_div(total / 4, EW_BLOCK), EW_BLOCK, 0, stream>>>(x, b, (unsigned)(n / 4), (unsigned)(total / 4));
+    else
+        add_row_vector_kernel<<<ceil_div(total, EW_BLOCK), EW_BLOCK, 0, stream>>>(x, b, n, total);
     ROCML_CHECK_LAUNCH("add_row_vector");
     return 0;
 }
@@ -1002,6 +1087,42 @@ __global__ void rope_heads_kernel(const float* __restrict__ q, int ldq, int head
     Elem<TO>::store(out + (size_t)t * ldo + (size_t)h * out_stride + out_offset + lead + e, v);
 }
 
+// The same, eight numbers a thread: parts, strides and offsets are multiples of 8 and the halves of a rotation too.  Bound by the
+// bytes: a number a thread (with three 64-bit divisions) took 95 us for 8,192 tokens of 16 heads of 128 + 64 numbers.
+template <typename TO>
+__global__ void __launch_bounds__(EW_BLOCK)
+rope_heads_vec_kernel(const float* __restrict__ q, int ldq, int head_stride, int offset, int dims, const float* __restrict__ cos_t,
+                      const float* __restrict__ sin_t, TO* __restrict__ out, int ldo, int out_stride, int out_offset, unsigned n_heads,
+                      int lead, unsigned pieces, unsigned total, int pairing) {
+    const unsigned idx = blockIdx.x * EW_BLOCK + threadIdx.x;
+    if (idx >= total) return;
+    const unsigned th = idx / pieces, t = th / n_heads, h = th - t * n_heads;
+    const int e = (int)(idx - th * pieces) * 8 - lead, half = dims / 2;
+    const float* src = q + (size_t)t * ldq + h * head_stride + offset;
+    float4 a = row4(src + e), b = row4(src + e + 4);
+    if (e >= 0 && e < dims) {
+        if (pairing == 1) {
+            const float4 c = row4(cos_t + (size_t)t * half + e / 2), s = row4(sin_t + (size_t)t * half + e / 2);
+            const float4 x = a, y = b;
+            a = make_float4(x.x * c.x - x.y * s.x, x.y * c.x + x.x * s.x, x.z * c.y - x.w * s.y, x.w * c.y + x.z * s.y);
+            b = make_float4(y.x * c.z - y.y * s.z, y.y * c.z + y.x * s.z, y.z * c.w - y.w * s.w, y.w * c.w + y.z * s.w);
+        } else {
+            const bool low = e < half;
+            const int at = low ? e : e - half;
+            const float* pair = src + (low ? e + half : e - half);
+            const float4 p = row4(pair), r = row4(pair + 4);
+            float4 c = row4(cos_t + (size_t)t * half + at), d = row4(cos_t + (size_t)t * half + at + 4);
+            float4 s = row4(sin_t + (size_t)t * half + at), u = row4(sin_t + (size_t)t * half + at + 4);
+            if (low) { s.x = -s.x; s.y = -s.y; s.z = -s.z; s.w = -s.w; u.x = -u.x; u.y = -u.y; u.z = -u.z; u.w = -u.w; }
+            a = make_float4(a.x * c.x + p.x * s.x, a.y * c.y + p.y * s.y, a.z * c.z + p.z * s.z, a.w * c.w + p.w * s.w);
+            b = make_float4(b.x * d.x + r.x * u.x, b.y * d.y + r.y * u.y, b.z * d.z + r.z * u.z, b.w * d.w + r.w * u.w);
+        }
+    }
+    TO* to = out + (size_t)t * ldo + h * out_stride + out_offset + lead + e;
+    store4(to, a.x, a.y, a.z, a.w);
+    store4(to + 4, b.x, b.y, b.z, b.w);
+}
+
 ROCML_EXPORT int rocml_rope_heads(const float* q, int ldq, int head_stride, int offset, int rot_part, int dims,
                                   const float* cos_t, const float* sin_t, void* out, int out_dtype, int ldo,
                                   int out_stride, int out_offset, int n_tokens, int n_heads, int lead, int pairing,
@@ -1016,6 +1137,17 @@ ROCML_EXPORT int rocml_rope_heads(const float* q, int ldq, int head_stride, int 
     long long total = (long long)n_tokens * n_heads * (lead + rot_part);
     if (total == 0) return 0;
     int grid = ceil_div(total, EW_BLOCK);
+    const uintptr_t aligned = (uintptr_t)q | (uintptr_t)out | (uintptr_t)cos_t | (uintptr_t)sin_t;
+    if ((out_dtype == ROCML_F32 || out_dtype == ROCML_BF16) && ((ldq | head_stride | offset | rot_part | lead | ldo | out_stride | out_offset) & 7) == 0 &&
+        dims % 16 == 0 && (aligned & 15) == 0 && total / 8 < 1ll << 31) {
+#define LAUNCH(TO) rope_heads_vec_kernel<TO><<<ceil_div(total / 8, EW_BLOCK), EW_BLOCK, 0, stream>>>(q, ldq, head_stride, offset, dims, cos_t, sin_t, \
+        (TO*)out, ldo, out_stride, out_offset, n_heads, lead, (lead + rot_part) / 8, (unsigned)(total / 8), pairing)
+        if (out_dtype == ROCML_F32) LAUNCH(float);
+        else LAUNCH(bf16_t);
+#undef LAUNCH
+        ROCML_CHECK_LAUNCH("rope_heads");
+        return 0;
+    }
     if (out_dtype == ROCML_F32)
         rope_heads_kernel<float><<<grid, EW_BLOCK, 0, stream>>>(q, ldq, head_stride, offset, rot_part, dims, cos_t, sin_t,
                                                                 (float*)out, ldo, out_stride, out_offset, n_heads, lead, total, pairing);
@@ -1165,6 +1297,29 @@ __global__ void gate_heads_kernel(const T* __restrict__ x, int ldx, int x_stride
     Elem<T>::store(out + idx, v);
 }
 
+// The same, eight numbers a thread where sizes and strides are multiples of 8 (8,192 rows of 2,048 of 3,072: 64 us a number a thread).
+template <typename T>
+__global__ void __launch_bounds__(EW_BLOCK)
+gate_heads_vec_kernel(const T* __restrict__ x, int ldx, int x_stride, const float* __restrict__ g, int ldg,
+                      T* __restrict__ out, unsigned n_heads, int n, unsigned total, int gate_one) {
+    const unsigned idx = blockIdx.x * EW_BLOCK + threadIdx.x;
+    if (idx >= total) return;
+    const unsigned pieces = n / 8, th = idx / pieces, t = th / n_heads, h = th - t * n_heads;
+    const int i = (int)(idx - th * pieces) * 8;
+    const T* from = x + (size_t)t * ldx + h * x_stride + i;
+    float4 a = row4(from), b = row4(from + 4);
+    if (g) {
+        const float* gp = g + (size_t)t * ldg + (gate_one ? h : h * n + i);
+        float4 p = gate_one ? make_float4(*gp, *gp, *gp, *gp) : row4(gp), r = gate_one ? p : row4(gp + 4);
+        auto gate = [](float v, float z) { return v * (1.0f / (1.0f + expf(-z))); };
+        a = make_float4(gate(a.x, p.x), gate(a.y, p.y), gate(a.z, p.z), gate(a.w, p.w));
+        b = make_float4(gate(b.x, r.x), gate(b.y, r.y), gate(b.z, r.z), gate(b.w, r.w));
+    }
+    T* to = out + (size_t)idx * 8;
+    store4(to, a.x, a.y, a.z, a.w);
+    store4(to + 4, b.x, b.y, b.z, b.w);
+}
+
 ROCML_EXPORT int rocml_gate_heads(const void* x, int dtype, int ldx, int x_stride, const float* g, int ldg, void* out,
                                   int n_rows, int n_heads, int n, int gate_one, hipStream_t stream) {
     ROCML_REQUIRE(n_rows >= 0 && n_heads > 0 && n > 0 && n <= x_stride && ldx >= n_heads * x_stride &&
@@ -1173,6 +1328,16 @@ ROCML_EXPORT int rocml_gate_heads(const void* x, int dtype, int ldx, int x_strid
     long long total = (long long)n_rows * n_heads * n;
     if (total == 0) return 0;
     int grid = ceil_div(total, EW_BLOCK);
+    if (((n | x_stride | ldx) & 7) == 0 && (gate_one || !g || ldg % 4 == 0) && ((uintptr_t)x & 15) == 0 && ((uintptr_t)out & 15) == 0 &&
+        (gate_one || ((uintptr_t)g & 15) == 0) && total / 8 < 1ll << 31 && (dtype == ROCML_F32 || dtype == ROCML_BF16)) {
+#define LAUNCH(T) gate_heads_vec_kernel<T><<<ceil_div(total / 8, EW_BLOCK), EW_BLOCK, 0, stream>>>((const T*)x, ldx, x_stride, g, ldg, (T*)out, n_heads, n, \
+                                                                                     (unsigned)(total / 8), gate_one)
+        if (dtype == ROCML_F32) LAUNCH(float);
+        else LAUNCH(bf16_t);
+#undef LAUNCH
+        ROCML_CHECK_LAUNCH("gate_heads");
+        return 0;
+    }
     if (dtype == ROCML_F32) gate_heads_kernel<float><<<grid, EW_BLOCK, 0, stream>>>((const float*)x, ldx, x_stride, g, ldg, (float*)out, n_heads, n, total, gate_one);
     else if (dtype == ROCML_BF16) gate_heads_kernel<bf16_t><<<grid, EW_BLOCK, 0, stream>>>((const bf16_t*)x, ldx, x_stride, g, ldg, (bf16_t*)out, n_heads, n, total, gate_one);
     else return rocml_fail("gate_heads: unknown dtype code %d", dtype);
