@@ -1191,7 +1191,40 @@ struct DecayScanArgs {
     float* state; const int* cu_seqlens; const int* seq_slots;
     float* out; int n_heads; int dk; int dv;
     float out_scale;                           // every output is multiplied by it (a scale of the queries)
+    // walks in segments (see below): tokens of one, sequences, [segment, H, dv, dk] states and [segment, H, dk] decays
+    int segment, n_seqs; float* seg_state; float* seg_decay;
 };
+
+// A long sequence in segments, where sequences, heads and columns alone are too few blocks: DECAY_PASS_STATE walks every segment
+// but a sequence's last from a state of zero and keeps the state it ends with and the product of its decays (no output, 0.6 of a
+// walk's work); decay_segments_kernel turns these into the state that every segment starts from; DECAY_PASS_OUT walks all
+// segments from there, side by side.  A sequence's segments are numbered behind those of the sequences before it.
+enum DecayPass : int { DECAY_PASS_ALL = 0, DECAY_PASS_STATE = 1, DECAY_PASS_OUT = 2 };
+struct DecaySegment { int seq, at, of, number; };        // its sequence, place in it, how many that has, the segment's number
+
+// The segment with this number (seq < 0: there are fewer), by a whole wave.
+__device__ __forceinline__ DecaySegment ds_segment(const int* __restrict__ cu_seqlens, int n_seqs, int segment, int number) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    int base = 0;
+    for (int b0 = 0; b0 < n_seqs; b0 += WAVE) {
+        const int b = min(b0 + lane, n_seqs - 1);
+        int mine = b0 + lane < n_seqs ? (cu_seqlens[b + 1] - cu_seqlens[b] + segment - 1) / segment : 0, upto = mine;
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1) {
+            int before = __shfl_up(upto, off, WAVE);
+            upto += lane >= off ? before : 0;
+        }
+        const int from = base + upto - mine;
+        const unsigned long long hit = __ballot(number >= from && number < from + mine);
+        if (hit) {
+            const int who = __ffsll((long long)hit) - 1;
+            return {__builtin_amdgcn_readfirstlane(b0 + who), __builtin_amdgcn_readfirstlane(number - __shfl(from, who, WAVE)),
+                    __builtin_amdgcn_readfirstlane(__shfl(mine, who, WAVE)), number};
+        }
+        base += __shfl(upto, WAVE - 1, WAVE);
+    }
+    return {-1, 0, 0, number};
+}
 
 // The sigmoid form a / (1 + e^x) by one hardware exponential and one hardware reciprocal: both are good to an ulp or so, and
 // where |x| is large enough for the exponent's own rounding to count the result is next to 0 or to a.
@@ -1209,7 +1242,7 @@ enum DecayMode : int { DECAY_HEAD = 0, DECAY_BONUS = 1, DECAY_GATE = 2, DECAY_TO
 // 16 CPL values, and with DECAY_HEAD the token's decay (the head's, or one for the rows beyond the sequence's last
 // token, which then leave the state as it is: with DECAY_BONUS and DECAY_TOKEN their decays are one and their keys zero, with DECAY_GATE their g is).  A lane reads its
 // R numbers of each part as whole vectors at fixed offsets, without a bound to check.
-template <int R, int CPL, int MODE>
+template <int R, int CPL, int MODE, int PASS = DECAY_PASS_ALL>
 __global__ void __launch_bounds__(DS_THREADS)
 decay_scan_kernel(DecayScanArgs a) {
     constexpr bool BONUS = MODE == DECAY_BONUS, GATE = MODE == DECAY_GATE, HEAD = MODE == DECAY_HEAD;
@@ -1226,7 +1259,17 @@ decay_scan_kernel(DecayScanArgs a) {
     int l = tid % DS_LANES, c = tid / DS_LANES;
     int dk = a.dk;
     int col0 = tile * TILE + c * CPL;
+    DecaySegment seg{b, 0, 1, 0};
+    if constexpr (PASS != DECAY_PASS_ALL) {
+        seg = ds_segment(a.cu_seqlens, a.n_seqs, a.segment, blockIdx.x);
+        b = seg.seq;
+        if (b < 0 || (PASS == DECAY_PASS_STATE && seg.at == seg.of - 1)) return;
+    }
     int first = a.cu_seqlens[b], n = a.cu_seqlens[b + 1] - first;
+    if constexpr (PASS != DECAY_PASS_ALL) {
+        first += seg.at * a.segment;
+        n = min(n - seg.at * a.segment, a.segment);
+    }
     float hd = HEAD ? a.head_decay[h] : 0.f;
     // the columns of a chunk's rows that this thread brings in: where they come from, per slot
     const float* src[SLOTS];
@@ -1272,15 +1315,27 @@ decay_scan_kernel(DecayScanArgs a) {
         }
     }
     float* st = a.state + ((size_t)a.seq_slots[b] * a.n_heads + h) * a.dv * dk;
+    if constexpr (PASS != DECAY_PASS_ALL) {          // where the walk's state comes from, or goes to
+        if (PASS == DECAY_PASS_STATE || seg.at > 0) st = a.seg_state + ((size_t)(seg.number - (PASS == DECAY_PASS_OUT)) * a.n_heads + h) * a.dv * dk;
+    }
     float s[CPL][R], u[R];
+    float prod[PASS == DECAY_PASS_STATE ? R : 1];     // the decays of the tokens so far, multiplied (first rows of lanes, first tile)
+    const bool products = PASS == DECAY_PASS_STATE && tile == 0 && tid < WAVE;
     // (a lane's R entries of a column lie side by side: 16-byte pieces where the sizes allow)
-    bool wide = R % 4 == 0 && dk % 4 == 0 && ((uintptr_t)a.state & 15) == 0;
+    bool wide = R % 4 == 0 && dk % 4 == 0 && (((uintptr_t)a.state | (PASS == DECAY_PASS_ALL ? 0 : (uintptr_t)a.seg_state)) & 15) == 0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         int i = l * R + r;
         u[r] = (BONUS && i < dk) ? a.bonus[(size_t)h * dk + i] : 0.f;
     }
-    if (wide) {
+    if constexpr (PASS == DECAY_PASS_STATE) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            prod[r] = 1.f;
+#pragma unroll
+            for (int p = 0; p < CPL; ++p) s[p][r] = 0.f;
+        }
+    } else if (wide) {
         if constexpr (R % 4 == 0) {
 #pragma unroll
             for (int p = 0; p < CPL; ++p)
@@ -1302,7 +1357,15 @@ decay_scan_kernel(DecayScanArgs a) {
     }
     // what a token does to the lane's columns: qq, kk, ww the lane's R numbers of the token's rows, vv its columns' values
     auto token = [&](const float (&qq)[R], const float (&kk)[R], const float (&ww)[R], const float (&vv)[CPL], float dec, float* sums) {
-        if constexpr (BONUS) {
+        if constexpr (PASS == DECAY_PASS_STATE) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+#pragma unroll
+                for (int p = 0; p < CPL; ++p)
+                    s[p][r] = GATE ? fmaf(kk[r], vv[p] - s[p][r], s[p][r]) : fmaf(ROWS ? ww[r] : dec, s[p][r], kk[r] * vv[p]);
+                if (products) prod[r] = GATE ? fmaf(-kk[r], prod[r], prod[r]) : prod[r] * (ROWS ? ww[r] : dec);
+            }
+        } else if constexpr (BONUS) {
             // (S + diag(u) k v^T)^T q = S^T q + v (u . k q): the second part is the same for every column
             float ukq = 0.f;
 #pragma unroll
@@ -1353,6 +1416,15 @@ decay_scan_kernel(DecayScanArgs a) {
         }
     };
     auto keep_state = [&]() {
+        if constexpr (PASS == DECAY_PASS_STATE) {
+            if (products && c == 0)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (l * R + r < dk) a.seg_decay[((size_t)seg.number * a.n_heads + h) * dk + l * R + r] = prod[r];
+        } else if constexpr (PASS == DECAY_PASS_OUT) {
+            if (seg.at < seg.of - 1) return;             // the sequence goes on
+            st = a.state + ((size_t)a.seq_slots[b] * a.n_heads + h) * a.dv * dk;
+        }
         if (wide) {
             if constexpr (R % 4 == 0) {
 #pragma unroll
@@ -1374,7 +1446,7 @@ decay_scan_kernel(DecayScanArgs a) {
                 if (col0 + p < a.dv && i < dk) st[(size_t)(col0 + p) * dk + i] = s[p][r];
         }
     };
-    if (n == 1) {
+    if (PASS == DECAY_PASS_ALL && n == 1) {
         // One token (a decode step): its numbers come straight from memory, beside the state's; the same arithmetic.
         float qq[R], kk[R], ww[R], vv[CPL], sums[CPL];
         size_t t = (size_t)first;
@@ -1504,6 +1576,7 @@ decay_scan_kernel(DecayScanArgs a) {
                 if constexpr (HEAD) dec = vals[TILE];
                 token(qq, kk, ww, vv, dec, acc + jj * CPL);
             }
+            if constexpr (PASS == DECAY_PASS_STATE) continue;
 #pragma unroll
             for (int i = 0; i < NV; ++i) acc[i] = row16_sum(acc[i]);
             float out_val = acc[0];
@@ -1518,23 +1591,73 @@ decay_scan_kernel(DecayScanArgs a) {
     keep_state();
 }
 
-template <int R, int CPL>
-static void launch_decay_scan_cols(const DecayScanArgs& a, int n_seqs, hipStream_t stream) {
-    dim3 grid(n_seqs, a.n_heads, ceil_div(a.dv, DS_GROUPS * CPL));
-    if (a.w && !a.bonus) decay_scan_kernel<R, CPL, DECAY_TOKEN><<<grid, DS_THREADS, 0, stream>>>(a);
-    else if (a.bonus) decay_scan_kernel<R, CPL, DECAY_BONUS><<<grid, DS_THREADS, 0, stream>>>(a);
-    else if (a.gate_lower) decay_scan_kernel<R, CPL, DECAY_GATE><<<grid, DS_THREADS, 0, stream>>>(a);
-    else decay_scan_kernel<R, CPL, DECAY_HEAD><<<grid, DS_THREADS, 0, stream>>>(a);
+// The states that the segments of a sequence start from, in place: the slot of segment i goes from what that segment adds to the state
+// behind it.  A thread has four entries of a head's state, dk along a column; the states of eight segments are asked for together.
+__global__ void __launch_bounds__(256)
+decay_segments_kernel(DecayScanArgs a) {
+    const int b = blockIdx.z, h = blockIdx.y, dk = a.dk, e = (blockIdx.x * 256 + threadIdx.x) * 4;
+    int number = 0;                                      // of the sequence's first segment
+    for (int i = threadIdx.x & (WAVE - 1); i < b; i += WAVE) number += (a.cu_seqlens[i + 1] - a.cu_seqlens[i] + a.segment - 1) / a.segment;
+#pragma unroll
+    for (int off = WAVE / 2; off > 0; off >>= 1) number += __shfl_xor(number, off, WAVE);
+    const int n_segs = (a.cu_seqlens[b + 1] - a.cu_seqlens[b] + a.segment - 1) / a.segment;
+    if (n_segs < 2 || e >= a.dv * dk) return;
+    float4 s = *(const float4*)(a.state + ((size_t)a.seq_slots[b] * a.n_heads + h) * a.dv * dk + e);
+    constexpr int AHEAD = 8;
+    for (int i0 = 0; i0 < n_segs - 1; i0 += AHEAD) {
+        float4 own[AHEAD], w[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const size_t row = (size_t)(number + min(i0 + i, n_segs - 2)) * a.n_heads + h;
+            own[i] = *(const float4*)(a.seg_state + row * a.dv * dk + e);
+            w[i] = *(const float4*)(a.seg_decay + row * dk + e % dk);
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            if (i0 + i >= n_segs - 1) break;
+            s.x = fmaf(w[i].x, s.x, own[i].x); s.y = fmaf(w[i].y, s.y, own[i].y);
+            s.z = fmaf(w[i].z, s.z, own[i].z); s.w = fmaf(w[i].w, s.w, own[i].w);
+            *(float4*)(a.seg_state + ((size_t)(number + i0 + i) * a.n_heads + h) * a.dv * dk + e) = s;
+        }
+    }
+}
+
+template <int R, int CPL, int PASS>
+static void launch_decay_scan_pass(const DecayScanArgs& a, int n_blocks, hipStream_t stream) {
+    dim3 grid(n_blocks, a.n_heads, ceil_div(a.dv, DS_GROUPS * CPL));
+    if (a.w && !a.bonus) decay_scan_kernel<R, CPL, DECAY_TOKEN, PASS><<<grid, DS_THREADS, 0, stream>>>(a);
+    else if (a.bonus) decay_scan_kernel<R, CPL, DECAY_BONUS, PASS><<<grid, DS_THREADS, 0, stream>>>(a);
+    else if (a.gate_lower) decay_scan_kernel<R, CPL, DECAY_GATE, PASS><<<grid, DS_THREADS, 0, stream>>>(a);
+    else decay_scan_kernel<R, CPL, DECAY_HEAD, PASS><<<grid, DS_THREADS, 0, stream>>>(a);
 }
 
 template <int R>
-static void launch_decay_scan(const DecayScanArgs& a, int n_seqs, hipStream_t stream) {
-        // Two columns per lane (a lane's reads of q, k and the decays then serve both) where blocks of 16 columns would be
+static void launch_decay_scan(const DecayScanArgs& a, int n_seqs, int n_segments, hipStream_t stream) {
+    // Two columns per lane (a lane's reads of q, k and the decays then serve both) where blocks of 16 columns would be
     // more than two a CU: measured on 8 x 2,048 tokens of 32 heads of 64 x 64 at 0.76 ms against 1.06 with one column
     // and 0.76 with four; a single sequence, whose blocks are fewer than the CUs, is faster with one (0.47 against 0.52).
+    if constexpr (R % 4 == 0 && R <= 8) {
+        if (a.segment) {
+            launch_decay_scan_pass<R, 2, DECAY_PASS_STATE>(a, n_segments, stream);
+            decay_segments_kernel<<<dim3(ceil_div(a.dv * a.dk, 1024), a.n_heads, n_seqs), 256, 0, stream>>>(a);
+            launch_decay_scan_pass<R, 2, DECAY_PASS_OUT>(a, n_segments, stream);
+            return;
+        }
+    }
     long long blocks = (long long)n_seqs * a.n_heads * ceil_div(a.dv, DS_GROUPS);
-    if (R <= 8 && a.dv > DS_GROUPS && blocks > 2ll * cu_count()) launch_decay_scan_cols<R, R <= 8 ? 2 : 1>(a, n_seqs, stream);
-    else launch_decay_scan_cols<R, 1>(a, n_seqs, stream);
+    if (R <= 8 && a.dv > DS_GROUPS && blocks > 2ll * cu_count()) launch_decay_scan_pass<R, R <= 8 ? 2 : 1, DECAY_PASS_ALL>(a, n_seqs, stream);
+    else launch_decay_scan_pass<R, 1, DECAY_PASS_ALL>(a, n_seqs, stream);
+}
+
+// Tokens of a segment, or 0 where whole sequences are faster.  A walk alone takes some 0.23 us a token of the longest sequence whatever
+// else the chip does (twice that with two blocks a CU); in segments the chip is full, and both passes together are bound by
+// their arithmetic: 0.26 us a token, head and 32 columns of 128 entries over all CUs, beside 30 us.  Microseconds whole and in segments (16 heads of
+// 128 x 128): one sequence of 8,192 tokens 1,861 and 512, of 700 161 and 75; five of 300 to 2,500 712 and 453; eight of 2,048
+// 683 and 1,040.  Segments of 64 for 128 are faster while they are few (700 tokens: 75 for 98), of 256 equal.
+static int decay_segment(int longest, int n_tokens, int n_heads, int dk, int dv) {
+    const int tokens = longest >= 1024 ? 128 : 64;
+    const double both = 30.0 + 0.26 * n_tokens * n_heads * ceil_div(dv, 2 * DS_GROUPS) * (dk > 64 ? 1.0 : 0.6) / cu_count();
+    return longest >= 4 * tokens && 0.23 * (dk > 64 ? 1.0 : 0.85) * longest > 1.1 * both ? tokens : 0;
 }
 
 ROCML_EXPORT int rocml_decay_scan(const float* q, int ldq, int q_col0, const float* k, int ldk, int k_col0, const float* v,
@@ -1542,7 +1665,9 @@ ROCML_EXPORT int rocml_decay_scan(const float* q, int ldq, int q_col0, const flo
                                   const float* head_decay, const float* bonus, const float* gate_lower, const float* gate_bias,
                                   float* state, int n_slots, const int* cu_seqlens,
                                   const int* seq_slots, int n_seqs, int n_tokens, float* out, int n_heads, int dk, int dv,
-                                  float out_scale, hipStream_t stream) {
+                                  float out_scale, void* workspace, long long workspace_bytes, int longest, int segment, hipStream_t stream) {
+    // workspace (may be null): memory for a walk in segments; longest: tokens of the longest sequence (0: not known, the mean is
+    // taken); segment: 0 = choose, -1 = never, else tokens of one (a multiple of 16)
     ROCML_REQUIRE(n_tokens >= 0 && n_seqs >= 0 && n_slots > 0 && n_heads > 0 && dk > 0 && dv > 0, "decay_scan: bad sizes T=%d B=%d H=%d",
                   n_tokens, n_seqs, n_heads);
     ROCML_REQUIRE(dk <= 16 * DS_LANES, "decay_scan: a key size of %d exceeds %d", dk, 16 * DS_LANES);
@@ -1556,13 +1681,27 @@ ROCML_EXPORT int rocml_decay_scan(const float* q, int ldq, int q_col0, const flo
                   "decay_scan: a row stride is too small for its columns");
     if (n_tokens == 0 || n_seqs == 0) return 0;
     DecayScanArgs a{q, ldq, q_col0, k, ldk, k_col0, v, ldv, v_col0, w, ldw, w_col0, w_offset, head_decay, bonus, gate_lower, gate_bias, state, cu_seqlens,
-                    seq_slots, out, n_heads, dk, dv, out_scale};
+                    seq_slots, out, n_heads, dk, dv, out_scale, 0, n_seqs, nullptr, nullptr};
     int r = ceil_div(dk, DS_LANES);
-    if (r <= 1) launch_decay_scan<1>(a, n_seqs, stream);
-    else if (r <= 2) launch_decay_scan<2>(a, n_seqs, stream);
-    else if (r <= 4) launch_decay_scan<4>(a, n_seqs, stream);
-    else if (r <= 8) launch_decay_scan<8>(a, n_seqs, stream);
-    else launch_decay_scan<16>(a, n_seqs, stream);
+    ROCML_REQUIRE(segment >= -1 && segment % DS_CHUNK == (segment < 0 ? -1 : 0), "decay_scan: segments of %d tokens", segment);
+    int n_segments = 0;
+    if (segment >= 0 && r > 2 && r <= 8 && dk % 4 == 0 && workspace && (((uintptr_t)state | (uintptr_t)workspace) & 15) == 0 && n_seqs < 65536) {
+        if (segment == 0) segment = decay_segment(longest > 0 ? longest : n_tokens / n_seqs, n_tokens, n_heads, dk, dv);
+        const long long most = workspace_bytes / ((long long)n_heads * (dv + 1) * dk * 4);
+        while (segment && segment < n_tokens && n_tokens / segment + n_seqs > most) segment *= 2;       // (as many as the memory holds)
+        const long long count = segment ? n_tokens / segment + n_seqs : 0;
+        if (count > n_seqs && count <= most && count < 1 << 24) {
+            n_segments = (int)count;
+            a.segment = segment;
+            a.seg_state = (float*)workspace;
+            a.seg_decay = a.seg_state + (size_t)count * n_heads * dv * dk;
+        }
+    }
+    if (r <= 1) launch_decay_scan<1>(a, n_seqs, 0, stream);
+    else if (r <= 2) launch_decay_scan<2>(a, n_seqs, 0, stream);
+    else if (r <= 4) launch_decay_scan<4>(a, n_seqs, n_segments, stream);
+    else if (r <= 8) launch_decay_scan<8>(a, n_seqs, n_segments, stream);
+    else launch_decay_scan<16>(a, n_seqs, 0, stream);
     ROCML_CHECK_LAUNCH("decay_scan");
     return 0;
 }

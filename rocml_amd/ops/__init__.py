@@ -63,7 +63,7 @@ _SIGNATURES = {
         "rocml_mlstm_scan": [_P, _I, _I, _I, _I, _I, _I, _P, _P, _F, _F, _F, _P, _P, _P, _I, _P, _P, _I, _I, _P, _I, _I, _I, _P],
         "rocml_mlstm_tile": [],
         "rocml_head_norm_gate": [_P, _P, _I, _I, _P, _P, _I, _I, _I, _I, _F, _I, _P],
-        "rocml_decay_scan": [_P, _I, _I, _P, _I, _I, _P, _I, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _P, _I, _I, _I, _F, _P],
+        "rocml_decay_scan": [_P, _I, _I, _P, _I, _I, _P, _I, _I, _P, _I, _I, _P, _P, _P, _P, _P, _P, _I, _P, _P, _I, _I, _P, _I, _I, _I, _F, _P, _LL, _I, _I, _P],
         "rocml_low_rank_decay": [_P, _I, _I, _P, _I, _P, _F, _P, _I, _I, _I, _P],
         "rocml_rotate_rows": [_P, _I, _I, _I, _I, _I, _I, _P, _P, _F, _I, _F, _P],
         "rocml_shift_mix": [_P, _I, _I, _I, _P, _I, _P, _I, _P, _P, _P, _I, _P, _P],
@@ -1489,7 +1489,8 @@ def decay_scan(q: torch.Tensor, q_col0: int, k: torch.Tensor, k_col0: int, v: to
                n_heads: int, head_dim: int, v_head_dim: int, head_decay: Optional[torch.Tensor] = None,
                decay: Optional[torch.Tensor] = None, decay_col0: int = 0, bonus: Optional[torch.Tensor] = None,
                decay_offset: Optional[torch.Tensor] = None, gate_lower: Optional[torch.Tensor] = None,
-               gate_bias: Optional[torch.Tensor] = None, out_scale: float = 1.0) -> None:
+               gate_bias: Optional[torch.Tensor] = None, out_scale: float = 1.0,
+               workspace: Optional[torch.Tensor] = None, longest: int = 0, segment: int = 0) -> None:
     """A recurrence whose state per head, ``S [dk, dv]``, decays row by row, over the step's tokens, per sequence in
     order: ``S <- diag(w_t) S + k_t v_t^T``.  With ``head_decay`` (one number per head) ``w_t`` is that constant and
     the output reads the new state, ``o_t = S_t^T q_t``; with ``decay`` (per token and key channel, columns
@@ -1498,8 +1499,10 @@ def decay_scan(q: torch.Tensor, q_col0: int, k: torch.Tensor, k_col0: int, v: to
     decay is ``exp(-exp(x + decay_offset))``.  With ``gate_lower`` ``l`` and ``gate_bias`` ``b`` (``[H * dk]`` each) ``k`` holds the
     logits of a forget gate ``f = l + (1 - l) sigmoid(k + b)`` that decides what is written too, ``S <- diag(f) S + (1 - f) v^T``,
     ``o = S^T silu(q)`` with the new state.  ``out_scale`` multiplies every output.  q, k, v are column ranges of 32-bit matrices ``[T, ld]``;
-    ``state [slots, H, dv, dk]``; ``out [T, H * dv]``; all 32-bit."""
-    _dev(q, k, v, state, cu_seqlens, seq_slots, out, head_decay, decay, bonus, decay_offset, gate_lower, gate_bias)
+    ``state [slots, H, dv, dk]``; ``out [T, H * dv]``; all 32-bit.  With ``workspace`` (device memory) long sequences are walked
+    in segments side by side where they alone would leave the chip idle; ``longest``: tokens of the longest (0: not known); ``segment``: tokens of one (a multiple of 16; 0: as the
+    kernels see fit, -1: never)."""
+    _dev(q, k, v, state, cu_seqlens, seq_slots, out, head_decay, decay, bonus, decay_offset, gate_lower, gate_bias, workspace)
     for t, what in ((q, "queries"), (k, "keys"), (v, "values"), (state, "recurrent state"), (out, "recurrence output")):
         _want(t, torch.float32, what)
     n_tokens, n_seqs = out.shape[0], seq_slots.numel()
@@ -1526,7 +1529,8 @@ def decay_scan(q: torch.Tensor, q_col0: int, k: torch.Tensor, k_col0: int, v: to
         0 if decay is None else decay.shape[1], decay_col0, _ptr(decay_offset), _ptr(head_decay), _ptr(bonus), _ptr(gate_lower),
         _ptr(gate_bias), _ptr(state),
         state.shape[0],
-        _ptr(cu_seqlens), _ptr(seq_slots), n_seqs, n_tokens, _ptr(out), n_heads, head_dim, v_head_dim, float(out_scale), _stream()))
+        _ptr(cu_seqlens), _ptr(seq_slots), n_seqs, n_tokens, _ptr(out), n_heads, head_dim, v_head_dim, float(out_scale),
+        _ptr(workspace), 0 if workspace is None else workspace.numel() * workspace.element_size(), int(longest), int(segment), _stream()))
 
 
 def low_rank_decay(low: torch.Tensor, low_col0: int, w: torch.Tensor, bias: Optional[torch.Tensor], tau: float, out: torch.Tensor) -> None:

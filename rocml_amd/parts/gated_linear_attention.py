@@ -98,7 +98,8 @@ class GatedLinearAttention(Mixer):
         ops.low_rank_decay(proj, c0 + self.low_col, self.a2, self.a2_bias, s.tau, decay)
         o = ws.get("gla.o", (n, self.v_dim), torch.float32)
         ops.decay_scan(proj, c0, proj, c0 + self.k_col, proj, c0 + self.v_col, cache.state, step.cu_seqlens, step.seq_slots, o,
-                       s.n_heads, s.head_dim, s.v_head_dim, decay=decay, out_scale=float(s.head_dim) ** -0.5)
+                       s.n_heads, s.head_dim, s.v_head_dim, decay=decay, out_scale=float(s.head_dim) ** -0.5,
+                       workspace=ws.scratch(), longest=step.max_new)
         gated = ws.get("gla.gated", (n, self.v_dim), self.dtype)
         ops.head_norm_gate(o, proj, c0 + self.g_col, self.norm_gain, gated, s.n_heads, s.eps, gate="silu")
         stream(step).add_product(gated, self.w_out, x_accum)

@@ -89,7 +89,8 @@ class Hgrn2(Mixer):
             ops.gemm(xn, self.w_in, proj, workspace=ws.scratch())
         o = ws.get("hgrn2.o", (n, self.v_dim), torch.float32)
         ops.decay_scan(proj, c0, proj, c0 + self.f_col, proj, c0 + self.v_col, cache.state, step.cu_seqlens, step.seq_slots, o,
-                       s.n_heads, s.head_dim, s.v_head_dim, gate_lower=self.lower, gate_bias=self.f_bias)
+                       s.n_heads, s.head_dim, s.v_head_dim, gate_lower=self.lower, gate_bias=self.f_bias,
+                       workspace=ws.scratch(), longest=step.max_new)
         normed = ws.get("hgrn2.normed", (n, self.v_dim), self.dtype)
         ops.head_norm_gate(o, None, 0, self.norm_gain, normed, s.n_heads, s.eps, gate=None)
         stream(step).add_product(normed, self.w_out, x_accum)

@@ -93,7 +93,7 @@ class Retention(Mixer):
                         scale_rest=float(s.head_dim) ** -0.5)
         o = ws.get("retention.o", (n, self.v_dim), torch.float32)
         ops.decay_scan(proj, 0, proj, self.k_col, proj, self.v_col, cache.state, step.cu_seqlens, step.seq_slots, o,
-                       s.n_heads, s.head_dim, s.v_head_dim, head_decay=self.decay)
+                       s.n_heads, s.head_dim, s.v_head_dim, head_decay=self.decay, workspace=ws.scratch(), longest=step.max_new)
         gated = ws.get("retention.gated", (n, self.v_dim), self.dtype)
         ops.head_norm_gate(o, proj, self.g_col, None, gated, s.n_heads, s.eps, gate="silu")
         stream(step).add_product(gated, self.w_out, x_accum)

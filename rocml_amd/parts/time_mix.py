@@ -97,7 +97,8 @@ class TimeMix(Mixer):
         o = ws.get("timemix.o", (n, self.inner), torch.float32)
         # (the recurrence kernel turns the logits into decays, exp(-exp(x + w0)), on their way into its LDS)
         ops.decay_scan(proj, 0, proj, self.inner, proj, 2 * self.inner, state.state, step.cu_seqlens, step.seq_slots, o,
-                       s.n_heads, s.head_dim, s.head_dim, decay=decay, decay_col0=0, bonus=self.bonus, decay_offset=self.w0)
+                       s.n_heads, s.head_dim, s.head_dim, decay=decay, decay_col0=0, bonus=self.bonus, decay_offset=self.w0,
+                       workspace=ws.scratch(), longest=step.max_new)
         gated = ws.get("timemix.gated", (n, self.inner), self.dtype)
         ops.head_norm_gate(o, proj, 3 * self.inner, self.norm_gain, gated, s.n_heads, s.eps, gate="silu")
         stream(step).add_product(gated, self.w_out, x_accum)
