@@ -142,6 +142,7 @@ struct LatentArgs {
     const bf16_t* q; bf16_t* out; const bf16_t* cache; const int* block_table; int bt_width;
     const int* cu_seqlens; int n_seqs; const int* token_pos; int n_tokens; int n_heads; int dk; int dv;
     float scale; int window; int tiles; void* workspace; long long workspace_bytes;
+    bool few;                                         // every sequence has 1 to 16 rows of work
 };
 
 template <int KD, int DT, int RT>
@@ -150,6 +151,7 @@ static int launch_latent(const LatentArgs& a, hipStream_t stream) {
     static bool ready = false;
     if (!ready) {
         if (allow_lds(attn_latent_mfma_kernel<KD, DT, RT>, L::BYTES)) return 1;
+        if (allow_lds(attn_latent_few_kernel<KD, DT>, L::BYTES)) return 1;
         ready = true;
     }
     // Splits of the key range: enough blocks for one a CU, at most one per two pieces the rows can see
@@ -166,9 +168,14 @@ static int launch_latent(const LatentArgs& a, hipStream_t stream) {
     if (n_splits < 1) n_splits = 1;
     float* part_o = (float*)a.workspace;
     float* part_ml = part_o ? part_o + rows * n_splits * a.dv : nullptr;
-    attn_latent_mfma_kernel<KD, DT, RT><<<dim3(a.tiles, n_splits), 256, L::BYTES, stream>>>(
-        a.q, a.out, a.cache, a.block_table, a.bt_width, a.cu_seqlens, a.n_seqs, a.token_pos, a.n_heads, a.dk, a.dv,
-        a.scale * LOG2E, a.window, n_splits, part_o, part_ml);
+    if (a.few)
+        attn_latent_few_kernel<KD, DT><<<dim3(a.n_seqs, n_splits), 256, L::BYTES, stream>>>(
+            a.q, a.out, a.cache, a.block_table, a.bt_width, a.cu_seqlens, a.token_pos, a.n_heads, a.dk, a.dv,
+            a.scale * LOG2E, a.window, n_splits, part_o, part_ml);
+    else
+        attn_latent_mfma_kernel<KD, DT, RT><<<dim3(a.tiles, n_splits), 256, L::BYTES, stream>>>(
+            a.q, a.out, a.cache, a.block_table, a.bt_width, a.cu_seqlens, a.n_seqs, a.token_pos, a.n_heads, a.dk, a.dv,
+            a.scale * LOG2E, a.window, n_splits, part_o, part_ml);
     if (n_splits > 1) {
         if (n_splits <= 8) launch_latent_reduce<1>(part_o, part_ml, a.out, rows, n_splits, a.dv, stream);
         else if (n_splits <= 16) launch_latent_reduce<2>(part_o, part_ml, a.out, rows, n_splits, a.dv, stream);
@@ -254,10 +261,14 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
         int kd = (d + 31) / 32, dt = (dv + 15) / 16;
         int rt = (long long)n_tokens * hq >= 128ll * n_seqs && kd <= 10 && dt <= 16 ? 2 : 1;
         long long tiles = 0;
-        for (int b = 0; b < n_seqs; ++b) tiles += ((long long)q_counts[b] * hq + AL_ROWS * rt - 1) / (AL_ROWS * rt);
+        bool few = true;
+        for (int b = 0; b < n_seqs; ++b) {
+            tiles += ((long long)q_counts[b] * hq + AL_ROWS * rt - 1) / (AL_ROWS * rt);
+            few = few && q_counts[b] >= 1 && (long long)q_counts[b] * hq <= 16;
+        }
         ROCML_REQUIRE(tiles > 0 && tiles < (1ll << 31), "attention: %lld row tiles", tiles);
         LatentArgs a{(const bf16_t*)q, (bf16_t*)out, (const bf16_t*)kcache, block_table, bt_width, cu_seqlens, n_seqs,
-                     token_pos, n_tokens, hq, d, dv, scale, window, (int)tiles, workspace, workspace_bytes};
+                     token_pos, n_tokens, hq, d, dv, scale, window, (int)tiles, workspace, workspace_bytes, few};
 #define BY_ROW_TILES(KD_, DT_) (rt == 2 ? launch_latent<KD_, DT_, 2>(a, stream) : launch_latent<KD_, DT_, 1>(a, stream))
         int rc = kd <= 3 && dt <= 4     ? BY_ROW_TILES(3, 4)
                  : kd <= 6 && dt <= 8   ? BY_ROW_TILES(6, 8)

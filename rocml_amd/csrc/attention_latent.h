@@ -48,6 +48,54 @@ struct LatentLds {
     static constexpr int BYTES = (AL_KEYS * K_ROW + DT * 16 * AL_VROW + DT * 2 * 32) * 2;
 };
 
+// A piece on its way from memory to LDS: a thread takes the two keys of a column (see above) and 8 numbers of both.
+template <int KD, int DT>
+struct LatentPiece {
+    using L = LatentLds<KD, DT>;
+    static constexpr int MAX_ITEMS = (AL_KEYS / 2) * (KD * 4) / 256 + 1;
+    const bf16_t* cache; const int* pages; int dk, dv, tid;
+    uint4 ra[MAX_ITEMS], rb[MAX_ITEMS];
+
+    __device__ __forceinline__ void request(int piece) {
+        const int key0 = piece * AL_KEYS, items = (AL_KEYS / 2) * (dk / 8);
+        int phys = max(pages[key0 / AM_PAGE], 0);       // (a page that is not there holds no visible key)
+        const bf16_t* base = cache + ((size_t)phys * AM_PAGE + key0 % AM_PAGE) * dk;
+#pragma unroll
+        for (int i = 0; i < MAX_ITEMS; ++i) {
+            int w = tid + i * 256;
+            if (w < items) {
+                int c = w & 15, dc = w >> 4;            // 16 neighbouring lanes: the 16 columns, the same 8 numbers
+                int ka = 8 * (c >> 2) + (c & 3);
+                ra[i] = *(const uint4*)(base + (size_t)ka * dk + dc * 8);
+                rb[i] = *(const uint4*)(base + (size_t)(ka + 4) * dk + dc * 8);
+            }
+        }
+    }
+    __device__ __forceinline__ void store(bf16_t* sk, bf16_t* sv) const {
+        const int items = (AL_KEYS / 2) * (dk / 8), dv8 = dv / 8;
+#pragma unroll
+        for (int i = 0; i < MAX_ITEMS; ++i) {
+            int w = tid + i * 256;
+            if (w < items) {
+                int c = w & 15, dc = w >> 4;
+                *(uint4*)(sk + c * L::K_ROW + dc * 8) = ra[i];
+                *(uint4*)(sk + (16 + c) * L::K_ROW + dc * 8) = rb[i];
+                if (dc < dv8) {
+                    const uint32_t a[4] = {ra[i].x, ra[i].y, ra[i].z, ra[i].w};
+                    const uint32_t bw[4] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
+                    uint32_t* dst = (uint32_t*)(sv + al_vrow_at(dc * 8) + 2 * c);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        // numbers 2j and 2j + 1 of both keys, the two keys side by side
+                        dst[(2 * j) * (AL_VROW / 2)] = (a[j] & 0xffffu) | (bw[j] << 16);
+                        dst[(2 * j + 1) * (AL_VROW / 2)] = (a[j] >> 16) | (bw[j] & 0xffff0000u);
+                    }
+                }
+            }
+        }
+    }
+};
+
 template <int KD, int DT, int RT>
 __global__ void __launch_bounds__(256)
 attn_latent_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ cache,
@@ -113,56 +161,14 @@ attn_latent_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, 
         for (int i = 0; i < DT; ++i) o[rt][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
 
-    // A piece on its way: a thread takes the two keys of a column (see above) and 8 numbers of both.
-    int dk8 = dk / 8, dv8 = dv / 8;
-    int items = (AL_KEYS / 2) * dk8;
-    constexpr int MAX_ITEMS = (AL_KEYS / 2) * (KD * 4) / 256 + 1;
-    uint4 ra[MAX_ITEMS], rb[MAX_ITEMS];
-    auto request_piece = [&](int piece) {
-        int key0 = piece * AL_KEYS;
-        int phys = max(pages[key0 / AM_PAGE], 0);       // (a page that is not there holds no visible key)
-        const bf16_t* base = cache + ((size_t)phys * AM_PAGE + key0 % AM_PAGE) * dk;
-#pragma unroll
-        for (int i = 0; i < MAX_ITEMS; ++i) {
-            int w = tid + i * 256;
-            if (w < items) {
-                int c = w & 15, dc = w >> 4;            // 16 neighbouring lanes: the 16 columns, the same 8 numbers
-                int ka = 8 * (c >> 2) + (c & 3);
-                ra[i] = *(const uint4*)(base + (size_t)ka * dk + dc * 8);
-                rb[i] = *(const uint4*)(base + (size_t)(ka + 4) * dk + dc * 8);
-            }
-        }
-    };
-    auto store_piece = [&]() {
-#pragma unroll
-        for (int i = 0; i < MAX_ITEMS; ++i) {
-            int w = tid + i * 256;
-            if (w < items) {
-                int c = w & 15, dc = w >> 4;
-                *(uint4*)(sk + c * L::K_ROW + dc * 8) = ra[i];
-                *(uint4*)(sk + (16 + c) * L::K_ROW + dc * 8) = rb[i];
-                if (dc < dv8) {
-                    const uint32_t a[4] = {ra[i].x, ra[i].y, ra[i].z, ra[i].w};
-                    const uint32_t bw[4] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
-                    uint32_t* dst = (uint32_t*)(sv + al_vrow_at(dc * 8) + 2 * c);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        // numbers 2j and 2j + 1 of both keys, the two keys side by side
-                        dst[(2 * j) * (AL_VROW / 2)] = (a[j] & 0xffffu) | (bw[j] << 16);
-                        dst[(2 * j + 1) * (AL_VROW / 2)] = (a[j] >> 16) | (bw[j] & 0xffff0000u);
-                    }
-                }
-            }
-        }
-    };
-
+    LatentPiece<KD, DT> next{cache, pages, dk, dv, tid};
     int piece = first_piece + split;
-    if (piece <= last_piece) request_piece(piece);
+    if (piece <= last_piece) next.request(piece);
     for (; piece <= last_piece; piece += n_splits) {
         __syncthreads();                 // the piece before has been multiplied (first round: the zeros are written)
-        store_piece();
+        next.store(sk, sv);
         __syncthreads();
-        if (piece + n_splits <= last_piece) request_piece(piece + n_splits);
+        if (piece + n_splits <= last_piece) next.request(piece + n_splits);
         int key0 = piece * AL_KEYS;
         if (!wave_active || key0 > wave_hi || key0 + AL_KEYS - 1 < wave_lo) continue;      // wave-uniform
         // scores of 2 x 16 keys: row r of tile u is key 8 (r / 4) + 4 u + r % 4, so that element i of
@@ -262,6 +268,118 @@ attn_latent_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, 
     }
 }
 
+// A decode step whose sequences have at most 16 rows of work each: one block per sequence and split, whose four waves share the rows.  Of a piece's
+// scores a wave forms 16 keys over half of the numbers, the halves meet in LDS, every wave forms the probabilities of all 32
+// keys (the same in each) and a quarter of the output's numbers.  Bound by its chain of trips and barriers: with the rows in one
+// wave (the other three only loading), the sequence looked up by one load after the other and the LDS zeroed ahead of every launch,
+// 8 sequences of 1,024 keys (16 heads, 576 and 512 numbers) took 17 us.  A split without a key writes no output: its weight is zero.
+template <int KD, int DT>
+__global__ void __launch_bounds__(256)
+attn_latent_few_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ cache,
+                       const int* __restrict__ block_table, int bt_width, const int* __restrict__ cu_seqlens,
+                       const int* __restrict__ token_pos, int n_heads, int dk, int dv,
+                       float scale_log2e, int window, int n_splits, float* __restrict__ part_o,
+                       float* __restrict__ part_ml) {
+    using L = LatentLds<KD, DT>;
+    constexpr int KH = (KD + 1) / 2, DW = DT / 4;     // steps of a half of the numbers, output tiles of a wave
+    extern __shared__ uint4 al_smem[];
+    __shared__ f32x4_t halves[2][2][64];              // [half of the numbers][16 keys]: sums of a wave
+    bf16_t* sk = (bf16_t*)al_smem;
+    bf16_t* sv = sk + AL_KEYS * L::K_ROW;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, col = lane & 15;
+    const int b = blockIdx.x, split = blockIdx.y;
+    const int tok0 = cu_seqlens[b], n_rows = (cu_seqlens[b + 1] - tok0) * n_heads, pos0 = token_pos[tok0];
+    const int* pages = block_table + (size_t)b * bt_width;
+    const bool row_ok = col < n_rows;
+    const int my_pos = pos0 + min(col, n_rows - 1) / n_heads, my_lo = window > 0 ? max(0, my_pos - window + 1) : 0;
+    const size_t grow = (size_t)tok0 * n_heads + min(col, n_rows - 1);
+    const int lo = window > 0 ? max(0, pos0 - window + 1) : 0, hi = pos0 + (n_rows - 1) / n_heads;     // keys that any row sees
+    const int last_piece = hi / AL_KEYS;
+    int piece = lo / AL_KEYS + split;
+    LatentPiece<KD, DT> next{cache, pages, dk, dv, tid};
+    if (piece <= last_piece) next.request(piece);
+    const int u_mine = wave & 1, half = wave >> 1;
+    bf16x8_t qf[KH];
+#pragma unroll
+    for (int i = 0; i < KH; ++i) {
+        const int at = (half * KH + i) * 32 + g * 8;
+        uint4 v = row_ok && half * KH + i < KD && at < dk ? *(const uint4*)(q + grow * dk + at) : make_uint4(0u, 0u, 0u, 0u);
+        qf[i] = __builtin_bit_cast(bf16x8_t, v);
+    }
+    if (dk < KD * 32 || dv < DT * 16) {               // zeros where the sizes stop short of the tiles: never written again
+        for (int i = tid; i < L::BYTES / 16; i += 256) al_smem[i] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    float m = -INFINITY, l = 0.f;
+    f32x4_t o[DW];
+#pragma unroll
+    for (int i = 0; i < DW; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const bool any = piece <= last_piece;
+    for (; piece <= last_piece; piece += n_splits) {
+        __syncthreads();                              // the piece before has been multiplied (first round: the zeros are written)
+        next.store(sk, sv);
+        __syncthreads();
+        if (piece + n_splits <= last_piece) next.request(piece + n_splits);
+        f32x4_t part = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        const bf16_t* krow = sk + (16 * u_mine + col) * L::K_ROW + half * KH * 32 + g * 8;
+#pragma unroll
+        for (int i = 0; i < KH; ++i)
+            if (half * KH + i < KD)
+                part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, *(const uint4*)(krow + i * 32)), qf[i], part, 0, 0, 0);
+        halves[half][u_mine][lane] = part;
+        __syncthreads();
+        f32x4_t s[2];
+        float mx = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            s[u] = halves[0][u][lane] + halves[1][u][lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int key = piece * AL_KEYS + g * 8 + u * 4 + i;
+                s[u][i] = row_ok && key >= my_lo && key <= my_pos ? s[u][i] * scale_log2e : -INFINITY;
+                mx = fmaxf(mx, s[u][i]);
+            }
+        }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float m_new = fmaxf(m, mx), m_use = m_new == -INFINITY ? 0.f : m_new, corr = fast_exp2(m - m_use);
+        float sum = 0.f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[u][i] = fast_exp2(s[u][i] - m_use);
+                sum += s[u][i];
+            }
+        sum += __shfl_xor(sum, 16, 64);
+        sum += __shfl_xor(sum, 32, 64);
+        l = l * corr + sum;
+        m = m_new;
+        // P^T operand: slot 2 i + u = key 8 g + 4 u + i, the order of the transposed copy
+        const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack_bf16x2(s[0][0], s[1][0]), pack_bf16x2(s[0][1], s[1][1]),
+                                                                     pack_bf16x2(s[0][2], s[1][2]), pack_bf16x2(s[0][3], s[1][3])));
+#pragma unroll
+        for (int i = 0; i < DW; ++i) {
+            const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, *(const uint4*)(sv + al_vrow_at((wave * DW + i) * 16 + col) + g * 8));
+            o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[i] * corr, 0, 0, 0);
+        }
+    }
+    if (!row_ok) return;
+    const size_t slot = grow * n_splits + split;
+    if (n_splits > 1 && wave == 0 && g == 0) {
+        part_ml[slot * 2] = m;
+        part_ml[slot * 2 + 1] = l;
+    }
+    if (!any && n_splits > 1) return;
+    const float inv = 1.0f / l;
+#pragma unroll
+    for (int i = 0; i < DW; ++i) {
+        const int d = (wave * DW + i) * 16 + 4 * g;   // (dv is a multiple of 8: four numbers are inside or outside together)
+        if (d >= dv) continue;
+        if (n_splits == 1) *(uint2*)(out + grow * dv + d) = make_uint2(pack_bf16x2(o[i][0] * inv, o[i][1] * inv), pack_bf16x2(o[i][2] * inv, o[i][3] * inv));
+        else *(float4*)(part_o + slot * dv + d) = make_float4(o[i][0], o[i][1], o[i][2], o[i][3]);
+    }
+}
+
 // Log-sum-exp merge of the splits of a row: one block per row.  At most 64 splits: lane s of every wave fetches split s's
 // reference and sum, so these loads go out together.  GROUPS groups of threads, one for every eight splits, take every GROUPS th
 // split each, four values a thread, all eight loads in one trip while the weights are formed, and meet in LDS in group order.
@@ -296,6 +414,7 @@ attn_latent_reduce_kernel(const float* __restrict__ part_o, const float* __restr
             int s = group + i * GROUPS;
             if (s >= n_splits) continue;
             float ws = wgt[s];
+            if (ws == 0.f) continue;                  // (a split without a key has left nothing)
             acc.x = fmaf(v[i].x, ws, acc.x); acc.y = fmaf(v[i].y, ws, acc.y);
             acc.z = fmaf(v[i].z, ws, acc.z); acc.w = fmaf(v[i].w, ws, acc.w);
         }

@@ -3,6 +3,7 @@
 // Norm statistics, angles and the SiLU are computed in 32-bit (angles in 64-bit) whatever
 // the storage type is.
 #include "common.h"
+#include "rotate.h"
 #include "gated_activation.h"
 
 ROCML_LAST_ERROR_FN(elementwise)
@@ -988,19 +989,6 @@ __device__ __forceinline__ float block_sum_256(float v, float* scratch) {
     return r;
 }
 
-// Number e of a part whose first `dims` numbers turn: pairs (e, e + dims/2), or with pairing 1 (2i, 2i + 1), by the
-// angle whose cosine and sine stand in c and s.
-__device__ __forceinline__ float turned(const float* __restrict__ v, int e, int dims, int pairing, const float* __restrict__ c,
-                                        const float* __restrict__ s) {
-    if (e >= dims) return v[e];
-    if (pairing == 1) {
-        int i = e >> 1;
-        return (e & 1) ? v[e] * c[i] + v[e - 1] * s[i] : v[e] * c[i] - v[e + 1] * s[i];
-    }
-    int half = dims / 2;
-    return e < half ? v[e] * c[e] - v[e + half] * s[e] : v[e] * c[e - half] + v[e - half] * s[e - half];
-}
-
 template <typename TO>
 __global__ void __launch_bounds__(EW_BLOCK)
 latent_prepare_kernel(const float* __restrict__ proj, int ld, int q_rank, int kv_rank, int rot_part, int dims,
@@ -1033,6 +1021,61 @@ latent_prepare_kernel(const float* __restrict__ proj, int ld, int q_rank, int kv
         Elem<TO>::store(dst + kv_rank + e, turned(kr, e, dims, pairing, cos_t + (size_t)t * half, sin_t + (size_t)t * half));
 }
 
+// The same for ranks of up to 1,024 that are multiples of 4: everything a token needs (its row, the gains, its page) is asked for
+// at once, the latents stay in registers and both sums cross the block together: one trip to memory and one barrier.  With a
+// pass for the sums and one for the results, a barrier pair each and the page's number behind them, a decode step's took 6.7 to 7.7 us
+// and 8,192 rows 30.
+template <typename TO>
+__global__ void __launch_bounds__(EW_BLOCK)
+latent_prepare_vec_kernel(const float* __restrict__ proj, int ld, int q_rank, int kv_rank, int rot_part, int dims,
+                          const float* __restrict__ q_gain, const float* __restrict__ kv_gain, float eps,
+                          const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+                          TO* __restrict__ cq_out, TO* __restrict__ cache, const int* __restrict__ block_table,
+                          int bt_width, const int* __restrict__ token_seq, const int* __restrict__ token_pos,
+                          int page_size, int write_cache, int pairing) {
+    __shared__ float red[2][EW_BLOCK / WAVE];
+    const int t = blockIdx.x, tid = threadIdx.x, e = tid * 4, half = dims / 2;
+    const float* row = proj + (size_t)t * ld;
+    const bool has_q = e < q_rank, has_k = write_cache && e < kv_rank;
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 q = has_q ? row4(row + e) : zero, qg = has_q ? row4(q_gain + e) : zero;
+    float4 k = has_k ? row4(row + q_rank + e) : zero, kg = has_k ? row4(kv_gain + e) : zero;
+    int page = -1, pos = 0;
+    float r[4];                                          // rotated numbers of this thread: EW_BLOCK apart
+    if (write_cache) {
+        pos = token_pos[t];
+        page = block_table[(size_t)token_seq[t] * bt_width + pos / page_size];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            int at = tid + i * EW_BLOCK;
+            r[i] = at < rot_part ? turned(row + q_rank + kv_rank, at, dims, pairing, cos_t + (size_t)t * half, sin_t + (size_t)t * half) : 0.f;
+        }
+    }
+    float sq = fmaf(q.x, q.x, fmaf(q.y, q.y, fmaf(q.z, q.z, q.w * q.w))), sk = fmaf(k.x, k.x, fmaf(k.y, k.y, fmaf(k.z, k.z, k.w * k.w)));
+    sq = wave_sum(sq);
+    sk = wave_sum(sk);
+    if (tid % WAVE == 0) {
+        red[0][tid / WAVE] = sq;
+        red[1][tid / WAVE] = sk;
+    }
+    __syncthreads();
+    sq = sk = 0.f;
+#pragma unroll
+    for (int w = 0; w < EW_BLOCK / WAVE; ++w) {
+        sq += red[0][w];
+        sk += red[1][w];
+    }
+    const float inv_q = 1.0f / sqrtf(sq / (float)q_rank + eps);
+    if (has_q) store4(cq_out + (size_t)t * q_rank + e, q.x * inv_q * qg.x, q.y * inv_q * qg.y, q.z * inv_q * qg.z, q.w * inv_q * qg.w);
+    if (page < 0) return;
+    TO* dst = cache + ((size_t)page * page_size + pos % page_size) * (kv_rank + rot_part);
+    const float inv_k = 1.0f / sqrtf(sk / (float)kv_rank + eps);
+    if (has_k) store4(dst + e, k.x * inv_k * kg.x, k.y * inv_k * kg.y, k.z * inv_k * kg.z, k.w * inv_k * kg.w);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (tid + i * EW_BLOCK < rot_part) Elem<TO>::store(dst + kv_rank + tid + i * EW_BLOCK, r[i]);
+}
+
 ROCML_EXPORT int rocml_latent_prepare(const float* proj, int ld, int n_tokens, int q_rank, int kv_rank, int rot_part,
                                       int dims, const float* q_gain, const float* kv_gain, float eps,
                                       const float* cos_t, const float* sin_t, void* cq_out, void* cache,
@@ -1049,12 +1092,19 @@ ROCML_EXPORT int rocml_latent_prepare(const float* proj, int ld, int n_tokens, i
     ROCML_REQUIRE(!write_cache || (cache && block_table && bt_width > 0 && page_size > 0 && token_seq && token_pos),
                   "latent_prepare: cache arguments missing");
     if (n_tokens == 0) return 0;
+    const uintptr_t aligned = (uintptr_t)proj | (uintptr_t)q_gain | (uintptr_t)kv_gain | (uintptr_t)cq_out | (uintptr_t)cache;
+    const bool vec = q_rank <= 4 * EW_BLOCK && kv_rank <= 4 * EW_BLOCK && rot_part <= 4 * EW_BLOCK &&
+                     ((q_rank | kv_rank | rot_part | ld) & 3) == 0 && (aligned & 15) == 0;
 #define LAUNCH(TO)                                                                                              \
-    latent_prepare_kernel<TO><<<n_tokens, EW_BLOCK, 0, stream>>>(proj, ld, q_rank, kv_rank, rot_part, dims,    \
+    if (vec)                                                                                                    \
+    latent_prepare_vec_kernel<TO><<<n_tokens, EW_BLOCK, 0, stream>>>(proj, ld, q_rank, kv_rank, rot_part, dims, \
+        q_gain, kv_gain, eps, cos_t, sin_t, (TO*)cq_out, (TO*)cache, block_table, bt_width, token_seq,         \
+        token_pos, page_size, write_cache, pairing);                                                            \
+    else latent_prepare_kernel<TO><<<n_tokens, EW_BLOCK, 0, stream>>>(proj, ld, q_rank, kv_rank, rot_part, dims,    \
         q_gain, kv_gain, eps, cos_t, sin_t, (TO*)cq_out, (TO*)cache, block_table, bt_width, token_seq,         \
         token_pos, page_size, write_cache, pairing)
-    if (out_dtype == ROCML_F32) LAUNCH(float);
-    else if (out_dtype == ROCML_BF16) LAUNCH(bf16_t);
+    if (out_dtype == ROCML_F32) { LAUNCH(float); }
+    else if (out_dtype == ROCML_BF16) { LAUNCH(bf16_t); }
     else return rocml_fail("latent_prepare: unknown dtype code %d", out_dtype);
 #undef LAUNCH
     ROCML_CHECK_LAUNCH("latent_prepare");

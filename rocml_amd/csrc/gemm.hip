@@ -835,3 +835,23 @@ ROCML_EXPORT int rocml_gemm_batched(const void* x, int x_dtype, int ldx, long lo
     ROCML_CHECK_LAUNCH("gemm_batched");
     return 0;
 }
+
+// The queries of a latent attention for at most 16 rows (latent_queries_kernel): out_h[M, 0 .. N) = q_h[M, 0 .. K) * w_h[N, K]^T and
+// out_h[M, N .. N + rot_part) = the rotated numbers q_h[M, offset ..) of which the first dims turn.  q is 32-bit, w and out bfloat16.
+ROCML_EXPORT int rocml_latent_queries(const float* q, int ldq, int q_stride, const void* w, void* out, int ldo, int o_stride, int heads,
+                                      int m, int n, int k, int offset, int rot_part, int dims, const float* cos_t, const float* sin_t,
+                                      int pairing, hipStream_t stream) {
+    ROCML_REQUIRE(heads > 0 && heads < 65536 && m >= 0 && m <= 16 && n > 0 && k > 0 && rot_part >= 0 && dims >= 0 && dims % 2 == 0 && dims <= rot_part,
+                  "latent_queries: bad sizes heads=%d M=%d N=%d K=%d part=%d dims=%d", heads, m, n, k, rot_part, dims);
+    ROCML_REQUIRE(offset >= 0 && k <= q_stride && offset + rot_part <= q_stride && n + rot_part <= o_stride && ldq >= heads * q_stride && ldo >= heads * o_stride,
+                  "latent_queries: a head does not hold its parts");
+    ROCML_REQUIRE(k % 8 == 0 && ldq % 4 == 0 && q_stride % 4 == 0 && (uintptr_t)q % 16 == 0 && (uintptr_t)w % 16 == 0,
+                  "latent_queries: rows and weights in 16-byte pieces are needed (K=%d ldq=%d)", k, ldq);
+    ROCML_REQUIRE(pairing == 0 || pairing == 1, "latent_queries: pairing %d (0: halves, 1: neighbours)", pairing);
+    ROCML_REQUIRE(q && w && out && (dims == 0 || (cos_t && sin_t)), "latent_queries: a pointer is missing");
+    if (m == 0) return 0;
+    latent_queries_kernel<<<dim3(ceil_div(n, 32) + 1, 1, heads), 256, 0, stream>>>(q, ldq, q_stride, (const bf16_t*)w, (bf16_t*)out, ldo, o_stride, m, n, k,
+                                                                                   offset, rot_part, dims, cos_t, sin_t, pairing);
+    ROCML_CHECK_LAUNCH("latent_queries");
+    return 0;
+}

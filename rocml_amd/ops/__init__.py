@@ -80,6 +80,7 @@ _SIGNATURES = {
         "rocml_gemm": [_P, _I, _I, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _LL, _P, _I, _F, _I, _P],
         "rocml_splitk_reduce": [_P, _P, _I, _I, _I, _I, _I, _I, _P],
         "rocml_gemm_batched": [_P, _I, _I, _LL, _P, _I, _I, _LL, _P, _I, _I, _LL, _I, _I, _I, _I, _P, _I, _LL, _I, _P],
+        "rocml_latent_queries": [_P, _I, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P],
         "rocml_gemm_residual_prescale_pays": [_I, _I, _I],
         "rocml_gemm_residual_prescale": [_P, _I, _P, _I, _P, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P, _P],
     },
@@ -851,6 +852,35 @@ def gemm_batched(x: torch.Tensor, x_head_stride: int, w: torch.Tensor, out: torc
     _check("gemm", library("gemm").rocml_gemm_batched(
         _ptr(x), _code(x), x.shape[1], x_head_stride, _ptr(w), _code(w), k, n * k, _ptr(out), _code(out),
         out.shape[1], out_head_stride, heads, x.shape[0], n, k, _ptr(gate), ldg, g_stride, 1 if gate_one else 0, _stream()))
+
+
+LATENT_QUERIES_MAX_ROWS = 16
+
+
+def latent_queries_fit(q: torch.Tensor, w: torch.Tensor, head_stride: int) -> bool:
+    """Whether ``latent_queries`` takes these operands."""
+    return (q.shape[0] <= LATENT_QUERIES_MAX_ROWS and w.dtype == torch.bfloat16 and w.shape[2] % 8 == 0 and head_stride % 4 == 0
+            and q.shape[1] % 4 == 0)
+
+
+def latent_queries(q: torch.Tensor, head_stride: int, w: torch.Tensor, out: torch.Tensor, out_stride: int, offset: int, rot_part: int,
+                   rot_dims: int, cos: Optional[torch.Tensor], sin: Optional[torch.Tensor], pairing: str = "halves") -> None:
+    """``gemm_batched(q, head_stride, w, out, out_stride)`` and ``rope_heads(q, heads, head_stride, offset, rot_part, rot_dims, cos, sin,
+    out, out_stride, N)`` in one launch, for at most 16 rows of 32-bit queries and bfloat16 weights ``[heads, N, K]``."""
+    if pairing not in ROPE_PAIRINGS:
+        raise KernelError(f"unknown rotation pairing {pairing!r}; known: {sorted(ROPE_PAIRINGS)}")
+    _dev(q, w, out, cos, sin)
+    _want(q, torch.float32, "queries")
+    _want(out, torch.bfloat16, "the attention's queries")
+    heads, n, k = w.shape
+    if q.dim() != 2 or out.dim() != 2 or q.shape[0] != out.shape[0] or not latent_queries_fit(q, w, head_stride):
+        raise KernelError("latent_queries takes at most 16 rows of 32-bit queries and bfloat16 weights [heads, N, K]")
+    if rot_dims and (cos is None or sin is None or cos.shape != (q.shape[0], rot_dims // 2) or sin.shape != cos.shape
+                     or cos.dtype != torch.float32 or sin.dtype != torch.float32):
+        raise KernelError(f"rotation tables must be float32 {(q.shape[0], rot_dims // 2)}")
+    _check("gemm", library("gemm").rocml_latent_queries(
+        _ptr(q), q.shape[1], head_stride, _ptr(w), _ptr(out), out.shape[1], out_stride, heads, q.shape[0], n, k, offset, rot_part, rot_dims,
+        _ptr(cos), _ptr(sin), ROPE_PAIRINGS[pairing], _stream()))
 
 
 PRESCALE_MAX_ROWS = 16      # most rows gemm_residual_prescale takes

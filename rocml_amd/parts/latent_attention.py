@@ -191,9 +191,12 @@ class LatentAttention(Mixer):
         if expanded:
             self._expanded_prompt(step, q, first, cos, sin, dims, cache, x_accum)
             return
-        ops.gemm_batched(q, self.qk_dim, self.w_uk_t, qa, self.row)
-        ops.rope_heads(q, s.n_heads, self.qk_dim, s.head_dim, s.rot_dim, dims, cos, sin, qa, self.row, s.kv_rank,
-                       pairing=self.pairing)
+        if self.dtype == torch.bfloat16 and ops.latent_queries_fit(q, self.w_uk_t, self.qk_dim):
+            ops.latent_queries(q, self.qk_dim, self.w_uk_t, qa, self.row, s.head_dim, s.rot_dim, dims, cos, sin, pairing=self.pairing)
+        else:
+            ops.gemm_batched(q, self.qk_dim, self.w_uk_t, qa, self.row)
+            ops.rope_heads(q, s.n_heads, self.qk_dim, s.head_dim, s.rot_dim, dims, cos, sin, qa, self.row, s.kv_rank,
+                           pairing=self.pairing)
         ol = ws.get("latent.ol", (n, s.n_heads * s.kv_rank), self.dtype)
         ops.attention(qa, ol, cache.k.unsqueeze(1), None, cache.block_table, step.token_seq, step.token_pos,
                       s.n_heads, 1, self.row, s.scale, s.window, workspace=ws.scratch(),

@@ -153,6 +153,8 @@ _COSTS: Dict[str, Tuple[str, Callable]] = {
     "gemm_batched": ("per-head products", _gemm_batched_cost),
     "latent_prepare": ("latent norms, rotation, append", lambda proj, *a, **kw: (
         proj.shape[0] * sum(a[:3]) * 6, proj.shape[0] * sum(a[:3]) * 4)),
+    "latent_queries": ("latent queries: per-head products and rotation", lambda q, head_stride, w, out, out_stride, *a, **kw: (
+        _nbytes(q, w, out), 2 * q.shape[0] * w.numel())),
     "rope_heads": ("rotation of the queries' part", lambda q, n_heads, head_stride, offset, rot_part, *a, **kw: (
         q.shape[0] * n_heads * rot_part * 6, q.shape[0] * n_heads * rot_part * 3)),
     "latent_window_plan": ("expanded prompt: plan of the visible rows", _tensor_args_cost(skip=(2,))),
