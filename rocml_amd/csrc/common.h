@@ -104,4 +104,46 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// Exchanges that stay in the vector registers (a shuffle is a trip through LDS, some 50 ns one after the other).  All 64 lanes are
+// active.  lane_xor1, lane_xor2: the neighbour's value one and two lanes across.
+template <int CTRL> __device__ __forceinline__ float lane_dpp(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float lane_xor1(float v) { return lane_dpp<0xB1>(v); }
+__device__ __forceinline__ float lane_xor2(float v) { return lane_dpp<0x4E>(v); }
+
+// sum over the 16 lanes of a row, the same in every lane: lanes 1 apart, 2 apart, mirrored inside a
+// half row, mirrored inside the row
+__device__ __forceinline__ float row16_sum(float v) {
+    v += lane_xor1(v);
+    v += lane_xor2(v);
+    v += lane_dpp<0x141>(v);
+    v += lane_dpp<0x140>(v);
+    return v;
+}
+
+// The two values of lanes 16 (32) apart, in both: swapping the odd rows (the upper half) of one copy with the even rows (the lower half) of the other.
+struct LanePair { float a, b; };
+__device__ __forceinline__ LanePair lane_pair16(float v) {
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+__device__ __forceinline__ LanePair lane_pair32(float v) {
+    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return {__uint_as_float(r[0]), __uint_as_float(r[1])};
+}
+
+// sum and maximum over the four rows' lanes of the same place, and over all lanes
+__device__ __forceinline__ float rows4_sum(float v) {
+    LanePair p = lane_pair16(v);
+    p = lane_pair32(p.a + p.b);
+    return p.a + p.b;
+}
+__device__ __forceinline__ float rows4_max(float v) {
+    LanePair p = lane_pair16(v);
+    p = lane_pair32(fmaxf(p.a, p.b));
+    return fmaxf(p.a, p.b);
+}
+__device__ __forceinline__ float lanes_sum(float v) { return rows4_sum(row16_sum(v)); }
+
 static inline int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }

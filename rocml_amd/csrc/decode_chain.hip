@@ -94,8 +94,7 @@ template <> struct DcType<float> {
     static __device__ __forceinline__ void finish(f32x4_t& acc) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            acc[e] += __shfl_xor(acc[e], 16, 64);
-            acc[e] += __shfl_xor(acc[e], 32, 64);
+            acc[e] = rows4_sum(acc[e]);
         }
     }
     static __device__ __forceinline__ int w_row(int lane) { return (lane >> 2) * 4; }
@@ -202,7 +201,7 @@ __device__ __forceinline__ float dc_row_scale(const DcArgs& a, const u64* ssq, i
         dc_collect<1>(a, epoch, mine, mine ? at * (8u * DC_APART) : 0u, [&](int, uint32_t o) { return dc_at(ssq, o); }, v);
         ss += mine ? __uint_as_float(v[0]) : 0.f;
     }
-    return 1.0f / sqrtf(wave_sum(ss) * a.inv_width + eps);
+    return 1.0f / sqrtf(lanes_sum(ss) * a.inv_width + eps);
 }
 
 // A block's place in the order: {launch, ticket} of its counter, handed on as {launch, item}; the items shard, shard + DC_SHARDS,
@@ -233,6 +232,7 @@ struct DcLds {
     uint32_t end;                               // see DcTickets
     // the waves' sums (two of them in turn: the other waves go on to the next item while the first finishes this one)
     alignas(16) float red[2][DC_MAX_TILES][W][DC_MAX_ROWS][DC_TILE];
+    float scale[2][DC_MAX_ROWS];                // the rows' norm scales (in turn, as red)
     alignas(16) float m[W][16], l[W][16];
     alignas(16) float o[W][DC_MAX_GROUP][DC_D + 4];
     alignas(16) float q[DC_MAX_GROUP][DC_D], k[DC_D], v[DC_D];      // (of the compute type)
@@ -403,56 +403,54 @@ __device__ __forceinline__ void dc_product(const DcArgs& a, const DcLayer& ly, c
         }
         hand_over(0);
     }
-    float scale = 1.0f;
     if (stage == DC_GU && wave == 0) {
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            float mine_ = dc_row_scale(a, st + p.ssqa + m * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch, a.eps_ffn, lane, 128, ss[m]);
-            scale = orow == m ? mine_ : scale;
+            const float scale = dc_row_scale(a, st + p.ssqa + m * (p.hidden / DC_TILE) * DC_APART, p.hidden / DC_TILE, epoch, a.eps_ffn, lane, 128, ss[m]);
+            if (lane == 0) sm.scale[turn][m] = scale;
         }
     }
     __syncthreads();
-    if (wave != 0) return;
-    for (int tile = 0; tile < tiles; ++tile) {
-        float v = 0.f;
+    // A row of lanes finishes a tile of one row of activations: four of them a wave (one after the other in the first wave, the three
+    // tiles of a gated item took a microsecond more).
+    const int part = wave * 4 + g;
+    if (wave * 4 >= tiles * M) return;
+    const int row = part % M, tile = part / M;
+    const bool in = tile < tiles;
+    float v = 0.f;
+    if (in) {
         const auto& red = sm.red[turn][tile];
-        if (orow < M) {
-            v = red[0][orow][col];
+        v = red[0][row][col];
 #pragma unroll
-            for (int i = 1; i < W; ++i) v += red[i][orow][col];
-        }
-        if (stage == DC_QKV) {
-            if (orow < M) dc_store(st + p.y + (size_t)orow * p.n_qkv + ocol + tile * DC_TILE, __float_as_uint(v), epoch);
-        } else if (stage == DC_GU) {
-            // gate and up rows in turn: even lanes have a gate, their neighbour its up value
-            v *= scale;
-            float up = __shfl_xor(v, 1, 64);
-            float hv = v / (1.0f + expf(-v)) * up;
-            u64* to = st + p.h + (size_t)orow * (p.inter / V) + (tile0 + tile) * (8 / V);
-            if constexpr (V == 2) {
-                float hn = __shfl_xor(hv, 2, 64);
-                if (orow < M && (col & 3) == 0) dc_store(to + col / 4, f32x2_to_bf16x2(hv, hn), epoch);
-            } else {
-                if (orow < M && (col & 1) == 0) dc_store(to + col / 2, __float_as_uint(hv), epoch);
-            }
+        for (int i = 1; i < W; ++i) v += red[i][row][col];
+    }
+    if (stage == DC_QKV) {
+        if (in) dc_store(st + p.y + (size_t)row * p.n_qkv + (tile0 + tile) * DC_TILE + col, __float_as_uint(v), epoch);
+    } else if (stage == DC_GU) {
+        // gate and up rows in turn: even lanes have a gate, their neighbour its up value
+        v *= sm.scale[turn][row];
+        const float up = lane_xor1(v), hv = v / (1.0f + expf(-v)) * up;
+        u64* to = st + p.h + (size_t)row * (p.inter / V) + (tile0 + tile) * (8 / V);
+        if constexpr (V == 2) {
+            const float hn = lane_xor2(hv);
+            if (in && (col & 3) == 0) dc_store(to + col / 4, f32x2_to_bf16x2(hv, hn), epoch);
         } else {
-            float r = x_old + v;
-            if (stage == DC_DOWN && layer == p.n_layers - 1) {
-                if (orow < M) a.x[(size_t)orow * p.hidden + ocol] = r;
-                return;
-            }
-            float xg = r * gv, xn = __shfl_xor(xg, 1, 64);
-            float sq = r * r;
-#pragma unroll
-            for (int off = 1; off < 16; off <<= 1) sq += __shfl_xor(sq, off, 64);
-            if (orow < M) {
-                const bool o = stage == DC_O;
-                u64* to = st + (o ? p.xga : p.xgb) + (size_t)orow * (p.hidden / V) + ocol / V;
-                if (V == 1) dc_store(to, __float_as_uint(xg), epoch);
-                else if ((col & 1) == 0) dc_store(to, f32x2_to_bf16x2(xg, xn), epoch);
-                if (col == 0) dc_store(st + (o ? p.ssqa : p.ssqb) + (orow * (p.hidden / DC_TILE) + tile0) * DC_APART, __float_as_uint(sq), epoch);
-                dc_store(st + (o ? p.xa : p.xb) + (size_t)orow * p.hidden + ocol, __float_as_uint(r), epoch);
-            }
+            if (in && (col & 1) == 0) dc_store(to + col / 2, __float_as_uint(hv), epoch);
+        }
+    } else {                                    // (one tile: the row is the one whose old value the lane holds)
+        const float r = x_old + v;
+        if (stage == DC_DOWN && layer == p.n_layers - 1) {
+            if (in) a.x[(size_t)row * p.hidden + ocol] = r;
+            return;
+        }
+        const float xg = r * gv, xn = lane_xor1(xg), sq = row16_sum(r * r);
+        if (in) {
+            const bool o = stage == DC_O;
+            u64* to = st + (o ? p.xga : p.xgb) + (size_t)row * (p.hidden / V) + ocol / V;
+            if (V == 1) dc_store(to, __float_as_uint(xg), epoch);
+            else if ((col & 1) == 0) dc_store(to, f32x2_to_bf16x2(xg, xn), epoch);
+            if (col == 0) dc_store(st + (o ? p.ssqa : p.ssqb) + (row * (p.hidden / DC_TILE) + tile0) * DC_APART, __float_as_uint(sq), epoch);
+            dc_store(st + (o ? p.xa : p.xb) + (size_t)row * p.hidden + ocol, __float_as_uint(r), epoch);
         }
     }
 }
@@ -519,8 +517,7 @@ template <int W> struct DcPieces<bf16_t, W> {
             for (int u = 0; u < 2; ++u)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[u][i]);
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            mx = rows4_max(mx);
             float m_new = fmaxf(m, mx);
             float m_use = m_new == -INFINITY ? 0.f : m_new;
             float corr = fast_exp2(m - m_use), sum = 0.f;
@@ -531,8 +528,7 @@ template <int W> struct DcPieces<bf16_t, W> {
                     s[u][i] = fast_exp2(s[u][i] - m_use);
                     sum += s[u][i];
                 }
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
+            sum = rows4_sum(sum);
             l = l * corr + sum;
             m = m_new;
             uint4 pv = make_uint4(pack_bf16x2(s[0][0], s[0][1]), pack_bf16x2(s[0][2], s[0][3]),
@@ -641,8 +637,7 @@ template <int W> struct DcPieces<float, W> {
             }
             multiply(new_pos, new_pos + 1);
         }
-        l += __shfl_xor(l, 16, 64);
-        l += __shfl_xor(l, 32, 64);
+        l = rows4_sum(l);
         const int row = lane & 15;
         if (lane < 16) {
             sm.m[wave][lane] = m;
@@ -714,7 +709,7 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
             if (r >= n_rows) break;
             float v0 = __uint_as_float(raw[2 * i]) * row_scale, v1 = __uint_as_float(raw[2 * i + 1]) * row_scale;
             if (r <= group) {
-                float inv = 1.0f / sqrtf(wave_sum(fmaf(v1, v1, v0 * v0)) / (float)D + a.qk_eps);
+                float inv = 1.0f / sqrtf(lanes_sum(fmaf(v1, v1, v0 * v0)) / (float)D + a.qk_eps);
                 v0 = v0 * inv * (r < group ? gq0 : gk0);
                 v1 = v1 * inv * (r < group ? gq1 : gk1);
                 // pairs (e, e + 64) are one lane's
@@ -860,6 +855,12 @@ __global__ void __launch_bounds__(64 * W) decode_chain_kernel(const DcArgs a) {
                 it.i -= p.items[s];
                 it.stage = s + 1;
             }
+        // (told to be the same in all lanes: the divisions leave them in vector registers, and a choice between two operands by the
+        // stage was then a load of the kernel's arguments by the lanes and a wait for everything on its way, the last store included: 1 to
+        // 2 us in every output and down item)
+        it.layer = __builtin_amdgcn_readfirstlane(it.layer);
+        it.i = __builtin_amdgcn_readfirstlane(it.i);
+        it.stage = __builtin_amdgcn_readfirstlane(it.stage);
         // (numbers start at 2: the state starts as zeros, and a layer reads what the one before it numbered)
         it.epoch = launch * (uint32_t)DC_LAYERS + (uint32_t)it.layer + 2u;
         const DcLayer& ly = a.layer[it.layer];

@@ -201,16 +201,6 @@ ROCML_EXPORT int rocml_causal_conv(const float* u, int ldu, int col0, int n_toke
 typedef float sc_f4 __attribute__((ext_vector_type(4)));      // 16 bytes as a native vector
 constexpr int SC_R = 16, SC_PP = 2, SC_PT = RC_BLOCK / SC_R * SC_PP, SC_MAX_TC = 32, SC_U = 4;
 
-// sum over the 16 lanes of a row, the same in every lane: lanes 1 apart, 2 apart, mirrored inside a
-// half row, mirrored inside the row
-__device__ __forceinline__ float row16_sum(float v) {
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xF, 0xF, false));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xF, 0xF, false));
-    return v;
-}
-
 // A thread's NI state entries of one column, n = r * NI ..: as 16-byte pieces where NI is a multiple of 4 and
 // the state is exactly 16 NI long (one load instruction of a wave then touches 16 memory lines, not 64).
 template <int NI>
