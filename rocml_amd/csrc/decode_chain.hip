@@ -8,9 +8,9 @@
 // order in which they depend on each other: it asks for its weights (or its pages) first, then waits for its operands, so that
 // the next stages' weights are in registers while this stage's results travel.  From a block's store to the waiting blocks that
 // read it some 1.5 us pass.  A step of the Qwen3-0.6B shape (28 layers, replayed, to the logits): one sequence of 40 tokens
-// 967 -> 530 us, of 500 978 -> 587, of 5,000 1,071 -> 894; two of 2,000 1,049 -> 747; four of 300 1,026 -> 773 (with how many keys it is
-// slower: rocml_decode_chain_reach).  What is left of a layer (15.3 us) is five times a result's way to the next stage, each with a
-// trip to memory behind its store.
+// 1,002 -> 474 us, of 500 1,011 -> 527, of 5,000 1,094 -> 703; two of 2,000 1,084 -> 761; four of 300 1,060 -> 697 (with how many keys it is
+// slower: rocml_decode_chain_reach).  What is left of a layer (some 13 us) is five times a result's way to the next stage (1 to 1.5 us from its
+// store to the operands behind it), 0.6 to 1 us of products and 0.3 to 0.6 of an epilogue.
 //
 // Measured on the way: two and three blocks a CU instead of one, 657 and 678 us against 558 (more weights ahead, but what asks
 // for operands is in the way of what answers); eight waves a block 648 against 548 (but see dc_plan); a wave of its own for
@@ -482,7 +482,7 @@ template <int W> struct DcPieces<bf16_t, W> {
     __device__ __forceinline__ void request_first() {
         if (wave < my_pages * 2) request(wave);
     }
-    __device__ __forceinline__ void run(DcLds<W>& sm, int cached, bool owner, int new_pos) {
+    __device__ __forceinline__ void run(DcLds<W>& sm, bool owner, int new_pos) {
         const int g = lane >> 4, col = lane & 15, n_pieces = my_pages * 2;
         const float scale_log2e = a.scale * AM_LOG2E;
         const bf16_t *sq = (const bf16_t*)sm.q, *sk = (const bf16_t*)sm.k, *sv = (const bf16_t*)sm.v;
@@ -540,28 +540,35 @@ template <int W> struct DcPieces<bf16_t, W> {
                 o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, vbuf[dt]), pf, o[dt], 0, 0, 0);
             }
         };
-        // (the step's own key is not yet in the cache where a block reads it; it comes last, from LDS)
+        // (the step's own key is not yet in the cache where a block reads it: it takes its place in its piece from LDS)
         for (int piece = wave; piece < n_pieces; piece += W) {
             f32x4_t s[2];
             if (piece != wave) request(piece);
-            scores((split + (piece >> 1) * a.p.splits) * AM_PAGE + (piece & 1) * 32, cached, s);
-            add_values(s);
-        }
-        asm volatile("" ::: "memory");
-        if (owner && wave == n_pieces % W) {
-            bool krow = col == 0, vrow = g == 0;
+            const int key0 = (split + (piece >> 1) * a.p.splits) * AM_PAGE + (piece & 1) * 32, at = new_pos - key0;
+            if (owner && at >= 0 && at < 32) {
+                const bool krow = col == (at >> 3) * 4 + (at & 3);
+                uint32_t half[4];                     // the value's half of a word of the lane's eight, if any
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
+                for (int i = 0; i < 4; ++i) half[i] = g == at >> 3 && at % 8 / 2 == i ? (at & 1 ? 0xffff0000u : 0xffffu) : 0u;
 #pragma unroll
                 for (int kd = 0; kd < KD; ++kd) {
-                    uint4 v = *(const uint4*)(sk + kd * 32 + g * 8);
-                    bool take = krow && u == 0;
-                    kbuf[u][kd] = make_uint4(take ? v.x : 0u, take ? v.y : 0u, take ? v.z : 0u, take ? v.w : 0u);
+                    const uint4 v = *(const uint4*)(sk + kd * 32 + g * 8);
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const bool take = krow && (at >> 2 & 1) == u;
+                        uint4& k = kbuf[u][kd];
+                        k = make_uint4(take ? v.x : k.x, take ? v.y : k.y, take ? v.z : k.z, take ? v.w : k.w);
+                    }
                 }
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) vbuf[dt] = make_uint4(vrow ? (uint32_t)sv[dt * 16 + col] : 0u, 0u, 0u, 0u);
-            f32x4_t s[2];
-            scores(new_pos, new_pos + 1, s);
+                for (int dt = 0; dt < DT; ++dt) {
+                    const uint32_t v = sv[dt * 16 + col] * 0x10001u;
+                    const uint4 old = vbuf[dt];
+                    vbuf[dt] = make_uint4((old.x & ~half[0]) | (v & half[0]), (old.y & ~half[1]) | (v & half[1]),
+                                          (old.z & ~half[2]) | (v & half[2]), (old.w & ~half[3]) | (v & half[3]));
+                }
+            }
+            scores(key0, new_pos + 1, s);
             add_values(s);
         }
         // the waves' results in wave order; element i of o[dt] is d = 16 dt + 4g + i, column = head
@@ -578,9 +585,11 @@ template <int W> struct DcPieces<bf16_t, W> {
     }
 };
 
-// 32-bit: a piece is 16 keys, the helpers are attn_f32_token_kernel's.
+// 32-bit: a piece is 16 keys, multiplied as the projections are (4x4x1 in sixteen blocks, four heads at a time): a block is four keys and four heads
+// at one place of the head size, or four values and four heads at one key, and the four rows of lanes add up.  16x16x4 with the two heads of a
+// group in use takes four times the clocks: 2 us a piece.
 template <int W> struct DcPieces<float, W> {
-    static constexpr int D = DC_D, KD = D / 16;
+    static constexpr int D = DC_D, KD = D / 16, HEADS = (DC_MAX_GROUP + 3) / 4;
     const DcArgs& a; const DcLayer& ly; const int* pages;
     int kvh, split, my_pages, group, wave, lane;
     af_f32x4_t k[KD], v[KD];
@@ -598,54 +607,99 @@ template <int W> struct DcPieces<float, W> {
     __device__ __forceinline__ void request_first() {
         if (wave < my_pages * 4) request(wave);
     }
-    __device__ __forceinline__ void run(DcLds<W>& sm, int cached, bool owner, int new_pos) {
-        AttnF32Args mask{};
-        mask.scale = a.scale;
-        const int n_pieces = my_pages * 4;
-        const float* q = sm.q[min(lane & 15, group - 1)] + (lane >> 4) * 4;
-        af_f32x4_t o[KD], s[1];
+    __device__ __forceinline__ void run(DcLds<W>& sm, bool owner, int new_pos) {
+        const int n_pieces = my_pages * 4, g = lane >> 4, quad = lane >> 2 & 3;
+        af_f32x4_t o[HEADS][KD];
+        float m[HEADS], l[HEADS];
 #pragma unroll
-        for (int c = 0; c < KD; ++c) o[c] = af_f32x4_t{0.f, 0.f, 0.f, 0.f};
-        float m = -INFINITY, l = 0.f;
-        // keys first .. first + 15, of which those before `to` are seen
-        auto multiply = [&](int first, int to) {
-            af_scores<KD, 1>([&](int c) { return *(const af_f32x4_t*)(q + c * 16); }, [&](int, int c) { return k[c]; }, s);
-            af_softmax<KD, 1>(s, o, m, l, mask, first, lane, to - 1, 0, 0.f);
-            bool seen[4];
+        for (int h = 0; h < HEADS; ++h) {
+            m[h] = -INFINITY;
+            l[h] = 0.f;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) seen[e] = first + (lane >> 4) * 4 + e < to;
-            af_values<KD, 1>(s, [&](int c, int) {
-                af_f32x4_t u = v[c];                  // a key that is not seen may hold anything: it is left out, not weighted by zero
-#pragma unroll
-                for (int e = 0; e < 4; ++e) u[e] = seen[e] ? u[e] : 0.f;
-                return u;
-            }, o);
-        };
-        for (int piece = wave; piece < n_pieces; piece += W) {
-            const int first = (split + (piece >> 2) * a.p.splits) * AF_PAGE + (piece & 3) * 16;
-            if (first >= cached) continue;
-            if (piece != wave) request(piece);
-            multiply(first, cached);
+            for (int c = 0; c < KD; ++c) o[h][c] = af_f32x4_t{0.f, 0.f, 0.f, 0.f};
         }
-        asm volatile("" ::: "memory");
-        // (the step's own key is not yet in the cache where a block reads it; it comes last, from LDS)
-        if (owner && wave == n_pieces % W) {
+        for (int piece = wave; piece < n_pieces; piece += W) {
+            const int first = (split + (piece >> 2) * a.p.splits) * AF_PAGE + (piece & 3) * 16, at = new_pos - first;
+            if (at < 0) continue;
+            if (piece != wave) request(piece);
+            // (the step's own key is not yet in the cache where a block reads it: it takes its place in its piece from LDS; a key that is
+            // not seen may hold anything: it is left out, not weighted by zero)
+            const bool own = owner && at < 16;
+            if (own) {
+#pragma unroll
+                for (int c = 0; c < KD; ++c) {
+                    const af_f32x4_t nk = *(const af_f32x4_t*)(sm.k + c * 16 + g * 4);
+                    const float nv = sm.v[c * 16 + (lane & 15)];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        k[c][e] = (lane & 15) == at ? nk[e] : k[c][e];
+                        v[c][e] = g * 4 + e == at ? nv : v[c][e];
+                    }
+                }
+            }
+            if (at < 15) {
+#pragma unroll
+                for (int c = 0; c < KD; ++c)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[c][e] = g * 4 + e <= at ? v[c][e] : 0.f;
+            }
+#pragma unroll
+            for (int h = 0; h < HEADS; ++h) {
+                if (h * 4 >= group) break;
+                const float* q = sm.q[min(h * 4 + (lane & 3), group - 1)] + g * 4;
+                f32x4_t s = {0.f, 0.f, 0.f, 0.f}, odd = s;
+#pragma unroll
+                for (int c = 0; c < KD; ++c) {
+                    const af_f32x4_t qv = *(const af_f32x4_t*)(q + c * 16);
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) {
+                        s = __builtin_amdgcn_mfma_f32_4x4x1f32(k[c][e], qv[e], s, 0, 0, 0);
+                        odd = __builtin_amdgcn_mfma_f32_4x4x1f32(k[c][e + 1], qv[e + 1], odd, 0, 0, 0);
+                    }
+                }
+                // element e: key 4 quad + e, head l%4, the same in every row of lanes
+                float top = -INFINITY;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    s[e] = quad * 4 + e <= at ? rows4_sum(s[e] + odd[e]) * a.scale : -INFINITY;
+                    top = fmaxf(top, s[e]);
+                }
+                top = fmaxf(top, lane_dpp<0x128>(top));             // (rotated by 8 and by 4 lanes inside the row)
+                top = fmaxf(top, lane_dpp<0x124>(top));
+                const float m_new = fmaxf(m[h], top), ref = m_new == -INFINITY ? 0.f : m_new, corr = expf(m[h] - ref);
+                l[h] *= corr;
+                af_f32x4_t p;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    s[e] = expf(s[e] - ref);
+                    l[h] += s[e];
+                    p[e] = __shfl(s[e], g * 20 + (lane & 3), 64);    // key 4 (l/16) + e: of this row's quad of that number
+                }
+                m[h] = m_new;
+#pragma unroll
+                for (int c = 0; c < KD; ++c) o[h][c] *= corr;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int c = 0; c < KD; ++c) o[h][c] = __builtin_amdgcn_mfma_f32_4x4x1f32(v[c][e], p[e], o[h][c], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < HEADS; ++h) {
+            if (h * 4 >= group) break;
+            const int row = h * 4 + (lane & 3);
+            l[h] += lane_dpp<0x128>(l[h]);
+            l[h] += lane_dpp<0x124>(l[h]);
+            if (lane < 4) {
+                sm.m[wave][row] = m[h];
+                sm.l[wave][row] = l[h];
+            }
 #pragma unroll
             for (int c = 0; c < KD; ++c) {
-                k[c] = *(const af_f32x4_t*)(sm.k + c * 16 + (lane >> 4) * 4);
-                v[c] = af_f32x4_t{sm.v[c * 16 + (lane & 15)], 0.f, 0.f, 0.f};
-            }
-            multiply(new_pos, new_pos + 1);
-        }
-        l = rows4_sum(l);
-        const int row = lane & 15;
-        if (lane < 16) {
-            sm.m[wave][lane] = m;
-            sm.l[wave][lane] = l;
-        }
-        if (row < group) {
 #pragma unroll
-            for (int c = 0; c < KD; ++c) *(af_f32x4_t*)(&sm.o[wave][row][c * 16 + (lane >> 4) * 4]) = o[c];
+                for (int e = 0; e < 4; ++e) o[h][c][e] = rows4_sum(o[h][c][e]);
+                if (g == 0 && row < group) *(af_f32x4_t*)(&sm.o[wave][row][c * 16 + quad * 4]) = o[h][c];
+            }
         }
     }
 };
@@ -739,7 +793,7 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
     }
     if (wave == W - 1 && lane == 0) tickets.drawn(drawn, sm.next + (turn ^ 1));
     __syncthreads();
-    piece.run(sm, owner ? new_pos : len, owner, new_pos);
+    piece.run(sm, owner, new_pos);
     __syncthreads();
     for (int head = wave; head < group; head += W) {
         const int d = lane * 2;
@@ -931,14 +985,15 @@ static bool dc_plan(DcPlan& p, int dtype, int rows, int hidden, int hq, int hkv,
 // long the weights' bytes take beside the stages' latencies, of how many words travel, and of how many keys are seen: the attention
 // kernels have a piece of keys on its way while they multiply another, the chain, whose registers hold weights, has not.  Steps to
 // the logits, replayed, us:
-//   bfloat16, 0.6B (31 MB a layer), one row: 40 keys 967 -> 530, 5,000 1,071 -> 894, 20,000 1,299 -> 1,266, 32,000 1,546 -> 1,502, 40,000
-//     (1,024 pages in the table) 1,646 -> 1,685; two rows: 2,000 1,049 -> 747, 3,900 1,132 -> 960, 4,200 (128 pages) 1,149 -> 1,259; three: 2,000
-//     1,146 -> 929, 2,100 (64 pages) 1,118 -> 1,144; four: 300 1,026 -> 773, 2,000 1,172 -> 1,023, 2,100 1,174 -> 1,330, 16,000 2,201 -> 2,937;
-//   1.7B (100 MB, 8 layers), one row: 500 505 -> 401, 32,000 648 -> 611; two: 2,000 503 -> 464, 3,900 544 -> 502, 4,200 548 -> 571; four:
-//     500 518 -> 497, 2,000 563 -> 532, 2,100 556 -> 594;
-//   4B (202 MB, 6 layers): one row 628 -> 623; 8B (386 MB, 6 layers): 841 -> 878: while weights stream, a word's way takes several us;
-//   32-bit, whose attention kernels walk a sequence's keys in few blocks: 0.6B (63 MB), one row of 500 1,827 -> 876, of 20,000 20,098 -> 2,053,
-//     four of 1,000 2,312 -> 1,447, of 20,000 20,499 -> 6,280; 1.7B (201 MB), one row of 500 944 -> 828, of 32,000 9,358 -> 1,219.
+//   bfloat16, 0.6B (31 MB a layer), one row: 40 keys 1,002 -> 474, 5,000 1,094 -> 703, 20,000 1,350 -> 1,228, 40,000 (626 pages) 1,724 -> 1,781; two rows: 2,000
+//     1,084 -> 761, 8,000 1,323 -> 1,101, 16,000 (251 pages) 1,601 -> 1,531; three: 2,100 1,162 -> 871, 4,000 1,287 -> 1,051; four: 2,100 1,227 -> 967, 4,000
+//     1,362 -> 1,195, 8,000 (126 pages) 1,654 -> 1,674;
+//   1.7B (100 MB, 8 layers), one row: 500 523 -> 391, 32,000 701 -> 684; two: 4,200 562 -> 515, 8,000 604 -> 572; four: 500 551 -> 489, 4,000 628 -> 601;
+//   4B (202 MB, 6 layers): one row 608 -> 597, four 641 -> 711; 8B (386 MB, 6 layers): one 806 -> 802, two 818 -> 845: while weights stream, a word's way takes several us;
+//   32-bit, whose attention kernels walk a sequence's keys in few blocks: 0.6B (63 MB), one row of 5,000 6,039 -> 1,187, four of 300 1,703 -> 1,016,
+//     of 4,000 5,210 -> 1,817; 1.7B (201 MB), one row of 500 962 -> 774, two 976 -> 804 (four do not fit the LDS).
+// The lines for several rows, and one row for large 32-bit layers, were drawn when the chain was slower; tests/test_gpu_decode_chain.py holds
+// them.  By the figures above they could lie at 250 pages for two rows and some 110 for four.
 ROCML_EXPORT int rocml_decode_chain_reach(int dtype, int rows, int hidden, int hq, int hkv, int head_dim, int inter) {
     DcPlan p;
     if (!dc_plan(p, dtype, rows, hidden, hq, hkv, head_dim, inter, 1, 1)) return 0;

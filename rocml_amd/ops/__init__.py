@@ -1255,11 +1255,13 @@ def decode_chain_max_layers() -> int:
     return library("decode_chain").rocml_decode_chain_max_layers()
 
 
-def decode_chain_splits(pages: int) -> int:
-    """Splits of the key range in ``decode_chain`` for a block table of ``pages`` pages: a block asks for two pages before it
-    waits for anything, and a second turn costs less than a merge.  It depends on the step's shape only, so a recorded step can be
+def decode_chain_splits(pages: int, pairs: int = 1) -> int:
+    """Splits of the key range in ``decode_chain`` for a block table of ``pages`` pages and ``pairs`` (token, kv head) pairs: a block asks
+    for two pages before it waits for anything, and a second turn costs less than a merge; with more than some 160 items the last ones start
+    when the first blocks are done with theirs (0.6B, one sequence of 5,000: 40 splits 822 us a step, 27 769, 20 703, 14 732; two of 1,000: 16 splits 674,
+    8 667, 6 663; four of 600 the same within 2 % from 2 to 6).  It depends on the step's shape only, so a recorded step can be
     replayed as the sequences grow."""
-    return 1 if pages <= 4 else min(64, (pages + 1) // 2)
+    return 1 if pages <= 4 else max(1, min(64, (pages + 1) // 2, 160 // pairs))
 
 
 @functools.lru_cache(maxsize=256)
@@ -1279,7 +1281,7 @@ def decode_chain_words(layer: ChainLayer, rows: int, n_layers: int) -> int:
     """64-bit words of state a chain of ``n_layers`` such layers needs for ``rows`` tokens (one per sequence); 0: not taken."""
     return library("decode_chain").rocml_decode_chain_words(
         _code(layer.w_qkv), rows, layer.hidden, layer.n_heads, layer.n_kv_heads, CHAIN_HEAD_DIM, layer.inter, n_layers,
-        decode_chain_splits(layer.block_table.shape[1]))
+        decode_chain_splits(layer.block_table.shape[1], rows * layer.n_kv_heads))
 
 
 def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer], token_pos: torch.Tensor, cos: torch.Tensor,
@@ -1336,7 +1338,7 @@ def decode_chain(x: torch.Tensor, xn: torch.Tensor, layers: Sequence[ChainLayer]
     _check("decode_chain", library("decode_chain").rocml_decode_chain(
         _code(first.w_qkv), _ptr(state), state.numel(), _ptr(x), _ptr(xn), pointers, len(layers), rows, hidden, first.n_heads, first.n_kv_heads,
         CHAIN_HEAD_DIM, first.inter, _ptr(first.block_table), first.block_table.shape[1], _ptr(token_pos), _ptr(cos), _ptr(sin),
-        first.scale, first.qk_eps, first.mix_eps, first.ffn_eps, decode_chain_splits(first.block_table.shape[1]),
+        first.scale, first.qk_eps, first.mix_eps, first.ffn_eps, decode_chain_splits(first.block_table.shape[1], rows * first.n_kv_heads),
         polls, -1 if patience < 0 else int(patience * 1e8), _ptr(late), blocks, _stream()))
 
 
