@@ -69,8 +69,7 @@ __device__ __forceinline__ void af_softmax(af_f32x4_t (&s)[NT], af_f32x4_t (&o)[
             s[t][e] = seen ? v : -INFINITY;
             top = fmaxf(top, s[t][e]);
         }
-    top = fmaxf(top, __shfl_xor(top, 16, 64));
-    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    top = rows4_max(top);
     float m_new = fmaxf(m, top);
     float ref = m_new == -INFINITY ? 0.f : m_new;     // nothing seen yet: every probability is exp(-inf)
     float corr = expf(m - ref);
@@ -201,8 +200,7 @@ attn_f32_prompt_kernel(AttnF32Args a) {
         af_values<KD, 4>(s, [&](int c, int kt) { return *(const af_f32x4_t*)(vs + (c * 16 + (lane & 15)) * VS + kt * 16 + (lane >> 4) * 4); }, o);
         if (repair) af_add_odd_values<KD>(s, a.vcache + at, o, a, p * AF_PAGE, lane, pos, lo);
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows4_sum(l);
     float down = 1.f;
     if (a.ex.sink) {
         float sink = a.ex.sinks ? a.ex.sinks[h] : 0.f, top = fmaxf(m, sink);
@@ -294,8 +292,7 @@ attn_f32_token_kernel(AttnF32Args a) {
             return u;
         }, o);
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = rows4_sum(l);
     if (lane < 16) {
         ms[wave * 16 + lane] = m;
         ls[wave * 16 + lane] = l;

@@ -200,8 +200,7 @@ attn_latent_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, 
                     s[rt][u][i] = v;
                     mx = fmaxf(mx, v);
                 }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            mx = rows4_max(mx);
             // The exponents' reference m follows a row's maximum only when that has grown by more than
             // AL_LAZY_MAX: any reference gives the same quotient at the end, the probabilities stay below
             // 2^AL_LAZY_MAX, and the sums and outputs so far are rescaled only for a row's first pieces
@@ -223,8 +222,7 @@ attn_latent_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, 
                     s[rt][u][i] = fast_exp2(s[rt][u][i] - m_use);
                     sum += s[rt][u][i];
                 }
-            sum += __shfl_xor(sum, 16, 64);
-            sum += __shfl_xor(sum, 32, 64);
+            sum = rows4_sum(sum);
             l[rt] += sum;
             // P^T operand: slot 2 i + u = key 8 g + 4 u + i, the order of the transposed copy
             pf[rt] = __builtin_bit_cast(bf16x8_t, make_uint4(pack_bf16x2(s[rt][0][0], s[rt][1][0]), pack_bf16x2(s[rt][0][1], s[rt][1][1]),
@@ -339,8 +337,7 @@ attn_latent_few_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, c
                 mx = fmaxf(mx, s[u][i]);
             }
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows4_max(mx);
         const float m_new = fmaxf(m, mx), m_use = m_new == -INFINITY ? 0.f : m_new, corr = fast_exp2(m - m_use);
         float sum = 0.f;
 #pragma unroll
@@ -350,8 +347,7 @@ attn_latent_few_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out, c
                 s[u][i] = fast_exp2(s[u][i] - m_use);
                 sum += s[u][i];
             }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
+        sum = rows4_sum(sum);
         l = l * corr + sum;
         m = m_new;
         // P^T operand: slot 2 i + u = key 8 g + 4 u + i, the order of the transposed copy

@@ -366,8 +366,7 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
                 s[u][i] = v;
                 mx = fmaxf(mx, v);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows4_max(mx);
         float m_new = fmaxf(m, mx);
         float m_use = m_new == -INFINITY ? 0.f : m_new;
         float corr = fast_exp2(m - m_use);
@@ -379,8 +378,7 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
                 s[u][i] = fast_exp2(s[u][i] - m_use);
                 sum += s[u][i];
             }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
+        sum = rows4_sum(sum);
         l = l * corr + sum;
         m = m_new;
         // P^T operand: slots 0..7 = keys 8g .. 8g+7.

@@ -201,7 +201,7 @@ __device__ __forceinline__ float dc_row_scale(const DcArgs& a, const u64* ssq, i
         dc_collect<1>(a, epoch, mine, mine ? at * (8u * DC_APART) : 0u, [&](int, uint32_t o) { return dc_at(ssq, o); }, v);
         ss += mine ? __uint_as_float(v[0]) : 0.f;
     }
-    return 1.0f / sqrtf(lanes_sum(ss) * a.inv_width + eps);
+    return 1.0f / sqrtf(wave_sum(ss) * a.inv_width + eps);
 }
 
 // A block's place in the order: {launch, ticket} of its counter, handed on as {launch, item}; the items shard, shard + DC_SHARDS,
@@ -763,7 +763,7 @@ __device__ __forceinline__ void dc_attention(const DcArgs& a, const DcLayer& ly,
             if (r >= n_rows) break;
             float v0 = __uint_as_float(raw[2 * i]) * row_scale, v1 = __uint_as_float(raw[2 * i + 1]) * row_scale;
             if (r <= group) {
-                float inv = 1.0f / sqrtf(lanes_sum(fmaf(v1, v1, v0 * v0)) / (float)D + a.qk_eps);
+                float inv = 1.0f / sqrtf(wave_sum(fmaf(v1, v1, v0 * v0)) / (float)D + a.qk_eps);
                 v0 = v0 * inv * (r < group ? gq0 : gk0);
                 v1 = v1 * inv * (r < group ? gq1 : gk1);
                 // pairs (e, e + 64) are one lane's

@@ -406,8 +406,7 @@ diff_decode_kernel(DiffArgs a, DiffProj pj, int n_splits, float* __restrict__ pa
                 s[u][i] = v;
                 mx = fmaxf(mx, v);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = rows4_max(mx);
         float m_new = fmaxf(m, mx);
         float m_use = m_new == -INFINITY ? 0.f : m_new;
         float corr = da_exp2(m - m_use), sum = 0.f;
@@ -418,8 +417,7 @@ diff_decode_kernel(DiffArgs a, DiffProj pj, int n_splits, float* __restrict__ pa
                 s[u][i] = da_exp2(s[u][i] - m_use);
                 sum += s[u][i];
             }
-        sum += __shfl_xor(sum, 16, 64);
-        sum += __shfl_xor(sum, 32, 64);
+        sum = rows4_sum(sum);
         l = l * corr + sum;
         m = m_new;
         uint4 pv = make_uint4(f32x2_to_bf16x2(s[0][0], s[0][1]), f32x2_to_bf16x2(s[0][2], s[0][3]),

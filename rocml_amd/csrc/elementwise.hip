@@ -646,8 +646,16 @@ qkv_rows_append_kernel(
                 float ss = lo[i].x * lo[i].x;
                 ss = fmaf(lo[i].y, lo[i].y, ss); ss = fmaf(lo[i].z, lo[i].z, ss); ss = fmaf(lo[i].w, lo[i].w, ss);
                 ss = fmaf(hi[i].x, hi[i].x, ss); ss = fmaf(hi[i].y, hi[i].y, ss); ss = fmaf(hi[i].z, hi[i].z, ss); ss = fmaf(hi[i].w, hi[i].w, ss);
+                if constexpr (LANES < 16) {
 #pragma unroll
-                for (int off = LANES / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
+                    for (int off = LANES / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
+                } else {
+                    if constexpr (LANES == 32) {
+                        const LanePair both = lane_pair16(ss);
+                        ss = both.a + both.b;
+                    }
+                    ss = row16_sum_far(ss);
+                }
                 inv = 1.0f / sqrtf(ss / (float)D + eps);
             }
             scale(lo[i], inv, row4(gain + e));

@@ -149,8 +149,7 @@ __device__ __forceinline__ float row_scale_finish(RowScale rs, int lane, int m, 
         float4 v = mine[j];
         s += (v.x + v.y) + (v.z + v.w);
     }
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
+    s = rows4_sum(s);
     return (lane & 15) < m ? 1.0f / sqrtf(s * rs.inv_width + rs.eps) : 1.0f;
 }
 
@@ -928,8 +927,7 @@ gemm_residual_prescale_kernel(const bf16_t* __restrict__ x, int ldx, const bf16_
             ss = fmaf(r, r, ss);
         }
     }
-    ss += __shfl_xor(ss, 16, 64);
-    ss += __shfl_xor(ss, 32, 64);
+    ss = rows4_sum(ss);
     if (row_ok && g == 0) ssq[(size_t)col * tiles + tile] = ss;
 }
 
