@@ -55,7 +55,8 @@ ROCML_EXPORT int rocml_embed_gather(const void* table, int table_dtype, const in
 }
 
 // ---- block reduction -------------------------------------------------------------
-// Sum over a block of EW_BLOCK threads in a fixed order: lanes by butterfly, waves in order.
+// Sum over a block of threads in a fixed order: lanes by butterfly, waves in order.
+template <int THREADS = EW_BLOCK>
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     v = wave_sum(v);
     int wave = threadIdx.x / WAVE;
@@ -64,7 +65,7 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     __syncthreads();
     float total = 0.f;
 #pragma unroll
-    for (int w = 0; w < EW_BLOCK / WAVE; ++w) total += scratch[w];
+    for (int w = 0; w < THREADS / WAVE; ++w) total += scratch[w];
     return total;
 }
 
@@ -104,6 +105,15 @@ __global__ void rmsnorm_kernel(float* x, const float* __restrict__ gain, TO* __r
 // Same result for rows of up to 8192 values that are a multiple of 4: the row stays in
 // registers between the two passes and all loads are issued at once (a loop of single loads
 // waits for each one in turn, which is what a one-row decode step would spend its time on).
+// RN_VEC: the vectors of a row that a thread holds; RN_GROUP: the splits whose loads are in flight
+// together.  A prompt is bound by memory, through how many rows a CU holds at once, which is a matter
+// of registers (eight splits of four vectors 172, one split 60, of one vector 16), a step of a few
+// rows by its loads' latency.  So both follow the call; with four vectors and eight splits for all,
+// threads loaded what the call has not over again (a row of 1024 values with 4 splits: 36 loads for 6).
+// In us, that against this, 1024 rows of 1024 values with 4 splits 9.0 -> 4.1, 2048 rows of 4096 with 1
+// 24.0 -> 17.4 (6.7 TB/s), 8192 of them 95.7 -> 68.4; one row of 1024 with 4 splits 3.5 -> 2.2.
+// (Skipping the absent splits of a larger group by branches instead took 6.7 for 4.3 at 8 rows of 4096
+// with 8 splits: the loads then wait for each other.)
 constexpr int RN_MAX_VEC = 8;
 
 __device__ __forceinline__ void store4(float* p, float a, float b, float c, float d) {
@@ -116,12 +126,12 @@ __device__ __forceinline__ void store4(bf16_t* p, float a, float b, float c, flo
     *(uint2*)p = v;
 }
 
-template <typename TO, int RN_VEC>
-__global__ void __launch_bounds__(EW_BLOCK)
+template <typename TO, int RN_VEC, int RN_GROUP, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 rmsnorm_vec_kernel(float* x, const float* __restrict__ gain, TO* __restrict__ out,
                    const int* __restrict__ rows, int n, float eps, const float* __restrict__ partials,
                    int n_splits, long long split_stride) {
-    __shared__ float scratch[EW_BLOCK / WAVE];
+    __shared__ float scratch[THREADS / WAVE];
     int r = blockIdx.x;
     int src = rows ? rows[r] : r;
     float4* xin = (float4*)(x + (size_t)src * n);
@@ -132,7 +142,7 @@ rmsnorm_vec_kernel(float* x, const float* __restrict__ gain, TO* __restrict__ ou
     float ss = 0.f;
 #pragma unroll
     for (int j = 0; j < RN_VEC; ++j) {
-        int idx = threadIdx.x + j * EW_BLOCK;
+        int idx = threadIdx.x + j * THREADS;
         bool ok = idx < nv;
         v[j] = xin[ok ? idx : 0];
         g[j] = g4[ok ? idx : 0];
@@ -141,29 +151,28 @@ rmsnorm_vec_kernel(float* x, const float* __restrict__ gain, TO* __restrict__ ou
     if (n_splits > 0) {
         const float4* p4 = (const float4*)(partials + (size_t)src * n);
         long long stride4 = split_stride / 4;
-        constexpr int GROUP = 32 / RN_VEC;              // splits whose loads are in flight together
-        for (int sp = 0; sp < n_splits; sp += GROUP) {  // loads of a group all issued, added in split order
-            float4 a[GROUP][RN_VEC];
+        for (int sp = 0; sp < n_splits; sp += RN_GROUP) {  // loads of a group all issued, added in split order
+            float4 a[RN_GROUP][RN_VEC];
 #pragma unroll
-            for (int q = 0; q < GROUP; ++q)
+            for (int q = 0; q < RN_GROUP; ++q)
 #pragma unroll
                 for (int j = 0; j < RN_VEC; ++j) {
-                    int idx = threadIdx.x + j * EW_BLOCK;
+                    int idx = threadIdx.x + j * THREADS;
                     int safe = idx < nv ? idx : 0;
                     a[q][j] = p4[(sp + q < n_splits ? sp + q : sp) * stride4 + safe];
                 }
 #pragma unroll
-            for (int q = 0; q < GROUP; ++q)
+            for (int q = 0; q < RN_GROUP; ++q)
 #pragma unroll
                 for (int j = 0; j < RN_VEC; ++j) {
-                    if ((int)threadIdx.x + j * EW_BLOCK >= nv || sp + q >= n_splits) continue;
+                    if ((int)threadIdx.x + j * THREADS >= nv || sp + q >= n_splits) continue;
                     v[j].x += a[q][j].x; v[j].y += a[q][j].y; v[j].z += a[q][j].z; v[j].w += a[q][j].w;
                 }
         }
         if (!rows) {
 #pragma unroll
             for (int j = 0; j < RN_VEC; ++j) {
-                int idx = threadIdx.x + j * EW_BLOCK;
+                int idx = threadIdx.x + j * THREADS;
                 if (idx < nv) xin[idx] = v[j];
             }
         }
@@ -171,15 +180,26 @@ rmsnorm_vec_kernel(float* x, const float* __restrict__ gain, TO* __restrict__ ou
 #pragma unroll
     for (int j = 0; j < RN_VEC; ++j)
         ss = fmaf(v[j].x, v[j].x, fmaf(v[j].y, v[j].y, fmaf(v[j].z, v[j].z, fmaf(v[j].w, v[j].w, ss))));
-    float total = block_sum(ss, scratch);
+    float total = block_sum<THREADS>(ss, scratch);
     float inv = 1.0f / sqrtf(total / (float)n + eps);
 #pragma unroll
     for (int j = 0; j < RN_VEC; ++j) {
-        int idx = threadIdx.x + j * EW_BLOCK;
+        int idx = threadIdx.x + j * THREADS;
         if (idx < nv)
             store4(o + 4 * idx, v[j].x * inv * g[j].x, v[j].y * inv * g[j].y, v[j].z * inv * g[j].z,
                    v[j].w * inv * g[j].w);
     }
+}
+
+template <typename TO, int RN_VEC, int THREADS>
+static void launch_rmsnorm_vec(float* x, const float* gain, TO* out, const int* rows, int n_rows, int n, float eps, const float* partials,
+                               int n_splits, long long split_stride, hipStream_t stream) {
+#define RN(GROUP_) rmsnorm_vec_kernel<TO, RN_VEC, GROUP_, THREADS><<<n_rows, THREADS, 0, stream>>>(x, gain, out, rows, n, eps, partials, n_splits, split_stride)
+    if (n_splits <= 1) RN(1);
+    else if (n_splits == 2) RN(2);
+    else if (n_splits <= 4) RN(4);
+    else RN((RN_VEC > 4 ? 4 : 8));
+#undef RN
 }
 
 ROCML_EXPORT int rocml_rmsnorm(float* x, const float* gain, void* out, int out_dtype, const int* rows,
@@ -193,16 +213,28 @@ ROCML_EXPORT int rocml_rmsnorm(float* x, const float* gain, void* out, int out_d
     bool vec = n % 4 == 0 && n <= 4 * RN_MAX_VEC * EW_BLOCK && (uintptr_t)x % 16 == 0 &&
                (uintptr_t)gain % 16 == 0 && (uintptr_t)out % 16 == 0 &&
                (n_splits == 0 || ((uintptr_t)partials % 16 == 0 && split_stride % 4 == 0));
+    int per = ceil_div(n, 4 * EW_BLOCK);     // vectors a thread
+    // Up to 512 rows are on the chip at once also with 1024 threads each, and a thread then has one or two vectors
+    // to wait for: 64 rows of 4096 values with 8 splits 4.5 -> 3.8 us, 512 rows with 4 10.3 -> 9.0.
+    bool few = n_rows <= 512;
+#define RN_ARGS rows, n_rows, n, eps, partials, n_splits, split_stride, stream
+#define RN_TYPE(TO_)                                                                              \
+    {                                                                                             \
+        if (per <= 1) launch_rmsnorm_vec<TO_, 1, EW_BLOCK>(x, gain, (TO_*)out, RN_ARGS);           \
+        else if (few && per <= 2) launch_rmsnorm_vec<TO_, 1, 512>(x, gain, (TO_*)out, RN_ARGS);    \
+        else if (few && per <= 4) launch_rmsnorm_vec<TO_, 1, 1024>(x, gain, (TO_*)out, RN_ARGS);   \
+        else if (few) launch_rmsnorm_vec<TO_, 2, 1024>(x, gain, (TO_*)out, RN_ARGS);               \
+        else if (per <= 2) launch_rmsnorm_vec<TO_, 2, EW_BLOCK>(x, gain, (TO_*)out, RN_ARGS);      \
+        else if (per <= 3) launch_rmsnorm_vec<TO_, 3, EW_BLOCK>(x, gain, (TO_*)out, RN_ARGS);      \
+        else if (per <= 4) launch_rmsnorm_vec<TO_, 4, EW_BLOCK>(x, gain, (TO_*)out, RN_ARGS);      \
+        else if (per <= 5) launch_rmsnorm_vec<TO_, 5, EW_BLOCK>(x, gain, (TO_*)out, RN_ARGS);      \
+        else launch_rmsnorm_vec<TO_, 8, EW_BLOCK>(x, gain, (TO_*)out, RN_ARGS);                    \
+    }
+    if (vec && out_dtype == ROCML_F32) RN_TYPE(float)
+    else if (vec && out_dtype == ROCML_BF16) RN_TYPE(bf16_t)
+#undef RN_TYPE
+#undef RN_ARGS
 #define RN_ARGS rows, n, eps, partials, n_splits, split_stride
-    bool small = n <= 4 * 4 * EW_BLOCK;      // rows of up to 4096 values: 4 vectors per thread
-    if (vec && out_dtype == ROCML_F32 && small)
-        rmsnorm_vec_kernel<float, 4><<<n_rows, EW_BLOCK, 0, stream>>>(x, gain, (float*)out, RN_ARGS);
-    else if (vec && out_dtype == ROCML_F32)
-        rmsnorm_vec_kernel<float, 8><<<n_rows, EW_BLOCK, 0, stream>>>(x, gain, (float*)out, RN_ARGS);
-    else if (vec && out_dtype == ROCML_BF16 && small)
-        rmsnorm_vec_kernel<bf16_t, 4><<<n_rows, EW_BLOCK, 0, stream>>>(x, gain, (bf16_t*)out, RN_ARGS);
-    else if (vec && out_dtype == ROCML_BF16)
-        rmsnorm_vec_kernel<bf16_t, 8><<<n_rows, EW_BLOCK, 0, stream>>>(x, gain, (bf16_t*)out, RN_ARGS);
     else if (out_dtype == ROCML_F32)
         rmsnorm_kernel<float><<<n_rows, EW_BLOCK, 0, stream>>>(x, gain, (float*)out, RN_ARGS);
     else if (out_dtype == ROCML_BF16)
