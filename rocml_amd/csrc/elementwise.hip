@@ -2118,12 +2118,13 @@ __global__ void __launch_bounds__(EW_BLOCK)
 added_conv_kernel(const T* __restrict__ h, T* __restrict__ out, int n, const float* __restrict__ w, T* __restrict__ state,
                   const int* __restrict__ cu_seqlens, const int* __restrict__ seq_slots, int n_seqs) {
     int c = (blockIdx.y * EW_BLOCK + threadIdx.x) * W;
-    int run = blockIdx.x, b = 0, first = 0, count = 0;
+    int run = blockIdx.x, b = 0, first = 0, count = 0, slot = 0;
     if (gridDim.x == (unsigned)n_seqs) {         // a run per sequence (a step of one token each, or short prompts)
         b = run;
         run = 0;
         first = cu_seqlens[b];
         count = cu_seqlens[b + 1] - first;
+        slot = seq_slots[b];
     } else {
         for (; b < n_seqs; ++b) {
             first = cu_seqlens[b];
@@ -2133,6 +2134,7 @@ added_conv_kernel(const T* __restrict__ h, T* __restrict__ out, int n, const flo
             run -= runs;
         }
         if (b >= n_seqs) return;
+        slot = seq_slots[b];
     }
     if (c >= n) return;
     int t0 = run * AC_RUN, t1 = min(count, t0 + AC_RUN);         // the run, in tokens of the sequence's part of the step
@@ -2142,11 +2144,32 @@ added_conv_kernel(const T* __restrict__ h, T* __restrict__ out, int n, const flo
     for (int j = 0; j < TAPS; ++j)
 #pragma unroll
         for (int i = 0; i < W; ++i) tap[j][i] = w[(size_t)j * n + c + i];
-    T* kept = state + (size_t)seq_slots[b] * KEPT * n + c;
+    T* kept = state + (size_t)slot * KEPT * n + c;
 #pragma unroll
     for (int j = 0; j < KEPT; ++j) {
         if (t0 == 0) ac_load<T, W>(past[j], kept + (size_t)j * n);
         else ac_load<T, W>(past[j], h + (size_t)(first + t0 - KEPT + j) * n + c);
+    }
+    if (KEPT > 0 && count == 1) {
+        // A step of one token: all that it reads is on its way in one trip, and no load stands behind a store (in the general
+        // form the token is read twice, the second time behind the kept rows' stores): twelve requests of 300 to 2,500 tokens and
+        // 32 steps of kakalorn-2b 37.16 -> 36.91 ms.
+        float cur[W], y[W];
+        size_t at = (size_t)first * n + c;
+        ac_load<T, W>(cur, h + at);
+#pragma unroll
+        for (int i = 0; i < W; ++i) {
+            float a = 0.f;
+#pragma unroll
+            for (int j = 0; j < KEPT; ++j) a = fmaf(tap[j][i], past[j][i], a);
+            a = fmaf(tap[KEPT][i], cur[i], a);
+            y[i] = cur[i] + a;
+        }
+        ac_store<T, W>(out + at, y);
+#pragma unroll
+        for (int j = 0; j + 1 < KEPT; ++j) ac_store<T, W>(kept + (size_t)j * n, past[j + 1]);
+        ac_store<T, W>(kept + (size_t)(KEPT > 0 ? KEPT - 1 : 0) * n, cur);
+        return;
     }
     if (KEPT > 0 && t0 == 0) {
         // the rows kept for the next step: the last of this step's, behind old ones where it brings fewer
