@@ -225,7 +225,7 @@ template <int V> struct DcInt { static constexpr int value = V; };
 // What a block works on, the same for all its threads.
 struct DcItem { int stage, layer, i; uint32_t epoch; };
 
-// LDS of a block.  (The arrays are read 16 bytes at a time; at an odd multiple of 8 a step of 526 us takes 695.)
+// LDS of a block.  (The arrays are read 16 bytes at a time; at an odd multiple of 8 a step takes a third longer.)
 template <int W>
 struct DcLds {
     u64 next[2];                                // the item after this one, in turn
