@@ -1189,6 +1189,9 @@ struct DecayScanArgs {
 // but a sequence's last from a state of zero and keeps the state it ends with and the product of its decays (no output, 0.6 of a
 // walk's work); decay_segments_kernel turns these into the state that every segment starts from; DECAY_PASS_OUT walks all
 // segments from there, side by side.  A sequence's segments are numbered behind those of the sequences before it.
+// Blocks of one launch come in any order, over several rounds, so no launch both reads and writes a sequence's state: the output pass,
+// whose last segment writes it, finds the state that the first one starts from in the last segment's place, which the first pass leaves
+// free.  (A sequence of one segment is one block's, which reads its columns before it writes them.)
 enum DecayPass : int { DECAY_PASS_ALL = 0, DECAY_PASS_STATE = 1, DECAY_PASS_OUT = 2 };
 struct DecaySegment { int seq, at, of, number; };        // its sequence, place in it, how many that has, the segment's number
 
@@ -1306,7 +1309,8 @@ decay_scan_kernel(DecayScanArgs a) {
     }
     float* st = a.state + ((size_t)a.seq_slots[b] * a.n_heads + h) * a.dv * dk;
     if constexpr (PASS != DECAY_PASS_ALL) {          // where the walk's state comes from, or goes to
-        if (PASS == DECAY_PASS_STATE || seg.at > 0) st = a.seg_state + ((size_t)(seg.number - (PASS == DECAY_PASS_OUT)) * a.n_heads + h) * a.dv * dk;
+        const int place = PASS == DECAY_PASS_STATE ? seg.number : seg.at > 0 ? seg.number - 1 : seg.number + seg.of - 1;
+        if (PASS == DECAY_PASS_STATE || seg.of > 1) st = a.seg_state + ((size_t)place * a.n_heads + h) * a.dv * dk;
     }
     float s[CPL][R], u[R];
     float prod[PASS == DECAY_PASS_STATE ? R : 1];     // the decays of the tokens so far, multiplied (first rows of lanes, first tile)
@@ -1582,7 +1586,7 @@ decay_scan_kernel(DecayScanArgs a) {
 }
 
 // The states that the segments of a sequence start from, in place: the slot of segment i goes from what that segment adds to the state
-// behind it.  A thread has four entries of a head's state, dk along a column; the states of eight segments are asked for together.
+// behind it, and the last one's takes the sequence's own state, from which its first segment starts.  A thread has four entries of a head's state, dk along a column; the states of eight segments are asked for together.
 __global__ void __launch_bounds__(256)
 decay_segments_kernel(DecayScanArgs a) {
     const int b = blockIdx.z, h = blockIdx.y, dk = a.dk, e = (blockIdx.x * 256 + threadIdx.x) * 4;
@@ -1593,6 +1597,7 @@ decay_segments_kernel(DecayScanArgs a) {
     const int n_segs = (a.cu_seqlens[b + 1] - a.cu_seqlens[b] + a.segment - 1) / a.segment;
     if (n_segs < 2 || e >= a.dv * dk) return;
     float4 s = *(const float4*)(a.state + ((size_t)a.seq_slots[b] * a.n_heads + h) * a.dv * dk + e);
+    *(float4*)(a.seg_state + ((size_t)(number + n_segs - 1) * a.n_heads + h) * a.dv * dk + e) = s;
     constexpr int AHEAD = 8;
     for (int i0 = 0; i0 < n_segs - 1; i0 += AHEAD) {
         float4 own[AHEAD], w[AHEAD];

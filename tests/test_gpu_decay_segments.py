@@ -90,3 +90,27 @@ def test_segments_fit_the_memory():
         assert torch.all(ws[room:] == 7)
         for a, b in zip(got, want):
             assert float((a - b).norm() / b.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("lens,H,segment", [([16 * 64 + 1], 32, 16), ([1, 40, 16, 0, 33], 2, 16)])
+def test_first_segments_start_from_the_state_before_the_step(lens, H, segment):
+    """The last segment's block may have written a sequence's new state before the first segment's block starts: many more blocks than
+    the chip holds, last segments of one token.  A first segment reads a copy, in the place that the last segment leaves free."""
+    dk, dv = 128, 128
+    case = _case(lens, H, dk, dv, "token")
+    _, cu, _, state, slots = case
+    numbers = [0]
+    for n in lens:
+        numbers.append(numbers[-1] + -(-n // segment))
+    count = sum(lens) // segment + len(lens)
+    ws = torch.full((count * H * (dv + 1) * dk * 4,), 0x7f, dtype=torch.uint8, device=DEV)
+    out, st = _run(lens, H, dk, dv, "token", case, workspace=ws, segment=segment)
+    whole, st_whole = _run(lens, H, dk, dv, "token", case, segment=-1)
+    places = ws[:count * H * dv * dk * 4].view(torch.float32).view(count, H, dv, dk).cpu()
+    for b, n in enumerate(lens):
+        if n > segment:
+            assert torch.equal(places[numbers[b + 1] - 1], state[slots[b]]), "the state before the step"
+        got, want = out[cu[b]:cu[b] + min(n, segment)], whole[cu[b]:cu[b] + min(n, segment)]
+        # the same walk from the same state: sums of 128 products at most in another order
+        assert n == 0 or float((got - want).norm() / want.norm()) < 2e-6
+    assert float((out - whole).norm() / whole.norm()) < 2e-6 and float((st - st_whole).norm() / st_whole.norm()) < 2e-6
