@@ -661,7 +661,8 @@ template <int W> struct DcPieces<float, W> {
                 float top = -INFINITY;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    s[e] = quad * 4 + e <= at ? rows4_sum(s[e] + odd[e]) * a.scale : -INFINITY;
+                    const float sum = rows4_sum(s[e] + odd[e]) * a.scale;       // (by all lanes, seen or not)
+                    s[e] = quad * 4 + e <= at ? sum : -INFINITY;
                     top = fmaxf(top, s[e]);
                 }
                 top = fmaxf(top, lane_dpp<0x128>(top));             // (rotated by 8 and by 4 lanes inside the row)
