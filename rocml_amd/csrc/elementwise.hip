@@ -620,6 +620,28 @@ __device__ __forceinline__ float4 row4(const bf16_t* p) {
     return make_float4(__uint_as_float(a.x << 16), __uint_as_float(a.x & 0xffff0000u), __uint_as_float(a.y << 16), __uint_as_float(a.y & 0xffff0000u));
 }
 
+// The sum of the squares of a row of D = 128 or 256 numbers, of which lane l of D/8 has 4l .. 4l + 3 (lo) and D/2 behind them (hi), in the
+// order of qk_norm_rope_append_kernel: there a lane has the numbers lane, lane + 64, ... and the wave adds up by a butterfly from 32
+// lanes apart to 1.  Here those lanes are the four numbers of a vector, four neighbours a lane, so the butterfly's first four steps
+// (32 to 4 apart) are steps of 8 to 1 lanes and its last two stay in the lane: a token's q and k are the same bits in a step of
+// few tokens and of many (rows of 128: 16 exchanges for 4, none of them through LDS; 8,192 tokens of 40 rows 62.1 us for 61.2).
+template <int D>
+__device__ __forceinline__ float head_squares(float4 lo, float4 hi) {
+    float ss[4];
+    const float a[4] = {lo.x, lo.y, lo.z, lo.w}, b[4] = {hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if constexpr (D == 128) {
+            ss[c] = fmaf(b[c], b[c], a[c] * a[c]);
+        } else {
+            const LanePair p = lane_pair16(a[c]), q = lane_pair16(b[c]);          // the numbers 64 apart are lanes 16 apart
+            ss[c] = fmaf(q.b, q.b, fmaf(q.a, q.a, fmaf(p.b, p.b, p.a * p.a)));
+        }
+        ss[c] = row16_sum_far(ss[c]);
+    }
+    return (ss[0] + ss[2]) + (ss[1] + ss[3]);
+}
+
 // Prompts: q and k rows of many tokens, whole heads of D = 128 or 256 rotated (pairs (e, e + D/2)) or none, complete projections, and
 // behind them in the same launch the values' tiles.  D/8 lanes have a row, eight values each: four pairs, so a rotation needs no
 // exchange and every load and store is 16 (or 8) bytes; a wave works on 64 / (D/8) rows at once and asks for PASSES
@@ -675,19 +697,7 @@ qkv_rows_append_kernel(
                 inv = span_inv[(size_t)tok[i] * 2 + (is_q ? 0 : 1)];
                 gain += (is_q ? rr[i] : rr[i] - hq) * D;
             } else {
-                float ss = lo[i].x * lo[i].x;
-                ss = fmaf(lo[i].y, lo[i].y, ss); ss = fmaf(lo[i].z, lo[i].z, ss); ss = fmaf(lo[i].w, lo[i].w, ss);
-                ss = fmaf(hi[i].x, hi[i].x, ss); ss = fmaf(hi[i].y, hi[i].y, ss); ss = fmaf(hi[i].z, hi[i].z, ss); ss = fmaf(hi[i].w, hi[i].w, ss);
-                if constexpr (LANES < 16) {
-#pragma unroll
-                    for (int off = LANES / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
-                } else {
-                    if constexpr (LANES == 32) {
-                        const LanePair both = lane_pair16(ss);
-                        ss = both.a + both.b;
-                    }
-                    ss = row16_sum_far(ss);
-                }
+                const float ss = head_squares<D>(lo[i], hi[i]);
                 inv = 1.0f / sqrtf(ss / (float)D + eps);
             }
             scale(lo[i], inv, row4(gain + e));
@@ -701,8 +711,9 @@ qkv_rows_append_kernel(
         }
         if (cos_t) {
             const float4 a = lo[i], b = hi[i], c = cs[i], n = sn[i];
-            lo[i] = make_float4(a.x * c.x - b.x * n.x, a.y * c.y - b.y * n.y, a.z * c.z - b.z * n.z, a.w * c.w - b.w * n.w);
-            hi[i] = make_float4(a.x * n.x + b.x * c.x, a.y * n.y + b.y * c.y, a.z * n.z + b.z * c.z, a.w * n.w + b.w * c.w);
+            // (which product is rounded before the sum is said here: left to the compiler it differed between the forms of this kernel)
+            lo[i] = make_float4(fmaf(a.x, c.x, -(b.x * n.x)), fmaf(a.y, c.y, -(b.y * n.y)), fmaf(a.z, c.z, -(b.z * n.z)), fmaf(a.w, c.w, -(b.w * n.w)));
+            hi[i] = make_float4(fmaf(b.x, c.x, a.x * n.x), fmaf(b.y, c.y, a.y * n.y), fmaf(b.z, c.z, a.z * n.z), fmaf(b.w, c.w, a.w * n.w));
         }
         if (row0 + i * SETS >= total) continue;
         TO* dst;
