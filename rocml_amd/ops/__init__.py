@@ -81,6 +81,7 @@ _SIGNATURES = {
         "rocml_splitk_reduce": [_P, _P, _I, _I, _I, _I, _I, _I, _P],
         "rocml_gemm_batched": [_P, _I, _I, _LL, _P, _I, _I, _LL, _P, _I, _I, _LL, _I, _I, _I, _I, _P, _I, _LL, _I, _P],
         "rocml_latent_queries": [_P, _I, _I, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P],
+        "rocml_gemm_tile_algo": [_I, _I, _I, _I],
         "rocml_gemm_residual_prescale_pays": [_I, _I, _I],
         "rocml_gemm_residual_prescale": [_P, _I, _P, _I, _P, _I, _P, _P, _I, _P, _I, _I, _I, _I, _P, _P],
     },
