@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 from rocml_amd import ops  # noqa: E402
 from rocml_amd.errors import KernelError  # noqa: E402
 
-PLAIN, TILE, SKINNY, KPAR, TILE256, TILE192, TILE128X192, TILE256X96, TILE64X256 = 1, 2, 3, 4, 5, 6, 7, 8, 9
+PLAIN, TILE, SKINNY, KPAR, TILE256, TILE256X192, TILE128X192, TILE256X128, TILE64X128 = 1, 2, 3, 4, 5, 6, 7, 8, 9
 
 
 def _operands(m, n, k, dtype, seed):
@@ -41,7 +41,7 @@ SHAPES = [(1, 64, 64), (5, 200, 72), (16, 130, 512), (17, 96, 264), (33, 4096, 1
           (1409, 300, 128), (2561, 200, 64)]       # 12 and 21 tile rows of 128, 6 and 11 of 256: whole bands of eight and a rest
 
 
-@pytest.mark.parametrize("algo", [PLAIN, TILE, SKINNY, KPAR, TILE256, TILE192, TILE128X192, TILE256X96, TILE64X256])
+@pytest.mark.parametrize("algo", [PLAIN, TILE, SKINNY, KPAR, TILE256, TILE256X192, TILE128X192, TILE256X128, TILE64X128])
 @pytest.mark.parametrize("m,n,k", SHAPES)
 def test_bfloat16_algorithms(m, n, k, algo):
     if (algo == SKINNY and m > 64) or (algo == KPAR and m > 16):
@@ -213,7 +213,7 @@ def test_few_rows_far_apart(m, n, k, which, sixteen_far_rows):
         assert float((h.double() - want).abs().max()) < 5e-3 * max(1.0, float(want.abs().max()))
 
 
-@pytest.mark.parametrize("algo", [PLAIN, TILE, SKINNY, KPAR, TILE256, TILE192, TILE128X192, TILE256X96, TILE64X256])
+@pytest.mark.parametrize("algo", [PLAIN, TILE, SKINNY, KPAR, TILE256, TILE256X192, TILE128X192, TILE256X128, TILE64X128])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (7, 448, 96), (25, 300, 520), (41, 130, 1032), (64, 1000, 264), (130, 256, 128), (300, 2048, 512)])
 def test_gated_epilogue(m, n, k, algo):
     """Rows of the weight are (gate, up) pairs; the output is silu(gate) * up, formed from
@@ -248,7 +248,7 @@ def test_float32_gated_by_the_plain_kernel(m, n, k, algo):
         assert float((out.double() - ref).abs().max()) < 2e-5 * max(1.0, float(ref.abs().max())), epilogue
 
 
-@pytest.mark.parametrize("m,algo", [(1, KPAR), (8, SKINNY), (40, SKINNY), (130, TILE), (130, TILE64X256), (130, TILE192), (300, TILE256)])
+@pytest.mark.parametrize("m,algo", [(1, KPAR), (8, SKINNY), (40, SKINNY), (130, TILE), (130, TILE64X128), (130, TILE256X192), (300, TILE256)])
 def test_gated_results_are_the_exact_ones_rounded_once(m, algo):
     """silu(gate) * up over the whole range in which exp(-gate) is finite, formed in 32-bit: the stored bfloat16 is the rounding of
     a number within four units in the last place (exponential, sum, division and product) of the exact one."""
@@ -505,7 +505,7 @@ def test_few_rows_products_with_chosen_blocks(m, n, k):
 
 
 # tiles of the ring kernel (rows x columns) by the algorithm that asks for them
-RING = {TILE: (128, 128), TILE128X192: (128, 192), TILE256X96: (256, 128), TILE64X256: (64, 128), 10: (64, 64), 11: (128, 64), 12: (128, 256)}
+RING = {TILE: (128, 128), TILE128X192: (128, 192), TILE256X128: (256, 128), TILE64X128: (64, 128), 10: (64, 64), 11: (128, 64), 12: (128, 256)}
 
 
 @pytest.mark.parametrize("algo", sorted(RING))
