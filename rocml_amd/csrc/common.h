@@ -142,8 +142,8 @@ __device__ __forceinline__ float rows4_max(float v) {
 
 // and over all lanes, in the order of a butterfly of shuffles from 32 lanes apart to 1: turns by 8 and by 4 in a row bring the value
 // 8 and 4 lanes across, as all rows are alike by then and a row repeats itself after 8.  A sum of 64 values waits for six
-// vector operations instead of six trips through LDS, some 50 ns each (with the attention kernels' sums over rows: one request of 8 billion
-// weights at batch 1 63.66 -> 63.01 ms, twelve of kakalorn-2b 37.42 -> 37.05 ms).
+// vector operations instead of six trips through LDS, some 50 ns each (of a whole request at most 1 %, little more than two runs of one
+// side differ by).
 __device__ __forceinline__ float row16_sum_far(float v) {
     v += lane_dpp<0x128>(v);
     v += lane_dpp<0x124>(v);

@@ -230,9 +230,11 @@ template <int W>
 struct DcLds {
     u64 next[2];                                // the item after this one, in turn
     uint32_t end;                               // see DcTickets
-    // the waves' sums (two of them in turn: the other waves go on to the next item while the first finishes this one)
+    // The waves' sums, two of them in turn: behind an item's barrier its first waves (one for every four rows of its tiles, up to three)
+    // read them while the others go on to the next item, which has the other place.  A place is written again two items later,
+    // behind the barrier of the item between, which those waves reach when they have read.
     alignas(16) float red[2][DC_MAX_TILES][W][DC_MAX_ROWS][DC_TILE];
-    float scale[2][DC_MAX_ROWS];                // the rows' norm scales (in turn, as red)
+    float scale[2][DC_MAX_ROWS];                // the rows' norm scales, likewise
     alignas(16) float m[W][16], l[W][16];
     alignas(16) float o[W][DC_MAX_GROUP][DC_D + 4];
     alignas(16) float q[DC_MAX_GROUP][DC_D], k[DC_D], v[DC_D];      // (of the compute type)
@@ -263,7 +265,8 @@ __device__ __forceinline__ void dc_take(const DcArgs& a, uint32_t epoch, const u
 
 // SHORT: a wave's weights are all in its ring at once (separate code: one ring for both would be held twice).
 // One to three tiles of 16 weight rows times all rows of activations.  A wave has an equal share of K: it asks for its weights, takes
-// its share of the operands into LDS (nobody else reads it) and multiplies; the waves meet once, and the first one finishes.
+// its share of the operands into LDS (nobody else reads it) and multiplies; the waves meet once, and the first ceil(tiles * rows / 4) of
+// them finish, a row of lanes a tile of one row of activations.
 __device__ __forceinline__ int dc_tiles(const DcPlan& p, int stage) { return stage == DC_QKV ? p.qkv_tiles : stage == DC_GU ? p.gu_tiles : 1; }
 
 template <typename E, int W, int M, bool SHORT>
@@ -893,7 +896,9 @@ __global__ void __launch_bounds__(64 * W) decode_chain_kernel(const DcArgs a) {
     }
     __syncthreads();
     uint32_t end = sm.end;
-    asm volatile("" : "+v"(end));               // (a vector register: scalar ones are scarcer, 535 us a step against 530)
+    // (a vector register: scalar ones are scarcer.  1 % of a step of 530 us when it was measured, before stages and layers were in scalar
+    // registers too)
+    asm volatile("" : "+v"(end));
     const DcTickets tickets = {a.state, end};
     for (int turn = 0;; turn ^= 1) {
         const u64 drawn = sm.next[turn];

@@ -177,8 +177,9 @@ static bool rows_near(int ldx, int ldw, int size) { return (long long)(ldx > ldw
 #include "gemm_f32.h"
 
 // algo: ALGO_AUTO = choose, else the tile kernel asked for (then K stays whole).  The choice is the smallest estimate over shapes and
-// pieces.  What counts is the CU with the most work: 6144 columns are 24 tiles of 256, which with 2048 rows leave a quarter of
-// the chip idle, or 32 tiles of 192, which fill it.  A product with few tiles (few rows, or a narrow output)
+// pieces.  What counts is the CU with the most work and how fast a tile's stage goes: 34816 columns at 192 rows are 136 tiles of
+// 256, little more than half of the chip, or 182 of 192 (105 us for 120); 6144 columns at 2,048 rows are 192 tiles of 256 or 256 of 192, whose
+// stages on a full chip are slower by more (91 us for 95).  A product with few tiles (few rows, or a narrow output)
 // leaves most CUs idle while a few walk through all of K: then K is cut into pieces of at least 256 (512 where more than eight).
 struct TileChoice { int algo, pieces; };
 
