@@ -1257,12 +1257,16 @@ def decode_chain_max_layers() -> int:
 
 
 def decode_chain_splits(pages: int, pairs: int = 1) -> int:
-    """Splits of the key range in ``decode_chain`` for a block table of ``pages`` pages and ``pairs`` (token, kv head) pairs: a block asks
-    for two pages before it waits for anything, and a second turn costs less than a merge; with more than some 160 items the last ones start
-    when the first blocks are done with theirs (0.6B, one sequence of 5,000: 40 splits 822 us a step, 27 769, 20 703, 14 732; two of 1,000: 16 splits 674,
-    8 667, 6 663; four of 600 the same within 2 % from 2 to 6).  It depends on the step's shape only, so a recorded step can be
+    """Splits of the key range in ``decode_chain`` for a block table of ``pages`` pages and ``pairs`` (token, kv head) pairs: two pages a
+    split, which a block asks for before it waits for anything, as long as these items are at most one a CU (0.6B, steps in us by
+    fewer splits with more pages and by these: one sequence of 4,000 keys 726 -> 632, in 32 bits 1,101 -> 948, two of 2,000 710 -> 648, four of
+    1,000 792 -> 726).  Beyond that some 160 items, each of several turns: more start when the first blocks are done with theirs (one
+    sequence of 5,000: 40 splits 822, 27 769, 20 703, 14 732).  It depends on the step's shape only, so a recorded step can be
     replayed as the sequences grow."""
-    return 1 if pages <= 4 else max(1, min(64, (pages + 1) // 2, 160 // pairs))
+    if pages <= 4:
+        return 1
+    two_pages = min(64, (pages + 1) // 2)
+    return two_pages if two_pages * pairs <= 256 else max(1, min(two_pages, 160 // pairs))
 
 
 @functools.lru_cache(maxsize=256)
