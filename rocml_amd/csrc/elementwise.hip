@@ -215,8 +215,9 @@ ROCML_EXPORT int rocml_rmsnorm(float* x, const float* gain, void* out, int out_d
                (n_splits == 0 || ((uintptr_t)partials % 16 == 0 && split_stride % 4 == 0));
     int per = ceil_div(n, 4 * EW_BLOCK);     // vectors a thread
     // Up to 512 rows are on the chip at once also with 1024 threads each, and a thread then has one or two vectors
-    // to wait for: 64 rows of 4096 values with 8 splits 4.5 -> 3.8 us, 512 rows with 4 10.3 -> 9.0.
-    bool few = n_rows <= 512;
+    // to wait for: 64 rows of 4096 values with 8 splits 4.5 -> 3.8 us, 512 rows with 4 10.3 -> 9.0.  (Without splits up to 256: 512 rows
+    // of 4096 3.2 us with 256 threads, 3.5 with 1024.)
+    bool few = n_rows <= (n_splits > 0 ? 512 : 256);
 #define RN_ARGS rows, n_rows, n, eps, partials, n_splits, split_stride, stream
 #define RN_TYPE(TO_)                                                                              \
     {                                                                                             \
