@@ -8,7 +8,7 @@
 // order in which they depend on each other: it asks for its weights (or its pages) first, then waits for its operands, so that
 // the next stages' weights are in registers while this stage's results travel.  From a block's store to the waiting blocks that
 // read it some 1.5 us pass.  A step of the Qwen3-0.6B shape (28 layers, replayed, to the logits): one sequence of 40 tokens
-// 1,002 -> 474 us, of 500 1,011 -> 527, of 5,000 1,094 -> 703; two of 2,000 1,084 -> 761; four of 300 1,060 -> 697 (with how many keys it is
+// 869 -> 437 us, of 500 938 -> 485, of 5,000 1,024 -> 749; two of 2,000 1,003 -> 650; four of 300 976 -> 660 (with how many keys it is
 // slower: rocml_decode_chain_reach).  What is left of a layer (some 13 us) is five times a result's way to the next stage (1 to 1.5 us from its
 // store to the operands behind it), 0.6 to 1 us of products and 0.3 to 0.6 of an epilogue.
 //
@@ -992,7 +992,7 @@ static bool dc_plan(DcPlan& p, int dtype, int rows, int hidden, int hq, int hkv,
 // kernels have a piece of keys on its way while they multiply another, the chain, whose registers hold weights, has not.  Steps to
 // the logits, replayed, us:
 //   bfloat16, 0.6B (31 MB a layer), one row: 40 keys 1,002 -> 474, 5,000 1,094 -> 703, 20,000 1,350 -> 1,228, 40,000 (626 pages) 1,724 -> 1,781; two rows: 2,000
-//     1,084 -> 761, 8,000 1,323 -> 1,101, 16,000 (251 pages) 1,601 -> 1,531; three: 2,100 1,162 -> 871, 4,000 1,287 -> 1,051; four: 2,100 1,227 -> 967, 4,000
+//     1,003 -> 650, 8,000 1,323 -> 1,101, 16,000 (251 pages) 1,601 -> 1,531; three: 2,100 1,162 -> 871, 4,000 1,287 -> 1,051; four: 2,100 1,227 -> 967, 4,000
 //     1,362 -> 1,195, 8,000 (126 pages) 1,654 -> 1,674;
 //   1.7B (100 MB, 8 layers), one row: 500 523 -> 391, 32,000 701 -> 684; two: 4,200 562 -> 515, 8,000 604 -> 572; four: 500 551 -> 489, 4,000 628 -> 601;
 //   4B (202 MB, 6 layers): one row 608 -> 597, four 641 -> 711; 8B (386 MB, 6 layers): one 806 -> 802, two 818 -> 845: while weights stream, a word's way takes several us;
