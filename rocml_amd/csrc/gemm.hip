@@ -129,7 +129,7 @@ static int launch_pingpong(const void* x, int ldx, const void* w, int ldw, void*
 // sums leave (`sums`).
 struct TileKind { int bm, bn, cap; double light, full, alone, fixed, round, weights, sums; int algo; };
 static const TileKind TILE_KINDS[] = {
-    {256, 256, 1, 1.16, 1.28, 0.0, 7.50, 2.85, 7.00, 5.00, ALGO_MFMA_TILE256},     {256, 192, 1, 1.02, 1.35, 0.0, 6.00, 7.80, 8.50, 6.50, ALGO_MFMA_TILE256X192},
+    {256, 256, 1, 1.06, 1.38, 0.0, 7.00, 2.05, 7.95, 5.15, ALGO_MFMA_TILE256},     {256, 192, 1, 0.91, 1.28, 0.0, 6.40, 8.90, 7.80, 6.35, ALGO_MFMA_TILE256X192},
     {128, 128, 1, 0.459, 0.529, 0.0, 3.68, 2.15, 5.26, 4.38, ALGO_MFMA_TILE},      {64, 64, 2, 0.474, 0.452, 0.253, 2.60, 0.69, 5.50, 5.08, ALGO_MFMA_TILE64},
     {128, 64, 2, 0.682, 0.677, 0.385, 2.64, 0.77, 4.98, 4.78, ALGO_MFMA_TILE128X64}, {128, 192, 1, 0.617, 0.697, 0.0, 4.56, 3.11, 5.53, 4.91, ALGO_MFMA_TILE128X192},
     {256, 128, 1, 0.665, 0.812, 0.0, 5.64, 4.17, 4.98, 6.29, ALGO_MFMA_TILE256X128}, {128, 256, 1, 0.780, 0.834, 0.0, 4.94, 3.35, 5.70, 5.39, ALGO_MFMA_TILE128X256},
@@ -144,7 +144,7 @@ static const TileKind TILE_KINDS[] = {
 // left to the next kernel, whole, gated; weights from memory), those within twice the best.  The estimate is 5 to 9 % off (root mean
 // square), the choice by it 0.9 % behind the best on average, more than 5 % for 186 products and 28 % at worst.
 // Those of the two 256-row kinds were searched for afterwards by the choice's loss, over 77,803 times of 1,874 products (outputs up to
-// 151936, every kind, whole and in pieces; the first fit had 256x256 a fifth too slow).  Microseconds, by the first choice and by this
+// 151936, every kind, whole and in pieces) and 5,316 of layers' own products at 512 to 16,384 rows (the first fit had 256x256 a fifth too slow).  Microseconds, by the first choice and by this
 // one: gated 384 rows x 24576 x 4096 104 -> 90 (256x256 for 128x192), 512 x 32768 x 2048 76 -> 59, 160 x 151936 x 2560 254 -> 221; on
 // average 0.5 % behind the best of the gated products (1.0), 1.0 of the whole (1.3) and 1.1 of those left to the next kernel (1.5).
 static double tile_cost(const TileKind& kind, int pieces, int m, int n, int k, int epi, bool defer, int cus) {

@@ -23,7 +23,7 @@ template <int SET> struct RingSet { static constexpr int value = SET; };
 // Against the kernels it replaced (registers, double-buffered LDS; microseconds): 670 rows x 4096 x 1024 16.5 -> 12.2, gated 6144 x
 // 1024 19.6 -> 16.4, 1024 x 3072 13.7 in four pieces -> 10.6 in two; 64 rows x 4096 x 12288 29 in eight pieces -> 22.5 in four,
 // 6144 x 4096 16.7 -> 13.6; 512 rows x 6144 x 4096 40 -> 33.  Over 2,454 whole and gated products of 17 to 3,000 rows 0.81 of the time
-// (geometric mean; 65 to 256 gated rows 0.58), one in forty more than 3 % slower and six more than 10 %: wide outputs at 40 to 128 rows,
+// (geometric mean; 65 to 256 gated rows 0.58), one in thirty or so more than 3 % slower and six more than 10 %: wide outputs at 40 to 128 rows,
 // whose blocks were two a CU (128 x 151936 x 1024 90 -> 97, 43 x 32768 x 2048 29 -> 32).  32-bit: 0.92 of the time over 400.
 // Sums are formed in the order of gemm_mfma_kernel's (the same bits); in 32 bits in runs of 512 of K.
 template <int EPI, typename T, typename E = bf16_t>
