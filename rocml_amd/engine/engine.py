@@ -20,6 +20,7 @@ import torch
 from ..cache import Cache
 from ..errors import CacheFullError, ContextOverflowError, RocmlError, StepFailedError
 from .. import profile
+from ..staging import Staging
 from .batch import StepContext, StepEntry, pack_step
 from .model import DecoderModel
 from .workspace import Workspace
@@ -49,6 +50,7 @@ class Engine:
         self.max_graph_prompt_tokens = 1024     # prompt steps of at most so many tokens may be recorded
         self.max_prompt_graphs = 32
         self._graphs: Dict[tuple, tuple] = {}
+        self._staging = Staging()
 
     # -- sequences -----------------------------------------------------------------------
     def new_sequence(self) -> int:
@@ -185,9 +187,14 @@ class Engine:
         tables = [self.cache.block_table(g, slots, width) for g in self.cache.kv_groups]
         # One upload for all integer tables of the step.
         parts = [ids, seq, pos, cu, lens, slot_arr, want_rows] + [t.reshape(-1) for t in tables]
-        host = np.concatenate(parts) if parts else np.zeros(0, np.int32)
-        meta = self.workspace.get("step.meta", (max(host.size, 1),), torch.int32)
-        meta[:host.size].copy_(torch.from_numpy(host))
+        size = sum(p.size for p in parts)
+        meta = self.workspace.get("step.meta", (size,), torch.int32)
+        if torch.cuda.is_current_stream_capturing():
+            # (the recorded copy would bring whatever lies in the staging memory at a replay)
+            raise RocmlError("a step cannot be recorded from outside: its tables come from the host")
+        staged = self._staging.take(size)
+        np.concatenate(parts, out=staged.numpy())
+        self._staging.send(staged, meta)
         if device_ids is not None:
             meta[:ids.size].copy_(device_ids)           # the ids lead the table
         max_new = max(len(t) for t in tokens)
@@ -254,9 +261,10 @@ class Engine:
 
     def _remember(self, key, entry) -> None:
         """Keeps a shape's graph; of the prompt shapes only the ``max_prompt_graphs`` seen last."""
-        self._graphs.pop(key, None)
+        gone = [self._graphs.pop(key, None)]
         self._graphs[key] = entry                      # (a dict keeps insertion order: last seen last)
         if key[0] == "prompt":
             prompts = [k for k in self._graphs if k[0] == "prompt"]
-            for k in prompts[:max(0, len(prompts) - self.max_prompt_graphs)]:
-                del self._graphs[k]
+            gone += [self._graphs.pop(k) for k in prompts[:max(0, len(prompts) - self.max_prompt_graphs)]]
+        if any(e is not None and e[1] is not None and e[1] is not entry[1] for e in gone):
+            torch.cuda.synchronize(self.model.device)  # the graph may still be running: the host does not wait for steps

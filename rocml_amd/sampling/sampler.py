@@ -19,6 +19,7 @@ import numpy as np
 import torch
 
 from .. import ops
+from ..staging import Staging
 from .params import Rng, SamplingParams, sequence_seed
 
 
@@ -41,7 +42,7 @@ class DeviceSampler:
         self._argmax_work: Optional[torch.Tensor] = None
         # the parameters of a call travel in one pinned buffer and one copy (32-bit words, floats
         # and integers side by side), the drawn ids come back through another
-        self._stage: Optional[torch.Tensor] = None
+        self._staging = Staging()
         self._stage_dev: Optional[torch.Tensor] = None
         self._ids_host: Optional[torch.Tensor] = None
 
@@ -85,10 +86,10 @@ class DeviceSampler:
             self._work = torch.empty(logits.numel(), dtype=torch.float32, device=self.device)
         window = max([s.params.repeat_penalty_window for s in seqs if s.params.penalty_active()] + [1])
         words = batch * (6 + window)
-        if self._stage is None or self._stage.numel() < words:
-            self._stage = torch.empty(2 * words, dtype=torch.int32, pin_memory=True)
+        if self._stage_dev is None or self._stage_dev.numel() < words:
             self._stage_dev = torch.empty(2 * words, dtype=torch.int32, device=self.device)
-        stage = self._stage[:words].numpy()
+        staged = self._staging.take(words)
+        stage = staged.numpy()
         stage[:] = 0
         temperature, uniform, top_p, penalty = (stage[i * batch:(i + 1) * batch].view(np.float32) for i in range(4))
         top_k, hist_len = stage[4 * batch:5 * batch], stage[5 * batch:6 * batch]
@@ -111,7 +112,7 @@ class DeviceSampler:
         drawing = top_k[temperature > 0]
         small_k = int(drawing.max()) if drawing.size and drawing.min() >= 1 and drawing.max() <= ops.SAMPLE_SMALL_K else 0
         dev = self._stage_dev[:words]
-        dev.copy_(self._stage[:words], non_blocking=True)
+        self._staging.send(staged, dev)
         floats = dev[:4 * batch].view(torch.float32)
         ops.sample(logits, self._work, floats[:batch], floats[batch:2 * batch], out,
                    top_k=dev[4 * batch:5 * batch], top_p=floats[2 * batch:3 * batch],
