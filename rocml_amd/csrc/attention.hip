@@ -7,11 +7,12 @@
 #include "attention_generic.h"
 #include "attention_f32.h"
 #include "attention_mfma.h"
+#include "attention_prompt.h"
 #include "attention_latent.h"
 
 ROCML_LAST_ERROR_FN(attention)
 
-enum AttnAlgo : int { ATTN_AUTO = 0, ATTN_PLAIN = 1, ATTN_MFMA = 2 };
+enum AttnAlgo : int { ATTN_AUTO = 0, ATTN_PLAIN = 1, ATTN_MFMA = 2, ATTN_PROMPT = 3 };
 
 static const float LOG2E = 1.4426950408889634f;
 
@@ -31,6 +32,8 @@ struct AttnArgs {
     int n_splits_hint;
     const DecodeProj* proj;     // decode only: the step's q/k/v projection instead of q and an appended cache
     const PrefillProj* prefill_proj = nullptr;      // prompts: the projection instead of prepared queries
+    const int* q_counts = nullptr;                  // prompts: query tokens of each sequence (host memory)
+    int algo = ATTN_AUTO;
     MaskExtra extra = MaskExtra{};                  // blocks of positions, distance slopes, sink
     bool has_extra = false;
 };
@@ -113,7 +116,53 @@ template <int D> static int launch_decode_plain(const AttnArgs& a, hipStream_t s
 template <int D> static int launch_decode_fused(const AttnArgs& a, hipStream_t s) { return launch_decode<D, true>(a, s); }
 
 template <int D>
+static int launch_prompt(const AttnArgs& a, hipStream_t stream) {
+    using L = prompt::Lds<D>;
+    static bool ready = false;
+    if (!ready) {
+        if (allow_lds(attn_prompt_kernel<D, false>, L::BYTES)) return 1;
+        if (allow_lds(attn_prompt_kernel<D, true>, L::BYTES)) return 1;
+        ready = true;
+    }
+    long long tiles = 0;
+    for (int b = 0; b < a.n_seqs; ++b) tiles += ceil_div(a.q_counts[b], prompt::TILE);
+    dim3 grid((unsigned)(tiles * a.hq));
+    if (a.prefill_proj)
+        attn_prompt_kernel<D, true><<<grid, AM_THREADS, L::BYTES, stream>>>(
+            nullptr, a.out, a.kcache, a.vcache, a.block_table, a.bt_width, a.cu_seqlens, a.n_seqs, a.token_pos,
+            a.hq, a.hkv, a.scale * LOG2E, *a.prefill_proj);
+    else
+        attn_prompt_kernel<D, false><<<grid, AM_THREADS, L::BYTES, stream>>>(
+            a.q, a.out, a.kcache, a.vcache, a.block_table, a.bt_width, a.cu_seqlens, a.n_seqs, a.token_pos,
+            a.hq, a.hkv, a.scale * LOG2E, PrefillProj{});
+    return 0;
+}
+
+// What attn_prompt_kernel takes: heads of 128 whose rows see every key before them.
+static bool prompt_takes(const AttnArgs& a, int d) { return d == 128 && !a.has_extra && a.window == 0 && a.q_counts; }
+
+// Whether it is the faster way.  Its blocks have twice the rows of attn_prefill_mfma_kernel's and a CU holds one, so each pays for its
+// start and end (some 10 us) by itself and a page takes 1.6 to 1.75 us for 256 rows where the other takes 1.8 to 2.4: it wants blocks of
+// many pages, and enough of them to fill the chip.  Measured (32 query heads on 8, us, the other kernel first): prompts of 1,024 tokens,
+// one 31 and 39, four 70 and 74; of 1,536, one 47 and 52, four 119 and 123; of 2,048 (18 pages a block), one (a block a CU) 62 and 67, two
+// 103 and 92, four 183 and 178; of 3,000 (26 pages), one 128 and 92, on 16 heads (192 blocks) 115 and 81; of 8,192 750 and 549, behind
+// 24,576 others 4,038 and 3,108.  With a window of 2,048 4,096 tokens take 136 and 148, which is why windows stay with the other.
+// The positions before the step's first token are not known here: a step behind many others counts as if it were the first.
+static bool prompt_pays(const AttnArgs& a) {
+    long long tiles = 0, pages = 0;
+    for (int b = 0; b < a.n_seqs; ++b)
+        for (long long n = prompt::TILE; n < a.q_counts[b] + (long long)prompt::TILE; n += prompt::TILE) {
+            ++tiles;
+            pages += ceil_div(n < a.q_counts[b] ? n : a.q_counts[b], AM_PAGE);
+        }
+    const long long blocks = tiles * a.hq, cus = cu_count();
+    return pages >= 24 * tiles ? 4 * blocks >= 3 * cus : pages >= 17 * tiles && blocks >= 2 * cus;
+}
+
+template <int D>
 static int launch_prefill(const AttnArgs& a, hipStream_t stream) {
+    if constexpr (D == 128)
+        if (prompt_takes(a, D) && (a.algo == ATTN_PROMPT || (a.algo == ATTN_AUTO && prompt_pays(a)))) return launch_prompt<D>(a, stream);
     static bool ready = false;
     if (!ready) {
         if (allow_lds(attn_prefill_mfma_kernel<D, false>, PrefillLds<D>::BYTES)) return 1;
@@ -194,7 +243,8 @@ static bool mfma_head_dim(int d) { return d == 32 || d == 64 || d == 96 || d == 
      : (d) == 128 ? fn<128>(__VA_ARGS__)              \
      : (d) == 192 ? fn<192>(__VA_ARGS__) : fn<256>(__VA_ARGS__))
 
-// algo: 0 = choose, 1 = plain kernel, 2 = MFMA kernels (error if they cannot take the shapes).
+// algo: 0 = choose, 1 = plain kernel, 2 = MFMA kernels without the one for long prompts, 3 = that one (error if they cannot take the
+// shapes).
 // cu_seqlens [n_seqs + 1] gives where each sequence's query tokens start (tokens of a sequence
 // are consecutive and in position order) and q_counts, an array in host memory, how many each has
 // (the prefill kernel's grid is sized from it); max_new is the most query tokens of any
@@ -229,7 +279,7 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
     ROCML_REQUIRE(window >= 0, "attention: negative window %d", window);
     ROCML_REQUIRE(d <= AG_BLOCK * AG_MAX_D_PER_THREAD, "attention: head_dim %d exceeds %d", d,
                   AG_BLOCK * AG_MAX_D_PER_THREAD);
-    ROCML_REQUIRE(algo >= ATTN_AUTO && algo <= ATTN_MFMA, "attention: unknown algorithm %d", algo);
+    ROCML_REQUIRE(algo >= ATTN_AUTO && algo <= ATTN_PROMPT, "attention: unknown algorithm %d", algo);
     if (n_tokens == 0) return 0;
     bool decode = max_new == 1;
     long long total_q_tiles = 0, counted = 0;
@@ -248,6 +298,10 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
         ROCML_REQUIRE(mfma_ok, "attention: the MFMA kernels need bfloat16, pages of 64 positions, a head size "
                                "of 32, 64, 96, 128, 192 or 256, at most 16 query heads per kv head in decode and "
                                "the sequence offsets in prefill (D=%d page=%d group=%d)", d, page_size, hq / hkv);
+    if (algo == ATTN_PROMPT)
+        ROCML_REQUIRE(mfma_ok && !decode && !has_extra && window == 0 && d == 128 && q_counts,
+                      "attention: the kernel for long prompts needs bfloat16, pages of 64 positions, a head size of 128, more than one query "
+                      "token of a sequence, the sequence offsets and counts, and rows that see every key before them (D=%d page=%d)", d, page_size);
     // one shared key/value head whose values lie in its key rows: the kernel for latent rows
     bool latent_ok = v_in_k && !has_extra && dtype == ROCML_BF16 && page_size == AM_PAGE && hkv == 1 && d % 8 == 0 &&
                      dv % 8 == 0 && d <= 576 && dv <= 512 && max_new >= 1 && cu_seqlens && n_seqs > 0 && q_counts;
@@ -285,6 +339,8 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
                    scale, window, workspace, workspace_bytes, n_splits, nullptr};
         a.extra = MaskExtra{chunk, slopes, sink, sinks, softcap, keep_first};
         a.has_extra = has_extra;
+        a.q_counts = q_counts;
+        a.algo = algo;
         int rc = decode ? BY_HEAD_DIM(launch_decode_plain, d, a, stream) : BY_HEAD_DIM(launch_prefill, d, a, stream);
         if (rc) return rc;
         ROCML_CHECK_LAUNCH("attention");
@@ -442,6 +498,7 @@ ROCML_EXPORT int rocml_attention_prefill_fused(const float* qkv, int ld, const f
                nullptr, token_pos, cu_seqlens, n_seqs, n_tokens, (int)total_q_tiles, 0, hq, hkv, scale, window, nullptr,
                0, 0, nullptr};
     a.prefill_proj = &pj;
+    a.q_counts = q_counts;
     int rc = BY_HEAD_DIM(launch_prefill, d, a, stream);
     if (rc) return rc;
     ROCML_CHECK_LAUNCH("fused prefill attention");

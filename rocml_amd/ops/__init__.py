@@ -945,7 +945,7 @@ def splitk_reduce(partials: torch.Tensor, out: torch.Tensor, accumulate: bool = 
 
 
 # ---- attention -----------------------------------------------------------------------
-ATTN_AUTO, ATTN_PLAIN, ATTN_MFMA = 0, 1, 2
+ATTN_AUTO, ATTN_PLAIN, ATTN_MFMA, ATTN_PROMPT = 0, 1, 2, 3
 
 
 def attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
