@@ -39,10 +39,11 @@ struct AttnArgs {
 };
 
 template <int D, bool FUSED, int AHEAD, int WAVES>
-static int launch_decode_kernel(const AttnArgs& a, int n_splits, float* part_o, float* part_ml, hipStream_t stream) {
+static int launch_decode_kernel(const AttnArgs& a, int n_splits, AmShared shared, float* part_o, float* part_ml, hipStream_t stream) {
     int group = a.hq / a.hkv;
     int lds = WAVES * group * (D + 4) * (int)sizeof(float);
-    dim3 grid(n_splits, a.hkv, a.n_tokens);
+    // blocks shared out by the tokens' lengths: n_splits is the room for the splits of one
+    dim3 grid(shared.n_tokens > 0 ? shared.slots : n_splits, a.hkv, shared.n_tokens > 0 ? 1 : a.n_tokens);
     if (a.has_extra) {
         static int allowed_extra = 0;
         if (lds > allowed_extra) {
@@ -51,7 +52,7 @@ static int launch_decode_kernel(const AttnArgs& a, int n_splits, float* part_o, 
         }
         attn_decode_mfma_kernel<D, FUSED, AHEAD, WAVES, true><<<grid, 64 * WAVES, lds, stream>>>(
             a.q, a.out, const_cast<bf16_t*>(a.kcache), const_cast<bf16_t*>(a.vcache), a.block_table, a.bt_width,
-            a.token_seq, a.token_pos, a.hq, a.hkv, a.scale * LOG2E, a.window, n_splits, part_o, part_ml,
+            a.token_seq, a.token_pos, a.hq, a.hkv, a.scale * LOG2E, a.window, n_splits, shared, part_o, part_ml,
             FUSED ? *a.proj : DecodeProj{}, a.extra);
         return 0;
     }
@@ -62,12 +63,29 @@ static int launch_decode_kernel(const AttnArgs& a, int n_splits, float* part_o, 
     }
     attn_decode_mfma_kernel<D, FUSED, AHEAD, WAVES><<<grid, 64 * WAVES, lds, stream>>>(
         a.q, a.out, const_cast<bf16_t*>(a.kcache), const_cast<bf16_t*>(a.vcache), a.block_table, a.bt_width,
-        a.token_seq, a.token_pos, a.hq, a.hkv, a.scale * LOG2E, a.window, n_splits, part_o, part_ml,
+        a.token_seq, a.token_pos, a.hq, a.hkv, a.scale * LOG2E, a.window, n_splits, shared, part_o, part_ml,
         FUSED ? *a.proj : DecodeProj{});
     return 0;
 }
 
 constexpr int WIDE_BLOCK_MIN_PIECES = 8;         // of a block: more than two a wave of four
+
+// Blocks a kv head that the tokens of a step share by their lengths, or 0: as many for every token.  By the launch's shape only, as a
+// recorded step is replayed while its sequences grow: batches of unequal lengths gain, those of one length pay for the working out
+// and for a merge (figures, even splits and shared ones, us with the merge, 32 heads on 8).
+// Up to half a block a CU without splits, a block of eight waves a CU: 6 sequences of 200 to 4,000 keys 21.0 and 17.4, 16 of them
+// 41.2 and 29.8, 16 of 100 to 1,000 17.0 and 15.6; of one length 6 of 2,070 18.6 and 19.0, 16 34.1 and 34.4.  Up to a
+// block for every eight CUs it does not pay: 3 of 2,070 13.2 and 13.9, 4 of 100 to 1,000 11.0 and 11.5.
+// Beyond, two blocks of four waves a CU (or what even splits are), where the block table has room for more than 1,024 keys: 24 of 200 to
+// 4,000 69.7 and 44.4, 32 75 and 57.7, 40 78.2 and 69.9, 56 133 and 120; of one length 24 of 2,070 48.3 and 52.6, 56 101.6 and 104.8; below, 32 of
+// 100 to 1,000 24.7 and 24.4, but 32 of 600 21.3 and 26.0.
+static int shared_slots(const AttnArgs& a, int n_splits) {
+    const long long pairs = (long long)a.n_tokens * a.hkv, cus = cu_count();
+    if (a.n_tokens > 64 || a.window > 0 || a.extra.chunk > 0 || 8 * pairs <= cus) return 0;
+    if (2 * pairs <= cus) return (int)(cus / a.hkv);
+    const long long slots = n_splits > 1 ? (long long)n_splits * a.n_tokens : 2 * cus / a.hkv;
+    return a.bt_width >= 32 && 8ll * a.n_tokens <= 7 * slots ? (int)slots : 0;
+}
 
 template <int D, bool FUSED>
 static int launch_decode(const AttnArgs& a, hipStream_t stream) {
@@ -84,6 +102,17 @@ static int launch_decode(const AttnArgs& a, hipStream_t stream) {
     if (n_splits > 1 && per_split * n_splits > a.workspace_bytes)
         n_splits = a.workspace ? (int)(a.workspace_bytes / per_split) : 1;
     if (n_splits < 1) n_splits = 1;
+    AmShared shared = {0, 0, 0};
+    if (const int slots = D <= 128 ? shared_slots(a, n_splits) : 0; slots > 0) {
+        // a token has at most so many splits: one for each of its pages, 64, what the other tokens leave, what the workspace holds
+        long long room = min(min(slots - a.n_tokens + 1, a.bt_width), 64);
+        if (room * per_split > a.workspace_bytes) room = a.workspace ? a.workspace_bytes / per_split : 0;
+        if (room >= 2) {
+            // (24 of 2,070 keys in blocks for one split each, the others empty: 78.9 us instead of 53.5, as the full ones meet on some CUs)
+            shared = {a.n_tokens, slots, min(slots / a.n_tokens, (int)room)};
+            n_splits = (int)room;
+        }
+    }
     float* part_o = (float*)a.workspace;
     float* part_ml = part_o ? part_o + (size_t)a.n_tokens * a.hq * n_splits * D : nullptr;
     // Many splits mean few pieces per block: then two of a wave's pieces travel at a time; so they
@@ -95,15 +124,17 @@ static int launch_decode(const AttnArgs& a, hipStream_t stream) {
     // two pieces each, over the splits and the waves: the launch's shape again, not the lengths).
     int rc;
     if constexpr (D <= 128) {
-        bool one_a_cu = (long long)a.n_tokens * a.hkv * n_splits <= cu_count();
+        const bool sharing = shared.n_tokens > 0;
+        bool one_a_cu = (sharing ? (long long)shared.slots * a.hkv : (long long)a.n_tokens * a.hkv * n_splits) <= cu_count();
         long long pieces = 2ll * ((a.bt_width + n_splits - 1) / n_splits);
-        if (one_a_cu && pieces > WIDE_BLOCK_MIN_PIECES)
-            rc = launch_decode_kernel<D, FUSED, 2, 8>(a, n_splits, part_o, part_ml, stream);
+        // (shared blocks of eight waves in any case: 8 sequences of 600 12.5 us with eight, 13.3 with four)
+        if (one_a_cu && (sharing || pieces > WIDE_BLOCK_MIN_PIECES))
+            rc = launch_decode_kernel<D, FUSED, 2, 8>(a, n_splits, shared, part_o, part_ml, stream);
         else
-            rc = n_splits >= 4 || one_a_cu ? launch_decode_kernel<D, FUSED, 2, 4>(a, n_splits, part_o, part_ml, stream)
-                                           : launch_decode_kernel<D, FUSED, 1, 4>(a, n_splits, part_o, part_ml, stream);
+            rc = (n_splits >= 4 && !sharing) || one_a_cu ? launch_decode_kernel<D, FUSED, 2, 4>(a, n_splits, shared, part_o, part_ml, stream)
+                                                                             : launch_decode_kernel<D, FUSED, 1, 4>(a, n_splits, shared, part_o, part_ml, stream);
     } else {
-        rc = launch_decode_kernel<D, FUSED, 1, 4>(a, n_splits, part_o, part_ml, stream);
+        rc = launch_decode_kernel<D, FUSED, 1, 4>(a, n_splits, shared, part_o, part_ml, stream);
     }
     if (rc) return rc;
     if (n_splits > 1)

@@ -61,6 +61,12 @@ struct DecodeProj {
 // grid (n_splits, Hkv, tokens), 4 or 8 waves; the block's pages are cut into 32-key pieces that the
 // waves take in turn; all query heads of the kv head ride in the 16 columns of the MFMA.
 //
+// shared.n_tokens > 0: grid (slots, Hkv), the blocks shared out among the step's tokens by their lengths (am_share; no window, no blocks
+// of positions), n_splits the room for a row's partial results.  With as many splits for every token the longest sequence of an
+// unequal batch was the whole kernel's time.  Us with the merge, 32 heads on 8 but the first, even splits and shared ones:
+// 16 of 128 to 4,096 keys on 40 heads 41.4 and 26.7 (their bytes: 16.6), 8 of 200 to 4,000 24.0 and 18.7, 24 of them 69.7 and 44.4; what
+// it costs where all are of one length: 8 of 2,070 20.9 and 21.5, 16 of 600 16.5 and 17.0.
+//
 // FUSED: the kernel takes the projection's output instead of q and a finished cache: every block
 // norms and rotates the q heads of its kv head itself and lays them out as the MFMA operand; the
 // block whose split holds the sequence's last page also norms and rotates the new key, writes it
@@ -86,13 +92,51 @@ __device__ __forceinline__ float am_tanh(float x) {
     return 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
 }
 
+// Which of `slots` blocks (of a kv head) takes which split of which token, when the splits go by the tokens' lengths: about the
+// fewest pages a split for which the splits of all tokens (at most `room` each) fit the blocks.  Every wave works it out for itself,
+// lane t for token t (n_tokens <= 64 and <= slots); blocks beyond the last split get t = -1.  Any count of splits is right, so the
+// divisions are approximate: they only have to come out alike in every wave.
+// Tokens of as many pages each keep the guess they come with (8 of 2,070 keys 22.1 us without this way out, 21.5 with it).
+struct AmShare { int t, split, n_splits; };
+__device__ __forceinline__ AmShare am_share(const int* token_pos, int n_tokens, int slots, int room, int slot, AmShare guess) {
+    const int lane = threadIdx.x & 63;
+    const bool has = lane < n_tokens;
+    const int n_pages = max(1, token_pos[has ? lane : 0] / AM_PAGE + 1);
+    if (__ballot(n_pages != __builtin_amdgcn_readfirstlane(n_pages)) == 0) {
+        if (slot >= n_tokens * guess.n_splits) guess.t = -1;
+        return guess;
+    }
+    const float pages = has ? (float)n_pages : 0.f;
+    float mine, each = fmaxf(wave_sum(pages) * __builtin_amdgcn_rcpf((float)slots), 1.f);
+    for (int tries = 0; tries < 64; ++tries, each *= 1.125f) {
+        // (a little less, so that a whole quotient stays what it is)
+        mine = has ? fminf(fmaxf(ceilf(pages * __builtin_amdgcn_rcpf(each) - 0.001f), 1.f), (float)room) : 0.f;
+        if (wave_sum(mine) <= (float)slots) break;
+        mine = has ? 1.f : 0.f;
+    }
+    // the splits up to and with this lane's token
+    int upto = (int)mine;
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xF, 0xF, false);        // from 1, 2, 4 and 8 lanes to the left in a row of 16,
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xF, 0xF, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xF, 0xF, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xF, 0xF, false);
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xA, 0xF, false);        // from the last lane of the row before, of the lower half
+    upto += __builtin_amdgcn_update_dpp(0, upto, 0x143, 0xC, 0xF, false);
+    const int t = __popcll(__ballot(upto <= slot));         // tokens whose splits all lie before this block
+    if (t >= n_tokens) return {-1, 0, 0};
+    const int n = __builtin_amdgcn_readlane((int)mine, t);
+    return {t, slot - (__builtin_amdgcn_readlane(upto, t) - n), n};
+}
+
+struct AmShared { int n_tokens, slots, even; };          // even: splits of a token of an equal batch; n_tokens 0: not shared
+
 template <int D, bool FUSED, int AHEAD, int WAVES, bool EXTRA = false>
 __global__ void __launch_bounds__(64 * WAVES)
 attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
                         bf16_t* kcache, bf16_t* vcache,
                         const int* __restrict__ block_table, int bt_width,
                         const int* __restrict__ token_seq, const int* __restrict__ token_pos, int hq,
-                        int hkv, float scale_log2e, int window, int n_splits,
+                        int hkv, float scale_log2e, int window, int n_splits, AmShared shared,
                         float* __restrict__ part_o, float* __restrict__ part_ml, DecodeProj pj,
                         MaskExtra mx = MaskExtra{}) {
     constexpr int KD = D / 32;      // MFMA steps along D for the scores
@@ -104,6 +148,12 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int g = lane >> 4, col = lane & 15;
     int group = hq / hkv;
+    const int room = n_splits;                      // for a row's partial results
+    if (shared.n_tokens > 0) {                      // (a guess that holds for tokens of one length)
+        n_splits = shared.even;
+        t = min((int)blockIdx.x / n_splits, shared.n_tokens - 1);
+        split = blockIdx.x - t * n_splits;
+    }
     // (token_seq null: token t is the one token of the step's sequence t)
     const int* pages = block_table + (size_t)(token_seq ? token_seq[t] : t) * bt_width;
     // Without a window a split's pages are split, split + n_splits, ... whatever the length: the
@@ -111,9 +161,19 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     int early[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) early[i] = pages[split + i * n_splits < bt_width ? split + i * n_splits : 0];
+    bool looked_up = true;
+    if (shared.n_tokens > 0) {
+        const AmShare share = am_share(token_pos, shared.n_tokens, shared.slots, room, blockIdx.x, {t, split, n_splits});
+        if (share.t < 0) return;
+        looked_up = share.t == t && share.split == split && share.n_splits == n_splits;
+        t = share.t;
+        split = share.split;
+        n_splits = share.n_splits;
+        pages = block_table + (size_t)(token_seq ? token_seq[t] : t) * bt_width;
+    }
     int len = token_pos[t] + 1;
     int lo = window > 0 ? max(0, len - window) : 0;
-    bool from_start = window == 0;                  // the sequence's first pages are the split's first pages
+    bool from_start = looked_up && window == 0;     // the sequence's first pages are the split's first pages
     float slope_l2 = 0.f;
     if constexpr (EXTRA) {
         if (mx.chunk > 0) {
@@ -447,10 +507,10 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
             acc += sm_o[((size_t)w * group + head) * (D + 4) + d] * wgt;
         }
         int h = kvh * group + head;
-        if (n_splits == 1) {
+        if (room == 1) {
             out[((size_t)t * hq + h) * D + d] = f32_to_bf16(acc / ll);
         } else {
-            size_t slot = ((size_t)t * hq + h) * n_splits + split;
+            size_t slot = ((size_t)t * hq + h) * room + split;
             part_o[slot * D + d] = acc;
             if (d == 0) {
                 part_ml[slot * 2] = mm;
@@ -458,9 +518,18 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
             }
         }
     }
+    const int absent = room - n_splits;
+    if (split == 0 && absent > 0)                   // the merge knows by these how many splits a row has
+        for (int idx = tid; idx < group * absent; idx += THREADS) {
+            const int head = idx / absent;
+            const size_t slot = ((size_t)t * hq + kvh * group + head) * room + n_splits + (idx - head * absent);
+            part_ml[slot * 2] = -INFINITY;
+            part_ml[slot * 2 + 1] = 0.f;
+        }
 }
 
-// Log-sum-exp merge of the splits in split order (rocml-kernels/kernels/attn_decode.hip:219-255).
+// Log-sum-exp merge of the splits in split order (rocml-kernels/kernels/attn_decode.hip:219-255).  n_splits: the room a row has for
+// them; a maximum of -inf with a sum of 0 marks those it does not have, whose partial outputs may be anything.
 template <int D>
 __global__ void attn_decode_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                           bf16_t* __restrict__ out, int n_splits) {
@@ -480,6 +549,8 @@ __global__ void attn_decode_reduce_kernel(const float* __restrict__ part_o, cons
     float first[8];
 #pragma unroll
     for (int s = 0; s < 8; ++s) first[s] = po[(size_t)min(s, n_splits - 1) * D + d];
+    const int room = n_splits;
+    n_splits = 64 - __builtin_clzll(__ballot(!(ms == -INFINITY && ls == 0.f)) | 1ull);
     float mm = wave_max(ms);
     float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mm);
     if (threadIdx.x < 64) wgt[lane] = w;
@@ -489,7 +560,7 @@ __global__ void attn_decode_reduce_kernel(const float* __restrict__ part_o, cons
     // finite values: no branches)
     float acc = 0.f;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) acc += first[s] * wgt[s];
+    for (int s = 0; s < 8; ++s) acc += (s < n_splits || n_splits == room ? first[s] : 0.f) * wgt[s];
     for (int s0 = 8; s0 < n_splits; s0 += 8) {
         float more[8];
 #pragma unroll

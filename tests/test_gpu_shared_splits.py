@@ -1,0 +1,70 @@
+"""Decode attention of batches whose blocks are shared out by the sequences' lengths: against plain softmax attention, at the edges of the
+rule that chooses it, with lengths that need most of the blocks for one sequence, and in a recorded launch whose sequences grow."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from rocml_amd import ops  # noqa: E402
+from tests.test_gpu_attention import MFMA, PAGE, _build, _check, _fused_case, _reference  # noqa: E402
+
+# (Hq, Hkv, D, lengths): on 256 CUs 8 kv heads share from 5 sequences on; 17 and more where the table has room for 32 pages
+SHARED = [(16, 8, 128, [1, 64, 65, 300, 2100]), (16, 8, 64, [1, 1, 1, 1, 1, 4000]), (8, 8, 128, [130] * 7), (32, 8, 128, [63, 64, 65, 127, 128, 129] * 2),
+          (40, 8, 128, [700, 1, 2, 3, 64, 128, 192, 256, 320, 1500, 30, 31, 32, 33, 34, 35]), (16, 2, 128, list(range(50, 1700, 50))),
+          (6, 3, 96, [5, 900, 17, 64, 200, 1, 33, 450, 128, 70, 1100, 12]), (4, 1, 32, [1 + 37 * i for i in range(40)]),
+          (8, 8, 128, [1 + 13 * i for i in range(23)] + [2049]), (8, 8, 128, [2000 + i for i in range(17)]), (8, 4, 64, [40 * i + 1 for i in range(63)] + [2050])]
+
+
+@pytest.mark.parametrize("hq,hkv,d,lengths", SHARED)
+def test_unequal_lengths(hq, hkv, d, lengths):
+    _check([(n, 1) for n in lengths], hq, hkv, d, torch.bfloat16, MFMA, n_splits=ops.decode_splits(len(lengths) * hkv, 256, 64), seed=5)
+    if d != 96 and d != 32:
+        _fused_case([(n, 1) for n in lengths], hq, hkv, d, 2, ops.decode_splits(len(lengths) * hkv, 256, 64), None, seed=7)
+
+
+@pytest.mark.parametrize("room", [1, 2, 5])
+def test_little_workspace(room):
+    """A workspace that holds so many splits of every token: no more are made, with one none."""
+    lengths, hq, hkv, d = [10, 2500, 64, 300, 1, 129, 600], 16, 8, 128
+    dev, ks, vs, qs = _build([(n, 1) for n in lengths], hq, hkv, d, torch.bfloat16, 3)
+    size = len(lengths) * hq * (d + 2) * 4 * room
+    ws = torch.full((size + 4096,), 0x7f, dtype=torch.uint8, device="cuda")
+    out = torch.full_like(dev["q"], float("nan"))
+    ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, d ** -0.5, None, algo=MFMA,
+                  workspace=ws[:size], cu_seqlens=dev["cu"], max_new=1, q_counts=[1] * len(lengths), max_len=max(lengths), n_splits=0)
+    assert bool((ws[size:] == 0x7f).all())
+    for b, n in enumerate(lengths):
+        want = _reference(qs[b], ks[b], vs[b], [n - 1], d ** -0.5, None)
+        assert float((out[b].cpu().double().view(1, hq, d) - want).abs().max()) < 1.5e-2
+
+
+def test_recorded_while_lengths_change():
+    """A recorded launch follows the positions it finds at each replay."""
+    lengths, hq, hkv, d = [1000, 64, 700, 65, 1400, 300, 2], 16, 8, 128
+    dev, ks, vs, qs = _build([(n, 1) for n in lengths], hq, hkv, d, torch.bfloat16, 9)
+    ws = torch.empty(16 << 20, dtype=torch.uint8, device="cuda")
+    out = torch.empty_like(dev["q"])
+
+    def step():
+        ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, d ** -0.5, None, algo=MFMA,
+                      workspace=ws, cu_seqlens=dev["cu"], max_new=1, q_counts=[1] * len(lengths), max_len=max(lengths), n_splits=5)
+    step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step()
+    for sub in (0, 1, 63, 900):
+        now = [max(1, n - sub) if n != 1400 else n for n in lengths]
+        dev["tok_pos"].copy_(torch.tensor(now, dtype=torch.int32) - 1)
+        ws.fill_(0xff)                              # what is left from before is NaN
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = out.clone()
+        step()
+        torch.cuda.synchronize()
+        assert torch.equal(out, replayed)
+        for b, n in enumerate(now):
+            want = _reference(qs[b], ks[b][:n], vs[b][:n], [n - 1], 1.0 / math.sqrt(d), None)
+            assert float((replayed[b].cpu().double().view(1, hq, d) - want).abs().max()) < 1.5e-2, (sub, n, PAGE)
