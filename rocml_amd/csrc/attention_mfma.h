@@ -92,6 +92,17 @@ __device__ __forceinline__ float am_tanh(float x) {
     return 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
 }
 
+// The sum of the lanes' numbers up to and with each lane's own.
+__device__ __forceinline__ int am_sums_upto(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);        // from 1, 2, 4 and 8 lanes to the left in a row of 16,
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);        // from the last lane of the row before, of the lower half
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
 // Which of `slots` blocks (of a kv head) takes which split of which token, when the splits go by the tokens' lengths: about the
 // fewest pages a split for which the splits of all tokens (at most `room` each) fit the blocks.  Every wave works it out for itself,
 // lane t for token t (n_tokens <= 64 and <= slots); blocks beyond the last split get t = -1.  Any count of splits is right, so the
@@ -114,14 +125,7 @@ __device__ __forceinline__ AmShare am_share(const int* token_pos, int n_tokens, 
         if (wave_sum(mine) <= (float)slots) break;
         mine = has ? 1.f : 0.f;
     }
-    // the splits up to and with this lane's token
-    int upto = (int)mine;
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x111, 0xF, 0xF, false);        // from 1, 2, 4 and 8 lanes to the left in a row of 16,
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x112, 0xF, 0xF, false);
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x114, 0xF, 0xF, false);
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x118, 0xF, 0xF, false);
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x142, 0xA, 0xF, false);        // from the last lane of the row before, of the lower half
-    upto += __builtin_amdgcn_update_dpp(0, upto, 0x143, 0xC, 0xF, false);
+    const int upto = am_sums_upto((int)mine);
     const int t = __popcll(__ballot(upto <= slot));         // tokens whose splits all lie before this block
     if (t >= n_tokens) return {-1, 0, 0};
     const int n = __builtin_amdgcn_readlane((int)mine, t);
@@ -667,6 +671,35 @@ __device__ __forceinline__ int am_first_key(int pos, int window, int chunk) {
     return window > 0 ? max(0, pos - window + 1) : 0;
 }
 
+// Tile `tile` of ROWS query rows over all sequences: its sequence, where that one's tokens start and how many they are, and the tile in
+// it; b is -1 beyond the last.  Beyond 16 sequences 64 at a time, one a lane: walked one by one, with a look at cu_seqlens each,
+// the last of 64 was some 3 us away (64 prompts of 40 tokens, 32 heads: 46.2 and 38.9 us); of 16 the walk is the nearer way (27.7 and 29.1).
+struct AmTile { int b, tok0, n_new, tile; };
+template <int ROWS>
+__device__ __forceinline__ AmTile am_find_tile(const int* cu_seqlens, int n_seqs, int tile) {
+    if (n_seqs <= 16) {
+        for (int b = 0; b < n_seqs; ++b) {
+            const int tok0 = cu_seqlens[b], n_new = cu_seqlens[b + 1] - tok0, tiles = (n_new + ROWS - 1) / ROWS;
+            if (tile < tiles) return {b, tok0, n_new, tile};
+            tile -= tiles;
+        }
+        return {-1, 0, 0, 0};
+    }
+    const int lane = threadIdx.x & 63;
+    for (int base = 0; base < n_seqs; base += 64) {
+        const int b = min(base + lane, n_seqs - 1), lo = cu_seqlens[b], n_new = cu_seqlens[b + 1] - lo;
+        const int tiles = base + lane < n_seqs ? (n_new + ROWS - 1) / ROWS : 0, upto = am_sums_upto(tiles);
+        const int all = __builtin_amdgcn_readlane(upto, 63);
+        if (tile < all) {
+            const int k = __popcll(__ballot(upto <= tile));
+            return {base + k, __builtin_amdgcn_readlane(lo, k), __builtin_amdgcn_readlane(n_new, k),
+                    tile - (__builtin_amdgcn_readlane(upto, k) - __builtin_amdgcn_readlane(tiles, k))};
+        }
+        tile -= all;
+    }
+    return {-1, 0, 0, 0};
+}
+
 template <int D, bool QPREP, bool EXTRA = false>
 __global__ void __launch_bounds__(AM_THREADS, D <= 128 ? 2 : 1)
 attn_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
@@ -675,6 +708,10 @@ attn_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
                          const int* __restrict__ cu_seqlens, int n_seqs,
                          const int* __restrict__ token_pos, int hq, int hkv, float scale_log2e,
                          int window, PrefillProj pj, MaskExtra mx = MaskExtra{}) {
+    // Pages on their way in registers while one is multiplied.  Two: what a lone block on a CU waits for beside its products (32 heads
+    // of 128, us with one and with two: a prompt of 700 31.4 and 29.5, of 1,500 64.3 and 58.7, 64 of 16 to 700 185 and 169, full rounds of
+    // blocks equal).  Heads of 64 and 96 gain as much alone and lose 2 % with all CUs full, 192 loses 4 to 8, 256 has no registers for it.
+    constexpr int AHEAD = D == 128 ? 2 : 1;
     static_assert(!(QPREP && EXTRA), "the kernel that prepares its queries knows plain layers only");
     using L = PrefillLds<D>;
     const int chunk = EXTRA ? mx.chunk : 0;
@@ -696,15 +733,9 @@ attn_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     int round_size = min(AM_ROUND, n_blocks - round0);
     int s = round0 + (((blockIdx.x / AM_ROUND) & 1) ? round_size - 1 - in_round : in_round);
     int h = s % hq, kvh = h / (hq / hkv);
-    int tile = total_tiles - 1 - s / hq, b = 0, tok0 = 0, n_new = 0;
-    for (; b < n_seqs; ++b) {
-        tok0 = cu_seqlens[b];
-        n_new = cu_seqlens[b + 1] - tok0;
-        int tiles = (n_new + AM_QTILE - 1) / AM_QTILE;
-        if (tile < tiles) break;
-        tile -= tiles;
-    }
-    if (b >= n_seqs) return;
+    const AmTile at = am_find_tile<AM_QTILE>(cu_seqlens, n_seqs, total_tiles - 1 - s / hq);
+    if (at.b < 0) return;
+    const int tile = at.tile, b = at.b, tok0 = at.tok0, n_new = at.n_new;
     const int* pages = block_table + (size_t)b * bt_width;
     int pos0 = token_pos[tok0];                        // position of the sequence's first new token
     int row_lo = tile * AM_QTILE, row_hi = min(n_new, row_lo + AM_QTILE) - 1;     // block's query rows
@@ -750,32 +781,34 @@ attn_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
 
-    // A page's keys and values wait in registers while the page before it is multiplied out of
-    // LDS: the loads of page p + 1 are issued right after page p has been written to LDS.
+    // A page's keys and values wait in registers while the AHEAD pages before it are multiplied out of
+    // LDS: the loads of page p + AHEAD are issued right after page p has been written to LDS.
     typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
     constexpr int K_PIECES = AM_PAGE * D / 8 / AM_THREADS, V_PIECES = D * AM_PAGE / 8 / AM_THREADS;
-    u32x4 kreg[K_PIECES], vreg[V_PIECES];
+    u32x4 kreg[AHEAD][K_PIECES], vreg[AHEAD][V_PIECES];
     int first_page = blk_first_key / AM_PAGE, last_page = blk_last_key / AM_PAGE;
     // kept first positions: their pages before the window's come first, then the window's
     const int keep = EXTRA ? mx.keep_first : 0;
     const int kept_pages = EXTRA ? min(first_page, (keep + AM_PAGE - 1) / AM_PAGE) : 0;
     auto logical_page = [&](int i) { return EXTRA && i < kept_pages ? i : first_page + i - kept_pages; };
     const int n_visits = last_page - first_page + 1 + kept_pages;
-#define AM_LOAD_PAGE(lp_)                                                                         \
-    {                                                                                             \
-        int phys_ = pages[lp_];                                                                   \
-        const u32x4* gk_ = (const u32x4*)(kcache + ((size_t)phys_ * hkv + kvh) * AM_PAGE * D);    \
-        const u32x4* gv_ = (const u32x4*)(vcache + ((size_t)phys_ * hkv + kvh) * D * AM_PAGE);    \
-        _Pragma("unroll") for (int i = 0; i < K_PIECES; ++i) kreg[i] = gk_[tid + i * AM_THREADS]; \
-        _Pragma("unroll") for (int i = 0; i < V_PIECES; ++i) vreg[i] = gv_[tid + i * AM_THREADS]; \
-    }
+    auto load_page = [&](int lp, u32x4 (&kr)[K_PIECES], u32x4 (&vr)[V_PIECES]) {
+        const int phys = pages[lp];
+        const u32x4* gk = (const u32x4*)(kcache + ((size_t)phys * hkv + kvh) * AM_PAGE * D);
+        const u32x4* gv = (const u32x4*)(vcache + ((size_t)phys * hkv + kvh) * D * AM_PAGE);
+#pragma unroll
+        for (int i = 0; i < K_PIECES; ++i) kr[i] = gk[tid + i * AM_THREADS];
+#pragma unroll
+        for (int i = 0; i < V_PIECES; ++i) vr[i] = gv[tid + i * AM_THREADS];
+    };
     // the wave's rows see every key of a 32-key piece when the piece lies at or below the first
     // row's position and at or above the last row's window start; only then masking is skipped
     int wave_min_pos = pos0 + w_lo;
     int wave_max_lo = am_first_key(pos0 + w_hi, window, chunk);
     bool wave_full = w_hi - w_lo == 31;
-    AM_LOAD_PAGE(logical_page(0))
-    for (int visit = 0; visit < n_visits; ++visit) {
+    load_page(logical_page(0), kreg[0], vreg[0]);
+    if (AHEAD == 2 && n_visits > 1) load_page(logical_page(1), kreg[AHEAD - 1], vreg[AHEAD - 1]);
+    auto visit_page = [&](int visit, u32x4 (&kreg)[K_PIECES], u32x4 (&vreg)[V_PIECES]) {
         const int lpage = logical_page(visit);
         __syncthreads();                                // the previous page has been consumed
 #pragma unroll
@@ -796,8 +829,8 @@ attn_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
             dst[2] = make_uint2(vreg[i][2], vreg[i][3]);
         }
         __syncthreads();
-        if (visit + 1 < n_visits) AM_LOAD_PAGE(logical_page(visit + 1))
-        if (!wave_active) continue;
+        if (visit + AHEAD < n_visits) load_page(logical_page(visit + AHEAD), kreg, vreg);
+        if (!wave_active) return;
         // The scores of both 32-key halves are started before either is finished: the softmax of
         // the first half (vector ALU) then runs while the matrix core still multiplies the second,
         // and the softmax of the second while the first half's values are multiplied.
@@ -894,8 +927,11 @@ attn_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
                 }
             }
         }
+    };
+    for (int visit = 0; visit < n_visits; visit += AHEAD) {
+        visit_page(visit, kreg[0], vreg[0]);
+        if (AHEAD == 2 && visit + 1 < n_visits) visit_page(visit + 1, kreg[AHEAD - 1], vreg[AHEAD - 1]);
     }
-#undef AM_LOAD_PAGE
     if (!row_ok) return;
     float inv = 1.0f / l;
     bf16_t* orow = out + ((size_t)(tok0 + my_row) * hq + h) * D;

@@ -80,15 +80,9 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     // Heavy tiles first.  Blocks go to the dies in turn: a die gets neighbouring heads, which share their keys.
     const int total_tiles = gridDim.x / hq, in_tile = blockIdx.x % hq;
     const int h = hq % 8 == 0 ? in_tile % 8 * (hq / 8) + in_tile / 8 : in_tile, kvh = h / (hq / hkv);
-    int tile = total_tiles - 1 - blockIdx.x / hq, b = 0, tok0 = 0, n_new = 0;
-    for (; b < n_seqs; ++b) {
-        tok0 = cu_seqlens[b];
-        n_new = cu_seqlens[b + 1] - tok0;
-        int tiles = (n_new + TILE - 1) / TILE;
-        if (tile < tiles) break;
-        tile -= tiles;
-    }
-    if (b >= n_seqs) return;
+    const AmTile at = am_find_tile<TILE>(cu_seqlens, n_seqs, total_tiles - 1 - (int)blockIdx.x / hq);
+    if (at.b < 0) return;
+    const int tile = at.tile, b = at.b, tok0 = at.tok0, n_new = at.n_new;
     const int* pages = block_table + (size_t)b * bt_width;
     const int pos0 = token_pos[tok0];
     const int row_lo = tile * TILE, row_hi = min(n_new, row_lo + TILE) - 1;
