@@ -1667,14 +1667,29 @@ norm_add_kernel(float* __restrict__ x, float* __restrict__ y, const float* __res
     }
 }
 
+__device__ __forceinline__ void row4_load(float (&v)[4], const float* p) {
+    const float4 r = *(const float4*)p;
+    v[0] = r.x; v[1] = r.y; v[2] = r.z; v[3] = r.w;
+}
+__device__ __forceinline__ void row4_load(float (&v)[4], const bf16_t* p) {
+    const uint2 r = *(const uint2*)p;
+    v[0] = bf16_to_f32((bf16_t)r.x); v[1] = bf16_to_f32((bf16_t)(r.x >> 16)); v[2] = bf16_to_f32((bf16_t)r.y); v[3] = bf16_to_f32((bf16_t)(r.y >> 16));
+}
+
 // The same for rows of up to 8192 values that are a multiple of 4: the row stays in registers and all
 // loads are issued at once.
-template <typename TC, bool LAYER, int VEC>
+//
+// TAPS > 0: row b is the one token of the step's sequence b, and what the next norm gives passes that layer's input convolution
+// (added_conv_kernel, in its order of operations: the same bits) before it is written.  The launch of its own that this saves
+// was 3.75 us of a step and layer (as traced, five rows of 2,048 channels with four taps: 3.6 us without, 5.4 with the convolution).
+template <typename TC> struct NormConv { const float* w; TC* state; const int* slots; };       // [TAPS, n], [slots, TAPS - 1, n], [rows]
+
+template <typename TC, bool LAYER, int VEC, int TAPS = 0>
 __global__ void __launch_bounds__(EW_BLOCK)
 norm_add_vec_kernel(float* __restrict__ x, const float* __restrict__ y, const float* __restrict__ gain,
                     const float* __restrict__ bias, float eps, int n, TC* __restrict__ copy,
                     const float* __restrict__ partials, int n_splits, long long split_stride, int replace,
-                    const float* __restrict__ next_gain, float next_eps) {
+                    const float* __restrict__ next_gain, float next_eps, NormConv<TC> conv = {}) {
     // With a few rows this is priced in trips to memory: everything the row needs is asked for at once (the next norm's
     // gain too), the K pieces GROUP at a time, and no load stands behind a branch or a select, where the wave would wait
     // for it: threads beyond the row's end read its start and count nothing.  Five rows of 2048 with four pieces: 9.2 -> 5.0 us.
@@ -1690,6 +1705,21 @@ norm_add_vec_kernel(float* __restrict__ x, const float* __restrict__ y, const fl
     const float* ng = prepare ? next_gain : gain;
     const float* src = replace ? x : y;               // (read and not counted: the pieces are the whole of y)
     vec4 yv[VEC], xv[VEC], gv[VEC], bv[VEC], nv4[VEC], sum[VEC];
+    constexpr int KEPT = TAPS > 1 ? TAPS - 1 : 1;
+    vec4 taps[VEC][TAPS > 0 ? TAPS : 1];
+    float past[VEC][KEPT][4];
+    TC* kept = nullptr;
+    if constexpr (TAPS > 0) {
+        kept = conv.state + (size_t)conv.slots[blockIdx.x] * KEPT * n;
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) {
+            const int i = threadIdx.x + j * EW_BLOCK, at = i < nv ? i : 0;
+#pragma unroll
+            for (int t = 0; t < TAPS; ++t) taps[j][t] = ((const vec4*)(conv.w + (size_t)t * n))[at];
+#pragma unroll
+            for (int t = 0; t < KEPT; ++t) row4_load(past[j][t], kept + (size_t)t * n + 4 * at);
+        }
+    }
 #pragma unroll
     for (int j = 0; j < VEC; ++j) yv[j] = xv[j] = gv[j] = bv[j] = nv4[j] = sum[j] = zero4;
     if (!idle) {
@@ -1773,6 +1803,25 @@ norm_add_vec_kernel(float* __restrict__ x, const float* __restrict__ y, const fl
             int i = threadIdx.x + j * EW_BLOCK;
             if (i >= nv) continue;
             vec4 g2 = nv4[j];
+            if constexpr (TAPS > 0) {
+                float cur[4] = {xv[j].x * inv2 * g2.x, xv[j].y * inv2 * g2.y, xv[j].z * inv2 * g2.z, xv[j].w * inv2 * g2.w}, o[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if constexpr (sizeof(TC) == 2) cur[e] = bf16_to_f32(f32_to_bf16(cur[e]));
+                    asm("" : "+v"(cur[e]));             // (a product, rounded, as the next kernel read it: no part of the sums' fused products)
+                    float a = 0.f;
+#pragma unroll
+                    for (int t = 0; t + 1 < TAPS; ++t) a = fmaf(taps[j][t][e], past[j][t][e], a);
+                    a = fmaf(taps[j][TAPS - 1][e], cur[e], a);
+                    o[e] = cur[e] + a;
+                }
+                store4(copy + row + 4 * (size_t)i, o[0], o[1], o[2], o[3]);
+#pragma unroll
+                for (int t = 0; t + 2 < TAPS; ++t)
+                    store4(kept + (size_t)t * n + 4 * i, past[j][t + 1][0], past[j][t + 1][1], past[j][t + 1][2], past[j][t + 1][3]);
+                store4(kept + (size_t)(KEPT - 1) * n + 4 * i, cur[0], cur[1], cur[2], cur[3]);
+                continue;
+            }
             store4(copy + row + 4 * (size_t)i, xv[j].x * inv2 * g2.x, xv[j].y * inv2 * g2.y, xv[j].z * inv2 * g2.z, xv[j].w * inv2 * g2.w);
         }
     }
@@ -1794,6 +1843,51 @@ static void launch_norm_add(float* x, float* y, const float* gain, const float* 
     else if (v <= 4) NAV(4);
     else NAV(8);
 #undef NAV
+}
+
+// Taps that norm_add_vec_kernel takes: more of them do not fit the registers beside a row's pieces.
+constexpr int NC_MIN_TAPS = 2, NC_MAX_TAPS = 4, NC_MAX_WIDTH = 8 * EW_BLOCK;
+
+ROCML_EXPORT int rocml_norm_add_conv_fits(int n, int taps) {
+    return n > 0 && n % 4 == 0 && n <= NC_MAX_WIDTH && taps >= NC_MIN_TAPS && taps <= NC_MAX_TAPS;
+}
+
+template <typename TC>
+static int launch_norm_add_conv(float* x, const float* y, const float* gain, float eps, int n_rows, int n, TC* copy, const float* partials,
+                                int n_splits, long long split_stride, int replace, const float* next_gain, float next_eps,
+                                const NormConv<TC>& conv, int taps, hipStream_t stream) {
+#define NAC(V_, T_) norm_add_vec_kernel<TC, false, V_, T_><<<n_rows, EW_BLOCK, 0, stream>>>(x, y, gain, nullptr, eps, n, copy, partials, n_splits, split_stride, replace, next_gain, next_eps, conv)
+    if (n <= 4 * EW_BLOCK) {
+        if (taps == 2) NAC(1, 2); else if (taps == 3) NAC(1, 3); else NAC(1, 4);
+    } else {
+        if (taps == 2) NAC(2, 2); else if (taps == 3) NAC(2, 3); else NAC(2, 4);
+    }
+#undef NAC
+    return 0;
+}
+
+// rocml_norm_add (root-mean-square norms) whose next norm passes an input convolution, for a step of one token per sequence: row b is the
+// token of the sequence whose kept rows are state[slots[b]]; no two rows name one slot.
+ROCML_EXPORT int rocml_norm_add_conv(float* x, const float* y, int n_rows, int n, const float* gain, float eps, void* copy, int dtype,
+                                     const float* partials, int n_splits, long long split_stride, int replace, const float* next_gain,
+                                     float next_eps, const float* w, int taps, void* state, const int* slots, hipStream_t stream) {
+    ROCML_REQUIRE(n_rows >= 0 && rocml_norm_add_conv_fits(n, taps), "norm_add_conv: %d rows of %d with %d taps", n_rows, n, taps);
+    ROCML_REQUIRE(x && y && gain && copy && next_gain && w && state && slots && n_splits >= 0 && (n_splits == 0 || partials) && (!replace || n_splits > 0),
+                  "norm_add_conv: missing arguments");
+    ROCML_REQUIRE((((uintptr_t)x | (uintptr_t)y | (uintptr_t)gain | (uintptr_t)copy | (uintptr_t)partials | (uintptr_t)next_gain | (uintptr_t)w | (uintptr_t)state) & 15) == 0 &&
+                      split_stride % 4 == 0, "norm_add_conv: buffers must be 16-byte aligned");
+    if (n_rows == 0) return 0;
+    int rc;
+    if (dtype == ROCML_F32)
+        rc = launch_norm_add_conv<float>(x, y, gain, eps, n_rows, n, (float*)copy, partials, n_splits, split_stride, replace, next_gain, next_eps,
+                                         {w, (float*)state, slots}, taps, stream);
+    else if (dtype == ROCML_BF16)
+        rc = launch_norm_add_conv<bf16_t>(x, y, gain, eps, n_rows, n, (bf16_t*)copy, partials, n_splits, split_stride, replace, next_gain, next_eps,
+                                          {w, (bf16_t*)state, slots}, taps, stream);
+    else return rocml_fail("norm_add_conv: unknown dtype code %d", dtype);
+    if (rc) return rc;
+    ROCML_CHECK_LAUNCH("norm_add_conv");
+    return 0;
 }
 
 // The same with the sublayer's output still in branches: y = c * sum_b y_b / sqrt(mean(y_b^2) + eps_b) * gain_b (one or two

@@ -259,7 +259,7 @@ class DecoderModel:
             if following is not None and (s.schedule[i + 1].offset_row is not None or s.schedule[i + 1].add_embedding):
                 following = None      # the stream changes between the two blocks: nothing can be prepared across
             if getattr(block, "takes_next_norm", False) and hasattr(following, "entry_hint") and i + 1 not in chains:
-                hint = following.entry_hint(step)
+                hint = following.entry_hint(step, self.entry_view(i + 1, cache, step)) if getattr(following, "conv_rides", False) else following.entry_hint(step)
             if hint is not None:
                 block.forward(step, x, view, entry.reads_cache_of is None, next_norm=hint)
             else:

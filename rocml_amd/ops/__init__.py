@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import ctypes
 import functools
-from typing import Dict, Optional, Sequence
+from typing import Dict, Optional, Sequence, Tuple
 
 import torch
 
@@ -38,6 +38,8 @@ _SIGNATURES = {
         "rocml_norm_add": [_P, _P, _I, _I, _P, _P, _F, _I, _P, _I, _P, _I, _LL, _I, _P, _F, _P],
         "rocml_added_conv": [_P, _P, _I, _I, _I, _P, _I, _P, _I, _P, _P, _I, _P, _P],
         "rocml_activate": [_P, _P, _I, _LL, _I, _P],
+        "rocml_norm_add_conv": [_P, _P, _I, _I, _P, _F, _P, _I, _P, _I, _LL, _I, _P, _F, _P, _I, _P, _P, _P],
+        "rocml_norm_add_conv_fits": [_I, _I],
         "rocml_norm_add_branches": [_P, _P, _P, _P, _P, _F, _F, _I, _I, _P, _P, _F, _I, _P, _I, _P],
         "rocml_norm_add_branches_fits": [_I],
         "rocml_layernorm": [_P, _P, _I, _I, _P, _P, _F, _P, _I, _P],
@@ -419,14 +421,16 @@ def qk_span_stats(qkv: torch.Tensor, q_width: int, k_width: int, bias: Optional[
 
 def norm_add(x: torch.Tensor, y: torch.Tensor, gain: torch.Tensor, bias: Optional[torch.Tensor], eps: float,
              layer: bool, copy: Optional[torch.Tensor] = None, partials: Optional[torch.Tensor] = None,
-             replace: bool = False, next_gain: Optional[torch.Tensor] = None, next_eps: float = 0.0) -> None:
+             replace: bool = False, next_gain: Optional[torch.Tensor] = None, next_eps: float = 0.0,
+             conv: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None) -> None:
     """``x += f(y)`` row by row in 32-bit: ``f`` a layer norm ``(y - mean) / sqrt(var + eps) * gain + bias``
     (``layer``) or ``y / sqrt(mean(y^2) + eps) * gain``.  ``copy`` gets the new ``x`` in its own type.
     ``partials`` (``[splits, rows, n]`` 32-bit): the K pieces of the product that made ``y``, added to ``y`` in
     split order first, or with ``replace`` all of ``y`` (what ``y`` holds is not read).  ``next_gain`` (with ``copy``):
     ``copy`` gets the root-mean-square norm of the new ``x`` instead, ``x / sqrt(mean(x^2) + next_eps) * next_gain``: the
-    norm that reads the stream next."""
-    _dev(x, y, gain, bias, copy, partials, next_gain)
+    norm that reads the stream next.  ``conv`` (``(w, state, slots)``, with ``next_gain``, where ``norm_add_conv_fits``): row ``b`` is
+    the one token of a sequence with the kept rows ``state[slots[b]]``, and what the next norm gives passes ``added_conv``."""
+    _dev(x, y, gain, bias, copy, partials, next_gain, *(conv or ()))
     if next_gain is not None and (copy is None or next_gain.dtype != torch.float32 or next_gain.numel() != x.shape[1]):
         raise KernelError("norm_add: the next norm needs a 32-bit gain of the row's size and a place for its output")
     n_splits = split_stride = 0
@@ -442,10 +446,27 @@ def norm_add(x: torch.Tensor, y: torch.Tensor, gain: torch.Tensor, bias: Optiona
     if x.dim() != 2 or y.shape != x.shape or gain.numel() != x.shape[1] or (copy is not None and copy.shape != x.shape) \
             or (bias is not None and (bias.dtype != torch.float32 or bias.numel() != x.shape[1])):
         raise KernelError("norm_add: shapes do not fit")
+    if conv is not None:
+        w, state, slots = conv
+        _want(w, torch.float32, "convolution weights")
+        _want(slots, torch.int32, "sequence slots")
+        taps, n = w.shape
+        if layer or bias is not None or next_gain is None or not norm_add_conv_fits(n, taps) or n != x.shape[1] or slots.numel() != x.shape[0] \
+                or state.dtype != copy.dtype or state.dim() != 3 or tuple(state.shape[1:]) != (taps - 1, n):
+            raise KernelError(f"norm_add: {taps} taps of {n} channels with kept rows {tuple(state.shape)} do not fit {tuple(x.shape)}")
+        _check("elementwise", library("elementwise").rocml_norm_add_conv(
+            _ptr(x), _ptr(y), x.shape[0], n, _ptr(gain), float(eps), _ptr(copy), _code(copy), _ptr(partials), n_splits, split_stride,
+            1 if replace else 0, _ptr(next_gain), float(next_eps), _ptr(w), taps, _ptr(state), _ptr(slots), _stream()))
+        return
     _check("elementwise", library("elementwise").rocml_norm_add(
         _ptr(x), _ptr(y), x.shape[0], x.shape[1], _ptr(gain), _ptr(bias), float(eps), 1 if layer else 0, _ptr(copy),
         _code(copy) if copy is not None else 0, _ptr(partials), n_splits, split_stride, 1 if replace else 0, _ptr(next_gain),
         float(next_eps), _stream()))
+
+
+def norm_add_conv_fits(n: int, taps: int) -> bool:
+    """Whether ``norm_add`` takes a convolution of ``taps`` taps behind the next norm of rows of ``n`` values."""
+    return bool(library("elementwise").rocml_norm_add_conv_fits(int(n), int(taps)))
 
 
 ADDED_CONV_MAX_TAPS = 16

@@ -151,7 +151,10 @@ class NormHint:
 @dataclass(frozen=True)
 class FullNormHint(NormHint):
     """The same norm, for a consumer that wants the norm's whole output (not an operand that still lacks its rows' scale):
-    a kernel that completes the stream may write ``x / sqrt(mean(x^2) + eps) * gain`` in the compute type beside it."""
+    a kernel that completes the stream may write ``x / sqrt(mean(x^2) + eps) * gain`` in the compute type beside it.
+    ``conv``: ``(weights, kept rows)`` of a convolution that the norm's output passes on its way to the consumer, in a step of one token
+    per sequence; the kernel may apply it too (the consumer is told, and does not apply it again)."""
+    conv: Optional[Tuple[torch.Tensor, torch.Tensor]] = None
 
 
 @dataclass(frozen=True)

@@ -18,6 +18,7 @@ convolution)``.  A schedule entry that reads another entry's cache line shares t
 convolution rows (``reader_request``, ``shared_view``, ``reader_view``)."""
 from __future__ import annotations
 
+import functools
 from typing import Dict
 
 from .. import ops
@@ -413,7 +414,7 @@ class SandwichNormBlock(ConvInput, Part):
     root-mean-square norms with a gain."""
     takes_pending = False
     takes_next_norm = True
-    _READY = "sandwich_norm.operand"      # in step.memo: (stream, gain, operand) of a norm that the kernel before formed
+    _READY = "sandwich_norm.operand"      # in step.memo: (stream, gain, operand, convolution) that the kernel before formed
 
     def __init__(self, spec: BlockSpec, ctx: BuildContext):
         if spec.mixer_out_norm is None or (spec.ffn is not None and (spec.ffn_norm is None or spec.ffn_out_norm is None)):
@@ -448,13 +449,23 @@ class SandwichNormBlock(ConvInput, Part):
             (self.ffn.activation_bytes(n_tokens) if self.ffn is not None else 0) + \
             (self.input_conv.activation_bytes(n_tokens) if self.input_conv is not None else 0)
 
-    def entry_hint(self, step):
-        """The norm this block reads the stream with first, for the kernel that completes the stream before it."""
+    def entry_hint(self, step, view=None):
+        """The norm this block reads the stream with first, for the kernel that completes the stream before it; with the
+        convolution behind it where that kernel takes it (``view``: this block's line of the cache)."""
         norm = self.children["mixer_norm"]
         gain = getattr(norm, "gain", None)
         if gain is None or not hasattr(norm, "eps") or getattr(norm, "centred", False):
             return None
-        return FullNormHint(gain, float(norm.eps), self.hidden)
+        conv = None
+        rows = self._views(view)[1]
+        if rows is not None and step.max_new == 1 and step.n_tokens == step.n_seqs and self.conv_rides:
+            conv = (self.input_conv.w, rows.state)
+        return FullNormHint(gain, float(norm.eps), self.hidden, conv)
+
+    @functools.cached_property
+    def conv_rides(self) -> bool:
+        """Whether the kernel that forms the first norm also takes this block's input convolution."""
+        return self.input_conv is not None and ops.norm_add_conv_fits(self.hidden, self.input_conv.taps)
 
     def _sublayer(self, step, x, norm, run, out_norm, following, conv_view=None) -> None:
         """``following``: a ``FullNormHint`` of the norm that reads the stream after this sublayer, or None.
@@ -466,9 +477,12 @@ class SandwichNormBlock(ConvInput, Part):
         if ready is not None and gain is not None and ready[0] == x.data_ptr() and ready[1] == gain.data_ptr():
             xn = ready[2]           # the kernel that completed the stream formed this norm on its way
         else:
+            if ready is not None and ready[3] is not None:
+                raise ConfigError("a convolution's kept rows were brought up to date for another layer than the one that reads it")
+            ready = None
             xn = ws.get("block.xn", tuple(x.shape), self.dtype)
             norm.forward(x, xn)
-        if conv_view is not None:
+        if conv_view is not None and (ready is None or ready[3] is None):
             xn = self.input_conv.forward(step, xn, conv_view[0])
         y = ws.get("block.sublayer", tuple(x.shape), torch.float32)
         rs.overwrite = rs.defer_overwrite = True
@@ -479,9 +493,10 @@ class SandwichNormBlock(ConvInput, Part):
         if isinstance(following, FullNormHint) and following.width == x.shape[1]:
             # (the sublayer is done with its operand: the buffer takes the next one)
             nxt = ws.get("block.xn", tuple(x.shape), self.dtype)
+            conv = following.conv
             ops.norm_add(x, y, out_norm.gain, None, out_norm.eps, layer=False, partials=partials, replace=replace, copy=nxt,
-                         next_gain=following.gain, next_eps=following.eps)
-            step.memo[self._READY] = (x.data_ptr(), following.gain.data_ptr(), nxt)
+                         next_gain=following.gain, next_eps=following.eps, conv=None if conv is None else (*conv, step.seq_slots))
+            step.memo[self._READY] = (x.data_ptr(), following.gain.data_ptr(), nxt, conv)
         else:
             ops.norm_add(x, y, out_norm.gain, None, out_norm.eps, layer=False, partials=partials, replace=replace)
 
