@@ -1061,7 +1061,8 @@ def decode_splits(pairs: int, n_cus: int, most: int) -> int:
     18 sequences 3,555 with 3, 3,375 with 5; 24 sequences 4,480 with none, 4,310 with 4;
     32 sequences 5,620 with none, 5,375 with 2; 40 sequences 5,990 with 3, 5,720 with none;
     56 sequences 7,330 with none, 7,000 with 2.  Below 8 sequences' worth of pairs (64) the
-    rule is about a block a CU."""
+    rule is about a block a CU.  (Where the kernel shares its blocks out by the sequences' lengths this is not their number:
+    ``shared_slots`` in ``attention.hip``.)"""
     if pairs * 4 < n_cus:
         # a few sequences: about a block a CU (two pieces of each wave are then on their way); measured,
         # one block a CU against two: one sequence 277.5 against 274.8 tokens a second, two 542 against
