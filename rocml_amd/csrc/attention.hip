@@ -175,8 +175,8 @@ static bool prompt_takes(const AttnArgs& a, int d) { return d == 128 && !a.has_e
 // Whether it is the faster way.  Its blocks have twice the rows of attn_prefill_mfma_kernel's and a CU holds one, so each pays for its
 // start and end (some 10 us) by itself and a page takes 1.6 to 1.75 us for 256 rows where the other takes 1.8 to 2.4: it wants blocks of
 // many pages, and enough of them to fill the chip.  Measured (32 query heads on 8, us, the other kernel first): prompts of 1,024 tokens,
-// one 31 and 39, four 70 and 74; of 1,536, one 47 and 52, four 119 and 123; of 2,048 (18 pages a block), one (a block a CU) 62 and 67, two
-// 103 and 92, four 183 and 178; of 3,000 (26 pages), one 128 and 92, on 16 heads (192 blocks) 115 and 81; of 8,192 750 and 549, behind
+// one 31 and 35, four 70 and 68; of 1,536, one 45 and 46, four 118 and 113; of 2,048 (18 pages a block), one (a block a CU) 60 and 59, two
+// 97 and 83, four 176 and 164; of 3,000 (26 pages), one 112 and 85, on 16 heads (192 blocks) 101 and 74; of 8,192 599 and 499, behind
 // 24,576 others 4,038 and 3,108.  With a window of 2,048 4,096 tokens take 136 and 148, which is why windows stay with the other.
 // The positions before the step's first token are not known here: a step behind many others counts as if it were the first.
 static bool prompt_pays(const AttnArgs& a) {

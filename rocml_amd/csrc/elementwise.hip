@@ -1681,7 +1681,7 @@ __device__ __forceinline__ void row4_load(float (&v)[4], const bf16_t* p) {
 //
 // TAPS > 0: row b is the one token of the step's sequence b, and what the next norm gives passes that layer's input convolution
 // (added_conv_kernel, in its order of operations: the same bits) before it is written.  The launch of its own that this saves
-// was 3.75 us of a step and layer (as traced, five rows of 2,048 channels with four taps: 3.6 us without, 5.4 with the convolution).
+// was 3.75 us of a step and layer (as traced, five rows of 2,048 channels with four taps: 5.0 us without, 5.6 with the convolution).
 template <typename TC> struct NormConv { const float* w; TC* state; const int* slots; };       // [TAPS, n], [slots, TAPS - 1, n], [rows]
 
 template <typename TC, bool LAYER, int VEC, int TAPS = 0>
