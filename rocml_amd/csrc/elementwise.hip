@@ -1874,8 +1874,10 @@ ROCML_EXPORT int rocml_norm_add_conv(float* x, const float* y, int n_rows, int n
     ROCML_REQUIRE(n_rows >= 0 && rocml_norm_add_conv_fits(n, taps), "norm_add_conv: %d rows of %d with %d taps", n_rows, n, taps);
     ROCML_REQUIRE(x && y && gain && copy && next_gain && w && state && slots && n_splits >= 0 && (n_splits == 0 || partials) && (!replace || n_splits > 0),
                   "norm_add_conv: missing arguments");
-    ROCML_REQUIRE((((uintptr_t)x | (uintptr_t)y | (uintptr_t)gain | (uintptr_t)copy | (uintptr_t)partials | (uintptr_t)next_gain | (uintptr_t)w | (uintptr_t)state) & 15) == 0 &&
-                      split_stride % 4 == 0, "norm_add_conv: buffers must be 16-byte aligned");
+    // (four values at a time: 16 bytes of 32-bit rows, 8 of bfloat16 ones)
+    ROCML_REQUIRE((((uintptr_t)x | (uintptr_t)y | (uintptr_t)gain | (uintptr_t)partials | (uintptr_t)next_gain | (uintptr_t)w) & 15) == 0 &&
+                      (((uintptr_t)copy | (uintptr_t)state) & (dtype == ROCML_BF16 ? 7 : 15)) == 0 && split_stride % 4 == 0,
+                  "norm_add_conv: buffers must be 16-byte aligned, bfloat16 rows 8");
     if (n_rows == 0) return 0;
     int rc;
     if (dtype == ROCML_F32)

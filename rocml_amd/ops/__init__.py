@@ -469,6 +469,14 @@ def norm_add_conv_fits(n: int, taps: int) -> bool:
     return bool(library("elementwise").rocml_norm_add_conv_fits(int(n), int(taps)))
 
 
+def norm_add_conv_takes(x: torch.Tensor, y: torch.Tensor, gain: torch.Tensor, copy: torch.Tensor, partials: Optional[torch.Tensor],
+                        next_gain: torch.Tensor, w: torch.Tensor, state: torch.Tensor) -> bool:
+    """Whether ``norm_add`` takes these operands with a convolution: their sizes, and where they start (it reads four values at a time;
+    ``norm_add`` and ``added_conv`` one after the other take any start)."""
+    return norm_add_conv_fits(x.shape[1], w.shape[0]) and all(
+        t is None or t.data_ptr() % (4 * t.element_size()) == 0 for t in (x, y, gain, copy, partials, next_gain, w, state))
+
+
 ADDED_CONV_MAX_TAPS = 16
 
 

@@ -494,6 +494,8 @@ class SandwichNormBlock(ConvInput, Part):
             # (the sublayer is done with its operand: the buffer takes the next one)
             nxt = ws.get("block.xn", tuple(x.shape), self.dtype)
             conv = following.conv
+            if conv is not None and not ops.norm_add_conv_takes(x, y, out_norm.gain, nxt, partials, following.gain, *conv):
+                conv = None             # (the layer that reads the norm applies it itself)
             ops.norm_add(x, y, out_norm.gain, None, out_norm.eps, layer=False, partials=partials, replace=replace, copy=nxt,
                          next_gain=following.gain, next_eps=following.eps, conv=None if conv is None else (*conv, step.seq_slots))
             step.memo[self._READY] = (x.data_ptr(), following.gain.data_ptr(), nxt, conv)
