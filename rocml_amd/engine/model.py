@@ -5,6 +5,7 @@ head (norm and output product) only for the rows whose logits are wanted.
 """
 from __future__ import annotations
 
+from dataclasses import replace
 from typing import Dict, List, Optional
 
 import torch
@@ -15,6 +16,7 @@ from ..cache.cache import HEADROOM_BYTES
 from ..config.spec import ModelSpec
 from ..errors import ConfigError
 from ..parts import BuildContext, ParamSpec, build_block, build_embedding, build_head
+from ..parts.base import FullNormHint
 from .batch import StepContext
 from .workspace import Workspace
 
@@ -214,6 +216,18 @@ class DecoderModel:
                 run = chains[i] = [layer]
         return chains
 
+    def next_hint(self, i: int, cache: Cache, step: StepContext):
+        """The norm that the block behind schedule entry ``i`` reads the stream with first, with the convolution behind it where it
+        rides along: what entry ``i``'s block may prepare.  None where the stream changes between the two."""
+        entry = self.spec.schedule[i + 1] if i + 1 < len(self.spec.schedule) else None
+        if entry is None or entry.offset_row is not None or entry.add_embedding:
+            return None
+        following = self.blocks[entry.layer]
+        hint = following.entry_hint(step) if hasattr(following, "entry_hint") else None
+        if isinstance(hint, FullNormHint) and getattr(following, "conv_rides", False):
+            hint = replace(hint, conv=following.entry_conv(step, self.entry_view(i + 1, cache, step)))
+        return hint
+
     # -- forward -----------------------------------------------------------------------
     def forward(self, step: StepContext, cache: Cache, block_tables: Dict[str, torch.Tensor],
                 want_rows: Optional[torch.Tensor], n_want: int) -> Optional[torch.Tensor]:
@@ -253,13 +267,7 @@ class DecoderModel:
                 ops.add_into(x, x0)
             if not getattr(block, "takes_pending", False):
                 ws.flush_pending()
-            # the block that runs next may let this block's last product prepare its first norm
-            following = self.blocks[s.schedule[i + 1].layer] if i + 1 < len(s.schedule) else None
-            hint = None
-            if following is not None and (s.schedule[i + 1].offset_row is not None or s.schedule[i + 1].add_embedding):
-                following = None      # the stream changes between the two blocks: nothing can be prepared across
-            if getattr(block, "takes_next_norm", False) and hasattr(following, "entry_hint") and i + 1 not in chains:
-                hint = following.entry_hint(step, self.entry_view(i + 1, cache, step)) if getattr(following, "conv_rides", False) else following.entry_hint(step)
+            hint = self.next_hint(i, cache, step) if getattr(block, "takes_next_norm", False) and i + 1 not in chains else None
             if hint is not None:
                 block.forward(step, x, view, entry.reads_cache_of is None, next_norm=hint)
             else:

@@ -449,18 +449,21 @@ class SandwichNormBlock(ConvInput, Part):
             (self.ffn.activation_bytes(n_tokens) if self.ffn is not None else 0) + \
             (self.input_conv.activation_bytes(n_tokens) if self.input_conv is not None else 0)
 
-    def entry_hint(self, step, view=None):
-        """The norm this block reads the stream with first, for the kernel that completes the stream before it; with the
-        convolution behind it where that kernel takes it (``view``: this block's line of the cache)."""
+    def entry_hint(self, step):
+        """The norm this block reads the stream with first, for the kernel that completes the stream before it."""
         norm = self.children["mixer_norm"]
         gain = getattr(norm, "gain", None)
         if gain is None or not hasattr(norm, "eps") or getattr(norm, "centred", False):
             return None
-        conv = None
+        return FullNormHint(gain, float(norm.eps), self.hidden)
+
+    def entry_conv(self, step, view):
+        """``(weights, kept rows)`` of the convolution that the first norm's output passes, where the kernel that forms the norm can
+        apply it in this step, or None.  ``view``: this block's line of the cache."""
         rows = self._views(view)[1]
-        if rows is not None and step.max_new == 1 and step.n_tokens == step.n_seqs and self.conv_rides:
-            conv = (self.input_conv.w, rows.state)
-        return FullNormHint(gain, float(norm.eps), self.hidden, conv)
+        if rows is None or step.max_new != 1 or step.n_tokens != step.n_seqs:
+            return None
+        return self.input_conv.w, rows.state
 
     @functools.cached_property
     def conv_rides(self) -> bool:
