@@ -43,7 +43,7 @@ static int launch_decode_kernel(const AttnArgs& a, int n_splits, AmShared shared
     int group = a.hq / a.hkv;
     int lds = WAVES * group * (D + 4) * (int)sizeof(float);
     // blocks shared out by the tokens' lengths: n_splits is the room for the splits of one
-    dim3 grid(shared.n_tokens > 0 ? shared.slots : n_splits, a.hkv, shared.n_tokens > 0 ? 1 : a.n_tokens);
+    const dim3 grid = shared.n_tokens > 0 ? dim3(a.hkv, shared.slots) : dim3(n_splits, a.hkv, a.n_tokens);
     if (a.has_extra) {
         static int allowed_extra = 0;
         if (lds > allowed_extra) {

@@ -61,8 +61,11 @@ struct DecodeProj {
 // grid (n_splits, Hkv, tokens), 4 or 8 waves; the block's pages are cut into 32-key pieces that the
 // waves take in turn; all query heads of the kv head ride in the 16 columns of the MFMA.
 //
-// shared.n_tokens > 0: grid (slots, Hkv), the blocks shared out among the step's tokens by their lengths (am_share; no window, no blocks
-// of positions), n_splits the room for a row's partial results.  With as many splits for every token the longest sequence of an
+// shared.n_tokens > 0: grid (Hkv, slots), the blocks shared out among the step's tokens by their lengths (am_share; no window, no blocks
+// of positions), n_splits the room for a row's partial results.  A page's kv heads lie side by side, so the blocks that run together have
+// to be of all of them: with the slots side by side and more blocks than run at once, one head's rows of every page were read, then the
+// next one's, 16 KB out of every 128, from a part of the memory's channels (56 sequences, a quarter of 4,000 keys and the others of 500:
+// 143.2 us, 95.4 this way; half of 4,000 151.9 and 110.3; 48, a third of 4,000, 88.2 and 74.3; 8 of 2,070 20.6 and 20.2).  With as many splits for every token the longest sequence of an
 // unequal batch was the whole kernel's time.  Us with the merge, 32 heads on 8 but the first, even splits and shared ones:
 // 16 of 128 to 4,096 keys on 40 heads 41.4 and 26.7 (their bytes: 16.6), 8 of 200 to 4,000 24.0 and 18.7, 24 of them 69.7 and 44.4; what
 // it costs where all are of one length: 8 of 2,070 20.9 and 21.5, 16 of 600 16.5 and 17.0.
@@ -154,9 +157,10 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     int group = hq / hkv;
     const int room = n_splits;                      // for a row's partial results
     if (shared.n_tokens > 0) {                      // (a guess that holds for tokens of one length)
+        kvh = blockIdx.x;
         n_splits = shared.even;
-        t = min((int)blockIdx.x / n_splits, shared.n_tokens - 1);
-        split = blockIdx.x - t * n_splits;
+        t = min((int)blockIdx.y / n_splits, shared.n_tokens - 1);
+        split = blockIdx.y - t * n_splits;
     }
     // (token_seq null: token t is the one token of the step's sequence t)
     const int* pages = block_table + (size_t)(token_seq ? token_seq[t] : t) * bt_width;
@@ -167,7 +171,7 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     for (int i = 0; i < 4; ++i) early[i] = pages[split + i * n_splits < bt_width ? split + i * n_splits : 0];
     bool looked_up = true;
     if (shared.n_tokens > 0) {
-        const AmShare share = am_share(token_pos, shared.n_tokens, shared.slots, room, blockIdx.x, {t, split, n_splits});
+        const AmShare share = am_share(token_pos, shared.n_tokens, shared.slots, room, blockIdx.y, {t, split, n_splits});
         if (share.t < 0) return;
         looked_up = share.t == t && share.split == split && share.n_splits == n_splits;
         t = share.t;
