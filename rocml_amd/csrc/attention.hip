@@ -30,6 +30,7 @@ struct AttnArgs {
     const int* cu_seqlens; int n_seqs; int n_tokens; int total_q_tiles; int max_len;
     int hq, hkv; float scale; int window; void* workspace; long long workspace_bytes;
     int n_splits_hint;
+    bool unequal;               // decode only: the tokens' lengths differ by much
     const DecodeProj* proj;     // decode only: the step's q/k/v projection instead of q and an appended cache
     const PrefillProj* prefill_proj = nullptr;      // prompts: the projection instead of prepared queries
     const int* q_counts = nullptr;                  // prompts: query tokens of each sequence (host memory)
@@ -70,18 +71,18 @@ static int launch_decode_kernel(const AttnArgs& a, int n_splits, AmShared shared
 
 constexpr int WIDE_BLOCK_MIN_PIECES = 8;         // of a block: more than two a wave of four
 
-// Blocks a kv head that the tokens of a step share by their lengths, or 0: as many for every token.  By the launch's shape only, as a
-// recorded step is replayed while its sequences grow: batches of unequal lengths gain, those of one length pay for the working out
-// and for a merge (figures, even splits and shared ones, us with the merge, 32 heads on 8).
-// Up to half a block a CU without splits, a block of eight waves a CU: 6 sequences of 200 to 4,000 keys 21.0 and 17.4, 16 of them
-// 41.2 and 29.8, 16 of 100 to 1,000 17.0 and 15.6; of one length 6 of 2,070 18.6 and 19.0, 16 34.1 and 34.4.  Up to a
-// block for every eight CUs it does not pay: 3 of 2,070 13.2 and 13.9, 4 of 100 to 1,000 11.0 and 11.5.
+// Blocks a kv head that the tokens of a step share by their lengths, or 0: as many for every token.  The caller says whether the lengths
+// differ by enough to gain (lengths_differ in ops has the line and its figures); a step of equal ones pays for the working out and for a
+// merge.  The rest goes by the launch's shape, as a recorded step is replayed while its sequences grow (us with the merge, 32 heads
+// on 8, even splits and shared ones).
+// Up to half a block a CU without splits, a block of eight waves a CU: 6 sequences of 200 to 4,000 keys 20.8 and 16.1, 16 of them
+// 42.1 and 34.0, 16 of 50 to 1,000 17.3 and 15.8.  Up to a block for every eight CUs it does not pay: 3 of 2,070 13.2 and 13.9, 4 of 100 to 1,000
+// 11.0 and 11.5.
 // Beyond, two blocks of four waves a CU (or what even splits are), where the block table has room for more than 1,024 keys: 24 of 200 to
-// 4,000 69.7 and 44.4, 32 75 and 57.7, 40 78.2 and 69.9, 56 133 and 120; of one length 24 of 2,070 48.3 and 52.6, 56 101.6 and 104.8; below, 32 of
-// 100 to 1,000 24.7 and 24.4, but 32 of 600 21.3 and 26.0.
+// 4,000 67.9 and 32.3, 32 72.0 and 52.8, 40 71.5 and 55.6, 56 127.4 and 92.3; below, 32 of 100 to 1,000 24.7 and 24.4, but 32 of 600 21.3 and 26.0.
 static int shared_slots(const AttnArgs& a, int n_splits) {
     const long long pairs = (long long)a.n_tokens * a.hkv, cus = cu_count();
-    if (a.n_tokens > 64 || a.window > 0 || a.extra.chunk > 0 || 8 * pairs <= cus) return 0;
+    if (!a.unequal || a.n_tokens > 64 || a.window > 0 || a.extra.chunk > 0 || 8 * pairs <= cus) return 0;
     if (2 * pairs <= cus) return (int)(cus / a.hkv);
     const long long slots = n_splits > 1 ? (long long)n_splits * a.n_tokens : 2 * cus / a.hkv;
     return a.bt_width >= 32 && 8ll * a.n_tokens <= 7 * slots ? (int)slots : 0;
@@ -286,7 +287,7 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
                                  const int* token_seq, const int* token_pos, int n_tokens, int hq,
                                  int hkv, int d, int page_size, float scale, int window, int algo,
                                  const int* cu_seqlens, int n_seqs, int max_new, const int* q_counts,
-                                 int max_len, int n_splits, void* workspace, long long workspace_bytes,
+                                 int max_len, int n_splits, int unequal, void* workspace, long long workspace_bytes,
                                  int dv, int v_in_k, int chunk, const float* slopes, int sink,
                                  const float* sinks, float softcap, int keep_first, hipStream_t stream) {
     // dv (0: the key head's size), v_in_k, chunk, slopes, sink, sinks, softcap and keep_first: see AttnExtra in attention_generic.h.
@@ -367,7 +368,7 @@ ROCML_EXPORT int rocml_attention(const void* q, void* out, const void* kcache, c
     if (mfma_ok && algo != ATTN_PLAIN) {
         AttnArgs a{(const bf16_t*)q, (bf16_t*)out, (const bf16_t*)kcache, (const bf16_t*)vcache, block_table,
                    bt_width, token_seq, token_pos, cu_seqlens, n_seqs, n_tokens, (int)total_q_tiles, max_len, hq, hkv,
-                   scale, window, workspace, workspace_bytes, n_splits, nullptr};
+                   scale, window, workspace, workspace_bytes, n_splits, unequal != 0, nullptr};
         a.extra = MaskExtra{chunk, slopes, sink, sinks, softcap, keep_first};
         a.has_extra = has_extra;
         a.q_counts = q_counts;
@@ -437,7 +438,7 @@ ROCML_EXPORT int rocml_attention_decode_fused(const float* qkv, int ld, int qkv_
                                               void* kcache, void* vcache, const int* block_table, int bt_width,
                                               const int* token_seq, const int* token_pos, int n_tokens, int hq,
                                               int hkv, int d, int page_size, float scale, int window,
-                                              int max_len, int n_splits, void* workspace,
+                                              int max_len, int n_splits, int unequal, void* workspace,
                                               long long workspace_bytes, const float* row_ssq, int row_parts,
                                               float row_eps, int row_width, const float* bias, int chunk,
                                               const float* slopes, int sink, const float* sinks, int keep_first, int rot,
@@ -474,7 +475,7 @@ ROCML_EXPORT int rocml_attention_decode_fused(const float* qkv, int ld, int qkv_
                   row_ssq, row_parts, row_eps, row_ssq ? 1.0f / (float)row_width : 0.f, bias, rot, v_is_k};
     AttnArgs a{nullptr, (bf16_t*)out, (const bf16_t*)kcache, (const bf16_t*)vcache, block_table, bt_width,
                token_seq, token_pos, nullptr, 0, n_tokens, 0, max_len, hq, hkv, scale, window, workspace,
-               workspace_bytes, n_splits, &pj};
+               workspace_bytes, n_splits, unequal != 0, &pj};
     a.extra = MaskExtra{chunk, slopes, sink, sinks, 0.f, keep_first};
     // (the bias, a rotation of a part of the head and values taken from the keys ride in the same instantiation)
     a.has_extra = chunk > 0 || slopes || sink || bias || keep_first > 0 || rot != d || v_is_k;
@@ -527,7 +528,7 @@ ROCML_EXPORT int rocml_attention_prefill_fused(const float* qkv, int ld, const f
     PrefillProj pj{qkv, ld, q_gain, eps, cos_t, sin_t};
     AttnArgs a{nullptr, (bf16_t*)out, (const bf16_t*)kcache, (const bf16_t*)vcache, block_table, bt_width,
                nullptr, token_pos, cu_seqlens, n_seqs, n_tokens, (int)total_q_tiles, 0, hq, hkv, scale, window, nullptr,
-               0, 0, nullptr};
+               0, 0, false, nullptr};
     a.prefill_proj = &pj;
     a.q_counts = q_counts;
     int rc = BY_HEAD_DIM(launch_prefill, d, a, stream);

@@ -65,10 +65,10 @@ struct DecodeProj {
 // of positions), n_splits the room for a row's partial results.  A page's kv heads lie side by side, so the blocks that run together have
 // to be of all of them: with the slots side by side and more blocks than run at once, one head's rows of every page were read, then the
 // next one's, 16 KB out of every 128, from a part of the memory's channels (56 sequences, a quarter of 4,000 keys and the others of 500:
-// 143.2 us, 95.4 this way; half of 4,000 151.9 and 110.3; 48, a third of 4,000, 88.2 and 74.3; 8 of 2,070 20.6 and 20.2).  With as many splits for every token the longest sequence of an
-// unequal batch was the whole kernel's time.  Us with the merge, 32 heads on 8 but the first, even splits and shared ones:
-// 16 of 128 to 4,096 keys on 40 heads 41.4 and 26.7 (their bytes: 16.6), 8 of 200 to 4,000 24.0 and 18.7, 24 of them 69.7 and 44.4; what
-// it costs where all are of one length: 8 of 2,070 20.9 and 21.5, 16 of 600 16.5 and 17.0.
+// 143.2 us, 95.4 this way; half of 4,000 151.9 and 110.3; 48, a third of 4,000, 88.2 and 74.3; 8 of 2,070 20.6 and 20.2).
+// With as many splits for every token the longest sequence of an unequal batch was the whole kernel's time.  Us with the merge, 32 heads
+// on 8 but the first, even splits and shared ones: 24 of 400 to 4,000 keys on 40 heads 72.2 and 48.4, 8 of 200 to 4,000 23.8 and 16.1,
+// 24 of them 67.9 and 32.3; where all are of one length (the callers then ask for even splits): 8 of 2,070 19.8 and 20.2, 24 48.7 and 55.5.
 //
 // FUSED: the kernel takes the projection's output instead of q and a finished cache: every block
 // norms and rotates the q heads of its kv head itself and lays them out as the MFMA operand; the

@@ -17,7 +17,9 @@ from typing import Dict, List, Optional, Sequence
 import numpy as np
 import torch
 
+from .. import ops
 from ..cache import Cache
+from ..cache.cache import KVGroup
 from ..errors import CacheFullError, ContextOverflowError, RocmlError, StepFailedError
 from .. import profile
 from ..staging import Staging
@@ -51,6 +53,9 @@ class Engine:
         self.max_prompt_graphs = 32
         self._graphs: Dict[tuple, tuple] = {}
         self._staging = Staging()
+        # most key/value heads of a layer whose decode steps may share their blocks out by the sequences' lengths
+        self._kv_heads = max([g.request.n_kv_heads for g in self.cache.kv_groups if isinstance(g, KVGroup) and g.span is None], default=0)
+        self._n_cus = ops.cu_count(model.device) if model.dtype == torch.bfloat16 else 0
 
     # -- sequences -----------------------------------------------------------------------
     def new_sequence(self) -> int:
@@ -199,6 +204,7 @@ class Engine:
             meta[:ids.size].copy_(device_ids)           # the ids lead the table
         max_new = max(len(t) for t in tokens)
         n_want = int(want_rows.size)
+        unequal = max_new == 1 and ops.may_share(len(slots), self._kv_heads, self._n_cus) and ops.lengths_differ(lens.tolist())
 
         def context() -> StepContext:
             views, at = [], 0
@@ -213,7 +219,7 @@ class Engine:
                                token_pos=d_pos, cu_seqlens=d_cu, seq_lens=d_lens, seq_slots=d_slots,
                                max_new=max_new, max_len=int(lens.max()),
                                new_counts=tuple(len(t) for t in tokens),
-                               workspace=self.workspace)
+                               workspace=self.workspace, unequal=unequal)
             step.block_tables = block_tables
             step.want_rows = d_want if n_want else None
             return step
@@ -227,13 +233,13 @@ class Engine:
             return run(context())
         # Steps of one shape run from a recorded graph: the launches of a step are the same every
         # time, only the integer tables change, and those lie at fixed addresses.  A decode step's
-        # shape is its number of sequences; a prompt step's is every sequence's number of tokens
-        # and first position (short prompts only: a long one keeps the GPU busy far longer than
+        # shape is its number of sequences and whether their lengths differ by much (another launch of the
+        # attention); a prompt step's is every sequence's number of tokens and first position (short prompts only: a long one keeps the GPU busy far longer than
         # the host needs to launch it).  A shape runs plainly the first time (kernels set
         # themselves up, buffers reach their size), is recorded the second time, and replayed
         # from then on.
         if max_new == 1:
-            key = (len(slots), n_want, width)
+            key = (len(slots), n_want, width, unequal)
         elif self.model.prompt_graph_safe and int(ids.size) <= self.max_graph_prompt_tokens:
             key = ("prompt", tuple(len(t) for t in tokens), tuple(starts), n_want, width)
         else:

@@ -89,9 +89,9 @@ _SIGNATURES = {
     },
     "attention": {
         "rocml_attention": [_P, _P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _I, _I, _I, _F, _I, _I,
-                            _P, _I, _I, _P, _I, _I, _P, _LL, _I, _I, _I, _P, _I, _P, _F, _I, _P],
+                            _P, _I, _I, _P, _I, _I, _I, _P, _LL, _I, _I, _I, _P, _I, _P, _F, _I, _P],
         "rocml_attention_decode_fused": [_P, _I, _I, _LL, _P, _P, _F, _P, _P, _I, _P, _P, _P, _P, _I, _P, _P,
-                                         _I, _I, _I, _I, _I, _F, _I, _I, _I, _P, _LL, _P, _I, _F, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
+                                         _I, _I, _I, _I, _I, _F, _I, _I, _I, _I, _P, _LL, _P, _I, _F, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
         "rocml_attention_prefill_fused": [_P, _I, _P, _F, _P, _P, _P, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _F, _I,
                                           _P, _I, _P, _P],
     },
@@ -985,7 +985,7 @@ def attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, v_cache
               q_counts: Optional[Sequence[int]] = None, max_len: int = 0, n_splits: int = 0,
               v_head_dim: Optional[int] = None, values_in_keys: bool = False, chunk: Optional[int] = None,
               slopes: Optional[torch.Tensor] = None, sink: bool = False, sinks: Optional[torch.Tensor] = None,
-              softcap: Optional[float] = None, keep_first: int = 0) -> None:
+              softcap: Optional[float] = None, keep_first: int = 0, unequal: bool = False) -> None:
     """Attention of the step's query tokens over the cache.  Keys are ``[pages, Hkv, page, D]``,
     values ``[pages, Hkv, D, page]``.  ``cu_seqlens`` (device), ``q_counts`` (the same knowledge on
     the host: query tokens of each sequence), ``max_new`` (the most of them) and ``max_len``
@@ -998,7 +998,11 @@ def attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, v_cache
     taken off the score of query ``i`` and key ``j``.  ``sink``: the denominator of the softmax has
     one more term ``exp(0)``, or with ``sinks`` (32-bit, one per query head) ``exp(sinks[h])``.
     ``softcap``: the scaled score ``s`` becomes ``softcap * tanh(s / softcap)`` before the mask.
-    ``keep_first``: with a window, the first so many positions are seen whatever their distance."""
+    ``keep_first``: with a window, the first so many positions are seen whatever their distance.
+
+    Decode: ``n_splits`` (0: chosen here) splits of every token's keys.  ``unequal``: the tokens see numbers of keys that differ by much
+    (``lengths_differ``), and the blocks may go by them instead (five to 64 tokens at 8 kv heads, no window, no blocks of positions;
+    ``n_splits`` is then no more than where their number starts from)."""
     _dev(q, out, k_cache, v_cache, block_table, token_seq, token_pos, cu_seqlens, slopes, sinks)
     if sinks is not None:
         _want(sinks, torch.float32, "sinks")
@@ -1043,7 +1047,7 @@ def attention(q: torch.Tensor, out: torch.Tensor, k_cache: torch.Tensor, v_cache
         _ptr(q), _ptr(out), _ptr(k_cache), _ptr(v_cache), _code(q), _ptr(block_table),
         block_table.shape[1], _ptr(token_seq), _ptr(token_pos), n_tokens, n_heads, n_kv_heads, head_dim,
         page, scale, 0 if window is None else int(window), algo, _ptr(cu_seqlens), n_seqs, max_new,
-        counts, max_len, n_splits, ws_ptr, ws_bytes, dv, 1 if values_in_keys else 0,
+        counts, max_len, n_splits, 1 if unequal else 0, ws_ptr, ws_bytes, dv, 1 if values_in_keys else 0,
         0 if chunk is None else int(chunk), _ptr(slopes), 1 if sink else 0, _ptr(sinks),
         0.0 if softcap is None else float(softcap), int(keep_first), _stream()))
 
@@ -1069,8 +1073,8 @@ def decode_splits(pairs: int, n_cus: int, most: int) -> int:
     18 sequences 3,555 with 3, 3,375 with 5; 24 sequences 4,480 with none, 4,310 with 4;
     32 sequences 5,620 with none, 5,375 with 2; 40 sequences 5,990 with 3, 5,720 with none;
     56 sequences 7,330 with none, 7,000 with 2.  Below 8 sequences' worth of pairs (64) the
-    rule is about a block a CU.  (Where the kernel shares its blocks out by the sequences' lengths this is not their number:
-    ``shared_slots`` in ``attention.hip``.)"""
+    rule is about a block a CU.  (Where the kernel shares its blocks out by the sequences' lengths, ``lengths_differ``, this is not
+    their number: ``shared_slots`` in ``attention.hip``.)"""
     if pairs * 4 < n_cus:
         # a few sequences: about a block a CU (two pieces of each wave are then on their way); measured,
         # one block a CU against two: one sequence 277.5 against 274.8 tokens a second, two 542 against
@@ -1084,6 +1088,27 @@ def decode_splits(pairs: int, n_cus: int, most: int) -> int:
         if cost < best_cost - 1e-9:
             best, best_cost = s, cost
     return best
+
+
+def may_share(n_tokens: int, n_kv_heads: int, n_cus: int) -> bool:
+    """Whether there is a decode step of so many tokens whose blocks go by the lengths (``shared_slots`` in ``attention.hip``)."""
+    return 2 <= n_tokens <= 64 and 0 < n_cus < 8 * n_tokens * n_kv_heads
+
+
+UNEQUAL_LENGTHS = 1.5       # longest over mean
+
+
+def lengths_differ(lengths: Sequence[int]) -> bool:
+    """Whether a decode step's sequences differ enough in length for blocks of attention that go by the lengths.  Asked before a step
+    is launched and part of what it is recorded under; sequences that grow together become more alike, so a batch changes sides at most once.
+
+    Even splits keep the longest sequence's blocks running alone, shared ones cost each block the working out and a merge.  Measured (us with
+    the merge, 32 heads on 8, even and shared, the longest so many times the mean long): 8 sequences of 2,070 on average 1.0 19.8 and 20.2,
+    1.35 20.8 and 21.3, 1.6 22.1 and 21.0; 16 1.35 37.1 and 38.9, 1.6 39.7 and 37.3; 24 1.0 48.7 and 55.5, 1.2 50.9 and 49.6, 1.6 61.4 and 50.8; 32 1.35
+    64.2 and 65.7, 1.6 69.6 and 69.3; 40 1.6 79.2 and 80.6; 56 1.6 113.4 and 117.3; 4,000 keys to a quarter of that, 28 (1.8) 75.2 and 62.3, 40 (2.0)
+    89.5 and 80.5, to a tenth, 24 (2.4) 69.8 and 44.5, 56 (2.5) 136.7 and 105.3.  What loses beyond the line: batches of 40 to 56 of which a
+    quarter to a half are 8 times as long as the others, up to 6 %, 20 of them 7."""
+    return len(lengths) > 0 and len(lengths) * max(lengths) >= UNEQUAL_LENGTHS * sum(lengths)
 
 
 def attention_decode_fusable(dtype: torch.dtype, n_heads: int, n_kv_heads: int, head_dim: int, page: int,
@@ -1162,7 +1187,7 @@ def attention_decode_fused(qkv: torch.Tensor, out: torch.Tensor, k_cache: torch.
                            max_len: int = 0, n_splits: int = 0, row_scale: Optional[RowScale] = None,
                            bias: Optional[torch.Tensor] = None, chunk: Optional[int] = None,
                            slopes: Optional[torch.Tensor] = None, sink: bool = False, sinks: Optional[torch.Tensor] = None,
-                           keep_first: int = 0, values_are_keys: bool = False) -> None:
+                           keep_first: int = 0, values_are_keys: bool = False, unequal: bool = False) -> None:
     """A decode step's attention straight from the q/k/v projection ``qkv`` (float32
     ``[tokens, ld]``, or its split-K partial sums ``[splits, tokens, ld]``): per-head norm,
     rotation, append of the new key and value to the cache and attention over the cache in one
@@ -1170,7 +1195,7 @@ def attention_decode_fused(qkv: torch.Tensor, out: torch.Tensor, k_cache: torch.
     ``t`` of the block table).  ``workspace`` must not overlap ``qkv``.  ``row_scale``: the
     projection's operand lacked its norm's scale, which is applied to the projection's sums here.
     ``bias`` (32-bit, one number per column of a projection row) is added behind that scale;
-    ``chunk``, ``slopes``, ``sink``, ``sinks`` and ``keep_first`` as in ``attention``.  The tables may be narrower than half a
+    ``chunk``, ``slopes``, ``sink``, ``sinks``, ``keep_first``, ``n_splits`` and ``unequal`` as in ``attention``.  The tables may be narrower than half a
     head: its leading values turn.  ``values_are_keys``: the rows hold no value columns, the new value is the projected key
     (with its bias) before norm and rotation."""
     _dev(qkv, out, k_cache, v_cache, block_table, token_seq, token_pos, q_gain, k_gain, cos, sin, bias, slopes, sinks)
@@ -1230,7 +1255,7 @@ def attention_decode_fused(qkv: torch.Tensor, out: torch.Tensor, k_cache: torch.
         _ptr(qkv), ld, qkv_splits, split_stride, _ptr(q_gain), _ptr(k_gain), eps, _ptr(cos), _ptr(sin),
         1 if write_kv else 0, _ptr(out), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1],
         _ptr(token_seq), _ptr(token_pos), n_tokens, n_heads, n_kv_heads, head_dim, page, scale,
-        0 if window is None else int(window), max_len, n_splits, ws_ptr, ws_bytes, ssq_ptr, parts, row_eps, width,
+        0 if window is None else int(window), max_len, n_splits, 1 if unequal else 0, ws_ptr, ws_bytes, ssq_ptr, parts, row_eps, width,
         _ptr(bias), 0 if chunk is None else int(chunk), _ptr(slopes), 1 if sink else 0, _ptr(sinks), int(keep_first),
         0 if cos is None else 2 * cos.shape[-1], 1 if values_are_keys else 0, _stream()))
 

@@ -320,7 +320,7 @@ class Attention(Mixer):
             ops.attention_decode_fused(qkv, o, cache.k, cache.v, cache.block_table, None, step.token_pos,
                                        s.n_heads, s.n_kv_heads, s.head_dim, s.scale, self.q_gain, self.k_gain, eps,
                                        cos, sin, write_kv=owns_cache, window=s.window, workspace=scratch[used:],
-                                       max_len=step.max_len, n_splits=self._decode_splits(step, cache),
+                                       max_len=step.max_len, n_splits=self._decode_splits(step, cache), unequal=step.unequal,
                                        row_scale=stream(step).row_scale,
                                        bias=None if self.b_qkv is None else self.b_qkv[:rows], chunk=s.chunk,
                                        slopes=self.slopes, sink=s.sink, sinks=self.sinks, keep_first=self.keep_first,
@@ -358,7 +358,7 @@ class Attention(Mixer):
                 ops.attention(q, o, cache.k, cache.v, cache.block_table, step.token_seq, step.token_pos,
                               s.n_heads, s.n_kv_heads, s.head_dim, s.scale, s.window, workspace=ws.scratch(),
                               cu_seqlens=step.cu_seqlens, max_new=step.max_new, q_counts=step.new_counts,
-                              max_len=step.max_len, n_splits=self._decode_splits(step, cache),
+                              max_len=step.max_len, n_splits=self._decode_splits(step, cache), unequal=step.unequal,
                               v_head_dim=self.v_head_dim, chunk=s.chunk, slopes=self.slopes, sink=s.sink, sinks=self.sinks,
                               softcap=self.softcap, keep_first=self.keep_first)
         if s.gate:

@@ -70,20 +70,20 @@ def _build(seqs, hq, hkv, d, dtype, seed, spare_pages=3):
     return dev, ks, vs, qs
 
 
-def _run(dev, seqs, hq, hkv, d, scale, window, algo, n_splits=0):
+def _run(dev, seqs, hq, hkv, d, scale, window, algo, n_splits=0, unequal=False):
     out = torch.full_like(dev["q"], float("nan"))
     ws = torch.empty(32 << 20, dtype=torch.uint8, device="cuda")
     ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv,
                   d, scale, window, algo=algo, workspace=ws, cu_seqlens=dev["cu"],
                   max_new=max(n for _, n in seqs), q_counts=[n for _, n in seqs],
-                  max_len=max(length for length, _ in seqs), n_splits=n_splits)
+                  max_len=max(length for length, _ in seqs), n_splits=n_splits, unequal=unequal)
     return out.cpu()
 
 
-def _check(seqs, hq, hkv, d, dtype, algo, window=None, n_splits=0, seed=0):
+def _check(seqs, hq, hkv, d, dtype, algo, window=None, n_splits=0, seed=0, unequal=False):
     dev, ks, vs, qs = _build(seqs, hq, hkv, d, dtype, seed)
     scale = 1.0 / math.sqrt(d)
-    got = _run(dev, seqs, hq, hkv, d, scale, window, algo, n_splits).double().reshape(-1, hq, d)
+    got = _run(dev, seqs, hq, hkv, d, scale, window, algo, n_splits, unequal).double().reshape(-1, hq, d)
     at = 0
     tol = 1e-4 if dtype == torch.float32 else 1.5e-2     # bfloat16: probabilities and output are rounded
     for (length, n_new), k, v, q in zip(seqs, ks, vs, qs):
@@ -163,7 +163,7 @@ def test_a_far_key_decides():
             assert float((got[:, h] - want[h // (hq // hkv)]).abs().max()) < 2e-2
 
 
-def _fused_case(seqs, hq, hkv, d, qkv_splits, attn_splits, window, seed, norm=True, rotate=True):
+def _fused_case(seqs, hq, hkv, d, qkv_splits, attn_splits, window, seed, norm=True, rotate=True, unequal=False):
     """A decode step through the fused kernel: random projection output (cut into partial sums),
     gains and rotation angles; the position of every sequence's new token holds a large value in
     the cache beforehand, so a row that is not replaced shows.  Checked against the two-kernel
@@ -211,17 +211,17 @@ def _fused_case(seqs, hq, hkv, d, qkv_splits, attn_splits, window, seed, norm=Tr
                             n_splits=qkv_splits)
     ops.attention(q_dev, out2, kc2, vc2, dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, scale, window,
                   algo=MFMA, workspace=ws, cu_seqlens=dev["cu"], max_new=1, q_counts=[1] * n, max_len=max_len,
-                  n_splits=attn_splits)
+                  n_splits=attn_splits, unequal=unequal)
     out = torch.full_like(q_dev, float("nan"))
     kc3, vc3 = dev["kc"].clone(), dev["vc"].clone()
     ops.attention_decode_fused(parts_dev, out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"],
                                hq, hkv, d, scale, cuda(q_gain), cuda(k_gain), eps, cuda(cos), cuda(sin),
-                               window=window, workspace=ws, max_len=max_len, n_splits=attn_splits)
+                               window=window, workspace=ws, max_len=max_len, n_splits=attn_splits, unequal=unequal)
     # without the sequence table: token t is sequence t, as in this step
     out3 = torch.full_like(q_dev, float("nan"))
     ops.attention_decode_fused(parts_dev, out3, kc3, vc3, dev["table"], None, dev["tok_pos"],
                                hq, hkv, d, scale, cuda(q_gain), cuda(k_gain), eps, cuda(cos), cuda(sin),
-                               window=window, workspace=ws, max_len=max_len, n_splits=attn_splits)
+                               window=window, workspace=ws, max_len=max_len, n_splits=attn_splits, unequal=unequal)
     torch.cuda.synchronize()
     assert torch.equal(out, out3) and torch.equal(kc3, dev["kc"]) and torch.equal(vc3, dev["vc"])
     # the cache: a 32-bit sum in another order may round a value to the neighbouring bfloat16

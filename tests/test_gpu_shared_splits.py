@@ -19,9 +19,9 @@ SHARED = [(16, 8, 128, [1, 64, 65, 300, 2100]), (16, 8, 64, [1, 1, 1, 1, 1, 4000
 
 @pytest.mark.parametrize("hq,hkv,d,lengths", SHARED)
 def test_unequal_lengths(hq, hkv, d, lengths):
-    _check([(n, 1) for n in lengths], hq, hkv, d, torch.bfloat16, MFMA, n_splits=ops.decode_splits(len(lengths) * hkv, 256, 64), seed=5)
+    _check([(n, 1) for n in lengths], hq, hkv, d, torch.bfloat16, MFMA, n_splits=ops.decode_splits(len(lengths) * hkv, 256, 64), seed=5, unequal=True)
     if d != 96 and d != 32:
-        _fused_case([(n, 1) for n in lengths], hq, hkv, d, 2, ops.decode_splits(len(lengths) * hkv, 256, 64), None, seed=7)
+        _fused_case([(n, 1) for n in lengths], hq, hkv, d, 2, ops.decode_splits(len(lengths) * hkv, 256, 64), None, seed=7, unequal=True)
 
 
 @pytest.mark.parametrize("room", [1, 2, 5])
@@ -33,7 +33,7 @@ def test_little_workspace(room):
     ws = torch.full((size + 4096,), 0x7f, dtype=torch.uint8, device="cuda")
     out = torch.full_like(dev["q"], float("nan"))
     ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, d ** -0.5, None, algo=MFMA,
-                  workspace=ws[:size], cu_seqlens=dev["cu"], max_new=1, q_counts=[1] * len(lengths), max_len=max(lengths), n_splits=0)
+                  workspace=ws[:size], cu_seqlens=dev["cu"], max_new=1, q_counts=[1] * len(lengths), max_len=max(lengths), n_splits=0, unequal=True)
     assert bool((ws[size:] == 0x7f).all())
     for b, n in enumerate(lengths):
         want = _reference(qs[b], ks[b], vs[b], [n - 1], d ** -0.5, None)
@@ -49,7 +49,7 @@ def test_recorded_while_lengths_change():
 
     def step():
         ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, d ** -0.5, None, algo=MFMA,
-                      workspace=ws, cu_seqlens=dev["cu"], max_new=1, q_counts=[1] * len(lengths), max_len=max(lengths), n_splits=5)
+                      workspace=ws, cu_seqlens=dev["cu"], max_new=1, q_counts=[1] * len(lengths), max_len=max(lengths), n_splits=5, unequal=True)
     step()
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()
@@ -68,3 +68,44 @@ def test_recorded_while_lengths_change():
         for b, n in enumerate(now):
             want = _reference(qs[b], ks[b][:n], vs[b][:n], [n - 1], 1.0 / math.sqrt(d), None)
             assert float((replayed[b].cpu().double().view(1, hq, d) - want).abs().max()) < 1.5e-2, (sub, n, PAGE)
+
+
+@pytest.mark.parametrize("hq,hkv,d,n,length", [(16, 8, 128, 8, 2070), (8, 8, 128, 24, 700), (16, 8, 64, 6, 130)])
+def test_as_many_splits_as_asked_for(hq, hkv, d, n, length):
+    """Without ``unequal`` every token has ``n_splits`` splits, with one no merge: the workspace stays as it is."""
+    dev, ks, vs, qs = _build([(length - i, 1) for i in range(n)], hq, hkv, d, torch.bfloat16, 4)
+    for splits in (1, 3):
+        ws = torch.full((32 << 20,), 0x7f, dtype=torch.uint8, device="cuda")
+        out = torch.full_like(dev["q"], float("nan"))
+        ops.attention(dev["q"], out, dev["kc"], dev["vc"], dev["table"], dev["tok_seq"], dev["tok_pos"], hq, hkv, d, d ** -0.5, None, algo=MFMA,
+                      workspace=ws, cu_seqlens=dev["cu"], max_new=1, q_counts=[1] * n, max_len=length, n_splits=splits)
+        used = n * hq * (d + 2) * 4 * splits if splits > 1 else 0
+        assert bool((ws[used:] == 0x7f).all()) and (used == 0 or not bool((ws[used - 4096:used] == 0x7f).all()))
+        for b in range(0, n, 5):
+            want = _reference(qs[b], ks[b], vs[b], [length - b - 1], d ** -0.5, None)
+            assert float((out[b].cpu().double().view(1, hq, d) - want).abs().max()) < 1.5e-2
+
+
+def test_engine_batches_that_become_alike(tmp_path):
+    """Steps of a batch whose lengths differ by much and less and less run, and are recorded, as one launch and then the other; steps of
+    one length only as the other.  Bit for bit the logits of steps that are not recorded."""
+    from rocml_amd.engine import Engine, StepEntry
+    from rocml_amd.weights import load_model
+    from tests import helpers
+    cfg = dict(helpers.TINY_H, hidden_size=128, num_attention_heads=8, num_key_value_heads=8, head_dim=64)
+    path = helpers.make_model_dir(tmp_path, cfg, 31, torch.bfloat16)
+
+    def run(lengths, steps, use_graphs):
+        engine = Engine(load_model(path, dtype="bfloat16", device="cuda:0"), max_tokens=4096, use_graphs=use_graphs)
+        texts = [helpers.random_tokens(n + steps, cfg["vocab_size"], 3 + i) for i, n in enumerate(lengths)]
+        slots = [engine.new_sequence() for _ in lengths]
+        engine.step([StepEntry(s, t[:n], []) for s, t, n in zip(slots, texts, lengths)])
+        out = []
+        for k in range(steps):
+            out.append(engine.step([StepEntry(s, [t[n + k]], [0]) for s, t, n in zip(slots, texts, lengths)]).cpu())
+        return torch.stack(out), {key[3] for key, entry in engine._graphs.items() if key[0] != "prompt" and entry[1] is not None}
+
+    got, sides = run([10, 10, 11, 12, 100, 10], 160, True)
+    want, none = run([10, 10, 11, 12, 100, 10], 160, False)
+    assert torch.equal(got, want) and sides == {True, False} and not none
+    assert run([70] * 6, 5, True)[1] == {False}
