@@ -69,7 +69,7 @@ class Engine:
 
     def check_steps(self) -> None:
         """Raises if a step that has ended on the GPU gave no result (its logits are NaN: a wait between the blocks of a
-        launch lasted for seconds).  Told once; a step asks for those before it, whoever fetches results asks for the step they
+        launch lasted for seconds).  Told once; a step asks for all before the last one, whoever fetches results asks for the step they
         came from.  The sequences of the step have to be released, the engine goes on."""
         if self.workspace.was_late():
             raise StepFailedError("a step ended without a result: its blocks waited for each other for too long")
@@ -86,6 +86,10 @@ class Engine:
         spec = self.model.spec
         if not entries:
             return None
+        if torch.cuda.is_current_stream_capturing():
+            # (the recorded copy would bring whatever lies in the staging memory at a replay)
+            raise RocmlError("a step cannot be recorded from outside: its tables come from the host")
+        self._staging.wait()            # (all before the last step has ended: what it has to tell is there)
         self.check_steps()
         if device_ids is not None:
             if any(len(e.tokens) != 1 for e in entries) or device_ids.numel() != len(entries) \
@@ -194,9 +198,6 @@ class Engine:
         parts = [ids, seq, pos, cu, lens, slot_arr, want_rows] + [t.reshape(-1) for t in tables]
         size = sum(p.size for p in parts)
         meta = self.workspace.get("step.meta", (size,), torch.int32)
-        if torch.cuda.is_current_stream_capturing():
-            # (the recorded copy would bring whatever lies in the staging memory at a replay)
-            raise RocmlError("a step cannot be recorded from outside: its tables come from the host")
         staged = self._staging.take(size)
         np.concatenate(parts, out=staged.numpy())
         self._staging.send(staged, meta)
