@@ -7,9 +7,7 @@ namespace prompt {
 constexpr int ROWS = 64;                              // query rows of a wave, two tiles of 32
 constexpr int SLOTS = 4;                              // pages of keys, and of values, in LDS
 constexpr int TILE = 4 * ROWS;                        // query rows of a block
-// The sum of 16 probabilities up to which their rows keep the reference of their exponents, whatever their maxima: any reference
-// gives the same quotient, and 2^19 keys of 2^60 each times values of up to 2^40 still are 32-bit and bfloat16 numbers of full precision.
-constexpr float FAR = 0x1p60f, NEAR = 0x1p-60f;
+constexpr float MOST = 0x1p120f;                      // of a row's sum: its reciprocal is a number of all digits, too
 
 template <int D>
 struct Lds {
@@ -51,8 +49,11 @@ __device__ __forceinline__ int value_place(int piece, int row) { return piece ^ 
 //  * pages go from memory straight into swizzled LDS rows, asked for three and four visits before they are read; a barrier a page;
 //  * nobody covers for a wave that waits, so its instructions are laid out one by one: behind each product two or three vector operations of
 //    the softmax of the last 32 keys, operands read six pairs of products ahead, across steps and the page's barrier too;
-//  * a row's reference stays what the maximum of its first page gave (any reference gives the same quotient, see FAR), so no step
-//    looks for a maximum, and none has a branch but the one that hides keys on the diagonal.
+//  * a row's reference stays what the maximum of its first page gave, so no step looks for a maximum, and none has a branch but the one that
+//    hides keys on the diagonal.  Any reference gives the same quotient as long as the sums are numbers: probabilities, as bfloat16 and as
+//    32-bit, have all their digits up to 2^127.  A wave with a row whose sums are not (scores some 80 above the first page's largest, or
+//    something that is not finite) does its rows again at the end, with references that follow.  Heads whose queries and keys are normed
+//    and have gains of one never come near it (|score| <= sqrt(128) = 11.3).
 // Measured (32 query heads on 8; us, before and now): 8,192 tokens behind 24,576 others 4,038 and 3,108 (953 and 1,238 TFLOP/s), 8,192
 // alone 626 and 496, four of 3,000 423 and 337; the rule in attention.hip has more.  The matrix cores are busy 59 % of the time at 1.95 GHz, where the chip's power
 // holds the clock; the wave issues something 69 % of the time (5.4 vector operations a product) and waits for counters or the barrier 16 %.
@@ -214,14 +215,13 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     };
     // 32 keys that all rows see: their exponentials beside the next scores (keys of slot ks, half kh) and the products of the last
     // probabilities with their values (slot vs, half vh).  An operand is read AHEAD products' pairs before its products, the first ones by the step
-    // before (ks2 ... vh2: the next step's).  The rows' references stay as they are; far: whether a sum left the range in which they may.
+    // before (ks2 ... vh2: the next step's).  The rows' references stay as they are.
     constexpr int PAIRS = KK + 2 * DT, RING = 8, AHEAD = 6;
     static_assert(KK == 2 * DT && PAIRS % RING == 0, "scores and values in turn");
     bf16x8_t ring[RING];
     auto operand = [&](int j, int ks, int kh, int vs, int vh) __attribute__((always_inline)) {
         return j & 1 ? value_frag(vs, vh, (j >> 1) / DT, (j >> 1) % DT) : key_frag(ks, kh, j >> 1);
     };
-    bool far = false;
     auto step = [&](f32x16_t (&s)[2], f32x16_t (&next)[2], int ks, int kh, int vs, int vh, int ks2, int kh2, int vs2, int vh2,
                     auto between) __attribute__((always_inline)) {
         uint32_t pn[2][8];
@@ -258,7 +258,6 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
         finish(PAIRS - 1);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            far |= !(sum[t] <= FAR);
             l[t] += sum[t];
 #pragma unroll
             for (int u = 0; u < 2; ++u) pf[t][u] = __builtin_bit_cast(bf16x8_t, make_uint4(pn[t][4 * u], pn[t][4 * u + 1], pn[t][4 * u + 2], pn[t][4 * u + 3]));
@@ -313,9 +312,7 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
         add_values(v & 3, 0, pf);
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
-            const float sum = exponentials(sc[1][t], m[t], pf[t]);
-            far |= !(sum <= FAR);
-            l[t] += sum;
+            l[t] += exponentials(sc[1][t], m[t], pf[t]);
         }
         add_values(v & 3, 1, pf);
         ++v;
@@ -323,13 +320,12 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
     for (; v < n_visits; ++v) pass_by(v);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");   // no load is on its way into LDS when the block ends
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        l[t] = sum_across_halves(l[t]);
-        if (__builtin_amdgcn_ballot_w64(far)) l[t] = __builtin_nanf("");
-    }
+    for (int t = 0; t < 2; ++t) l[t] = sum_across_halves(l[t]);
     if (!active) return;
-    // Where a reference was too far from its row's maximum, or something is no finite number, the wave does its rows again: page after
-    // page straight from memory, with references that follow.
+    // Where a reference was too far from its row's maximum, or something is no finite number, the wave does its rows again: 32 keys at a
+    // time straight from memory, with references that follow.  Where all rows do (8,192 tokens, 32 heads, scores some 130 apart) the
+    // kernel takes 1,500 us (without it 489, attn_prefill_mfma_kernel 600); each of the wave's two tiles by itself 2,290, the
+    // next keys asked for ahead 1,520, references that follow inside the first pass 10 % more for all others.
     bool bad = false;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -338,26 +334,36 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int e = 0; e < 16; ++e) finite = fmaf(o[t][dt][e], 0.f, finite);
-        bad |= row_ok[t] && !(l[t] >= NEAR && l[t] < INFINITY && finite == 0.f);
+        bad |= row_ok[t] && !(l[t] > 0.f && l[t] < MOST && finite == 0.f);
     }
     if (__builtin_amdgcn_ballot_w64(bad)) {
+        int hi[2];                                      // the last key that a tile's rows see, -1: it has no rows
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             m[t] = -INFINITY;
             l[t] = 0.f;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) o[t][dt] = zero;
-            const int t_lo = w_lo + t * 32, t_hi = min(n_new - 1, t_lo + 31);
-            if (t_lo >= n_new) continue;
+            hi[t] = w_lo + t * 32 < n_new ? pos0 + min(n_new - 1, w_lo + t * 32 + 31) : -1;
+        }
 #pragma unroll 1
-            for (int key0 = 0; key0 <= pos0 + t_hi; key0 += 32) {
-                const size_t page = (size_t)pages[key0 / AM_PAGE] * hkv + kvh;
-                const bf16_t* krow = kcache + (page * AM_PAGE + key0 % AM_PAGE + key_of_row(col)) * D + h2 * 8;
-                const bf16_t* vrow = vcache + (page * D + col) * AM_PAGE + key0 % AM_PAGE + h2 * 8;
+        for (int key0 = 0; key0 <= max(hi[0], hi[1]); key0 += 32) {
+            const size_t page = (size_t)pages[key0 / AM_PAGE] * hkv + kvh;
+            const bf16_t* krow = kcache + (page * AM_PAGE + key0 % AM_PAGE + key_of_row(col)) * D + h2 * 8;
+            const bf16_t* vrow = vcache + (page * D + col) * AM_PAGE + key0 % AM_PAGE + h2 * 8;
+            bf16x8_t kf[KK], vf[DT][2];
+#pragma unroll
+            for (int kk = 0; kk < KK; ++kk) kf[kk] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(krow + kk * 16));
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) vf[dt][u] = __builtin_bit_cast(bf16x8_t, *(const uint4*)(vrow + dt * 32 * AM_PAGE + u * 16));
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                if (key0 > hi[t]) continue;             // (what is not finite there is none of these rows')
                 f32x16_t s = zero;
 #pragma unroll
-                for (int kk = 0; kk < KK; ++kk)
-                    s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, *(const uint4*)(krow + kk * 16)), qf[t][kk], s, 0, 0, 0);
+                for (int kk = 0; kk < KK; ++kk) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[kk], qf[t][kk], s, 0, 0, 0);
                 float mx = -INFINITY;
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
@@ -374,13 +380,12 @@ attn_prompt_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
 #pragma unroll
                     for (int e = 0; e < 16; ++e) o[t][dt][e] *= corr;
 #pragma unroll
-                    for (int u = 0; u < 2; ++u)
-                        o[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8_t, *(const uint4*)(vrow + dt * 32 * AM_PAGE + u * 16)), pf[t][u], o[t][dt], 0, 0, 0);
+                    for (int u = 0; u < 2; ++u) o[t][dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt][u], pf[t][u], o[t][dt], 0, 0, 0);
                 }
             }
-            l[t] = sum_across_halves(l[t]);
         }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) l[t] = sum_across_halves(l[t]);
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {

@@ -102,6 +102,28 @@ def test_references_that_are_left_behind(jump):
     _check(got, _exact(q, k, vs[0], 0, 1.0))
 
 
+@pytest.mark.parametrize("a_page", [3.0, 25.0, 55.0])
+def test_references_that_stay_or_follow(a_page):
+    """Scores that climb by so much a page (in all by 4 to 76, and by 47 to 860), for some rows and heads, and fall or stay for the others:
+    up to some 80 the first page's reference does, beyond it the rows are done again, beside rows that keep theirs."""
+    seqs = [(1000, 1000)]
+    dev, ks, vs, qs = _build(seqs, 4, 2, D, torch.bfloat16, seed=10)
+    q, k = qs[0], ks[0]
+    q[..., 0] = 8.0
+    q[::3, :, 0] = 0.0
+    q[1::7, :, 0] = -8.0
+    q[:, 3, 0] = 1.0
+    k[:, 0, 0] = torch.arange(1000) // 16 * (a_page / 4.0 / 8.0)
+    dev["q"].copy_(q.view(1000, -1))
+    for page in range((1000 + PAGE - 1) // PAGE):
+        rows = k[page * PAGE:(page + 1) * PAGE]
+        dev["kc"][int(dev["table"][0, page]), :, :rows.shape[0]] = rows.transpose(0, 1).cuda()
+    got = _run(dev, seqs, 4, 2, D, SCALE, None, ops.ATTN_PROMPT).view(-1, 4, D)
+    _check(got, _exact(q, k, vs[0], 0))
+    got = _run(dev, seqs, 4, 2, D, 1.0, None, ops.ATTN_PROMPT).view(-1, 4, D)
+    _check(got, _exact(q, k, vs[0], 0, 1.0))
+
+
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 @pytest.mark.parametrize("where", ["key", "value"])
 def test_numbers_that_are_not_finite_stay_with_the_rows_that_see_them(where, value):
