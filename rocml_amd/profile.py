@@ -131,6 +131,12 @@ def _tensor_args_cost(skip: Tuple[int, ...] = (), flops_per_byte: float = 0.0) -
     return cost
 
 
+def _added_conv_cost(h, w, state, slots) -> Tuple[int, int]:
+    """The taps and the kept rows of a convolution on a mixer's input, without the rows themselves."""
+    kept = 0 if state is None else 2 * slots.numel() * state.shape[1] * state.shape[2] * state.element_size()
+    return _nbytes(w) + kept, 2 * w.shape[0] * h.numel()
+
+
 # launch helper -> (label of the report row, bytes and flops of a call)
 _COSTS: Dict[str, Tuple[str, Callable]] = {
     "gemm": ("product", _gemm_cost),
@@ -163,12 +169,13 @@ _COSTS: Dict[str, Tuple[str, Callable]] = {
     "sigmoid_gate": ("output gate", lambda y, gate, **kw: (2 * _nbytes(y) + gate.numel() * 4, 4 * y.numel())),
     "qk_span_stats": ("q/k norm factors", lambda qkv, q_width, k_width, bias, eps, out: (
         qkv.shape[0] * (q_width + k_width) * qkv.element_size() + _nbytes(out), 2 * qkv.shape[0] * (q_width + k_width))),
-    "norm_add": (lambda *a, **kw: "sublayer norm, residual sum and the next norm" if kw.get("next_gain") is not None
-                 else "sublayer norm and residual sum", lambda x, y, gain, bias, eps, **kw: (
-        2 * _nbytes(x) + _nbytes(kw.get("copy"), kw.get("partials")) + (0 if kw.get("replace") else _nbytes(y)), 8 * x.numel())),
-    "added_conv": ("convolution on the mixer's input", lambda h, w, state, cu, slots, counts, out: (
-        _nbytes(h, out, w) + (0 if state is None else 2 * slots.numel() * state.shape[1] * state.shape[2] * state.element_size()),
-        2 * w.shape[0] * h.numel())),
+    "norm_add": (lambda *a, **kw: "sublayer norm, residual sum, next norm and convolution" if kw.get("conv") is not None
+                 else "sublayer norm, residual sum and the next norm" if kw.get("next_gain") is not None
+                 else "sublayer norm and residual sum", lambda x, y, gain, bias, eps, **kw: tuple(a + b for a, b in zip((
+                     2 * _nbytes(x) + _nbytes(kw.get("copy"), kw.get("partials")) + (0 if kw.get("replace") else _nbytes(y)), 8 * x.numel()),
+                     (0, 0) if kw.get("conv") is None else _added_conv_cost(x, *kw["conv"])))),
+    "added_conv": ("convolution on the mixer's input", lambda h, w, state, cu, slots, counts, out: tuple(a + b for a, b in zip(
+        (_nbytes(h, out), 0), _added_conv_cost(h, w, state, slots)))),
     "activate": ("activation", lambda x, out, activation: (_nbytes(x, out), 4 * x.numel())),
     "norm_add_branches": ("branch norms, sublayer norm and residual sum", lambda x, branches, gains, weight, beps, gain, bias, eps, layer, **kw: (
         2 * _nbytes(x) + _nbytes(*branches) + _nbytes(kw.get("copy")), 8 * x.numel() * (1 + len(branches)))),
