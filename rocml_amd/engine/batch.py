@@ -54,7 +54,7 @@ def pack_step(slots: Sequence[int], starts: Sequence[int], tokens: Sequence[Sequ
     """Host arrays of a packed step: ids, sequence index and position per token, offsets,
     final lengths."""
     if all(len(t) == 1 for t in tokens):        # a decode step: the host may be what it waits for
-        first, n = np.asarray(starts, dtype=np.int32), len(tokens)
+        first, n = np.array(starts, dtype=np.int32), len(tokens)       # (a copy: it is the table of positions)
         return (np.asarray([t[0] for t in tokens], dtype=np.int32), np.arange(n, dtype=np.int32), first,
                 np.arange(n + 1, dtype=np.int32), first + 1, np.asarray(slots, dtype=np.int32))
     counts = np.asarray([len(t) for t in tokens], dtype=np.int32)
