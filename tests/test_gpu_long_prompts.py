@@ -48,6 +48,22 @@ def test_tiles_pages_and_cuts(seqs, hq, hkv):
         at += n
 
 
+@pytest.mark.parametrize("algo", [ops.ATTN_MFMA, ops.ATTN_PROMPT])
+@pytest.mark.parametrize("n_seqs,longer", [(16, {0: 300, 15: 513}), (17, {0: 513, 15: 129, 16: 257}), (64, {15: 257, 16: 300, 63: 513}),
+                                           (65, {0: 130, 63: 300, 64: 600}), (70, {16: 129, 62: 257, 64: 300, 69: 513})])
+def test_many_sequences_of_more_than_a_tile(n_seqs, longer, algo):
+    """A tile's sequence and place in it are found in a walk up to 16 sequences and 64 at a time beyond: sequences of several tiles first,
+    last and at the edges of those groups, beside some of one token."""
+    counts = [longer.get(i, 1 + 5 * i % 97) for i in range(n_seqs)]
+    seqs = [(n + (0 if i % 3 else 40), n) for i, n in enumerate(counts)]
+    dev, ks, vs, qs = _build(seqs, 2, 1, D, torch.bfloat16, seed=n_seqs)
+    got = _run(dev, seqs, 2, 1, D, SCALE, None, algo).view(-1, 2, D)
+    at = 0
+    for (length, n), k, v, q in zip(seqs, ks, vs, qs):
+        _check(got[at:at + n], _exact(q, k, v, length - n))
+        at += n
+
+
 def test_the_rule_takes_it_and_both_ways_agree():
     """A prompt that the library's own rule gives to this kernel (its bits are those of the forced one, not of the other kernel)."""
     seqs = [(3100, 3100)]
