@@ -712,10 +712,6 @@ attn_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
                          const int* __restrict__ cu_seqlens, int n_seqs,
                          const int* __restrict__ token_pos, int hq, int hkv, float scale_log2e,
                          int window, PrefillProj pj, MaskExtra mx = MaskExtra{}) {
-    // Pages on their way in registers while one is multiplied.  Two: what a lone block on a CU waits for beside its products (32 heads
-    // of 128, us with one and with two: a prompt of 700 31.4 and 29.5, of 1,500 64.3 and 58.7, 64 of 16 to 700 185 and 169, full rounds of
-    // blocks equal).  Heads of 64 and 96 gain as much alone and lose 2 % with all CUs full, 192 loses 4 to 8, 256 has no registers for it.
-    constexpr int AHEAD = D == 128 ? 2 : 1;
     static_assert(!(QPREP && EXTRA), "the kernel that prepares its queries knows plain layers only");
     using L = PrefillLds<D>;
     const int chunk = EXTRA ? mx.chunk : 0;
@@ -785,157 +781,51 @@ attn_prefill_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[i][e] = 0.f;
 
-    // A page's keys and values wait in registers while the AHEAD pages before it are multiplied out of
-    // LDS: the loads of page p + AHEAD are issued right after page p has been written to LDS.
+    // A page's keys and values wait in registers while the page before it is multiplied out of
+    // LDS: the loads of page p + 1 are issued right after page p has been written to LDS.  (Two pages on their way: 300 tokens on 32
+    // heads of 128 14.5 -> 14.8 us, 12 prompts of 20 to 660 14.6 -> 15.8, with a sink 1,500 tokens 61.0 -> 65.7.)
     typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
     constexpr int K_PIECES = AM_PAGE * D / 8 / AM_THREADS, V_PIECES = D * AM_PAGE / 8 / AM_THREADS;
-    u32x4 kreg[AHEAD][K_PIECES], vreg[AHEAD][V_PIECES];
+    u32x4 kreg[K_PIECES], vreg[V_PIECES];
     int first_page = blk_first_key / AM_PAGE, last_page = blk_last_key / AM_PAGE;
     // kept first positions: their pages before the window's come first, then the window's
     const int keep = EXTRA ? mx.keep_first : 0;
     const int kept_pages = EXTRA ? min(first_page, (keep + AM_PAGE - 1) / AM_PAGE) : 0;
     auto logical_page = [&](int i) { return EXTRA && i < kept_pages ? i : first_page + i - kept_pages; };
     const int n_visits = last_page - first_page + 1 + kept_pages;
-    auto load_page = [&](int lp, u32x4 (&kr)[K_PIECES], u32x4 (&vr)[V_PIECES]) {
-        const int phys = pages[lp];
-        const u32x4* gk = (const u32x4*)(kcache + ((size_t)phys * hkv + kvh) * AM_PAGE * D);
-        const u32x4* gv = (const u32x4*)(vcache + ((size_t)phys * hkv + kvh) * D * AM_PAGE);
-#pragma unroll
-        for (int i = 0; i < K_PIECES; ++i) kr[i] = gk[tid + i * AM_THREADS];
-#pragma unroll
-        for (int i = 0; i < V_PIECES; ++i) vr[i] = gv[tid + i * AM_THREADS];
-    };
+#define AM_LOAD_PAGE(lp_)                                                                         \
+    {                                                                                             \
+        int phys_ = pages[lp_];                                                                   \
+        const u32x4* gk_ = (const u32x4*)(kcache + ((size_t)phys_ * hkv + kvh) * AM_PAGE * D);    \
+        const u32x4* gv_ = (const u32x4*)(vcache + ((size_t)phys_ * hkv + kvh) * D * AM_PAGE);    \
+        _Pragma("unroll") for (int i = 0; i < K_PIECES; ++i) kreg[i] = gk_[tid + i * AM_THREADS]; \
+        _Pragma("unroll") for (int i = 0; i < V_PIECES; ++i) vreg[i] = gv_[tid + i * AM_THREADS]; \
+    }
     // the wave's rows see every key of a 32-key piece when the piece lies at or below the first
     // row's position and at or above the last row's window start; only then masking is skipped
     int wave_min_pos = pos0 + w_lo;
     int wave_max_lo = am_first_key(pos0 + w_hi, window, chunk);
     bool wave_full = w_hi - w_lo == 31;
-    load_page(logical_page(0), kreg[0], vreg[0]);
-    if (AHEAD == 2 && n_visits > 1) load_page(logical_page(1), kreg[AHEAD - 1], vreg[AHEAD - 1]);
-    auto visit_page = [&](int visit, u32x4 (&kreg)[K_PIECES], u32x4 (&vreg)[V_PIECES]) {
-        const int lpage = logical_page(visit);
-        __syncthreads();                                // the previous page has been consumed
-#pragma unroll
-        for (int i = 0; i < K_PIECES; ++i) {
-            int piece = tid + i * AM_THREADS;
-            int key = piece / (D / 8), dc = piece % (D / 8);
-            *(u32x4*)(sk + key * L::K_ROW + dc * 8) = kreg[i];
+    AM_LOAD_PAGE(logical_page(0))
+    // A visit, as a function or in the loop: the compiler gives the two different registers.  As a function 128 a lane instead of 136 for
+    // heads of 64, 164 and 178 for 96, and fewer moves (us in the loop and as a function: a prompt of 300 tokens on 32 heads of 128 15.6 and
+    // 14.5, 64 of 20 to 540 90.9 and 88.2; of 64 12.9 and 11.9, 44.9 and 40.4; 128 tokens of 64 behind 3,000 53.5 and 57.3), but 388 and 372 for
+    // 192 and moves between the register files (1,500 tokens 78.0 and 80.4; of 256 97.2 and 102.0).
+    if constexpr (D <= 128) {
+        auto visit_page = [&](int visit, u32x4 (&kreg)[K_PIECES], u32x4 (&vreg)[V_PIECES]) {
+#define AM_LEAVE return
+#include "attention_prefill_visit.h"
+#undef AM_LEAVE
+        };
+        for (int visit = 0; visit < n_visits; ++visit) visit_page(visit, kreg, vreg);
+    } else {
+        for (int visit = 0; visit < n_visits; ++visit) {
+#define AM_LEAVE continue
+#include "attention_prefill_visit.h"
+#undef AM_LEAVE
         }
-#pragma unroll
-        for (int i = 0; i < V_PIECES; ++i) {
-            int piece = tid + i * AM_THREADS;
-            // Within 16 keys the four groups of 4 stand in the order 0, 2, 1, 3: the second product
-            // wants keys {4h .. 4h+3, 8+4h .. 8+4h+3} per lane (the order the scores come in), and
-            // so finds them side by side, one 16-byte read.
-            int d = piece / 8, kc = piece % 8;
-            uint2* dst = (uint2*)(sv + d * L::V_ROW + (kc >> 1) * 16 + (kc & 1) * 4);
-            dst[0] = make_uint2(vreg[i][0], vreg[i][1]);
-            dst[2] = make_uint2(vreg[i][2], vreg[i][3]);
-        }
-        __syncthreads();
-        if (visit + AHEAD < n_visits) load_page(logical_page(visit + AHEAD), kreg, vreg);
-        if (!wave_active) return;
-        // The scores of both 32-key halves are started before either is finished: the softmax of
-        // the first half (vector ALU) then runs while the matrix core still multiplies the second,
-        // and the softmax of the second while the first half's values are multiplied.
-        // S^T: element e of s is key 8(e/4) + 4 h2 + e%4, column = query row.
-        int page_key0 = lpage * AM_PAGE;
-        bool live[2];
-        f32x16_t sc[2];
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            int key0 = page_key0 + half * 32;
-            live[half] = !(key0 > wave_last_key || (key0 + 31 < wave_first_key && !(EXTRA && key0 < keep)));   // wave-uniform
-            if (!live[half]) continue;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) sc[half][e] = 0.f;
-            const bf16_t* krow = sk + (half * 32 + col) * L::K_ROW + h2 * 8;
-#pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                bf16x8_t kf = __builtin_bit_cast(bf16x8_t, *(const uint4*)(krow + kk * 16));
-                sc[half] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[kk], sc[half], 0, 0, 0);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            if (!live[half]) continue;
-            int key0 = page_key0 + half * 32;
-            f32x16_t& s = sc[half];
-            bool need_mask = !wave_full || key0 + 31 > wave_min_pos || key0 < wave_max_lo;   // wave-uniform
-            if constexpr (EXTRA) {
-                if (cap_out != 0.f) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) s[e] = am_tanh(s[e] * cap_in) * cap_out;
-                }
-            }
-            if (need_mask) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    int key = key0 + 8 * (e >> 2) + 4 * h2 + (e & 3);
-                    s[e] = (row_ok && key <= my_pos && (key >= my_lo || (EXTRA && key < keep))) ? s[e] : -INFINITY;
-                }
-            }
-            if constexpr (EXTRA) {
-                if (kslope != 0.f) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        int key = key0 + 8 * (e >> 2) + 4 * h2 + (e & 3);
-                        s[e] -= kslope * (float)(my_pos - key);
-                    }
-                }
-            }
-            float mx = s[0];
-#pragma unroll
-            for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
-            mx = max_across_halves(mx) * scale_log2e;       // the scale is positive
-            // The exponents' reference m follows a row's maximum only when that has grown by more
-            // than AM_LAZY_MAX (powers of two): any reference gives the same quotient at the end,
-            // the probabilities stay below 2^AM_LAZY_MAX, which bfloat16 and the 32-bit sums hold
-            // with room to spare, and the sums and outputs so far have to be rescaled (64 products
-            // a lane) only for the first pieces of a row instead of whenever one of a wave's 32
-            // rows meets a new maximum, which with a thousand keys behind it is still every other piece.
-            if (__builtin_amdgcn_ballot_w64(mx > m + AM_LAZY_MAX)) {
-                float m_new = fmaxf(m, mx);
-                float corr = fast_exp2(m - (m_new == -INFINITY ? 0.f : m_new));
-                l *= corr;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) o[dt][e] *= corr;
-                m = m_new;
-            }
-            float m_use = m == -INFINITY ? 0.f : m;
-            float sum = 0.f;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                s[e] = fast_exp2(fmaf(s[e], scale_log2e, -m_use));
-                sum += s[e];
-            }
-            sum = sum_across_halves(sum);
-            l += sum;
-            // P^T operands: MFMA u takes elements 8u..8u+7 = keys 16u + {4 h2 .. +3, 8 + 4 h2 .. +3}.
-            bf16x8_t pf[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-                pf[u] = __builtin_bit_cast(bf16x8_t, make_uint4(
-                    pack_bf16x2(s[8 * u + 0], s[8 * u + 1]), pack_bf16x2(s[8 * u + 2], s[8 * u + 3]),
-                    pack_bf16x2(s[8 * u + 4], s[8 * u + 5]), pack_bf16x2(s[8 * u + 6], s[8 * u + 7])));
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) {
-                    const bf16_t* vrow = sv + (dt * 32 + col) * L::V_ROW + half * 32 + 16 * u + 8 * h2;
-                    bf16x8_t vf = __builtin_bit_cast(bf16x8_t, *(const uint4*)vrow);
-                    o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf[u], o[dt], 0, 0, 0);
-                }
-            }
-        }
-    };
-    for (int visit = 0; visit < n_visits; visit += AHEAD) {
-        visit_page(visit, kreg[0], vreg[0]);
-        if (AHEAD == 2 && visit + 1 < n_visits) visit_page(visit + 1, kreg[AHEAD - 1], vreg[AHEAD - 1]);
     }
+#undef AM_LOAD_PAGE
     if (!row_ok) return;
     float inv = 1.0f / l;
     bf16_t* orow = out + ((size_t)(tok0 + my_row) * hq + h) * D;
