@@ -536,9 +536,9 @@ attn_decode_mfma_kernel(const bf16_t* __restrict__ q, bf16_t* __restrict__ out,
         }
 }
 
-// Log-sum-exp merge of the splits in split order (rocml-kernels/kernels/attn_decode.hip:219-255).  n_splits: the room a row has for
-// them; a maximum of -inf with a sum of 0 marks those it does not have, whose partial outputs may be anything.
-template <int D>
+// Log-sum-exp merge of the splits in split order (rocml-kernels/kernels/attn_decode.hip:219-255).  MARKED: n_splits is the room a row has
+// for them; a maximum of -inf with a sum of 0 marks those it does not have, whose partial outputs may be anything.
+template <int D, bool MARKED>
 __global__ void attn_decode_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                           bf16_t* __restrict__ out, int n_splits) {
     // At most 64 splits: lane s of every wave fetches split s's maximum and sum, so the loads
@@ -558,7 +558,7 @@ __global__ void attn_decode_reduce_kernel(const float* __restrict__ part_o, cons
 #pragma unroll
     for (int s = 0; s < 8; ++s) first[s] = po[(size_t)min(s, n_splits - 1) * D + d];
     const int room = n_splits;
-    n_splits = 64 - __builtin_clzll(__ballot(!(ms == -INFINITY && ls == 0.f)) | 1ull);
+    if constexpr (MARKED) n_splits = 64 - __builtin_clzll(__ballot(!(ms == -INFINITY && ls == 0.f)) | 1ull);
     float mm = wave_max(ms);
     float w = ms == -INFINITY ? 0.f : fast_exp2(ms - mm);
     if (threadIdx.x < 64) wgt[lane] = w;
@@ -568,7 +568,7 @@ __global__ void attn_decode_reduce_kernel(const float* __restrict__ part_o, cons
     // finite values: no branches)
     float acc = 0.f;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) acc += (s < n_splits || n_splits == room ? first[s] : 0.f) * wgt[s];
+    for (int s = 0; s < 8; ++s) acc += (!MARKED || s < n_splits || n_splits == room ? first[s] : 0.f) * wgt[s];
     for (int s0 = 8; s0 < n_splits; s0 += 8) {
         float more[8];
 #pragma unroll
