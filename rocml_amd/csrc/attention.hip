@@ -181,10 +181,14 @@ static bool prompt_takes(const AttnArgs& a, int d) { return d == 128 && !a.has_e
 
 // Whether it is the faster way.  Its blocks have twice the rows of attn_prefill_mfma_kernel's and a CU holds one, so each pays for its
 // start and end (some 10 us) by itself and a page takes 1.6 to 1.75 us for 256 rows where the other takes 1.8 to 2.4: it wants blocks of
-// many pages, and enough of them to fill the chip.  Measured (32 query heads on 8, us, the other kernel first): prompts of 1,024 tokens,
-// one 31 and 35, four 70 and 68; of 1,536, one 45 and 46, four 118 and 113; of 2,048 (18 pages a block), one (a block a CU) 60 and 59, two
-// 97 and 83, four 176 and 164; of 3,000 (26 pages), one 112 and 85, on 16 heads (192 blocks) 101 and 74; of 8,192 599 and 499, behind
-// 24,576 others 4,038 and 3,108.  With a window of 2,048 4,096 tokens take 136 and 148, which is why windows stay with the other.
+// many pages, and enough of them to fill the chip.  Measured (32 query heads on 8, us, the other kernel first; a tile's pages on average):
+// taken, 24 pages and three quarters of a block a CU: one prompt of 3,000 108 and 81, on 16 heads 98 and 73, on 40 114 and 100; of 4,096
+// 158 and 134, on 16 heads (a block a CU) 100 and 100; of 8,192 572 and 479, behind 24,576 others 4,038 and 3,108; 17 pages and two blocks a
+// CU: two prompts of 2,048 93 and 79, four 167 and 157, eight 338 and 313.  Not taken: one prompt of 2,048 54 and 57, of 1,536 42 and 45, of
+// 1,024 31 and 35, four 64 and 62, on 40 heads 66 and 73, sixteen 206 and 213.  Between, it goes by how either kernel's tiles fall into rounds of
+// blocks, and the lines leave out what gains in some places: one prompt of 2,304 64 and 64, on 64 heads 104 and 106, of 2,500 89 and 70, of 2,560 73 and
+// 72; two of 1,700 75 and 64; four of 1,536 104 and 100; three of 1,800 117 and 113, on 40 heads 141 and 147.
+// With a window of 2,048 4,096 tokens take 136 and 148, which is why windows stay with the other.
 // The positions before the step's first token are not known here: a step behind many others counts as if it were the first.
 static bool prompt_pays(const AttnArgs& a) {
     long long tiles = 0, pages = 0;
