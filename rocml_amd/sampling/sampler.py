@@ -88,7 +88,8 @@ class DeviceSampler:
         words = batch * (6 + window)
         if self._stage_dev is None or self._stage_dev.numel() < words:
             self._stage_dev = torch.empty(2 * words, dtype=torch.int32, device=self.device)
-        staged = self._staging.take(words)
+        recorded = torch.cuda.is_current_stream_capturing()
+        staged = self._staging.take(words, recorded)
         stage = staged.numpy()
         stage[:] = 0
         temperature, uniform, top_p, penalty = (stage[i * batch:(i + 1) * batch].view(np.float32) for i in range(4))
@@ -112,7 +113,7 @@ class DeviceSampler:
         drawing = top_k[temperature > 0]
         small_k = int(drawing.max()) if drawing.size and drawing.min() >= 1 and drawing.max() <= ops.SAMPLE_SMALL_K else 0
         dev = self._stage_dev[:words]
-        self._staging.send(staged, dev)
+        self._staging.send(staged, dev, recorded)
         floats = dev[:4 * batch].view(torch.float32)
         ops.sample(logits, self._work, floats[:batch], floats[batch:2 * batch], out,
                    top_k=dev[4 * batch:5 * batch], top_p=floats[2 * batch:3 * batch],

@@ -16,7 +16,7 @@ class Staging:
     """One pinned buffer of 32-bit words, filled again only when its copy has ended: the host is at most one copy ahead of the
     device, whichever streams they went to.  (Four buffers in turn: 16.01 and 16.05, 62.48 and 62.47, 34.48 and 34.51 ms of the above.)
 
-    Under a stream capture nothing is waited for and the copy is recorded as it is: a replay brings what then lies in the buffer."""
+    ``recorded``: under a stream capture.  Nothing is waited for and the copy is recorded as it is: a replay brings what then lies in the buffer."""
 
     def __init__(self):
         self._buffer: Optional[torch.Tensor] = None
@@ -27,19 +27,19 @@ class Staging:
         if self._sent is not None:
             self._sent.synchronize()
 
-    def take(self, words: int) -> torch.Tensor:
+    def take(self, words: int, recorded: bool = False) -> torch.Tensor:
         """``words`` 32-bit integers of pinned memory to fill and hand to ``send``."""
-        if not torch.cuda.is_current_stream_capturing():
+        if not recorded:
             self.wait()
         if self._buffer is None or self._buffer.numel() < words:
             # (sizes differ from step to step: room for twice as many, so that they settle soon)
             self._buffer = torch.empty(max(2 * words, 64), dtype=torch.int32, pin_memory=True)
         return self._buffer[:words]
 
-    def send(self, staged: torch.Tensor, dest: torch.Tensor) -> None:
+    def send(self, staged: torch.Tensor, dest: torch.Tensor, recorded: bool = False) -> None:
         """Queues the copy of what ``take`` gave to ``dest`` on the current stream."""
         dest.copy_(staged, non_blocking=True)
-        if torch.cuda.is_current_stream_capturing():
+        if recorded:
             return
         if self._sent is None:
             self._sent = torch.cuda.Event()

@@ -46,10 +46,9 @@ def test_a_capture_waits_for_nothing(device):
     staging, dest = Staging(), torch.zeros(8, dtype=torch.int32)
     staging.send(staging.take(8), dest)
     before = list(device.said)
-    device.capturing = True
-    staged = staging.take(8)
-    assert staged.data_ptr() == staging.take(8).data_ptr()          # the buffer that a replay will read
-    staging.send(staged, dest)
+    staged = staging.take(8, recorded=True)
+    assert staged.data_ptr() == staging.take(8, recorded=True).data_ptr()          # the buffer that a replay will read
+    staging.send(staged, dest, recorded=True)
     assert device.said == before
 
 
