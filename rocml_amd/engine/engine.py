@@ -79,7 +79,9 @@ class Engine:
         """Runs the entries' tokens; returns ``[n_wanted, vocab]`` 32-bit logits on the
         device in the order of the entries and of their ``want`` lists, or None when
         nothing is wanted.  The result is a buffer of the engine and holds until the next
-        step.  ``device_ids`` (int32 on the device, one per entry, every entry bringing one
+        step.  Which kernels run, and into how many pieces their sums are cut, goes by the whole step: the last bits of a
+        sequence's logits depend on how many others it brings, and in decode, where lengths differ by much
+        (``ops.lengths_differ``), on their lengths.  ``device_ids`` (int32 on the device, one per entry, every entry bringing one
         token): the token ids are taken from there instead of from the entries, whose tokens
         only stand for their number; for ids that a sampler has just drawn and the host has not
         seen yet."""
