@@ -1107,7 +1107,7 @@ def lengths_differ(lengths: Sequence[int]) -> bool:
     1.35 20.8 and 21.3, 1.6 22.1 and 21.0; 16 1.35 37.1 and 38.9, 1.6 39.7 and 37.3; 24 1.0 48.7 and 55.5, 1.2 50.9 and 49.6, 1.6 61.4 and 50.8; 32 1.35
     64.2 and 65.7, 1.6 69.6 and 69.3; 40 1.6 79.2 and 80.6; 56 1.6 113.4 and 117.3; 4,000 keys to a quarter of that, 28 (1.8) 75.2 and 62.3, 40 (2.0)
     89.5 and 80.5, to a tenth, 24 (2.4) 69.8 and 44.5, 56 (2.5) 136.7 and 105.3.  What loses beyond the line: batches of 40 to 56 of which a
-    quarter to a half are 8 times as long as the others, up to 6 %, 20 of them 7."""
+    quarter to a half are 8 times as long as the others, up to 6 %, 20 of them 7, 16 with one of twice the others' length 4."""
     return len(lengths) > 0 and len(lengths) * max(lengths) >= UNEQUAL_LENGTHS * sum(lengths)
 
 
